@@ -646,30 +646,17 @@ static bool run_mul_mat_q(exec_state & st, const ggml_tensor * w, const ggml_ten
         c->st.kernel_launches++;
         return true;
     }
-    const bool q80_skinny = w->type == GGML_TYPE_Q8_0 && !w2 && !add2 && mmq_q80_skinny_supported(w->type, K, N, M);
-    // the prompt GEMM over Q8_0 weights reads both operands in panel order when the weights have their panel copy (GGML_MI355X_Q80_GEMM_PANELS=0: as before round 6)
-    static const bool gemm_panels = !getenv("GGML_MI355X_Q80_GEMM_PANELS") || atoi(getenv("GGML_MI355X_Q80_GEMM_PANELS")) != 0;
-    const bool q80_gemm = !q80_skinny && w->type == GGML_TYPE_Q8_0 && M >= c->opt.q80_min_cols && !w2 && !add2 && mmq_q80_supported(w->type, K, N, M);
-    const uint8_t * q80_gemm_wp = (q80_gemm && gemm_panels) ? q80_panel_copy(c, w) : nullptr;
-    const void * act = quantized_src1(st, b, (q80_skinny || q80_gemm_wp) ? MI_ACT_Q80_PANEL : w->type);
-    if (q80_skinny) {  // 9 .. 32 columns of a -np decode step (round 6)
+    const bool q80_batch = w->type == GGML_TYPE_Q8_0 && !w2 && !add2 && mmq_q80_batch_supported(w->type, K, N, M);
+    const void * act = quantized_src1(st, b, q80_batch ? MI_ACT_Q80_PANEL : w->type);
+    if (q80_batch) {  // a -np decode step, a prompt
         const uint8_t * wp = q80_panel_copy(c, w);
         c->st.decode_copy_launches += wp != nullptr;
-        timed_scope ts(c, "mmq_q8_0_skinny", wbytes);
+        timed_scope ts(c, M <= 32 ? "mmq_q8_0_skinny" : "mmq_q8_0", wbytes);
         const int64_t arows = add ? add->ne[1] * add->ne[2] * add->ne[3] : 0;
-        launch_mmq_q80_skinny(c->stream, (const uint8_t *) w->data, wp, (int64_t) w->nb[1], (int) K, (int) N, (int) M, act, (float *) dst->data, (int64_t) (dst->nb[1] / 4),
+        launch_mmq_q80(c->stream, (const uint8_t *) w->data, wp, (int64_t) w->nb[1], (int) K, (int) N, (int) M, act, (float *) dst->data, (int64_t) (dst->nb[1] / 4),
                               add ? (const float *) add->data : nullptr, (!add || arows == 1) ? 0 : (int64_t) (add->nb[1] / 4));
         c->st.kernel_launches++;
         c->st.skinny_launches++;
-        return true;
-    }
-    if (q80_gemm) {
-        timed_scope ts(c, "mmq_q8_0", wbytes);
-        const int64_t arows = add ? add->ne[1] * add->ne[2] * add->ne[3] : 0;
-        c->st.decode_copy_launches += q80_gemm_wp != nullptr;
-        launch_mmq_q80(c->stream, (const uint8_t *) w->data, q80_gemm_wp, (int64_t) w->nb[1], (int) K, (int) N, (int) M, act, (float *) dst->data, (int64_t) (dst->nb[1] / 4),
-                       add ? (const float *) add->data : nullptr, (!add || arows == 1) ? 0 : (int64_t) (add->nb[1] / 4));
-        c->st.kernel_launches++;
         return true;
     }
     const bool i8 = c->opt.mmq_i8 && mmq_i8_supported(w->type, K, N, M);
@@ -795,7 +782,7 @@ static bool quant_consumers_only(const exec_state & st, int at, const ggml_tenso
     }
     return true;
 }
-// ... and the same question for Q8_0 weights (round 6): every reader of t is a Q8_0 mat-mul that takes the 9 .. 128-column matrix-core kernel (its activations in panel
+// ... and the same question for Q8_0 weights (round 6): every reader of t is a Q8_0 mat-mul that takes a matrix-core kernel (9 columns and up) (its activations in panel
 // order), so a producer may leave Q8_0 panel blocks instead of f32
 static bool q80_panel_consumers_only(const exec_state & st, int at, const ggml_tensor * t) {
     if ((t->flags & GGML_TENSOR_FLAG_OUTPUT) || t->type != GGML_TYPE_F32 || (t->ne[0] % 128) != 0) return false;
@@ -808,7 +795,7 @@ static bool q80_panel_consumers_only(const exec_state & st, int at, const ggml_t
             if (u->src[s] != t) continue;
             const ggml_tensor * wt = u->src[0];
             if (!(u->op == GGML_OP_MUL_MAT && s == 1 && wt->type == GGML_TYPE_Q8_0 && wt->ne[2] == 1 && wt->ne[3] == 1 && rows_contig(wt) && !buffer_is_split(wt->buffer) &&
-                  mmq_q80_skinny_supported(wt->type, wt->ne[0], wt->ne[1], M) && u->type == GGML_TYPE_F32 && ggml_abi_is_contiguous(u)))
+                  mmq_q80_batch_supported(wt->type, wt->ne[0], wt->ne[1], M) && u->type == GGML_TYPE_F32 && ggml_abi_is_contiguous(u)))
                 return false;
             if (tp_active(st.c) && buffer_is_rowpar(wt->view_src ? wt->view_src->buffer : wt->buffer)) return false;
             last = j;
@@ -1389,7 +1376,7 @@ static int try_merge_mm_batch(exec_state & st, int i) {  // returns the number o
     return ms[0].n_nodes;
 }
 
-// Q8_0 weights, 9 .. 128 columns (round 6): wq / wk / wv (and gate / up) of a batch multiply the same activations — one launch of the weight-streaming matrix-core
+// Q8_0 weights, 9 columns and up: wq / wk / wv (and gate / up) of a batch multiply the same activations — one launch of the matrix-core
 // kernel over the concatenated 32-row panels (mmq_q80.hip), bias ADDs folded into the store.  The member search is try_merge_mm_batch's (same dependence rules);
 // no K split, no epilogues: with the K / V projections out of the way the ropes and cache stores that follow fuse as they do for the K-quants (try_fuse_rope_store).
 static int try_merge_q80_skinny(exec_state & st, int i) {  // returns the number of nodes consumed at position i (0: not merged)
@@ -1402,7 +1389,7 @@ static int try_merge_q80_skinny(exec_state & st, int i) {  // returns the number
     auto eligible = [&](const ggml_tensor * t) {
         const ggml_tensor * w = t->src[0];
         return t->op == GGML_OP_MUL_MAT && t->src[1] == X && w->type == GGML_TYPE_Q8_0 && w->ne[0] == K && w->ne[2] == 1 && w->ne[3] == 1 && rows_contig(w) && !buffer_is_split(w->buffer) &&
-               mmq_q80_skinny_supported(w->type, K, w->ne[1], M) && t->type == GGML_TYPE_F32 && ggml_abi_is_contiguous(t) && !(tp_active(c) && buffer_is_rowpar(w->view_src ? w->view_src->buffer : w->buffer));
+               mmq_q80_batch_supported(w->type, K, w->ne[1], M) && t->type == GGML_TYPE_F32 && ggml_abi_is_contiguous(t) && !(tp_active(c) && buffer_is_rowpar(w->view_src ? w->view_src->buffer : w->buffer));
     };
     auto with_add = [&](int k) {  // member at node k, with the ADD that directly follows it folded in
         ggml_tensor * t = g->nodes[k];
@@ -1455,8 +1442,8 @@ static int try_merge_q80_skinny(exec_state & st, int i) {  // returns the number
     for (size_t q = 1; q < ms.size(); ++q)
         for (int d = 0; d < ms[q].n_nodes; ++d) { mark_done(st, ms[q].k + d); c->st.fused_nodes++; }
     {
-        timed_scope ts(c, (std::string("mmq_q8_0_skinny") + (ms.size() == 3 ? "_x3" : "_x2") + "_n" + std::to_string(n_total) + "_k" + std::to_string(K)).c_str(), wbytes, true);
-        launch_mmq_q80_skinny_multi(c->stream, (int) ms.size(), mats, (int) K, (int) M, act);
+        timed_scope ts(c, (std::string(M <= 32 ? "mmq_q8_0_skinny" : "mmq_q8_0") + (ms.size() == 3 ? "_x3" : "_x2") + "_n" + std::to_string(n_total) + "_k" + std::to_string(K)).c_str(), wbytes, true);
+        launch_mmq_q80_multi(c->stream, (int) ms.size(), mats, (int) K, (int) M, act);
     }
     c->st.decode_copy_launches += with_copy != 0;
     c->st.skinny_launches++;
@@ -2758,7 +2745,7 @@ static int run_node(exec_state & st, int i) {
                     return 2;
                 }
             }
-            if (fuse && !rowpar && c->opt.mm_merge && a->type == GGML_TYPE_Q8_0 && mmq_q80_skinny_supported(a->type, a->ne[0], a->ne[1], M)) {
+            if (fuse && !rowpar && c->opt.mm_merge && a->type == GGML_TYPE_Q8_0 && mmq_q80_batch_supported(a->type, a->ne[0], a->ne[1], M)) {
                 const int used = try_merge_q80_skinny(st, i);
                 if (used != 0) return used;
             }
@@ -2767,7 +2754,7 @@ static int run_node(exec_state & st, int i) {
                 if (used != 0) return used;
             }
             if (fuse && !rowpar && ((M >= mmq_min_cols_for(c, a->type) && c->opt.mmq_i8 && mmq_i8_supported(a->type, a->ne[0], a->ne[1], M)) ||
-                                    (M >= c->opt.q80_min_cols && mmq_q80_supported(a->type, a->ne[0], a->ne[1], M)) || mmq_q80_skinny_supported(a->type, a->ne[0], a->ne[1], M))) {
+                                    mmq_q80_batch_supported(a->type, a->ne[0], a->ne[1], M))) {
                 // batches: MUL_MAT -> ADD (bias row or residual) rides in the GEMM's store
                 ggml_tensor * a1 = next(1);
                 const ggml_tensor * o1 = (a1 && single_use(st, n)) ? add_partner(a1, n) : nullptr;

@@ -27,7 +27,7 @@ inline tdesc TD(const ggml_tensor * t) {
 // kind: GGML_TYPE_Q8_K -> q8k_dev[rows][K/256]; GGML_TYPE_Q8_0 -> q80_dev[rows][K/32]
 size_t quantized_act_bytes(int kind, int64_t K, int64_t rows);
 void launch_quantize_act(hipStream_t s, int kind, const tdesc & src, void * dst);
-// Q8_0 activations of up to 32 columns in PANEL order (mmq_q80.hip: k_mmq_q80_skinny): per block of 32 values [K half][column 0 .. 31][16 quants] + [column] f32 scales, 1152 B
+// Q8_0 activations in PANEL order, columns in groups of 32 (mmq_q80.hip): per block of 32 values [K half][column 0 .. 31][16 quants] + [column] f32 scales, 1152 B
 #define MI_ACT_Q80_PANEL 1008
 void launch_quantize_q80_panel(hipStream_t s, const tdesc & src, void * dst);
 // producers fused with that quantisation (ops.hip; same arithmetic as the unfused kernels): RMS_NORM(x) * w, SwiGLU
@@ -229,13 +229,11 @@ int launch_mmq_i8(hipStream_t s, int type, const uint8_t * W, int64_t w_nb1, int
 bool mmq_skinny_supported(int type, int64_t K, int64_t N, int64_t M, int64_t w_nb1);
 int mmq_skinny_ksplit(int64_t K, int64_t n_total);
 // Q8_0 weights x Q8_0 activations, one int8 MFMA per 32-value block + immediate f32 scale-accumulate (mmq_q80.hip)
-bool mmq_q80_supported(int type, int64_t K, int64_t N, int64_t M);
-void launch_mmq_q80(hipStream_t s, const uint8_t * W, const uint8_t * W_panels, int64_t w_nb1, int K, int N, int M, const void * act_q80, float * dst, int64_t dst_stride, const float * add, int64_t add_stride);
-// 9 .. 32 columns: the weights streamed once, 32-row panels, K split over the waves of a workgroup (mmq_q80.hip; round 6)
-bool mmq_q80_skinny_supported(int type, int64_t K, int64_t N, int64_t M);
+// 9 columns and up: up to 32 with the weights streamed once, above in tiles of 32 rows x 64 columns; activations in panel order
+bool mmq_q80_batch_supported(int type, int64_t K, int64_t N, int64_t M);
 struct mmq80s_desc { const uint8_t * W; const uint8_t * W_panels; int64_t w_nb1; int N; float * dst; int64_t dst_stride; const float * add; int64_t add_stride; };
-void launch_mmq_q80_skinny_multi(hipStream_t s, int n, const mmq80s_desc * mats, int K, int M, const void * act_q80_panel);  // up to three matrices over the same activations
-void launch_mmq_q80_skinny(hipStream_t s, const uint8_t * W, const uint8_t * W_panels, int64_t w_nb1, int K, int N, int M, const void * act_q80_panel, float * dst, int64_t dst_stride, const float * add, int64_t add_stride);
+void launch_mmq_q80_multi(hipStream_t s, int n, const mmq80s_desc * mats, int K, int M, const void * act_q80_panel);  // up to three matrices over the same activations
+void launch_mmq_q80(hipStream_t s, const uint8_t * W, const uint8_t * W_panels, int64_t w_nb1, int K, int N, int M, const void * act_q80_panel, float * dst, int64_t dst_stride, const float * add, int64_t add_stride);
 void launch_mmq(hipStream_t s, int type, const uint8_t * W, int64_t w_nb1, int K, int N, int M, const void * act_q8k, float * dst, int64_t dst_stride, int ksplit, float * part);
 
 // ---- element-wise / normalisation / data movement (ops.hip)

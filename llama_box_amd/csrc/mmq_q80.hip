@@ -1,15 +1,19 @@
-// mmq_q80.hip — batched mat-mul for Q8_0 weights on the gfx950 INTEGER matrix cores.
+// mmq_q80.hip — batched mat-mul (9 columns and up) for Q8_0 weights on the gfx950 INTEGER matrix cores.
 //
 // ggml-cpu's ggml_vec_dot_q8_0_q8_0 quantises the activations to Q8_0 as well and sums,
 // per 32-value block, sumi * (d_w * d_x) in f32.  A block is exactly the K extent of v_mfma_i32_32x32x32_i8, so one MFMA
 // with a zero accumulator yields the 32x32 integer block sums, and the f32 scale-accumulate follows at once — there is no
-// super-block to amortise it over, which makes this kernel VALU-bound (4 VALU per output and block against one MFMA per
-// 1024 outputs): the matrix core only replaces the 32 multiply-adds per output and block.  Still an order of magnitude
-// faster than running the batch as 8-column mat-vec passes, which re-stream the weights once per pass.
-// Tile 128 weight rows x 128 columns x 128 K (4 blocks) per trip, 8 waves (32 x 64 each), double-buffered LDS: raw int8 of
-// both operands in the XOR-swizzled [row][128 B] image of mmq_i8.hip plus the 4 block scales of every row / column.
+// super-block to amortise it over, which makes these kernels VALU-bound (3 VALU per output and block: convert, d_w * d_x,
+// fused multiply-add — 192 issue cycles beside the MFMA's 32, 0.84 POP/s for the chip).
+//
+// Both kernels take their operands straight from global memory into the MFMA's registers: the weights from their panel copy
+// (repack.hip: k_repack_q80_panels; or, without one, from the 2-byte-aligned blocks), the activations in panel order
+// (quantize.hip) — a wave-instruction reads 1 KB of consecutive bytes either way, no LDS tile and no barrier per K step.
+// An output is eight partial sums — chunk c of four blocks goes to sum c mod 8 — added in order, whatever the number of
+// columns, the wave that made them and the matrices that share the launch: the same bits in every form.
 #include <algorithm>
 #include <cstdlib>
+#include <type_traits>
 
 #include "dev_util.h"
 #include "kernels.h"
@@ -19,190 +23,15 @@ namespace mi355x {
 typedef float float16q __attribute__((ext_vector_type(16)));
 typedef int int4q __attribute__((ext_vector_type(4)));
 typedef int int16q __attribute__((ext_vector_type(16)));
+typedef float float32q __attribute__((ext_vector_type(32)));
 
-struct mmq80_args {
-    const uint8_t * W;
-    int64_t w_nb1;
-    int K, N, M;
-    const q80_dev * act;  // [M][K/32]
-    float * dst;
-    int64_t dst_stride;
-    int n_panels, m_tiles;
-    const float * add;
-    int64_t add_stride;
-};
-
-constexpr int Q80_T = 128 * 128;                // bytes of one operand tile
-constexpr int Q80_STAGE = 2 * Q80_T + 2 * 128 * 16;  // A | B | dw[128][4] | da[128][4]
-
-__device__ __forceinline__ int sw_offq(const int row, const int chunk) { return row * 128 + ((chunk ^ ((row >> 1) & 7)) << 4); }
-
-// PANEL (round 6): the weights come from their panel copy (repack.hip: k_repack_q80_panels) and the activations in panel order (quantize.hip: k_quantize_q8_0<true>) —
-// a thread's block is two aligned 16-byte loads + its scale instead of eight 2-byte-aligned dwords + the scale, consecutive threads read consecutive bytes
-template <bool PANEL> __global__ void __launch_bounds__(512, 1) k_mmq_q80(const mmq80_args a) {
-    extern __shared__ __attribute__((aligned(16))) char smem[];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int xcd = blockIdx.x & 7, qb = blockIdx.x >> 3;
-    const int panel = (qb / a.m_tiles) * 8 + xcd, mt = qb % a.m_tiles;
-    if (panel >= a.n_panels) return;
-    const int n0 = panel * 128, m0 = mt * 128;
-    const int nb32 = a.K / 32, trips = a.K / 128;
-    const int nslab = wave & 3, mhalf = wave >> 2;
-
-    // staging roles: thread -> (row | column, block of the trip)
-    const int srow = tid >> 2, sq = tid & 3;
-    const uint8_t * wblk = a.W + (size_t) min(n0 + srow, a.N - 1) * a.w_nb1 + (size_t) sq * 34;
-    const q80_dev * yblk = a.act + (size_t) min(m0 + srow, a.M - 1) * nb32 + sq;
-    const int off0 = sw_offq(srow, 2 * sq), off1 = sw_offq(srow, 2 * sq + 1);
-
-    uint32_t ga0, ga1, ga2, ga3, ga4, ga5, ga6, ga7, gb0, gb1, gb2, gb3, gb4, gb5, gb6, gb7;
-    uint16_t gad = 0;
-    float gbd = 0.0f;
-    // PANEL: the (32 rows, 4 blocks) tile of this thread's row for trip t, and the (block, 32 columns) tile of its column
-    const int wrow_c = min(n0 + srow, a.N - 1), ycol_c = min(m0 + srow, a.M - 1);
-    const uint8_t * wtile = a.W + (size_t) (wrow_c >> 5) * (size_t) trips * 4352 + (size_t) sq * 1024 + (size_t) (wrow_c & 31) * 16;
-    const uint8_t * wtile_d = a.W + (size_t) (wrow_c >> 5) * (size_t) trips * 4352 + 4096 + (size_t) sq * 64 + (size_t) (wrow_c & 31) * 2;
-    const char * ytile = (const char *) a.act + ((size_t) (ycol_c >> 5) * (size_t) nb32 + (size_t) sq) * 1152 + (size_t) (ycol_c & 31) * 16;
-    auto issue_loads = [&](const int t) {
-        if constexpr (PANEL) {
-            const uint4 a0 = *(const uint4 *) (wtile + (size_t) t * 4352), a1 = *(const uint4 *) (wtile + (size_t) t * 4352 + 512);
-            ga0 = a0.x; ga1 = a0.y; ga2 = a0.z; ga3 = a0.w; ga4 = a1.x; ga5 = a1.y; ga6 = a1.z; ga7 = a1.w;
-            gad = *(const uint16_t *) (wtile_d + (size_t) t * 4352);
-            const char * yt = ytile + (size_t) t * 4 * 1152;
-            const uint4 b0 = *(const uint4 *) yt, b1 = *(const uint4 *) (yt + 512);
-            gb0 = b0.x; gb1 = b0.y; gb2 = b0.z; gb3 = b0.w; gb4 = b1.x; gb5 = b1.y; gb6 = b1.z; gb7 = b1.w;
-            gbd = *(const float *) (yt + 1024 - (size_t) (ycol_c & 31) * 16 + (size_t) (ycol_c & 31) * 4);
-            return;
-        }
-        const uint8_t * p = wblk + (size_t) t * 4 * 34;  // Q8_0 blocks are 2-byte aligned: dword loads typed accordingly
-        gad = ld16(p);
-        ga0 = ld32_a2(p + 2); ga1 = ld32_a2(p + 6); ga2 = ld32_a2(p + 10); ga3 = ld32_a2(p + 14);
-        ga4 = ld32_a2(p + 18); ga5 = ld32_a2(p + 22); ga6 = ld32_a2(p + 26); ga7 = ld32_a2(p + 30);
-        const q80_dev * y = yblk + (size_t) t * 4;
-        const uint32_t * yq = (const uint32_t *) y->qs;
-        gb0 = yq[0]; gb1 = yq[1]; gb2 = yq[2]; gb3 = yq[3]; gb4 = yq[4]; gb5 = yq[5]; gb6 = yq[6]; gb7 = yq[7];
-        gbd = y->d;
-    };
-    auto stage = [&](const int t) {
-        char * buf = smem + (t & 1) * Q80_STAGE;
-        *(uint4 *) (buf + off0) = make_uint4(ga0, ga1, ga2, ga3);
-        *(uint4 *) (buf + off1) = make_uint4(ga4, ga5, ga6, ga7);
-        *(uint4 *) (buf + Q80_T + off0) = make_uint4(gb0, gb1, gb2, gb3);
-        *(uint4 *) (buf + Q80_T + off1) = make_uint4(gb4, gb5, gb6, gb7);
-        ((float *) (buf + 2 * Q80_T))[sq * 128 + srow] = h2f(gad);              // scales are stored [block][row] so that the four
-        ((float *) (buf + 2 * Q80_T + 128 * 16))[sq * 128 + srow] = gbd;        // consecutive rows of an accumulator quad are one 16-byte read
-    };
-
-    const int fr = lane & 31, kg = lane >> 5;
-    const int swz = (fr >> 1) & 7;
-    const int arow_off = (nslab * 32 + fr) * 128;
-    const int brow_off0 = (mhalf * 64 + fr) * 128, brow_off1 = (mhalf * 64 + 32 + fr) * 128;
-    float16q C0, C1;
-    int16q zi;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) { C0[r] = 0.0f; C1[r] = 0.0f; zi[r] = 0; }
-
-    issue_loads(0);
-    stage(0);
-    if (trips > 1) issue_loads(1);
-    __syncthreads();
-    for (int t = 0; t < trips; ++t) {
-        if (t + 1 < trips) {
-            stage(t + 1);
-            if (t + 2 < trips) issue_loads(t + 2);
-        }
-        const char * buf = smem + (t & 1) * Q80_STAGE;
-        const float * dwt = (const float *) (buf + 2 * Q80_T);
-        const float * dat = (const float *) (buf + 2 * Q80_T + 128 * 16);
-#pragma unroll
-        for (int blk = 0; blk < 4; ++blk) {
-            const int co = ((2 * blk + kg) ^ swz) << 4;
-            const int4q fa = *(const int4q *) (buf + arow_off + co);
-            const int4q fb0 = *(const int4q *) (buf + Q80_T + brow_off0 + co), fb1 = *(const int4q *) (buf + Q80_T + brow_off1 + co);
-            const float y0 = dat[blk * 128 + mhalf * 64 + fr], y1 = dat[blk * 128 + mhalf * 64 + 32 + fr];
-            float x[16];  // block scale of the 16 rows this lane's accumulator registers belong to
-#pragma unroll
-            for (int g4 = 0; g4 < 4; ++g4) {
-                const float4 v = *(const float4 *) (dwt + blk * 128 + nslab * 32 + 8 * g4 + 4 * kg);
-                x[4 * g4] = v.x; x[4 * g4 + 1] = v.y; x[4 * g4 + 2] = v.z; x[4 * g4 + 3] = v.w;
-            }
-            const int16q s0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa, fb0, zi, 0, 0, 0);
-            const int16q s1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa, fb1, zi, 0, 0, 0);
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                C0[r] += (float) s0[r] * (x[r] * y0);  // sumf += sumi * (d_w * d_x), as the CPU does
-                C1[r] += (float) s1[r] * (x[r] * y1);
-            }
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int tt = 0; tt < 2; ++tt) {
-        const int m = m0 + mhalf * 64 + tt * 32 + fr;
-        if (m >= a.M) continue;
-        float * out = a.dst + (size_t) m * a.dst_stride;
-        const float * ad = a.add ? a.add + (size_t) m * a.add_stride : nullptr;
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            const int n = n0 + nslab * 32 + 8 * g + 4 * kg;
-            float c4[4];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) c4[r] = tt ? C1[4 * g + r] : C0[4 * g + r];
-            if (ad) {
-#pragma unroll
-                for (int r = 0; r < 4; ++r) if (n + r < a.N) c4[r] += ad[n + r];
-            }
-            if (n + 3 < a.N && ((((uintptr_t) (out + n)) & 15) == 0)) {
-                *(float4 *) (out + n) = make_float4(c4[0], c4[1], c4[2], c4[3]);
-            } else {
-#pragma unroll
-                for (int r = 0; r < 4; ++r) if (n + r < a.N) out[n + r] = c4[r];
-            }
-        }
-    }
-}
-
-bool mmq_q80_supported(int type, int64_t K, int64_t N, int64_t M) {
-    (void) N;
-    return type == GGML_TYPE_Q8_0 && (K % 128) == 0 && M >= 9;
-}
-
-void launch_mmq_q80(hipStream_t s, const uint8_t * W, const uint8_t * W_panels, int64_t w_nb1, int K, int N, int M, const void * act_q80, float * dst, int64_t dst_stride, const float * add,
-                    int64_t add_stride) {  // W_panels != nullptr: the panel copy, and act_q80 holds the activations in panel order
-    mmq80_args a;
-    a.W = W_panels ? W_panels : W;
-    a.w_nb1 = w_nb1;
-    a.K = K;
-    a.N = N;
-    a.M = M;
-    a.act = (const q80_dev *) act_q80;
-    a.dst = dst;
-    a.dst_stride = dst_stride;
-    a.n_panels = (N + 127) / 128;
-    a.m_tiles = (M + 127) / 128;
-    a.add = add;
-    a.add_stride = add_stride;
-    const size_t lds = 2 * (size_t) Q80_STAGE;
-    static std::atomic<uint32_t> lds_raised{0};  // one bit per device (common.h: ensure_dyn_lds)
-    static std::atomic<uint32_t> lds_raised_p{0};
-    const unsigned grid = (unsigned) (((a.n_panels + 7) / 8) * 8 * a.m_tiles);
-    if (W_panels) {
-        (void) ensure_dyn_lds((const void *) k_mmq_q80<true>, lds, lds_raised_p);  // on failure the launch below fails and graph_compute reports it
-        hipLaunchKernelGGL(k_mmq_q80<true>, dim3(grid), dim3(512), lds, s, a);
-    } else {
-        (void) ensure_dyn_lds((const void *) k_mmq_q80<false>, lds, lds_raised);
-        hipLaunchKernelGGL(k_mmq_q80<false>, dim3(grid), dim3(512), lds, s, a);
-    }
-}
-
-// ------------------------------------------------------------------------------------------------ 9 .. 32 columns (round 6)
-// A -np decode step of a Q8_0 model: until this round every such mat-mul ran as 8-column mat-vec passes (the weights streamed once per pass, the dot products
-// on the vector ALU: 61 us per matrix of Llama-3-8B Q8_0 at 32 columns, a 16 ms step) and the 128 x 128-tile GEMM above has too few workgroups for 32 columns
-// (97 us).  Here the WEIGHTS stream once: a workgroup owns 32 weight rows, its eight waves take the K range in interleaved chunks of four blocks (128 values:
-// one cache line of every row), one v_mfma_i32_32x32x32_i8 per block gives the 32 x 32 integer block sums, and the f32 scale-accumulate follows as in the GEMM
-// (sumf += sumi * (d_w * d_x), ggml_vec_dot_q8_0_q8_0's expression).  Weight bytes go from global memory straight into the MFMA operand registers (a lane = a
-// row and a 16-value half of the block, 2-byte aligned 16-byte loads); the activations' blocks (32 columns x K / 32 x 36 B: L2-resident) likewise; the 32 row
-// scales of a block reach the 16 accumulator rows of a lane through a wave-private LDS line.  The eight partial tiles meet in LDS and are added in wave order.
+// ------------------------------------------------------------------------------------------------ 9 .. 32 columns
+// A -np decode step of a Q8_0 model (as 8-column mat-vec passes the weights streamed once per pass: 61 us per matrix of Llama-3-8B Q8_0 at 32 columns, a 16 ms
+// step).  Here the WEIGHTS stream once: a workgroup owns 32 weight rows, its eight waves take the K range in interleaved chunks of four blocks (128 values:
+// one cache line of every row), one v_mfma_i32_32x32x32_i8 per block gives the 32 x 32 integer block sums, and the f32 scale-accumulate follows
+// (sumf += sumi * (d_w * d_x), ggml_vec_dot_q8_0_q8_0's expression, with the fused multiply-add its SIMD builds use).  Weight bytes go from global memory straight
+// into the MFMA operand registers (a lane = a row and a 16-value half of the block); the activations' blocks (32 columns x K / 32 x 36 B: L2-resident) likewise; the
+// 32 row scales of a block reach the 16 accumulator rows of a lane through a wave-private LDS line.  The eight partial tiles meet in LDS and are added in wave order.
 struct mmq80s_mat {
     const uint8_t * W;   // the tensor (block layout), or its panel copy (repack.hip: k_repack_q80_panels) — template WP
     int64_t w_nb1;
@@ -285,7 +114,7 @@ template <bool WP> __global__ void __launch_bounds__(Q80S_WV * 64, 2) k_mmq_q80_
             }
             const int16q s = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[b], fb[b], zi, 0, 0, 0);
 #pragma unroll
-            for (int r = 0; r < 16; ++r) C[r] += (float) s[r] * (x[r] * dy[b]);  // sumf += sumi * (d_w * d_x), as the CPU does
+            for (int r = 0; r < 16; ++r) C[r] = __builtin_fmaf((float) s[r], x[r] * dy[b], C[r]);
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();  // (the next chunk's scales overwrite the line)
@@ -314,13 +143,126 @@ template <bool WP> __global__ void __launch_bounds__(Q80S_WV * 64, 2) k_mmq_q80_
     }
 }
 
-bool mmq_q80_skinny_supported(int type, int64_t K, int64_t N, int64_t M) {
+// ------------------------------------------------------------------------------------------------ 33 columns and up
+// A prompt's micro-batch, drafts of several sequences.  A workgroup owns 32 weight rows x 64 columns, its four waves take the K range in interleaved chunks of four
+// blocks and make one partial sum each, added in wave order: an output has the same bits whatever matrices and columns share the launch.  Per two blocks and 32
+// columns: two v_mfma_i32_32x32x32_i8 for the integer block sums, and ONE v_mfma_f32_32x32x1 (two outer products) for the factors d_w * d_x of all 2 x 1024 outputs —
+// the multiplication that would be a third VALU instruction per output and block, and the row scales need no way through LDS to the accumulator's rows.  Two VALU
+// are left (convert, fused multiply-add): 128 issue cycles per block beside the matrix core's 64, 1.26 POP/s for the chip.  The next step of two blocks is in flight
+// while one is multiplied, three waves per SIMD (160 registers; three steps in flight at two waves per SIMD: 55 us below).  Workgroups that read the same weights
+// (the column tiles of a panel) follow one another on one XCD, so the weights cross HBM once.
+// TinyLlama, 512 columns: wq + wk + wv / gate + up / a whole 700-token prompt.  128 x 128 LDS tiles, one launch per matrix: 3 x 45 us / 2 x 45 us / 17.2 ms; this kernel
+// with the factors on the VALU: 40 / 66 us / 9.1 ms; as it is: 15 / 44 us / 6.3 ms (23.6 GFLOP in 44 us: 0.53 POP/s).
+constexpr int Q80C_WV = 4;
+template <bool WP> __global__ void __launch_bounds__(Q80C_WV * 64, 3) k_mmq_q80_cols(const mmq80s_args a, const int n_panels, const int m_tiles) {
+    __shared__ float red[Q80C_WV][16][65];                         // the waves' partial tiles, one 32-column half at a time
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int fr = lane & 31, kg = lane >> 5;
+    const int xcd = blockIdx.x & 7, qb = blockIdx.x >> 3;
+    const int gp = (qb / m_tiles) * 8 + xcd, m0 = (qb % m_tiles) * 64;  // the panel, counted over all matrices
+    if (gp >= n_panels) return;
+    const int mi = gp < a.m[0].panel_end ? 0 : (gp < a.m[1].panel_end ? 1 : 2);
+    const mmq80s_mat & mt = a.m[mi];
+    const int panel = gp - (mi ? a.m[mi - 1].panel_end : 0);
+    const int n0 = panel * 32;
+    const int nchunk = a.K / 128;
+    const bool two = m0 + 32 < a.M;                                // (uniform) the second half of the tile has columns
+    // uniform bases + a lane's offset (columns are clamped inside the tile's own groups of 32: group m0 / 32, and the next one when it has columns)
+    const uint8_t * wbase = WP ? mt.W + (size_t) panel * nchunk * 4352 : mt.W;
+    const size_t wlane = WP ? 0 : (size_t) min(n0 + fr, mt.N - 1) * mt.w_nb1;
+    const size_t ygroup = (size_t) (a.K / 32) * 1152;
+    const char * y0 = a.act + (size_t) (m0 >> 5) * ygroup, * y1 = two ? y0 + ygroup : y0;
+    const int f0 = min(fr, a.M - 1 - m0), f1 = two ? min(fr, a.M - 1 - m0 - 32) : f0;
+
+    int16q zi;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) zi[r] = 0;
+    float32q zp;
+#pragma unroll
+    for (int r = 0; r < 32; ++r) zp[r] = 0.0f;
+    // the operands of two blocks (scales: lanes 0 .. 31 the first block's, lanes 32 .. 63 the second's); two sets: one multiplied, one in flight
+    struct opset { int4q A[2], B0[2], B1[2]; uint32_t dW; float dY0, dY1; };
+    auto load2 = [&](const int c, const int half, opset & o) {
+        const size_t yo = (size_t) (c * 4 + 2 * half) * 1152;
+        if constexpr (WP) o.dW = *(const uint16_t *) (wbase + (size_t) c * 4352 + 4096 + half * 128 + lane * 2);
+        else o.dW = ld16(wbase + wlane + (size_t) (c * 4 + 2 * half + kg) * 34);
+        o.dY0 = *(const float *) (y0 + yo + (kg * 1152 + 1024 + f0 * 4));
+        o.dY1 = *(const float *) (y1 + yo + (kg * 1152 + 1024 + f1 * 4));
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int b = 2 * half + u;
+            if constexpr (WP) o.A[u] = *(const int4q *) (wbase + (size_t) c * 4352 + b * 1024 + lane * 16);  // [K half][row][16]
+            else o.A[u] = __builtin_bit_cast(int4q, *(const q80s_u32x4_a2 *) (wbase + wlane + (size_t) (c * 4 + b) * 34 + 2 + 16 * kg));
+            o.B0[u] = *(const int4q *) (y0 + yo + u * 1152 + (kg * 512 + f0 * 16));
+            o.B1[u] = *(const int4q *) (y1 + yo + u * 1152 + (kg * 512 + f1 * 16));
+        }
+    };
+    float C0[16], C1[16];
+    auto mul2 = [&](const opset & o, const auto both) {
+        const float dw = h2f((uint16_t) o.dW);
+        auto tile = [&](const int4q * B, const float dy, float (&C)[16]) {
+            // d_w * d_x of two blocks' 32 x 32 outputs in one matrix instruction (two outer products; a product of two 11-bit significands is exact)
+            const float32q p = __builtin_amdgcn_mfma_f32_32x32x1f32(dw, dy, zp, 0, 0, 0);
+            const int16q s0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(o.A[0], B[0], zi, 0, 0, 0);
+            const int16q s1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(o.A[1], B[1], zi, 0, 0, 0);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) C[r] = __builtin_fmaf((float) s0[r], p[r], C[r]);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) C[r] = __builtin_fmaf((float) s1[r], p[16 + r], C[r]);
+        };
+        tile(o.B0, o.dY0, C0);
+        if constexpr (decltype(both)::value) tile(o.B1, o.dY1, C1);
+    };
+    auto sums = [&](const auto both) {
+        if (wave >= nchunk) return;
+        const int steps = 2 * ((nchunk - wave + 3) / 4);           // step h: half h & 1 of chunk wave + 4 (h >> 1)
+        auto fetch = [&](const int h, opset & o) {                 // (past the last step: the last one's again, read and not used)
+            const int hc = min(h, steps - 1);
+            load2(wave + 4 * (hc >> 1), hc & 1, o);
+            __builtin_amdgcn_sched_barrier(0);                     // (the scheduler would move the loads down to their uses)
+        };
+        opset o0, o1;
+        fetch(0, o0);
+        for (int h = 0; h < steps; h += 2) {                       // (an even number of steps)
+            fetch(h + 1, o1);
+            mul2(o0, both);
+            fetch(h + 2, o0);
+            mul2(o1, both);
+        }
+    };
+#pragma unroll
+    for (int r = 0; r < 16; ++r) { C0[r] = 0.0f; C1[r] = 0.0f; }
+    if (two) sums(std::true_type{});
+    else sums(std::false_type{});
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        if (h == 1 && !two) break;
+        if (h == 1) __syncthreads();
+#pragma unroll
+        for (int r = 0; r < 16; ++r) red[wave][r][lane] = h ? C1[r] : C0[r];
+        __syncthreads();
+        // the sums of a column's 32 rows go to consecutive threads: whole 128-byte lines
+        for (int e = tid; e < 32 * 32; e += Q80C_WV * 64) {
+            const int row = e & 31, col = e >> 5;
+            const int r = (row & 3) + 4 * (row >> 3), l = col + 32 * ((row >> 2) & 1);
+            float v = red[0][r][l];
+#pragma unroll
+            for (int w = 1; w < Q80C_WV; ++w) v += red[w][r][l];
+            const int m = m0 + 32 * h + col, n = n0 + row;
+            if (m < a.M && n < mt.N) {
+                if (mt.add) v += mt.add[(size_t) m * mt.add_stride + n];
+                mt.dst[(size_t) m * mt.dst_stride + n] = v;
+            }
+        }
+    }
+}
+
+bool mmq_q80_batch_supported(int type, int64_t K, int64_t N, int64_t M) {
     static const bool on = !getenv("GGML_MI355X_Q80_SKINNY") || atoi(getenv("GGML_MI355X_Q80_SKINNY")) != 0;
-    static const int max_cols = getenv("GGML_MI355X_Q80_SKINNY_MAX") ? atoi(getenv("GGML_MI355X_Q80_SKINNY_MAX")) : 128;  // (up to 128 columns: four passes of 32 still beat the 128 x 128-tile GEMM's few workgroups — Llama-3-8B Q8_0, 128-token micro-batches: 8.5 k against 5.1 k tok/s)
-    return on && type == GGML_TYPE_Q8_0 && (K % 128) == 0 && N >= 1 && M >= 9 && M <= std::min(max_cols, 128);
+    return on && type == GGML_TYPE_Q8_0 && (K % 128) == 0 && N >= 1 && M >= 9;
 }
 // n matrices (1 .. 3) over the same activations; panels[q] != nullptr for ALL of them or for none (the template form is per launch)
-void launch_mmq_q80_skinny_multi(hipStream_t s, int n, const mmq80s_desc * mats, int K, int M, const void * act_q80) {
+void launch_mmq_q80_multi(hipStream_t s, int n, const mmq80s_desc * mats, int K, int M, const void * act_q80) {
     mmq80s_args a;
     int pe = 0;
     const bool wp = mats[0].W_panels != nullptr;
@@ -330,22 +272,22 @@ void launch_mmq_q80_skinny_multi(hipStream_t s, int n, const mmq80s_desc * mats,
         a.m[q] = {wp ? d.W_panels : d.W, d.w_nb1, d.N, pe, d.dst, d.dst_stride, d.add, d.add_stride};
     }
     a.K = K;
-    for (int m0 = 0; m0 < M; m0 += 32) {  // groups of 32 columns: the activations' panel tiles of group g follow those of group g - 1 (quantize.hip)
-        a.M = std::min(32, M - m0);
-        a.act = (const char *) act_q80 + (size_t) (m0 / 32) * (size_t) (K / 32) * 1152;
-        for (int q = 0; q < 3; ++q) {
-            const mmq80s_desc & d = mats[q < n ? q : n - 1];
-            a.m[q].dst = d.dst + (size_t) m0 * d.dst_stride;
-            a.m[q].add = d.add ? d.add + (size_t) m0 * d.add_stride : nullptr;
-        }
+    a.M = M;
+    a.act = (const char *) act_q80;
+    if (M <= 32) {
         if (wp) hipLaunchKernelGGL(k_mmq_q80_skinny<true>, dim3((unsigned) pe), dim3(Q80S_WV * 64), 0, s, a);
         else hipLaunchKernelGGL(k_mmq_q80_skinny<false>, dim3((unsigned) pe), dim3(Q80S_WV * 64), 0, s, a);
+        return;
     }
+    const int m_tiles = (M + 63) / 64;
+    const dim3 grid((unsigned) ((pe + 7) / 8 * 8 * m_tiles)), block(Q80C_WV * 64);
+    if (wp) hipLaunchKernelGGL(k_mmq_q80_cols<true>, grid, block, 0, s, a, pe, m_tiles);
+    else hipLaunchKernelGGL(k_mmq_q80_cols<false>, grid, block, 0, s, a, pe, m_tiles);
 }
-void launch_mmq_q80_skinny(hipStream_t s, const uint8_t * W, const uint8_t * W_panels, int64_t w_nb1, int K, int N, int M, const void * act_q80, float * dst, int64_t dst_stride, const float * add,
+void launch_mmq_q80(hipStream_t s, const uint8_t * W, const uint8_t * W_panels, int64_t w_nb1, int K, int N, int M, const void * act_q80, float * dst, int64_t dst_stride, const float * add,
                            int64_t add_stride) {
     const mmq80s_desc d{W, W_panels, w_nb1, N, dst, dst_stride, add, add_stride};
-    launch_mmq_q80_skinny_multi(s, 1, &d, K, M, act_q80);
+    launch_mmq_q80_multi(s, 1, &d, K, M, act_q80);
 }
 
 MI_TU_TOUCH(mmq_q80)
