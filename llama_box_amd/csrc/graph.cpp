@@ -325,6 +325,8 @@ struct ws_plan {
     size_t aux_bytes = 0;  // region B: attention partials
 };
 
+static bool mm_tile_applies(const ggml_tensor * n);
+static bool mm_id_tile_applies(const ggml_tensor * n);
 static size_t fa_image_offset(const tdesc & q, const tdesc & k, const tdesc & v) { return (fattn_workspace_bytes(q, k, v, 64, GGML_TYPE_F16) + 255) & ~(size_t) 255; }
 static ws_plan plan_ws(backend_ctx * c, const ggml_cgraph * g) {
     ws_plan p;
@@ -350,6 +352,8 @@ static ws_plan plan_ws(backend_ctx * c, const ggml_cgraph * g) {
         } else if (n->op == GGML_OP_MUL_MAT && mm_cache_image_ok(n) && !buffer_is_split(n->src[0]->buffer)) {
             const tdesc a16 = kv_image_desc(TD(n->src[0]), nullptr);
             p.aux_bytes = std::max(p.aux_bytes, ((mul_mat_f_workspace_bytes(a16, TD(n->src[1])) + 255) & ~(size_t) 255) + kv_image_bytes(a16));
+        } else if (n->op == GGML_OP_MUL_MAT && mm_tile_applies(n)) {
+            p.act_bytes = std::max(p.act_bytes, (size_t) (n->src[1]->ne[0] * n->src[1]->ne[1]) * 2);
         } else if (n->op == GGML_OP_MUL_MAT && n->src[0]->type == GGML_TYPE_F16) {
             p.aux_bytes = std::max(p.aux_bytes, mul_mat_f_workspace_bytes(TD(n->src[0]), TD(n->src[1])));
             if (c->opt.attn_nf) p.aux_bytes = std::max(p.aux_bytes, attn_nf_list_scratch_bytes(TD(n->src[1]), TD(n->src[0]), nullptr));
@@ -358,6 +362,7 @@ static ws_plan plan_ws(backend_ctx * c, const ggml_cgraph * g) {
                 p.aux_bytes = std::max(p.aux_bytes, attn_nf_mma_ws_bytes(TD(n->src[1]), fattn_mma_pick_splits(TD(n->src[1]), TD(n->src[0]))));
         } else if (n->op == GGML_OP_MUL_MAT_ID && n->src[2]) {
             p.aux_bytes = std::max(p.aux_bytes, mul_mat_id_workspace_bytes(TD(n->src[0]), TD(n->src[2])));
+            if (mm_id_tile_applies(n)) p.act_bytes = std::max(p.act_bytes, (size_t) ggml_abi_nelements(n->src[1]) * 2);
         } else if (n->op == GGML_OP_GATED_LINEAR_ATTN && n->op_params[3] == MI_SEQ_OP_TAG && (n->op_params[0] == SEQ_DELTA_CH || n->op_params[0] == SEQ_LINEAR) && n->src[0] && n->src[3]) {
             p.aux_bytes = std::max(p.aux_bytes, seq_recurrence_scratch_bytes(n->op_params[0], n->op_params[1], (int) (n->src[0]->ne[0] / std::max(1, n->op_params[2])), n->src[3]->ne[1]));
         } else if (n->op == GGML_OP_FLASH_ATTN_EXT && fa_route(n) == 4) {
@@ -550,6 +555,38 @@ static const void * quantized_src1(exec_state & st, const ggml_tensor * b, int w
         timed_scope ts(c, "quantize_act", (double) ggml_abi_nbytes(b));
         if (kind == MI_ACT_Q80_PANEL) launch_quantize_q80_panel(c->stream, TD(b), dst);
         else launch_quantize_act(c->stream, kind, TD(b), dst);
+        c->st.kernel_launches++;
+    }
+    c->q8_src = b->data;
+    c->q8_kind = kind;
+    c->q8_bytes = ggml_abi_nbytes(b);
+    return dst;
+}
+
+// MUL_MAT of a batch of columns by a 16-bit weight matrix on the LDS-tiled kernels (mmf_tile.hip): src1 goes through a copy in the matrix's type.  Up to 16 columns the
+// kernel that splits K over the waves of a 16-row tile is faster (4096 x 4096: 17.5 us for 16 columns, 28.6 for 32; tiles: 23 and 22.6), whatever shares the launch
+static constexpr int64_t MM_TILE_MIN_COLS = 17;
+static bool mm_tile_applies(const ggml_tensor * n) {
+    const ggml_tensor * a = n->src[0], * b = n->src[1];
+    return (a->type == GGML_TYPE_F16 || a->type == GGML_TYPE_BF16) && n->type == GGML_TYPE_F32 && b->type == GGML_TYPE_F32 && b->ne[1] >= MM_TILE_MIN_COLS && a->ne[2] * a->ne[3] * b->ne[2] * b->ne[3] == 1 &&
+           !buffer_is_split(a->buffer) && b->nb[0] == 4 && (b->nb[1] % 16) == 0 && (((uintptr_t) b->data) & 15) == 0 && n->nb[0] == 4 &&
+           mul_mat_tile_ok(a->type, a->ne[0], a->ne[1], (int64_t) a->nb[0], (int64_t) a->nb[1], a->data);
+}
+// ... and MUL_MAT_ID of as many (expert, token) columns as its batched form takes (src1's rows of all tokens dense)
+static bool mm_id_tile_applies(const ggml_tensor * n) {
+    const ggml_tensor * a = n->src[0], * b = n->src[1], * ids = n->src[2];
+    return mul_mat_id_batched(TD(a), TD(b), TD(ids)) && ggml_abi_is_contiguous(b) && b->ne[3] == 1 && n->nb[0] == 4 && (size_t) ggml_abi_nelements(b) * 2 < ((size_t) 1 << 32) &&
+           mul_mat_tile_ok(a->type, a->ne[0], a->ne[1], (int64_t) a->nb[0], (int64_t) a->nb[1], a->data);
+}
+// src1 rounded to the 16-bit type of src0, unless the scratch already holds exactly that (projections of one input)
+static const void * rounded_src1(exec_state & st, const ggml_tensor * b, int wtype) {
+    backend_ctx * c = st.c;
+    const int kind = MI_ACT_16 + wtype;
+    void * dst = (char *) c->ws + st.act_off;
+    if (c->q8_src == b->data && c->q8_kind == kind && c->q8_bytes == ggml_abi_nbytes(b)) return dst;
+    {
+        timed_scope ts(c, "round_act", (double) ggml_abi_nbytes(b));
+        launch_to_16(c->stream, wtype, (const char *) b->data, (int64_t) b->nb[1], b->ne[0], b->ne[1] * b->ne[2], dst);
         c->st.kernel_launches++;
     }
     c->q8_src = b->data;
@@ -777,7 +814,7 @@ static bool quant_consumers_only(const exec_state & st, int at, const ggml_tenso
     if (n_cons == 0 || n_cons != use_count(st, t)) return false;
     for (int j = at + 1; j <= last; ++j) {
         const ggml_tensor * u = g->nodes[j];
-        if (u->op == GGML_OP_MUL_MAT && is_quant(u->src[0]->type) && u->src[1] != t) return false;
+        if (u->op == GGML_OP_MUL_MAT && (is_quant(u->src[0]->type) || mm_tile_applies(u)) && u->src[1] != t) return false;
         if (u->op == GGML_OP_MUL_MAT_ID) return false;
     }
     return true;
@@ -805,7 +842,7 @@ static bool q80_panel_consumers_only(const exec_state & st, int at, const ggml_t
     if (n_cons == 0 || n_cons != use_count(st, t)) return false;
     for (int j = at + 1; j <= last; ++j) {  // (the activation area is shared: no other quantised mat-mul may run before the last reader)
         const ggml_tensor * u = g->nodes[j];
-        if (u->op == GGML_OP_MUL_MAT && is_quant(u->src[0]->type) && u->src[1] != t) return false;
+        if (u->op == GGML_OP_MUL_MAT && (is_quant(u->src[0]->type) || mm_tile_applies(u)) && u->src[1] != t) return false;
         if (u->op == GGML_OP_MUL_MAT_ID) return false;
     }
     return true;
@@ -1776,20 +1813,23 @@ static bool try_fuse_attn_nf_mma(exec_state & st, int i) {
     return true;
 }
 
-// A decode step's bf16 projections of the same activations (q, k, v and the gate of a layer): the siblings that follow node i are executed EARLY, at node i,
+// Projections of the same activations by bf16 matrices (q, k, v and the gate of a layer): the siblings that follow node i are executed EARLY, at node i,
 // as one launch — legal when nothing between node i and a sibling's own position reads or occupies the memory the sibling's result goes to (the graph
 // allocator may have given it a block that an earlier tensor still owns at node i's time).  Returns true when node i and at least one sibling were served.
-static bool try_merge_matvec_bf16(exec_state & st, int i) {
+// One column, 2 .. 16 and more each have their kernel; all of them give a matrix the bits it gets alone.
+static bool try_merge_mm_16(exec_state & st, int i) {
     backend_ctx * c = st.c;
     ggml_cgraph * g = st.g;
     const ggml_tensor * n0 = g->nodes[i];
     const ggml_tensor * X = n0->src[1];
-    const int64_t K = n0->src[0]->ne[0];
-    if (!is_f32_contig(X) || ggml_abi_nelements(X) != K || (K % 8) != 0 || K < 256 || (((uintptr_t) X->data) & 15)) return false;
+    const int64_t K = n0->src[0]->ne[0], M = X->ne[1];
+    if (!is_f32_contig(X) || ggml_abi_nelements(X) != K * M || (K % 8) != 0 || K < 256 || (((uintptr_t) X->data) & 15)) return false;
+    const bool tile = M >= MM_TILE_MIN_COLS;
     auto eligible = [&](const ggml_tensor * t) {
         const ggml_tensor * w = t->src[0];
-        return t->op == GGML_OP_MUL_MAT && t->src[1] == X && w->type == GGML_TYPE_BF16 && w->ne[0] == K && w->ne[2] == 1 && w->ne[3] == 1 && w->nb[0] == 2 && (w->nb[1] % 16) == 0 &&
-               !(((uintptr_t) w->data) & 15) && !buffer_is_split(w->buffer) && is_f32_contig(t) && !mm_cache_image_ok(t);
+        return t->op == GGML_OP_MUL_MAT && t->src[1] == X && (w->type == GGML_TYPE_BF16 || (tile && w->type == GGML_TYPE_F16)) && w->type == n0->src[0]->type && w->ne[0] == K && w->ne[2] == 1 &&
+               w->ne[3] == 1 && w->nb[0] == 2 && (w->nb[1] % 16) == 0 && !(((uintptr_t) w->data) & 15) && !buffer_is_split(w->buffer) && is_f32_contig(t) && !mm_cache_image_ok(t) &&
+               (tile ? mm_tile_applies(t) : mul_mat_bf16_multi_ok(w->ne[1], K, M));
     };
     if (!eligible(n0)) return false;
     std::vector<int> ms{i};
@@ -1810,6 +1850,21 @@ static bool try_merge_matvec_bf16(exec_state & st, int i) {
         if (ok) ms.push_back(k);
     }
     if (ms.size() < 2) return false;
+    if (tile) {
+        const void * x16 = rounded_src1(st, X, n0->src[0]->type);
+        mul_mat_tile_desc m[4];
+        double bytes = 0;
+        for (size_t q = 0; q < ms.size(); ++q) {
+            const ggml_tensor * t = g->nodes[ms[q]], * w = t->src[0];
+            m[q] = {w->data, (int64_t) w->nb[1], w->ne[1], t->data, (int64_t) t->nb[1]};
+            bytes += (double) ggml_abi_nbytes(w);
+        }
+        timed_scope ts(c, "mul_mat_f_siblings", bytes);
+        launch_mul_mat_tile(c->stream, n0->src[0]->type, m, (int) ms.size(), K, M, x16);
+        c->st.kernel_launches++;
+        for (size_t q = 1; q < ms.size(); ++q) { mark_done(st, ms[q]); c->st.fused_nodes++; }
+        return true;
+    }
     matvec_multi mm{};
     mm.n = (int) ms.size();
     double bytes = 0;
@@ -1822,7 +1877,8 @@ static bool try_merge_matvec_bf16(exec_state & st, int i) {
         bytes += (double) ggml_abi_nbytes(t->src[0]);
     }
     timed_scope ts(c, "mul_mat_f_siblings", bytes);
-    launch_matvec_bf16_multi(c->stream, mm, (const float *) X->data, K);
+    if (M == 1) launch_matvec_bf16_multi(c->stream, mm, (const float *) X->data, K);
+    else launch_mul_mat_bf16_multi(c->stream, mm, (const char *) X->data, (int64_t) X->nb[1], K, M);
     c->st.kernel_launches++;
     for (size_t q = 1; q < ms.size(); ++q) { mark_done(st, ms[q]); c->st.fused_nodes++; }
     return true;
@@ -2674,7 +2730,15 @@ static int run_node(exec_state & st, int i) {
             }
             if (!is_quant(a->type) && fuse && c->opt.attn_nf && try_fuse_attn_nf(st, i)) return 1;
             if (!is_quant(a->type) && fuse && c->opt.attn_nf && try_fuse_attn_nf_mma(st, i)) return 1;
-            if (a->type == GGML_TYPE_BF16 && fuse && try_merge_matvec_bf16(st, i)) return 1;
+            if ((a->type == GGML_TYPE_BF16 || a->type == GGML_TYPE_F16) && fuse && try_merge_mm_16(st, i)) return 1;
+            if (mm_tile_applies(n)) {
+                const void * x16 = rounded_src1(st, b, a->type);
+                const mul_mat_tile_desc m{a->data, (int64_t) a->nb[1], a->ne[1], n->data, (int64_t) n->nb[1]};
+                timed_scope ts(c, "mul_mat_f", (double) ggml_abi_nbytes(a));
+                launch_mul_mat_tile(s, a->type, &m, 1, a->ne[0], b->ne[1], x16);
+                c->st.kernel_launches++;
+                return 1;
+            }
             if (!is_quant(a->type)) {
                 timed_scope ts(c, "mul_mat_f", (double) ggml_abi_nbytes(a));
                 launch_mul_mat_f(s, TD(a), TD(b), TD(n), (float *) ((char *) c->ws + st.aux_off), c->ws ? c->ws_size - st.aux_off : 0);
@@ -3090,7 +3154,8 @@ static int run_node(exec_state & st, int i) {
             const size_t need = mul_mat_id_workspace_bytes(TD(a), TD(ids));
             void * ws = (c->ws && st.aux_off + need <= c->ws_size) ? (char *) c->ws + st.aux_off : nullptr;
             timed_scope ts(c, "mul_mat_id", (double) ggml_abi_nbytes(a) / (double) std::max<int64_t>(1, a->ne[2]) * (double) std::min<int64_t>(a->ne[2], ggml_abi_nelements(ids)));
-            const bool grouped = launch_mul_mat_id(s, TD(a), TD(b), TD(ids), TD(n), ws, ws ? c->ws_size - st.aux_off : 0, valid && ws);
+            const void * x16 = (ws && mm_id_tile_applies(n)) ? rounded_src1(st, b, a->type) : nullptr;
+            const bool grouped = launch_mul_mat_id(s, TD(a), TD(b), TD(ids), TD(n), ws, ws ? c->ws_size - st.aux_off : 0, valid && ws, x16);
             st.moe_ids = grouped ? ids : nullptr;  // (only a launch that made or used the lists vouches for them: the per-column forms leave the scratch alone)
             st.moe_node = grouped ? i : -1;
             c->st.kernel_launches++;

@@ -29,6 +29,7 @@ size_t quantized_act_bytes(int kind, int64_t K, int64_t rows);
 void launch_quantize_act(hipStream_t s, int kind, const tdesc & src, void * dst);
 // Q8_0 activations in PANEL order, columns in groups of 32 (mmq_q80.hip): per block of 32 values [K half][column 0 .. 31][16 quants] + [column] f32 scales, 1152 B
 #define MI_ACT_Q80_PANEL 1008
+#define MI_ACT_16 2000  // + the 16-bit type: f32 rows rounded to it (mmf_tile.hip)
 void launch_quantize_q80_panel(hipStream_t s, const tdesc & src, void * dst);
 // producers fused with that quantisation (ops.hip; same arithmetic as the unfused kernels): RMS_NORM(x) * w, SwiGLU
 bool rms_norm_q80_panel_ok(const tdesc & src, const float * w);
@@ -162,12 +163,22 @@ void launch_qkv(hipStream_t s, const qkv_args & a, int type_a, int type_b);
 void launch_mul_mat_f(hipStream_t s, const tdesc & src0, const tdesc & src1, const tdesc & dst, float * ws = nullptr, size_t ws_bytes = 0);  // ws: scratch for K-split partial tiles
 size_t mul_mat_f_workspace_bytes(const tdesc & src0, const tdesc & src1);
 // up to four bf16 matrices (rows of K values, 16-byte aligned) against ONE f32 column of K values (K a multiple of 8), one launch
+// a batch of M columns by up to four f16 / bf16 matrices of K columns, LDS-tiled (mmf_tile.hip); x16: the columns in the matrices' type, dense rows (launch_to_16; x rows 16-byte aligned)
+struct mul_mat_tile_desc { const void * W; int64_t nb1; int64_t N; void * dst; int64_t dst_nb1; };
+bool mul_mat_tile_ok(int type, int64_t K, int64_t N, int64_t nb0, int64_t nb1, const void * W);
+void launch_to_16(hipStream_t s, int type, const char * x, int64_t nb1, int64_t K, int64_t rows, void * out);
+// the experts' columns (lists: k_moe_group); x16 rows: src1's [n_b, T]
+void launch_mul_mat_id_tile(hipStream_t s, const tdesc & as, int64_t n_b, int64_t n_used, int64_t T, const tdesc & d, const int32_t * cnt, const int32_t * off, const int32_t * list, const void * x16);
+bool mul_mat_id_batched(const tdesc & as, const tdesc & b, const tdesc & ids);  // does launch_mul_mat_id group the columns by expert?
+void launch_mul_mat_tile(hipStream_t s, int type, const mul_mat_tile_desc * m, int n, int64_t K, int64_t M, const void * x16);
 struct matvec_multi { const char * W[4]; int64_t nb1[4]; int64_t N[4]; float * dst[4]; int blk0[5]; int n; };
 void launch_matvec_bf16_multi(hipStream_t s, matvec_multi mm, const float * x, int64_t K);
+bool mul_mat_bf16_multi_ok(int64_t N, int64_t K, int64_t M);  // one column, or the columns launch_mul_mat_f gives the kernel whose sums the launch below repeats
+void launch_mul_mat_bf16_multi(hipStream_t s, matvec_multi mm, const char * x, int64_t x_nb1, int64_t K, int64_t M);  // ... 2 .. 16 columns
 // MUL_MAT_ID: as [K, N, n_expert] (f32 / f16 / bf16), b [K, 1 or n_used, T] f32, ids [n_used, T] i32 -> d [N, n_used, T].  ws: scratch for the
 // per-expert column lists of the batched form; lists_valid: an earlier call left the lists of these same ids there
 size_t mul_mat_id_workspace_bytes(const tdesc & as, const tdesc & ids);
-bool launch_mul_mat_id(hipStream_t s, const tdesc & as, const tdesc & b, const tdesc & ids, const tdesc & d, void * ws, size_t ws_bytes, bool lists_valid);  // true: the batched form ran and left the lists in ws
+bool launch_mul_mat_id(hipStream_t s, const tdesc & as, const tdesc & b, const tdesc & ids, const tdesc & d, void * ws, size_t ws_bytes, bool lists_valid, const void * x16 = nullptr);  // x16: src1 in the experts' 16-bit type (mmf_tile.hip); true: the batched form ran and left the lists in ws
 // MUL_MAT of ONE column / MUL_MAT_ID of few columns by a bf16 matrix whose operand is silu(g f) (u f) of rows gu [2 K, n_used, T] (f: one factor per row, or null)
 bool matvec_glu_ok(const tdesc & a, const void * gu, const tdesc * ids);
 void launch_matvec_glu(hipStream_t s, const tdesc & a, const float * gu, const float * f, const tdesc * ids, const tdesc & d);
@@ -485,6 +496,7 @@ void tu_touch_quantize(hipStream_t s);
 void tu_touch_mmvq(hipStream_t s);
 void tu_touch_qkv(hipStream_t s);
 void tu_touch_mmf(hipStream_t s);
+void tu_touch_mmf_tile(hipStream_t s);
 void tu_touch_attn_nf(hipStream_t s);
 void tu_touch_mmq(hipStream_t s);
 void tu_touch_mmq_i8(hipStream_t s);
@@ -506,6 +518,7 @@ inline void preload_kernel_files(hipStream_t s) {
     tu_touch_mmvq(s);
     tu_touch_qkv(s);
     tu_touch_mmf(s);
+    tu_touch_mmf_tile(s);
     tu_touch_attn_nf(s);
     tu_touch_mmq(s);
     tu_touch_mmq_i8(s);

@@ -238,17 +238,8 @@ template <int GH> static void launch_xres_t(hipStream_t s, const tdesc & a, cons
 // over thousands of cells — 128 waves of the kernel above, each walking all of K, took 170 us), and for 2..15 columns: 16 x 16 tiles
 // on v_mfma_f32_16x16x32_f16 (A: src1 column m = lane & 15, B: src0 row n = lane & 15, k-group lane >> 4), the NWK waves of a
 // workgroup take the K steps of ONE tile in turn and add up through LDS in wave order (deterministic).
-template <int NWK, bool BF>
-__global__ void __launch_bounds__(64 * NWK) k_mul_mat_f16_mma16(const tdesc a, const tdesc b, const tdesc d) {
-    __shared__ mmf_float4 red[NWK][64];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int r16 = lane & 15, kg = lane >> 4;
-    const int64_t row0 = (int64_t) blockIdx.x * 16, col0 = (int64_t) blockIdx.y * 16;
-    const int64_t i12 = blockIdx.z % b.ne[2], i13 = blockIdx.z / b.ne[2];
-    const int64_t i02 = i12 / (b.ne[2] / a.ne[2]), i03 = i13 / (b.ne[3] / a.ne[3]);
-    const int64_t K = a.ne[0];
-    const char * wrow = a.data + std::min<int64_t>(row0 + r16, a.ne[1] - 1) * a.nb[1] + i02 * a.nb[2] + i03 * a.nb[3] + kg * 16;
-    const char * xcol = b.data + std::min<int64_t>(col0 + r16, b.ne[1] - 1) * b.nb[1] + i12 * b.nb[2] + i13 * b.nb[3] + kg * 32;
+template <int NWK, bool BF> __device__ __forceinline__ mmf_float4 mma16_tile(const char * wrow, const char * xcol, const int64_t K, mmf_float4 (&red)[NWK][64]) {  // the sums: in wave 0
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, kg = lane >> 4;
     mmf_float4 acc = {0, 0, 0, 0};
     for (int64_t k = (int64_t) wave * 32; k < K; k += 32 * NWK * 4) {  // 4 steps' loads in flight
         uint4 w[4], x0[4], x1[4];
@@ -270,9 +261,24 @@ __global__ void __launch_bounds__(64 * NWK) k_mul_mat_f16_mma16(const tdesc a, c
     }
     red[wave][lane] = acc;
     __syncthreads();
-    if (wave != 0) return;
+    if (wave == 0) {
 #pragma unroll
-    for (int w = 1; w < NWK; ++w) acc += red[w][lane];
+        for (int w = 1; w < NWK; ++w) acc += red[w][lane];
+    }
+    return acc;
+}
+template <int NWK, bool BF>
+__global__ void __launch_bounds__(64 * NWK) k_mul_mat_f16_mma16(const tdesc a, const tdesc b, const tdesc d) {
+    __shared__ mmf_float4 red[NWK][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int r16 = lane & 15, kg = lane >> 4;
+    const int64_t row0 = (int64_t) blockIdx.x * 16, col0 = (int64_t) blockIdx.y * 16;
+    const int64_t i12 = blockIdx.z % b.ne[2], i13 = blockIdx.z / b.ne[2];
+    const int64_t i02 = i12 / (b.ne[2] / a.ne[2]), i03 = i13 / (b.ne[3] / a.ne[3]);
+    const char * wrow = a.data + std::min<int64_t>(row0 + r16, a.ne[1] - 1) * a.nb[1] + i02 * a.nb[2] + i03 * a.nb[3] + kg * 16;
+    const char * xcol = b.data + std::min<int64_t>(col0 + r16, b.ne[1] - 1) * b.nb[1] + i12 * b.nb[2] + i13 * b.nb[3] + kg * 32;
+    const mmf_float4 acc = mma16_tile<NWK, BF>(wrow, xcol, a.ne[0], red);
+    if (wave != 0) return;
     // lane: src0 row row0 + r16; register i: src1 column col0 + 4 kg + i
     const int64_t row = row0 + r16;
     if (row >= a.ne[1]) return;
@@ -282,6 +288,30 @@ __global__ void __launch_bounds__(64 * NWK) k_mul_mat_f16_mma16(const tdesc a, c
         const int64_t col = col0 + 4 * kg + i;
         if (col < b.ne[1]) *(float *) (out + col * d.nb[1]) = acc[i];
     }
+}
+// ... up to four bf16 matrices against the same 2 .. 16 columns in one launch (a step's q / k / v / gate projections: four launches of 8.7 us each, of which the weights'
+// bytes are 1 .. 2): the workgroups are dealt over the matrices' 16-row tiles; results dense rows
+template <int NWK>
+__global__ void __launch_bounds__(64 * NWK) k_mul_mat_bf16_mma16_multi(const matvec_multi mm, const char * __restrict__ x, const int64_t x_nb1, const int64_t K, const int M) {
+    __shared__ mmf_float4 red[NWK][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int r16 = lane & 15, kg = lane >> 4;
+    int q = 0;
+    while (q + 1 < mm.n && (int) blockIdx.x >= mm.blk0[q + 1]) ++q;
+    const int64_t row0 = (int64_t) ((int) blockIdx.x - mm.blk0[q]) * 16, N = mm.N[q];
+    const mmf_float4 acc = mma16_tile<NWK, true>(mm.W[q] + std::min<int64_t>(row0 + r16, N - 1) * mm.nb1[q] + kg * 16, x + (int64_t) min(r16, M - 1) * x_nb1 + kg * 32, K, red);
+    if (wave != 0 || row0 + r16 >= N) return;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        if (4 * kg + i < M) mm.dst[q][(int64_t) (4 * kg + i) * N + row0 + r16] = acc[i];
+}
+static bool mma16_applies(int64_t M, int64_t K, int64_t waves32) { return M < 16 || (K >= 1024 && waves32 < 2048); }
+bool mul_mat_bf16_multi_ok(int64_t N, int64_t K, int64_t M) { return M == 1 || (M <= 16 && mma16_applies(M, K, (N + 31) / 32)); }
+void launch_mul_mat_bf16_multi(hipStream_t s, matvec_multi mm, const char * x, int64_t x_nb1, int64_t K, int64_t M) {
+    mm.blk0[0] = 0;
+    for (int q = 0; q < mm.n; ++q) mm.blk0[q + 1] = mm.blk0[q] + (int) ((mm.N[q] + 15) / 16);
+    if (K >= 4096) hipLaunchKernelGGL(k_mul_mat_bf16_mma16_multi<16>, dim3((unsigned) mm.blk0[mm.n]), dim3(1024), 0, s, mm, x, x_nb1, K, (int) M);
+    else hipLaunchKernelGGL(k_mul_mat_bf16_mma16_multi<8>, dim3((unsigned) mm.blk0[mm.n]), dim3(512), 0, s, mm, x, x_nb1, K, (int) M);
 }
 
 // ---- ... and when scratch is at hand (few columns, at most 128 rows, long rows — V^T.p of a -np decode batch): 16 x 16 tiles fetch
@@ -767,7 +797,7 @@ void launch_mul_mat_f(hipStream_t s, const tdesc & a, const tdesc & b, const tde
     }
     if (w16 && vec_ok && b.ne[1] >= 2) {
         const int64_t waves32 = ((a.ne[1] + 31) / 32) * ((b.ne[1] + 31) / 32) * b.ne[2] * b.ne[3];
-        if (b.ne[1] < 16 || (K >= 1024 && waves32 < 2048)) {  // few tiles, long rows (or a handful of columns): split K inside the workgroup
+        if (mma16_applies(b.ne[1], K, waves32)) {  // few tiles, long rows (or a handful of columns): split K inside the workgroup
             dim3 grid((unsigned) ((a.ne[1] + 15) / 16), (unsigned) ((b.ne[1] + 15) / 16), (unsigned) (b.ne[2] * b.ne[3]));
             if (bf) {
                 if (K >= 4096) hipLaunchKernelGGL((k_mul_mat_f16_mma16<16, true>), grid, dim3(1024), 0, s, a, b, d);
@@ -1080,15 +1110,24 @@ size_t mul_mat_id_workspace_bytes(const tdesc & as, const tdesc & ids) {
 }
 // grouped: the column lists made by an earlier call over the same ids (the down projection follows the up projection) are used again
 // returns true when the batched form ran: the column lists of these ids are then in ws (false: ws was not touched)
-bool launch_mul_mat_id(hipStream_t s, const tdesc & as, const tdesc & b, const tdesc & ids, const tdesc & d, void * ws, size_t ws_bytes, bool lists_valid) {
+static bool mul_mat_id_vec_ok(const tdesc & as, const tdesc & b) {
+    bool ok = (as.type == GGML_TYPE_BF16 || as.type == GGML_TYPE_F16) && as.nb[0] == 2 && b.nb[0] == 4 && (as.ne[0] % 8) == 0 && (((uintptr_t) as.data) & 15) == 0 && (((uintptr_t) b.data) & 15) == 0;
+    for (int i = 1; i < 3; ++i) ok = ok && (as.nb[i] % 16) == 0 && (b.nb[i] % 16) == 0;
+    return ok;
+}
+bool mul_mat_id_batched(const tdesc & as, const tdesc & b, const tdesc & ids) { return mul_mat_id_vec_ok(as, b) && ids.ne[0] * ids.ne[1] >= 64 && as.ne[2] <= 65535; }
+bool launch_mul_mat_id(hipStream_t s, const tdesc & as, const tdesc & b, const tdesc & ids, const tdesc & d, void * ws, size_t ws_bytes, bool lists_valid, const void * x16) {
     const int64_t K = as.ne[0], n_used = ids.ne[0], T = ids.ne[1];
     if (as.ne[1] == 0 || n_used * T == 0) return false;
     const bool bf = as.type == GGML_TYPE_BF16, w16 = bf || as.type == GGML_TYPE_F16;
-    bool vec_ok = w16 && as.nb[0] == 2 && b.nb[0] == 4 && (K % 8) == 0 && (((uintptr_t) as.data) & 15) == 0 && (((uintptr_t) b.data) & 15) == 0;
-    for (int i = 1; i < 3; ++i) vec_ok = vec_ok && (as.nb[i] % 16) == 0 && (b.nb[i] % 16) == 0;
-    if (vec_ok && n_used * T >= 64 && as.ne[2] <= 65535 && ws && mul_mat_id_workspace_bytes(as, ids) <= ws_bytes) {
+    const bool vec_ok = mul_mat_id_vec_ok(as, b);
+    if (mul_mat_id_batched(as, b, ids) && ws && mul_mat_id_workspace_bytes(as, ids) <= ws_bytes) {
         int32_t * cnt = (int32_t *) ws, * off = cnt + as.ne[2], * list = off + as.ne[2];
         if (!lists_valid) hipLaunchKernelGGL(k_moe_group, dim3((unsigned) as.ne[2]), dim3(256), 0, s, ids, (int) as.ne[2], cnt, off, list);
+        if (x16) {
+            launch_mul_mat_id_tile(s, as, b.ne[1], n_used, T, d, cnt, off, list, x16);
+            return true;
+        }
         // column tiles per expert in the grid: enough for an even spread (the loop inside covers an expert that drew more)
         const int64_t even = (n_used * T + as.ne[2] - 1) / as.ne[2];
         const dim3 grid((unsigned) ((as.ne[1] + 63) / 64), (unsigned) std::max<int64_t>(1, std::min<int64_t>(64, (even + 63) / 64 * 2)), (unsigned) as.ne[2]);

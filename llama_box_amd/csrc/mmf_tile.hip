@@ -1,0 +1,269 @@
+// mmf_tile.hip — MUL_MAT / MUL_MAT_ID of a batch of columns by f16 / bf16 matrices: LDS-tiled, on v_mfma_f32_32x32x16_{f16,bf16}.
+//
+// The contract is mmf.hip's (ggml_compute_forward_mul_mat): src1 is rounded to src0's 16-bit type (nearest even), products
+// are exact in f32 and accumulated in f32.  One accumulator per output walks K in steps of 16, in order, whatever the tile: the result does not depend on the tile
+// chosen, on the matrices that share the launch or on the other columns.
+//
+// A workgroup of four waves owns TM src1 columns x TN src0 rows and advances K by 64.  Both operands arrive by LDS-DMA (global_load_lds_dwordx4, 1 KB = 8 rows of
+// 128 bytes per wave-instruction) into a ring of S stages, S - 1 of them in flight: with one stage ahead in registers a step of 128 x 128 took 1.7 us, the latency of
+// its loads, against 0.2 us of matrix work.  src1 is rounded to 16 bits once per tensor (k_to_16: the q / k / v / gate projections read the same copy), which halves
+// its share of the 64 bytes per clock a CU can fetch — what bounds a 64 x 128 tile.  LDS rows hold the 16-byte chunk index XORed by (row >> 1) & 7 (the lanes
+// of the DMA fetch the permuted chunks): the 16 lanes a ds_read_b128 serves at once hit 16 distinct slots.  One barrier per step.  Workgroups that read the same src0
+// rows follow one another on one XCD.
+#include <algorithm>
+#include <atomic>
+#include <cstdlib>
+
+#include "dev_util.h"
+#include "kernels.h"
+
+namespace mi355x {
+
+typedef _Float16 mt_half8 __attribute__((ext_vector_type(8)));
+typedef __bf16 mt_bf8 __attribute__((ext_vector_type(8)));
+typedef float mt_float16 __attribute__((ext_vector_type(16)));
+
+// lane i's 16 bytes at base + off land at LDS[lds + 16 i]; base and lds are wave-uniform (M0 is written in the statement that uses it).  No memory clobber: the stage
+// written is one that nobody reads before the next barrier, so the compiler may move LDS reads across
+__device__ __forceinline__ void mt_dma16(const char * base, const uint32_t off, const uint32_t lds) {
+    uint32_t keep;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0" : "=&s"(keep) : "v"(off), "s"(base), "s"(lds));
+}
+
+// f32 rows -> dense rows of src0's 16-bit type, nearest even.  Two float4 in, one uint4 out per thread
+template <bool BF> __global__ void __launch_bounds__(256) k_to_16(const char * __restrict__ x, const int64_t nb1, const int64_t K8, const int64_t total, uint4 * __restrict__ out) {
+    const int64_t i = (int64_t) blockIdx.x * 256 + threadIdx.x;
+    if (i >= total) return;
+    const int64_t r = i / K8, c = i - r * K8;
+    const float4 p = *(const float4 *) (x + r * nb1 + c * 32), q = *(const float4 *) (x + r * nb1 + c * 32 + 16);
+    const float v[8] = {p.x, p.y, p.z, p.w, q.x, q.y, q.z, q.w};
+    uint4 o;
+    if constexpr (BF) {
+        mt_bf8 h;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) h[k] = (__bf16) v[k];
+        o = __builtin_bit_cast(uint4, h);
+    } else {
+        mt_half8 h;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) h[k] = (_Float16) v[k];
+        o = __builtin_bit_cast(uint4, h);
+    }
+    out[i] = o;
+}
+
+struct mt_mat {
+    const char * W;
+    int64_t nb1;
+    int64_t N;
+    int tile_end;  // row tiles [previous matrix's tile_end, tile_end) are this matrix's
+    char * dst;
+    int64_t dst_nb1;
+};
+struct mt_args {
+    mt_mat m[4];    // up to four matrices over the same columns
+    int64_t K, M;
+    const char * x;  // src1 in 16 bits, dense rows
+    int n_tiles, m_tiles;
+    // ID: the columns of expert blockIdx.z are list[off[e] .. off[e] + cnt[e]), entry u + n_used t: src1 row (u % ne11) + ne11 t, result row (u, t)
+    const int32_t * cnt, * off, * list;
+    int64_t n_used, ne11, w_nb2, d_nb2;
+};
+
+template <bool BF, int TM, int TN, int S, bool ID> __global__ void __launch_bounds__(256, 1) k_mul_mat_tile(const mt_args a) {
+    constexpr int MT = TM / 64, NT = TN / 64;
+    constexpr int STAGE = (TM + TN) * 128, L = (TM + TN) / 32;  // bytes of a stage, DMA instructions per wave and stage
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int fr = lane & 31, g = lane >> 5, wm = wave & 1, wn = wave >> 1;
+    int tile, mt0, e = 0;
+    int64_t M = a.M;
+    if constexpr (ID) {
+        tile = blockIdx.x;
+        mt0 = blockIdx.y;
+        e = blockIdx.z;
+        M = a.cnt[e];
+    } else {
+        const int xcd = blockIdx.x & 7, q = blockIdx.x >> 3;
+        tile = (q / a.m_tiles) * 8 + xcd;
+        mt0 = q % a.m_tiles;
+        if (tile >= a.n_tiles) return;
+    }
+    int mi = 0;
+    if constexpr (!ID) mi = tile < a.m[0].tile_end ? 0 : (tile < a.m[1].tile_end ? 1 : (tile < a.m[2].tile_end ? 2 : 3));
+    const mt_mat & mat = a.m[mi];
+    const int64_t n0 = (int64_t) (tile - (mi ? a.m[mi - 1].tile_end : 0)) * TN, N = mat.N, K = a.K;
+    const int32_t * cols = ID ? a.list + a.off[e] : nullptr;
+    const char * const wbase = mat.W + n0 * mat.nb1 + (ID ? e * a.w_nb2 : 0);
+    const int swz = (fr >> 1) & 7, steps = (int) (K / 64);
+    const char * const fx = smem + (wm * (TM / 2) + fr) * 128, * const fw = smem + (TM + wn * (TN / 2) + fr) * 128;
+    const uint32_t lds0 = (uint32_t) (uintptr_t) smem;
+
+    // (a workgroup of an expert walks the expert's column tiles, the grid's second dimension strides them)
+    for (int mt = mt0; ; mt += ID ? (int) gridDim.y : 0) {
+        const int64_t m0 = (int64_t) mt * TM;
+        if (ID && m0 >= M) return;
+        auto uniform = [](const char * q) {  // (wave-uniform by construction; into scalar registers)
+            const uint64_t v = (uint64_t) (uintptr_t) q;
+            return (const char *) (uintptr_t) (((uint64_t) (uint32_t) __builtin_amdgcn_readfirstlane((int) (v >> 32)) << 32) | (uint32_t) __builtin_amdgcn_readfirstlane((int) v));
+        };
+        // this wave's DMA instructions: 8 rows each, of src1 below TM and of src0 from there; lane -> row lane / 8, the permuted chunk of slot lane % 8
+        const char * base[L];
+        uint32_t off[L];
+#pragma unroll
+        for (int j = 0; j < L; ++j) {
+            const int r0 = (wave * L + j) * 8, row = r0 + (lane >> 3), chunk = (lane & 7) ^ ((row >> 1) & 7);
+            if (r0 < TM) {
+                int64_t m = std::min<int64_t>(m0 + row, M - 1);
+                if constexpr (ID) {
+                    const int32_t ci = cols[m];
+                    m = (ci % a.n_used) % a.ne11 + (ci / a.n_used) * a.ne11;
+                    base[j] = uniform(a.x);
+                    off[j] = (uint32_t) (m * K * 2 + chunk * 16);
+                } else {
+                    base[j] = uniform(a.x + m0 * K * 2);
+                    off[j] = (uint32_t) ((m - m0) * K * 2 + chunk * 16);
+                }
+            } else {
+                base[j] = uniform(wbase);
+                off[j] = (uint32_t) (std::min<int64_t>(row - TM, N - 1 - n0) * mat.nb1 + chunk * 16);
+            }
+        }
+        auto issue = [&](const int s, const int j0, const int j1) {
+            const uint32_t to = lds0 + (uint32_t) (s % S) * STAGE + (uint32_t) wave * L * 1024;
+#pragma unroll
+            for (int j = j0; j < j1; ++j) mt_dma16(base[j] + (int64_t) s * 128, off[j], to + j * 1024);
+        };
+        mt_float16 acc[MT][NT];
+#pragma unroll
+        for (int t = 0; t < MT; ++t)
+#pragma unroll
+            for (int u = 0; u < NT; ++u) acc[t][u] = (mt_float16){0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+        if (ID && mt != mt0) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");  // (the ring is free, no store is counted in vmcnt)
+#pragma unroll
+        for (int s = 0; s < S - 1; ++s)
+            if (s < steps) issue(s, 0, L);
+        for (int s = 0; s < steps; ++s) {
+            // this wave's pieces of step s have landed (in-order vmcnt: only the S - 2 steps behind it may still fly), then everybody's have, and nobody reads step
+            // s - 1 any more: its stage is the one requested next
+            if (s + S - 2 < steps) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((S - 2) * L) : "memory");
+            else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            const int bo = (s % S) * STAGE;
+            uint4 xa[2][MT], wb[2][NT];
+            auto frags = [&](const int ks) {
+                const int co = ((2 * ks + g) ^ swz) << 4;
+#pragma unroll
+                for (int t = 0; t < MT; ++t) xa[ks & 1][t] = *(const uint4 *) (fx + bo + t * 32 * 128 + co);
+#pragma unroll
+                for (int u = 0; u < NT; ++u) wb[ks & 1][u] = *(const uint4 *) (fw + bo + u * 32 * 128 + co);
+            };
+            frags(0);
+#pragma unroll
+            for (int ks = 0; ks < 4; ++ks) {
+                if (ks < 3) frags(ks + 1);
+                if (s + S - 1 < steps) issue(s + S - 1, ks * L / 4, (ks + 1) * L / 4);  // (a quarter at a time: the CU's one address pipeline takes 16 clocks for each)
+#pragma unroll
+                for (int t = 0; t < MT; ++t)
+#pragma unroll
+                    for (int u = 0; u < NT; ++u) {
+                        if constexpr (BF) acc[t][u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(mt_bf8, xa[ks & 1][t]), __builtin_bit_cast(mt_bf8, wb[ks & 1][u]), acc[t][u], 0, 0, 0);
+                        else acc[t][u] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(mt_half8, xa[ks & 1][t]), __builtin_bit_cast(mt_half8, wb[ks & 1][u]), acc[t][u], 0, 0, 0);
+                    }
+            }
+        }
+        // lane: src0 row; register i: src1 column (i & 3) + 8 (i >> 2) + 4 g — 32 lanes store a whole 128-byte line
+#pragma unroll
+        for (int u = 0; u < NT; ++u) {
+            const int64_t n = n0 + wn * (TN / 2) + u * 32 + fr;
+            if (n >= N) continue;
+#pragma unroll
+            for (int t = 0; t < MT; ++t)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {
+                    const int64_t m = m0 + wm * (TM / 2) + t * 32 + (i & 3) + 8 * (i >> 2) + 4 * g;
+                    if (m < M) {
+                        char * out;
+                        if constexpr (ID) {
+                            const int32_t ci = cols[m];
+                            out = mat.dst + (ci % a.n_used) * mat.dst_nb1 + (ci / a.n_used) * a.d_nb2;
+                        } else out = mat.dst + m * mat.dst_nb1;
+                        *(float *) (out + n * 4) = acc[t][u][i];
+                    }
+                }
+        }
+        if constexpr (!ID) return;
+    }
+}
+
+// The tile and its ring.  Measured (us; bf16, 512 columns unless stated; 128 x 128 with two stages and two workgroups per CU / 64 x 128 with five / 64 x 64 with four; before: one wave
+// per 32 x 32 tile, operands straight from global memory): K 4096 N 14336: 90 / 136 / 125 (623), N 10240: 86 / 102 / 92 (453), N 4096: 57 / 36 / 33 (184); K 14336 N 4096: 224 / 113 /
+// 128 (645); 128 columns, N 14336: 76 / 44 / 46 (313), N 4096: 55 / 32 / 23 (94); 64 columns, N 14336: 74 / 43 / 34 (163), N 4096: 54 / 32 / 22 (51).
+static void mt_pick(const mul_mat_tile_desc * m, int n, int64_t M, int * tm, int * tn) {
+    auto count = [&](int64_t TM, int64_t TN) {
+        int64_t t = 0;
+        for (int q = 0; q < n; ++q) t += (m[q].N + TN - 1) / TN;
+        return t * ((M + TM - 1) / TM);
+    };
+    *tm = 64;
+    *tn = 64;
+    if (M > 64 && count(128, 128) >= 288) { *tm = 128; *tn = 128; }     // more than one workgroup per CU: the fewest bytes per product
+    else if (M > 64 && count(64, 128) >= 192) *tn = 128;                // most CUs have one
+}
+template <bool BF, int TM, int TN, int S, bool ID> static void mt_launch_t(hipStream_t s, const dim3 grid, const mt_args & a) {
+    const size_t lds = (size_t) S * (TM + TN) * 128;
+    static std::atomic<uint32_t> raised{0};  // one bit per device (common.h: ensure_dyn_lds)
+    (void) ensure_dyn_lds((const void *) k_mul_mat_tile<BF, TM, TN, S, ID>, lds, raised);  // on failure the launch below fails and graph_compute reports it
+    hipLaunchKernelGGL((k_mul_mat_tile<BF, TM, TN, S, ID>), grid, dim3(256), lds, s, a);
+}
+bool mul_mat_tile_ok(int type, int64_t K, int64_t N, int64_t nb0, int64_t nb1, const void * W) {
+    return (type == GGML_TYPE_F16 || type == GGML_TYPE_BF16) && nb0 == 2 && K >= 64 && (K % 64) == 0 && N >= 1 && (nb1 % 16) == 0 && (((uintptr_t) W) & 15) == 0 && 128 * nb1 < ((int64_t) 1 << 31);
+}
+void launch_to_16(hipStream_t s, int type, const char * x, int64_t nb1, int64_t K, int64_t rows, void * out) {
+    const int64_t total = rows * (K / 8);
+    const dim3 grid((unsigned) ((total + 255) / 256));
+    if (type == GGML_TYPE_BF16) hipLaunchKernelGGL(k_to_16<true>, grid, dim3(256), 0, s, x, nb1, K / 8, total, (uint4 *) out);
+    else hipLaunchKernelGGL(k_to_16<false>, grid, dim3(256), 0, s, x, nb1, K / 8, total, (uint4 *) out);
+}
+void launch_mul_mat_tile(hipStream_t s, int type, const mul_mat_tile_desc * m, int n, int64_t K, int64_t M, const void * x16) {
+    mt_args a{};
+    int tm, tn;
+    mt_pick(m, n, M, &tm, &tn);
+    int64_t t = 0;
+    for (int q = 0; q < 4; ++q) {
+        const mul_mat_tile_desc & d = m[q < n ? q : n - 1];
+        if (q < n) t += (d.N + tn - 1) / tn;
+        a.m[q] = {(const char *) d.W, d.nb1, d.N, (int) t, (char *) d.dst, d.dst_nb1};
+    }
+    a.K = K;
+    a.M = M;
+    a.x = (const char *) x16;
+    a.n_tiles = (int) t;
+    a.m_tiles = (int) ((M + tm - 1) / tm);
+    const dim3 grid((unsigned) ((a.n_tiles + 7) / 8 * 8 * a.m_tiles));
+    const bool bf = type == GGML_TYPE_BF16;
+#define MT(TM_, TN_, S_) { if (bf) mt_launch_t<true, TM_, TN_, S_, false>(s, grid, a); else mt_launch_t<false, TM_, TN_, S_, false>(s, grid, a); }
+    if (tm == 128) MT(128, 128, 2)
+    else if (tn == 128) MT(64, 128, 5)
+    else MT(64, 64, 4)
+#undef MT
+}
+
+void launch_mul_mat_id_tile(hipStream_t s, const tdesc & as, int64_t n_b, int64_t n_used, int64_t T, const tdesc & d, const int32_t * cnt, const int32_t * off, const int32_t * list, const void * x16) {
+    mt_args a{};
+    const int64_t even = (n_used * T + as.ne[2] - 1) / as.ne[2];  // columns per expert when they are spread evenly (the loop inside covers an expert that drew more)
+    for (int q = 0; q < 4; ++q) a.m[q] = {as.data, as.nb[1], as.ne[1], 0, d.data, d.nb[1]};
+    a.K = as.ne[0];
+    a.x = (const char *) x16;
+    a.cnt = cnt; a.off = off; a.list = list;
+    a.n_used = n_used; a.ne11 = n_b; a.w_nb2 = as.nb[2]; a.d_nb2 = d.nb[2];
+    const int64_t slots = std::max<int64_t>(1, std::min<int64_t>(64, (even + 63) / 64 * 2));
+    const int tn = (as.ne[1] + 127) / 128 * std::max<int64_t>(1, even / 64) * as.ne[2] >= 192 ? 128 : 64;
+    const dim3 grid((unsigned) ((as.ne[1] + tn - 1) / tn), (unsigned) slots, (unsigned) as.ne[2]);
+    const bool bf = as.type == GGML_TYPE_BF16;
+    if (tn == 128) { if (bf) mt_launch_t<true, 64, 128, 3, true>(s, grid, a); else mt_launch_t<false, 64, 128, 3, true>(s, grid, a); }
+    else { if (bf) mt_launch_t<true, 64, 64, 4, true>(s, grid, a); else mt_launch_t<false, 64, 64, 4, true>(s, grid, a); }
+}
+
+MI_TU_TOUCH(mmf_tile)
+
+}  // namespace mi355x

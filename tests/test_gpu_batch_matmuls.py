@@ -3,6 +3,7 @@ import numpy as np
 import pytest
 
 import harness as T
+import nigozen_ref as R
 import llama_box_amd as L
 
 pytestmark = pytest.mark.gpu
@@ -36,3 +37,75 @@ def test_q8_0_batches_of_33_columns_and_up(backend, H, K, N, M):
     wr, br = np.ascontiguousarray(w[rows]), np.ascontiguousarray(b[:, rows])
     ref = T.run_case(lambda g: H.ggml_add(g.ctx, H.ggml_mul_mat(g.ctx, g.new(L.Q8_0, [K, len(rows)], wr), g.new(L.F32, [K, M], x)), g.new(L.F32, [len(rows), M], br)), "oracle")[0].reshape(M, -1)
     assert T.nmse(got[:, rows], ref) <= 1e-10
+
+
+def round16(a, wt):
+    return R.bf16_round(a) if wt == L.BF16 else a.astype(np.float16).astype(np.float32)
+
+
+def bits16(a, wt):
+    return (np.ascontiguousarray(a, np.float32).view(np.uint32) >> 16).astype(np.uint16) if wt == L.BF16 else a.astype(np.float16)
+
+
+# one step of K and many, row tiles of 64 / 128 with a remainder, column tiles with one column too many or too few, and sizes on both sides of the tiles' dispatch
+@pytest.mark.parametrize("wt", [L.BF16, L.F16])
+@pytest.mark.parametrize("K,N,M", [(64, 30, 17), (128, 64, 63), (192, 65, 64), (1024, 200, 65), (320, 129, 127), (64, 4100, 330), (256, 12300, 200), (128, 18500, 257), (4096, 96, 40)])
+def test_16_bit_matrices_with_batches(backend, H, wt, K, N, M):
+    """mmf_tile.hip against float64 over the rounded operands.  f32 sums of K products of size ~1 / sqrt(K): off by at most K eps |x| |w| ~ K 6e-8, in practice its root."""
+    rng = np.random.default_rng(K + N + M)
+    w = round16((rng.standard_normal((N, K)) / np.sqrt(K)).astype(np.float32), wt)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+
+    def build(g):
+        return H.ggml_mul_mat(g.ctx, g.new(wt, [K, N], bits16(w, wt)), g.new(L.F32, [K, M], x))
+
+    got = T.run_case(build, backend)[0].reshape(M, N)
+    ref = round16(x, wt).astype(np.float64) @ w.astype(np.float64).T
+    assert np.abs(got - ref).max() <= 6e-8 * np.sqrt(K) * 8
+
+
+@pytest.mark.parametrize("M", [2, 16, 17, 150])
+def test_16_bit_siblings_have_the_bits_of_single_launches(backend, H, M):
+    """three bf16 matrices over one input: one launch (and one rounding of the input), the results of three"""
+    rng = np.random.default_rng(M)
+    K, Ns = 1024, (300, 64, 70)
+    ws = [round16((rng.standard_normal((n, K)) / np.sqrt(K)).astype(np.float32), L.BF16) for n in Ns]
+    x = rng.standard_normal((M, K)).astype(np.float32)
+
+    def build(g):
+        cur = g.new(L.F32, [K, M], x)
+        return [H.ggml_mul_mat(g.ctx, g.new(L.BF16, [K, n], bits16(w, L.BF16)), cur) for n, w in zip(Ns, ws)]
+
+    k0 = backend.stat("kernel_launches")
+    got = T.run_case(build, backend)
+    merged = backend.stat("kernel_launches") - k0
+    backend.set_option("fusion", 0)
+    try:
+        plain = T.run_case(build, backend)
+    finally:
+        backend.set_option("fusion", 1)
+    assert merged == (1 if M < 17 else 2)
+    for a, b, w in zip(got, plain, ws):
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+        ref = round16(x, L.BF16).astype(np.float64) @ w.astype(np.float64).T
+        assert np.abs(a.reshape(M, -1) - ref).max() <= 6e-8 * np.sqrt(K) * 8
+
+
+# columns of an expert: none, fewer than a tile, several tiles (one expert draws most)
+@pytest.mark.parametrize("K,N,n_exp,top,T_", [(64, 40, 5, 2, 40), (128, 200, 8, 1, 300), (192, 130, 3, 3, 70), (256, 4160, 6, 2, 100)])
+def test_experts_with_batches(backend, H, K, N, n_exp, top, T_):
+    rng = np.random.default_rng(K + N + T_)
+    w = round16((rng.standard_normal((n_exp, N, K)) / np.sqrt(K)).astype(np.float32), L.BF16)
+    x = rng.standard_normal((T_, 1, K)).astype(np.float32)
+    ids = np.stack([rng.permutation(n_exp - 1 if n_exp > top else n_exp)[:top] for _ in range(T_)]).astype(np.int32)  # (the last expert draws nothing when it can be left out)
+    ids[: T_ // 2, 0], swap = 0, ids[: T_ // 2, 0].copy()
+    for t in range(T_ // 2):
+        ids[t, 1:][ids[t, 1:] == 0] = swap[t]
+
+    def build(g):
+        return H.ggml_mul_mat_id(g.ctx, g.new(L.BF16, [K, N, n_exp], bits16(w, L.BF16)), g.new(L.F32, [K, 1, T_], x), g.new(L.I32, [top, T_], ids))
+
+    got = T.run_case(build, backend)[0].reshape(T_, top, N)
+    xr = round16(x, L.BF16).astype(np.float64)[:, 0]
+    ref = np.stack([[w[ids[t, u]].astype(np.float64) @ xr[t] for u in range(top)] for t in range(T_)])
+    assert np.abs(got - ref).max() <= 6e-8 * np.sqrt(K) * 8
