@@ -392,21 +392,58 @@ __device__ __forceinline__ uint32_t att_bf16_bits(const float f) {
     const uint32_t u = __float_as_uint(f);
     return (u + 0x7FFFu + ((u >> 16) & 1u)) >> 16;
 }
-template <int DK16, int DVT>
-__global__ void __launch_bounds__(256) k_attn_mma_bf16(const tdesc q, const tdesc k, const tdesc v, const tdesc mask, const float * __restrict__ sinks, const float * __restrict__ r12, const tdesc dst,
+typedef __bf16 att_bf2 __attribute__((ext_vector_type(2)));
+typedef float att_f2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t att_bf16_pack(const float a, const float b) {  // two values to bf16, nearest even, in one instruction
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((att_f2){a, b}, att_bf2));
+}
+// NV: value shares of 8 entries x 4 cells per thread and block (8 x DVT x 4 of them over the workgroup's threads).  PLAIN: scores are q.k x scale + mask (no sigmoid, cap or distance
+// penalty), head sizes exactly 16 DK16 / 32 DVT.
+// First the mask is scanned for the blocks of 32 cells that anybody in the workgroup sees (a bit each), then the visible ones are walked: the next one's K operands, V entries
+// and mask terms travel while the current one is multiplied, V^T alternates between two LDS copies, one barrier per block.  A 2000-token prompt in portions of 512, 32 heads of 128
+// on 8 key heads, per launch: 217 us with the mask, the K and V of a block read one after the other and the variants' branches inside, 97 us as it is.
+constexpr int ATT_SCAN_BITS = 16384;  // blocks beyond these are taken as visible (a wave that sees nothing of a block still skips it)
+template <int DK16, int DVT, int NV, bool PLAIN>
+__global__ void __launch_bounds__(256, 2) k_attn_mma_bf16(const tdesc q, const tdesc k, const tdesc v, const tdesc mask, const float * __restrict__ sinks, const float * __restrict__ r12, const tdesc dst,
                                                        const float scale, const float * __restrict__ sig, const float softcap, const int pen_kind) {
     constexpr int VS = 36;  // V^T row stride in LDS (bf16 elements): 72 bytes keeps the 8-byte reads aligned and spreads the rows over the banks
-    __shared__ __attribute__((aligned(16))) uint16_t Vt[DVT * 32 * VS];
-    __shared__ int flag[2];
+    __shared__ __attribute__((aligned(16))) uint16_t Vt2[2][DVT * 32 * VS];
+    __shared__ uint32_t bits[ATT_SCAN_BITS / 32];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int n = lane & 31, g = lane >> 5;
     const int64_t h = blockIdx.y, n_q = q.ne[1], n_kv = k.ne[1];
-    const int DK = (int) q.ne[0], DV = (int) v.ne[0];
+    const int DK = PLAIN ? 16 * DK16 : (int) q.ne[0], DV = PLAIN ? 32 * DVT : (int) v.ne[0];
     const int64_t tq = (int64_t) blockIdx.x * (blockDim.x / 2) + wave * 32 + n;  // this lane's query (a workgroup of 1, 2 or 4 waves: 32 queries a wave)
     const bool q_live = tq < n_q;
     const int64_t kvh = h / (q.ne[2] / k.ne[2]);
-    const char * kbase = k.data + kvh * k.nb[2];
+    const char * kbase = k.data + kvh * k.nb[2] + g * 16;
     const char * vbase = v.data + kvh * v.nb[2];
+    const char * mrow = mask.data + (q_live ? tq : n_q - 1) * mask.nb[1];
+    const int n_blk = (int) ((n_kv + 31) / 32), n_scan = min(n_blk, ATT_SCAN_BITS);
+    // this lane's 16 mask terms of a block: cells 32 blk + 8 b + 4 g .. + 3, b = 0 .. 3 (register i = 4 b + r)
+    auto load_mask = [&](const int blk, float (&mv)[16]) {
+        const int64_t j0 = (int64_t) blk * 32 + 4 * g;
+        if ((int64_t) blk * 32 + 32 <= n_kv) {  // (uniform)
+#pragma unroll
+            for (int b = 0; b < 4; ++b) {
+                const float4 t = *(const float4 *) (mrow + (j0 + 8 * b) * 4);
+                mv[4 * b] = t.x; mv[4 * b + 1] = t.y; mv[4 * b + 2] = t.z; mv[4 * b + 3] = t.w;
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const int64_t j = j0 + 8 * (i >> 2) + (i & 3);
+                mv[i] = j < n_kv ? ((const float *) mrow)[j] : -INFINITY;
+            }
+        }
+    };
+    auto seen = [&](const float (&mv)[16]) {
+        float t = mv[0];
+#pragma unroll
+        for (int i = 1; i < 16; ++i) t = fmaxf(t, mv[i]);
+        return __ballot(q_live && t > -INFINITY) != 0;
+    };
+    for (int i = threadIdx.x; i < (n_scan + 31) / 32; i += blockDim.x) bits[i] = 0;
     // the wave's queries as second operands: element group (16 s + 8 g .. + 7) of query n
     uint4 qf[DK16];
     {
@@ -414,15 +451,37 @@ __global__ void __launch_bounds__(256) k_attn_mma_bf16(const tdesc q, const tdes
 #pragma unroll
         for (int s = 0; s < DK16; ++s) {
             const int i0 = 16 * s + 8 * g;
-            uint32_t b[8];
+            uint32_t b[4];
 #pragma unroll
-            for (int e = 0; e < 8; ++e) b[e] = (q_live && i0 + e < DK) ? att_bf16_bits(qrow[i0 + e]) : 0u;
-            qf[s] = make_uint4(b[0] | (b[1] << 16), b[2] | (b[3] << 16), b[4] | (b[5] << 16), b[6] | (b[7] << 16));
+            for (int e = 0; e < 4; ++e) {
+                const float x = (q_live && i0 + 2 * e < DK) ? qrow[i0 + 2 * e] : 0.0f, y = (q_live && i0 + 2 * e + 1 < DK) ? qrow[i0 + 2 * e + 1] : 0.0f;
+                b[e] = att_bf16_pack(x, y);
+            }
+            qf[s] = make_uint4(b[0], b[1], b[2], b[3]);
         }
     }
-    const int pen = r12 ? pen_kind : 0;
+    __syncthreads();
+    for (int blk = 0; blk < n_scan; blk += 4) {  // (four blocks' loads in flight; past the end the last block again)
+        float t0[16], t1[16], t2[16], t3[16];
+        load_mask(blk, t0);
+        load_mask(min(blk + 1, n_blk - 1), t1);
+        load_mask(min(blk + 2, n_blk - 1), t2);
+        load_mask(min(blk + 3, n_blk - 1), t3);
+        const uint32_t w = (seen(t0) ? 1u : 0u) | (seen(t1) ? 2u : 0u) | (seen(t2) ? 4u : 0u) | (seen(t3) ? 8u : 0u);
+        if (lane == 0 && w) atomicOr(&bits[blk >> 5], w << (blk & 31));
+    }
+    __syncthreads();
+    auto next_block = [&](int blk) {  // the first visible block from blk on (n_blk: none); uniform
+        while (blk < n_scan) {
+            const uint32_t w = (uint32_t) __builtin_amdgcn_readfirstlane((int) bits[blk >> 5]) >> (blk & 31);
+            if (w) { blk += __builtin_ctz(w); break; }
+            blk = (blk | 31) + 1;
+        }
+        return blk < n_blk ? (blk < n_scan || n_scan < n_blk ? blk : n_blk) : n_blk;
+    };
+    const int pen = PLAIN ? 0 : (r12 ? pen_kind : 0);
     const float r1 = pen ? r12[h] : 0.0f, r2 = pen == ATTN_PEN_LOG ? r12[q.ne[2] + h] : 0.0f;
-    const bool sgm = sig != nullptr;
+    const bool sgm = PLAIN ? false : sig != nullptr;
     const float s_temp = sgm ? sig[h] : 1.0f, s_bias = sgm ? sig[q.ne[2] + h] : 0.0f;
     float m = sgm ? 0.0f : (sinks ? sinks[h] : ATTN_F32_LOW), l = (sinks && !sgm) ? 1.0f : 0.0f;
     att_f16v O[DVT];
@@ -430,79 +489,83 @@ __global__ void __launch_bounds__(256) k_attn_mma_bf16(const tdesc q, const tdes
     for (int dt = 0; dt < DVT; ++dt)
 #pragma unroll
         for (int i = 0; i < 16; ++i) O[dt][i] = 0.0f;
-    const char * mrow = mask.data + (q_live ? tq : 0) * mask.nb[1];
-    if (threadIdx.x < 2) flag[threadIdx.x] = 0;
-    __syncthreads();
-    // this lane's 16 mask terms of a block: cells j0 + 8 b + 4 g .. + 3, b = 0 .. 3 (register i = 4 b + r); the NEXT block's terms are requested while the
-    // current block is worked on (three dependent trips to memory per block — mask, V, K — were what bound this kernel)
-    auto load_mask = [&](const int64_t j0, float (&mv)[16]) {
-#pragma unroll
-        for (int b = 0; b < 4; ++b) {
-            const int64_t j = j0 + 8 * b + 4 * g;
-            float4 t = make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
-            if (q_live && j + 3 < n_kv) t = *(const float4 *) (mrow + j * 4);
-            else if (q_live) {
-                if (j < n_kv) t.x = ((const float *) mrow)[j];
-                if (j + 1 < n_kv) t.y = ((const float *) mrow)[j + 1];
-                if (j + 2 < n_kv) t.z = ((const float *) mrow)[j + 2];
-            }
-            mv[4 * b] = t.x; mv[4 * b + 1] = t.y; mv[4 * b + 2] = t.z; mv[4 * b + 3] = t.w;
-        }
-    };
+    uint4 kn[DK16], vn[NV][4];
     float mv_next[16];
-    load_mask(0, mv_next);
-    for (int64_t j0 = 0, blk = 0; j0 < n_kv; j0 += 32, ++blk) {
-        float mv[16];
-        bool any = false;
+    auto fetch = [&](const int blk) {  // a block's K operands, this thread's share of its V (8 consecutive entries of FOUR neighbouring cells), its mask terms
+        const int64_t j0 = (int64_t) blk * 32;
+        const char * krow = kbase + std::min<int64_t>(j0 + n, n_kv - 1) * k.nb[1];
 #pragma unroll
-        for (int i = 0; i < 16; ++i) { mv[i] = mv_next[i]; any = any || mv[i] > -INFINITY; }
-        if (j0 + 32 < n_kv) load_mask(j0 + 32, mv_next);
-        const bool wave_any = __ballot(any) != 0;
-        if (threadIdx.x == 0) flag[(blk + 1) & 1] = 0;
-        if (wave_any && lane == 0) flag[blk & 1] = 1;
-        __syncthreads();
-        if (!flag[blk & 1]) continue;  // (the same answer for every thread of the workgroup)
-        // the block's K operands are requested first, so that they travel while V^T is staged
-        uint4 kf[DK16];
-        {
-            const int64_t cell = j0 + n < n_kv ? j0 + n : n_kv - 1;
-            const char * krow = kbase + cell * k.nb[1] + g * 16;
-#pragma unroll
-            for (int s = 0; s < DK16; ++s) {
-                kf[s] = make_uint4(0, 0, 0, 0);
-                if (wave_any && 16 * s + 8 * g < DK) kf[s] = *(const uint4 *) (krow + s * 32);
+        for (int s = 0; s < DK16; ++s) {
+            if constexpr (PLAIN) kn[s] = *(const uint4 *) (krow + s * 32);
+            else {
+                kn[s] = make_uint4(0, 0, 0, 0);
+                if (16 * s + 8 * g < DK) kn[s] = *(const uint4 *) (krow + s * 32);
             }
         }
-        // V^T of the block into LDS: a thread takes 8 consecutive value entries of FOUR neighbouring cells and writes eight 8-byte groups (4 cells of one entry)
-        for (int e0 = threadIdx.x; e0 < 8 * (DVT * 4); e0 += blockDim.x) {
-            const int cg = e0 / (DVT * 4), c8 = e0 % (DVT * 4);
-            uint32_t u[4][4];
+#pragma unroll
+        for (int r = 0; r < NV; ++r) {
+            const int e0 = min((int) threadIdx.x + r * (int) blockDim.x, 32 * DVT - 1), cg = e0 / (DVT * 4), c8 = e0 % (DVT * 4);
 #pragma unroll
             for (int cc = 0; cc < 4; ++cc) {
-                uint4 t = make_uint4(0, 0, 0, 0);
-                if (j0 + 4 * cg + cc < n_kv && 8 * c8 < DV) t = *(const uint4 *) (vbase + (j0 + 4 * cg + cc) * v.nb[1] + c8 * 16);
-                u[cc][0] = t.x; u[cc][1] = t.y; u[cc][2] = t.z; u[cc][3] = t.w;
-            }
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                // entries 2 e (low halves) and 2 e + 1 (high halves) of the four cells
-                const uint2 lo2 = make_uint2((u[0][e] & 0xFFFFu) | (u[1][e] << 16), (u[2][e] & 0xFFFFu) | (u[3][e] << 16));
-                const uint2 hi2 = make_uint2((u[0][e] >> 16) | (u[1][e] & 0xFFFF0000u), (u[2][e] >> 16) | (u[3][e] & 0xFFFF0000u));
-                *(uint2 *) (Vt + (8 * c8 + 2 * e) * VS + 4 * cg) = lo2;
-                *(uint2 *) (Vt + (8 * c8 + 2 * e + 1) * VS + 4 * cg) = hi2;
+                const int64_t j = j0 + 4 * cg + cc;
+                if constexpr (PLAIN) vn[r][cc] = *(const uint4 *) (vbase + std::min<int64_t>(j, n_kv - 1) * v.nb[1] + c8 * 16);
+                else {
+                    vn[r][cc] = make_uint4(0, 0, 0, 0);
+                    if (8 * c8 < DV) vn[r][cc] = *(const uint4 *) (vbase + std::min<int64_t>(j, n_kv - 1) * v.nb[1] + c8 * 16);
+                }
             }
         }
-        __syncthreads();
-        if (!wave_any) continue;  // (wave-uniform; no barrier follows inside this iteration)
+        load_mask(blk, mv_next);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    int blk = next_block(0);
+    if (blk < n_blk) fetch(blk);
+    for (int it = 0; blk < n_blk; ++it) {
+        uint16_t * const Vt = Vt2[it & 1];
+        const int64_t j0 = (int64_t) blk * 32;
+        const bool tail = j0 + 32 > n_kv;  // (cells past the end: weight 0 and value 0 — a value read for them may be anything)
+#pragma unroll
+        for (int r = 0; r < NV; ++r) {
+            const int e0 = threadIdx.x + r * blockDim.x, cg = e0 / (DVT * 4), c8 = e0 % (DVT * 4);
+            if (cg < 8) {  // eight 8-byte groups: 4 cells of one entry
+                uint32_t u[4][4] = {{vn[r][0].x, vn[r][0].y, vn[r][0].z, vn[r][0].w}, {vn[r][1].x, vn[r][1].y, vn[r][1].z, vn[r][1].w},
+                                    {vn[r][2].x, vn[r][2].y, vn[r][2].z, vn[r][2].w}, {vn[r][3].x, vn[r][3].y, vn[r][3].z, vn[r][3].w}};
+                if (tail) {
+#pragma unroll
+                    for (int cc = 0; cc < 4; ++cc)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) u[cc][e] = j0 + 4 * cg + cc < n_kv ? u[cc][e] : 0u;
+                }
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    // entries 2 e (low halves) and 2 e + 1 (high halves) of the four cells
+                    const uint2 lo2 = make_uint2(__builtin_amdgcn_perm(u[1][e], u[0][e], 0x05040100u), __builtin_amdgcn_perm(u[3][e], u[2][e], 0x05040100u));
+                    const uint2 hi2 = make_uint2(__builtin_amdgcn_perm(u[1][e], u[0][e], 0x07060302u), __builtin_amdgcn_perm(u[3][e], u[2][e], 0x07060302u));
+                    *(uint2 *) (Vt + (8 * c8 + 2 * e) * VS + 4 * cg) = lo2;
+                    *(uint2 *) (Vt + (8 * c8 + 2 * e + 1) * VS + 4 * cg) = hi2;
+                }
+            }
+        }
+        float mv[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) mv[i] = q_live ? mv_next[i] : -INFINITY;
+        const bool wave_any = seen(mv);
+        __syncthreads();  // V^T of this block is staged; nobody reads the other copy any more
         att_f16v S;
 #pragma unroll
         for (int i = 0; i < 16; ++i) S[i] = 0.0f;
+        if (wave_any) {
 #pragma unroll
-        for (int s = 0; s < DK16; ++s) S = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(att_bf8, kf[s]), __builtin_bit_cast(att_bf8, qf[s]), S, 0, 0, 0);
+            for (int s = 0; s < DK16; ++s) S = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(att_bf8, kn[s]), __builtin_bit_cast(att_bf8, qf[s]), S, 0, 0, 0);
+        }
+        blk = next_block(blk + 1);
+        if (blk < n_blk) fetch(blk);
+        if (!wave_any) continue;
         float mx = ATTN_F32_LOW;
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-            S[i] = mv[i] > -INFINITY ? attn_score(S[i], scale, s_temp, softcap) + mask_term(mv[i], pen, r1, r2) : -INFINITY;
+            if constexpr (PLAIN) S[i] = mv[i] > -INFINITY ? S[i] * scale + mv[i] : -INFINITY;
+            else S[i] = mv[i] > -INFINITY ? attn_score(S[i], scale, s_temp, softcap) + mask_term(mv[i], pen, r1, r2) : -INFINITY;
             mx = fmaxf(mx, S[i]);
         }
         mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
@@ -512,32 +575,41 @@ __global__ void __launch_bounds__(256) k_attn_mma_bf16(const tdesc q, const tdes
         uint32_t hi[8], lo[8];
 #pragma unroll
         for (int i = 0; i < 16; i += 2) {
-            const float p0 = sgm ? (S[i] > -INFINITY ? attn_sigmoid(S[i] + s_bias) : 0.0f) : expf(S[i] - m_new);
-            const float p1 = sgm ? (S[i + 1] > -INFINITY ? attn_sigmoid(S[i + 1] + s_bias) : 0.0f) : expf(S[i + 1] - m_new);
+            float p0, p1;
+            if constexpr (PLAIN) { p0 = expf(S[i] - m_new); p1 = expf(S[i + 1] - m_new); }
+            else {
+                p0 = sgm ? (S[i] > -INFINITY ? attn_sigmoid(S[i] + s_bias) : 0.0f) : expf(S[i] - m_new);
+                p1 = sgm ? (S[i + 1] > -INFINITY ? attn_sigmoid(S[i + 1] + s_bias) : 0.0f) : expf(S[i + 1] - m_new);
+            }
             ps += p0 + p1;
-            const uint32_t h0 = att_bf16_bits(p0), h1 = att_bf16_bits(p1);
-            hi[i >> 1] = h0 | (h1 << 16);
-            lo[i >> 1] = att_bf16_bits(p0 - __uint_as_float(h0 << 16)) | (att_bf16_bits(p1 - __uint_as_float(h1 << 16)) << 16);
+            const uint32_t h2 = att_bf16_pack(p0, p1);
+            hi[i >> 1] = h2;
+            lo[i >> 1] = att_bf16_pack(p0 - __uint_as_float(h2 << 16), p1 - __uint_as_float(h2 & 0xFFFF0000u));
         }
         ps += __shfl_xor(ps, 32, 64);
         l = l * corr + ps;
         m = m_new;
+        if (__ballot(corr != 1.0f) != 0) {  // (a running maximum that stays rescales by 1)
 #pragma unroll
-        for (int dt = 0; dt < DVT; ++dt)
+            for (int dt = 0; dt < DVT; ++dt)
 #pragma unroll
-            for (int i = 0; i < 16; ++i) O[dt][i] *= corr;
+                for (int i = 0; i < 16; ++i) O[dt][i] *= corr;
+        }
 #pragma unroll
         for (int s2 = 0; s2 < 2; ++s2) {
             const uint4 ph = make_uint4(hi[4 * s2], hi[4 * s2 + 1], hi[4 * s2 + 2], hi[4 * s2 + 3]);
             const uint4 pl = make_uint4(lo[4 * s2], lo[4 * s2 + 1], lo[4 * s2 + 2], lo[4 * s2 + 3]);
+            uint4 vf[DVT];
 #pragma unroll
             for (int dt = 0; dt < DVT; ++dt) {
                 const uint16_t * vr = Vt + (32 * dt + n) * VS + 16 * s2 + 4 * g;
                 const uint2 a0 = *(const uint2 *) vr, a1 = *(const uint2 *) (vr + 8);
-                const uint4 vf = make_uint4(a0.x, a0.y, a1.x, a1.y);
-                O[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(att_bf8, vf), __builtin_bit_cast(att_bf8, ph), O[dt], 0, 0, 0);
-                O[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(att_bf8, vf), __builtin_bit_cast(att_bf8, pl), O[dt], 0, 0, 0);
+                vf[dt] = make_uint4(a0.x, a0.y, a1.x, a1.y);
             }
+#pragma unroll
+            for (int dt = 0; dt < DVT; ++dt) O[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(att_bf8, vf[dt]), __builtin_bit_cast(att_bf8, ph), O[dt], 0, 0, 0);
+#pragma unroll
+            for (int dt = 0; dt < DVT; ++dt) O[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(att_bf8, vf[dt]), __builtin_bit_cast(att_bf8, pl), O[dt], 0, 0, 0);
         }
     }
     if (!q_live) return;
@@ -548,7 +620,7 @@ __global__ void __launch_bounds__(256) k_attn_mma_bf16(const tdesc q, const tdes
 #pragma unroll
         for (int b = 0; b < 4; ++b) {
             const int d0 = 32 * dt + 8 * b + 4 * g;
-            if (d0 + 3 < DV) *(float4 *) (out + d0) = make_float4(O[dt][4 * b] * inv, O[dt][4 * b + 1] * inv, O[dt][4 * b + 2] * inv, O[dt][4 * b + 3] * inv);
+            if (PLAIN || d0 + 3 < DV) *(float4 *) (out + d0) = make_float4(O[dt][4 * b] * inv, O[dt][4 * b + 1] * inv, O[dt][4 * b + 2] * inv, O[dt][4 * b + 3] * inv);
             else
                 for (int r = 0; r < 4; ++r) if (d0 + r < DV) out[d0 + r] = O[dt][4 * b + r] * inv;
         }
@@ -803,7 +875,12 @@ static void attn_f32_launch_t(hipStream_t s, const tdesc & q, const tdesc & k, c
             const dim3 grid((unsigned) ((n_q + 32 * nw - 1) / (32 * nw)), (unsigned) H);
             const dim3 block((unsigned) (64 * nw));
             const int dk16 = (DK + 15) / 16, dvt = (DV + 31) / 32;
-#define MI_ATT_MMA(A, B) hipLaunchKernelGGL((k_attn_mma_bf16<A, B>), grid, block, 0, s, q, k, v, *mask, sinks, r12, dst, scale, sig, softcap, pen_kind)
+            const bool plain = !sig && !r12 && softcap <= 0.0f && DK == 16 * dk16 && DV == 32 * dvt;
+#define MI_ATT_MMA2(A, B, P) do { \
+                if (B >= 3 && nw == 1) hipLaunchKernelGGL((k_attn_mma_bf16<A, B, B >= 3 ? 2 : 1, P>), grid, block, 0, s, q, k, v, *mask, sinks, r12, dst, scale, sig, softcap, pen_kind); \
+                else hipLaunchKernelGGL((k_attn_mma_bf16<A, B, 1, P>), grid, block, 0, s, q, k, v, *mask, sinks, r12, dst, scale, sig, softcap, pen_kind); \
+            } while (0)
+#define MI_ATT_MMA(A, B) do { if (plain && dk16 == A && dvt == B) MI_ATT_MMA2(A, B, true); else MI_ATT_MMA2(A, B, false); } while (0)
             const int a = dk16 <= 2 ? 2 : (dk16 <= 4 ? 4 : (dk16 <= 6 ? 6 : 8)), b = dvt <= 1 ? 1 : (dvt <= 2 ? 2 : (dvt <= 3 ? 3 : 4));
             if (a == 2 && b == 1) MI_ATT_MMA(2, 1); else if (a == 2 && b == 2) MI_ATT_MMA(2, 2); else if (a == 2) MI_ATT_MMA(2, 4);
             else if (a == 6 && b == 3) MI_ATT_MMA(6, 3);
@@ -814,6 +891,7 @@ static void attn_f32_launch_t(hipStream_t s, const tdesc & q, const tdesc & k, c
             else if (a == 4 && b == 1) MI_ATT_MMA(4, 1); else if (a == 4 && b == 2) MI_ATT_MMA(4, 2); else if (a == 4) MI_ATT_MMA(4, 4);
             else if (b == 1) MI_ATT_MMA(8, 1); else if (b == 2) MI_ATT_MMA(8, 2); else MI_ATT_MMA(8, 4);
 #undef MI_ATT_MMA
+#undef MI_ATT_MMA2
             return;
         }
     }
