@@ -23,6 +23,9 @@
 //     /root/reference/llama.cpp/ggml/src/ggml-cpu/quants.c), exact in int32.
 //   * mins (Q4_K / Q5_K) and the -32 offset of Q6_K are sum_j m_j * bsum_j over the activation block's 16-value sums — one
 //     f16 MFMA per unit on the f16 bsums the quantisers store (exact: |.| < 2^24), as in mmq_i8.hip.
+//   * the columns come in TQ groups of eight (1, 2 or 4: launch_skinny_tq): a launch fetches, folds and sums the accumulators of whole groups only.  With 32
+//     columns' worth of work on every launch a step of 3 columns cost what one of 32 does; now (MI355X, us a launch, 3 / 9 / 32 columns; the first figure is
+//     the same launch before): gate/up 28672 x 4096 Q4_K 21.9 -> 18.7 / 20.6 / 22.6, 4096 x 14336 Q6_K 18.8 -> 16.4 / 17.4 / 21.5, wq + wk + wv (Q4_K, Q6_K) 15.4 -> 12.4 / 13.1 / 16.1.
 //   * Q6_K blocks are 210 bytes at 2-byte alignment: the unit is fetched as 4-byte-aligned 16-byte pieces (dwordx4 only needs
 //     dword alignment) and shifted by 0 / 2 bytes on the way into LDS (v_alignbyte + the neighbour lane's first dword).
 // Forms in this file: the K-parallel kernel above for any shape (k_mmq_skinny<QA, QB, EPI>; QA != QB: matrices of two formats in one
@@ -49,11 +52,12 @@ typedef uint32_t u32x2s __attribute__((ext_vector_type(2)));
 constexpr int SK_NW = 8;            // waves per workgroup
 constexpr int SK_BTOK = 304;        // LDS bytes per token of the activation unit: 256 qs + 32 bsums (f16) + 16 pad (76 dwords = 4 * 19)
 constexpr int SK_B_BYTES = 32 * SK_BTOK;
+template <int TQ> constexpr int sk_b_bytes() { return 8 * TQ * SK_BTOK; }  // ... of TQ groups of eight tokens
 template <int QT> struct sk_fmt;
 template <> struct sk_fmt<4> { static constexpr int BYTES = 144, PIECES = 9, ROW = 144; };   // 36 dwords = 4 * 9
 template <> struct sk_fmt<5> { static constexpr int BYTES = 176, PIECES = 11, ROW = 176; };  // 44 dwords = 4 * 11
 template <> struct sk_fmt<6> { static constexpr int BYTES = 210, PIECES = 14, ROW = 240; };  // 14 pieces + 16 pad: 60 dwords = 4 * 15
-template <int QT> constexpr int sk_wave_lds() { return 32 * sk_fmt<QT>::ROW + SK_B_BYTES + 128; }
+template <int QT, int TQ> constexpr int sk_wave_lds() { return 32 * sk_fmt<QT>::ROW + sk_b_bytes<TQ>() + 128; }
 
 __device__ __forceinline__ uint32_t sk_pack_h2(const float a, const float b) {
     typedef _Float16 half2s __attribute__((ext_vector_type(2)));
@@ -79,7 +83,10 @@ template <int K> __device__ __forceinline__ uint32_t sk_rep_byte(const uint32_t 
 // q <= 15, digits <= 7, products <= 105) or 16 s2 + 4 s1 + s0 (Q5_K: q <= 31, digits <= 3, products <= 93), one int8 weight operand per
 // digit (four nibbles x digit = ONE v_pk_mul_lo_u16), and the digit planes accumulate over all eight sub-blocks INSIDE the matrix
 // cores (C operand): sum_j sc_j (q . y)_j = 8 P1 + P0, the same integers ggml-cpu computes, with no per-sub-block fold at all.
-template <int QT> __device__ __forceinline__ void sk_unit_k45(const char * __restrict__ arow, const char * __restrict__ btok, const float * __restrict__ dAs, const int g, float (&acc)[16]) {
+// Up to eight columns (TQ = 1) only four of the sixteen accumulators are wanted: there the fold is 32 v_mad_i32_i24 against 64 (Q5_K: 96) digit products and
+// twice the MFMAs, and the plain nibbles go to the matrix cores; from nine columns on both forms take the same time and the digits stay.
+template <int QT, int TQ> __device__ __forceinline__ void sk_unit_k45(const char * __restrict__ arow, const char * __restrict__ btok, const float * __restrict__ dAs, const int g, float (&acc)[4 * TQ]) {
+    constexpr bool DIGITS = TQ > 1;
     constexpr int NP = QT == 4 ? 2 : 3;              // digit planes
     constexpr uint32_t DM = QT == 4 ? 0x07070707u : 0x03030303u;
     constexpr int DS = QT == 4 ? 3 : 2;              // bits per digit
@@ -115,6 +122,7 @@ template <int QT> __device__ __forceinline__ void sk_unit_k45(const char * __res
     uint4 qh = make_uint4(0, 0, 0, 0);
     if constexpr (QT == 5) qh = *(const uint4 *) (arow + 16 + 16 * g);
     int16s pl[NP];
+    int fold[4 * TQ] = {};
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
         const uint4 raw = *(const uint4 *) (arow + (QT == 5 ? 48 : 16) + 32 * p + 16 * g);
@@ -130,6 +138,15 @@ template <int QT> __device__ __forceinline__ void sk_unit_k45(const char * __res
         }
         const int4s y0 = *(const int4s *) (btok + 64 * p + 16 * g);
         const int4s y1 = *(const int4s *) (btok + 64 * p + 32 + 16 * g);
+        if constexpr (!DIGITS) {
+            const uint32_t src = p < 2 ? slo : shi;
+            const int s0 = (int) ((src >> (16 * (p & 1))) & 0xFF), s1 = (int) ((src >> (16 * (p & 1) + 8)) & 0xFF);
+            const int4s a0 = {(int) wlo[0], (int) wlo[1], (int) wlo[2], (int) wlo[3]}, a1 = {(int) whi[0], (int) whi[1], (int) whi[2], (int) whi[3]};
+            const int16s t0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(y0, a0, zeroi, 0, 0, 0);
+            const int16s t1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(y1, a1, zeroi, 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < 4 * TQ; ++i) fold[i] += __mul24(t0[i], s0) + __mul24(t1[i], s1);
+        } else
 #pragma unroll
         for (int n = 0; n < NP; ++n) {
             // sub-blocks 2p (low nibbles) and 2p + 1 (high nibbles): their digit n, replicated into both 16-bit lanes
@@ -147,14 +164,15 @@ template <int QT> __device__ __forceinline__ void sk_unit_k45(const char * __res
     }
     // ---- fold the unit
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
+    for (int q = 0; q < TQ; ++q) {
         const float4 dy = *(const float4 *) (dAs + 8 * q + 4 * g);
         const float dyv[4] = {dy.x, dy.y, dy.z, dy.w};
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int i = 4 * q + r;
             int isum;
-            if constexpr (QT == 4) isum = (pl[1][i] << 3) + pl[0][i];
+            if constexpr (!DIGITS) isum = fold[i];
+            else if constexpr (QT == 4) isum = (pl[1][i] << 3) + pl[0][i];
             else isum = (pl[2][i] << 4) + (pl[1][i] << 2) + pl[0][i];
             const float v = __builtin_fmaf(-dmin, ms[i], d * (float) isum);
             acc[i] = __builtin_fmaf(dyv[r], v, acc[i]);
@@ -169,7 +187,7 @@ template <int QT> __device__ __forceinline__ void sk_unit_k45(const char * __res
 // this pass serves the items whose matrix is stored as QT and walks past the others (k_mmq_skinny_mix runs one pass per format)
 // (the pass is a lambda INSIDE the kernel: as a device function taking the argument block, by value or by reference, it made the compiler
 // copy the block into scratch memory — 408 bytes per lane — and read every pointer of the launch from there)
-template <int QA, int QB, bool EPI>
+template <int QA, int QB, bool EPI, int TQ, bool TILE = false>
 __global__ void __launch_bounds__(SK_NW * 64, 1) k_mmq_skinny(const mmq8_args a) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     constexpr bool MIXED = QA != QB;
@@ -187,9 +205,9 @@ __global__ void __launch_bounds__(SK_NW * 64, 1) k_mmq_skinny(const mmq8_args a)
     // the row stride is the same for every matrix of one format (checked by the launcher)
     const int w_nb1 = !MIXED || a.mat[0].qt == QT ? (int) a.mat[0].w_nb1 : (a.mat[1].qt == QT ? (int) a.mat[1].w_nb1 : (int) a.mat[2].w_nb1);
 
-    char * const As = smem + wave * sk_wave_lds<QT>();
+    char * const As = smem + wave * sk_wave_lds<QT, TQ>();
     char * const Bs = As + 32 * F::ROW;
-    float * const dAs = (float *) (Bs + SK_B_BYTES);
+    float * const dAs = (float *) (Bs + sk_b_bytes<TQ>());
 
     // ---- fetch roles.  Every offset is linear in the fetch index u, so a handful of registers address the whole unit:
     //   weights, last 8 pieces of a row (Q4_K / Q5_K: the 128 qs bytes): u = 0..3, row = (lane >> 3) + 8 u, piece = HEAD + (lane & 7)
@@ -250,27 +268,28 @@ __global__ void __launch_bounds__(SK_NW * 64, 1) k_mmq_skinny(const mmq8_args a)
         _Pragma("unroll") for (int u = 0; u < NLT; ++u) ga[u] = *(const u32x4s *) (wb + at_off + u * at_step);          \
         _Pragma("unroll") for (int u = 0; u < NLH; ++u) ga[NLT + u] = *(const u32x4s *) (wb + ah_off[u]);               \
         const char * ab = act_base + (size_t) (sb) * sizeof(q8k_dev);                                                   \
-        _Pragma("unroll") for (int u = 0; u < 8; ++u)                                                                   \
-            if (4 * u < a.M) gb[u] = *(const u32x4s *) (ab + bq_off + u * bq_step); /* tokens 4u .. 4u+3: skipped beyond M */ \
-        gb[8] = *(const u32x4s *) (ab + bs_off);                                                                        \
+        _Pragma("unroll") for (int u = 0; u < 2 * TQ; ++u)                                                              \
+            if (TQ < 4 || 4 * u < a.M) gb[u] = *(const u32x4s *) (ab + bq_off + u * bq_step); /* tokens 4u .. 4u+3: skipped beyond M */ \
+        if (TQ == 4 || lane < 16 * TQ) gb[8] = *(const u32x4s *) (ab + bs_off);                                         \
         gd = *(const float *) (ab + d_off);                                                                             \
     }
     // the unit whose loads are in flight: (nx_item, nx_sb); wave w takes super-blocks lo + w, lo + w + 8, .. of every item
-    int nx_item = blockIdx.x, nx_sb = 0;
+    const int first = TILE ? (int) blockIdx.x * SK_NW + wave : (int) blockIdx.x, stride = TILE ? (int) gridDim.x * SK_NW : (int) gridDim.x;
+    int nx_item = first, nx_sb = 0;
 #define SK_NORMALISE()                                                                 \
     while (nx_item < n_items && (nx_sb >= item_hi(nx_item) || !mine(nx_item))) {       \
-        nx_item += gridDim.x;                                                          \
-        if (nx_item < n_items) nx_sb = item_lo(nx_item) + wave;                        \
+        nx_item += stride;                                                             \
+        if (nx_item < n_items) nx_sb = item_lo(nx_item) + (TILE ? 0 : wave);           \
     }
-    if (nx_item < n_items) nx_sb = item_lo(nx_item) + wave;
+    if (nx_item < n_items) nx_sb = item_lo(nx_item) + (TILE ? 0 : wave);
     SK_NORMALISE()
     if (nx_item < n_items) SK_ISSUE(item_rows(nx_item), nx_sb)
 
-    for (int item = blockIdx.x; item < n_items; item += gridDim.x) {
+    for (int item = first; item < n_items; item += stride) {
         if (!mine(item)) continue;
-        float acc[16];
+        float acc[4 * TQ];
 #pragma unroll
-        for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
+        for (int i = 0; i < 4 * TQ; ++i) acc[i] = 0.0f;
         while (nx_item == item) {
             const int sb = nx_sb;
             // ---- registers -> the wave's LDS area
@@ -294,23 +313,23 @@ __global__ void __launch_bounds__(SK_NW * 64, 1) k_mmq_skinny(const mmq8_args a)
                     if (u + 1 < NLH || ah_last_live) *(u32x4s *) (As + ah_lds[u]) = ga[NLT + u];
             }
 #pragma unroll
-            for (int u = 0; u < 8; ++u)
-                if (4 * u < a.M) *(u32x4s *) (Bs + bq_lds + u * 4 * SK_BTOK) = gb[u];
-            *(u32x4s *) (Bs + bs_lds) = gb[8];
+            for (int u = 0; u < 2 * TQ; ++u)
+                if (TQ < 4 || 4 * u < a.M) *(u32x4s *) (Bs + bq_lds + u * 4 * SK_BTOK) = gb[u];
+            if (TQ == 4 || lane < 16 * TQ) *(u32x4s *) (Bs + bs_lds) = gb[8];
             if (g == 0) dAs[row] = gd;
             // ---- the next unit's loads (of this item or of the workgroup's next one) fly while this one is multiplied
-            nx_sb += SK_NW;
+            nx_sb += TILE ? 1 : SK_NW;
             SK_NORMALISE()
             if (nx_item < n_items) SK_ISSUE(item_rows(nx_item), nx_sb)
 
             const char * const arow = As + row * F::ROW;   // this lane's weight row (B operand: n = row)
-            const char * const btok = Bs + row * SK_BTOK;  // this lane's token (A operand: m = token)
+            const char * const btok = Bs + (row & (8 * TQ - 1)) * SK_BTOK;  // this lane's token (A operand: m = token; the operand rows beyond 8 TQ repeat, their results are not used)
             if constexpr (QT == 4 || QT == 5) {
-                sk_unit_k45<QT>(arow, btok, dAs, g, acc);
+                sk_unit_k45<QT, TQ>(arow, btok, dAs, g, acc);
             } else {
                 // (the fold stays on v_mad_i32_i24 here although it issues at ~6.8 clocks (scripts/ubench/valu_probe.hip): the fp32 form of it —
                 // cvt + fma, 2 clocks each — was built and made the compiler park the prefetched unit in scratch (156 bytes per lane))
-                int16s isum = zeroi;
+                int isum[4 * TQ] = {};
                 float16s ms;
                 float d;
                 const uint4 scb = *(const uint4 *) (arow + 192);
@@ -342,8 +361,9 @@ __global__ void __launch_bounds__(SK_NW * 64, 1) k_mmq_skinny(const mmq8_args a)
                             const int2s y = *(const int2s *) (btok + 16 * s + 8 * g);
                             const int16s tk = __builtin_amdgcn_mfma_i32_32x32x16_i8(__builtin_bit_cast(long, y), __builtin_bit_cast(long, v[k]), zeroi, 0, 0, 0);
 #pragma unroll
-                            for (int i = 0; i < 16; ++i) isum[i] += __mul24(tk[i], sc[s]);
+                            for (int i = 0; i < 4 * TQ; ++i) isum[i] += __mul24(tk[i], sc[s]);
                         }
+
                     }
                 // the codes are q + 32: subtract 32 * sum_s sc_s * bsum_s (one f16 MFMA, exact integers)
                 const half8s bsf = *(const half8s *) (btok + 256 + 16 * g);
@@ -355,7 +375,7 @@ __global__ void __launch_bounds__(SK_NW * 64, 1) k_mmq_skinny(const mmq8_args a)
                 ms = __builtin_amdgcn_mfma_f32_32x32x16_f16(bsf, __builtin_bit_cast(half8s, sfu), zerof, 0, 0, 0);
                 // fold the unit: tokens of register i are (i & 3) + 8 (i >> 2) + 4 g
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
+                for (int q = 0; q < TQ; ++q) {
                     const float4 dy = *(const float4 *) (dAs + 8 * q + 4 * g);
                     const float dyv[4] = {dy.x, dy.y, dy.z, dy.w};
 #pragma unroll
@@ -368,11 +388,28 @@ __global__ void __launch_bounds__(SK_NW * 64, 1) k_mmq_skinny(const mmq8_args a)
             }
         }
 
+        if constexpr (TILE) {  // the wave has the whole of K: lane = weight row, register i = token (i & 3) + 8 (i >> 2) + 4 g
+            const int mi = MAT_OF(item), n = (item - MAT_SEL(mi, panel0)) * 32 + row;
+            float * const m_dst = MAT_SEL(mi, dst);
+            const int64_t m_dst_stride = MAT_SEL(mi, dst_stride);
+            const float * const m_add = MAT_SEL(mi, add);
+            const int64_t m_add_stride = MAT_SEL(mi, add_stride);
+            if (m_add) {
+#pragma unroll
+                for (int i = 0; i < 4 * TQ; ++i) acc[i] += m_add[(size_t) min((i & 3) + 8 * (i >> 2) + 4 * g, a.M - 1) * m_add_stride + n];
+            }
+#pragma unroll
+            for (int i = 0; i < 4 * TQ; ++i) {
+                const int tok = (i & 3) + 8 * (i >> 2) + 4 * g;
+                if (tok < a.M) m_dst[(size_t) tok * m_dst_stride + n] = acc[i];
+            }
+            continue;
+        }
         // ---- the eight K slices of the tile meet in LDS: each wave leaves its 32 x 32 partial [token][row] at the start of its
         // own area (no other wave touches that), then every thread sums two outputs over the waves in a fixed order
         float * const own = (float *) As;
 #pragma unroll
-        for (int i = 0; i < 16; ++i) own[((i & 3) + 8 * (i >> 2) + 4 * g) * 32 + row] = acc[i];
+        for (int i = 0; i < 4 * TQ; ++i) own[((i & 3) + 8 * (i >> 2) + 4 * g) * 32 + row] = acc[i];
         __syncthreads();
         const int tile = item >> ksl, ky = item & (a.ksplit - 1), mi = MAT_OF(tile);
         const int mN = MAT_SEL(mi, N);
@@ -383,12 +420,12 @@ __global__ void __launch_bounds__(SK_NW * 64, 1) k_mmq_skinny(const mmq8_args a)
         const float * const m_add = MAT_SEL(mi, add);
         const int64_t m_add_stride = MAT_SEL(mi, add_stride);
 #pragma unroll
-        for (int q = 0; q < 1024 / (SK_NW * 64); ++q) {
+        for (int q = 0; q < (256 * TQ + SK_NW * 64 - 1) / (SK_NW * 64); ++q) {
             const int o = tid + q * SK_NW * 64;
             const int tok = o >> 5, n = n0 + (o & 31);
             float v = *(const float *) (smem + o * 4);
 #pragma unroll
-            for (int w = 1; w < SK_NW; ++w) v += *(const float *) (smem + w * sk_wave_lds<QT>() + o * 4);
+            for (int w = 1; w < SK_NW; ++w) v += *(const float *) (smem + w * sk_wave_lds<QT, TQ>() + o * 4);
             if (a.ksplit > 1) {
                 if (tok < a.M) m_part[((size_t) ky * a.M + tok) * mN + n] = v;
                 continue;
@@ -543,7 +580,7 @@ __global__ void __launch_bounds__(TP_NW * 64, 2) k_mmq_skinny_tp(const mmq8_args
         __syncthreads();                                    // ... everybody's have, and nobody reads step s - 1 any more
         if (s + TP_NS - 1 < total) TP_ISSUE_NEXT()
         const int slot = s % TP_NS;
-        sk_unit_k45<QT>(a_ring_p + slot * tp_a_stage<QT>() + row * F::ROW, smem + slot * SK_B_BYTES + row * SK_BTOK, (const float *) (smem + TP_NS * SK_B_BYTES + slot * 128), g, acc);
+        sk_unit_k45<QT, 4>(a_ring_p + slot * tp_a_stage<QT>() + row * F::ROW, smem + slot * SK_B_BYTES + row * SK_BTOK, (const float *) (smem + TP_NS * SK_B_BYTES + slot * 128), g, acc);
         if (++cu_sb == nblk) {
             // ---- the tile is complete: lane = weight row, register i = token (i & 3) + 8 (i >> 2) + 4 g
             const int mi = MAT_OF(cu_item);
@@ -582,18 +619,17 @@ __global__ void __launch_bounds__(TP_NW * 64, 2) k_mmq_skinny_tp(const mmq8_args
 // weights 8 waves x 3 stages x 4.5 KB + activations 2 stages x 2 blocks x 9.5 KB = 146.5 KB — the activations (L2 hits) run one step
 // ahead, the weights two.  The halves of a tile meet once, at the end: wave t + 4 leaves its sums in the weight stage it consumed last.
 // (Q5_K's 5.5 KB units do not fit that way: it stays on the four-wave form.)
-constexpr int TP8_NW = 8, TP8_NSA = 3, TP8_NSB = 2;
-constexpr int TP8_B_STAGE = 2 * SK_B_BYTES, TP8_D_STAGE = 256;
-template <int QT> constexpr int tp8_lds_bytes() { return TP8_NSB * (TP8_B_STAGE + TP8_D_STAGE) + TP8_NW * TP8_NSA * tp_a_stage<QT>(); }
+constexpr int TP8_NW = 8, TP8_NSA = 3, TP8_NSB = 2, TP8_D_STAGE = 256;
+template <int QT, int TQ> constexpr int tp8_lds_bytes() { return TP8_NSB * (2 * sk_b_bytes<TQ>() + TP8_D_STAGE) + TP8_NW * TP8_NSA * tp_a_stage<QT>(); }
 
-template <int QT>
+template <int QT, int TQ>
 __global__ void __launch_bounds__(TP8_NW * 64, 1) k_mmq_skinny_tp8(const mmq8_args a) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     typedef sk_fmt<QT> F;
     constexpr int NPA = 32 * F::PIECES, NLA = (NPA + 63) / 64;  // weight pieces per unit and the wave-instructions fetching them
-    constexpr int NPB = 2 * 32 * 19 / TP8_NW;                    // activation pieces per wave and step: 152 = 2 x 64 + 24
-    constexpr int A_STAGE = tp_a_stage<QT>();
-    static_assert(tp8_lds_bytes<QT>() <= 160 * 1024, "LDS");
+    constexpr int NPB = 2 * 8 * TQ * 19 / TP8_NW, NLB = (NPB + 63) / 64;  // activation pieces per wave and step (32 tokens: 152 = 2 x 64 + 24) and the wave-instructions fetching them
+    constexpr int A_STAGE = tp_a_stage<QT>(), TP8_B_STAGE = 2 * sk_b_bytes<TQ>();
+    static_assert(tp8_lds_bytes<QT, TQ>() <= 160 * 1024, "LDS");
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int tile = wave & 3, kh = wave >> 2;  // this wave's tile of the group and its parity of super-blocks
     const int row = lane & 31, g = lane >> 5;
@@ -612,12 +648,12 @@ __global__ void __launch_bounds__(TP8_NW * 64, 1) k_mmq_skinny_tp8(const mmq8_ar
         const int pi = min(lane + 64 * u, NPA - 1);
         a_off[u] = (pi / F::PIECES) * w_nb1 + (pi % F::PIECES) * 16;
     }
-    // the stage's 1216 activation pieces in LDS order [block][token][19 pieces]; this wave requests 152 consecutive ones
-    int b_off[3];
+    // the stage's activation pieces (1216 of 32 tokens) in LDS order [block][token][19 pieces]; this wave requests NPB consecutive ones
+    int b_off[NLB];
 #pragma unroll
-    for (int u = 0; u < 3; ++u) {
+    for (int u = 0; u < NLB; ++u) {
         const int pi = wave * NPB + min(lane + 64 * u, NPB - 1);
-        const int blk = pi / 608, rem = pi - blk * 608;
+        const int blk = pi / (152 * TQ), rem = pi - blk * (152 * TQ);
         b_off[u] = (rem / 19) * tok_bytes + blk * (int) sizeof(q8k_dev) + (rem % 19) * 16;
     }
     const int d_off = row * tok_bytes + g * (int) sizeof(q8k_dev) + 304;  // q8k_dev::d of (block g, token row): 64 lanes
@@ -639,15 +675,15 @@ __global__ void __launch_bounds__(TP8_NW * 64, 1) k_mmq_skinny_tp8(const mmq8_ar
     auto issue_b = [&](const int j, const int slot) {
         const char * ab = (const char *) a.act + (size_t) (2 * j) * sizeof(q8k_dev);
         const uint32_t bl = b_ring + slot * TP8_B_STAGE + wave * NPB * 16;
-        tp_dma16(ab + b_off[0], bl);
-        tp_dma16(ab + b_off[1], bl + 1024);
-        if (lane < NPB - 128) tp_dma16(ab + b_off[2], bl + 2048);
+#pragma unroll
+        for (int u = 0; u < NLB; ++u)
+            if (u + 1 < NLB || (NPB % 64) == 0 || lane < (NPB % 64)) tp_dma16(ab + b_off[u], bl + u * 1024);
         tp_dma4(ab + d_off, d_ring + slot * TP8_D_STAGE);  // (every wave: identical bytes to the same place, and one wait count for all)
     };
 
-    float acc[16];
+    float acc[4 * TQ];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
+    for (int i = 0; i < 4 * TQ; ++i) acc[i] = 0.0f;
     // request cursors: weights run two steps ahead, activations one; queue order per step [activations s + 1, weights s + 2] — what
     // step s + 1 consumes is then older than the one thing that may still fly when it starts (in-order vmcnt)
     int ia_item = blockIdx.x, ia_j = 0, na = 0, sa = 0;  // next weight step to request (item, step of the item, running number, slot)
@@ -664,7 +700,7 @@ __global__ void __launch_bounds__(TP8_NW * 64, 1) k_mmq_skinny_tp8(const mmq8_ar
         __syncthreads();  // everything of step s is in LDS, and nobody reads step s - 1 any more
         if (nb < total) TP8_ISSUE_B()
         if (na < total) TP8_ISSUE_A()
-        sk_unit_k45<QT>(a_ring_p + ca * A_STAGE + row * F::ROW, smem + cb * TP8_B_STAGE + kh * SK_B_BYTES + row * SK_BTOK,
+        sk_unit_k45<QT, TQ>(a_ring_p + ca * A_STAGE + row * F::ROW, smem + cb * TP8_B_STAGE + kh * sk_b_bytes<TQ>() + (row & (8 * TQ - 1)) * SK_BTOK,
                         (const float *) (smem + TP8_NSB * TP8_B_STAGE + cb * TP8_D_STAGE + kh * 128), g, acc);
         if (++cu_j == nst) {
             // ---- the tile is complete: the odd half's sums cross over through the weight stage that wave has just consumed (its next
@@ -672,13 +708,13 @@ __global__ void __launch_bounds__(TP8_NW * 64, 1) k_mmq_skinny_tp8(const mmq8_ar
             if (kh) {
                 float * const own = (float *) (a_ring_p + ca * A_STAGE);
 #pragma unroll
-                for (int i = 0; i < 16; ++i) own[i * 64 + lane] = acc[i];
+                for (int i = 0; i < 4 * TQ; ++i) own[i * 64 + lane] = acc[i];
             }
             __syncthreads();
             if (!kh) {
                 const float * const other = (const float *) (a_ring_p + 4 * TP8_NSA * A_STAGE + ca * A_STAGE);
 #pragma unroll
-                for (int i = 0; i < 16; ++i) acc[i] += other[i * 64 + lane];
+                for (int i = 0; i < 4 * TQ; ++i) acc[i] += other[i * 64 + lane];
                 const int mi = MAT_OF(cu_item);
                 const int n = (cu_item - MAT_SEL(mi, panel0)) * 128 + tile * 32 + row;
                 float * const m_dst = MAT_SEL(mi, dst);
@@ -687,10 +723,10 @@ __global__ void __launch_bounds__(TP8_NW * 64, 1) k_mmq_skinny_tp8(const mmq8_ar
                 const int64_t m_add_stride = MAT_SEL(mi, add_stride);
                 if (m_add) {
 #pragma unroll
-                    for (int i = 0; i < 16; ++i) acc[i] += m_add[(size_t) min((i & 3) + 8 * (i >> 2) + 4 * g, a.M - 1) * m_add_stride + n];
+                    for (int i = 0; i < 4 * TQ; ++i) acc[i] += m_add[(size_t) min((i & 3) + 8 * (i >> 2) + 4 * g, a.M - 1) * m_add_stride + n];
                 }
 #pragma unroll
-                for (int i = 0; i < 16; ++i) {
+                for (int i = 0; i < 4 * TQ; ++i) {
                     const int tok = (i & 3) + 8 * (i >> 2) + 4 * g;
                     if (tok < a.M) m_dst[(size_t) tok * m_dst_stride + n] = acc[i];
                 }
@@ -699,7 +735,7 @@ __global__ void __launch_bounds__(TP8_NW * 64, 1) k_mmq_skinny_tp8(const mmq8_ar
                 if (s + 1 < total) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             }
 #pragma unroll
-            for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
+            for (int i = 0; i < 4 * TQ; ++i) acc[i] = 0.0f;
             cu_j = 0;
             cu_item += gridDim.x;
         }
@@ -1067,9 +1103,9 @@ bool mmq_skinny_supported(int type, int64_t K, int64_t N, int64_t M, int64_t w_n
     // rows packed back to back (then every matrix of a launch has the same row stride)
     if (type == GGML_TYPE_Q4_K) return w_nb1 == (K / 256) * 144;
     if (type == GGML_TYPE_Q5_K) return w_nb1 == (K / 256) * 176;
-    // (a Q6_K matrix of 64 k rows and more — the output matrix — stays on the tiled GEMM: 144 us against 170 us here for 128256 x 4096 at
-    // 32 columns, profiles/r03_np32_ab_q6_tiled.txt; this kernel's Q6_K unit is bound by its integer VALU, the tiled one converts once per 64 columns)
-    if (type == GGML_TYPE_Q6_K) return N < 65536 && w_nb1 == (K / 256) * 210 && (w_nb1 % 4) == 0;  // dword-aligned rows: the 0 / 2-byte shift of a super-block is the same in every row
+    // (a Q6_K matrix of 64 k rows and more — the output matrix — comes here with up to 16 columns only, in the one-wave-per-tile form: 128256 x 4096 takes 113 us
+    // at 3 columns against 135 us on the tiled GEMM; at 32 columns both take 148 us, and the tiled GEMM keeps them)
+    if (type == GGML_TYPE_Q6_K) return (N < 65536 || M <= 16) && w_nb1 == (K / 256) * 210 && (w_nb1 % 4) == 0;  // dword-aligned rows: the 0 / 2-byte shift of a super-block is the same in every row
     return false;
 }
 
@@ -1091,7 +1127,7 @@ static int skinny_n_cu() {
     return n_cu.load(std::memory_order_relaxed);
 }
 
-template <int QT> static void launch_skinny_t(hipStream_t s, mmq8_args a) {
+template <int QT, int TQ> static void launch_skinny_t(hipStream_t s, mmq8_args a) {
     const int n_cu = skinny_n_cu();
     a.m_tiles = 1;
     if constexpr (QT == 4 || QT == 5) {
@@ -1105,9 +1141,10 @@ template <int QT> static void launch_skinny_t(hipStream_t s, mmq8_args a) {
                 // two waves per tile (GGML_MI355X_SKINNY_TP=1: the four-wave form)
                 static const bool tp8 = !getenv("GGML_MI355X_SKINNY_TP") || atoi(getenv("GGML_MI355X_SKINNY_TP")) != 1;
                 if (tp8 && (a.K % 512) == 0) {
+                    constexpr size_t lds8 = (size_t) tp8_lds_bytes<QT, TQ>();
                     static std::atomic<uint32_t> lds_raised_tp8{0};
-                    (void) ensure_dyn_lds((const void *) k_mmq_skinny_tp8<QT>, (size_t) tp8_lds_bytes<QT>(), lds_raised_tp8);
-                    MI_LAUNCH_PROBED((k_mmq_skinny_tp8<QT>), dim3((unsigned) std::min(a.n_panels, n_cu)), dim3(TP8_NW * 64), (size_t) tp8_lds_bytes<QT>(), s, a);
+                    (void) ensure_dyn_lds((const void *) k_mmq_skinny_tp8<QT, TQ>, lds8, lds_raised_tp8);
+                    MI_LAUNCH_PROBED((k_mmq_skinny_tp8<QT, TQ>), dim3((unsigned) std::min(a.n_panels, n_cu)), dim3(TP8_NW * 64), lds8, s, a);
                     return;
                 }
             }
@@ -1117,26 +1154,35 @@ template <int QT> static void launch_skinny_t(hipStream_t s, mmq8_args a) {
             return;
         }
     }
-    const size_t lds = (size_t) SK_NW * sk_wave_lds<QT>();
+    const size_t lds = (size_t) SK_NW * sk_wave_lds<QT, TQ>();
     static std::atomic<uint32_t> lds_raised{0}, lds_raised_epi{0};
-    const void * fn_plain = (const void *) k_mmq_skinny<QT, QT, false>;
-    const void * fn_epi = (const void *) k_mmq_skinny<QT, QT, true>;
+    const void * fn_plain = (const void *) k_mmq_skinny<QT, QT, false, TQ>;
+    const void * fn_epi = (const void *) k_mmq_skinny<QT, QT, true, TQ>;
     (void) ensure_dyn_lds(a.has_epi ? fn_epi : fn_plain, lds, a.has_epi ? lds_raised_epi : lds_raised);
     a.n_panels = 0;
     for (int i = 0; i < a.n_mat; ++i) {
         a.mat[i].panel0 = a.n_panels;
         a.n_panels += a.mat[i].N / 32;
     }
+    if constexpr (QT == 6 && TQ < 4) {
+        // a tile per wave where that fills three quarters of the chip's wave slots: no barrier and no sum over the waves (135 us K-parallel, 113 us so: 128256 x 4096 x 3)
+        if (!a.has_epi && a.ksplit == 1 && a.n_panels >= 6 * n_cu) {
+            static std::atomic<uint32_t> lds_raised_tile{0};
+            (void) ensure_dyn_lds((const void *) k_mmq_skinny<QT, QT, false, TQ, true>, lds, lds_raised_tile);
+            MI_LAUNCH_PROBED((k_mmq_skinny<QT, QT, false, TQ, true>), dim3((unsigned) n_cu), dim3(SK_NW * 64), lds, s, a);
+            return;
+        }
+    }
     // one workgroup per CU (its LDS areas fill the CU), walking the (tile, K slice) items with a stride of the grid
     const int items = a.n_panels * a.ksplit;
-    if (a.has_epi) MI_LAUNCH_PROBED((k_mmq_skinny<QT, QT, true>), dim3((unsigned) std::min(items, n_cu)), dim3(SK_NW * 64), lds, s, a);
-    else MI_LAUNCH_PROBED((k_mmq_skinny<QT, QT, false>), dim3((unsigned) std::min(items, n_cu)), dim3(SK_NW * 64), lds, s, a);
+    if (a.has_epi) MI_LAUNCH_PROBED((k_mmq_skinny<QT, QT, true, TQ>), dim3((unsigned) std::min(items, n_cu)), dim3(SK_NW * 64), lds, s, a);
+    else MI_LAUNCH_PROBED((k_mmq_skinny<QT, QT, false, TQ>), dim3((unsigned) std::min(items, n_cu)), dim3(SK_NW * 64), lds, s, a);
 }
 
-template <int QA, int QB> static void launch_skinny_mix_t(hipStream_t s, mmq8_args a) {
-    constexpr size_t lds = (size_t) SK_NW * (size_t) std::max(sk_wave_lds<QA>(), sk_wave_lds<QB>());
+template <int QA, int QB, int TQ> static void launch_skinny_mix_t(hipStream_t s, mmq8_args a) {
+    constexpr size_t lds = (size_t) SK_NW * (size_t) std::max(sk_wave_lds<QA, TQ>(), sk_wave_lds<QB, TQ>());
     static std::atomic<uint32_t> lds_raised{0}, lds_raised_epi{0};
-    const void * fn = a.has_epi ? (const void *) k_mmq_skinny<QA, QB, true> : (const void *) k_mmq_skinny<QA, QB, false>;
+    const void * fn = a.has_epi ? (const void *) k_mmq_skinny<QA, QB, true, TQ> : (const void *) k_mmq_skinny<QA, QB, false, TQ>;
     (void) ensure_dyn_lds(fn, lds, a.has_epi ? lds_raised_epi : lds_raised);
     a.m_tiles = 1;
     a.n_panels = 0;
@@ -1145,8 +1191,18 @@ template <int QA, int QB> static void launch_skinny_mix_t(hipStream_t s, mmq8_ar
         a.n_panels += a.mat[i].N / 32;
     }
     const int items = a.n_panels * a.ksplit;
-    if (a.has_epi) MI_LAUNCH_PROBED((k_mmq_skinny<QA, QB, true>), dim3((unsigned) std::min(items, skinny_n_cu())), dim3(SK_NW * 64), lds, s, a);
-    else MI_LAUNCH_PROBED((k_mmq_skinny<QA, QB, false>), dim3((unsigned) std::min(items, skinny_n_cu())), dim3(SK_NW * 64), lds, s, a);
+    if (a.has_epi) MI_LAUNCH_PROBED((k_mmq_skinny<QA, QB, true, TQ>), dim3((unsigned) std::min(items, skinny_n_cu())), dim3(SK_NW * 64), lds, s, a);
+    else MI_LAUNCH_PROBED((k_mmq_skinny<QA, QB, false, TQ>), dim3((unsigned) std::min(items, skinny_n_cu())), dim3(SK_NW * 64), lds, s, a);
+}
+// the form for a's columns, in whole groups of eight
+template <int QA, int QB, int TQ> static void launch_skinny_one(hipStream_t s, const mmq8_args & a) {
+    if constexpr (QA == QB) launch_skinny_t<QA, TQ>(s, a);
+    else launch_skinny_mix_t<QA, QB, TQ>(s, a);
+}
+template <int QA, int QB> static void launch_skinny_tq(hipStream_t s, const mmq8_args & a) {
+    if (a.M <= 8) launch_skinny_one<QA, QB, 1>(s, a);
+    else if (a.M <= 16) launch_skinny_one<QA, QB, 2>(s, a);
+    else launch_skinny_one<QA, QB, 4>(s, a);
 }
 bool launch_mmq_skinny_mixed(hipStream_t s, const mmq8_args & a) {
     bool has[7] = {};
@@ -1154,15 +1210,15 @@ bool launch_mmq_skinny_mixed(hipStream_t s, const mmq8_args & a) {
         if (a.mat[i].qt < 4 || a.mat[i].qt > 6) return false;
         has[a.mat[i].qt] = true;
     }
-    if (has[4] && has[6] && !has[5]) { launch_skinny_mix_t<4, 6>(s, a); return true; }
-    if (has[5] && has[6] && !has[4]) { launch_skinny_mix_t<5, 6>(s, a); return true; }
+    if (has[4] && has[6] && !has[5]) { launch_skinny_tq<4, 6>(s, a); return true; }
+    if (has[5] && has[6] && !has[4]) { launch_skinny_tq<5, 6>(s, a); return true; }
     return false;
 }
 
 void launch_mmq_skinny(hipStream_t s, int type, const mmq8_args & a) {
-    if (type == GGML_TYPE_Q4_K) launch_skinny_t<4>(s, a);
-    else if (type == GGML_TYPE_Q5_K) launch_skinny_t<5>(s, a);
-    else launch_skinny_t<6>(s, a);
+    if (type == GGML_TYPE_Q4_K) launch_skinny_tq<4, 4>(s, a);
+    else if (type == GGML_TYPE_Q5_K) launch_skinny_tq<5, 5>(s, a);
+    else launch_skinny_tq<6, 6>(s, a);
 }
 
 MI_TU_TOUCH(mmq_skinny)

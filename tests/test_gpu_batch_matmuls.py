@@ -109,3 +109,26 @@ def test_experts_with_batches(backend, H, K, N, n_exp, top, T_):
     xr = round16(x, L.BF16).astype(np.float64)[:, 0]
     ref = np.stack([[w[ids[t, u]].astype(np.float64) @ xr[t] for u in range(top)] for t in range(T_)])
     assert np.abs(got - ref).max() <= 6e-8 * np.sqrt(K) * 8
+
+
+# every form of the small-batch kernel (K over the waves, with and without a K split; four tiles a workgroup; a tile per wave) and both sides of its groups of eight columns
+@pytest.mark.parametrize("qt,K,N", [(L.Q4_K, 2816, 96), (L.Q5_K, 2048, 64), (L.Q6_K, 4096, 160), (L.Q4_K, 1024, 24576), (L.Q6_K, 768, 49152), (L.Q6_K, 256, 70016)])
+def test_k_quant_batches_by_groups_of_eight_columns(backend, H, qt, K, N):
+    """mmq_skinny.hip: a column's bits do not depend on how many others there are (the integer sums are exact, the f32 sums in the same order), and match the oracle."""
+    rng = np.random.default_rng(K + N)
+    w = T.rand_weight(qt, K, N, rng)
+    x = (rng.standard_normal((32, K)) * rng.uniform(0.2, 3.0, (32, 1))).astype(np.float32)
+
+    def run(M, where, ww):
+        return T.run_case(lambda g: H.ggml_mul_mat(g.ctx, g.new(qt, [K, ww.shape[0]], ww), g.new(L.F32, [K, M], x[:M])), where)[0].reshape(M, -1)
+
+    rows = np.unique(np.concatenate([np.arange(min(N, 40)), np.arange(max(0, N - 40), N)]))
+    w = w.reshape(N, -1)
+    ref = run(32, "oracle", np.ascontiguousarray(w[rows]))
+    full = run(32 if N < 65536 else 16, backend, w)  # (65536 rows and up: 17 columns and more run on another kernel)
+    for M in (2, 3, 7, 8, 9, 15, 16, 17, 24):
+        if M > len(full) or (qt == L.Q5_K and M == 2):  # (two columns of Q5_K: the mat-vec)
+            continue
+        got = run(M, backend, w)
+        assert np.array_equal(got.view(np.uint32), full[:M].view(np.uint32)), M
+    assert T.nmse(full[:, rows], ref[: len(full)]) <= 1e-10
