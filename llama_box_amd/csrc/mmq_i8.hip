@@ -426,7 +426,7 @@ template <int QT, int BN, int BM = 128> static void launch_mmq8_t(hipStream_t s,
 int mmq_pick_ksplit(int64_t K, int64_t N, int64_t M, bool skinny, int type) {
     if (skinny && M >= 2 && M <= 32 && (N % 32) == 0) return mmq_skinny_ksplit(K, N);
     // prompt batches the wide form of mmq_skinny.hip serves run without a K split (its grid fills the chip by token-tile groups)
-    if (skinny && mmq_wide_tiles(type, K, &N, 1, M, (K / 256) * (type == GGML_TYPE_Q4_K ? 144 : 176), 1) != 0) return 1;
+    if (const int ks = skinny ? mmq_wide_ksplit(type, K, N, M) : 0) return ks;
     const int64_t wgs = ((N + 63) / 64) * ((M + 127) / 128), nblk = K / 256;
     static const int ks_target = getenv("GGML_MI355X_MMQ_KS_TARGET") ? atoi(getenv("GGML_MI355X_MMQ_KS_TARGET")) : 512;
     if (M <= 64) return (int) std::max<int64_t>(1, std::min<int64_t>(nblk, ks_target / std::max<int64_t>(1, wgs)));
@@ -546,7 +546,8 @@ int launch_mmq_i8_multi(hipStream_t s, int type, int n_mat, const mmq_mat_desc *
         const int tt = same ? mmq_wide_tiles(type, K, Ns, n_mat, M, mats[0].w_nb1, a.ksplit) : 0;
         if (tt) {
             launch_mmq_wide(s, type, tt, a);
-            return 2;
+            if (a.ksplit > 1 && reduce) launch_splitk_reduce_multi(s, a);
+            return mmq_wide_fills(type, panels128, M) ? 2 : 0;  // (the counters: a launch whose row groups and token tiles alone fill the chip, or a split one)
         }
     }
     skinny = skinny && (a.ksplit & (a.ksplit - 1)) == 0;  // (its K split is a power of two: mmq_skinny_ksplit)

@@ -766,11 +766,11 @@ static int skinny_n_cu();
 
 // ------------------------------------------------------------------------------------------------ wide form (prompt batches)
 // The same unit for 33 .. thousands of columns: a workgroup = NW computing waves = NW row tiles x TT token tiles (32 TT columns)
-// x the whole K range (+ loader waves, below).  Per step (super-block) a wave converts ITS weight unit once, in registers — nibbles x scale digits = the
+// x the whole K range or a slice of it (+ loader waves, below).  Per step (super-block) a wave converts ITS weight unit once, in registers — nibbles x scale digits = the
 // int8 B operands of all eight sub-blocks, 64 registers for Q4_K — and multiplies it with TT token tiles whose activations sit in
 // LDS exactly as the quantisers wrote them ([token][256 qs | bsums]: LDS-DMA, no conversion, no ds_write anywhere in the kernel).
 // mmq_i8.hip, which this replaces where it applies, stages both operands through registers into LDS every 128 values of K and
-// runs at 24 % of the matrix pipe with its components adding up serially (DESIGN.md: fragment reads 4.0, conversion + LDS writes
+// runs at 24 % of the matrix pipe with its components adding up serially (fragment reads 4.0, conversion + LDS writes
 // 2.6, global loads 2.0 ms of a 13 ms prefill GEMM budget); here an MFMA operand costs one LDS read per TT/1 use on the weight
 // side and one per use on the activation side, and a step is 17 TT MFMAs against ~180 + 80 TT VALU.
 //   rings: weights 3 stages per wave (requested two steps ahead), activations 2 stages per workgroup (one step ahead: they come from
@@ -778,20 +778,131 @@ static int skinny_n_cu();
 //   (in-order vmcnt).  Items (128-row group, token tile group) of one weight group run on the same XCD at the same time: its L2
 //   serves the weight bytes to all of them.
 constexpr int WD_NB = 2;  // stages of the activation ring (3 = requested two steps ahead, like the weights: measured equal, A/B on one box)
-template <int QT, int TT, int NW> constexpr int wd_lds_bytes() { return WD_NB * TT * (SK_B_BYTES + 128) + NW * 3 * tp_a_stage<QT>(); }
-constexpr int WD_NL = 2;  // loader waves per workgroup
+constexpr int WD_NA = 3;  // ... of the weight rings
+// Up to this many columns the K range may be split and Q6_K comes here too (k_mmq_wide_few).  Whole prompts of Llama-3-8B Q4_K_M, us, before / with it: 64 columns
+// 4106 / 3942, 77: 5336 / 4505, 112: 5648 / 5145, 160: 7691 / 6846, 256: 8673 / 7812, 288: 10371 / 8600, 384: 11613 / 11309; at 448 the split products cost what they
+// bring (12259 / 12708), and a Q6_K 14336 x 4096 takes 121 us here against 95 on the tiled GEMM at 512.
+constexpr int64_t WD_FEW = 384;
+constexpr int WD_NW = 4, WD_NL = 2;  // computing waves (one 32-row tile each) and loader waves of a workgroup
+template <int QT, int TT, int NSA = WD_NA> constexpr int wd_lds_bytes() { return WD_NB * TT * (SK_B_BYTES + 128) + WD_NW * NSA * 32 * 16 * sk_fmt<QT>::PIECES; }
+
+// A weight unit on its way to int8 matrix operands, sub-block by sub-block (Q6_K: pair by pair): next(j) yields the planes of values 32 j .. 32 j + 31 of this lane's row
+// (its half of them: 16 g ..), j = 0 .. 7 in turn.  Q4_K / Q5_K: digits of the sub-block scale times the codes (sk_unit_k45).
+template <int QT> struct sk_conv {
+    static constexpr int NP = QT == 4 ? 2 : 3;
+    static constexpr uint32_t DM = QT == 4 ? 0x07070707u : 0x03030303u;
+    static constexpr int DS = QT == 4 ? 3 : 2;
+    float d, dmin;
+    uint4 mins;  // the lane's f16 operand of the mins
+    const char * p;
+    uint32_t dlo[NP], dhi[NP];
+    uint4 qh, raw, nraw;
+    __device__ __forceinline__ void start(const char * arow, const int g, const int) {
+        typedef _Float16 half2s __attribute__((ext_vector_type(2)));
+        p = arow + (QT == 5 ? 48 : 16) + 16 * g;
+        const uint4 hdr = *(const uint4 *) arow;
+        raw = *(const uint4 *) p;
+        if constexpr (QT == 5) qh = *(const uint4 *) (arow + 16 + 16 * g);
+        d = h2f((uint16_t) (hdr.x & 0xFFFF));
+        dmin = h2f((uint16_t) (hdr.x >> 16));
+        const uint32_t slo = hdr.y & 0x3F3F3F3Fu, shi = (hdr.w & 0x0F0F0F0Fu) | ((hdr.y >> 2) & 0x30303030u);
+        const uint32_t mlo = hdr.z & 0x3F3F3F3Fu, mhi = ((hdr.w >> 4) & 0x0F0F0F0Fu) | ((hdr.z >> 2) & 0x30303030u);
+        const uint32_t msrc = g ? mhi : mlo;
+        const half2s k1024 = {(_Float16) 1024.0f, (_Float16) 1024.0f};
+        mins.x = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2s, sk_rep_byte<0>(msrc) | 0x64006400u) - k1024);
+        mins.y = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2s, sk_rep_byte<1>(msrc) | 0x64006400u) - k1024);
+        mins.z = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2s, sk_rep_byte<2>(msrc) | 0x64006400u) - k1024);
+        mins.w = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2s, sk_rep_byte<3>(msrc) | 0x64006400u) - k1024);
+#pragma unroll
+        for (int n = 0; n < NP; ++n) {
+            dlo[n] = (slo >> (DS * n)) & DM;
+            dhi[n] = (shi >> (DS * n)) & DM;
+        }
+    }
+    __device__ __forceinline__ void next(const int j, int4s (&W)[NP]) {  // (j is a constant after unrolling)
+        if (!(j & 1) && j < 6) nraw = *(const uint4 *) (p + 16 * j + 32);
+        const uint32_t r[4] = {raw.x, raw.y, raw.z, raw.w}, q5[4] = {qh.x, qh.y, qh.z, qh.w};
+        uint32_t w[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            w[k] = ((j & 1) ? r[k] >> 4 : r[k]) & 0x0F0F0F0Fu;
+            if constexpr (QT == 5) w[k] |= ((q5[k] >> j) & 0x01010101u) << 4;
+        }
+#pragma unroll
+        for (int n = 0; n < NP; ++n) {
+            const uint32_t src = j < 4 ? dlo[n] : dhi[n];
+            const uint32_t e = (j & 3) == 0 ? sk_rep_byte<0>(src) : (j & 3) == 1 ? sk_rep_byte<1>(src) : (j & 3) == 2 ? sk_rep_byte<2>(src) : sk_rep_byte<3>(src);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) W[n][k] = (int) sk_pk_mul(w[k], e);
+        }
+        if (j & 1) raw = nraw;
+    }
+};
+// Q6_K: 6-bit code x 8-bit scale is a 14-bit product: its low seven bits and the rest are the two planes.  The code's offset of 32 is taken off through the activations'
+// 16-value sums (mins = -32 x scales: all terms are multiples of 32 below 2^28, exact in f32).  Values 32 j + 16 g .. are sub-block 2 j + g.  sh: the block starts that
+// many bytes into the fetched row (210-byte blocks, whole dwords fetched).
+template <> struct sk_conv<6> {
+    static constexpr int NP = 2;
+    float d, dmin;
+    uint4 mins;
+    const char * a;
+    int g, sh;
+    uint32_t sc4[4], qa[4], qb[4], qc[4];
+    __device__ __forceinline__ void piece(const int o, uint32_t (&x)[4]) const {
+        const uint4 v = *(const uint4 *) (a + o);
+        const uint32_t nx = *(const uint32_t *) (a + o + 16);
+        x[0] = __builtin_amdgcn_alignbyte(v.y, v.x, sh);
+        x[1] = __builtin_amdgcn_alignbyte(v.z, v.y, sh);
+        x[2] = __builtin_amdgcn_alignbyte(v.w, v.z, sh);
+        x[3] = __builtin_amdgcn_alignbyte(nx, v.w, sh);
+    }
+    __device__ __forceinline__ void start(const char * arow, const int g_, const int sh_) {
+        typedef _Float16 half2s __attribute__((ext_vector_type(2)));
+        a = arow;
+        g = g_;
+        sh = sh_;
+        piece(192, sc4);
+        d = h2f((uint16_t) (*(const uint32_t *) (arow + 208) >> (8 * sh)));
+        dmin = 0.0f;
+        const uint32_t m0 = (g ? sc4[2] : sc4[0]) ^ 0x80808080u, m1 = (g ? sc4[3] : sc4[1]) ^ 0x80808080u;  // scale + 128; 0x6400 | n == 1024 + n in f16
+        const half2s k1152 = {(_Float16) 1152.0f, (_Float16) 1152.0f}, k32 = {(_Float16) -32.0f, (_Float16) -32.0f};
+        mins.x = __builtin_bit_cast(uint32_t, (__builtin_bit_cast(half2s, __builtin_amdgcn_perm(0u, m0, 0x0c010c00u) | 0x64006400u) - k1152) * k32);
+        mins.y = __builtin_bit_cast(uint32_t, (__builtin_bit_cast(half2s, __builtin_amdgcn_perm(0u, m0, 0x0c030c02u) | 0x64006400u) - k1152) * k32);
+        mins.z = __builtin_bit_cast(uint32_t, (__builtin_bit_cast(half2s, __builtin_amdgcn_perm(0u, m1, 0x0c010c00u) | 0x64006400u) - k1152) * k32);
+        mins.w = __builtin_bit_cast(uint32_t, (__builtin_bit_cast(half2s, __builtin_amdgcn_perm(0u, m1, 0x0c030c02u) | 0x64006400u) - k1152) * k32);
+#pragma unroll
+        for (int w = 0; w < 4; ++w) sc4[w] >>= 8 * g;
+    }
+    __device__ __forceinline__ void next(const int j, int4s (&W)[2]) {
+        typedef short short2s __attribute__((ext_vector_type(2)));
+        const int hf = j >> 2, k = j & 3;
+        if (k == 0) {
+            piece(64 * hf + 16 * g, qa);
+            piece(64 * hf + 32 + 16 * g, qb);
+            piece(128 + 32 * hf + 16 * g, qc);
+        }
+        const short e1 = (short) (int8_t) (sc4[2 * hf + (k >> 1)] >> (16 * (k & 1)));
+        const short2s e = {e1, e1};
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+            const uint32_t lo4 = (k & 1) ? qb[x] : qa[x];
+            const uint32_t q = ((k < 2 ? lo4 : lo4 >> 4) & 0x0F0F0F0Fu) | ((k < 2 ? qc[x] << (4 - 2 * k) : qc[x] >> (2 * k - 4)) & 0x30303030u);
+            const short2s pe = __builtin_bit_cast(short2s, q & 0x00FF00FFu) * e, po = __builtin_bit_cast(short2s, (q >> 8) & 0x00FF00FFu) * e;
+            W[0][x] = (int) ((__builtin_bit_cast(uint32_t, pe) & 0x007F007Fu) | ((__builtin_bit_cast(uint32_t, po) & 0x007F007Fu) << 8));
+            W[1][x] = (int) __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, po >> 7), __builtin_bit_cast(uint32_t, pe >> 7), 0x06020400u);
+        }
+    }
+};
 
 // NW computing waves (one 32-row tile each) + WD_NL loader waves.  In-kernel timestamps of the first version, where every wave
 // requested its own operands: per step and wave 1 050 clocks issuing 9 LDS-DMA instructions (each waits for room in the CU's one
 // address pipeline), 1 650 at the barrier (for the slowest issuer), 430 converting the weight unit, 2 700 in the 34 MFMAs of its two
 // token tiles — the matrix pipe busy 37 %.  The loaders take the first two off the computing waves: they request, wait (vmcnt) and
 // meet the others at the step's barrier; the computing waves only convert and multiply.
-// NL = 0: no loader waves — every computing wave requests its own weight tile and its share of the activations (NW waves = one per
-// SIMD: 512 registers each, accumulators in AGPRs, room for 4 token tiles per converted weight unit).  Measured (A/B, 2048-token
-// prefill): 23.2 k tok/s against 31.6 k for 4 + 2 waves x 2 tiles — the requests' issue stalls sit in the computing waves' own
-// instruction streams again.  Kept behind GGML_MI355X_MMQ_WIDE_SELF=1 (correct: the wide tests pass with it).
-template <int QT, int TT, int NW, int NL>
-__global__ void __launch_bounds__((NW + NL) * 64, 1) k_mmq_wide(const mmq8_args a) {
+// NL = 0: no loaders, but two workgroups a CU (the weight ring one stage shorter, so that both fit the LDS): one's arithmetic covers the other's requests and barrier.
+// Q4_K from 385 columns on: 28672 x 4096 at 512 columns 155 -> 149 us, a 2048-token prompt of Llama-3-8B 52.7 -> 51.9 ms.  (Q5_K's units do not fit twice.)
+template <int QT, int TT, int NW, int NL, int NSA>
+__global__ void __launch_bounds__((NW + NL) * 64, NSA == 2 ? 2 : 1) k_mmq_wide(const mmq8_args a) {
     constexpr bool SELF = NL == 0;
     constexpr int NLD = SELF ? NW : NL;  // waves that request
     extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -817,7 +928,7 @@ __global__ void __launch_bounds__((NW + NL) * 64, 1) k_mmq_wide(const mmq8_args 
     const uint32_t b_ring = lds0, d_ring = lds0 + WD_NB * B_STAGE, a_rings = d_ring + WD_NB * TT * 128;
     const char * const b_ring_p = smem;
     const char * const d_ring_p = smem + WD_NB * B_STAGE;
-    const char * const a_ring_p = smem + WD_NB * B_STAGE + WD_NB * TT * 128 + (loader ? 0 : wave) * 3 * A_STAGE;
+    const char * const a_ring_p = smem + WD_NB * B_STAGE + WD_NB * TT * 128 + (loader ? 0 : wave) * NSA * A_STAGE;
 
     // loader fetch roles (offsets from the unit's first byte)
     int a_off[NLA];
@@ -866,7 +977,7 @@ __global__ void __launch_bounds__((NW + NL) * 64, 1) k_mmq_wide(const mmq8_args 
         for (int k = 0; k < TPL; ++k) {
             const int t = ld * TPL + k;
             const uint8_t * wb = wg + (size_t) t * 32 * (size_t) w_nb1;
-            const uint32_t al = a_rings + (t * 3 + slot) * A_STAGE;
+            const uint32_t al = a_rings + (t * NSA + slot) * A_STAGE;
 #pragma unroll
             for (int u = 0; u < NLA; ++u)
                 if (u + 1 < NLA || (NPA % 64) == 0 || lane < (NPA % 64)) tp_dma16(wb + a_off[u], al + u * 1024);
@@ -901,11 +1012,10 @@ __global__ void __launch_bounds__((NW + NL) * 64, 1) k_mmq_wide(const mmq8_args 
     int vc = va, sc_ = 0;                             // the step being multiplied (computing waves)
 #define WD_ADV(v, sb) { if (++(sb) == nblk) { (sb) = 0; (v) = next_valid((v) + gridDim.x); } }
     if (loader || SELF) {
-        if (va < n_virtual) { issue_a(va, sa, na % 3); ++na; WD_ADV(va, sa) }
+        if (va < n_virtual) { issue_a(va, sa, na % NSA); ++na; WD_ADV(va, sa) }
         if (vb < n_virtual) { issue_b(vb, sbb, nb % WD_NB); ++nb; WD_ADV(vb, sbb) }
-        if (va < n_virtual) { issue_a(va, sa, na % 3); ++na; WD_ADV(va, sa) }
-        if (WD_NB == 3 && vb < n_virtual) { issue_b(vb, sbb, nb % WD_NB); ++nb; WD_ADV(vb, sbb) }
-    }
+        if (NSA == 3 && va < n_virtual) { issue_a(va, sa, na % NSA); ++na; WD_ADV(va, sa) }
+            }
     const int16s zeroi = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
     const float16s zerof = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
     if constexpr (!SELF) {
@@ -915,29 +1025,28 @@ __global__ void __launch_bounds__((NW + NL) * 64, 1) k_mmq_wide(const mmq8_args 
             for (int s = 0; s < total; ++s) {
                 // this loader's pieces of step s (weights requested two steps ago, activations one) have landed; only its weight requests of
                 // step s + 1 may still fly
-                // (WD_NB == 3: the activations run two steps ahead as well; what may still fly is step s + 1 of both kinds, requested together)
-                if (na > s + 1) tp_wait_c<WD_NB == 3 ? n_ops_a + NLB + DCNT : n_ops_a>();
+                if (NSA == 3 && na > s + 1) tp_wait_c<n_ops_a>();
                 else tp_wait_c<0>();
                 __syncthreads();  // everything of step s is in LDS, and nobody reads step s - 1 any more
                 if (vb < n_virtual) { issue_b(vb, sbb, nb % WD_NB); ++nb; WD_ADV(vb, sbb) }
-                if (va < n_virtual) { issue_a(va, sa, na % 3); ++na; WD_ADV(va, sa) }
+                if (va < n_virtual) { issue_a(va, sa, na % NSA); ++na; WD_ADV(va, sa) }
             }
             return;
         }
     }
     for (int s = 0; s < total; ++s) {
         if (SELF) {
-            if (na > s + 1) tp_wait_c<WD_NB == 3 ? n_ops_a + NLB + DCNT : n_ops_a>();
+            if (NSA == 3 && na > s + 1) tp_wait_c<n_ops_a>();
             else tp_wait_c<0>();
         }
         __syncthreads();  // everything of step s is in LDS, and nobody reads step s - 1 any more
         if (SELF) {
             if (vb < n_virtual) { issue_b(vb, sbb, nb % WD_NB); ++nb; WD_ADV(vb, sbb) }
-            if (va < n_virtual) { issue_a(va, sa, na % 3); ++na; WD_ADV(va, sa) }
+            if (va < n_virtual) { issue_a(va, sa, na % NSA); ++na; WD_ADV(va, sa) }
         }
 
         // ---- this wave's weight unit -> digit-plane operands, once per step
-        const char * const arow = a_ring_p + (s % 3) * A_STAGE + row * F::ROW;
+        const char * const arow = a_ring_p + (s % NSA) * A_STAGE + row * F::ROW;
         const uint4 hdr = *(const uint4 *) arow;
         const float d = h2f((uint16_t) (hdr.x & 0xFFFF)), dmin = h2f((uint16_t) (hdr.x >> 16));
         const uint32_t slo = hdr.y & 0x3F3F3F3Fu, shi = (hdr.w & 0x0F0F0F0Fu) | ((hdr.y >> 2) & 0x30303030u);
@@ -1057,29 +1166,337 @@ __global__ void __launch_bounds__((NW + NL) * 64, 1) k_mmq_wide(const mmq8_args 
 #undef MAT_OF
 }
 
-// Prompt batches (33 columns and up) take the wide form when every matrix is whole 128-row groups of Q4_K / Q5_K, there is no K
-// split and (row groups x 64-column groups) can occupy the chip.  One workgroup shape is in use — 4 computing waves (128 rows) x 2
-// token tiles (64 columns) + 2 loaders; measured on the 512-token prefill of Llama-3-8B Q4_K_M against the tiled GEMM at 28.9 k tok/s:
-// this shape 30.5 k; 8 computing waves x 2 tiles, everyone requesting its own operands, 28.7 k; the same with 2 / 4 loaders 26.1 /
-// 28.9 k (one address pipeline per CU: 52 LDS-DMA instructions per step); 4 waves x 4 tiles 20.2 k (spills at the 256-register cap
-// of six waves).  Qwen2-7B Q5_K_M (three digit planes: the tiled GEMM spills there) 20.5 -> 25.3 k.  Returns the shape code
-// NW * 16 + TT, or 0.  The caller's activation area must hold whole 128-column groups (columns beyond M are fetched, never stored).
+// ------------------------------------------------------------------------------------------------ wide form, up to WD_FEW columns
+// The same workgroup (4 computing waves + 2 loaders) where the columns are too few for the grid above: a K slice is part of the item, so that 4096 rows x 77 columns
+// fill the chip with 8 slices of two super-blocks (partial products to [slice][M][N], summed by the consumer as ever), three token tiles a workgroup where that wastes
+// less than two (65 .. 96 columns), and Q6_K.  What bounds a launch is the computing waves' instruction stream — one wave a SIMD: the ALU's ~175 + 90 TT instructions
+// and 17 TT MFMAs of a step in one queue — so LAP puts the one behind the other: the weight unit is converted chunk by chunk while the first token tile is
+// multiplied, a tile's sums are folded while the next one is.  MI355X, 77 columns: gate/up 28672 x 4096 50 -> 36 us, wo and ffn_down Q4_K 21 -> 17,
+// ffn_down Q6_K 39 .. 51 -> 29, wq + wk (+ wv) 22 -> 17.  (At 512 columns the chunks gain nothing over k_mmq_wide.)
+template <int QT, int TT, bool LAP>
+__global__ void __launch_bounds__((WD_NW + WD_NL) * 64, 1) k_mmq_wide_few(const mmq8_args a) {
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    typedef sk_fmt<QT> F;
+    constexpr int NP = QT == 5 ? 3 : 2;
+    constexpr int NPA = 32 * F::PIECES, NLA = (NPA + 63) / 64;
+    constexpr int NPB = TT * 32 * 19 / WD_NL, NLB = (NPB + 63) / 64;  // activation pieces per loader and step, and the instructions fetching them
+    constexpr int TPL = WD_NW / WD_NL;                               // weight tiles per loader
+    constexpr int DCNT = (TT + WD_NL - 1) / WD_NL;                   // scale requests per loader and step
+    constexpr int B_STAGE = TT * SK_B_BYTES, A_STAGE = 32 * 16 * F::PIECES;  // (LDS-DMA is lane-linear: rows of whole pieces)
+    static_assert(WD_NW % WD_NL == 0 && (TT * 32 * 19) % WD_NL == 0, "loader roles");
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const bool loader = wave >= WD_NW;
+    const int ld = wave - WD_NW;  // loader index
+    const int row = lane & 31, g = lane >> 5;
+    const int nblk = a.K / 256;
+    const int w_nb1 = (int) a.mat[0].w_nb1;
+    const int tok_bytes = nblk * (int) sizeof(q8k_dev);
+    const uint32_t lds0 = (uint32_t) (uintptr_t) smem;
+    // LDS: [activation ring 2 x TT x 9728][scale ring 2 x TT x 128][weight rings: tile x 3 x stage]
+    const uint32_t b_ring = lds0, d_ring = lds0 + WD_NB * B_STAGE, a_rings = d_ring + WD_NB * TT * 128;
+    const char * const b_ring_p = smem;
+    const char * const d_ring_p = smem + WD_NB * B_STAGE;
+    const char * const a_ring_p = smem + WD_NB * B_STAGE + WD_NB * TT * 128 + (loader ? 0 : wave) * WD_NA * A_STAGE;
+
+    // loader fetch roles (offsets from the unit's first byte)
+    int a_off[NLA];
+#pragma unroll
+    for (int u = 0; u < NLA; ++u) {
+        const int pi = min(lane + 64 * u, NPA - 1);
+        a_off[u] = (pi / F::PIECES) * w_nb1 + (pi % F::PIECES) * 16;
+    }
+    int b_off[NLB];
+#pragma unroll
+    for (int u = 0; u < NLB; ++u) {
+        const int pi = max(ld, 0) * NPB + min(lane + 64 * u, NPB - 1);
+        b_off[u] = (pi / 19) * tok_bytes + (pi % 19) * 16;
+    }
+    const int d_off = row * tok_bytes + 304;  // q8k_dev::d of token `row` of a token tile
+    constexpr int n_ops_a = TPL * NLA;        // a loader's weight requests of one step
+
+#define MAT_OF(t) ((a.n_mat > 2 && (t) >= a.mat[2].panel0) ? 2 : ((a.n_mat > 1 && (t) >= a.mat[1].panel0) ? 1 : 0))
+#define MAT_SEL(mi, f) ((mi) == 0 ? a.mat[0].f : ((mi) == 1 ? a.mat[1].f : a.mat[2].f))
+    // virtual items v = blockIdx.x + gridDim.x r: XCD v % 8 (workgroups go round the XCDs) serves groups xcd, xcd + 8, ..; the token-tile
+    // groups of one weight group are consecutive there
+    const int n_groups = a.n_panels, m_tiles = a.m_tiles;
+    const int n_virtual = ((n_groups + 7) / 8) * 8 * m_tiles * a.ksplit;
+    // the item v: row group, K slice and token tile (token tiles innermost: they share the weights)
+    auto decode = [&](const int v, int & group, int & ks, int & mt) {
+        const int xcd = v & 7, q = v >> 3, per = m_tiles * a.ksplit;
+        const int gq = q / per, rem = q - gq * per;
+        group = gq * 8 + xcd;
+        ks = rem / m_tiles;
+        mt = rem - ks * m_tiles;
+    };
+    auto next_valid = [&](int v) {
+        for (; v < n_virtual; v += gridDim.x)
+            if (((v >> 3) / (m_tiles * a.ksplit)) * 8 + (v & 7) < n_groups) return v;
+        return n_virtual;
+    };
+    auto slice = [&](const int ks) { return ks * nblk / a.ksplit; };  // first super-block of a K slice
+    int total = 0;  // steps of this workgroup (the same number in every wave: one barrier each)
+    for (int v = next_valid(blockIdx.x); v < n_virtual; v = next_valid(v + gridDim.x)) {
+        int gr, ks, mt;
+        decode(v, gr, ks, mt);
+        total += slice(ks + 1) - slice(ks);
+    }
+    // request cursors: the item, what is left of its K slice, and where its next block is (decoded once per item)
+    struct cursor { int v, left; const char * at; };
+    auto seek_a = [&](cursor & c) {
+        if (c.v >= n_virtual) return;
+        int gr, ks, mt;
+        decode(c.v, gr, ks, mt);
+        const int mi = MAT_OF(gr), sb = slice(ks);
+        c.left = slice(ks + 1) - sb;
+        c.at = (const char *) MAT_SEL(mi, W) + (size_t) (gr - MAT_SEL(mi, panel0)) * (32 * WD_NW) * (size_t) w_nb1 + (size_t) sb * F::BYTES;
+    };
+    auto seek_b = [&](cursor & c) {
+        if (c.v >= n_virtual) return;
+        int gr, ks, mt;
+        decode(c.v, gr, ks, mt);
+        const int sb = slice(ks);
+        c.left = slice(ks + 1) - sb;
+        c.at = (const char *) a.act + (size_t) mt * (32 * TT) * (size_t) tok_bytes + (size_t) sb * sizeof(q8k_dev);
+    };
+
+    auto issue_a = [&](const char * wg, const int slot) {
+#pragma unroll
+        for (int k = 0; k < TPL; ++k) {
+            const int t = ld * TPL + k;
+            const char * wb = wg + (size_t) t * 32 * (size_t) w_nb1;
+            if constexpr (QT == 6) wb -= (uintptr_t) wb & 2;  // (a block of an odd index starts two bytes into its first dword)
+            const uint32_t al = a_rings + (t * WD_NA + slot) * A_STAGE;
+#pragma unroll
+            for (int u = 0; u < NLA; ++u)
+                if (u + 1 < NLA || (NPA % 64) == 0 || lane < (NPA % 64)) tp_dma16(wb + a_off[u], al + u * 1024);
+        }
+    };
+    auto issue_b = [&](const char * ab, const int slot) {
+        const uint32_t bl = b_ring + slot * B_STAGE + ld * NPB * 16;
+#pragma unroll
+        for (int u = 0; u < NLB; ++u)
+            if (u + 1 < NLB || (NPB % 64) == 0 || lane < (NPB % 64)) tp_dma16(ab + b_off[u], bl + u * 1024);
+        // the block scales of token tile tt: loader tt % WD_NL — every loader issues DCNT of these instructions (a duplicate when it has
+        // no tile of its own), so that the wait counts are the same compile-time constants for all
+#pragma unroll
+        for (int t = 0; t < DCNT; ++t) {
+            const int tt = min(ld + t * WD_NL, TT - 1);
+            if (lane < 32) tp_dma4(ab + (size_t) tt * 32 * (size_t) tok_bytes + d_off, d_ring + slot * TT * 128 + tt * 128);
+        }
+    };
+
+    float acc[TT][16];
+#pragma unroll
+    for (int t = 0; t < TT; ++t)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[t][i] = 0.0f;
+
+    // weights run WD_NA - 1 steps ahead, activations one
+    cursor ca{next_valid(blockIdx.x), 0, nullptr}, cb = ca;
+    int na = 0, nb = 0, sa = 0, sb_ = 0;  // steps requested so far and the slots of the next
+    int vc = ca.v, lc = 0, mc = 0, nc = 0, kc = 0, sbc = 0;  // the item being multiplied (computing waves): steps left, token tile, row group, K slice; its super-block
+    if (vc < n_virtual) {
+        decode(vc, nc, kc, mc);
+        sbc = slice(kc);
+        lc = slice(kc + 1) - sbc;
+    }
+#define WD_ISSUE_A() { issue_a(ca.at, sa); ++na; sa = sa + 1 == WD_NA ? 0 : sa + 1; ca.at += F::BYTES; if (--ca.left == 0) { ca.v = next_valid(ca.v + gridDim.x); seek_a(ca); } }
+#define WD_ISSUE_B() { issue_b(cb.at, sb_); ++nb; sb_ ^= 1; cb.at += sizeof(q8k_dev); if (--cb.left == 0) { cb.v = next_valid(cb.v + gridDim.x); seek_b(cb); } }
+    const int16s zeroi = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+    const float16s zerof = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+    // the loaders' loop, apart from the computing waves' (one barrier per step in both): its address registers are not live in the
+    // multiply loop and the operands are not live here (239 -> 183 registers for Q4_K)
+    if (loader) {
+        seek_a(ca);
+        seek_b(cb);
+        if (na < total) WD_ISSUE_A()
+        if (nb < total) WD_ISSUE_B()
+        if (na < total) WD_ISSUE_A()
+        for (int s = 0; s < total; ++s) {
+            // this loader's pieces of step s (weights requested two steps ago, activations one) have landed; only its weight requests of
+            // step s + 1 may still fly
+            if (na > s + 1) tp_wait_c<n_ops_a>();
+            else tp_wait_c<0>();
+            __syncthreads();  // everything of step s is in LDS, and nobody reads step s - 1 any more
+            if (nb < total) WD_ISSUE_B()
+            if (na < total) WD_ISSUE_A()
+        }
+        return;
+    }
+    int slot_a = 0, slot_b = 0;  // the slots of the step being multiplied
+    for (int s = 0; s < total; ++s) {
+        __syncthreads();  // everything of step s is in LDS, and nobody reads step s - 1 any more
+
+        const char * const arow = a_ring_p + slot_a * A_STAGE + row * 16 * F::PIECES;
+        const char * const brow = b_ring_p + slot_b * B_STAGE + row * SK_BTOK + 16 * g;
+        const float * const dst_ = (const float *) (d_ring_p + slot_b * TT * 128) + 4 * g;
+        auto Y = [&](const int c) { return *(const int4s *) (brow + (c >> 3) * 32 * SK_BTOK + 32 * (c & 7)); };  // chunk c = 8 t + j: values 32 j .. of token tile t
+        auto BS = [&](const int t) { return *(const half8s *) (brow + t * 32 * SK_BTOK + 256); };
+        auto DY = [&](const int t, const int q) { return *(const float4 *) (dst_ + t * 32 + 8 * q); };
+        // LAP: the step in chunks of NP MFMAs with the arithmetic that hides behind them; the operands of the chunk after the next are on their way from LDS.
+        // (sched_barrier: the compiler would sort the chunks back into runs.  Q5_K goes without: a second set of its three planes' sums does not fit in the registers)
+        sk_conv<QT> cv;
+        cv.start(arow, g, 2 * (sbc & 1));
+        int4s W[8][NP];
+        int16s pl[LAP ? 2 : 1][NP];
+        float16s ms;
+        auto fold = [&](const int t, const int i, const float dy) {
+            const int16s * const P = pl[LAP ? t & 1 : 0];
+            int isum;
+            if constexpr (QT == 4) isum = (P[1][i] << 3) + P[0][i];
+            else if constexpr (QT == 6) isum = (int) ((uint32_t) P[1][i] << 7) + P[0][i];
+            else isum = (P[NP - 1][i] << 4) + (P[1][i] << 2) + P[0][i];
+            const float v = QT == 6 ? cv.d * (float) isum : __builtin_fmaf(-cv.dmin, ms[i], cv.d * (float) isum);
+            acc[t][i] = __builtin_fmaf(dy, v, acc[t][i]);
+        };
+        if constexpr (LAP) {
+            int4s y0 = Y(0), y1 = Y(1);
+            float4 dy0 = DY(0, 0), dy1;
+            half8s bs = BS(0);
+#pragma unroll
+            for (int c = 0; c < 8 * TT; ++c) {
+                const int t = c >> 3, j = c & 7;
+                const int4s y = (c & 1) ? y1 : y0;
+                if (c + 2 < 8 * TT) { if (c & 1) y1 = Y(c + 2); else y0 = Y(c + 2); }
+                if (t == 0) cv.next(j, W[j]);
+                if (QT == 6 && j == 0) {
+                    const float16s m = __builtin_amdgcn_mfma_f32_32x32x16_f16(bs, __builtin_bit_cast(half8s, cv.mins), zerof, 0, 0, 0);
+                    if (t + 1 < TT) bs = BS(t + 1);
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) pl[LAP ? t & 1 : 0][0][i] = (int) m[i];
+                }
+#pragma unroll
+                for (int n = 0; n < NP; ++n) pl[LAP ? t & 1 : 0][n] = __builtin_amdgcn_mfma_i32_32x32x32_i8(y, W[j][n], j == 0 && (QT != 6 || n > 0) ? zeroi : pl[LAP ? t & 1 : 0][n], 0, 0, 0);
+                if (t > 0) {
+                    const float4 dy = ((j >> 1) & 1) ? dy1 : dy0;
+                    if (!(j & 1)) { if ((j >> 1) & 1) dy0 = DY(j == 6 ? t : t - 1, ((j >> 1) + 1) & 3); else dy1 = DY(t - 1, (j >> 1) + 1); }
+                    fold(t - 1, 2 * j, (j & 1) ? dy.z : dy.x);
+                    fold(t - 1, 2 * j + 1, (j & 1) ? dy.w : dy.y);
+                }
+                if (QT != 6 && j == 7) {
+                    ms = __builtin_amdgcn_mfma_f32_32x32x16_f16(bs, __builtin_bit_cast(half8s, cv.mins), zerof, 0, 0, 0);
+                    if (t + 1 < TT) bs = BS(t + 1);
+                }
+                if (c + 1 == 8 * TT) {
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        const float4 dy = q == 0 ? dy0 : DY(t, q);
+                        fold(t, 4 * q, dy.x);
+                        fold(t, 4 * q + 1, dy.y);
+                        fold(t, 4 * q + 2, dy.z);
+                        fold(t, 4 * q + 3, dy.w);
+                    }
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) cv.next(j, W[j]);
+#pragma unroll
+            for (int t = 0; t < TT; ++t) {
+                if (QT == 6) {
+                    const float16s m = __builtin_amdgcn_mfma_f32_32x32x16_f16(BS(t), __builtin_bit_cast(half8s, cv.mins), zerof, 0, 0, 0);
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) pl[0][0][i] = (int) m[i];
+                }
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    const int4s y = Y(8 * t + j);
+#pragma unroll
+                    for (int n = 0; n < NP; ++n) pl[0][n] = __builtin_amdgcn_mfma_i32_32x32x32_i8(y, W[j][n], j == 0 && (QT != 6 || n > 0) ? zeroi : pl[0][n], 0, 0, 0);
+                }
+                if (QT != 6) ms = __builtin_amdgcn_mfma_f32_32x32x16_f16(BS(t), __builtin_bit_cast(half8s, cv.mins), zerof, 0, 0, 0);
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const float4 dy = DY(t, q);
+                    fold(t, 4 * q, dy.x);
+                    fold(t, 4 * q + 1, dy.y);
+                    fold(t, 4 * q + 2, dy.z);
+                    fold(t, 4 * q + 3, dy.w);
+                }
+            }
+        }
+        slot_a = slot_a + 1 == WD_NA ? 0 : slot_a + 1;
+        slot_b ^= 1;
+        ++sbc;
+        if (--lc == 0) {
+            // ---- the tiles are complete: lane = weight row, register i = token (i & 3) + 8 (i >> 2) + 4 g of token tile t
+            const int mi = MAT_OF(nc);
+            const int n = (nc - MAT_SEL(mi, panel0)) * (32 * WD_NW) + wave * 32 + row;
+            const int mN = MAT_SEL(mi, N);
+            const bool split = a.ksplit > 1;
+            float * const m_dst = split ? MAT_SEL(mi, part) + (size_t) kc * a.M * mN : MAT_SEL(mi, dst);
+            const int64_t m_dst_stride = split ? mN : MAT_SEL(mi, dst_stride);
+            const float * const m_add = split ? nullptr : MAT_SEL(mi, add);
+            const int64_t m_add_stride = MAT_SEL(mi, add_stride);
+            // (addends first, all of them in flight, then nothing but stores: with the optional load inside the store loop the compiler
+            // waited vmcnt(0) before every store — stores count in vmcnt on this ISA, so each of the 32 waited for its predecessor's
+            // write acknowledgement, ~16k clocks per item)
+            if (m_add) {
+#pragma unroll
+                for (int t = 0; t < TT; ++t)
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) {
+                        const int tok = min(mc * 32 * TT + t * 32 + (i & 3) + 8 * (i >> 2) + 4 * g, a.M - 1);
+                        acc[t][i] += m_add[(size_t) tok * m_add_stride + n];
+                    }
+            }
+#pragma unroll
+            for (int t = 0; t < TT; ++t)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {
+                    const int tok = mc * 32 * TT + t * 32 + (i & 3) + 8 * (i >> 2) + 4 * g;
+                    if (tok < a.M) m_dst[(size_t) tok * m_dst_stride + n] = acc[t][i];
+                    acc[t][i] = 0.0f;
+                }
+            vc = next_valid(vc + gridDim.x);
+            if (vc < n_virtual) {
+                decode(vc, nc, kc, mc);
+                sbc = slice(kc);
+                lc = slice(kc + 1) - slice(kc);
+            }
+        }
+    }
+#undef WD_ISSUE_A
+#undef WD_ISSUE_B
+#undef MAT_SEL
+#undef MAT_OF
+}
+
+// Prompt batches (33 columns and up) take a wide form when every matrix is whole 128-row groups, rows packed back to back: up to WD_FEW columns Q4_K, Q5_K and Q6_K with
+// as many K slices as fill the chip; beyond, Q4_K and Q5_K without a K split where (row groups x 64-column groups) occupy half of it.  Measured on the 512-token prefill
+// of Llama-3-8B Q4_K_M against the tiled GEMM at 28.9 k tok/s: 4 computing waves x 2 token tiles + 2 loaders 30.5 k; 8 computing waves x 2 tiles, everyone requesting its
+// own operands, 28.7 k; the same with 2 / 4 loaders 26.1 / 28.9 k (one address pipeline per CU: 52 LDS-DMA instructions per step); 4 waves x 4 tiles 20.2 k (spills at
+// the 256-register cap of six waves).  Qwen2-7B Q5_K_M (three digit planes: the tiled GEMM spills there) 20.5 -> 25.3 k.  Returns the token tiles of a workgroup, or 0.
+// The caller's activation area must hold whole 128-column groups (columns beyond M are fetched, never stored).
+bool mmq_wide_fills(int type, int64_t g128, int64_t M) { return type != GGML_TYPE_Q6_K && g128 * ((M + 63) / 64) * 2 >= skinny_n_cu(); }
 int mmq_wide_tiles(int type, int64_t K, const int64_t * N, int n_mat, int64_t M, int64_t w_nb1, int ksplit) {
     static const bool on = !getenv("GGML_MI355X_MMQ_WIDE") || atoi(getenv("GGML_MI355X_MMQ_WIDE")) != 0;
-    if (!on || !(type == GGML_TYPE_Q4_K || type == GGML_TYPE_Q5_K) || ksplit != 1 || M < 33 || (K % 256) != 0) return 0;
-    if (w_nb1 != (K / 256) * (type == GGML_TYPE_Q4_K ? 144 : 176)) return 0;
+    if (!on || M < 33 || (K % 256) != 0 || ksplit > K / 256) return 0;
+    if (!(type == GGML_TYPE_Q4_K || type == GGML_TYPE_Q5_K || type == GGML_TYPE_Q6_K)) return 0;
+    if (w_nb1 != (K / 256) * (type == GGML_TYPE_Q4_K ? 144 : type == GGML_TYPE_Q5_K ? 176 : 210)) return 0;
+    if (type == GGML_TYPE_Q6_K && (K % 512) != 0) return 0;  // rows of whole dwords: the two-byte shift of a block is the same in every row
     int64_t g128 = 0;
     for (int i = 0; i < n_mat; ++i) {
         if (N[i] % 128) return 0;
         g128 += N[i] / 128;
     }
-    return g128 * ((M + 63) / 64) * 2 >= skinny_n_cu() ? 4 * 16 + 2 : 0;
+    // three tiles where they waste fewer columns than two (Q5_K: their registers do not fit)
+    if (M <= WD_FEW) return type != GGML_TYPE_Q5_K && (M + 95) / 96 * 96 < (M + 63) / 64 * 64 ? 3 : 2;
+    return ksplit == 1 && mmq_wide_fills(type, g128, M) ? 2 : 0;
+}
+int mmq_wide_ksplit(int type, int64_t K, int64_t N, int64_t M) {
+    const int tt = mmq_wide_tiles(type, K, &N, 1, M, (K / 256) * (type == GGML_TYPE_Q4_K ? 144 : type == GGML_TYPE_Q5_K ? 176 : 210), 1);
+    if (!tt) return 0;
+    if (M > WD_FEW) return 1;
+    const int64_t items = N / 128 * ((M + 32 * tt - 1) / (32 * tt));
+    return (int) std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(8, K / 512), skinny_n_cu() / items));
 }
 
-template <int QT, int TT, int NW, int NL> static void launch_wide_t(hipStream_t s, mmq8_args a) {
+template <int QT, int TT, int NW, int NL, int NSA> static void launch_wide_t(hipStream_t s, mmq8_args a) {
     static std::atomic<uint32_t> lds_raised{0};
-    const void * fn = (const void *) k_mmq_wide<QT, TT, NW, NL>;
-    const size_t lds = (size_t) wd_lds_bytes<QT, TT, NW>();
+    const void * fn = (const void *) k_mmq_wide<QT, TT, NW, NL, NSA>;
+    const size_t lds = (size_t) wd_lds_bytes<QT, TT, NSA>();
     (void) ensure_dyn_lds(fn, lds, lds_raised);
     a.n_panels = 0;
     for (int i = 0; i < a.n_mat; ++i) {
@@ -1088,14 +1505,31 @@ template <int QT, int TT, int NW, int NL> static void launch_wide_t(hipStream_t 
     }
     a.m_tiles = (a.M + 32 * TT - 1) / (32 * TT);
     const int n_virtual = ((a.n_panels + 7) / 8) * 8 * a.m_tiles;
-    MI_LAUNCH_PROBED((k_mmq_wide<QT, TT, NW, NL>), dim3((unsigned) std::min(n_virtual, skinny_n_cu())), dim3((NW + NL) * 64), lds, s, a);
+    MI_LAUNCH_PROBED((k_mmq_wide<QT, TT, NW, NL, NSA>), dim3((unsigned) std::min(n_virtual, skinny_n_cu() * (NSA == 2 ? 2 : 1))), dim3((NW + NL) * 64), lds, s, a);
 }
-void launch_mmq_wide(hipStream_t s, int type, int shape, const mmq8_args & a) {
-    static const int self4 = getenv("GGML_MI355X_MMQ_WIDE_SELF") ? atoi(getenv("GGML_MI355X_MMQ_WIDE_SELF")) : 0;  // experiment: 4 waves x 4 token tiles, no loaders
-    (void) shape;
-    if (self4 && type == GGML_TYPE_Q4_K) { launch_wide_t<4, 4, 4, 0>(s, a); return; }
-    if (type == GGML_TYPE_Q4_K) launch_wide_t<4, 2, 4, WD_NL>(s, a);
-    else launch_wide_t<5, 2, 4, WD_NL>(s, a);
+template <int QT, int TT, bool LAP> static void launch_wide_few_t(hipStream_t s, mmq8_args a) {
+    static std::atomic<uint32_t> lds_raised{0};
+    constexpr size_t lds = (size_t) wd_lds_bytes<QT, TT>();
+    (void) ensure_dyn_lds((const void *) k_mmq_wide_few<QT, TT, LAP>, lds, lds_raised);
+    a.n_panels = 0;
+    for (int i = 0; i < a.n_mat; ++i) {
+        a.mat[i].panel0 = a.n_panels;
+        a.n_panels += a.mat[i].N / (32 * WD_NW);
+    }
+    a.m_tiles = (a.M + 32 * TT - 1) / (32 * TT);
+    const int n_virtual = ((a.n_panels + 7) / 8) * 8 * a.m_tiles * a.ksplit;
+    MI_LAUNCH_PROBED((k_mmq_wide_few<QT, TT, LAP>), dim3((unsigned) std::min(n_virtual, skinny_n_cu())), dim3((WD_NW + WD_NL) * 64), lds, s, a);
+}
+void launch_mmq_wide(hipStream_t s, int type, int tt, const mmq8_args & a) {
+    if (a.M > WD_FEW) {
+        if (type == GGML_TYPE_Q5_K) launch_wide_t<5, 2, WD_NW, WD_NL, WD_NA>(s, a);
+        else launch_wide_t<4, 2, WD_NW, 0, 2>(s, a);
+    } else if (type == GGML_TYPE_Q5_K) launch_wide_few_t<5, 2, false>(s, a);
+    else if (type == GGML_TYPE_Q6_K) {
+        if (tt == 3) launch_wide_few_t<6, 3, true>(s, a);
+        else launch_wide_few_t<6, 2, true>(s, a);
+    } else if (tt == 3) launch_wide_few_t<4, 3, true>(s, a);
+    else launch_wide_few_t<4, 2, true>(s, a);
 }
 
 bool mmq_skinny_supported(int type, int64_t K, int64_t N, int64_t M, int64_t w_nb1) {

@@ -132,3 +132,27 @@ def test_k_quant_batches_by_groups_of_eight_columns(backend, H, qt, K, N):
         got = run(M, backend, w)
         assert np.array_equal(got.view(np.uint32), full[:M].view(np.uint32)), M
     assert T.nmse(full[:, rows], ref[: len(full)]) <= 1e-10
+
+
+# one super-block and many, K slices of unequal lengths, two and three token tiles a workgroup with ragged ends, both sides of the line to the unsplit form, Q6_K rows of an odd number of blocks
+@pytest.mark.parametrize("qt", [L.Q4_K, L.Q5_K, L.Q6_K])
+@pytest.mark.parametrize("K,N,M", [(256, 128, 33), (512, 256, 65), (4608, 128, 77), (2560, 384, 96), (1024, 4096, 97), (768, 512, 129), (2048, 1024, 190), (512, 8192, 288), (1536, 640, 384), (1536, 16384, 385)])
+def test_k_quant_batches_of_33_columns_and_up(backend, H, qt, K, N, M):
+    """mmq_skinny.hip: k_mmq_wide_few / k_mmq_wide against the oracle and, the sums of the K slices apart, the tiled GEMM: exact integer block sums, f32 sums over K / 256 terms."""
+    rng = np.random.default_rng(K + N + M)
+    w = T.rand_weight(qt, K, N, rng).reshape(N, -1)
+    x = (rng.standard_normal((M, K)) * rng.uniform(0.2, 3.0, (M, 1))).astype(np.float32)
+    b = rng.standard_normal((M, N)).astype(np.float32)
+
+    def run(where, ww, bb):
+        return T.run_case(lambda g: H.ggml_add(g.ctx, H.ggml_mul_mat(g.ctx, g.new(qt, [K, ww.shape[0]], ww), g.new(L.F32, [K, M], x)), g.new(L.F32, [ww.shape[0], M], bb)), where)[0].reshape(M, -1)
+
+    got = run(backend, w, b)
+    backend.set_option("mmq_skinny", 0)
+    try:
+        tiled = run(backend, w, b)
+    finally:
+        backend.set_option("mmq_skinny", 1)
+    assert T.nmse(got, tiled) <= 1e-12
+    rows = np.unique(np.concatenate([np.arange(min(N, 40)), np.arange(max(0, N - 40), N)]))
+    assert T.nmse(got[:, rows], run("oracle", np.ascontiguousarray(w[rows]), np.ascontiguousarray(b[:, rows]))) <= 1e-10
