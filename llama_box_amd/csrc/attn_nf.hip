@@ -24,16 +24,16 @@ namespace mi355x {
 
 #define NF_CAP 1024  // visible cells per token served from registers and LDS
 struct __attribute__((aligned(4))) u32x4a { uint32_t x, y, z, w; };  // a 16-byte load that only promises dword alignment
-template <int G>
-__global__ void __launch_bounds__(256) k_attn_nf_list(const tdesc q, const tdesc k, const tdesc v, const tdesc mask, const tdesc dst, const int * __restrict__ lists,
+template <int G, int NW>
+__global__ void __launch_bounds__(NW * 64) k_attn_nf_list(const tdesc q, const tdesc k, const tdesc v, const tdesc mask, const tdesc dst, const int * __restrict__ lists,
                                                       const int list_stride, float * __restrict__ scratch, const float scale, const int dq_n, q8k_dev * __restrict__ q8, const int nf_groups_on) {
     // q8 != null (only with dq_n == 1 and an even G): the result's only readers are quantised mat-muls (wo) — it leaves the kernel as the
     // Q8_K blocks quantize_row_q8_K builds of the token's row (a block = two heads), through the q area of the LDS, and not as f32
-    constexpr int D = 128;
+    constexpr int D = 128, NT = NW * 64;
     const bool nf_groups = nf_groups_on;
     extern __shared__ __attribute__((aligned(16))) float nf_smem[];  // q [G][128] | positions [NF_CAP] | probabilities [G][NF_CAP]
-    __shared__ float shf[4];
-    __shared__ double shd[4];
+    __shared__ float shf[NW];
+    __shared__ double shd[NW];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int tok = blockIdx.x, kvh = blockIdx.y, dq = blockIdx.z;
     const int n_kv = (int) k.ne[1], nkv_heads = (int) k.ne[2];
@@ -57,7 +57,7 @@ __global__ void __launch_bounds__(256) k_attn_nf_list(const tdesc q, const tdesc
         }
     };
     if (cnt == 0) {  // a token that sees nothing: the CPU's row is expf(-inf - -inf) = NaN throughout
-        for (int e = tid; e < G * rows_per; e += 256) put(e / rows_per, d0 + e % rows_per, __builtin_nanf(""));
+        for (int e = tid; e < G * rows_per; e += NT) put(e / rows_per, d0 + e % rows_per, __builtin_nanf(""));
         finish();
         return;
     }
@@ -72,18 +72,18 @@ __global__ void __launch_bounds__(256) k_attn_nf_list(const tdesc q, const tdesc
         float * qs = nf_smem;                       // [G][128] q rounded to f16
         int * pos_s = (int *) (nf_smem + G * D);    // [NF_CAP]
         float * p_s = nf_smem + G * D + NF_CAP;     // [G][NF_CAP]
-        for (int e = tid; e < G * D; e += 256) {
+        for (int e = tid; e < G * D; e += NT) {
             const int g = e / D, i = e % D;
             qs[e] = h2f(f2h(*((const float *) (q.data + (int64_t) tok * q.nb[1] + (int64_t) (kvh * G + g) * q.nb[2]) + i)));
         }
-        for (int c = tid; c < cnt; c += 256) pos_s[c] = pos[c];
+        for (int c = tid; c < cnt; c += NT) pos_s[c] = pos[c];
         __syncthreads();
         float mx[G];
 #pragma unroll
         for (int g = 0; g < G; ++g) mx[g] = -INFINITY;
         const char * kbase = k.data + (int64_t) kvh * k.nb[2];
 #pragma unroll 1
-        for (int c = tid; c < cnt; c += 256) {
+        for (int c = tid; c < cnt; c += NT) {
             const int pc = pos_s[c];
             const uint4 * kr = (const uint4 *) (kbase + (int64_t) pc * k.nb[1]);
             uint4 kv[16];  // the K row: 128 halves, all 16 loads in flight
@@ -110,12 +110,12 @@ __global__ void __launch_bounds__(256) k_attn_nf_list(const tdesc q, const tdesc
                 p_s[g * NF_CAP + c] = t;  // (this thread's own slot until the probabilities are published below)
             }
         }
-        for (int c = tid; c < cnt; c += 256) {
+        for (int c = tid; c < cnt; c += NT) {
 #pragma unroll
             for (int g = 0; g < G; ++g) mx[g] = fmaxf(mx[g], p_s[g * NF_CAP + c]);
         }
-        __shared__ float shm[4][G];
-        __shared__ double shs[4][G];
+        __shared__ float shm[NW][G];
+        __shared__ double shs[NW][G];
 #pragma unroll
         for (int g = 0; g < G; ++g) {
             const float t = wave_max(mx[g]);
@@ -125,10 +125,12 @@ __global__ void __launch_bounds__(256) k_attn_nf_list(const tdesc q, const tdesc
         double sum[G];
 #pragma unroll
         for (int g = 0; g < G; ++g) {
-            mx[g] = fmaxf(fmaxf(shm[0][g], shm[1][g]), fmaxf(shm[2][g], shm[3][g]));
+            mx[g] = shm[0][g];
+#pragma unroll
+            for (int w = 1; w < NW; ++w) mx[g] = fmaxf(mx[g], shm[w][g]);
             sum[g] = 0.0;
         }
-        for (int c = tid; c < cnt; c += 256) {
+        for (int c = tid; c < cnt; c += NT) {
 #pragma unroll
             for (int g = 0; g < G; ++g) {
                 const float e = expf(p_s[g * NF_CAP + c] - mx[g]);
@@ -144,46 +146,48 @@ __global__ void __launch_bounds__(256) k_attn_nf_list(const tdesc q, const tdesc
         __syncthreads();
 #pragma unroll
         for (int g = 0; g < G; ++g) {
-            double t = ((shs[0][g] + shs[1][g]) + shs[2][g]) + shs[3][g];
+            double t = shs[0][g];
+#pragma unroll
+            for (int w = 1; w < NW; ++w) t += shs[w][g];
             if (isnan(t) || t == 0.0) t = -INFINITY;
             const float inv = (float) (1.0 / t);
-            for (int c = tid; c < cnt; c += 256) p_s[g * NF_CAP + c] = h2f(f2h(p_s[g * NF_CAP + c] * inv));
+            for (int c = tid; c < cnt; c += NT) p_s[g * NF_CAP + c] = h2f(f2h(p_s[g * NF_CAP + c] * inv));
         }
         __syncthreads();
         // 3. V^T.p: lanes take cells (4 per lane and group of 256), a wave takes RB rows of the transposed cache at a time — all RB x 4 two-byte
         // loads of a block are requested before the first is used (one row pair at a time, each trip waited for its own loads: 16 round
         // trips per wave were 30 of the launch's 52 us)
         auto vtp = [&](auto rb_tag) {
-        constexpr int RB = decltype(rb_tag)::value;
-        for (int r0 = wave * RB; r0 < rows_per; r0 += 4 * RB) {
+        constexpr int RB = decltype(rb_tag)::value, J = NW == 4 ? 4 : 16 / RB;  // cells a lane takes per trip
+        for (int r0 = wave * RB; r0 < rows_per; r0 += NW * RB) {
             float acc[RB][G];
 #pragma unroll
             for (int r = 0; r < RB; ++r)
 #pragma unroll
                 for (int g = 0; g < G; ++g) acc[r][g] = 0.0f;
             const char * vr0 = vbase + (int64_t) (d0 + r0) * v.nb[1];
-            for (int cg = 0; cg < cnt; cg += 256) {
-                int64_t o[4];
-                float pp[G][4];
+            for (int cg = 0; cg < cnt; cg += 64 * J) {
+                int64_t o[J];
+                float pp[G][J];
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
+                for (int j = 0; j < J; ++j) {
                     const int c = cg + lane + 64 * j;
                     const bool in = c < cnt;
                     o[j] = in ? (int64_t) pos_s[c] * 2 : (int64_t) pos_s[0] * 2;
 #pragma unroll
                     for (int g = 0; g < G; ++g) pp[g][j] = in ? p_s[g * NF_CAP + c] : 0.0f;
                 }
-                uint16_t xv[RB][4];
+                uint16_t xv[RB][J];
 #pragma unroll
                 for (int r = 0; r < RB; ++r) {
                     const char * vr = vr0 + (int64_t) min(r, rows_per - 1 - r0) * v.nb[1];
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) xv[r][j] = *(const uint16_t *) (vr + o[j]);
+                    for (int j = 0; j < J; ++j) xv[r][j] = *(const uint16_t *) (vr + o[j]);
                 }
 #pragma unroll
                 for (int r = 0; r < RB; ++r)
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) {
+                    for (int j = 0; j < J; ++j) {
                         const float x = h2f(xv[r][j]);
 #pragma unroll
                         for (int g = 0; g < G; ++g) acc[r][g] = fmaf(x, pp[g][j], acc[r][g]);
@@ -206,7 +210,7 @@ __global__ void __launch_bounds__(256) k_attn_nf_list(const tdesc q, const tdesc
         // instructions is what matters: at 128 + 72 cells a wave issues 8 + 36 of them instead of 128, and a lane owns its row's sums (no
         // 64-lane reductions).  Waves 0 / 1 take the even groups of rows 0..63 / 64..127, waves 2 / 3 the odd groups; the halves meet in LDS.
         // One slice of the head dimensions and at most 512 cells (64 groups: one ballot); the form above serves the rest.
-        if (dq_n == 1 && cnt <= 512 && nf_groups) {
+        if (NW == 4 && dq_n == 1 && cnt <= 512 && nf_groups) {
             const int ngr = (cnt + 7) / 8, gi_l = lane;
             const bool in = gi_l < ngr;
             const int p_first = pos_s[min(8 * gi_l, cnt - 1)], p_last = pos_s[min(8 * gi_l + 7, cnt - 1)];
@@ -283,7 +287,11 @@ __global__ void __launch_bounds__(256) k_attn_nf_list(const tdesc q, const tdesc
             finish();
             return;
         }
-        if (G <= 4 && rows_per >= 64) vtp(std::integral_constant<int, 16>{});
+        if constexpr (NW == 8) {  // (two slices and more: 64 rows at the most, two to eight a wave, sixteen loads a row group in flight)
+            if (rows_per >= 64) vtp(std::integral_constant<int, 8>{});
+            else if (rows_per >= 32) vtp(std::integral_constant<int, 4>{});
+            else vtp(std::integral_constant<int, 2>{});
+        } else if (G <= 4 && rows_per >= 64) vtp(std::integral_constant<int, 16>{});
         else if (rows_per >= 32) vtp(std::integral_constant<int, 8>{});
         else vtp(std::integral_constant<int, 4>{});
         finish();
@@ -303,7 +311,7 @@ __global__ void __launch_bounds__(256) k_attn_nf_list(const tdesc q, const tdesc
             for (int i = 0; i < 8; ++i) qf[g][i] = h2f(f2h(t[i]));
         }
         const char * kbase = k.data + (int64_t) kvh * k.nb[2] + sl * 16;
-        for (int c0 = wave * 4; c0 < cnt; c0 += 16) {
+        for (int c0 = wave * 4; c0 < cnt; c0 += 4 * NW) {
             const int c = min(c0 + sub, cnt - 1);
             const uint4 kr = *(const uint4 *) (kbase + (int64_t) pos[c] * k.nb[1]);
             const uint32_t u[4] = {kr.x, kr.y, kr.z, kr.w};
@@ -330,7 +338,7 @@ __global__ void __launch_bounds__(256) k_attn_nf_list(const tdesc q, const tdesc
     for (int g = 0; g < G; ++g) {
         float * row = sc + (int64_t) g * n_kv;
         float mx = -INFINITY;
-        for (int c = tid; c < cnt; c += 256) {
+        for (int c = tid; c < cnt; c += NT) {
             float w = row[c] * scale;
             w += m16 ? h2f(((const uint16_t *) mrow)[pos[c]]) : ((const float *) mrow)[pos[c]];
             row[c] = w;
@@ -340,9 +348,11 @@ __global__ void __launch_bounds__(256) k_attn_nf_list(const tdesc q, const tdesc
         __syncthreads();
         if (lane == 0) shf[wave] = mx;
         __syncthreads();
-        mx = fmaxf(fmaxf(shf[0], shf[1]), fmaxf(shf[2], shf[3]));
+        mx = shf[0];
+#pragma unroll
+        for (int w = 1; w < NW; ++w) mx = fmaxf(mx, shf[w]);
         double sum = 0.0;
-        for (int c = tid; c < cnt; c += 256) {
+        for (int c = tid; c < cnt; c += NT) {
             const float e = expf(row[c] - mx);
             row[c] = e;
             sum += (double) e;
@@ -351,15 +361,17 @@ __global__ void __launch_bounds__(256) k_attn_nf_list(const tdesc q, const tdesc
         __syncthreads();
         if (lane == 0) shd[wave] = sum;
         __syncthreads();
-        sum = ((shd[0] + shd[1]) + shd[2]) + shd[3];
+        sum = shd[0];
+#pragma unroll
+        for (int w = 1; w < NW; ++w) sum += shd[w];
         if (isnan(sum) || sum == 0.0) sum = -INFINITY;
         const float inv = (float) (1.0 / sum);
-        for (int c = tid; c < cnt; c += 256) row[c] = h2f(f2h(row[c] * inv));
+        for (int c = tid; c < cnt; c += NT) row[c] = h2f(f2h(row[c] * inv));
     }
     __threadfence_block();
     __syncthreads();
     // ---- 3. V^T.p: wave w takes rows d0 + w, d0 + w + 4, ..; lanes take listed cells
-    for (int r = wave; r < rows_per; r += 4) {
+    for (int r = wave; r < rows_per; r += NW) {
         const int d = d0 + r;
         const char * vrow = vbase + (int64_t) d * v.nb[1];
         float acc[G];
@@ -410,9 +422,15 @@ bool launch_attn_nf_list(hipStream_t s, const tdesc & q, const tdesc & k, const 
     if (q8_out && (dq != 1 || (G & 1))) return false;  // Q8_K blocks are head pairs of whole rows
     static const int groups_on = !getenv("GGML_MI355X_NF_GROUPS") || atoi(getenv("GGML_MI355X_NF_GROUPS")) != 0;
     dim3 grid((unsigned) q.ne[1], (unsigned) k.ne[2], (unsigned) dq);
-#define NF(G_) case G_: hipLaunchKernelGGL(k_attn_nf_list<G_>, grid, dim3(256), (size_t) (G_ * 128 + NF_CAP + G_ * NF_CAP) * 4, s, q, k, v, mask, dst, lists, list_stride, scratch, scale, dq, (q8k_dev *) q8_out, groups_on); return true;
+    // Few tokens: every slice of the head dimensions computes ALL the logits of its heads, one wave a SIMD, and that is most of the launch.  While the grid is no more than
+    // one workgroup a CU, eight waves share the logits and the gathers (3 tokens x 700 cells of Llama-3-8B: 26.5 -> 19.5 us a launch; with sixteen waves, 128 registers
+    // and spills, 29.2); more workgroups than that already have the company of another (20 tokens: a step of 3.9 ms with four waves, 4.0 with eight).
+    const bool few = dq > 1 && q.ne[1] * k.ne[2] * dq <= 256;
+#define NF_GO(G_, W_) hipLaunchKernelGGL((k_attn_nf_list<G_, W_>), grid, dim3(W_ * 64), (size_t) (G_ * 128 + NF_CAP + G_ * NF_CAP) * 4, s, q, k, v, mask, dst, lists, list_stride, scratch, scale, dq, (q8k_dev *) q8_out, groups_on)
+#define NF(G_) case G_: if (few) NF_GO(G_, 8); else NF_GO(G_, 4); return true;
     switch (G) { NF(1) NF(2) NF(3) NF(4) NF(5) NF(6) NF(7) NF(8) default: break; }
 #undef NF
+#undef NF_GO
     return false;
 }
 

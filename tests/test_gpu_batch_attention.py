@@ -2,6 +2,7 @@
 import numpy as np
 import pytest
 
+import harness as T
 import llama_box_amd as L
 from test_gpu_nigozen import attention_case
 
@@ -20,3 +21,39 @@ def test_prompt_attention_at_block_edges(backend, H, n_q, n_kv, heads, kv_heads,
     v = rng.standard_normal((n_kv, kv_heads, dv)).astype(np.float32)
     got, ref = attention_case(backend, H, L.BF16, n_q, n_kv, heads, kv_heads, dk, dv, chunk, sink, q, k, v, np.arange(n_kv - n_q, n_kv))
     assert np.abs(got - ref).max() <= 2e-5 * max(1.0, np.abs(ref).max())
+
+
+# two tokens (eight slices of a head's dimensions) to more workgroups than CUs; lists of one cell, ragged, a full eight-wave trip and more than fit the chip's memory
+@pytest.mark.parametrize("T_,NKV,G,per", [(2, 2, 4, 1), (3, 8, 4, 700), (5, 2, 7, 513), (2, 8, 8, 1024), (3, 4, 1, 1100), (16, 8, 2, 70), (17, 8, 4, 100)])
+def test_few_tokens_over_listed_cells(backend, H, T_, NKV, G, per):
+    """K.q -> SOFT_MAX -> V^T.p of a few tokens over scattered cells (attn_nf.hip), against float64 with the chain's two f16 roundings (queries, probabilities):
+    sums of at most 1100 products in f32, and a probability next to a rounding boundary may round the other way: 2^-11 of it."""
+    rng = np.random.default_rng(T_ + 31 * per + G)
+    HD, NH = 128, NKV * G
+    n_kv = min(max(256, (T_ * per + 255) // 256 * 256), 1024 * T_)  # (more cells a token: another route)
+    k = rng.standard_normal((n_kv, NKV, HD)).astype(np.float16)
+    v = rng.standard_normal((NKV, HD, n_kv)).astype(np.float16)
+    q = rng.standard_normal((T_, NH, HD)).astype(np.float32)
+    mask = np.full((T_, n_kv), -np.inf, np.float32)
+    for t in range(T_):
+        mask[t, rng.choice(n_kv, per - t % min(per, 3), replace=False)] = 0
+
+    def build(g):
+        kc, vc = g.new(L.F16, [NKV * HD, n_kv], k.reshape(n_kv, -1)), g.new(L.F16, [n_kv, NKV * HD], v.reshape(-1, n_kv))
+        qp = H.ggml_permute(g.ctx, g.new(L.F32, [HD, NH, T_], q), 0, 2, 1, 3)
+        kv = H.ggml_view_3d(g.ctx, kc, HD, n_kv, NKV, NKV * HD * 2, HD * 2, 0)
+        vv = H.ggml_view_3d(g.ctx, vc, n_kv, HD, NKV, n_kv * 2, n_kv * 2 * HD, 0)
+        p = H.ggml_soft_max_ext(g.ctx, H.ggml_mul_mat(g.ctx, kv, qp), g.new(L.F32, [n_kv, T_], mask), HD ** -0.5, 0.0)
+        return H.ggml_mul_mat(g.ctx, vv, p)
+
+    s0 = backend.stat("kernel_launches")
+    got = T.run_case(build, backend)[0].reshape(NH, T_, HD)
+    launches = backend.stat("kernel_launches") - s0
+    assert launches <= 2, launches  # (the lists and the chain)
+    qh = q.astype(np.float16).astype(np.float64)
+    for h in range(NH):
+        s = qh[:, h] @ k[:, h // G].astype(np.float64).T * HD ** -0.5 + mask
+        p = np.exp(s - s.max(1, keepdims=True))
+        p = (p / p.sum(1, keepdims=True)).astype(np.float16).astype(np.float64)
+        ref = p @ v[h // G].astype(np.float64).T
+        assert np.abs(got[h] - ref).max() <= 2e-3 * np.abs(ref).max() + 1e-5, h
