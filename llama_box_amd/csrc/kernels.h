@@ -272,6 +272,7 @@ void launch_swiglu(hipStream_t s, const tdesc & a, const tdesc * b, const tdesc 
 struct splitk_src { const float * part; int ks; int64_t mn; const float * add; int64_t add_stride; float * out; int64_t out_stride; };
 void launch_splitk_rms_norm_mul_quantize(hipStream_t s, const splitk_src & sk, int rows, int K, const float * w, float eps, void * dst);
 void launch_rms_norm_mul_quantize(hipStream_t s, const tdesc & x, const float * w, float eps, void * dst_q8k);
+void launch_quantize_heads(hipStream_t s, const tdesc & x, void * dst);  // [128, tokens, heads (even)] contiguous f32 -> Q8_K rows [128 x heads] of the tokens
 void launch_swiglu_quantize(hipStream_t s, const tdesc & a, const tdesc * b, int64_t nc, int swapped, void * dst_q8k);
 void launch_cpy(hipStream_t s, const tdesc & src, const tdesc & dst);
 void launch_concat(hipStream_t s, const tdesc & a, const tdesc & b, const tdesc & dst, int dim);  // f32, any strides

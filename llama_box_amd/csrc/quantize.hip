@@ -163,6 +163,18 @@ void launch_swiglu_quantize(hipStream_t s, const tdesc & a, const tdesc * b, int
     hipLaunchKernelGGL(k_swiglu_q8_K, dim3((unsigned) ((total + 3) / 4)), dim3(256), 0, s, pa, pb, a.nb[1], b ? b->nb[1] : a.nb[1], nb, total, (q8k_dev *) dst);
 }
 
+// [128, tokens, heads] f32 -> Q8_K rows of the token-major copy [128 x heads, tokens]: a block is two heads of one token
+__global__ void __launch_bounds__(64) k_quantize_heads_q8_K(const char * __restrict__ src, const int64_t nb1, const int64_t nb2, const int nb_per_row, q8k_dev * __restrict__ dst) {
+    const int lane = threadIdx.x, row = (int) blockIdx.x / nb_per_row, ib = (int) blockIdx.x - row * nb_per_row;
+    const float4 a = ((const float4 *) (src + (int64_t) row * nb1 + (int64_t) (2 * ib + (lane >> 5)) * nb2))[lane & 31];
+    const float t[4] = {a.x, a.y, a.z, a.w};
+    wave_quantize_q8_K(t, lane, dst + blockIdx.x);
+}
+void launch_quantize_heads(hipStream_t s, const tdesc & x, void * dst) {
+    const int nb = (int) (x.ne[2] / 2);
+    hipLaunchKernelGGL(k_quantize_heads_q8_K, dim3((unsigned) (x.ne[1] * nb)), dim3(64), 0, s, x.data, x.nb[1], x.nb[2], nb, (q8k_dev *) dst);
+}
+
 size_t quantized_act_bytes(int kind, int64_t K, int64_t rows) {
     if (kind == GGML_TYPE_Q8_K) return (size_t) rows * (size_t) (K / 256) * sizeof(q8k_dev);
     return (size_t) rows * (size_t) (K / 32) * sizeof(q80_dev);
