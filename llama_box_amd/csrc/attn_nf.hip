@@ -64,7 +64,7 @@ __global__ void __launch_bounds__(NW * 64) k_attn_nf_list(const tdesc q, const t
     const char * mrow = mask.data + (int64_t) tok * mask.nb[1];
     const bool m16 = mask.type == GGML_TYPE_F16;
     const char * vbase = v.data + (int64_t) kvh * v.nb[2];
-    // ---- up to NF_CAP visible cells (every -np decode step): everything stays on chip.  A thread owns cells tid, tid + 256, ..: it reads
+    // ---- up to NF_CAP visible cells (every -np decode step): everything stays on chip.  A thread owns cells tid, tid + NT, ..: it reads
     // their K rows whole (16 independent 16-byte loads, the q rows come from LDS by broadcast), so a logit needs no cross-lane sum and
     // the soft-max runs on registers; probabilities and positions go to LDS for step 3.  (The first version walked the list with one
     // dependent load pair per trip in every phase: 102 us per launch, all of it memory latency.)
