@@ -1170,13 +1170,25 @@ static const ggml_tensor * through_views(const ggml_tensor * t);
 // ------------------------------------------------------------------------------------------------ batches: sibling mat-muls
 // A batch's wq / wk / wv (and ffn_gate / ffn_up) multiply the same activations.  Launched one by one, the small ones cannot
 // fill the chip without a K split and its second kernel; as ONE launch over the concatenated row panels they can (mmq_i8.hip).
-// The siblings that follow node i in the graph are executed EARLY, at node i: legal when nothing between node i and a
-// sibling's own position reads or occupies the memory the sibling's result is written to (the graph allocator may have given
-// it a block that an earlier tensor still owns at node i's time).  Bias / residual ADDs directly after a member ride in its store.
+// The siblings that follow node i in the graph are executed EARLY, at node i, where may_run_early allows it (the graph allocator
+// may have given a result a block that an earlier tensor still owns at node i's time).  Bias / residual ADDs directly after a member ride in its store.
 static bool ranges_overlap(const ggml_tensor * x, const ggml_tensor * y) {
     if (!x->data || !y->data) return false;
     const char * x0 = (const char *) x->data, * y0 = (const char *) y->data;
     return x0 < y0 + ggml_abi_nbytes(y) && y0 < x0 + ggml_abi_nbytes(x);
+}
+// May the sibling mat-mul t (node k), whose result goes to dst, run at node i's place?  Its result must not sit in memory that node i or one in between still uses (the block
+// of a matrix that node i is the last to read, say), and what it reads must already be what it is at node k: a matrix that the graph itself writes on the way (a cast, rows of a
+// cache) or an input changed in place is not.  member(j): node j is part of the launch.
+template <class F> static bool may_run_early(const exec_state & st, int i, int k, const ggml_tensor * t, const ggml_tensor * dst, F member) {
+    for (int j = i; j < k; ++j) {
+        const ggml_tensor * u = st.g->nodes[j];
+        if (!is_view_op(u) && !st.done[j] && (ranges_overlap(u, t->src[0]) || ranges_overlap(u, t->src[1]))) return false;
+        if (j > i && !is_view_op(u) && !member(j) && ranges_overlap(dst, u)) return false;
+        for (int sidx = 0; sidx < (j == i ? 1 : GGML_MAX_SRC); ++sidx)  // (node i's input is t's own: it cannot be gone before t)
+            if (u->src[sidx] && ranges_overlap(dst, u->src[sidx])) return false;
+    }
+    return true;
 }
 static int try_merge_mm_batch(exec_state & st, int i) {  // returns the number of nodes consumed at position i (0: not merged)
     backend_ctx * c = st.c;
@@ -1219,15 +1231,12 @@ static int try_merge_mm_batch(exec_state & st, int i) {  // returns the number o
         bool ok = true;
         for (auto & o : ms) ok = ok && !ranges_overlap(m.dst, o.dst) && !ranges_overlap(m.dst, g->nodes[o.k]);
         for (auto & o : others) ok = ok && !ranges_overlap(m.dst, o.dst) && !ranges_overlap(m.dst, g->nodes[o.k]);
-        for (int j = i + 1; j < k && ok; ++j) {  // everything that runs between node i and the sibling's own position
-            const ggml_tensor * u = g->nodes[j];
+        ok = ok && may_run_early(st, i, k, t, m.dst, [&](int j) {
             bool is_member = false;
             for (auto & o : ms) is_member = is_member || j == o.k || (o.n_nodes == 2 && j == o.k + 1);
             for (auto & o : others) is_member = is_member || j == o.k || (o.n_nodes == 2 && j == o.k + 1);
-            if (!is_view_op(u) && !is_member && ranges_overlap(m.dst, u)) ok = false;
-            for (int sidx = 0; sidx < GGML_MAX_SRC && ok; ++sidx)
-                if (u->src[sidx] && ranges_overlap(m.dst, u->src[sidx])) ok = false;
-        }
+            return is_member;
+        });
         if (ok && m.add && ranges_overlap(m.dst, m.add) && m.add->data != m.dst->data) ok = false;
         if (ok) (same ? ms : others).push_back(m);
     }
@@ -1448,14 +1457,11 @@ static int try_merge_q80_skinny(exec_state & st, int i) {  // returns the number
         const member m = with_add(k);
         bool ok = true;
         for (auto & o : ms) ok = ok && !ranges_overlap(m.dst, o.dst) && !ranges_overlap(m.dst, g->nodes[o.k]);
-        for (int j = i + 1; j < k && ok; ++j) {  // everything that runs between node i and the sibling's own position
-            const ggml_tensor * u = g->nodes[j];
+        ok = ok && may_run_early(st, i, k, t, m.dst, [&](int j) {
             bool is_member = false;
             for (auto & o : ms) is_member = is_member || j == o.k || (o.n_nodes == 2 && j == o.k + 1);
-            if (!is_view_op(u) && !is_member && ranges_overlap(m.dst, u)) ok = false;
-            for (int sidx = 0; sidx < GGML_MAX_SRC && ok; ++sidx)
-                if (u->src[sidx] && ranges_overlap(m.dst, u->src[sidx])) ok = false;
-        }
+            return is_member;
+        });
         if (ok && m.add && ranges_overlap(m.dst, m.add) && m.add->data != m.dst->data) ok = false;
         if (ok) ms.push_back(m);
     }
@@ -1825,8 +1831,7 @@ static bool try_fuse_attn_nf_mma(exec_state & st, int i) {
 }
 
 // Projections of the same activations by bf16 matrices (q, k, v and the gate of a layer): the siblings that follow node i are executed EARLY, at node i,
-// as one launch — legal when nothing between node i and a sibling's own position reads or occupies the memory the sibling's result goes to (the graph
-// allocator may have given it a block that an earlier tensor still owns at node i's time).  Returns true when node i and at least one sibling were served.
+// as one launch (may_run_early).  Returns true when node i and at least one sibling were served.
 // One column, 2 .. 16 and more each have their kernel; all of them give a matrix the bits it gets alone.
 static bool try_merge_mm_16(exec_state & st, int i) {
     backend_ctx * c = st.c;
@@ -1850,14 +1855,7 @@ static bool try_merge_mm_16(exec_state & st, int i) {
         if (st.done[k] || !eligible(t)) continue;
         bool ok = true;
         for (int mi : ms) ok = ok && !ranges_overlap(t, g->nodes[mi]);
-        for (int j = i + 1; j < k && ok; ++j) {  // everything that runs between node i and the sibling's own position
-            const ggml_tensor * u = g->nodes[j];
-            bool member = false;
-            for (int mi : ms) member = member || mi == j;
-            if (!is_view_op(u) && !member && ranges_overlap(t, u)) ok = false;
-            for (int sidx = 0; sidx < GGML_MAX_SRC && ok; ++sidx)
-                if (u->src[sidx] && ranges_overlap(t, u->src[sidx])) ok = false;
-        }
+        ok = ok && may_run_early(st, i, k, t, t, [&](int j) { return std::find(ms.begin(), ms.end(), j) != ms.end(); });
         if (ok) ms.push_back(k);
     }
     if (ms.size() < 2) return false;

@@ -143,11 +143,12 @@ class G:
             self.inputs.append((t, raw))
         return t
 
-    def compute(self, outs, n_threads=4, expand_first=(), cuts=None):
+    def compute(self, outs, n_threads=4, expand_first=(), cuts=None, same_block=()):
         """Allocates every tensor, uploads inputs, evaluates the graph for `outs`, returns numpy copies of `outs`.
         expand_first: tensors added to the graph before the outputs, unflagged (llama.cpp's build_attn expands q, k, v together
         before the cache stores); cuts: node indices at which the graph is handed to the backend in pieces — ggml_graph_view of
-        the full graph, what ggml_backend_sched gives a backend for each of its splits."""
+        the full graph, what ggml_backend_sched gives a backend for each of its splits; same_block: pairs (t, u) of which t is placed
+        at u's address, as the graph allocator does with the block of a tensor that nobody reads any more."""
         H = self.H
         gf = H.ggml_new_graph_custom(self.ctx, 4096, False)
         for o in expand_first:
@@ -166,6 +167,9 @@ class G:
         self.buf = H.ggml_backend_alloc_ctx_tensors_from_buft(self.ctx, buft)
         assert self.buf, "buffer allocation failed"
         H.ggml_backend_buffer_clear(self.buf, 0)
+        for t, u in same_block:
+            assert H.ggml_nbytes(t) <= H.ggml_nbytes(u)
+            t.contents.data = u.contents.data
         for t, raw in self.inputs:
             H.ggml_backend_tensor_set(t, raw.ctypes.data_as(C.c_void_p), 0, raw.nbytes)
         if self.target == "oracle":

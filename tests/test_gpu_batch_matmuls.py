@@ -156,3 +156,70 @@ def test_k_quant_batches_of_33_columns_and_up(backend, H, qt, K, N, M):
     assert T.nmse(got, tiled) <= 1e-12
     rows = np.unique(np.concatenate([np.arange(min(N, 40)), np.arange(max(0, N - 40), N)]))
     assert T.nmse(got[:, rows], run("oracle", np.ascontiguousarray(w[rows]), np.ascontiguousarray(b[:, rows]))) <= 1e-10
+
+
+# one column and more, both sides of the lines between the kernels; matrices that the graph makes: a cast, rows stored into a matrix
+@pytest.mark.parametrize("wt,M", [(L.BF16, 1), (L.BF16, 2), (L.BF16, 17), (L.BF16, 60), (L.F16, 16), (L.F16, 17), (L.F16, 60), (L.Q8_0, 9), (L.Q8_0, 33), (L.Q8_0, 140)])
+@pytest.mark.parametrize("made", ["cast", "rows", "input"])
+def test_siblings_wait_for_what_they_read(backend, H, wt, M, made):
+    """A sibling is run with the first product of its input only if its matrix and the input are then what they are at its own place: the bits of the same graph node by node."""
+    rng = np.random.default_rng(M)
+    K, N = 256, 96
+    w = [(rng.standard_normal((N, K)) / 16).astype(np.float32) for _ in range(2)]
+    x, x2 = rng.standard_normal((M, K)).astype(np.float32), rng.standard_normal((M, K)).astype(np.float32)
+
+    def run():
+        g = T.G(backend)
+        try:
+            xt, first = g.new(L.F32, [K, M], x), []
+
+            def matrix(q):
+                f = g.new(L.F32, [K, N], w[q])
+                if made != "rows":
+                    return H.ggml_cast(g.ctx, f, wt)
+                return H.ggml_set_rows(g.ctx, g.new(wt, [K, N]), f, g.new(L.I64, [N], np.arange(N, dtype=np.int64)))
+
+            ms = [matrix(0), matrix(1)]
+            outs = [H.ggml_mul_mat(g.ctx, ms[0], xt)]
+            if made == "input":  # both matrices are there before the first product, the input's rows change behind it
+                first = [*ms, outs[0], H.ggml_set_rows(g.ctx, xt, g.new(L.F32, [K, M], x2), g.new(L.I64, [M], np.arange(M, dtype=np.int64)))]
+            outs.append(H.ggml_mul_mat(g.ctx, ms[1], xt))
+            return g.compute(outs, expand_first=first)
+        finally:
+            g.free()
+
+    got = run()
+    backend.set_option("fusion", 0)
+    try:
+        plain = run()
+    finally:
+        backend.set_option("fusion", 1)
+    for a, b, wq, xq in zip(got, plain, w, (x, x2 if made == "input" else x)):
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+        assert T.nmse(a.reshape(M, N), xq.astype(np.float64) @ wq.T) < 1e-3  # (8-bit codes of both operands: 1e-4)
+
+
+@pytest.mark.parametrize("wt", [L.BF16, L.F16, L.Q8_0])
+def test_sibling_in_the_block_of_the_first_matrix(backend, H, wt):
+    """The first product is the last reader of its matrix, and the sibling's result got that block: the sibling runs behind it."""
+    rng = np.random.default_rng(3)
+    K, N, M = 1024, 4096, 150
+    w = [(rng.standard_normal((N, K)) / 32).astype(np.float32) for _ in range(2)]
+    x = rng.standard_normal((M, K)).astype(np.float32)
+
+    def run(recycled):
+        g = T.G(backend)
+        try:
+            xt = g.new(L.F32, [K, M], x)
+            ms = [H.ggml_cast(g.ctx, g.new(L.F32, [K, N], v), wt) for v in w]
+            outs = [H.ggml_mul_mat(g.ctx, m, xt) for m in ms]
+            k0 = backend.stat("kernel_launches")
+            r = g.compute(outs, expand_first=ms, same_block=[(outs[1], ms[0])] if recycled else [])
+            return r, backend.stat("kernel_launches") - k0
+        finally:
+            g.free()
+
+    (got, n_got), (plain, n_plain) = run(True), run(False)
+    assert n_got == n_plain + 1, (n_got, n_plain)
+    for a, b in zip(got, plain):
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
