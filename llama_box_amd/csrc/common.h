@@ -192,6 +192,28 @@ struct timing_slot {
     int64_t count = 0;
 };
 
+// A src1 converted into the activation scratch for a mat-mul.  It serves another product of the same memory only if that product reads the same rows: two views may agree in
+// address and extent and differ in their rows' number, length or distance.
+struct act_image {
+    const void * src = nullptr;
+    int kind = 0;
+    size_t bytes = 0;
+    int64_t ne[4] = {};
+    size_t nb[4] = {};
+    void set(const ggml_tensor * t, int k) {
+        src = t->data;
+        kind = k;
+        bytes = ggml_abi_nbytes(t);
+        memcpy(ne, t->ne, sizeof(ne));
+        memcpy(nb, t->nb, sizeof(nb));
+    }
+    bool holds(const ggml_tensor * t, int k) const {
+        if (src != t->data || kind != k || bytes != ggml_abi_nbytes(t) || ne[0] != t->ne[0] || nb[0] != t->nb[0] || nb[1] != t->nb[1]) return false;
+        if (memcmp(ne, t->ne, sizeof(ne)) == 0 && memcmp(nb, t->nb, sizeof(nb)) == 0) return true;
+        // (dense rows, arranged differently over the higher dimensions)
+        return ggml_abi_is_contiguous(t) && ne[1] * ne[2] * ne[3] == t->ne[1] * t->ne[2] * t->ne[3] && nb[2] == nb[1] * (size_t) ne[1] && nb[3] == nb[2] * (size_t) ne[2];
+    }
+};
 struct backend_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -201,11 +223,7 @@ struct backend_ctx {
     // scratch (quantised activations, attention partials); grown outside capture only
     void * ws = nullptr;
     size_t ws_size = 0;
-    // activation-quantisation cache: which src1 tensor the q8 scratch currently holds
-    const void * q8_src = nullptr;
-    int q8_kind = 0;
-    size_t q8_bytes = 0;
-    uint64_t q8_epoch = 0;
+    act_image act;  // what the activation scratch currently holds
     // hipGraph cache
     std::unordered_map<uint64_t, cached_graph> graphs;
     cached_graph * last_graph = nullptr;  // the entry looked up last: compared first, in place (graph.cpp: key_equals)

@@ -315,7 +315,7 @@ static bool ensure_ws(backend_ctx * c, size_t need) {
         return false;
     }
     c->ws_size = sz;
-    c->q8_src = nullptr;
+    c->act.src = nullptr;
     free_graph_cache(c);  // captured graphs hold the old scratch address
     return true;
 }
@@ -550,16 +550,14 @@ static const void * quantized_src1(exec_state & st, const ggml_tensor * b, int w
     backend_ctx * c = st.c;
     const int kind = wtype == MI_ACT_Q80_PANEL ? MI_ACT_Q80_PANEL : act_kind(wtype);
     void * dst = (char *) c->ws + st.act_off;
-    if (c->q8_src == b->data && c->q8_kind == kind && c->q8_bytes == ggml_abi_nbytes(b)) return dst;
+    if (c->act.holds(b, kind)) return dst;
     {
         timed_scope ts(c, "quantize_act", (double) ggml_abi_nbytes(b));
         if (kind == MI_ACT_Q80_PANEL) launch_quantize_q80_panel(c->stream, TD(b), dst);
         else launch_quantize_act(c->stream, kind, TD(b), dst);
         c->st.kernel_launches++;
     }
-    c->q8_src = b->data;
-    c->q8_kind = kind;
-    c->q8_bytes = ggml_abi_nbytes(b);
+    c->act.set(b, kind);
     return dst;
 }
 
@@ -583,15 +581,13 @@ static const void * rounded_src1(exec_state & st, const ggml_tensor * b, int wty
     backend_ctx * c = st.c;
     const int kind = MI_ACT_16 + wtype;
     void * dst = (char *) c->ws + st.act_off;
-    if (c->q8_src == b->data && c->q8_kind == kind && c->q8_bytes == ggml_abi_nbytes(b)) return dst;
+    if (c->act.holds(b, kind)) return dst;
     {
         timed_scope ts(c, "round_act", (double) ggml_abi_nbytes(b));
         launch_to_16(c->stream, wtype, (const char *) b->data, (int64_t) b->nb[1], b->ne[0], b->ne[1] * b->ne[2], dst);
         c->st.kernel_launches++;
     }
-    c->q8_src = b->data;
-    c->q8_kind = kind;
-    c->q8_bytes = ggml_abi_nbytes(b);
+    c->act.set(b, kind);
     return dst;
 }
 
@@ -849,9 +845,7 @@ static bool q80_panel_consumers_only(const exec_state & st, int at, const ggml_t
 }
 static void mark_q8_cache(exec_state & st, const ggml_tensor * t, int kind = GGML_TYPE_Q8_K);
 static void mark_q8_cache(exec_state & st, const ggml_tensor * t, int kind) {
-    st.c->q8_src = t->data;
-    st.c->q8_kind = kind;
-    st.c->q8_bytes = ggml_abi_nbytes(t);
+    st.c->act.set(t, kind);
     st.q8_fresh = true;
 }
 
@@ -3584,7 +3578,7 @@ static bool run_nodes(backend_ctx * c, ggml_cgraph * g, const ws_plan & wp) {
     for (int i = 0; i < g->n_nodes; ++i)
         for (int s = 0; s < GGML_MAX_SRC; ++s)
             if (g->nodes[i]->src[s]) st.uses[g->nodes[i]->src[s]]++;
-    c->q8_src = nullptr;  // inputs change between graph launches
+    c->act.src = nullptr;  // inputs change between graph launches
     st.done.assign((size_t) g->n_nodes, 0);
     for (int i = 0; i < g->n_nodes;) {
         ggml_tensor * n = g->nodes[i];
@@ -3597,8 +3591,8 @@ static bool run_nodes(backend_ctx * c, ggml_cgraph * g, const ws_plan & wp) {
         if (used < 0) return false;
         for (int k = 0; k < used; ++k)  // (mask statistics describe uploaded bytes only: common.h)
             if (!is_view_op(g->nodes[i + k]) && g->nodes[i + k]->data) forget_mask_stats(g->nodes[i + k]->data, ggml_abi_nbytes(g->nodes[i + k]));
-        if (!st.q8_fresh && c->q8_src) {
-            const char * q0 = (const char *) c->q8_src, * q1 = q0 + c->q8_bytes;
+        if (!st.q8_fresh && c->act.src) {
+            const char * q0 = (const char *) c->act.src, * q1 = q0 + c->act.bytes;
             auto hits = [&](const ggml_tensor * t) {
                 if (is_view_op(t) || !t->data) return false;  // (views write nothing)
                 const char * t0 = (const char *) t->data;
@@ -3607,7 +3601,7 @@ static bool run_nodes(backend_ctx * c, ggml_cgraph * g, const ws_plan & wp) {
             bool hit = false;
             for (int k = 0; k < used && !hit; ++k) hit = hits(g->nodes[i + k]);
             for (size_t k = 0; k < st.ooo.size() && !hit; ++k) hit = hits(g->nodes[st.ooo[k]]);
-            if (hit) c->q8_src = nullptr;
+            if (hit) c->act.src = nullptr;
         }
         st.q8_fresh = false;
         i += used;

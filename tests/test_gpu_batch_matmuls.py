@@ -223,3 +223,28 @@ def test_sibling_in_the_block_of_the_first_matrix(backend, H, wt):
     assert n_got == n_plain + 1, (n_got, n_plain)
     for a, b in zip(got, plain):
         assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+
+
+# two views of one address and one extent whose rows are not the same: fewer rows further apart, or half as many rows of twice the length
+@pytest.mark.parametrize("wt", [L.BF16, L.F16, L.Q8_0, L.Q4_K])
+@pytest.mark.parametrize("form", ["stride", "length"])
+def test_inputs_of_one_address_and_extent(backend, H, wt, form):
+    """A converted input is used again for a product over the same rows only: the bits each product has alone."""
+    rng = np.random.default_rng(5)
+    K, N = 256, 96
+    K2 = K if form == "stride" else 2 * K
+    M, M2 = (33, 17) if form == "stride" else (40, 20)
+    ws = [bits16((rng.standard_normal((N, k)) / 16).astype(np.float32), wt) if wt in (L.BF16, L.F16) else T.rand_weight(wt, k, N, rng) for k in (K, K2)]
+    x = rng.standard_normal(40 * 512).astype(np.float32)
+
+    def build(which):
+        def f(g):
+            xt = g.new(L.F32, [x.size], x)
+            v = [H.ggml_view_2d(g.ctx, xt, K, M, K * (8 if form == "stride" else 4), 0), H.ggml_view_2d(g.ctx, xt, K2, M2, K * (16 if form == "stride" else 8), 0)]
+            assert H.ggml_nbytes(v[0]) == H.ggml_nbytes(v[1])
+            return [H.ggml_mul_mat(g.ctx, g.new(wt, [k, N], w), u) for k, w, u, q in zip((K, K2), ws, v, (0, 1)) if q in which]
+        return f
+
+    got = T.run_case(build((0, 1)), backend)
+    for q in (0, 1):
+        assert np.array_equal(got[q].view(np.uint32), T.run_case(build((q,)), backend)[0].view(np.uint32)), q
