@@ -342,6 +342,8 @@ static ws_plan plan_ws(backend_ctx * c, const ggml_cgraph * g) {
     }
     for (int i = 0; i < g->n_nodes; ++i) {
         const ggml_tensor * n = g->nodes[i];
+        // (besides what follows: K.q of one head on one key head has this form, and the attention chain that may start at it has its own scratch)
+        if (n->op == GGML_OP_MUL_MAT && mm_tile_applies(n)) p.act_bytes = std::max(p.act_bytes, (size_t) (n->src[1]->ne[0] * n->src[1]->ne[1]) * 2);
         if (n->op == GGML_OP_MUL_MAT && is_quant(n->src[0]->type)) {
             const ggml_tensor * b = n->src[1];
             const int64_t Mc = b->ne[1] * b->ne[2] * b->ne[3];
@@ -352,8 +354,6 @@ static ws_plan plan_ws(backend_ctx * c, const ggml_cgraph * g) {
         } else if (n->op == GGML_OP_MUL_MAT && mm_cache_image_ok(n) && !buffer_is_split(n->src[0]->buffer)) {
             const tdesc a16 = kv_image_desc(TD(n->src[0]), nullptr);
             p.aux_bytes = std::max(p.aux_bytes, ((mul_mat_f_workspace_bytes(a16, TD(n->src[1])) + 255) & ~(size_t) 255) + kv_image_bytes(a16));
-        } else if (n->op == GGML_OP_MUL_MAT && mm_tile_applies(n)) {
-            p.act_bytes = std::max(p.act_bytes, (size_t) (n->src[1]->ne[0] * n->src[1]->ne[1]) * 2);
         } else if (n->op == GGML_OP_MUL_MAT && n->src[0]->type == GGML_TYPE_F16) {
             p.aux_bytes = std::max(p.aux_bytes, mul_mat_f_workspace_bytes(TD(n->src[0]), TD(n->src[1])));
             if (c->opt.attn_nf) p.aux_bytes = std::max(p.aux_bytes, attn_nf_list_scratch_bytes(TD(n->src[1]), TD(n->src[0]), nullptr));

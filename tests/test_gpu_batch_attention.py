@@ -89,3 +89,34 @@ def test_few_tokens_feed_a_quantised_matrix(backend, H, T_, NKV, G, per):
     finally:
         backend.set_option("fusion", 1)
     assert T.nmse(got, plain) <= 1e-5
+
+
+@pytest.mark.parametrize("T_,n_kv", [(32, 32768), (512, 16384)])
+def test_one_head_over_one_key_head(H, T_, n_kv):
+    """K.q -> SOFT_MAX -> V^T.p with one query head on one key head: plain 2-D products by their shapes, and the chain's scratch is there for them too (more of it than a new
+    backend's first allocation leaves over).  Against float64 with the chain's two f16 roundings: 2^-11 of a probability next to a rounding boundary."""
+    rng = np.random.default_rng(T_)
+    HD, backend = 128, L.Backend(0)
+    k, v = rng.standard_normal((n_kv, HD)).astype(np.float16), rng.standard_normal((HD, n_kv)).astype(np.float16)
+    q = rng.standard_normal((T_, 1, HD)).astype(np.float32)
+    mask = np.full((T_, n_kv), -np.inf, np.float32)
+    for t in range(T_):
+        mask[t, rng.choice(n_kv, 40, replace=False)] = 0
+
+    def build(g):
+        kc, vc = g.new(L.F16, [HD, n_kv], k), g.new(L.F16, [n_kv, HD], v)
+        qp = H.ggml_permute(g.ctx, g.new(L.F32, [HD, 1, T_], q), 0, 2, 1, 3)
+        kv, vv = H.ggml_view_3d(g.ctx, kc, HD, n_kv, 1, HD * 2, HD * 2, 0), H.ggml_view_3d(g.ctx, vc, n_kv, HD, 1, n_kv * 2, n_kv * 2 * HD, 0)
+        p = H.ggml_soft_max_ext(g.ctx, H.ggml_mul_mat(g.ctx, kv, qp), g.new(L.F32, [n_kv, T_], mask), HD ** -0.5, 0.0)
+        return H.ggml_mul_mat(g.ctx, vv, p)
+
+    try:
+        f0 = backend.stat("fused_nodes")
+        got = T.run_case(build, backend)[0].reshape(T_, HD)
+        assert backend.stat("fused_nodes") == f0 + 2  # (the soft-max and the second product)
+    finally:
+        backend.close()
+    s = q[:, 0].astype(np.float16).astype(np.float64) @ k.astype(np.float64).T * HD ** -0.5 + mask
+    p = np.exp(s - s.max(1, keepdims=True))
+    ref = (p / p.sum(1, keepdims=True)).astype(np.float16).astype(np.float64) @ v.astype(np.float64).T
+    assert np.abs(got - ref).max() <= 2e-3 * np.abs(ref).max() + 1e-5
