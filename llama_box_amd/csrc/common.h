@@ -223,7 +223,7 @@ struct backend_ctx {
     // scratch (quantised activations, attention partials); grown outside capture only
     void * ws = nullptr;
     size_t ws_size = 0;
-    act_image act;  // what the activation scratch currently holds
+    act_image act, act16;  // what the activation scratch currently holds: a quantised src1, one rounded to 16 bits
     // hipGraph cache
     std::unordered_map<uint64_t, cached_graph> graphs;
     cached_graph * last_graph = nullptr;  // the entry looked up last: compared first, in place (graph.cpp: key_equals)

@@ -315,13 +315,14 @@ static bool ensure_ws(backend_ctx * c, size_t need) {
         return false;
     }
     c->ws_size = sz;
-    c->act.src = nullptr;
+    c->act.src = c->act16.src = nullptr;
     free_graph_cache(c);  // captured graphs hold the old scratch address
     return true;
 }
 
 struct ws_plan {
     size_t act_bytes = 0;  // region A: quantised activations
+    size_t act16_bytes = 0;  // ... and activations rounded to 16 bits (an input of both kinds of matrices is converted once for each)
     size_t aux_bytes = 0;  // region B: attention partials
 };
 
@@ -343,7 +344,7 @@ static ws_plan plan_ws(backend_ctx * c, const ggml_cgraph * g) {
     for (int i = 0; i < g->n_nodes; ++i) {
         const ggml_tensor * n = g->nodes[i];
         // (besides what follows: K.q of one head on one key head has this form, and the attention chain that may start at it has its own scratch)
-        if (n->op == GGML_OP_MUL_MAT && mm_tile_applies(n)) p.act_bytes = std::max(p.act_bytes, (size_t) (n->src[1]->ne[0] * n->src[1]->ne[1]) * 2);
+        if (n->op == GGML_OP_MUL_MAT && mm_tile_applies(n)) p.act16_bytes = std::max(p.act16_bytes, (size_t) (n->src[1]->ne[0] * n->src[1]->ne[1]) * 2);
         if (n->op == GGML_OP_MUL_MAT && is_quant(n->src[0]->type)) {
             const ggml_tensor * b = n->src[1];
             const int64_t Mc = b->ne[1] * b->ne[2] * b->ne[3];
@@ -362,7 +363,7 @@ static ws_plan plan_ws(backend_ctx * c, const ggml_cgraph * g) {
                 p.aux_bytes = std::max(p.aux_bytes, attn_nf_mma_ws_bytes(TD(n->src[1]), fattn_mma_pick_splits(TD(n->src[1]), TD(n->src[0]))));
         } else if (n->op == GGML_OP_MUL_MAT_ID && n->src[2]) {
             p.aux_bytes = std::max(p.aux_bytes, mul_mat_id_workspace_bytes(TD(n->src[0]), TD(n->src[2])));
-            if (mm_id_tile_applies(n)) p.act_bytes = std::max(p.act_bytes, (size_t) ggml_abi_nelements(n->src[1]) * 2);
+            if (mm_id_tile_applies(n)) p.act16_bytes = std::max(p.act16_bytes, (size_t) ggml_abi_nelements(n->src[1]) * 2);
         } else if (n->op == GGML_OP_GATED_LINEAR_ATTN && n->op_params[3] == MI_SEQ_OP_TAG && (n->op_params[0] == SEQ_DELTA_CH || n->op_params[0] == SEQ_LINEAR) && n->src[0] && n->src[3]) {
             p.aux_bytes = std::max(p.aux_bytes, seq_recurrence_scratch_bytes(n->op_params[0], n->op_params[1], (int) (n->src[0]->ne[0] / std::max(1, n->op_params[2])), n->src[3]->ne[1]));
         } else if (n->op == GGML_OP_FLASH_ATTN_EXT && fa_route(n) == 4) {
@@ -382,6 +383,7 @@ static ws_plan plan_ws(backend_ctx * c, const ggml_cgraph * g) {
         }
     }
     p.act_bytes = (p.act_bytes + 255) & ~(size_t) 255;
+    p.act16_bytes = (p.act16_bytes + 255) & ~(size_t) 255;
     return p;
 }
 
@@ -457,7 +459,7 @@ struct exec_state {
     ggml_cgraph * g;
     std::unordered_map<const ggml_tensor *, int> uses;
     mutable std::unordered_map<const ggml_tensor *, int> uses_global;  // memo of graph_use_count()
-    size_t act_off = 0, aux_off = 0;
+    size_t act_off = 0, act16_off = 0, aux_off = 0;
     // [RMS_NORM -> MUL] pairs whose result is consumed only by single-column K-quant mat-vecs: nothing is launched
     // for them; each consumer recomputes norm*w in its prologue (mmvq.hip PRO=2)
     std::unordered_map<const ggml_tensor *, deferred_norm> deferred;
@@ -580,14 +582,14 @@ static bool mm_id_tile_applies(const ggml_tensor * n) {
 static const void * rounded_src1(exec_state & st, const ggml_tensor * b, int wtype) {
     backend_ctx * c = st.c;
     const int kind = MI_ACT_16 + wtype;
-    void * dst = (char *) c->ws + st.act_off;
-    if (c->act.holds(b, kind)) return dst;
+    void * dst = (char *) c->ws + st.act16_off;
+    if (c->act16.holds(b, kind)) return dst;
     {
         timed_scope ts(c, "round_act", (double) ggml_abi_nbytes(b));
         launch_to_16(c->stream, wtype, (const char *) b->data, (int64_t) b->nb[1], b->ne[0], b->ne[1] * b->ne[2], dst);
         c->st.kernel_launches++;
     }
-    c->act.set(b, kind);
+    c->act16.set(b, kind);
     return dst;
 }
 
@@ -810,7 +812,7 @@ static bool quant_consumers_only(const exec_state & st, int at, const ggml_tenso
     if (n_cons == 0 || n_cons != use_count(st, t)) return false;
     for (int j = at + 1; j <= last; ++j) {
         const ggml_tensor * u = g->nodes[j];
-        if (u->op == GGML_OP_MUL_MAT && (is_quant(u->src[0]->type) || mm_tile_applies(u)) && u->src[1] != t) return false;
+        if (u->op == GGML_OP_MUL_MAT && is_quant(u->src[0]->type) && u->src[1] != t) return false;
         if (u->op == GGML_OP_MUL_MAT_ID) return false;
     }
     return true;
@@ -838,7 +840,7 @@ static bool q80_panel_consumers_only(const exec_state & st, int at, const ggml_t
     if (n_cons == 0 || n_cons != use_count(st, t)) return false;
     for (int j = at + 1; j <= last; ++j) {  // (the activation area is shared: no other quantised mat-mul may run before the last reader)
         const ggml_tensor * u = g->nodes[j];
-        if (u->op == GGML_OP_MUL_MAT && (is_quant(u->src[0]->type) || mm_tile_applies(u)) && u->src[1] != t) return false;
+        if (u->op == GGML_OP_MUL_MAT && is_quant(u->src[0]->type) && u->src[1] != t) return false;
         if (u->op == GGML_OP_MUL_MAT_ID) return false;
     }
     return true;
@@ -3573,12 +3575,13 @@ static bool run_nodes(backend_ctx * c, ggml_cgraph * g, const ws_plan & wp) {
     exec_state st{};
     st.c = c;
     st.g = g;
-    st.aux_off = wp.act_bytes;
+    st.act16_off = wp.act_bytes;
+    st.aux_off = wp.act_bytes + wp.act16_bytes;
     st.uses.reserve((size_t) g->n_nodes * 2);
     for (int i = 0; i < g->n_nodes; ++i)
         for (int s = 0; s < GGML_MAX_SRC; ++s)
             if (g->nodes[i]->src[s]) st.uses[g->nodes[i]->src[s]]++;
-    c->act.src = nullptr;  // inputs change between graph launches
+    c->act.src = c->act16.src = nullptr;  // inputs change between graph launches
     st.done.assign((size_t) g->n_nodes, 0);
     for (int i = 0; i < g->n_nodes;) {
         ggml_tensor * n = g->nodes[i];
@@ -3591,18 +3594,21 @@ static bool run_nodes(backend_ctx * c, ggml_cgraph * g, const ws_plan & wp) {
         if (used < 0) return false;
         for (int k = 0; k < used; ++k)  // (mask statistics describe uploaded bytes only: common.h)
             if (!is_view_op(g->nodes[i + k]) && g->nodes[i + k]->data) forget_mask_stats(g->nodes[i + k]->data, ggml_abi_nbytes(g->nodes[i + k]));
-        if (!st.q8_fresh && c->act.src) {
-            const char * q0 = (const char *) c->act.src, * q1 = q0 + c->act.bytes;
+        auto written = [&](const act_image & im) {
+            const char * q0 = (const char *) im.src, * q1 = q0 + im.bytes;
             auto hits = [&](const ggml_tensor * t) {
                 if (is_view_op(t) || !t->data) return false;  // (views write nothing)
                 const char * t0 = (const char *) t->data;
                 return t0 < q1 && q0 < t0 + ggml_abi_nbytes(t);
             };
-            bool hit = false;
-            for (int k = 0; k < used && !hit; ++k) hit = hits(g->nodes[i + k]);
-            for (size_t k = 0; k < st.ooo.size() && !hit; ++k) hit = hits(g->nodes[st.ooo[k]]);
-            if (hit) c->act.src = nullptr;
-        }
+            for (int k = 0; k < used; ++k)
+                if (hits(g->nodes[i + k])) return true;
+            for (int k : st.ooo)
+                if (hits(g->nodes[k])) return true;
+            return false;
+        };
+        if (!st.q8_fresh && c->act.src && written(c->act)) c->act.src = nullptr;
+        if (c->act16.src && written(c->act16)) c->act16.src = nullptr;
         st.q8_fresh = false;
         i += used;
     }
@@ -3746,7 +3752,7 @@ enum ggml_status graph_compute(backend_ctx * c, ggml_cgraph * g) {
         if (handled) return st_ip;
     }
     const ws_plan wp = plan_ws(c, g);
-    if (!ensure_ws(c, wp.act_bytes + wp.aux_bytes + 256)) return GGML_STATUS_ALLOC_FAILED;
+    if (!ensure_ws(c, wp.act_bytes + wp.act16_bytes + wp.aux_bytes + 256)) return GGML_STATUS_ALLOC_FAILED;
     bool has_split = false;  // multi-device launches + peer copies: executed eagerly (capture across devices is left for a box that has them)
     for (int i = 0; i < g->n_nodes && !has_split; ++i) has_split = g->nodes[i]->op == GGML_OP_MUL_MAT && buffer_is_split(g->nodes[i]->src[0]->buffer);
     // (graphs that launch on several devices' streams: captured only on request — GGML_MI355X_SPLIT_GRAPHS=1 — until that has run on a box

@@ -248,3 +248,32 @@ def test_inputs_of_one_address_and_extent(backend, H, wt, form):
     got = T.run_case(build((0, 1)), backend)
     for q in (0, 1):
         assert np.array_equal(got[q].view(np.uint32), T.run_case(build((q,)), backend)[0].view(np.uint32)), q
+
+
+@pytest.mark.parametrize("M", [20, 70])
+def test_input_of_16_bit_and_quantised_matrices(backend, H, M):
+    """An input that both kinds of matrices read in turn (adapters beside a quantised matrix) is converted once for each kind."""
+    rng = np.random.default_rng(M)
+    K, N = 512, 96
+    ws = [(wt, T.rand_weight(wt, K, N, rng) if wt == L.Q8_0 else bits16((rng.standard_normal((N, K)) / 22).astype(np.float32), wt)) for wt in (L.Q8_0, L.F16) * 3]
+    x = rng.standard_normal((M, K)).astype(np.float32)
+
+    def run(which):
+        k0 = backend.stat("kernel_launches")
+
+        def build(g):
+            cur = g.new(L.F32, [K, M], x)
+            return [H.ggml_mul_mat(g.ctx, g.new(wt, [K, N], w), cur) for wt, w in (ws[q] for q in which)]
+
+        r = T.run_case(build, backend)
+        return r, backend.stat("kernel_launches") - k0
+
+    backend.set_option("fusion", 0)  # (node by node)
+    try:
+        got, n = run(range(6))
+        alone = [run([q]) for q in range(6)]
+    finally:
+        backend.set_option("fusion", 1)
+    assert n == sum(k for _, k in alone) - 4  # (two conversions instead of six)
+    for q in range(6):
+        assert np.array_equal(got[q].view(np.uint32), alone[q][0][0].view(np.uint32)), q
