@@ -326,7 +326,7 @@ struct ws_plan {
     size_t aux_bytes = 0;  // region B: attention partials
 };
 
-static bool mm_tile_applies(const ggml_tensor * n);
+static bool mm_tile_form(const ggml_tensor * n);
 static bool mm_id_tile_applies(const ggml_tensor * n);
 static size_t fa_image_offset(const tdesc & q, const tdesc & k, const tdesc & v) { return (fattn_workspace_bytes(q, k, v, 64, GGML_TYPE_F16) + 255) & ~(size_t) 255; }
 static ws_plan plan_ws(backend_ctx * c, const ggml_cgraph * g) {
@@ -344,7 +344,7 @@ static ws_plan plan_ws(backend_ctx * c, const ggml_cgraph * g) {
     for (int i = 0; i < g->n_nodes; ++i) {
         const ggml_tensor * n = g->nodes[i];
         // (besides what follows: K.q of one head on one key head has this form, and the attention chain that may start at it has its own scratch)
-        if (n->op == GGML_OP_MUL_MAT && mm_tile_applies(n)) p.act16_bytes = std::max(p.act16_bytes, (size_t) (n->src[1]->ne[0] * n->src[1]->ne[1]) * 2);
+        if (n->op == GGML_OP_MUL_MAT && mm_tile_form(n)) p.act16_bytes = std::max(p.act16_bytes, (size_t) (n->src[1]->ne[0] * n->src[1]->ne[1]) * 2);
         if (n->op == GGML_OP_MUL_MAT && is_quant(n->src[0]->type)) {
             const ggml_tensor * b = n->src[1];
             const int64_t Mc = b->ne[1] * b->ne[2] * b->ne[3];
@@ -563,15 +563,16 @@ static const void * quantized_src1(exec_state & st, const ggml_tensor * b, int w
     return dst;
 }
 
-// MUL_MAT of a batch of columns by a 16-bit weight matrix on the LDS-tiled kernels (mmf_tile.hip): src1 goes through a copy in the matrix's type.  Up to 16 columns the
-// kernel that splits K over the waves of a 16-row tile is faster (4096 x 4096: 17.5 us for 16 columns, 28.6 for 32; tiles: 23 and 22.6), whatever shares the launch
+// MUL_MAT of a batch of columns by a 16-bit weight matrix on the LDS-tiled kernels (mmf_tile.hip): src1 goes through a copy in the matrix's type.  Which products have that form
 static constexpr int64_t MM_TILE_MIN_COLS = 17;
-static bool mm_tile_applies(const ggml_tensor * n) {
+static bool mm_tile_form(const ggml_tensor * n) {
     const ggml_tensor * a = n->src[0], * b = n->src[1];
     return (a->type == GGML_TYPE_F16 || a->type == GGML_TYPE_BF16) && n->type == GGML_TYPE_F32 && b->type == GGML_TYPE_F32 && b->ne[1] >= MM_TILE_MIN_COLS && a->ne[2] * a->ne[3] * b->ne[2] * b->ne[3] == 1 &&
            !buffer_is_split(a->buffer) && b->nb[0] == 4 && (b->nb[1] % 16) == 0 && (((uintptr_t) b->data) & 15) == 0 && n->nb[0] == 4 &&
            mul_mat_tile_ok(a->type, a->ne[0], a->ne[1], (int64_t) a->nb[0], (int64_t) a->nb[1], a->data);
 }
+// ... and one such product alone takes it where that is the faster way (mul_mat_tile_pays); siblings: try_merge_mm_16
+static bool mm_tile_applies(const ggml_tensor * n) { return mm_tile_form(n) && mul_mat_tile_pays(n->src[0]->ne[0], n->src[0]->ne[1], n->src[1]->ne[1]); }
 // ... and MUL_MAT_ID of as many (expert, token) columns as its batched form takes (src1's rows of all tokens dense)
 static bool mm_id_tile_applies(const ggml_tensor * n) {
     const ggml_tensor * a = n->src[0], * b = n->src[1], * ids = n->src[2];
@@ -1828,7 +1829,7 @@ static bool try_fuse_attn_nf_mma(exec_state & st, int i) {
 
 // Projections of the same activations by bf16 matrices (q, k, v and the gate of a layer): the siblings that follow node i are executed EARLY, at node i,
 // as one launch (may_run_early).  Returns true when node i and at least one sibling were served.
-// One column, 2 .. 16 and more each have their kernel; all of them give a matrix the bits it gets alone.
+// One column, 2 .. 16 and more each have their kernel; a matrix gets the bits of that kernel alone (17 columns and up: the tiles, which a product without siblings may not take).
 static bool try_merge_mm_16(exec_state & st, int i) {
     backend_ctx * c = st.c;
     ggml_cgraph * g = st.g;
@@ -1841,7 +1842,7 @@ static bool try_merge_mm_16(exec_state & st, int i) {
         const ggml_tensor * w = t->src[0];
         return t->op == GGML_OP_MUL_MAT && t->src[1] == X && (w->type == GGML_TYPE_BF16 || (tile && w->type == GGML_TYPE_F16)) && w->type == n0->src[0]->type && w->ne[0] == K && w->ne[2] == 1 &&
                w->ne[3] == 1 && w->nb[0] == 2 && (w->nb[1] % 16) == 0 && !(((uintptr_t) w->data) & 15) && !buffer_is_split(w->buffer) && is_f32_contig(t) && !mm_cache_image_ok(t) &&
-               (tile ? mm_tile_applies(t) : mul_mat_bf16_multi_ok(w->ne[1], K, M));
+               (tile ? mm_tile_form(t) : mul_mat_bf16_multi_ok(w->ne[1], K, M));
     };
     if (!eligible(n0)) return false;
     std::vector<int> ms{i};
@@ -1856,6 +1857,9 @@ static bool try_merge_mm_16(exec_state & st, int i) {
     }
     if (ms.size() < 2) return false;
     if (tile) {
+        // (one launch and one rounding for all: that pays for matrices that would not alone, but for two narrow f16 ones over long rows — K 11008, 8 rows, 17 columns: 2 x 16 us
+        // on the kernel that splits K over the chip, 46 tiled)
+        if (ms.size() == 2 && n0->src[0]->type == GGML_TYPE_F16 && K > 4096 && n0->ne[0] <= 128 && g->nodes[ms[1]]->ne[0] <= 128 && !mm_tile_applies(n0) && !mm_tile_applies(g->nodes[ms[1]])) return false;
         const void * x16 = rounded_src1(st, X, n0->src[0]->type);
         mul_mat_tile_desc m[4];
         double bytes = 0;
@@ -2736,7 +2740,8 @@ static int run_node(exec_state & st, int i) {
             if (!is_quant(a->type) && fuse && c->opt.attn_nf && try_fuse_attn_nf(st, i)) return 1;
             if (!is_quant(a->type) && fuse && c->opt.attn_nf && try_fuse_attn_nf_mma(st, i)) return 1;
             if ((a->type == GGML_TYPE_BF16 || a->type == GGML_TYPE_F16) && fuse && try_merge_mm_16(st, i)) return 1;
-            if (mm_tile_applies(n)) {
+            // (node by node, fusion off, every product of the form: then a merged launch can be compared with its products one by one, bit for bit)
+            if (fuse ? mm_tile_applies(n) : mm_tile_form(n)) {
                 const void * x16 = rounded_src1(st, b, a->type);
                 const mul_mat_tile_desc m{a->data, (int64_t) a->nb[1], a->ne[1], n->data, (int64_t) n->nb[1]};
                 timed_scope ts(c, "mul_mat_f", (double) ggml_abi_nbytes(a));

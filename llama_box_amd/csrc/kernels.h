@@ -166,6 +166,7 @@ size_t mul_mat_f_workspace_bytes(const tdesc & src0, const tdesc & src1);
 // a batch of M columns by up to four f16 / bf16 matrices of K columns, LDS-tiled (mmf_tile.hip); x16: the columns in the matrices' type, dense rows (launch_to_16; x rows 16-byte aligned)
 struct mul_mat_tile_desc { const void * W; int64_t nb1; int64_t N; void * dst; int64_t dst_nb1; };
 bool mul_mat_tile_ok(int type, int64_t K, int64_t N, int64_t nb0, int64_t nb1, const void * W);
+bool mul_mat_tile_pays(int64_t K, int64_t N, int64_t M);  // ... faster than launch_mul_mat_f for one matrix of N rows, M > 16 columns
 void launch_to_16(hipStream_t s, int type, const char * x, int64_t nb1, int64_t K, int64_t rows, void * out);
 // the experts' columns (lists: k_moe_group); x16 rows: src1's [n_b, T]
 void launch_mul_mat_id_tile(hipStream_t s, const tdesc & as, int64_t n_b, int64_t n_used, int64_t T, const tdesc & d, const int32_t * cnt, const int32_t * off, const int32_t * list, const void * x16);

@@ -218,6 +218,21 @@ template <bool BF, int TM, int TN, int S, bool ID> static void mt_launch_t(hipSt
 bool mul_mat_tile_ok(int type, int64_t K, int64_t N, int64_t nb0, int64_t nb1, const void * W) {
     return (type == GGML_TYPE_F16 || type == GGML_TYPE_BF16) && nb0 == 2 && K >= 64 && (K % 64) == 0 && N >= 1 && (nb1 % 16) == 0 && (((uintptr_t) W) & 15) == 0 && 128 * nb1 < ((int64_t) 1 << 31);
 }
+// Rounding and tiles (a workgroup of 64 x 64 walks all of K) against one launch of mmf.hip's kernels.  Measured (us for one product of 17 .. 2048 columns, the rounding included; mmf.hip / tiles):
+// - K >= 1024: mmf.hip gives a 16 x 16 tile to 8 waves (16 from K = 4096), which share K in trips of 1024 (2048) values.  While all tiles run at once that is the faster way: K 4096, 512 rows,
+//   64 columns 14.5 / 22.0; N 2048 x 32 14.7 / 23.8; K 11008, 8 rows x 17 16 / 46.  With more it is not: N 2048 x 64 25.4 / 25.5, N 4096 x 64 45.8 / 22.6.  The line, in 16 x 16 tiles'
+//   worth of outputs: 512 for K of one or two whole trips (K 2048: 448 14.3 / 15.3, 516 17.0 / 14.7), 288 where the last trip is part empty (K 1536: 272 11.7 / 12.0, 320 14.4 / 12.7),
+//   304 up to K = 4096 (258 19.6 / 22.9, 384 22.5 / 21.6), 256 beyond (K 11008: 256 35.7 / 49, 272 52 / 47).
+// - K below 1024: mmf.hip has one wave walk K for 32 x 32 outputs.  K 512, 128 rows x 64 14.0 / 7.7; K 256 9.0 / 6.8, but x 32 6.4 / 6.8, x 17 5.5 / 6.4; K 128, 1024 rows x 64 6.5 / 6.5, 128 rows
+//   x 512 6.4 / 6.6, 11008 x 128 10.1 / 8.2; K 64, 4096 x 256 6.5 / 6.8, 11008 x 512 17.9 / 14.5; at most 32 rows leave the tiles half empty: K 256, 8 rows x 128 5.9 / 6.8, K 512 8.0 / 7.6.
+bool mul_mat_tile_pays(int64_t K, int64_t N, int64_t M) {
+    if (K >= 1024) return (N + 15) / 16 * M > 16 * (K <= 2048 ? (K % 1024 == 0 ? 512 : 288) : K <= 4096 ? 304 : 256);
+    if (N <= 32) return K >= 512 && M <= 1024;
+    if (K < 128) return N * M >= (int64_t) 3 << 20;
+    if (K < 192) return N >= 256 && M > 48;
+    if (K < 384) return M > 32;
+    return true;
+}
 void launch_to_16(hipStream_t s, int type, const char * x, int64_t nb1, int64_t K, int64_t rows, void * out) {
     const int64_t total = rows * (K / 8);
     const dim3 grid((unsigned) ((total + 255) / 256));

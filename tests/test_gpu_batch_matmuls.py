@@ -277,3 +277,33 @@ def test_input_of_16_bit_and_quantised_matrices(backend, H, M):
     assert n == sum(k for _, k in alone) - 4  # (two conversions instead of six)
     for q in range(6):
         assert np.array_equal(got[q].view(np.uint32), alone[q][0][0].view(np.uint32)), q
+
+
+# both sides of every line of the choice between the tiles and the kernels without them (mul_mat_tile_pays): two launches (rounding, tiles) or one (or two: K slices and their sum)
+@pytest.mark.parametrize("wt", [L.BF16, L.F16])
+@pytest.mark.parametrize("K,N,M,tiled", [
+    (1024, 1024, 128, False), (1024, 1024, 129, True), (1536, 1024, 72, False), (1536, 1024, 73, True), (2048, 512, 256, False), (2048, 512, 257, True), (3072, 1024, 76, False), (3072, 1024, 77, True),
+    (4352, 512, 128, False), (4352, 512, 129, True), (512, 32, 40, True), (448, 32, 40, False), (64, 4096, 300, False), (128, 256, 48, False), (128, 256, 49, True), (192, 70, 32, False), (192, 70, 33, True),
+    (384, 40, 17, True)])
+def test_16_bit_matrices_around_the_lines_of_the_choice(backend, H, wt, K, N, M, tiled):
+    rng = np.random.default_rng(K + N + M)
+    w = round16((rng.standard_normal((N, K)) / np.sqrt(K)).astype(np.float32), wt)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+
+    def run():
+        k0 = backend.stat("kernel_launches")
+        r = T.run_case(lambda g: H.ggml_mul_mat(g.ctx, g.new(wt, [K, N], bits16(w, wt)), g.new(L.F32, [K, M], x)), backend)[0].reshape(M, N)
+        return r, backend.stat("kernel_launches") - k0
+
+    got, n = run()
+    assert n == (2 if tiled else 1)
+    backend.set_option("fusion", 0)
+    try:
+        tiles, _ = run()
+    finally:
+        backend.set_option("fusion", 1)
+    ref = round16(x, wt).astype(np.float64) @ w.astype(np.float64).T
+    for r in (got, tiles):
+        assert np.abs(r - ref).max() <= 6e-8 * np.sqrt(K) * 8
+    if tiled:
+        assert np.array_equal(got.view(np.uint32), tiles.view(np.uint32))
