@@ -145,7 +145,8 @@ struct stats {
     int64_t p2p_allreduces = 0;        // row-parallel sums served by the one-shot peer-to-peer kernel (tp_p2p.hip) instead of RCCL
     int64_t ss_handoffs = 0;           // RMS_NORM prologues that took the sum of squares from the producing mat-vec's partial sums
     int64_t skinny_launches = 0;       // mat-muls of 2..32 columns served by the weight-streaming matrix-core kernel
-    int64_t wide_launches = 0;         // prompt-batch mat-muls served by its wide form
+    int64_t wide_launches = 0;         // prompt-batch mat-muls served by its wide forms (k_mmq_wide, k_mmq_wide_few)
+    int64_t wide_few_launches = 0;     // ... by k_mmq_wide_few (few columns: K slices, Q6_K too)
     int64_t tiled_launches = 0;        // batch mat-muls served by the LDS-tiled int8 GEMM (mmq_i8.hip)
     int64_t nf_mma_chains = 0;         // non-flash K.q -> SOFT_MAX -> V^T.p chains of a prompt micro-batch served by the two-pass matrix-core kernel (round 4)
     int64_t fa_list_launches = 0;      // FLASH_ATTN_EXT nodes served over per-token position lists (2..32 tokens; 33..256 when the mask is known to be sparse)

@@ -724,7 +724,8 @@ static bool run_mul_mat_q(exec_state & st, const ggml_tensor * w, const ggml_ten
             const int served = launch_mmq_i8(c->stream, w->type, (const uint8_t *) w->data, (int64_t) w->nb[1], (int) K, (int) N, (int) M, act, (float *) dst->data, (int64_t) (dst->nb[1] / 4), c->opt.mmq_bn, epi ? 1 : ks, part,
                                              add ? (const float *) add->data : nullptr, add_stride, !defer, c->opt.mmq_skinny, epi);
             c->st.skinny_launches += served == 1;
-            c->st.wide_launches += served == 2;
+            c->st.wide_launches += served >= 2;
+            c->st.wide_few_launches += served == 3;
             c->st.tiled_launches += served == 0;
             if (defer) {
                 st.sk_dst = dst;
@@ -1378,8 +1379,9 @@ static int try_merge_mm_batch(exec_state & st, int i) {  // returns the number o
         }
         const int served = launch_mmq_i8_multi(c->stream, type, (int) ms.size(), mats, (int) K, (int) M, act, c->opt.mmq_bn, ks, part, !defer, c->opt.mmq_skinny, epi_node >= 0 ? &epi : nullptr);
         c->st.skinny_launches += served == 1;
-        c->st.wide_launches += served == 2;
-            c->st.tiled_launches += served == 0;
+        c->st.wide_launches += served >= 2;
+        c->st.wide_few_launches += served == 3;
+        c->st.tiled_launches += served == 0;
     }
     c->st.kernel_launches += (ks > 1 && !defer) ? 2 : 1;
     c->st.fused_nodes += ms[0].n_nodes - 1;

@@ -37,7 +37,7 @@ bool launch_mmq_skinny_mixed(hipStream_t s, const mmq8_args & a);
 // prompt batches on the same unit (mmq_skinny.hip, wide form): token tiles per workgroup (4 / 2) when it applies, 0 when it does not
 int mmq_wide_tiles(int type, int64_t K, const int64_t * N, int n_mat, int64_t M, int64_t w_nb1, int ksplit);
 int mmq_wide_ksplit(int type, int64_t K, int64_t N, int64_t M);  // K slices of such a launch (0: it does not apply)
-bool mmq_wide_fills(int type, int64_t g128, int64_t M);           // do its row groups of 128 and column groups of 64 occupy half the chip?
+int64_t mmq_wide_few_max();                                       // up to this many columns: k_mmq_wide_few
 void launch_mmq_wide(hipStream_t s, int type, int tt, const mmq8_args & a);  // mmq_skinny.hip; a.mat[].panel0 / n_panels are set by the launcher
 
 }  // namespace mi355x

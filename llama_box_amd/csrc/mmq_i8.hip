@@ -547,7 +547,7 @@ int launch_mmq_i8_multi(hipStream_t s, int type, int n_mat, const mmq_mat_desc *
         if (tt) {
             launch_mmq_wide(s, type, tt, a);
             if (a.ksplit > 1 && reduce) launch_splitk_reduce_multi(s, a);
-            return mmq_wide_fills(type, panels128, M) ? 2 : 0;  // (the counters: a launch whose row groups and token tiles alone fill the chip, or a split one)
+            return M <= mmq_wide_few_max() ? 3 : 2;
         }
     }
     skinny = skinny && (a.ksplit & (a.ksplit - 1)) == 0;  // (its K split is a power of two: mmq_skinny_ksplit)

@@ -1469,7 +1469,8 @@ __global__ void __launch_bounds__((WD_NW + WD_NL) * 64, 1) k_mmq_wide_few(const 
 // own operands, 28.7 k; the same with 2 / 4 loaders 26.1 / 28.9 k (one address pipeline per CU: 52 LDS-DMA instructions per step); 4 waves x 4 tiles 20.2 k (spills at
 // the 256-register cap of six waves).  Qwen2-7B Q5_K_M (three digit planes: the tiled GEMM spills there) 20.5 -> 25.3 k.  Returns the token tiles of a workgroup, or 0.
 // The caller's activation area must hold whole 128-column groups (columns beyond M are fetched, never stored).
-bool mmq_wide_fills(int type, int64_t g128, int64_t M) { return type != GGML_TYPE_Q6_K && g128 * ((M + 63) / 64) * 2 >= skinny_n_cu(); }
+static bool mmq_wide_fills(int type, int64_t g128, int64_t M) { return type != GGML_TYPE_Q6_K && g128 * ((M + 63) / 64) * 2 >= skinny_n_cu(); }
+int64_t mmq_wide_few_max() { return WD_FEW; }
 int mmq_wide_tiles(int type, int64_t K, const int64_t * N, int n_mat, int64_t M, int64_t w_nb1, int ksplit) {
     static const bool on = !getenv("GGML_MI355X_MMQ_WIDE") || atoi(getenv("GGML_MI355X_MMQ_WIDE")) != 0;
     if (!on || M < 33 || (K % 256) != 0 || ksplit > K / 256) return 0;

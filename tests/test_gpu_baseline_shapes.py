@@ -715,7 +715,7 @@ def test_layer_teacher_forced_batch(backend, H, plog, li, mode, fa):
         y = H.ggml_mul_mat(g.ctx, g.new(sp.t_d, [FF, E], W["wd"]), a)
         return dict(outs=[H.ggml_add(g.ctx, y, g.new(L.F32, [E, M], inp["ffn_inp"]))], first=[])
 
-    COUNTERS = ("kernel_launches", "skinny_launches", "wide_launches", "tiled_launches", "rope_epilogues", "fa_list_launches")
+    COUNTERS = ("kernel_launches", "skinny_launches", "wide_launches", "wide_few_launches", "tiled_launches", "rope_epilogues", "fa_list_launches")
 
     def run(seg, target, inp):
         g = T.G(target)
@@ -742,12 +742,11 @@ def test_layer_teacher_forced_batch(backend, H, plog, li, mode, fa):
                 assert cnt["tiled_launches"] >= 1, (group, cnt)
             assert cnt["skinny_launches"] == 0, (group, cnt)
         else:
-            # 33 .. 160 columns, or a rank's narrow shards: the wide form where its grid fills the chip (mmq_wide_tiles), the tiled int8 GEMM
-            # otherwise — never the 32-column skinny kernel, never a column-by-column mat-vec fall-back (one launch per matrix group at most,
+            # 33 .. 160 columns, or a rank's narrow shards: a wide form where it applies, the tiled int8 GEMM otherwise — never the 32-column skinny kernel, never a column-by-column mat-vec fall-back (one launch per matrix group at most,
             # + split-K reduce / quantiser launches)
             assert cnt["skinny_launches"] == 0 and cnt["wide_launches"] + cnt["tiled_launches"] >= 1, (group, cnt)
-            if L.Q6_K in wtypes:
-                assert cnt["tiled_launches"] >= 1, (group, cnt)
+            if L.Q6_K in wtypes:  # (up to 384 columns: the wide form with K slices)
+                assert cnt["wide_few_launches" if M <= 384 else "tiled_launches"] >= 1, (group, cnt)
             assert cnt["kernel_launches"] <= 12, (group, cnt)
 
     tag = f"{sp.name} [{mode}, {M} tokens, n_kv {n_kv}, fa={fa}]"

@@ -147,12 +147,19 @@ def test_k_quant_batches_of_33_columns_and_up(backend, H, qt, K, N, M):
     def run(where, ww, bb):
         return T.run_case(lambda g: H.ggml_add(g.ctx, H.ggml_mul_mat(g.ctx, g.new(qt, [K, ww.shape[0]], ww), g.new(L.F32, [K, M], x)), g.new(L.F32, [ww.shape[0], M], bb)), where)[0].reshape(M, -1)
 
+    COUNTERS = ("skinny_launches", "wide_launches", "wide_few_launches", "tiled_launches")
+    c0 = [backend.stat(k) for k in COUNTERS]
     got = run(backend, w, b)
+    served = [backend.stat(k) - c for k, c in zip(COUNTERS, c0)]
+    few = M <= 384 and (qt != L.Q6_K or K % 512 == 0)
+    assert served == ([0, 1, 1, 0] if few else [0, 0, 0, 1] if qt == L.Q6_K else [0, 1, 0, 0]), served
+    c0 = backend.stat("tiled_launches")
     backend.set_option("mmq_skinny", 0)
     try:
         tiled = run(backend, w, b)
     finally:
         backend.set_option("mmq_skinny", 1)
+    assert backend.stat("tiled_launches") == c0 + 1
     assert T.nmse(got, tiled) <= 1e-12
     rows = np.unique(np.concatenate([np.arange(min(N, 40)), np.arange(max(0, N - 40), N)]))
     assert T.nmse(got[:, rows], run("oracle", np.ascontiguousarray(w[rows]), np.ascontiguousarray(b[:, rows]))) <= 1e-10

@@ -290,7 +290,7 @@ def test_mul_mat_q_skinny_batches(backend, H, plog, qt, K, N, M, epi):
 @pytest.mark.parametrize("K,N,M,epi,served", [
     (512, 4096, 512, "res", 1), (1024, 8192, 300, "bias", 1), (256, 12288, 130, "none", 1), (2048, 16384, 33, "none", 1), (4096, 16384, 64, "res", 1),
     (512, 28672, 128, "none", 1), (1024, 16384, 200, "bias", 1),  # many row groups, ragged columns
-    (2048, 4096, 100, "none", 0),  # too few (row group, token tile) pairs to fill the chip: the tiled GEMM keeps it
+    (2048, 4096, 100, "none", 1),  # too few (row group, token tile) pairs to fill the chip: slices of K (k_mmq_wide_few)
 ])
 def test_mul_mat_q_wide_batches(backend, H, plog, qt, K, N, M, epi, served):
     """Prompt batches (33 columns and up) on the wide form of the skinny unit (mmq_skinny.hip, k_mmq_wide): four row tiles x two
