@@ -34,10 +34,9 @@ struct mmq8_args {
 void launch_mmq_skinny(hipStream_t s, int type, const mmq8_args & a);
 // matrices of two K-quant formats in one launch (a.mat[].qt set); false: this pair of formats is not built
 bool launch_mmq_skinny_mixed(hipStream_t s, const mmq8_args & a);
-// prompt batches on the same unit (mmq_skinny.hip, wide form): token tiles per workgroup (4 / 2) when it applies, 0 when it does not
-int mmq_wide_tiles(int type, int64_t K, const int64_t * N, int n_mat, int64_t M, int64_t w_nb1, int ksplit);
+// prompt batches on the same unit (mmq_skinny.hip): 0 = not there, 1 = k_mmq_wide (no K split), 2 / 3 = k_mmq_wide_few with that many token tiles a workgroup
+int mmq_wide_form(int type, int64_t K, const int64_t * N, int n_mat, int64_t M, int64_t w_nb1);
 int mmq_wide_ksplit(int type, int64_t K, int64_t N, int64_t M);  // K slices of such a launch (0: it does not apply)
-int64_t mmq_wide_few_max();                                       // up to this many columns: k_mmq_wide_few
-void launch_mmq_wide(hipStream_t s, int type, int tt, const mmq8_args & a);  // mmq_skinny.hip; a.mat[].panel0 / n_panels are set by the launcher
+void launch_mmq_wide(hipStream_t s, int type, int form, const mmq8_args & a);  // mmq_skinny.hip; a.mat[].panel0 / n_panels are set by the launcher
 
 }  // namespace mi355x

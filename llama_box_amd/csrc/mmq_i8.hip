@@ -425,7 +425,7 @@ template <int QT, int BN, int BM = 128> static void launch_mmq8_t(hipStream_t s,
 // the K range is split over blockIdx.y and the partial products are summed in a fixed order by a second tiny kernel
 int mmq_pick_ksplit(int64_t K, int64_t N, int64_t M, bool skinny, int type) {
     if (skinny && M >= 2 && M <= 32 && (N % 32) == 0) return mmq_skinny_ksplit(K, N);
-    // prompt batches the wide form of mmq_skinny.hip serves run without a K split (its grid fills the chip by token-tile groups)
+    // prompt batches on the wide forms of mmq_skinny.hip: without a K split where the grid fills the chip by token-tile groups, with their own slices otherwise
     if (const int ks = skinny ? mmq_wide_ksplit(type, K, N, M) : 0) return ks;
     const int64_t wgs = ((N + 63) / 64) * ((M + 127) / 128), nblk = K / 256;
     static const int ks_target = getenv("GGML_MI355X_MMQ_KS_TARGET") ? atoi(getenv("GGML_MI355X_MMQ_KS_TARGET")) : 512;
@@ -543,11 +543,11 @@ int launch_mmq_i8_multi(hipStream_t s, int type, int n_mat, const mmq_mat_desc *
             Ns[i] = mats[i].N;
             same = same && mats[i].w_nb1 == mats[0].w_nb1;
         }
-        const int tt = same ? mmq_wide_tiles(type, K, Ns, n_mat, M, mats[0].w_nb1, a.ksplit) : 0;
-        if (tt) {
-            launch_mmq_wide(s, type, tt, a);
+        const int form = same ? mmq_wide_form(type, K, Ns, n_mat, M, mats[0].w_nb1) : 0;
+        if (form == 1 ? a.ksplit == 1 : form != 0 && a.ksplit <= K / 256) {
+            launch_mmq_wide(s, type, form, a);
             if (a.ksplit > 1 && reduce) launch_splitk_reduce_multi(s, a);
-            return M <= mmq_wide_few_max() ? 3 : 2;
+            return form == 1 ? 2 : 3;
         }
     }
     skinny = skinny && (a.ksplit & (a.ksplit - 1)) == 0;  // (its K split is a power of two: mmq_skinny_ksplit)

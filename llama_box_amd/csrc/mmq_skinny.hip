@@ -779,7 +779,7 @@ static int skinny_n_cu();
 //   serves the weight bytes to all of them.
 constexpr int WD_NB = 2;  // stages of the activation ring (3 = requested two steps ahead, like the weights: measured equal, A/B on one box)
 constexpr int WD_NA = 3;  // ... of the weight rings
-// Up to this many columns the K range may be split and Q6_K comes here too (k_mmq_wide_few).  Whole prompts of Llama-3-8B Q4_K_M, us, before / with it: 64 columns
+// Up to this many columns the K range may be split and Q6_K comes here too (k_mmq_wide_few, where few_pays says so).  Whole prompts of Llama-3-8B Q4_K_M, us, before / with it: 64 columns
 // 4106 / 3942, 77: 5336 / 4505, 112: 5648 / 5145, 160: 7691 / 6846, 256: 8673 / 7812, 288: 10371 / 8600, 384: 11613 / 11309; at 448 the split products cost what they
 // bring (12259 / 12708), and a Q6_K 14336 x 4096 takes 121 us here against 95 on the tiled GEMM at 512.
 constexpr int64_t WD_FEW = 384;
@@ -900,7 +900,7 @@ template <> struct sk_conv<6> {
 // token tiles — the matrix pipe busy 37 %.  The loaders take the first two off the computing waves: they request, wait (vmcnt) and
 // meet the others at the step's barrier; the computing waves only convert and multiply.
 // NL = 0: no loaders, but two workgroups a CU (the weight ring one stage shorter, so that both fit the LDS): one's arithmetic covers the other's requests and barrier.
-// Q4_K from 385 columns on: 28672 x 4096 at 512 columns 155 -> 149 us, a 2048-token prompt of Llama-3-8B 52.7 -> 51.9 ms.  (Q5_K's units do not fit twice.)
+// Q4_K with more items than CUs: 28672 x 4096 at 512 columns 155 -> 149 us, a 2048-token prompt of Llama-3-8B 52.7 -> 51.9 ms.  (Q5_K's units do not fit twice.)
 template <int QT, int TT, int NW, int NL, int NSA>
 __global__ void __launch_bounds__((NW + NL) * 64, NSA == 2 ? 2 : 1) k_mmq_wide(const mmq8_args a) {
     constexpr bool SELF = NL == 0;
@@ -1463,35 +1463,62 @@ __global__ void __launch_bounds__((WD_NW + WD_NL) * 64, 1) k_mmq_wide_few(const 
 #undef MAT_OF
 }
 
-// Prompt batches (33 columns and up) take a wide form when every matrix is whole 128-row groups, rows packed back to back: up to WD_FEW columns Q4_K, Q5_K and Q6_K with
-// as many K slices as fill the chip; beyond, Q4_K and Q5_K without a K split where (row groups x 64-column groups) occupy half of it.  Measured on the 512-token prefill
-// of Llama-3-8B Q4_K_M against the tiled GEMM at 28.9 k tok/s: 4 computing waves x 2 token tiles + 2 loaders 30.5 k; 8 computing waves x 2 tiles, everyone requesting its
-// own operands, 28.7 k; the same with 2 / 4 loaders 26.1 / 28.9 k (one address pipeline per CU: 52 LDS-DMA instructions per step); 4 waves x 4 tiles 20.2 k (spills at
-// the 256-register cap of six waves).  Qwen2-7B Q5_K_M (three digit planes: the tiled GEMM spills there) 20.5 -> 25.3 k.  Returns the token tiles of a workgroup, or 0.
-// The caller's activation area must hold whole 128-column groups (columns beyond M are fetched, never stored).
-static bool mmq_wide_fills(int type, int64_t g128, int64_t M) { return type != GGML_TYPE_Q6_K && g128 * ((M + 63) / 64) * 2 >= skinny_n_cu(); }
-int64_t mmq_wide_few_max() { return WD_FEW; }
-int mmq_wide_tiles(int type, int64_t K, const int64_t * N, int n_mat, int64_t M, int64_t w_nb1, int ksplit) {
+// Prompt batches (33 columns and up) of whole 128-row groups, rows packed back to back, have two wide forms: k_mmq_wide (Q4_K, Q5_K; the whole of K; where row groups x 64-column
+// groups occupy half the chip) and, up to WD_FEW columns, k_mmq_wide_few (Q6_K too; slices of K).  The caller's activation area must hold whole 128-column groups (columns
+// beyond M are fetched, never stored).  k_mmq_wide's shape, measured on the 512-token prefill of Llama-3-8B Q4_K_M against the tiled GEMM at 28.9 k tok/s: 4 computing waves x
+// 2 token tiles + 2 loaders 30.5 k; 8 computing waves x 2 tiles, everyone requesting its own operands, 28.7 k; the same with 2 / 4 loaders 26.1 / 28.9 k (one address pipeline
+// per CU: 52 LDS-DMA instructions per step); 4 waves x 4 tiles 20.2 k (spills at the 256-register cap of six waves).  Qwen2-7B Q5_K_M (three digit planes: the tiled GEMM
+// spills there) 20.5 -> 25.3 k.
+static int64_t wide_row_bytes(int type, int64_t K) { return K / 256 * (type == GGML_TYPE_Q4_K ? 144 : type == GGML_TYPE_Q5_K ? 176 : 210); }
+// three token tiles a workgroup where they waste fewer columns than two (Q5_K: their registers do not fit)
+static int few_tiles(int type, int64_t M) { return type != GGML_TYPE_Q5_K && (M + 95) / 96 * 96 < (M + 63) / 64 * 64 ? 3 : 2; }
+static int64_t few_slices(int64_t K, int64_t items) { return std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(8, K / 512), skinny_n_cu() / items)); }
+// Is k_mmq_wide_few the fastest for n rows in all?  Both sides measured, one product with its quantiser and its sum of slices, at 2748 points of K 256 .. 14336, n 128 .. 28672,
+// 33 .. 384 columns (us, other kernel / k_mmq_wide_few, n x K); what this rule picks is within 5 % of the better one at all but 40 of them.
+// - Against k_mmq_wide: by steps of a workgroup, (token tiles + 2) quarters each, the slices' sum as six steps.  Q4_K, 77 columns, 28672 x 4096 51.1 / 39.4 (one round of three
+//   tiles for two of two), 8192 x 4096 28.9 / 26.2 (4 slices), 14336 x 2048 20.5 / 25.8; 257 columns, 8192 x 4096 51.9 / 39.4, 6144 x 4096 32.8 / 38.0.
+// - Against the tiled GEMM, whose own K split and small tiles win where a slice is short or the rows are few: by format and columns.
+//   64: Q4_K 2048 x 2048 14.5 / 15.7, 3072 x 2048 16.6 / 16.1, 512 x 8192 21.3 / 19.3; Q6_K 4096 x 4096 21.3 / 23.1, 14336 x 4096 35.6 / 32.4.
+//   77: Q4_K 1024 x 1024 14.3 / 14.9, 2048 x 2048 17.8 / 17.3, 6144 x 2048 19.4 / 20.1, 4096 x 4096 20.8 / 23.3, 6144 x 4096 28.9 / 24.4; Q5_K 1024 x 1024 17.4 / 14.5;
+//   Q6_K 2048 x 2048 18.9 / 19.3, 4096 x 14336 46.8 / 38.0.
+//   160: Q4_K 4096 x 512 11.0 / 11.9, 4096 x 2048 20.8 / 20.0; Q6_K 1024 x 1024 15.8 / 16.0, 4096 x 2048 22.1 / 23.4, 14336 x 4096 (two rounds) 63.1 / 79.7.
+//   300: eight slices' sum is too much for few rows: Q4_K 256 x 4096 21.1 / 24.6.
+static bool few_pays(int type, int64_t K, int64_t n, int64_t M) {
+    const int64_t cu = skinny_n_cu(), nblk = K / 256, tt = few_tiles(type, M), items = n / 128 * ((M + 32 * tt - 1) / (32 * tt)), ks = few_slices(K, items), rounds = (items * ks + cu - 1) / cu;
+    const bool q5 = type == GGML_TYPE_Q5_K, q6 = type == GGML_TYPE_Q6_K;
+    const int64_t wide_items = n / 128 * ((M + 63) / 64);
+    if (!q6 && wide_items * 2 >= cu) return rounds * ((nblk + ks - 1) / ks) * (tt + 2) + (ks > 1 ? 24 : 0) < (wide_items + cu - 1) / cu * nblk * 4;
+    if (q6 && !(rounds == 1 || (tt == 3 && items * 8 >= rounds * cu * 7))) return false;
+    if (M <= 64) return n * K >= (q6 ? (int64_t) 36 << 20 : (int64_t) 6 << 20) || (!q6 && K >= 8192);
+    if (M <= 96) {
+        if (q5) return K >= 1024;
+        if (q6) return K >= 8192 || n * K >= (int64_t) 20 << 20;
+        return K >= 2048 && !(K < 3584 && n > 4096) && !(K >= 4096 && K < 8192 && n > 1024 && n < 6144);
+    }
+    if (M <= 256) {
+        if (q6) return K >= 8192 ? n <= 6144 || M <= 128 : K >= 2048 && (n <= 1024 || (K >= 3584 && n >= 6144));
+        return K >= 2048 || (K >= 1024 && (q5 || n <= 1024));
+    }
+    if (q6) return K >= 8192 ? n >= 1024 : (K >= 3584 && n >= 3072) || (K >= 2048 && n >= 6144);
+    return K >= (q5 ? 1024 : 2048) && !(n <= 768 && K >= 3072 && K < 8192);
+}
+int mmq_wide_form(int type, int64_t K, const int64_t * N, int n_mat, int64_t M, int64_t w_nb1) {
     static const bool on = !getenv("GGML_MI355X_MMQ_WIDE") || atoi(getenv("GGML_MI355X_MMQ_WIDE")) != 0;
-    if (!on || M < 33 || (K % 256) != 0 || ksplit > K / 256) return 0;
+    if (!on || M < 33 || (K % 256) != 0) return 0;
     if (!(type == GGML_TYPE_Q4_K || type == GGML_TYPE_Q5_K || type == GGML_TYPE_Q6_K)) return 0;
-    if (w_nb1 != (K / 256) * (type == GGML_TYPE_Q4_K ? 144 : type == GGML_TYPE_Q5_K ? 176 : 210)) return 0;
+    if (w_nb1 != wide_row_bytes(type, K)) return 0;
     if (type == GGML_TYPE_Q6_K && (K % 512) != 0) return 0;  // rows of whole dwords: the two-byte shift of a block is the same in every row
     int64_t g128 = 0;
     for (int i = 0; i < n_mat; ++i) {
         if (N[i] % 128) return 0;
         g128 += N[i] / 128;
     }
-    // three tiles where they waste fewer columns than two (Q5_K: their registers do not fit)
-    if (M <= WD_FEW) return type != GGML_TYPE_Q5_K && (M + 95) / 96 * 96 < (M + 63) / 64 * 64 ? 3 : 2;
-    return ksplit == 1 && mmq_wide_fills(type, g128, M) ? 2 : 0;
+    if (M <= WD_FEW && few_pays(type, K, 128 * g128, M)) return few_tiles(type, M);
+    return type != GGML_TYPE_Q6_K && g128 * ((M + 63) / 64) * 2 >= skinny_n_cu() ? 1 : 0;
 }
 int mmq_wide_ksplit(int type, int64_t K, int64_t N, int64_t M) {
-    const int tt = mmq_wide_tiles(type, K, &N, 1, M, (K / 256) * (type == GGML_TYPE_Q4_K ? 144 : type == GGML_TYPE_Q5_K ? 176 : 210), 1);
-    if (!tt) return 0;
-    if (M > WD_FEW) return 1;
-    const int64_t items = N / 128 * ((M + 32 * tt - 1) / (32 * tt));
-    return (int) std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(8, K / 512), skinny_n_cu() / items));
+    const int form = mmq_wide_form(type, K, &N, 1, M, wide_row_bytes(type, K));
+    return form <= 1 ? form : (int) few_slices(K, N / 128 * ((M + 32 * form - 1) / (32 * form)));
 }
 
 template <int QT, int TT, int NW, int NL, int NSA> static void launch_wide_t(hipStream_t s, mmq8_args a) {
@@ -1521,15 +1548,19 @@ template <int QT, int TT, bool LAP> static void launch_wide_few_t(hipStream_t s,
     const int n_virtual = ((a.n_panels + 7) / 8) * 8 * a.m_tiles * a.ksplit;
     MI_LAUNCH_PROBED((k_mmq_wide_few<QT, TT, LAP>), dim3((unsigned) std::min(n_virtual, skinny_n_cu())), dim3((WD_NW + WD_NL) * 64), lds, s, a);
 }
-void launch_mmq_wide(hipStream_t s, int type, int tt, const mmq8_args & a) {
-    if (a.M > WD_FEW) {
+void launch_mmq_wide(hipStream_t s, int type, int form, const mmq8_args & a) {
+    if (form == 1) {
+        int64_t items = 0;
+        for (int i = 0; i < a.n_mat; ++i) items += a.mat[i].N / 128 * ((a.M + 63) / 64);
+        // (two workgroups a CU need two items a CU: 4096 x 4096 at 512 columns, 256 items, 35.5 us with loaders, 39.8 without; 6144 x 4096, 384 items, 54.5 / 51.1)
         if (type == GGML_TYPE_Q5_K) launch_wide_t<5, 2, WD_NW, WD_NL, WD_NA>(s, a);
+        else if (items <= skinny_n_cu()) launch_wide_t<4, 2, WD_NW, WD_NL, WD_NA>(s, a);
         else launch_wide_t<4, 2, WD_NW, 0, 2>(s, a);
     } else if (type == GGML_TYPE_Q5_K) launch_wide_few_t<5, 2, false>(s, a);
     else if (type == GGML_TYPE_Q6_K) {
-        if (tt == 3) launch_wide_few_t<6, 3, true>(s, a);
+        if (form == 3) launch_wide_few_t<6, 3, true>(s, a);
         else launch_wide_few_t<6, 2, true>(s, a);
-    } else if (tt == 3) launch_wide_few_t<4, 3, true>(s, a);
+    } else if (form == 3) launch_wide_few_t<4, 3, true>(s, a);
     else launch_wide_few_t<4, 2, true>(s, a);
 }
 

@@ -134,10 +134,15 @@ def test_k_quant_batches_by_groups_of_eight_columns(backend, H, qt, K, N):
     assert T.nmse(full[:, rows], ref[: len(full)]) <= 1e-10
 
 
-# one super-block and many, K slices of unequal lengths, two and three token tiles a workgroup with ragged ends, both sides of the line to the unsplit form, Q6_K rows of an odd number of blocks
+# one super-block and many, K slices of unequal lengths, two and three token tiles a workgroup with ragged ends, both sides of the lines between the kernels (f: k_mmq_wide_few,
+# w: k_mmq_wide, t: the tiled GEMM; for Q4_K, Q5_K, Q6_K), Q6_K rows of an odd number of blocks
 @pytest.mark.parametrize("qt", [L.Q4_K, L.Q5_K, L.Q6_K])
-@pytest.mark.parametrize("K,N,M", [(256, 128, 33), (512, 256, 65), (4608, 128, 77), (2560, 384, 96), (1024, 4096, 97), (768, 512, 129), (2048, 1024, 190), (512, 8192, 288), (1536, 640, 384), (1536, 16384, 385)])
-def test_k_quant_batches_of_33_columns_and_up(backend, H, qt, K, N, M):
+@pytest.mark.parametrize("K,N,M,kernels", [
+    (256, 128, 33, "ttt"), (512, 256, 65, "ttt"), (4608, 128, 77, "fft"), (2560, 384, 96, "fft"), (1024, 4096, 97, "tft"), (768, 512, 129, "ttt"), (2048, 1024, 190, "fff"), (512, 8192, 288, "fwt"),
+    (1536, 640, 384, "tft"), (1536, 16384, 385, "wwt"),
+    (8192, 128, 33, "fft"), (8448, 256, 64, "fft"), (8704, 128, 65, "fff"), (1280, 256, 96, "tft"), (2560, 384, 97, "fff"), (2304, 512, 129, "fft"), (2048, 896, 256, "fff"), (2560, 896, 257, "fft"),
+    (3584, 3072, 288, "fff"), (8192, 1024, 384, "fff"), (8192, 4608, 33, "fff"), (512, 16384, 33, "wwt"), (512, 4096, 512, "wwt")])
+def test_k_quant_batches_of_33_columns_and_up(backend, H, qt, K, N, M, kernels):
     """mmq_skinny.hip: k_mmq_wide_few / k_mmq_wide against the oracle and, the sums of the K slices apart, the tiled GEMM: exact integer block sums, f32 sums over K / 256 terms."""
     rng = np.random.default_rng(K + N + M)
     w = T.rand_weight(qt, K, N, rng).reshape(N, -1)
@@ -151,8 +156,7 @@ def test_k_quant_batches_of_33_columns_and_up(backend, H, qt, K, N, M):
     c0 = [backend.stat(k) for k in COUNTERS]
     got = run(backend, w, b)
     served = [backend.stat(k) - c for k, c in zip(COUNTERS, c0)]
-    few = M <= 384 and (qt != L.Q6_K or K % 512 == 0)
-    assert served == ([0, 1, 1, 0] if few else [0, 0, 0, 1] if qt == L.Q6_K else [0, 1, 0, 0]), served
+    assert served == {"f": [0, 1, 1, 0], "w": [0, 1, 0, 0], "t": [0, 0, 0, 1]}[kernels[(L.Q4_K, L.Q5_K, L.Q6_K).index(qt)]], served
     c0 = backend.stat("tiled_launches")
     backend.set_option("mmq_skinny", 0)
     try:
