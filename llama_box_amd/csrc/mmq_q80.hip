@@ -259,7 +259,7 @@ template <bool WP> __global__ void __launch_bounds__(Q80C_WV * 64, 3) k_mmq_q80_
 
 bool mmq_q80_batch_supported(int type, int64_t K, int64_t N, int64_t M) {
     static const bool on = !getenv("GGML_MI355X_Q80_SKINNY") || atoi(getenv("GGML_MI355X_Q80_SKINNY")) != 0;
-    return on && type == GGML_TYPE_Q8_0 && (K % 128) == 0 && N >= 1 && M >= 9;
+    return (on || M > 32) && type == GGML_TYPE_Q8_0 && (K % 128) == 0 && N >= 1 && M >= 9;  // (off: the mat-vec passes up to 32 columns)
 }
 // n matrices (1 .. 3) over the same activations; panels[q] != nullptr for ALL of them or for none (the template form is per launch)
 void launch_mmq_q80_multi(hipStream_t s, int n, const mmq80s_desc * mats, int K, int M, const void * act_q80) {

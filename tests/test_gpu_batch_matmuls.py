@@ -1,4 +1,8 @@
 """Mat-muls of prompts and batches at the edges of their kernels' tiles, against the oracle."""
+import os
+import subprocess
+import sys
+
 import numpy as np
 import pytest
 
@@ -318,3 +322,20 @@ def test_16_bit_matrices_around_the_lines_of_the_choice(backend, H, wt, K, N, M,
         assert np.abs(r - ref).max() <= 6e-8 * np.sqrt(K) * 8
     if tiled:
         assert np.array_equal(got.view(np.uint32), tiles.view(np.uint32))
+
+
+def test_q8_0_batches_without_the_skinny_kernel(built):
+    """GGML_MI355X_Q80_SKINNY=0 turns off the kernel of 9 .. 32 columns; 33 and more stay on the matrix cores."""
+    code = """if 1:
+        import numpy as np, harness as T, llama_box_amd as L
+        be, H, rng = L.Backend(0), L.host(), np.random.default_rng(1)
+        w, x = T.rand_weight(L.Q8_0, 256, 64, rng), rng.standard_normal((33, 256)).astype(np.float32)
+        for M in (32, 33):
+            f = lambda g: H.ggml_mul_mat(g.ctx, g.new(L.Q8_0, [256, 64], w), g.new(L.F32, [256, M], x[:M]))
+            s = be.stat("skinny_launches")
+            got = T.run_case(f, be)[0]
+            print(be.stat("skinny_launches") - s, T.nmse(got, T.run_case(f, "oracle")[0]) <= 1e-10)
+    """
+    env = dict(os.environ, GGML_MI355X_Q80_SKINNY="0", PYTHONPATH=os.pathsep.join([T.REPO, os.path.join(T.REPO, "tests")]))
+    r = subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0 and r.stdout.split() == ["0", "True", "1", "True"], (r.stdout, r.stderr[-1000:])
