@@ -1485,11 +1485,10 @@ static int try_merge_q80_skinny(exec_state & st, int i) {  // returns the number
         for (int d = 0; d < ms[q].n_nodes; ++d) { mark_done(st, ms[q].k + d); c->st.fused_nodes++; }
     {
         timed_scope ts(c, (std::string(M <= 32 ? "mmq_q8_0_skinny" : "mmq_q8_0") + (ms.size() == 3 ? "_x3" : "_x2") + "_n" + std::to_string(n_total) + "_k" + std::to_string(K)).c_str(), wbytes, true);
-        launch_mmq_q80_multi(c->stream, (int) ms.size(), mats, (int) K, (int) M, act);
+        c->st.kernel_launches += launch_mmq_q80_multi(c->stream, (int) ms.size(), mats, (int) K, (int) M, act);
     }
     c->st.decode_copy_launches += with_copy != 0;
     c->st.skinny_launches++;
-    c->st.kernel_launches++;
     c->st.fused_nodes += ms[0].n_nodes - 1;
     return ms[0].n_nodes;
 }

@@ -3,14 +3,14 @@
 // ggml-cpu's ggml_vec_dot_q8_0_q8_0 quantises the activations to Q8_0 as well and sums,
 // per 32-value block, sumi * (d_w * d_x) in f32.  A block is exactly the K extent of v_mfma_i32_32x32x32_i8, so one MFMA
 // with a zero accumulator yields the 32x32 integer block sums, and the f32 scale-accumulate follows at once — there is no
-// super-block to amortise it over, which makes these kernels VALU-bound (3 VALU per output and block: convert, d_w * d_x,
-// fused multiply-add — 192 issue cycles beside the MFMA's 32, 0.84 POP/s for the chip).
+// super-block to amortise it over, which makes these kernels VALU-bound: 3 VALU per output and block up to 32 columns (convert, d_w * d_x,
+// fused multiply-add), 2 in the column kernel above that (the factors come from the matrix core), 4 with the 128 x 128 tiles.
 //
-// Both kernels take their operands straight from global memory into the MFMA's registers: the weights from their panel copy
+// The first two take their operands straight from global memory into the MFMA's registers: the weights from their panel copy
 // (repack.hip: k_repack_q80_panels; or, without one, from the 2-byte-aligned blocks), the activations in panel order
 // (quantize.hip) — a wave-instruction reads 1 KB of consecutive bytes either way, no LDS tile and no barrier per K step.
-// An output is eight partial sums — chunk c of four blocks goes to sum c mod 8 — added in order, whatever the number of
-// columns, the wave that made them and the matrices that share the launch: the same bits in every form.
+// An output is a few partial sums, added in order, over interleaved chunks of four blocks: eight (chunk c to sum c mod 8) up to 32 columns, four (c mod 4) above.  Its bits depend on
+// which side of that line the batch is, not on the number of columns otherwise, the kernel, the wave or the matrices that share the launch.
 #include <algorithm>
 #include <cstdlib>
 #include <type_traits>
@@ -150,17 +150,19 @@ template <bool WP> __global__ void __launch_bounds__(Q80S_WV * 64, 2) k_mmq_q80_
 // the multiplication that would be a third VALU instruction per output and block, and the row scales need no way through LDS to the accumulator's rows.  Two VALU
 // are left (convert, fused multiply-add): 128 issue cycles per block beside the matrix core's 64, 1.26 POP/s for the chip.  The next step of two blocks is in flight
 // while one is multiplied, three waves per SIMD (160 registers; three steps in flight at two waves per SIMD: 55 us below).  Workgroups that read the same weights
-// (the column tiles of a panel) follow one another on one XCD, so the weights cross HBM once.
+// (the column tiles of a panel) follow one another on one XCD, so the weights cross HBM once per 1024 columns: an XCD runs about 96 workgroups at once, and 6 panels x 16 tiles draw
+// fewer different operands than 3 x 32 (2048 columns in two groups / in one, 128 x 128 tiles: 14336 x 4096 385 / 571 / 473 us, 4096 x 4096 124 / 175 / 149).
 // TinyLlama, 512 columns: wq + wk + wv / gate + up / a whole 700-token prompt.  128 x 128 LDS tiles, one launch per matrix: 3 x 45 us / 2 x 45 us / 17.2 ms; this kernel
-// with the factors on the VALU: 40 / 66 us / 9.1 ms; as it is: 15 / 44 us / 6.3 ms (23.6 GFLOP in 44 us: 0.53 POP/s).
+// with the factors on the VALU: 40 / 66 us / 9.1 ms; as it is: 15 / 44 us / 5.9 ms (23.6 GFLOP in 44 us: 0.53 POP/s).
 constexpr int Q80C_WV = 4;
 template <bool WP> __global__ void __launch_bounds__(Q80C_WV * 64, 3) k_mmq_q80_cols(const mmq80s_args a, const int n_panels, const int m_tiles) {
     __shared__ float red[Q80C_WV][16][65];                         // the waves' partial tiles, one 32-column half at a time
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int fr = lane & 31, kg = lane >> 5;
     const int xcd = blockIdx.x & 7, qb = blockIdx.x >> 3;
-    const int gp = (qb / m_tiles) * 8 + xcd, m0 = (qb % m_tiles) * 64;  // the panel, counted over all matrices
-    if (gp >= n_panels) return;
+    // m_tiles: the column tiles of one group of them (blockIdx.y)
+    const int gp = (qb / m_tiles) * 8 + xcd, m0 = ((int) blockIdx.y * m_tiles + qb % m_tiles) * 64;  // the panel, counted over all matrices
+    if (gp >= n_panels || m0 >= a.M) return;
     const int mi = gp < a.m[0].panel_end ? 0 : (gp < a.m[1].panel_end ? 1 : 2);
     const mmq80s_mat & mt = a.m[mi];
     const int panel = gp - (mi ? a.m[mi - 1].panel_end : 0);
@@ -257,12 +259,162 @@ template <bool WP> __global__ void __launch_bounds__(Q80C_WV * 64, 3) k_mmq_q80_
     }
 }
 
+// ------------------------------------------------------------------------------------------------ 33 columns and up: 128 x 128 tiles
+// Tile 128 weight rows x 128 columns x 128 K (4 blocks) per trip, 8 waves (32 x 64 each), double-buffered LDS: raw int8 of both operands in the XOR-swizzled [row][128 B] image of
+// mmq_i8.hip plus the 4 block scales of every row / column.  Four VALU per output and block, one workgroup a CU — but an operand is fetched once for 128 outputs, where the kernel
+// above fetches it for 32 or 64: for rows without a panel copy, whose 34-byte blocks come in pieces, and for K of one or two chunks, where that kernel has work for one or
+// two of its four waves.  The chunks are taken in its order (sum c mod 4, sums added in order): the same bits.
+constexpr int Q80_T = 128 * 128;                // bytes of one operand tile
+constexpr int Q80_STAGE = 2 * Q80_T + 2 * 128 * 16;  // A | B | dw[4][128] | da[4][128]
+__device__ __forceinline__ int sw_offq(const int row, const int chunk) { return row * 128 + ((chunk ^ ((row >> 1) & 7)) << 4); }
+
+template <bool WP> __global__ void __launch_bounds__(512, 1) k_mmq_q80_tile(const mmq80s_args a, const int n_panels, const int m_tiles) {
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int xcd = blockIdx.x & 7, qb = blockIdx.x >> 3;
+    const int panel = (qb / m_tiles) * 8 + xcd, mt = qb % m_tiles;
+    if (panel >= n_panels) return;
+    const mmq80s_mat & w = a.m[0];
+    const int n0 = panel * 128, m0 = mt * 128;
+    const int nb32 = a.K / 32, trips = a.K / 128;
+    const int nslab = wave & 3, mhalf = wave >> 2;
+
+    // staging roles: thread -> (row | column, block of the trip)
+    const int srow = tid >> 2, sq = tid & 3;
+    const int wrow_c = min(n0 + srow, w.N - 1), ycol_c = min(m0 + srow, a.M - 1);
+    const uint8_t * const wblk = WP ? w.W + (size_t) (wrow_c >> 5) * (size_t) trips * 4352 + (size_t) sq * 1024 + (size_t) (wrow_c & 31) * 16 : w.W + (size_t) wrow_c * w.w_nb1 + (size_t) sq * 34;
+    const uint8_t * const wscale = WP ? w.W + (size_t) (wrow_c >> 5) * (size_t) trips * 4352 + 4096 + (size_t) sq * 64 + (size_t) (wrow_c & 31) * 2 : wblk;
+    const char * const ytile = a.act + ((size_t) (ycol_c >> 5) * (size_t) nb32 + (size_t) sq) * 1152;
+    const int off0 = sw_offq(srow, 2 * sq), off1 = sw_offq(srow, 2 * sq + 1);
+
+    uint4 ga0, ga1, gb0, gb1;
+    uint16_t gad = 0;
+    float gbd = 0.0f;
+    auto issue_loads = [&](const int c) {
+        if constexpr (WP) {
+            ga0 = *(const uint4 *) (wblk + (size_t) c * 4352);
+            ga1 = *(const uint4 *) (wblk + (size_t) c * 4352 + 512);
+            gad = *(const uint16_t *) (wscale + (size_t) c * 4352);
+        } else {
+            const uint8_t * p = wblk + (size_t) c * 4 * 34;  // (blocks are 2-byte aligned)
+            gad = ld16(p);
+            ga0 = make_uint4(ld32_a2(p + 2), ld32_a2(p + 6), ld32_a2(p + 10), ld32_a2(p + 14));
+            ga1 = make_uint4(ld32_a2(p + 18), ld32_a2(p + 22), ld32_a2(p + 26), ld32_a2(p + 30));
+        }
+        const char * yt = ytile + (size_t) c * 4 * 1152;
+        gb0 = *(const uint4 *) (yt + (ycol_c & 31) * 16);
+        gb1 = *(const uint4 *) (yt + 512 + (ycol_c & 31) * 16);
+        gbd = *(const float *) (yt + 1024 + (ycol_c & 31) * 4);
+    };
+    auto stage = [&](const int t) {
+        char * buf = smem + (t & 1) * Q80_STAGE;
+        *(uint4 *) (buf + off0) = ga0;
+        *(uint4 *) (buf + off1) = ga1;
+        *(uint4 *) (buf + Q80_T + off0) = gb0;
+        *(uint4 *) (buf + Q80_T + off1) = gb1;
+        ((float *) (buf + 2 * Q80_T))[sq * 128 + srow] = h2f(gad);              // scales are stored [block][row] so that the four
+        ((float *) (buf + 2 * Q80_T + 128 * 16))[sq * 128 + srow] = gbd;        // consecutive rows of an accumulator quad are one 16-byte read
+    };
+    auto next = [&](const int c) { return c + 4 < trips ? c + 4 : (c & 3) + 1; };  // the chunk behind chunk c: 0, 4, 8, .., 1, 5, ..
+
+    const int fr = lane & 31, kg = lane >> 5;
+    const int swz = (fr >> 1) & 7;
+    const int arow_off = (nslab * 32 + fr) * 128;
+    const int brow_off0 = (mhalf * 64 + fr) * 128, brow_off1 = (mhalf * 64 + 32 + fr) * 128;
+    float C0[16], C1[16], S0[16], S1[16];
+    int16q zi;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) { C0[r] = 0.0f; C1[r] = 0.0f; zi[r] = 0; }
+
+    int c = 0, cl = 0;  // the chunk multiplied, the chunk loaded last
+    issue_loads(0);
+    stage(0);
+    if (trips > 1) { cl = next(0); issue_loads(cl); }
+    __syncthreads();
+    for (int t = 0; t < trips; ++t) {
+        if (t + 1 < trips) {
+            stage(t + 1);
+            if (t + 2 < trips) { cl = next(cl); issue_loads(cl); }
+        }
+        const char * buf = smem + (t & 1) * Q80_STAGE;
+        const float * dwt = (const float *) (buf + 2 * Q80_T);
+        const float * dat = (const float *) (buf + 2 * Q80_T + 128 * 16);
+#pragma unroll
+        for (int blk = 0; blk < 4; ++blk) {
+            const int co = ((2 * blk + kg) ^ swz) << 4;
+            const int4q fa = *(const int4q *) (buf + arow_off + co);
+            const int4q fb0 = *(const int4q *) (buf + Q80_T + brow_off0 + co), fb1 = *(const int4q *) (buf + Q80_T + brow_off1 + co);
+            const float y0 = dat[blk * 128 + mhalf * 64 + fr], y1 = dat[blk * 128 + mhalf * 64 + 32 + fr];
+            float x[16];  // block scale of the 16 rows this lane's accumulator registers belong to
+#pragma unroll
+            for (int g4 = 0; g4 < 4; ++g4) {
+                const float4 v = *(const float4 *) (dwt + blk * 128 + nslab * 32 + 8 * g4 + 4 * kg);
+                x[4 * g4] = v.x; x[4 * g4 + 1] = v.y; x[4 * g4 + 2] = v.z; x[4 * g4 + 3] = v.w;
+            }
+            const int16q s0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa, fb0, zi, 0, 0, 0);
+            const int16q s1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa, fb1, zi, 0, 0, 0);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                C0[r] = __builtin_fmaf((float) s0[r], x[r] * y0, C0[r]);
+                C1[r] = __builtin_fmaf((float) s1[r], x[r] * y1, C1[r]);
+            }
+        }
+        const int cn = next(c);
+        if ((cn & 3) != (c & 3)) {  // (the last chunk of a sum; past the last sum nothing reads C)
+            const bool first = (c & 3) == 0;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                S0[r] = first ? C0[r] : S0[r] + C0[r];
+                S1[r] = first ? C1[r] : S1[r] + C1[r];
+                C0[r] = 0.0f;
+                C1[r] = 0.0f;
+            }
+        }
+        c = cn;
+        __syncthreads();
+    }
+#pragma unroll
+    for (int tt = 0; tt < 2; ++tt) {
+        const int m = m0 + mhalf * 64 + tt * 32 + fr;
+        if (m >= a.M) continue;
+        float * out = w.dst + (size_t) m * w.dst_stride;
+        const float * ad = w.add ? w.add + (size_t) m * w.add_stride : nullptr;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const int n = n0 + nslab * 32 + 8 * g + 4 * kg;
+            float c4[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) c4[r] = tt ? S1[4 * g + r] : S0[4 * g + r];
+            if (ad) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) if (n + r < w.N) c4[r] += ad[n + r];
+            }
+            if (n + 3 < w.N && ((((uintptr_t) (out + n)) & 15) == 0)) {
+                *(float4 *) (out + n) = make_float4(c4[0], c4[1], c4[2], c4[3]);
+            } else {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) if (n + r < w.N) out[n + r] = c4[r];
+            }
+        }
+    }
+}
+
 bool mmq_q80_batch_supported(int type, int64_t K, int64_t N, int64_t M) {
     static const bool on = !getenv("GGML_MI355X_Q80_SKINNY") || atoi(getenv("GGML_MI355X_Q80_SKINNY")) != 0;
     return (on || M > 32) && type == GGML_TYPE_Q8_0 && (K % 128) == 0 && N >= 1 && M >= 9;  // (off: the mat-vec passes up to 32 columns)
 }
-// n matrices (1 .. 3) over the same activations; panels[q] != nullptr for ALL of them or for none (the template form is per launch)
-void launch_mmq_q80_multi(hipStream_t s, int n, const mmq80s_desc * mats, int K, int M, const void * act_q80) {
+// Tiles of 128 x 128 instead of the column kernel (N: rows of all matrices of the launch)?  Measured (us, one product with its quantiser, tiles / columns):
+// - K of one or two chunks: from about two million outputs on.  K 128, 5632 x 256 10.8 / 9.2, 4096 x 512 10.6 / 12.5, 14336 x 512 19.9 / 27.4; K 256, 4096 x 384 12.9 / 10.5,
+//   4096 x 512 13.4 / 13.5, 14336 x 512 24.4 / 29.5.  K 512, up to 512 columns: 14336 x 384 31.2 / 27.5, 14336 x 512 31.9 / 33.3, 32000 x 256 32.4 / 36.2.
+// - without a panel copy, any K: K 2048, 4000 x 512 47.8 / 41.6, 5600 x 512 45.8 / 56.4, 14000 x 256 45.2 / 65.8; K 5632, 5600 x 512 104.8 / 110.8, 14000 x 512 197 / 244.
+// With a panel copy and longer rows the column kernel wins everywhere: K 2048, 14336 x 512 77.4 / 61.1, 32000 x 2048 570 / 438.
+static bool q80_tile_pays(int64_t K, int64_t N, int64_t M, bool panels) {
+    if (K <= 256) return N * M >= ((int64_t) 15 << 17);
+    if (!panels) return N * M >= ((int64_t) 5 << 19);
+    return K <= 512 && M <= 512 && N * M >= ((int64_t) 7 << 20);
+}
+// n matrices (1 .. 3) over the same activations; returns the launches; panels[q] != nullptr for ALL of them or for none (the template form is per launch)
+int launch_mmq_q80_multi(hipStream_t s, int n, const mmq80s_desc * mats, int K, int M, const void * act_q80) {
     mmq80s_args a;
     int pe = 0;
     const bool wp = mats[0].W_panels != nullptr;
@@ -277,12 +429,28 @@ void launch_mmq_q80_multi(hipStream_t s, int n, const mmq80s_desc * mats, int K,
     if (M <= 32) {
         if (wp) hipLaunchKernelGGL(k_mmq_q80_skinny<true>, dim3((unsigned) pe), dim3(Q80S_WV * 64), 0, s, a);
         else hipLaunchKernelGGL(k_mmq_q80_skinny<false>, dim3((unsigned) pe), dim3(Q80S_WV * 64), 0, s, a);
-        return;
+        return 1;
     }
-    const int m_tiles = (M + 63) / 64;
-    const dim3 grid((unsigned) ((pe + 7) / 8 * 8 * m_tiles)), block(Q80C_WV * 64);
+    int64_t n_total = 0;
+    for (int q = 0; q < n; ++q) n_total += mats[q].N;
+    if (q80_tile_pays(K, n_total, M, wp)) {
+        for (int q = 0; q < n; ++q) {
+            mmq80s_args one = a;
+            one.m[0] = a.m[q];
+            const int np = (mats[q].N + 127) / 128, mt = (M + 127) / 128;
+            static std::atomic<uint32_t> raised{0}, raised_p{0};  // one bit per device (common.h: ensure_dyn_lds)
+            (void) ensure_dyn_lds(wp ? (const void *) k_mmq_q80_tile<true> : (const void *) k_mmq_q80_tile<false>, 2 * (size_t) Q80_STAGE, wp ? raised_p : raised);  // on failure the launch below fails and graph_compute reports it
+            const dim3 grid((unsigned) ((np + 7) / 8 * 8 * mt));
+            if (wp) hipLaunchKernelGGL(k_mmq_q80_tile<true>, grid, dim3(512), 2 * Q80_STAGE, s, one, np, mt);
+            else hipLaunchKernelGGL(k_mmq_q80_tile<false>, grid, dim3(512), 2 * Q80_STAGE, s, one, np, mt);
+        }
+        return n;
+    }
+    const int tiles = (M + 63) / 64, groups = (tiles + 15) / 16, m_tiles = (tiles + groups - 1) / groups;
+    const dim3 grid((unsigned) ((pe + 7) / 8 * 8 * m_tiles), (unsigned) groups), block(Q80C_WV * 64);
     if (wp) hipLaunchKernelGGL(k_mmq_q80_cols<true>, grid, block, 0, s, a, pe, m_tiles);
     else hipLaunchKernelGGL(k_mmq_q80_cols<false>, grid, block, 0, s, a, pe, m_tiles);
+    return 1;
 }
 void launch_mmq_q80(hipStream_t s, const uint8_t * W, const uint8_t * W_panels, int64_t w_nb1, int K, int N, int M, const void * act_q80, float * dst, int64_t dst_stride, const float * add,
                            int64_t add_stride) {

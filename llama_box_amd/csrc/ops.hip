@@ -40,7 +40,7 @@ __device__ __forceinline__ float block_max_f(float v, float * sh) {
 // ggml_compute_forward_rms_norm_f32: sum of squares accumulated in double, scale = 1/sqrtf(mean + eps), y = x*scale;
 // optional fused `* w` (the MUL node that always follows in llm_build_*)
 // one 32-value block of a row, held four values a lane by eight consecutive lanes, quantised as k_quantize_q8_0 does it and written in PANEL order (quantize.hip;
-// mmq_q80.hip: the 9 .. 128-column kernel's activations): row = column index, blk = block index along K
+// mmq_q80.hip: the activations of its kernels): row = column index, blk = block index along K
 __device__ __forceinline__ void q80_panel_store(const float r0, const float r1, const float r2, const float r3, const int w8, const int64_t row, const int64_t blk, const int64_t nblk, char * __restrict__ dst) {
     float amax = fmaxf(fmaxf(fabsf(r0), fabsf(r1)), fmaxf(fabsf(r2), fabsf(r3)));
     amax = fmaxf(amax, __shfl_xor(amax, 1, 64));

@@ -13,11 +13,10 @@ import llama_box_amd as L
 pytestmark = pytest.mark.gpu
 
 
-# (K, N, M): one column tile and its neighbours, a half-empty tile, K of fewer chunks than partial sums, rows that are no whole panel (no panel copy),
-# and tile counts on both sides of the line between the two splits
+# (K, N, M): one column tile and its neighbours, a half-empty tile, K of fewer chunks than partial sums, rows that are no whole panel (no panel copy), many rows and columns (128 x 128 tiles)
 @pytest.mark.parametrize("K,N,M", [(128, 32, 33), (256, 33, 64), (1024, 96, 65), (2048, 160, 97), (640, 70, 129), (1152, 64, 200), (256, 4096, 960), (384, 4096, 1024), (256, 4128, 1057), (128, 4100, 1030)])
 def test_q8_0_batches_of_33_columns_and_up(backend, H, K, N, M):
-    """mmq_q80.hip: k_mmq_q80_cols — the same bits for a column whatever batch it is in (one wave per tile or four), and the oracle's values."""
+    """mmq_q80.hip: k_mmq_q80_cols / k_mmq_q80_tile — the same bits for a column in any batch of 33 columns and more, and the oracle's values."""
     rng = np.random.default_rng(K + N + M)
     w = T.rand_weight(L.Q8_0, K, N, rng)
     x = (rng.standard_normal((M, K)) * rng.uniform(0.2, 3.0, (M, 1))).astype(np.float32)
@@ -34,7 +33,7 @@ def test_q8_0_batches_of_33_columns_and_up(backend, H, K, N, M):
     assert backend.stat("skinny_launches") == s0 + 1
     for c, e in {(0, 33), (max(0, M - 63), M), (M // 2, min(M, M // 2 + 40))}:
         if e - c < 33:
-            continue  # (another kernel)
+            continue  # (another kernel: eight partial sums, not four)
         part = T.run_case(build(c, e), backend)[0].reshape(e - c, N)
         assert np.array_equal(got[c:e].view(np.uint32), part.view(np.uint32)), (c, e)
     rows = np.unique(np.concatenate([np.arange(min(N, 40)), np.arange(max(0, N - 40), N)]))  # (the oracle on the first and last rows)
@@ -322,6 +321,44 @@ def test_16_bit_matrices_around_the_lines_of_the_choice(backend, H, wt, K, N, M,
         assert np.abs(r - ref).max() <= 6e-8 * np.sqrt(K) * 8
     if tiled:
         assert np.array_equal(got.view(np.uint32), tiles.view(np.uint32))
+
+
+# 128 x 128 tiles (short rows and many outputs; without a panel copy at any length) and the column kernel in one and two groups of column tiles; rows and columns that end inside a tile
+@pytest.mark.parametrize("panels", [False, True])
+@pytest.mark.parametrize("K,N,M", [(128, 4128, 600), (256, 2080, 1025), (384, 96, 1030), (1152, 1088, 2500), (128, 64, 1100), (640, 3008, 1090), (512, 14336, 512)])
+def test_q8_0_batches_with_and_without_the_panel_copy(backend, H, panels, K, N, M):
+    """mmq_q80.hip from 33 columns: the bits of a column are those of 40 columns alone (always the column kernel), and its values the oracle's."""
+    rng = np.random.default_rng(K + N + M)
+    w = T.rand_weight(L.Q8_0, K, N, rng)
+    x = (rng.standard_normal((M, K)) * rng.uniform(0.2, 3.0, (M, 1))).astype(np.float32)
+    r = rng.standard_normal((M, N)).astype(np.float32)
+
+    def run(c0, c1):
+        g = T.G(backend)
+        try:
+            out = H.ggml_add(g.ctx, H.ggml_mul_mat(g.ctx, g.new(L.Q8_0, [K, N], w), g.new(L.F32, [K, c1 - c0], x[c0:c1])), g.new(L.F32, [N, c1 - c0], r[c0:c1]))
+            got = g.compute([out])[0]
+            if panels:  # the same graph again, over a weights buffer
+                p0 = backend.stat("decode_copy_launches")
+                H.ggml_backend_buffer_set_usage(g.buf, 1)
+                assert H.ggml_backend_graph_compute(backend.backend, g.gf) == 0
+                assert backend.stat("decode_copy_launches") == p0 + 1
+                got = g.read(out)
+            return got.reshape(c1 - c0, N)
+        finally:
+            g.free()
+
+    backend.set_option("graphs", 0)
+    try:
+        got = run(0, M)
+        for c in (0, M // 2, M - 40):
+            assert np.array_equal(got[c:c + 40].view(np.uint32), run(c, c + 40).view(np.uint32)), c
+    finally:
+        backend.set_option("graphs", 1)
+    rows = np.unique(np.concatenate([np.arange(40), np.arange(N - 40, N)]))
+    wr, rr = np.ascontiguousarray(w[rows]), np.ascontiguousarray(r[:, rows])
+    ref = T.run_case(lambda g: H.ggml_add(g.ctx, H.ggml_mul_mat(g.ctx, g.new(L.Q8_0, [K, len(rows)], wr), g.new(L.F32, [K, M], x)), g.new(L.F32, [len(rows), M], rr)), "oracle")[0].reshape(M, -1)
+    assert T.nmse(got[:, rows], ref) <= 1e-10
 
 
 def test_q8_0_batches_without_the_skinny_kernel(built):
