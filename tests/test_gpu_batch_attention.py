@@ -59,10 +59,13 @@ def test_few_tokens_over_listed_cells(backend, H, T_, NKV, G, per):
         assert np.abs(got[h] - ref).max() <= 2e-3 * np.abs(ref).max() + 1e-5, h
 
 
-@pytest.mark.parametrize("T_,NKV,G,per", [(2, 2, 1, 9), (3, 8, 4, 300), (17, 2, 3, 40), (32, 8, 4, 30)])
-def test_few_tokens_feed_a_quantised_matrix(backend, H, T_, NKV, G, per):
-    """... -> CONT(PERMUTE) -> MUL_MAT with a K-quant: the copy and its quantiser as one launch, or none, against the same graph node by node: only a Q8_K code next to a
-    rounding boundary may differ (1e-5 of the product's size)."""
+# slices of the head dimensions (dq > 1: few tokens) and whole rows, an even and an odd number of heads on a key head
+@pytest.mark.parametrize("recycled", [False, True])
+@pytest.mark.parametrize("T_,NKV,G,per,dq", [(2, 2, 1, 9, 8), (3, 8, 4, 300, 8), (17, 2, 3, 40, 8), (20, 8, 2, 12, 2), (32, 8, 4, 30, 1), (32, 8, 3, 30, 1)])
+def test_few_tokens_feed_a_quantised_matrix(backend, H, T_, NKV, G, per, dq, recycled):
+    """... -> CONT(PERMUTE) -> MUL_MAT with a K-quant, the copy in a block of its own or in q's (where the graph allocator puts it).  No launch copies: the attention kernel writes the
+    copy or, from whole rows of head pairs, its Q8_K blocks; where it may not write to q's block because other slices still read it, the quantiser takes the heads from the
+    product.  Against the same graph node by node: only a Q8_K code next to a rounding boundary may differ (1e-5 of the product's size)."""
     rng = np.random.default_rng(T_ + 31 * per + G)
     HD, NH, n_kv, N = 128, NKV * G, max(256, (T_ * per + 255) // 256 * 256), 96
     k = rng.standard_normal((n_kv, NKV * HD)).astype(np.float16)
@@ -73,19 +76,29 @@ def test_few_tokens_feed_a_quantised_matrix(backend, H, T_, NKV, G, per):
     for t in range(T_):
         mask[t, rng.choice(n_kv, per, replace=False)] = 0
 
-    def build(g):
-        q = H.ggml_mul_mat(g.ctx, g.new(L.Q4_K, [256, NH * HD], wq), g.new(L.F32, [256, T_], x))  # (the allocator may give q's block to the copy)
-        qp = H.ggml_permute(g.ctx, H.ggml_reshape_3d(g.ctx, q, HD, NH, T_), 0, 2, 1, 3)
-        kv = H.ggml_view_3d(g.ctx, g.new(L.F16, [NKV * HD, n_kv], k), HD, n_kv, NKV, NKV * HD * 2, HD * 2, 0)
-        vv = H.ggml_view_3d(g.ctx, g.new(L.F16, [n_kv, NKV * HD], v), n_kv, HD, NKV, n_kv * 2, n_kv * 2 * HD, 0)
-        p = H.ggml_soft_max_ext(g.ctx, H.ggml_mul_mat(g.ctx, kv, qp), g.new(L.F32, [n_kv, T_], mask), HD ** -0.5, 0.0)
-        o = H.ggml_cont_2d(g.ctx, H.ggml_permute(g.ctx, H.ggml_mul_mat(g.ctx, vv, p), 0, 2, 1, 3), NH * HD, T_)
-        return H.ggml_mul_mat(g.ctx, g.new(L.Q4_K, [NH * HD, N], wo), o)
+    def run(whole):  # the launches up to wo's product, or the product
+        g = T.G(backend)
+        try:
+            q = H.ggml_mul_mat(g.ctx, g.new(L.Q4_K, [256, NH * HD], wq), g.new(L.F32, [256, T_], x))
+            qp = H.ggml_permute(g.ctx, H.ggml_reshape_3d(g.ctx, q, HD, NH, T_), 0, 2, 1, 3)
+            kv = H.ggml_view_3d(g.ctx, g.new(L.F16, [NKV * HD, n_kv], k), HD, n_kv, NKV, NKV * HD * 2, HD * 2, 0)
+            vv = H.ggml_view_3d(g.ctx, g.new(L.F16, [n_kv, NKV * HD], v), n_kv, HD, NKV, n_kv * 2, n_kv * 2 * HD, 0)
+            p = H.ggml_soft_max_ext(g.ctx, H.ggml_mul_mat(g.ctx, kv, qp), g.new(L.F32, [n_kv, T_], mask), HD ** -0.5, 0.0)
+            o = H.ggml_cont_2d(g.ctx, H.ggml_permute(g.ctx, H.ggml_mul_mat(g.ctx, vv, p), 0, 2, 1, 3), NH * HD, T_)
+            r = H.ggml_mul_mat(g.ctx, g.new(L.Q4_K, [NH * HD, N], wo), o) if whole else H.ggml_mul_mat(g.ctx, g.new(L.Q4_K, [256, NH * HD], wq), g.new(L.F32, [256, T_], x))
+            k0 = backend.stat("kernel_launches")
+            out = g.compute([r], same_block=[(o, q)] if recycled else [])[0]
+            return out, backend.stat("kernel_launches") - k0
+        finally:
+            g.free()
 
-    got = T.run_case(build, backend)[0]
+    got, launches = run(True)
+    product = 1 + (NH * HD // 256 >= 8)  # wo: K slices and their sum from eight super-blocks on
+    quantised = 0 if dq == 1 and G % 2 == 0 else 1
+    assert launches == run(False)[1] + 2 + quantised + product, launches  # (q; the lists, the chain)
     backend.set_option("fusion", 0)
     try:
-        plain = T.run_case(build, backend)[0]
+        plain, _ = run(True)
     finally:
         backend.set_option("fusion", 1)
     assert T.nmse(got, plain) <= 1e-5
