@@ -423,10 +423,7 @@ template <int QT, int BN, int BM = 128> static void launch_mmq8_t(hipStream_t s,
 
 // few activation columns (continuous-batching decode, M <= 64) leave N/64 x 1 workgroups — far fewer than 256 CUs — so
 // the K range is split over blockIdx.y and the partial products are summed in a fixed order by a second tiny kernel
-int mmq_pick_ksplit(int64_t K, int64_t N, int64_t M, bool skinny, int type) {
-    if (skinny && M >= 2 && M <= 32 && (N % 32) == 0) return mmq_skinny_ksplit(K, N);
-    // prompt batches on the wide forms of mmq_skinny.hip: without a K split where the grid fills the chip by token-tile groups, with their own slices otherwise
-    if (const int ks = skinny ? mmq_wide_ksplit(type, K, N, M) : 0) return ks;
+int mmq_tiled_ksplit(int64_t K, int64_t N, int64_t M) {
     const int64_t wgs = ((N + 63) / 64) * ((M + 127) / 128), nblk = K / 256;
     static const int ks_target = getenv("GGML_MI355X_MMQ_KS_TARGET") ? atoi(getenv("GGML_MI355X_MMQ_KS_TARGET")) : 512;
     if (M <= 64) return (int) std::max<int64_t>(1, std::min<int64_t>(nblk, ks_target / std::max<int64_t>(1, wgs)));
@@ -435,6 +432,12 @@ int mmq_pick_ksplit(int64_t K, int64_t N, int64_t M, bool skinny, int type) {
     if (wgs < 256) return (int) std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(4, nblk / 4), 256 / wgs));
     if (wgs == 256 && nblk >= 32) return 2;
     return 1;
+}
+int mmq_pick_ksplit(int64_t K, int64_t N, int64_t M, bool skinny, int type) {
+    if (skinny && M >= 2 && M <= 32 && (N % 32) == 0) return mmq_skinny_ksplit(K, N);
+    // prompt batches on the wide forms of mmq_skinny.hip: without a K split where the grid fills the chip by token-tile groups, with their own slices otherwise
+    if (const int ks = skinny ? mmq_wide_ksplit(type, K, N, M) : 0) return ks;
+    return mmq_tiled_ksplit(K, N, M);
 }
 // can matrices of these K-quant types (same K, same activations) share one launch of 2..32 columns?
 bool mmq_skinny_mix_ok(const int * types, const int64_t * N, const int64_t * w_nb1, int n, int64_t K, int64_t M) {

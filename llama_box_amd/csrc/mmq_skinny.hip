@@ -1472,35 +1472,39 @@ __global__ void __launch_bounds__((WD_NW + WD_NL) * 64, 1) k_mmq_wide_few(const 
 static int64_t wide_row_bytes(int type, int64_t K) { return K / 256 * (type == GGML_TYPE_Q4_K ? 144 : type == GGML_TYPE_Q5_K ? 176 : 210); }
 // three token tiles a workgroup where they waste fewer columns than two (Q5_K: their registers do not fit)
 static int few_tiles(int type, int64_t M) { return type != GGML_TYPE_Q5_K && (M + 95) / 96 * 96 < (M + 63) / 64 * 64 ? 3 : 2; }
+// (row group, token tile) items of n rows as the kernels deal them out: row groups in eights, one per XCD, the last eight not always whole.  36 groups are dealt as 40: seven slices of
+// them would be a second round for the workgroups that draw the 257th item and up (4608 x 4096 x 77, Q4_K: 20.8 us against 13.7 for the 4096 rows beside it)
+static int64_t dealt_items(int64_t n, int64_t M, int64_t tt) { return (n / 128 + 7) / 8 * 8 * ((M + 32 * tt - 1) / (32 * tt)); }
 static int64_t few_slices(int64_t K, int64_t items) { return std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(8, K / 512), skinny_n_cu() / items)); }
-// Is k_mmq_wide_few the fastest for n rows in all?  Both sides measured, one product with its quantiser and its sum of slices, at 2748 points of K 256 .. 14336, n 128 .. 28672,
-// 33 .. 384 columns (us, other kernel / k_mmq_wide_few, n x K); what this rule picks is within 5 % of the better one at all but 40 of them.
-// - Against k_mmq_wide: by steps of a workgroup, (token tiles + 2) quarters each, the slices' sum as six steps.  Q4_K, 77 columns, 28672 x 4096 51.1 / 39.4 (one round of three
-//   tiles for two of two), 8192 x 4096 28.9 / 26.2 (4 slices), 14336 x 2048 20.5 / 25.8; 257 columns, 8192 x 4096 51.9 / 39.4, 6144 x 4096 32.8 / 38.0.
-// - Against the tiled GEMM, whose own K split and small tiles win where a slice is short or the rows are few: by format and columns.
-//   64: Q4_K 2048 x 2048 14.5 / 15.7, 3072 x 2048 16.6 / 16.1, 512 x 8192 21.3 / 19.3; Q6_K 4096 x 4096 21.3 / 23.1, 14336 x 4096 35.6 / 32.4.
-//   77: Q4_K 1024 x 1024 14.3 / 14.9, 2048 x 2048 17.8 / 17.3, 6144 x 2048 19.4 / 20.1, 4096 x 4096 20.8 / 23.3, 6144 x 4096 28.9 / 24.4; Q5_K 1024 x 1024 17.4 / 14.5;
-//   Q6_K 2048 x 2048 18.9 / 19.3, 4096 x 14336 46.8 / 38.0.
-//   160: Q4_K 4096 x 512 11.0 / 11.9, 4096 x 2048 20.8 / 20.0; Q6_K 1024 x 1024 15.8 / 16.0, 4096 x 2048 22.1 / 23.4, 14336 x 4096 (two rounds) 63.1 / 79.7.
-//   300: eight slices' sum is too much for few rows: Q4_K 256 x 4096 21.1 / 24.6.
+// do k_mmq_wide's row groups (g128 of them) and 64-column groups occupy half the chip?
+static bool wide_fills(int type, int64_t g128, int64_t M) { return type != GGML_TYPE_Q6_K && g128 * ((M + 63) / 64) * 2 >= skinny_n_cu(); }
+// Is k_mmq_wide_few the fastest for n rows in all?  By the time each kernel takes in its own steps: a start, the steps one after the other (super-blocks of a K slice x rounds over the chip), what a
+// further round adds.  Constants in us, fitted to the median launches of all of them over 5096 points (Q4_K, Q5_K, Q6_K; K 256 .. 14336, n 128 .. 28672, 33 .. 384 columns) whose weights came
+// from memory, as in a pass over a model: repeated over weights that the last-level cache holds, the tiled GEMM looks up to a quarter better than it is.  The sum of K slices counts half
+// (2.4 us): more often than not the next kernel makes it.  The pick is the slower one by more than 5 % at 74 of the points, by 15 % at most; what it decides, other kernel / this one:
+// - Against k_mmq_wide: Q4_K, 77 columns, 28672 x 4096 53.8 / 38.8 (one round of three tiles for two of two), 14336 x 2048 17.5 / 16.5 and the sum of two slices.
+// - Against the tiled GEMM, whose workgroups share a CU and whose own K slices are at most four from 65 columns on: Q4_K, 77 columns, 5120 x 4096 18.8 / 15.1, 1024 x 2048 12.6 / 10.0,
+//   4096 x 512 8.1 / 9.8; Q6_K, 160 columns, 5120 x 4096 43.4 / 26.3, 14336 x 4096 66.1 / 81.4; up to 64 columns it slices as finely as this one: Q6_K, 128 x 5120 x 64 6.2 / 12.6.
 static bool few_pays(int type, int64_t K, int64_t n, int64_t M) {
-    const int64_t cu = skinny_n_cu(), nblk = K / 256, tt = few_tiles(type, M), items = n / 128 * ((M + 32 * tt - 1) / (32 * tt)), ks = few_slices(K, items), rounds = (items * ks + cu - 1) / cu;
-    const bool q5 = type == GGML_TYPE_Q5_K, q6 = type == GGML_TYPE_Q6_K;
-    const int64_t wide_items = n / 128 * ((M + 63) / 64);
-    if (!q6 && wide_items * 2 >= cu) return rounds * ((nblk + ks - 1) / ks) * (tt + 2) + (ks > 1 ? 24 : 0) < (wide_items + cu - 1) / cu * nblk * 4;
-    if (q6 && !(rounds == 1 || (tt == 3 && items * 8 >= rounds * cu * 7))) return false;
-    if (M <= 64) return n * K >= (q6 ? (int64_t) 36 << 20 : (int64_t) 6 << 20) || (!q6 && K >= 8192);
-    if (M <= 96) {
-        if (q5) return K >= 1024;
-        if (q6) return K >= 8192 || n * K >= (int64_t) 20 << 20;
-        return K >= 2048 && !(K < 3584 && n > 4096) && !(K >= 4096 && K < 8192 && n > 1024 && n < 6144);
+    const int64_t cu = skinny_n_cu(), nblk = K / 256, tt = few_tiles(type, M), items = dealt_items(n, M, tt), ks = few_slices(K, items);
+    const int f = type == GGML_TYPE_Q4_K ? 0 : type == GGML_TYPE_Q5_K ? 1 : 2;
+    auto up = [](int64_t a, int64_t b) { return (double) ((a + b - 1) / b); };
+    struct form { double start, step, round; };
+    static const form FEW2[3] = {{6.2, 1.48, 2.5}, {6.1, 2.04, 2.5}, {6.6, 2.42, 2.1}}, FEW3[3] = {{6.9, 1.96, 3.1}, {0, 0, 0}, {7.8, 2.94, 2.2}}, WIDE[2] = {{5.5, 1.40, 2.3}, {5.6, 1.89, 2.4}};
+    // a step with r workgroups on a CU: step + shared r; up to 64 columns (tiles of 64) and beyond (of 128)
+    struct tile { double start, per_wg, step, shared; };
+    static const tile TILE64[3] = {{3.5, 0.93, 0.18, 1.28}, {3.2, 0.97, 0.0, 2.53}, {3.5, 0.95, 0.0, 1.63}}, TILE128[3] = {{2.9, 1.0, 1.13, 1.13}, {3.4, 0.4, 1.45, 1.45}, {2.0, 2.0, 1.06, 1.52}};
+    const double slices_sum = 2.4;
+    const form & w = tt == 3 ? FEW3[f] : FEW2[f];
+    const double rounds = up(items * ks, cu), few = w.start + w.step * up(nblk, ks) * rounds + w.round * (rounds - 1) + (ks > 1 ? slices_sum : 0);
+    if (wide_fills(type, n / 128, M)) {
+        const double r = up(dealt_items(n, M, 2), cu);
+        return few < WIDE[f].start + WIDE[f].step * nblk * r + WIDE[f].round * (r - 1);
     }
-    if (M <= 256) {
-        if (q6) return K >= 8192 ? n <= 6144 || M <= 128 : K >= 2048 && (n <= 1024 || (K >= 3584 && n >= 6144));
-        return K >= 2048 || (K >= 1024 && (q5 || n <= 1024));
-    }
-    if (q6) return K >= 8192 ? n >= 1024 : (K >= 3584 && n >= 3072) || (K >= 2048 && n >= 6144);
-    return K >= (q5 ? 1024 : 2048) && !(n <= 768 && K >= 3072 && K < 8192);
+    const int64_t tks = mmq_tiled_ksplit(K, n, M);
+    const tile & t = M <= 64 ? TILE64[f] : TILE128[f];
+    const double r = up((n + 63) / 64 * ((M + 127) / 128) * tks, cu);
+    return few < t.start + t.per_wg * r + (t.step + t.shared * r) * up(nblk, tks) + (tks > 1 ? slices_sum : 0);
 }
 int mmq_wide_form(int type, int64_t K, const int64_t * N, int n_mat, int64_t M, int64_t w_nb1) {
     static const bool on = !getenv("GGML_MI355X_MMQ_WIDE") || atoi(getenv("GGML_MI355X_MMQ_WIDE")) != 0;
@@ -1514,11 +1518,11 @@ int mmq_wide_form(int type, int64_t K, const int64_t * N, int n_mat, int64_t M, 
         g128 += N[i] / 128;
     }
     if (M <= WD_FEW && few_pays(type, K, 128 * g128, M)) return few_tiles(type, M);
-    return type != GGML_TYPE_Q6_K && g128 * ((M + 63) / 64) * 2 >= skinny_n_cu() ? 1 : 0;
+    return wide_fills(type, g128, M) ? 1 : 0;
 }
 int mmq_wide_ksplit(int type, int64_t K, int64_t N, int64_t M) {
     const int form = mmq_wide_form(type, K, &N, 1, M, wide_row_bytes(type, K));
-    return form <= 1 ? form : (int) few_slices(K, N / 128 * ((M + 32 * form - 1) / (32 * form)));
+    return form <= 1 ? form : (int) few_slices(K, dealt_items(N, M, form));
 }
 
 template <int QT, int TT, int NW, int NL, int NSA> static void launch_wide_t(hipStream_t s, mmq8_args a) {

@@ -138,13 +138,14 @@ def test_k_quant_batches_by_groups_of_eight_columns(backend, H, qt, K, N):
 
 
 # one super-block and many, K slices of unequal lengths, two and three token tiles a workgroup with ragged ends, both sides of the lines between the kernels (f: k_mmq_wide_few,
-# w: k_mmq_wide, t: the tiled GEMM; for Q4_K, Q5_K, Q6_K), Q6_K rows of an odd number of blocks
+# w: k_mmq_wide, t: the tiled GEMM; for Q4_K, Q5_K, Q6_K), row groups that are not whole eights with as many slices as those allow, Q6_K rows of an odd number of blocks
 @pytest.mark.parametrize("qt", [L.Q4_K, L.Q5_K, L.Q6_K])
 @pytest.mark.parametrize("K,N,M,kernels", [
-    (256, 128, 33, "ttt"), (512, 256, 65, "ttt"), (4608, 128, 77, "fft"), (2560, 384, 96, "fft"), (1024, 4096, 97, "tft"), (768, 512, 129, "ttt"), (2048, 1024, 190, "fff"), (512, 8192, 288, "fwt"),
-    (1536, 640, 384, "tft"), (1536, 16384, 385, "wwt"),
-    (8192, 128, 33, "fft"), (8448, 256, 64, "fft"), (8704, 128, 65, "fff"), (1280, 256, 96, "tft"), (2560, 384, 97, "fff"), (2304, 512, 129, "fft"), (2048, 896, 256, "fff"), (2560, 896, 257, "fft"),
-    (3584, 3072, 288, "fff"), (8192, 1024, 384, "fff"), (8192, 4608, 33, "fff"), (512, 16384, 33, "wwt"), (512, 4096, 512, "wwt")])
+    (256, 128, 33, "ttt"), (512, 256, 65, "ttt"), (4608, 128, 77, "fff"), (2560, 384, 96, "fff"), (1024, 4096, 97, "fff"), (768, 512, 129, "fft"), (2048, 1024, 190, "fff"),
+    (512, 8192, 288, "fwf"), (1536, 640, 384, "fff"), (1536, 16384, 385, "wwt"), (8192, 128, 33, "ttt"), (8448, 256, 64, "ttt"), (8704, 128, 65, "fff"),
+    (1024, 1024, 77, "tft"), (2560, 384, 97, "fff"), (768, 2048, 77, "tft"), (2048, 896, 256, "fff"), (2560, 896, 257, "fff"), (3584, 3072, 288, "fff"),
+    (8192, 1024, 384, "fff"), (8192, 4608, 33, "fff"), (512, 16384, 33, "wwt"), (512, 4096, 512, "wwt"), (4096, 4608, 77, "fff"), (4096, 128, 384, "fft"),
+    (1536, 20480, 65, "fwf"), (1024, 24576, 64, "wwf")])
 def test_k_quant_batches_of_33_columns_and_up(backend, H, qt, K, N, M, kernels):
     """mmq_skinny.hip: k_mmq_wide_few / k_mmq_wide against the oracle and, the sums of the K slices apart, the tiled GEMM: exact integer block sums, f32 sums over K / 256 terms."""
     rng = np.random.default_rng(K + N + M)
