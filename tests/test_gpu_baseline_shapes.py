@@ -745,8 +745,9 @@ def test_layer_teacher_forced_batch(backend, H, plog, li, mode, fa):
             # 33 .. 160 columns, or a rank's narrow shards: a wide form where it applies, the tiled int8 GEMM otherwise — never the 32-column skinny kernel, never a column-by-column mat-vec fall-back (one launch per matrix group at most,
             # + split-K reduce / quantiser launches)
             assert cnt["skinny_launches"] == 0 and cnt["wide_launches"] + cnt["tiled_launches"] >= 1, (group, cnt)
-            if L.Q6_K in wtypes:  # (up to 384 columns: the wide form with K slices)
-                assert cnt["wide_few_launches" if M <= 384 else "tiled_launches"] >= 1, (group, cnt)
+            if L.Q6_K in wtypes:  # (up to 384 columns: the wide form with K slices, but for 8192 x 3584 x 160, which would be a second round of it for a few items)
+                tiled = M > 384 or (group.startswith("ffn_down") and (FF, E, M) == (3584, 8192, 160))
+                assert cnt["tiled_launches" if tiled else "wide_few_launches"] >= 1, (group, cnt)
             assert cnt["kernel_launches"] <= 12, (group, cnt)
 
     tag = f"{sp.name} [{mode}, {M} tokens, n_kv {n_kv}, fa={fa}]"
