@@ -576,7 +576,7 @@ static bool mm_tile_applies(const ggml_tensor * n) { return mm_tile_form(n) && m
 // ... and MUL_MAT_ID of as many (expert, token) columns as its batched form takes (src1's rows of all tokens dense)
 static bool mm_id_tile_applies(const ggml_tensor * n) {
     const ggml_tensor * a = n->src[0], * b = n->src[1], * ids = n->src[2];
-    return mul_mat_id_batched(TD(a), TD(b), TD(ids)) && ggml_abi_is_contiguous(b) && b->ne[3] == 1 && n->nb[0] == 4 && (size_t) ggml_abi_nelements(b) * 2 < ((size_t) 1 << 32) &&
+    return mul_mat_id_batched(TD(a), TD(b), TD(ids)) && mul_mat_id_tile_pays(a->ne[0], a->ne[1], (ids->ne[0] * ids->ne[1] + a->ne[2] - 1) / a->ne[2]) && ggml_abi_is_contiguous(b) && b->ne[3] == 1 && n->nb[0] == 4 && (size_t) ggml_abi_nelements(b) * 2 < ((size_t) 1 << 32) &&
            mul_mat_tile_ok(a->type, a->ne[0], a->ne[1], (int64_t) a->nb[0], (int64_t) a->nb[1], a->data);
 }
 // src1 rounded to the 16-bit type of src0, unless the scratch already holds exactly that (projections of one input)

@@ -170,6 +170,7 @@ bool mul_mat_tile_pays(int64_t K, int64_t N, int64_t M);  // ... faster than lau
 void launch_to_16(hipStream_t s, int type, const char * x, int64_t nb1, int64_t K, int64_t rows, void * out);
 // the experts' columns (lists: k_moe_group); x16 rows: src1's [n_b, T]
 void launch_mul_mat_id_tile(hipStream_t s, const tdesc & as, int64_t n_b, int64_t n_used, int64_t T, const tdesc & d, const int32_t * cnt, const int32_t * off, const int32_t * list, const void * x16);
+bool mul_mat_id_tile_pays(int64_t K, int64_t N, int64_t even);  // ... faster than mmf.hip's form for `even` columns an expert?
 bool mul_mat_id_batched(const tdesc & as, const tdesc & b, const tdesc & ids);  // does launch_mul_mat_id group the columns by expert?
 void launch_mul_mat_tile(hipStream_t s, int type, const mul_mat_tile_desc * m, int n, int64_t K, int64_t M, const void * x16);
 struct matvec_multi { const char * W[4]; int64_t nb1[4]; int64_t N[4]; float * dst[4]; int blk0[5]; int n; };

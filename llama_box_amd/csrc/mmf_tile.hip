@@ -233,6 +233,17 @@ bool mul_mat_tile_pays(int64_t K, int64_t N, int64_t M) {
     if (K < 384) return M > 32;
     return true;
 }
+// ... and the experts' columns, `even` of them for each when they are spread evenly: the rounding and tiles against mmf.hip's launch of one wave per 32 x 32 outputs, which lists and tiles of
+// few columns hardly fill.  The longer K, the earlier the tiles win.  Measured at 1592 shapes of 4 .. 128 experts of 32 .. 4096 rows (us, mmf.hip / tiles): K 64, 64 x 2048 x 16 columns 17.7 / 41.5
+// (every workgroup of 64 x 128 waits for its first stage); K 128 within 10 % from 64 columns on, 1.1 .. 1.5 times as long below; K 192, 128 rows x 32 1.03 times, x 64 0.97; K 256, 8 x 2048 x
+// 16 columns 11.8 / 12.1, x 32 17.0 / 13.5, 64 x 2048 x 2 22.3 / 33.7; K 384, 512 rows x 16 1.0 .. 1.08 times, 1408 rows 0.76 .. 0.94; K 512 at most 1.05 times, 0.4 .. 0.9 mostly; up to 32 rows, which
+// leave half a tile empty, K 512 x 16 1.05 times, x 32 0.94 .. 1.02, K 768 0.95.
+bool mul_mat_id_tile_pays(int64_t K, int64_t N, int64_t even) {
+    if (N < 64) return K >= 768 || (K >= 512 && even >= 32);
+    if (K >= 512) return true;
+    if (K >= 384) return even >= 24 || N >= 1024;
+    return (K >= 256 && even >= 24) || (K >= 192 && even >= 48);
+}
 void launch_to_16(hipStream_t s, int type, const char * x, int64_t nb1, int64_t K, int64_t rows, void * out) {
     const int64_t total = rows * (K / 8);
     const dim3 grid((unsigned) ((total + 255) / 256));

@@ -94,9 +94,12 @@ def test_16_bit_siblings_have_the_bits_of_single_launches(backend, H, M):
         assert np.abs(a.reshape(M, -1) - ref).max() <= 6e-8 * np.sqrt(K) * 8
 
 
-# columns of an expert: none, fewer than a tile, several tiles (one expert draws most)
-@pytest.mark.parametrize("K,N,n_exp,top,T_", [(64, 40, 5, 2, 40), (128, 200, 8, 1, 300), (192, 130, 3, 3, 70), (256, 4160, 6, 2, 100)])
-def test_experts_with_batches(backend, H, K, N, n_exp, top, T_):
+# columns of an expert: none, fewer than a tile, several tiles (one expert draws most); both sides of the lines between the tiles (whose input is rounded by a launch of its own) and mmf.hip's form
+@pytest.mark.parametrize("K,N,n_exp,top,T_,tiled", [
+    (64, 40, 5, 2, 40, False), (128, 200, 8, 1, 300, False), (192, 130, 3, 3, 70, True), (256, 4160, 6, 2, 100, True), (192, 130, 3, 3, 47, False), (192, 64, 4, 2, 96, True), (256, 70, 4, 1, 92, False),
+    (256, 70, 4, 1, 93, True), (384, 1000, 8, 2, 92, False), (384, 1024, 16, 1, 64, True), (448, 96, 8, 2, 93, True), (512, 64, 64, 4, 16, True), (512, 40, 8, 2, 124, False), (512, 40, 8, 2, 125, True),
+    (768, 33, 32, 2, 32, True), (1024, 300, 8, 2, 70, True)])
+def test_experts_with_batches(backend, H, K, N, n_exp, top, T_, tiled):
     rng = np.random.default_rng(K + N + T_)
     w = round16((rng.standard_normal((n_exp, N, K)) / np.sqrt(K)).astype(np.float32), L.BF16)
     x = rng.standard_normal((T_, 1, K)).astype(np.float32)
@@ -108,7 +111,9 @@ def test_experts_with_batches(backend, H, K, N, n_exp, top, T_):
     def build(g):
         return H.ggml_mul_mat_id(g.ctx, g.new(L.BF16, [K, N, n_exp], bits16(w, L.BF16)), g.new(L.F32, [K, 1, T_], x), g.new(L.I32, [top, T_], ids))
 
+    k0 = backend.stat("kernel_launches")
     got = T.run_case(build, backend)[0].reshape(T_, top, N)
+    assert backend.stat("kernel_launches") - k0 == (2 if tiled else 1)
     xr = round16(x, L.BF16).astype(np.float64)[:, 0]
     ref = np.stack([[w[ids[t, u]].astype(np.float64) @ xr[t] for u in range(top)] for t in range(T_)])
     assert np.abs(got - ref).max() <= 6e-8 * np.sqrt(K) * 8
