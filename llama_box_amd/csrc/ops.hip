@@ -141,71 +141,101 @@ void launch_rms_norm_mul_q80_panel(hipStream_t s, const tdesc & src, float eps, 
 // like RMS_NORM's).  w: optional weight of the MUL that follows; r: optional residual rows of the ADD behind that (same shape as the output).
 // second stage (w2 != nullptr): the row just written is normalised once more into d2, y2 = LN(y) * w2 — the norm in front of the next sublayer, which reads
 // the residual stream this kernel has just updated (a thread re-reads the elements it wrote itself)
+// Rows of up to 4096 values in whole, aligned pieces of four (k_layer_norm_held, R pieces a thread): the row, its weights, the residual row and the second stage's
+// weights are ALL requested before anything waits, so a row costs one round trip to memory and the barriers of its sums.  With the weights and the residual loaded behind
+// the sums, value by value under the bounds check, each of the sixteen values of a thread waited for its own two loads.  MI355X, us a launch, before / now: 2 rows of 2048
+// with both stages 12.2 / 4.2, 512 rows of 4096 13.8 / 7.2.  Any other row: k_layer_norm.
+template <int R>
+__global__ void __launch_bounds__(256) k_layer_norm_held(const tdesc a, const tdesc d, const float eps, const float * __restrict__ w, const tdesc r, const int has_r,
+                                                         const float * __restrict__ w2, const float eps2, const tdesc d2) {
+    __shared__ double sh[4][4];
+    const int64_t row = blockIdx.x;
+    const int64_t i1 = row % a.ne[1], i2 = (row / a.ne[1]) % a.ne[2], i3 = row / (a.ne[1] * a.ne[2]);
+    const float4 * const x = (const float4 *) (a.data + i1 * a.nb[1] + i2 * a.nb[2] + i3 * a.nb[3]);
+    const float4 * const rr = (const float4 *) (r.data + i1 * r.nb[1] + i2 * r.nb[2] + i3 * r.nb[3]);
+    const int n4 = (int) (a.ne[0] >> 2);
+    const double inv = (double) a.ne[0];
+    float4 xv[R], wv[R], rv[R], w2v[R];
+#pragma unroll
+    for (int u = 0; u < R; ++u) {  // (lanes beyond the row read its last piece and add nothing)
+        const int i = min((int) threadIdx.x + 256 * u, n4 - 1);
+        xv[u] = x[i];
+        wv[u] = w ? ((const float4 *) w)[i] : make_float4(1.f, 1.f, 1.f, 1.f);
+        rv[u] = has_r ? rr[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+        w2v[u] = w2 ? ((const float4 *) w2)[i] : make_float4(1.f, 1.f, 1.f, 1.f);
+    }
+    auto total = [&](const double part, double * const s4) {
+        const double v = wave_sum_d(part);
+        if ((threadIdx.x & 63) == 0) s4[threadIdx.x >> 6] = v;
+        __syncthreads();
+        return ((s4[0] + s4[1]) + s4[2]) + s4[3];
+    };
+    auto live = [&](const int u) { return (int) threadIdx.x + 256 * u < n4; };
+    auto norm = [&](const float e, const int stage, float & mean, float & scale) {
+        double s = 0.0, q = 0.0;
+#pragma unroll
+        for (int u = 0; u < R; ++u)
+            if (live(u)) s += ((double) xv[u].x + (double) xv[u].y) + ((double) xv[u].z + (double) xv[u].w);
+        mean = (float) (total(s, sh[2 * stage]) / inv);
+#pragma unroll
+        for (int u = 0; u < R; ++u) {
+            const float dx = xv[u].x - mean, dy = xv[u].y - mean, dz = xv[u].z - mean, dw = xv[u].w - mean;
+            if (live(u)) q += ((double) (dx * dx) + (double) (dy * dy)) + ((double) (dz * dz) + (double) (dw * dw));
+        }
+        scale = 1.0f / sqrtf((float) (total(q, sh[2 * stage + 1]) / inv) + e);
+    };
+    float mean, scale;
+    norm(eps, 0, mean, scale);
+    float4 * const y = (float4 *) (d.data + i1 * d.nb[1] + i2 * d.nb[2] + i3 * d.nb[3]);
+#pragma unroll
+    for (int u = 0; u < R; ++u) {
+        float4 v;
+        v.x = (xv[u].x - mean) * scale; v.y = (xv[u].y - mean) * scale; v.z = (xv[u].z - mean) * scale; v.w = (xv[u].w - mean) * scale;
+        if (w) { v.x *= wv[u].x; v.y *= wv[u].y; v.z *= wv[u].z; v.w *= wv[u].w; }
+        if (has_r) { v.x += rv[u].x; v.y += rv[u].y; v.z += rv[u].z; v.w += rv[u].w; }
+        if (live(u)) y[threadIdx.x + 256 * u] = v;
+        xv[u] = v;
+    }
+    if (w2 == nullptr) return;
+    norm(eps2, 1, mean, scale);
+    float4 * const y2 = (float4 *) (d2.data + i1 * d2.nb[1] + i2 * d2.nb[2] + i3 * d2.nb[3]);
+#pragma unroll
+    for (int u = 0; u < R; ++u) {
+        float4 v;
+        v.x = (xv[u].x - mean) * scale * w2v[u].x; v.y = (xv[u].y - mean) * scale * w2v[u].y; v.z = (xv[u].z - mean) * scale * w2v[u].z; v.w = (xv[u].w - mean) * scale * w2v[u].w;
+        if (live(u)) y2[threadIdx.x + 256 * u] = v;
+    }
+}
+// y = (x - mean) / sqrt(var + eps) per row for rows that are longer, odd or not aligned: the row is read again in every pass
 __global__ void __launch_bounds__(256) k_layer_norm(const tdesc a, const tdesc d, const float eps, const float * __restrict__ w, const tdesc r, const int has_r,
-                                                    const float * __restrict__ w2 = nullptr, const float eps2 = 0.0f, const tdesc d2 = tdesc()) {
+                                                    const float * __restrict__ w2, const float eps2, const tdesc d2) {
     __shared__ double sh[4];
     const int64_t row = blockIdx.x;
     const int64_t i1 = row % a.ne[1], i2 = (row / a.ne[1]) % a.ne[2], i3 = row / (a.ne[1] * a.ne[2]);
-    const float * __restrict__ x = (const float *) (a.data + i1 * a.nb[1] + i2 * a.nb[2] + i3 * a.nb[3]);
-    float * __restrict__ y = (float *) (d.data + i1 * d.nb[1] + i2 * d.nb[2] + i3 * d.nb[3]);
-    const float * __restrict__ rr = has_r ? (const float *) (r.data + i1 * r.nb[1] + i2 * r.nb[2] + i3 * r.nb[3]) : nullptr;
+    const float * x = (const float *) (a.data + i1 * a.nb[1] + i2 * a.nb[2] + i3 * a.nb[3]);
+    float * y = (float *) (d.data + i1 * d.nb[1] + i2 * d.nb[2] + i3 * d.nb[3]);
+    const float * rr = has_r ? (const float *) (r.data + i1 * r.nb[1] + i2 * r.nb[2] + i3 * r.nb[3]) : nullptr;
     const int64_t n = a.ne[0];
-    // rows of up to 4096 values are read ONCE and kept in registers (16 a thread); longer rows are re-read from L2 in every pass
-    constexpr int RC = 16;
-    const bool held = n <= 256 * RC;
-    float xv[RC];
     double s = 0.0;
-    if (held) {
-#pragma unroll
-        for (int u = 0; u < RC; ++u) {
-            const int64_t i = threadIdx.x + 256 * u;
-            xv[u] = i < n ? x[i] : 0.0f;
-            s += (double) xv[u];
-        }
-    } else {
-        for (int64_t i = threadIdx.x; i < n; i += blockDim.x) s += (double) x[i];
-    }
+    for (int64_t i = threadIdx.x; i < n; i += blockDim.x) s += (double) x[i];
     s = block_sum_d(s, sh);
     const float mean = (float) (s / (double) n);
     __syncthreads();
     double q = 0.0;
-    if (held) {
-#pragma unroll
-        for (int u = 0; u < RC; ++u) {
-            const float dv = xv[u] - mean;
-            if (threadIdx.x + 256 * u < n) q += (double) (dv * dv);
-        }
-    } else {
-        for (int64_t i = threadIdx.x; i < n; i += blockDim.x) {
-            const float dv = x[i] - mean;
-            q += (double) (dv * dv);
-        }
+    for (int64_t i = threadIdx.x; i < n; i += blockDim.x) {
+        const float dv = x[i] - mean;
+        q += (double) (dv * dv);
     }
     q = block_sum_d(q, sh);
     const float var = (float) (q / (double) n);
     const float scale = 1.0f / sqrtf(var + eps);
     double s2 = 0.0;
-    if (held) {
-#pragma unroll
-        for (int u = 0; u < RC; ++u) {
-            const int64_t i = threadIdx.x + 256 * u;
-            if (i < n) {
-                float v = (xv[u] - mean) * scale;
-                if (w) v *= w[i];
-                if (rr) v += rr[i];
-                y[i] = v;
-                xv[u] = v;
-                s2 += (double) v;
-            }
-        }
-    } else {
-        for (int64_t i = threadIdx.x; i < n; i += blockDim.x) {
-            float v = (x[i] - mean) * scale;
-            if (w) v *= w[i];
-            if (rr) v += rr[i];
-            y[i] = v;
-            s2 += (double) v;
-        }
+    for (int64_t i = threadIdx.x; i < n; i += blockDim.x) {
+        float v = (x[i] - mean) * scale;
+        if (w) v *= w[i];
+        if (rr) v += rr[i];
+        y[i] = v;
+        s2 += (double) v;
     }
     if (w2 == nullptr) return;
     __syncthreads();
@@ -213,40 +243,32 @@ __global__ void __launch_bounds__(256) k_layer_norm(const tdesc a, const tdesc d
     const float mean2 = (float) (s2 / (double) n);
     __syncthreads();
     double q2 = 0.0;
-    if (held) {
-#pragma unroll
-        for (int u = 0; u < RC; ++u) {
-            const float dv = xv[u] - mean2;
-            if (threadIdx.x + 256 * u < n) q2 += (double) (dv * dv);
-        }
-    } else {
-        for (int64_t i = threadIdx.x; i < n; i += blockDim.x) {
-            const float dv = y[i] - mean2;
-            q2 += (double) (dv * dv);
-        }
+    for (int64_t i = threadIdx.x; i < n; i += blockDim.x) {
+        const float dv = y[i] - mean2;
+        q2 += (double) (dv * dv);
     }
     q2 = block_sum_d(q2, sh);
     const float scale2 = 1.0f / sqrtf((float) (q2 / (double) n) + eps2);
-    float * __restrict__ y2 = (float *) (d2.data + i1 * d2.nb[1] + i2 * d2.nb[2] + i3 * d2.nb[3]);
-    if (held) {
-#pragma unroll
-        for (int u = 0; u < RC; ++u) {
-            const int64_t i = threadIdx.x + 256 * u;
-            if (i < n) y2[i] = (xv[u] - mean2) * scale2 * w2[i];
-        }
-    } else {
-        for (int64_t i = threadIdx.x; i < n; i += blockDim.x) y2[i] = (y[i] - mean2) * scale2 * w2[i];
-    }
+    float * y2 = (float *) (d2.data + i1 * d2.nb[1] + i2 * d2.nb[2] + i3 * d2.nb[3]);
+    for (int64_t i = threadIdx.x; i < n; i += blockDim.x) y2[i] = (y[i] - mean2) * scale2 * w2[i];
+}
+static void launch_layer_norm_rows(hipStream_t s, const tdesc & src, const tdesc & dst, const float eps, const float * mul_w, const tdesc * residual, const float * w2, const float eps2, const tdesc & dst2) {
+    const int64_t rows = src.ne[1] * src.ne[2] * src.ne[3], n = src.ne[0];
+    if (rows == 0) return;
+    const tdesc r = residual ? *residual : src;
+    auto al = [](const tdesc & t) { return (((uintptr_t) t.data | (uintptr_t) t.nb[1] | (uintptr_t) t.nb[2] | (uintptr_t) t.nb[3]) & 15) == 0; };
+    const bool held = n > 0 && n <= 4096 && (n & 3) == 0 && al(src) && al(dst) && al(r) && al(dst2) && (((uintptr_t) mul_w | (uintptr_t) w2) & 15) == 0;
+    const dim3 g((unsigned) rows), b(256);
+    if (!held) hipLaunchKernelGGL(k_layer_norm, g, b, 0, s, src, dst, eps, mul_w, r, residual ? 1 : 0, w2, eps2, dst2);
+    else if (n <= 1024) hipLaunchKernelGGL(k_layer_norm_held<1>, g, b, 0, s, src, dst, eps, mul_w, r, residual ? 1 : 0, w2, eps2, dst2);
+    else if (n <= 2048) hipLaunchKernelGGL(k_layer_norm_held<2>, g, b, 0, s, src, dst, eps, mul_w, r, residual ? 1 : 0, w2, eps2, dst2);
+    else hipLaunchKernelGGL(k_layer_norm_held<4>, g, b, 0, s, src, dst, eps, mul_w, r, residual ? 1 : 0, w2, eps2, dst2);
 }
 void launch_layer_norm(hipStream_t s, const tdesc & src, const tdesc & dst, float eps, const float * mul_w, const tdesc * residual) {
-    const int64_t rows = src.ne[1] * src.ne[2] * src.ne[3];
-    if (rows == 0) return;
-    hipLaunchKernelGGL(k_layer_norm, dim3((unsigned) rows), dim3(256), 0, s, src, dst, eps, mul_w, residual ? *residual : src, residual ? 1 : 0, (const float *) nullptr, 0.0f, src);
+    launch_layer_norm_rows(s, src, dst, eps, mul_w, residual, nullptr, 0.0f, dst);
 }
 void launch_layer_norm_twice(hipStream_t s, const tdesc & src, const tdesc & dst, float eps, const float * mul_w, const tdesc * residual, const float * w2, float eps2, const tdesc & dst2) {
-    const int64_t rows = src.ne[1] * src.ne[2] * src.ne[3];
-    if (rows == 0) return;
-    hipLaunchKernelGGL(k_layer_norm, dim3((unsigned) rows), dim3(256), 0, s, src, dst, eps, mul_w, residual ? *residual : src, residual ? 1 : 0, w2, eps2, dst2);
+    launch_layer_norm_rows(s, src, dst, eps, mul_w, residual, w2, eps2, dst2);
 }
 
 // ------------------------------------------------------------------------------------------------ router: top-k and soft-max over the chosen logits

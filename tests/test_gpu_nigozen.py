@@ -308,6 +308,25 @@ def test_layer_norm_with_weight_and_residual(backend, H):
         assert np.abs(got[1].reshape(rows, n) - R.layer_norm(x.astype(np.float64), 1.0, 1e-5)).max() <= 1e-5
 
 
+# rows at the edges of the pieces that a thread holds (1024, 2048, 4096 values), ones that are no whole pieces of four, and one that is longer than the held form takes
+@pytest.mark.parametrize("n", [4, 1020, 1024, 1028, 1027, 2048, 2052, 4092, 4096, 4097, 4100])
+def test_layer_norm_two_stages_at_the_edges_of_its_pieces(backend, H, n):
+    rng = np.random.default_rng(n)
+    rows = 3
+    x = (rng.standard_normal((rows, n)) * 3 + 1.5).astype(np.float32)
+    r = rng.standard_normal((rows, n)).astype(np.float32)
+    w, w2 = (rng.standard_normal(n).astype(np.float32) for _ in range(2))
+
+    def build(g):
+        s = H.ggml_add(g.ctx, H.ggml_mul(g.ctx, H.ggml_norm(g.ctx, g.new(L.F32, [n, rows], x), 1e-5), g.new(L.F32, [n], w)), g.new(L.F32, [n, rows], r))
+        return [H.ggml_mul(g.ctx, H.ggml_norm(g.ctx, s, 1e-6), g.new(L.F32, [n], w2))]
+
+    s = R.layer_norm(x.astype(np.float64), w.astype(np.float64), 1e-5) + r
+    got = run(backend, build)[0].reshape(rows, n)
+    # the first stage rounds values of up to ~15 to f32 (1e-6 each), the second divides by a deviation near 1
+    assert np.abs(got - R.layer_norm(s, w2.astype(np.float64), 1e-6)).max() <= 2e-5
+
+
 def test_rotary_on_the_leading_pairs(backend, H):
     rng = np.random.default_rng(6)
     x = rng.standard_normal((9, 3, 20)).astype(np.float32)
