@@ -4,10 +4,11 @@
 // are exact in f32 and accumulated in f32.  One accumulator per output walks K in steps of 16, in order, whatever the tile: the result does not depend on the tile
 // chosen, on the matrices that share the launch or on the other columns.
 //
-// A workgroup of four waves owns TM src1 columns x TN src0 rows and advances K by 64.  Both operands arrive by LDS-DMA (global_load_lds_dwordx4, 1 KB = 8 rows of
-// 128 bytes per wave-instruction) into a ring of S stages, S - 1 of them in flight: with one stage ahead in registers a step of 128 x 128 took 1.7 us, the latency of
-// its loads, against 0.2 us of matrix work.  src1 is rounded to 16 bits once per tensor (k_to_16: the q / k / v / gate projections read the same copy), which halves
-// its share of the 64 bytes per clock a CU can fetch — what bounds a 64 x 128 tile.  LDS rows hold the 16-byte chunk index XORed by (row >> 1) & 7 (the lanes
+// A workgroup of four waves owns TM src1 columns x TN src0 rows, a quarter of them each, and advances K by 64.  Both operands arrive by LDS-DMA (global_load_lds_dwordx4, 1 KB = 8 rows of
+// 128 bytes per wave-instruction) into a ring of S stages, up to S - 1 of them in flight: with one stage ahead in registers a step of 128 x 128 took 1.7 us, the latency of
+// its loads, against 0.2 us of matrix work.  The operands of the next 16 values of K leave LDS under the products of these, across the steps too: a step's one barrier lies ahead of its
+// last products (128 x 128, K 4096, 6144 rows, 512 columns: 43 us, 70 with the first reads of a step behind its barrier).  src1 is rounded to 16 bits once per tensor (k_to_16: the q / k / v / gate projections read the same copy), which halves
+// its share of what a CU fetches.  LDS rows hold the 16-byte chunk index XORed by (row >> 1) & 7 (the lanes
 // of the DMA fetch the permuted chunks): the 16 lanes a ds_read_b128 serves at once hit 16 distinct slots.  One barrier per step.  Workgroups that read the same src0
 // rows follow one another on one XCD.
 #include <algorithm>
@@ -72,10 +73,11 @@ struct mt_args {
 
 template <bool BF, int TM, int TN, int S, bool ID> __global__ void __launch_bounds__(256, 1) k_mul_mat_tile(const mt_args a) {
     constexpr int MT = TM / 64, NT = TN / 64;
-    constexpr int STAGE = (TM + TN) * 128, L = (TM + TN) / 32;  // bytes of a stage, DMA instructions per wave and stage
+    constexpr int STAGE = (TM + TN) * 128, L = (TM + TN) / 32, Q = L / 4;  // bytes of a stage, DMA instructions per wave and stage, of which the first quarter
+    static_assert(S >= 3 && (S - 1) * L <= 63, "ring");
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int fr = lane & 31, g = lane >> 5, wm = wave & 1, wn = wave >> 1;
+    const int fr = lane & 31, g = lane >> 5;
     int tile, mt0, e = 0;
     int64_t M = a.M;
     if constexpr (ID) {
@@ -95,7 +97,8 @@ template <bool BF, int TM, int TN, int S, bool ID> __global__ void __launch_boun
     const int64_t n0 = (int64_t) (tile - (mi ? a.m[mi - 1].tile_end : 0)) * TN, N = mat.N, K = a.K;
     const int32_t * cols = ID ? a.list + a.off[e] : nullptr;
     const char * const wbase = mat.W + n0 * mat.nb1 + (ID ? e * a.w_nb2 : 0);
-    const int swz = (fr >> 1) & 7, steps = (int) (K / 64);
+    const int steps = (int) (K / 64);
+    const int swz = (fr >> 1) & 7, wm = wave & 1, wn = wave >> 1;
     const char * const fx = smem + (wm * (TM / 2) + fr) * 128, * const fw = smem + (TM + wn * (TN / 2) + fr) * 128;
     const uint32_t lds0 = (uint32_t) (uintptr_t) smem;
 
@@ -129,10 +132,8 @@ template <bool BF, int TM, int TN, int S, bool ID> __global__ void __launch_boun
                 off[j] = (uint32_t) (std::min<int64_t>(row - TM, N - 1 - n0) * mat.nb1 + chunk * 16);
             }
         }
-        auto issue = [&](const int s, const int j0, const int j1) {
-            const uint32_t to = lds0 + (uint32_t) (s % S) * STAGE + (uint32_t) wave * L * 1024;
-#pragma unroll
-            for (int j = j0; j < j1; ++j) mt_dma16(base[j] + (int64_t) s * 128, off[j], to + j * 1024);
+        auto issue = [&](const int s, const int j) __attribute__((always_inline)) {
+            mt_dma16(base[j] + (int64_t) s * 128, off[j], lds0 + (uint32_t) (s % S) * STAGE + (uint32_t) (wave * L + j) * 1024);
         };
         mt_float16 acc[MT][NT];
 #pragma unroll
@@ -141,35 +142,63 @@ template <bool BF, int TM, int TN, int S, bool ID> __global__ void __launch_boun
             for (int u = 0; u < NT; ++u) acc[t][u] = (mt_float16){0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
         if (ID && mt != mt0) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");  // (the ring is free, no store is counted in vmcnt)
 #pragma unroll
-        for (int s = 0; s < S - 1; ++s)
-            if (s < steps) issue(s, 0, L);
-        for (int s = 0; s < steps; ++s) {
-            // this wave's pieces of step s have landed (in-order vmcnt: only the S - 2 steps behind it may still fly), then everybody's have, and nobody reads step
-            // s - 1 any more: its stage is the one requested next
-            if (s + S - 2 < steps) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((S - 2) * L) : "memory");
-            else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-            const int bo = (s % S) * STAGE;
-            uint4 xa[2][MT], wb[2][NT];
-            auto frags = [&](const int ks) {
-                const int co = ((2 * ks + g) ^ swz) << 4;
+        for (int s = 0; s < S; ++s)
+            if (s < steps)
 #pragma unroll
-                for (int t = 0; t < MT; ++t) xa[ks & 1][t] = *(const uint4 *) (fx + bo + t * 32 * 128 + co);
+                for (int j = 0; j < (s < S - 1 ? L : Q); ++j) issue(s, j);
+        if (steps >= S) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((S - 2) * L + Q) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+        uint4 xa[2][MT], wb[2][NT];
+        auto frags = [&](const int s, const int ks, const int set) __attribute__((always_inline)) {
+            const int bo = (s % S) * STAGE + (((2 * ks + g) ^ swz) << 4);
 #pragma unroll
-                for (int u = 0; u < NT; ++u) wb[ks & 1][u] = *(const uint4 *) (fw + bo + u * 32 * 128 + co);
-            };
-            frags(0);
+            for (int t = 0; t < MT; ++t) xa[set][t] = *(const uint4 *) (fx + bo + t * 4096);
+#pragma unroll
+            for (int u = 0; u < NT; ++u) wb[set][u] = *(const uint4 *) (fw + bo + u * 4096);
+        };
+        frags(0, 0, 0);
+        auto products = [&](const int set, const int req, const int j0, const int j1) __attribute__((always_inline)) {  // ... and the requests j0 .. j1 - 1 of step req on the way
+#pragma unroll
+            for (int t = 0; t < MT; ++t)
+#pragma unroll
+                for (int u = 0; u < NT; ++u) {
+                    if constexpr (BF) acc[t][u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(mt_bf8, xa[set][t]), __builtin_bit_cast(mt_bf8, wb[set][u]), acc[t][u], 0, 0, 0);
+                    else acc[t][u] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(mt_half8, xa[set][t]), __builtin_bit_cast(mt_half8, wb[set][u]), acc[t][u], 0, 0, 0);
+                    const int i = t * NT + u;  // (spread over the products: the CU's one address pipeline takes 16 clocks for each)
+#pragma unroll
+                    for (int j = j0 + (j1 - j0) * i / (MT * NT); j < j0 + (j1 - j0) * (i + 1) / (MT * NT); ++j) {
+                        issue(req, j);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+        };
+        int s = 0;
+        for (; s + S < steps; ++s) {
 #pragma unroll
             for (int ks = 0; ks < 4; ++ks) {
-                if (ks < 3) frags(ks + 1);
-                if (s + S - 1 < steps) issue(s + S - 1, ks * L / 4, (ks + 1) * L / 4);  // (a quarter at a time: the CU's one address pipeline takes 16 clocks for each)
-#pragma unroll
-                for (int t = 0; t < MT; ++t)
-#pragma unroll
-                    for (int u = 0; u < NT; ++u) {
-                        if constexpr (BF) acc[t][u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(mt_bf8, xa[ks & 1][t]), __builtin_bit_cast(mt_bf8, wb[ks & 1][u]), acc[t][u], 0, 0, 0);
-                        else acc[t][u] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(mt_half8, xa[ks & 1][t]), __builtin_bit_cast(mt_half8, wb[ks & 1][u]), acc[t][u], 0, 0, 0);
-                    }
+                if (ks == 3) {
+                    // this wave has the rest of step s in registers and its pieces of step s + 1 have landed (in-order vmcnt: only the S - 2 steps behind it may still fly);
+                    // then so has everybody: the stage of step s is the one requested next
+                    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((S - 2) * L) : "memory");
+                    frags(s + 1, 0, 0);
+                } else frags(s, ks + 1, (ks + 1) & 1);
+                __builtin_amdgcn_sched_barrier(0);  // (the reads of the next products travel under these)
+                if (ks == 3) products(1, s + S, 0, Q);
+                else products(ks & 1, s + S - 1, Q + (L - Q) * ks / 3, Q + (L - Q) * (ks + 1) / 3);
             }
+        }
+        if (steps >= S)
+#pragma unroll
+            for (int j = Q; j < L; ++j) issue(steps - 1, j);
+        while (true) {  // the rest has been requested
+#pragma unroll
+            for (int ks = 0; ks < 4; ++ks) {
+                if (ks < 3) frags(s, ks + 1, (ks + 1) & 1);
+                products(ks & 1, 0, 0, 0);
+            }
+            if (++s >= steps) break;
+            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            frags(s, 0, 0);
         }
         // lane: src0 row; register i: src1 column (i & 3) + 8 (i >> 2) + 4 g — 32 lanes store a whole 128-byte line
 #pragma unroll
@@ -195,19 +224,30 @@ template <bool BF, int TM, int TN, int S, bool ID> __global__ void __launch_boun
     }
 }
 
-// The tile and its ring.  Measured (us; bf16, 512 columns unless stated; 128 x 128 with two stages and two workgroups per CU / 64 x 128 with five / 64 x 64 with four; before: one wave
-// per 32 x 32 tile, operands straight from global memory): K 4096 N 14336: 90 / 136 / 125 (623), N 10240: 86 / 102 / 92 (453), N 4096: 57 / 36 / 33 (184); K 14336 N 4096: 224 / 113 /
-// 128 (645); 128 columns, N 14336: 76 / 44 / 46 (313), N 4096: 55 / 32 / 23 (94); 64 columns, N 14336: 74 / 43 / 34 (163), N 4096: 54 / 32 / 22 (51).
+// The tile and its ring: the form whose rounds over the 256 CUs take least.  A round of a form costs the same whatever the shape, in proportion to K (us for K = 4096, weights from
+// memory): 256 x 128 in three stages 66, 128 x 128 in four 43, 128 x 64 in five 33, 64 x 64 in four 23 with one workgroup per CU and 38 with two.  Measured (us; bf16, 512 columns unless
+// stated; 256 x 128 / 128 x 128 / 128 x 64 / 64 x 64; before, where a step's first operands were read behind its barrier: 128 x 128 in two stages, 64 x 128 in five or 64 x 64):
+// K 4096 N 14336: 70 / 87 / 117 / 116 (84), N 28672: 139 / 173 / 208 / 227 (161), N 10240: 66 / 85 / 88 / 85 (78), N 6144: 63 / 43 / 59 / 53 (63), N 4096: 62 / 42 / 33 / 38 (34);
+// K 14336 N 4096: 192 / 130 / 96 / 119 (107); K 8192 N 2048: 107 / 71 / 51 / 39 (56); K 2048 N 8192: 40 / 28 / 39 / 39 (39), N 2048: 33 / 19 / 14 / 11 (17); 256 columns, K 4096 N 14336:
+// 69 / 50 / 63 / 69 (65); 128 columns, N 14336: 60 / 49 / 38 / 42 (39), N 4096: 56 / 42 / 31 / 23 (23).  What bounds a round: from memory a CU fetches at most 50 KB per us however deep
+// the ring (142 from L2), so a tile's share of src0 is 0.3 us a step whatever its columns.
 static void mt_pick(const mul_mat_tile_desc * m, int n, int64_t M, int * tm, int * tn) {
     auto count = [&](int64_t TM, int64_t TN) {
         int64_t t = 0;
         for (int q = 0; q < n; ++q) t += (m[q].N + TN - 1) / TN;
         return t * ((M + TM - 1) / TM);
     };
+    auto rounds = [](int64_t c, int64_t at_once) { return (c + at_once - 1) / at_once; };
+    const int64_t small = count(64, 64);
+    int64_t best = small <= 256 ? 23 : 38 * rounds(small, 512);
     *tm = 64;
     *tn = 64;
-    if (M > 64 && count(128, 128) >= 288) { *tm = 128; *tn = 128; }     // more than one workgroup per CU: the fewest bytes per product
-    else if (M > 64 && count(64, 128) >= 192) *tn = 128;                // most CUs have one
+    if (M <= 64) return;  // (wider tiles would be half empty)
+    const struct { int tm, tn, cost; } forms[3] = {{128, 64, 33}, {128, 128, 43}, {256, 128, 66}};
+    for (const auto & f : forms) {
+        const int64_t cost = f.cost * rounds(count(f.tm, f.tn), 256);
+        if (cost < best) { best = cost; *tm = f.tm; *tn = f.tn; }
+    }
 }
 template <bool BF, int TM, int TN, int S, bool ID> static void mt_launch_t(hipStream_t s, const dim3 grid, const mt_args & a) {
     const size_t lds = (size_t) S * (TM + TN) * 128;
@@ -268,8 +308,9 @@ void launch_mul_mat_tile(hipStream_t s, int type, const mul_mat_tile_desc * m, i
     const dim3 grid((unsigned) ((a.n_tiles + 7) / 8 * 8 * a.m_tiles));
     const bool bf = type == GGML_TYPE_BF16;
 #define MT(TM_, TN_, S_) { if (bf) mt_launch_t<true, TM_, TN_, S_, false>(s, grid, a); else mt_launch_t<false, TM_, TN_, S_, false>(s, grid, a); }
-    if (tm == 128) MT(128, 128, 2)
-    else if (tn == 128) MT(64, 128, 5)
+    if (tm == 256) MT(256, 128, 3)
+    else if (tn == 128) MT(128, 128, 4)
+    else if (tm == 128) MT(128, 64, 5)
     else MT(64, 64, 4)
 #undef MT
 }

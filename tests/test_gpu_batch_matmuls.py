@@ -67,6 +67,19 @@ def test_16_bit_matrices_with_batches(backend, H, wt, K, N, M):
     assert np.abs(got - ref).max() <= 6e-8 * np.sqrt(K) * 8
 
 
+# every tile of mmf_tile.hip (256 x 128, 128 x 128, 128 x 64, 64 x 64 columns x rows) with fewer steps of K than its ring has stages, as many, one and two more, and remainders on both sides
+@pytest.mark.parametrize("N,M,stages", [(14401, 500, 3), (9000, 190, 4), (4100, 330, 5), (130, 70, 4)])
+@pytest.mark.parametrize("more", [-1, 0, 1, 2])
+def test_16_bit_tiles_and_their_rings(backend, H, N, M, stages, more):
+    rng = np.random.default_rng(N + M + more)
+    K = 64 * (stages + more)
+    w = round16((rng.standard_normal((N, K)) / np.sqrt(K)).astype(np.float32), L.BF16)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    got = T.run_case(lambda g: H.ggml_mul_mat(g.ctx, g.new(L.BF16, [K, N], bits16(w, L.BF16)), g.new(L.F32, [K, M], x)), backend)[0].reshape(M, N)
+    ref = round16(x, L.BF16).astype(np.float64) @ w.astype(np.float64).T
+    assert np.abs(got - ref).max() <= 6e-8 * np.sqrt(K) * 8  # (as above)
+
+
 @pytest.mark.parametrize("M", [2, 16, 17, 150])
 def test_16_bit_siblings_have_the_bits_of_single_launches(backend, H, M):
     """three bf16 matrices over one input: one launch (and one rounding of the input), the results of three"""
