@@ -377,15 +377,19 @@ __global__ void __launch_bounds__(256) k_attn_f32_tile(const tdesc q, const tdes
 }
 
 // ------------------------------------------------------------------------------------------------ prompt batches over a bf16 cache: the matrix cores
-// k_attn_mma_bf16: a wave owns 32 query tokens of one head; a workgroup is 1, 2 or 4 such waves sharing the staged V^T block.  Per block of 32 cells
-//   S^T = K . Q^T   on v_mfma_f32_32x32x16_bf16 (first operand: the cells' bf16 rows straight from the cache, 16 bytes a lane; second: the wave's queries,
-//                   rounded to bf16 once and kept in registers) — a lane then holds 16 scores of ITS query (its half-wave's cells), so the running maximum,
-//                   the sum and the rescaling are per-lane scalars and one exchange with the other half-wave;
+// k_attn_mma_bf16: a workgroup of four waves owns 32 query tokens of one head; wave w takes every fourth block of 32 cells (w, w + 4, ..), alone, and the four meet at the end.  Per block
+//   S^T = K . Q^T   on v_mfma_f32_32x32x16_bf16 (first operand: the cells' bf16 rows; second: the queries, rounded to bf16 once and kept in registers) — a lane
+//                   then holds 16 scores of ITS query (its half-wave's cells), so the running maximum, the sum and the rescaling are per-lane scalars and one
+//                   exchange with the other half-wave;
 //   scores, maxima, exponentials and sums are f32;
-//   O^T += V^T . P^T  on the same instruction, V^T staged through LDS (bf16, transposed on the way in), the weights P given as TWO bf16 terms
-//                   (p = hi + lo, |lo| <= 2^-9 |p|): the f32 weights enter the sum to 2^-17, not rounded to 8 bits.
+//   O^T += V^T . P^T  on the same instruction, the weights P given as TWO bf16 terms (p = hi + lo, |lo| <= 2^-9 |p|): the f32 weights enter the sum to 2^-17, not rounded to 8 bits.
 // The key order inside the second product is the order the first product's registers come in (both operands permuted alike).
-// Blocks that the mask hides from all of a workgroup's queries are skipped after the mask read.  Head sizes: multiples of 8 up to 16 DK16 / 32 DVT.
+// K and V rows reach the wave's own LDS by LDS-DMA as they lie (a lane-per-row load of K touches 32 lines an instruction), V is transposed by ds_read_b64_tr_b16 on the way out; a wave needs
+// no barrier: the next block's K is requested when this one's has left LDS, its V when the second product has read this one's.  First the mask of the 32 queries is scanned, row by row, for
+// the blocks that any of them sees, and for those where its terms are not all zero: only these read it again.  Head sizes: multiples of 8 up to 16 DK16 / 32 DVT.
+// What bounds it: the vector ALU, about 350 instructions a block beside 24 matrix ones, with two waves a SIMD.  512 queries x 32 heads of 128 on 8 key heads, the last of n cells (us; before:
+// 32 queries a wave, all cells, V^T staged by the workgroup): n = 512 20.9 (44.5), 1024 33.5 (79.7), 2048 60 (150), 8192 210 (545); 16 heads on 4, n = 2048 52 (143); 2048 queries x 64 heads
+// 319 (525); 64 queries x 16 heads, n = 512 17 (41).
 typedef __bf16 att_bf8 __attribute__((ext_vector_type(8)));
 typedef float att_f16v __attribute__((ext_vector_type(16)));
 __device__ __forceinline__ uint32_t att_bf16_bits(const float f) {
@@ -397,26 +401,47 @@ typedef float att_f2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint32_t att_bf16_pack(const float a, const float b) {  // two values to bf16, nearest even, in one instruction
     return __builtin_bit_cast(uint32_t, __builtin_convertvector((att_f2){a, b}, att_bf2));
 }
-// NV: value shares of 8 entries x 4 cells per thread and block (8 x DVT x 4 of them over the workgroup's threads).  PLAIN: scores are q.k x scale + mask (no sigmoid, cap or distance
-// penalty), head sizes exactly 16 DK16 / 32 DVT.
-// First the mask is scanned for the blocks of 32 cells that anybody in the workgroup sees (a bit each), then the visible ones are walked: the next one's K operands, V entries
-// and mask terms travel while the current one is multiplied, V^T alternates between two LDS copies, one barrier per block.  A 2000-token prompt in portions of 512, 32 heads of 128
-// on 8 key heads, per launch: 217 us with the mask, the K and V of a block read one after the other and the variants' branches inside, 97 us as it is.
-constexpr int ATT_SCAN_BITS = 16384;  // blocks beyond these are taken as visible (a wave that sees nothing of a block still skips it)
-template <int DK16, int DVT, int NV, bool PLAIN>
+// e^t for t <= 88: 2^(t log2 e) with the rounding error of the product put back (v_exp_f32's own last place remains, as in expf); 0 from -150 down, NaN stays NaN
+__device__ __forceinline__ float att_exp(float t) {
+    constexpr float L2E = 1.44269504f, L2E_LO = 1.92596299e-8f, LN2 = 0.693147181f;
+    t = t < -150.0f ? -150.0f : t;
+    const float a = t * L2E, p = __builtin_amdgcn_exp2f(a);
+    return fmaf(p, fmaf(t, L2E_LO, fmaf(t, L2E, -a)) * LN2, p);
+}
+// lane i's 16 bytes at base + off land at LDS[lds + 16 i]; base and lds are wave-uniform
+__device__ __forceinline__ void att_dma16(const char * base, const uint32_t off, const uint32_t lds) {
+    uint32_t keep;
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0" : "=&s"(keep) : "v"(off), "s"(base), "s"(lds) : "memory");
+}
+typedef short att_s4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ att_s4 att_read_tr(const uint16_t * at) {  // 16 lanes read 4 rows of 16 values (4 lanes a row, 4 values each), lane i of them receives column i
+    return __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) att_s4 *) (__attribute__((address_space(3))) void *) at);
+}
+// PLAIN: scores are q.k x scale + mask (no sigmoid, cap or distance penalty), head sizes exactly 16 DK16 / 32 DVT.
+constexpr int ATT_SCAN_BITS = 16384;  // blocks beyond these are taken as visible, with a bias
+template <int DK16, int DVT, bool PLAIN>
 __global__ void __launch_bounds__(256, 2) k_attn_mma_bf16(const tdesc q, const tdesc k, const tdesc v, const tdesc mask, const float * __restrict__ sinks, const float * __restrict__ r12, const tdesc dst,
                                                        const float scale, const float * __restrict__ sig, const float softcap, const int pen_kind) {
-    constexpr int VS = 36;  // V^T row stride in LDS (bf16 elements): 72 bytes keeps the 8-byte reads aligned and spreads the rows over the banks
-    __shared__ __attribute__((aligned(16))) uint16_t Vt2[2][DVT * 32 * VS];
-    __shared__ uint32_t bits[ATT_SCAN_BITS / 32];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    constexpr int W = 4;  // waves
+    // 16-byte pieces of a cell's K and V rows in LDS, a piece's index XORed by the cell's: the 16 K rows read at once, and the 4 x 64 bytes of V, hit all banks once
+    constexpr int CP = DK16 <= 2 ? 4 : DK16 <= 4 ? 8 : 16, CV = DVT <= 1 ? 4 : DVT <= 2 ? 8 : 16;
+    constexpr int KT = 32 * CP * 8, VB = 32 * CV * 8;  // elements of a block's K, V
+    __shared__ __attribute__((aligned(16))) uint16_t pool[W * std::max(KT + VB, DVT * 32 * 64)];  // K and V of a wave, in the end its 32 x 32 DVT sums as f32
+    __shared__ uint32_t bits[ATT_SCAN_BITS / 32], mixed[ATT_SCAN_BITS / 32];  // block seen by any query; by some only, or with a bias
+    __shared__ float meet[W][2][32];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int) threadIdx.x >> 6);
     const int n = lane & 31, g = lane >> 5;
-    const int64_t h = blockIdx.y, n_q = q.ne[1], n_kv = k.ne[1];
+    int h = blockIdx.y, qt = blockIdx.x;
+    if (gridDim.y % 8 == 0) {  // an XCD has neighbouring heads, so that their K and V stay in its L2; the late query tiles first, then the early ones upward: a CU's two see equally much
+        const int id = blockIdx.x + gridDim.x * blockIdx.y, hx = gridDim.y / 8, t = (id >> 3) / hx, half = (gridDim.x + 1) / 2;
+        h = (id & 7) * hx + (id >> 3) % hx;
+        qt = t < half ? (int) gridDim.x - 1 - t : t - half;
+    }
+    const int64_t n_q = q.ne[1], n_kv = k.ne[1];
     const int DK = PLAIN ? 16 * DK16 : (int) q.ne[0], DV = PLAIN ? 32 * DVT : (int) v.ne[0];
-    const int64_t tq = (int64_t) blockIdx.x * (blockDim.x / 2) + wave * 32 + n;  // this lane's query (a workgroup of 1, 2 or 4 waves: 32 queries a wave)
+    const int64_t tq = (int64_t) qt * 32 + n;  // this lane's query
     const bool q_live = tq < n_q;
-    const int64_t kvh = h / (q.ne[2] / k.ne[2]);
-    const char * kbase = k.data + kvh * k.nb[2] + g * 16;
+    const int kvh = h / ((int) q.ne[2] / (int) k.ne[2]);
     const char * vbase = v.data + kvh * v.nb[2];
     const char * mrow = mask.data + (q_live ? tq : n_q - 1) * mask.nb[1];
     const int n_blk = (int) ((n_kv + 31) / 32), n_scan = min(n_blk, ATT_SCAN_BITS);
@@ -437,149 +462,189 @@ __global__ void __launch_bounds__(256, 2) k_attn_mma_bf16(const tdesc q, const t
             }
         }
     };
-    auto seen = [&](const float (&mv)[16]) {
-        float t = mv[0];
-#pragma unroll
-        for (int i = 1; i < 16; ++i) t = fmaxf(t, mv[i]);
-        return __ballot(q_live && t > -INFINITY) != 0;
-    };
-    for (int i = threadIdx.x; i < (n_scan + 31) / 32; i += blockDim.x) bits[i] = 0;
-    // the wave's queries as second operands: element group (16 s + 8 g .. + 7) of query n
+    for (int i = threadIdx.x; i < (n_scan + 31) / 32; i += blockDim.x) {
+        bits[i] = 0;
+        mixed[i] = 0;
+    }
+    // the queries as second operands: element group (16 s + 8 g .. + 7) of query n
     uint4 qf[DK16];
     {
         const float * qrow = (const float *) (q.data + (q_live ? tq : 0) * q.nb[1] + h * q.nb[2]);
+        const bool quads = PLAIN && (((uintptr_t) q.data | (uintptr_t) q.nb[1] | (uintptr_t) q.nb[2]) & 15) == 0;  // (uniform)
 #pragma unroll
         for (int s = 0; s < DK16; ++s) {
             const int i0 = 16 * s + 8 * g;
             uint32_t b[4];
+            if (quads) {
+                float4 x = *(const float4 *) (qrow + i0), y = *(const float4 *) (qrow + i0 + 4);
+                if (!q_live) x = y = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                b[0] = att_bf16_pack(x.x, x.y); b[1] = att_bf16_pack(x.z, x.w); b[2] = att_bf16_pack(y.x, y.y); b[3] = att_bf16_pack(y.z, y.w);
+            } else {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const float x = (q_live && i0 + 2 * e < DK) ? qrow[i0 + 2 * e] : 0.0f, y = (q_live && i0 + 2 * e + 1 < DK) ? qrow[i0 + 2 * e + 1] : 0.0f;
-                b[e] = att_bf16_pack(x, y);
+                for (int e = 0; e < 4; ++e) {
+                    const float x = (q_live && i0 + 2 * e < DK) ? qrow[i0 + 2 * e] : 0.0f, y = (q_live && i0 + 2 * e + 1 < DK) ? qrow[i0 + 2 * e + 1] : 0.0f;
+                    b[e] = att_bf16_pack(x, y);
+                }
             }
             qf[s] = make_uint4(b[0], b[1], b[2], b[3]);
         }
     }
     __syncthreads();
-    for (int blk = 0; blk < n_scan; blk += 4) {  // (four blocks' loads in flight; past the end the last block again)
-        float t0[16], t1[16], t2[16], t3[16];
-        load_mask(blk, t0);
-        load_mask(min(blk + 1, n_blk - 1), t1);
-        load_mask(min(blk + 2, n_blk - 1), t2);
-        load_mask(min(blk + 3, n_blk - 1), t3);
-        const uint32_t w = (seen(t0) ? 1u : 0u) | (seen(t1) ? 2u : 0u) | (seen(t2) ? 4u : 0u) | (seen(t3) ? 8u : 0u);
-        if (lane == 0 && w) atomicOr(&bits[blk >> 5], w << (blk & 31));
+    {  // a wave reads eight of the 32 rows, 256 cells at a time
+        const char * const m0 = mask.data + (int64_t) qt * 32 * mask.nb[1];
+        const int rows = (int) std::min<int64_t>(32, n_q - (int64_t) qt * 32) - 1;
+        for (int c = 0; c < n_scan; c += 8) {
+            const int64_t j = (int64_t) c * 32 + 4 * lane;
+            float4 t[8];
+#pragma unroll
+            for (int r = 0; r < 8; ++r) {
+                const float * p = (const float *) (m0 + (int64_t) std::min(8 * wave + r, rows) * mask.nb[1]);
+                if (j + 4 <= n_kv) t[r] = *(const float4 *) (p + j);
+                else t[r] = make_float4(j < n_kv ? p[j] : -INFINITY, j + 1 < n_kv ? p[j + 1] : -INFINITY, j + 2 < n_kv ? p[j + 2] : -INFINITY, -INFINITY);
+            }
+            bool any = false, odd = false;
+#pragma unroll
+            for (int r = 0; r < 8; ++r) {
+                any |= t[r].x > -INFINITY || t[r].y > -INFINITY || t[r].z > -INFINITY || t[r].w > -INFINITY;
+                odd |= t[r].x != 0.0f || t[r].y != 0.0f || t[r].z != 0.0f || t[r].w != 0.0f;
+            }
+            uint64_t va = __ballot(any), vo = __ballot(odd);  // eight lanes a block
+            uint32_t wa = 0, wo = 0;
+#pragma unroll
+            for (int b = 0; b < 8; ++b) {
+                wa |= ((va >> (8 * b)) & 0xFF) ? 1u << b : 0u;
+                wo |= ((vo >> (8 * b)) & 0xFF) ? 1u << b : 0u;
+            }
+            if (lane == 0) {
+                const uint32_t in = n_scan - c >= 8 ? 0xFFu : (1u << (n_scan - c)) - 1u;
+                if (wa & in) atomicOr(&bits[c >> 5], (wa & in) << (c & 31));
+                if (wo & in) atomicOr(&mixed[c >> 5], (wo & in) << (c & 31));
+            }
+        }
     }
     __syncthreads();
-    auto next_block = [&](int blk) {  // the first visible block from blk on (n_blk: none); uniform
+    auto next_block = [&](int blk) {  // this wave's first visible block from blk on (n_blk: none); uniform
         while (blk < n_scan) {
-            const uint32_t w = (uint32_t) __builtin_amdgcn_readfirstlane((int) bits[blk >> 5]) >> (blk & 31);
+            const uint32_t w = (uint32_t) __builtin_amdgcn_readfirstlane((int) (bits[blk >> 5] & (0x11111111u << wave))) >> (blk & 31);
             if (w) { blk += __builtin_ctz(w); break; }
             blk = (blk | 31) + 1;
         }
-        return blk < n_blk ? (blk < n_scan || n_scan < n_blk ? blk : n_blk) : n_blk;
+        if (blk >= n_scan) blk += (wave - blk) & (W - 1);
+        return min(blk, n_blk);
     };
     const int pen = PLAIN ? 0 : (r12 ? pen_kind : 0);
     const float r1 = pen ? r12[h] : 0.0f, r2 = pen == ATTN_PEN_LOG ? r12[q.ne[2] + h] : 0.0f;
     const bool sgm = PLAIN ? false : sig != nullptr;
     const float s_temp = sgm ? sig[h] : 1.0f, s_bias = sgm ? sig[q.ne[2] + h] : 0.0f;
-    float m = sgm ? 0.0f : (sinks ? sinks[h] : ATTN_F32_LOW), l = (sinks && !sgm) ? 1.0f : 0.0f;
+    float m = sgm ? 0.0f : (sinks && wave == 0 ? sinks[h] : ATTN_F32_LOW), l = (sinks && wave == 0 && !sgm) ? 1.0f : 0.0f;
     att_f16v O[DVT];
 #pragma unroll
     for (int dt = 0; dt < DVT; ++dt)
 #pragma unroll
         for (int i = 0; i < 16; ++i) O[dt][i] = 0.0f;
-    uint4 kn[DK16], vn[NV][4];
-    float mv_next[16];
-    auto fetch = [&](const int blk) {  // a block's K operands, this thread's share of its V (8 consecutive entries of FOUR neighbouring cells), its mask terms
-        const int64_t j0 = (int64_t) blk * 32;
-        const char * krow = kbase + std::min<int64_t>(j0 + n, n_kv - 1) * k.nb[1];
-#pragma unroll
-        for (int s = 0; s < DK16; ++s) {
-            if constexpr (PLAIN) kn[s] = *(const uint4 *) (krow + s * 32);
-            else {
-                kn[s] = make_uint4(0, 0, 0, 0);
-                if (16 * s + 8 * g < DK) kn[s] = *(const uint4 *) (krow + s * 32);
-            }
-        }
-#pragma unroll
-        for (int r = 0; r < NV; ++r) {
-            const int e0 = min((int) threadIdx.x + r * (int) blockDim.x, 32 * DVT - 1), cg = e0 / (DVT * 4), c8 = e0 % (DVT * 4);
-#pragma unroll
-            for (int cc = 0; cc < 4; ++cc) {
-                const int64_t j = j0 + 4 * cg + cc;
-                if constexpr (PLAIN) vn[r][cc] = *(const uint4 *) (vbase + std::min<int64_t>(j, n_kv - 1) * v.nb[1] + c8 * 16);
-                else {
-                    vn[r][cc] = make_uint4(0, 0, 0, 0);
-                    if (8 * c8 < DV) vn[r][cc] = *(const uint4 *) (vbase + std::min<int64_t>(j, n_kv - 1) * v.nb[1] + c8 * 16);
-                }
-            }
-        }
-        load_mask(blk, mv_next);
-        __builtin_amdgcn_sched_barrier(0);
+    float mv[16];
+    bool bias = true;  // the fetched block's mask terms are not all zero
+    auto fetch_mask = [&](const int blk) {
+        bias = blk >= n_scan || (__builtin_amdgcn_readfirstlane((int) mixed[blk >> 5]) >> (blk & 31) & 1) != 0;
+        if (bias) load_mask(blk, mv);
     };
-    int blk = next_block(0);
-    if (blk < n_blk) fetch(blk);
-    for (int it = 0; blk < n_blk; ++it) {
-        uint16_t * const Vt = Vt2[it & 1];
+    // Lane and instruction -> cell 64 / C i + lane / C, the piece that slot lane % C holds (past the row's end: its first one, which nobody uses)
+    uint16_t * const Kt = pool + wave * (KT + VB), * const Vl = Kt + KT;
+    uint32_t koff[CP / 4], voff;  // (the XOR patterns of K repeat every 16 cells, those of V every four)
+    auto kpiece = [&](const int i, const int64_t last) {
+        const int c = i * (64 / CP) + lane / CP, p = (lane % CP) ^ ((c / (16 / CP)) & (CP - 1));
+        return (uint32_t) std::min<int64_t>(c, last) * (uint32_t) k.nb[1] + (p < DK / 8 ? p * 16 : 0);
+    };
+    auto vpiece = [&](const int i, const int64_t last) {
+        const int c = i * (64 / CV) + lane / CV, p = (lane % CV) ^ (4 * ((c / (16 / CV)) & (CV / 4 - 1)));
+        return (uint32_t) std::min<int64_t>(c, last) * (uint32_t) v.nb[1] + (p < DV / 8 ? p * 16 : 0);
+    };
+#pragma unroll
+    for (int i = 0; i < CP / 4; ++i) koff[i] = kpiece(i, 31);
+    voff = vpiece(0, 31);
+    auto dma_k = [&](const int blk) {
+        const int64_t j0 = (int64_t) blk * 32;
+        const char * const from = k.data + kvh * k.nb[2] + j0 * k.nb[1];
+        const uint32_t to = (uint32_t) (uintptr_t) Kt;
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // (the block before has left LDS)
+        if (j0 + 32 <= n_kv) {
+#pragma unroll
+            for (int i = 0; i < CP / 2; ++i) att_dma16(from + (i / (CP / 4)) * 16 * k.nb[1], koff[i % (CP / 4)], to + i * 1024);
+        } else {
+#pragma unroll
+            for (int i = 0; i < CP / 2; ++i) att_dma16(from, kpiece(i, n_kv - 1 - j0), to + i * 1024);
+        }
+    };
+    auto dma_v = [&](const int blk) {
+        const int64_t j0 = (int64_t) blk * 32;
+        const char * const from = vbase + j0 * v.nb[1];
+        const uint32_t to = (uint32_t) (uintptr_t) Vl;
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        if (j0 + 32 <= n_kv) {
+#pragma unroll
+            for (int i = 0; i < CV / 2; ++i) att_dma16(from + i * (64 / CV) * v.nb[1], voff, to + i * 1024);
+        } else {
+#pragma unroll
+            for (int i = 0; i < CV / 2; ++i) att_dma16(from, vpiece(i, n_kv - 1 - j0), to + i * 1024);
+        }
+    };
+    int blk = next_block(wave);
+    if (blk < n_blk) {
+        fetch_mask(blk);
+        dma_k(blk);
+        dma_v(blk);
+    }
+    while (blk < n_blk) {
         const int64_t j0 = (int64_t) blk * 32;
         const bool tail = j0 + 32 > n_kv;  // (cells past the end: weight 0 and value 0 — a value read for them may be anything)
+        if (bias)
 #pragma unroll
-        for (int r = 0; r < NV; ++r) {
-            const int e0 = threadIdx.x + r * blockDim.x, cg = e0 / (DVT * 4), c8 = e0 % (DVT * 4);
-            if (cg < 8) {  // eight 8-byte groups: 4 cells of one entry
-                uint32_t u[4][4] = {{vn[r][0].x, vn[r][0].y, vn[r][0].z, vn[r][0].w}, {vn[r][1].x, vn[r][1].y, vn[r][1].z, vn[r][1].w},
-                                    {vn[r][2].x, vn[r][2].y, vn[r][2].z, vn[r][2].w}, {vn[r][3].x, vn[r][3].y, vn[r][3].z, vn[r][3].w}};
-                if (tail) {
-#pragma unroll
-                    for (int cc = 0; cc < 4; ++cc)
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) u[cc][e] = j0 + 4 * cg + cc < n_kv ? u[cc][e] : 0u;
-                }
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    // entries 2 e (low halves) and 2 e + 1 (high halves) of the four cells
-                    const uint2 lo2 = make_uint2(__builtin_amdgcn_perm(u[1][e], u[0][e], 0x05040100u), __builtin_amdgcn_perm(u[3][e], u[2][e], 0x05040100u));
-                    const uint2 hi2 = make_uint2(__builtin_amdgcn_perm(u[1][e], u[0][e], 0x07060302u), __builtin_amdgcn_perm(u[3][e], u[2][e], 0x07060302u));
-                    *(uint2 *) (Vt + (8 * c8 + 2 * e) * VS + 4 * cg) = lo2;
-                    *(uint2 *) (Vt + (8 * c8 + 2 * e + 1) * VS + 4 * cg) = hi2;
-                }
-            }
-        }
-        float mv[16];
-#pragma unroll
-        for (int i = 0; i < 16; ++i) mv[i] = q_live ? mv_next[i] : -INFINITY;
-        const bool wave_any = seen(mv);
-        __syncthreads();  // V^T of this block is staged; nobody reads the other copy any more
+            for (int i = 0; i < 16; ++i) mv[i] = q_live ? mv[i] : -INFINITY;
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(CV / 2) : "memory");  // (its K has landed: only its V may still fly)
         att_f16v S;
 #pragma unroll
         for (int i = 0; i < 16; ++i) S[i] = 0.0f;
-        if (wave_any) {
 #pragma unroll
-            for (int s = 0; s < DK16; ++s) S = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(att_bf8, kn[s]), __builtin_bit_cast(att_bf8, qf[s]), S, 0, 0, 0);
+        for (int s = 0; s < DK16; ++s) {
+            uint4 kf = *(const uint4 *) ((const char *) Kt + (n * CP + ((2 * s + g) ^ ((n / (16 / CP)) & (CP - 1)))) * 16);
+            if (!PLAIN && 16 * s + 8 * g >= DK) kf = make_uint4(0, 0, 0, 0);
+            S = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(att_bf8, kf), __builtin_bit_cast(att_bf8, qf[s]), S, 0, 0, 0);
+        }
+        float mx = ATTN_F32_LOW;
+        if (!bias) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                if constexpr (PLAIN) S[i] = S[i] * scale;
+                else S[i] = attn_score(S[i], scale, s_temp, softcap) + mask_term(0.0f, pen, r1, r2);
+                mx = fmaxf(mx, S[i]);
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                if constexpr (PLAIN) S[i] = mv[i] > -INFINITY ? S[i] * scale + mv[i] : -INFINITY;
+                else S[i] = mv[i] > -INFINITY ? attn_score(S[i], scale, s_temp, softcap) + mask_term(mv[i], pen, r1, r2) : -INFINITY;
+                mx = fmaxf(mx, S[i]);
+            }
         }
         blk = next_block(blk + 1);
-        if (blk < n_blk) fetch(blk);
-        if (!wave_any) continue;
-        float mx = ATTN_F32_LOW;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            if constexpr (PLAIN) S[i] = mv[i] > -INFINITY ? S[i] * scale + mv[i] : -INFINITY;
-            else S[i] = mv[i] > -INFINITY ? attn_score(S[i], scale, s_temp, softcap) + mask_term(mv[i], pen, r1, r2) : -INFINITY;
-            mx = fmaxf(mx, S[i]);
+        if (blk < n_blk) {
+            fetch_mask(blk);
+            dma_k(blk);
         }
+        __builtin_amdgcn_sched_barrier(0);
         mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-        const float m_new = sgm ? 0.0f : fmaxf(m, mx);
+        // the reference of the exponents follows the maximum only when that is e^8 ahead: weights stay below e^8, and the sums are rescaled a few times a row instead of at almost every block
+        const float m_new = sgm ? 0.0f : (mx > m + 8.0f ? mx : m);
         const float corr = sgm ? 1.0f : expf(m - m_new);
         float ps = 0.0f;
         uint32_t hi[8], lo[8];
 #pragma unroll
         for (int i = 0; i < 16; i += 2) {
             float p0, p1;
-            if constexpr (PLAIN) { p0 = expf(S[i] - m_new); p1 = expf(S[i + 1] - m_new); }
+            if constexpr (PLAIN) { p0 = att_exp(S[i] - m_new); p1 = att_exp(S[i + 1] - m_new); }
             else {
-                p0 = sgm ? (S[i] > -INFINITY ? attn_sigmoid(S[i] + s_bias) : 0.0f) : expf(S[i] - m_new);
-                p1 = sgm ? (S[i + 1] > -INFINITY ? attn_sigmoid(S[i + 1] + s_bias) : 0.0f) : expf(S[i + 1] - m_new);
+                p0 = sgm ? (S[i] > -INFINITY ? attn_sigmoid(S[i] + s_bias) : 0.0f) : att_exp(S[i] - m_new);
+                p1 = sgm ? (S[i + 1] > -INFINITY ? attn_sigmoid(S[i + 1] + s_bias) : 0.0f) : att_exp(S[i + 1] - m_new);
             }
             ps += p0 + p1;
             const uint32_t h2 = att_bf16_pack(p0, p1);
@@ -595,6 +660,13 @@ __global__ void __launch_bounds__(256, 2) k_attn_mma_bf16(const tdesc q, const t
 #pragma unroll
                 for (int i = 0; i < 16; ++i) O[dt][i] *= corr;
         }
+        if (blk < n_blk) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(CP / 2) : "memory");  // (the V of this block has landed: only the next one's K may still fly)
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        if (tail) {  // cells past the end: weight 0 and value 0 (a value read for them may be anything)
+            for (int i = lane; i < 32 * CV; i += 64)
+                if (j0 + i / CV >= n_kv) *(uint4 *) (Vl + i * 8) = make_uint4(0, 0, 0, 0);
+            asm volatile("" ::: "memory");  // (a wave's LDS accesses happen in the order they are written down in)
+        }
 #pragma unroll
         for (int s2 = 0; s2 < 2; ++s2) {
             const uint4 ph = make_uint4(hi[4 * s2], hi[4 * s2 + 1], hi[4 * s2 + 2], hi[4 * s2 + 3]);
@@ -602,8 +674,10 @@ __global__ void __launch_bounds__(256, 2) k_attn_mma_bf16(const tdesc q, const t
             uint4 vf[DVT];
 #pragma unroll
             for (int dt = 0; dt < DVT; ++dt) {
-                const uint16_t * vr = Vt + (32 * dt + n) * VS + 16 * s2 + 4 * g;
-                const uint2 a0 = *(const uint2 *) vr, a1 = *(const uint2 *) (vr + 8);
+                // a lane reads entries 4 (l & 3) .. + 3 of 16 of one cell and receives one entry (its lane's, l & 15) of four cells: 4 g .. + 3 and 8 + 4 g .. + 3 of the half block
+                const int l = lane & 15, c = 16 * s2 + 4 * g + (l >> 2), p = 4 * dt + 2 * ((lane >> 4) & 1) + ((l & 3) >> 1);
+                const uint16_t * vr = Vl + (c * CV + (p ^ (4 * ((c / (16 / CV)) & (CV / 4 - 1))))) * 8 + 4 * (l & 1);
+                const uint2 a0 = __builtin_bit_cast(uint2, att_read_tr(vr)), a1 = __builtin_bit_cast(uint2, att_read_tr(vr + 8 * CV * 8));
                 vf[dt] = make_uint4(a0.x, a0.y, a1.x, a1.y);
             }
 #pragma unroll
@@ -611,20 +685,44 @@ __global__ void __launch_bounds__(256, 2) k_attn_mma_bf16(const tdesc q, const t
 #pragma unroll
             for (int dt = 0; dt < DVT; ++dt) O[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(att_bf8, vf[dt]), __builtin_bit_cast(att_bf8, pl), O[dt], 0, 0, 0);
         }
+        if (blk < n_blk) dma_v(blk);
     }
+    // the waves' sums, relative to the largest of their references, added in the waves' order; a wave stores DVT of the 4 DVT groups of 8 entries
+    if (g == 0) {
+        meet[wave][0][n] = m;
+        meet[wave][1][n] = l;
+    }
+    __syncthreads();  // (nobody reads K or V any more)
+    float mm = meet[0][0][n];
+#pragma unroll
+    for (int w = 1; w < W; ++w) mm = fmaxf(mm, meet[w][0][n]);
+    l = 0.0f;
+#pragma unroll
+    for (int w = 0; w < W; ++w) l += meet[w][1][n] * (sgm ? 1.0f : expf(meet[w][0][n] - mm));
+    const float f = sgm ? 1.0f : expf(m - mm);
+    float4 * const sums = (float4 *) pool;
+#pragma unroll
+    for (int dt = 0; dt < DVT; ++dt)
+#pragma unroll
+        for (int b = 0; b < 4; ++b) sums[(wave * DVT * 4 + dt * 4 + b) * 64 + lane] = make_float4(O[dt][4 * b] * f, O[dt][4 * b + 1] * f, O[dt][4 * b + 2] * f, O[dt][4 * b + 3] * f);
+    __syncthreads();
     if (!q_live) return;
     const float inv = sgm ? 1.0f : (l > 0.0f ? 1.0f / l : 0.0f);
     float * out = (float *) (dst.data + h * dst.nb[1] + tq * dst.nb[2]);
 #pragma unroll
-    for (int dt = 0; dt < DVT; ++dt)
+    for (int i = 0; i < DVT; ++i) {
+        const int gi = wave * DVT + i, d0 = 32 * (gi >> 2) + 8 * (gi & 3) + 4 * g;
+        float4 p[W];
 #pragma unroll
-        for (int b = 0; b < 4; ++b) {
-            const int d0 = 32 * dt + 8 * b + 4 * g;
-            if (PLAIN || d0 + 3 < DV) *(float4 *) (out + d0) = make_float4(O[dt][4 * b] * inv, O[dt][4 * b + 1] * inv, O[dt][4 * b + 2] * inv, O[dt][4 * b + 3] * inv);
-            else
-                for (int r = 0; r < 4; ++r) if (d0 + r < DV) out[d0 + r] = O[dt][4 * b + r] * inv;
-        }
+        for (int w = 0; w < W; ++w) p[w] = sums[(w * DVT * 4 + gi) * 64 + lane];
+        const float v[4] = {((p[0].x + p[1].x) + (p[2].x + p[3].x)) * inv, ((p[0].y + p[1].y) + (p[2].y + p[3].y)) * inv, ((p[0].z + p[1].z) + (p[2].z + p[3].z)) * inv,
+                            ((p[0].w + p[1].w) + (p[2].w + p[3].w)) * inv};
+        if (PLAIN || d0 + 3 < DV) *(float4 *) (out + d0) = make_float4(v[0], v[1], v[2], v[3]);
+        else
+            for (int r = 0; r < 4; ++r) if (d0 + r < DV) out[d0 + r] = v[r];
+    }
 }
+
 // k_attn_mma_bf16_wide: the same scheme for ONE key/value head shared by all query heads and rows wider than a wave can hold — a latent cache row [latent | rotated part] of
 // several hundred values, its leading part the value.  The queries of a workgroup are 32 (token, head) pairs (head fastest); its four waves share them: wave w computes the
 // partial scores over a quarter of the key entries, the partials meet in LDS (every wave adds them in the order 0 .. 3 and so holds the same scores), every wave runs the f32
@@ -812,6 +910,7 @@ static bool attn_mma_bf16_ok(const tdesc & q, const tdesc & k, const tdesc & v, 
     if (!mask || mask->type != GGML_TYPE_F32 || (mask->nb[1] % 16) != 0 || (((uintptr_t) mask->data) & 15)) return false;
     if (k.type != GGML_TYPE_BF16 || v.type != GGML_TYPE_BF16 || q.ne[1] < 32) return false;
     if ((q.ne[0] % 8) != 0 || (v.ne[0] % 8) != 0 || q.ne[0] > 128 || v.ne[0] > 128) return false;
+    if (k.nb[1] >= (1 << 26) || v.nb[1] >= (1 << 26)) return false;  // (a block's offsets in 32 bits)
     if ((k.nb[1] % 16) || (k.nb[2] % 16) || (v.nb[1] % 16) || (v.nb[2] % 16) || (((uintptr_t) k.data | (uintptr_t) v.data | (uintptr_t) dst.data) & 15)) return false;
     if ((dst.nb[1] % 16) || (dst.nb[2] % 16)) return false;
     return true;
@@ -866,20 +965,10 @@ static void attn_f32_launch_t(hipStream_t s, const tdesc & q, const tdesc & k, c
             return;
         }
         if (mma_on && attn_mma_bf16_ok(q, k, v, mask, dst)) {  // prompt portions over a bf16 cache: the matrix cores
-            // waves per workgroup: four share a staged V^T block; two when four would leave most of the chip's 256 CUs without a workgroup (measured at 512 queries x 16
-            // heads: 1.87 ms for 16 launches with two waves, 2.12 with four, 1.99 with one)
-            int nw = ((n_q + 127) / 128) * H < 256 ? 2 : 4;
-            static const int nw_env = getenv("GGML_MI355X_ATTN_NW") ? atoi(getenv("GGML_MI355X_ATTN_NW")) : 0;
-            if (nw_env == 1 || nw_env == 2 || nw_env == 4) nw = nw_env;
-            while (nw > 1 && 32 * (nw / 2) >= n_q) nw >>= 1;  // (no more waves than the batch has groups of 32 queries)
-            const dim3 grid((unsigned) ((n_q + 32 * nw - 1) / (32 * nw)), (unsigned) H);
-            const dim3 block((unsigned) (64 * nw));
+            const dim3 grid((unsigned) ((n_q + 31) / 32), (unsigned) H);
             const int dk16 = (DK + 15) / 16, dvt = (DV + 31) / 32;
             const bool plain = !sig && !r12 && softcap <= 0.0f && DK == 16 * dk16 && DV == 32 * dvt;
-#define MI_ATT_MMA2(A, B, P) do { \
-                if (B >= 3 && nw == 1) hipLaunchKernelGGL((k_attn_mma_bf16<A, B, B >= 3 ? 2 : 1, P>), grid, block, 0, s, q, k, v, *mask, sinks, r12, dst, scale, sig, softcap, pen_kind); \
-                else hipLaunchKernelGGL((k_attn_mma_bf16<A, B, 1, P>), grid, block, 0, s, q, k, v, *mask, sinks, r12, dst, scale, sig, softcap, pen_kind); \
-            } while (0)
+#define MI_ATT_MMA2(A, B, P) hipLaunchKernelGGL((k_attn_mma_bf16<A, B, P>), grid, dim3(256), 0, s, q, k, v, *mask, sinks, r12, dst, scale, sig, softcap, pen_kind)
 #define MI_ATT_MMA(A, B) do { if (plain && dk16 == A && dvt == B) MI_ATT_MMA2(A, B, true); else MI_ATT_MMA2(A, B, false); } while (0)
             const int a = dk16 <= 2 ? 2 : (dk16 <= 4 ? 4 : (dk16 <= 6 ? 6 : 8)), b = dvt <= 1 ? 1 : (dvt <= 2 ? 2 : (dvt <= 3 ? 3 : 4));
             if (a == 2 && b == 1) MI_ATT_MMA(2, 1); else if (a == 2 && b == 2) MI_ATT_MMA(2, 2); else if (a == 2) MI_ATT_MMA(2, 4);

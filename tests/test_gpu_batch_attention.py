@@ -133,3 +133,46 @@ def test_one_head_over_one_key_head(H, T_, n_kv):
     p = np.exp(s - s.max(1, keepdims=True))
     ref = (p / p.sum(1, keepdims=True)).astype(np.float16).astype(np.float64) @ v.astype(np.float64).T
     assert np.abs(got - ref).max() <= 2e-3 * np.abs(ref).max() + 1e-5
+
+
+# k_attn_mma_bf16 (attn_f32.hip): blocks of 32 cells, every fourth one a wave's.  Fewer blocks than waves, a last block of 1 and of 31 cells, masks that leave a wave nothing, holes between requests,
+# biases, a row that sees nothing, rows of the f32's lowest value; heads in eights (the launch's other order) and not; head sizes of whole tiles and not
+@pytest.mark.parametrize("n_q,n_kv,heads,kv_heads,dk,dv", [(32, 32, 8, 2, 128, 128), (33, 97, 3, 1, 64, 64), (70, 287, 16, 4, 32, 128), (64, 1000, 8, 8, 96, 96), (100, 130, 5, 5, 72, 40), (257, 700, 8, 1, 128, 64),
+                                                           (40, 33, 6, 3, 24, 32)])
+@pytest.mark.parametrize("kind", ["causal", "holes", "bias", "lowest"])
+def test_prompts_over_a_bf16_cache(backend, H, n_q, n_kv, heads, kv_heads, dk, dv, kind):
+    rng = np.random.default_rng(n_q + n_kv + dk)
+    r16 = lambda a: (np.ascontiguousarray(a, np.float32).view(np.uint32) & 0xFFFF0000).view(np.float32)
+    bits = lambda a: (np.ascontiguousarray(a, np.float32).view(np.uint32) >> 16).astype(np.uint16)
+    q, k, v = (r16(rng.standard_normal(s) * f) for s, f in (((n_q, heads, dk), 2.0), ((n_kv, kv_heads, dk), 1.0), ((n_kv, kv_heads, dv), 1.0)))
+    low = np.finfo(np.float32).min if kind == "lowest" else -np.inf
+    t, j = np.arange(n_q)[:, None], np.arange(n_kv)[None, :]
+    ok = j <= t + max(0, n_kv - n_q)
+    if kind == "holes":
+        ok = ok & ((j // 40) % 3 == t % 3)
+    m = np.full((n_q, n_kv), low, np.float32)
+    m[ok] = 0.0
+    if kind == "bias":
+        m = np.where(ok, -0.01 * np.abs(t - j), -np.inf).astype(np.float32)
+        m[5] = -np.inf  # (a row that sees nothing: zeros)
+    mask = np.full((64 * ((n_q + 63) // 64), n_kv), -np.inf, np.float32)
+    mask[:n_q] = m
+    scale = 1.0 / np.sqrt(dk)
+
+    def build(g):
+        tk, tv = (g.new(L.BF16, [d * kv_heads, n_kv], bits(x)) for d, x in ((dk, k), (dv, v)))
+        kk = H.ggml_view_3d(g.ctx, tk, dk, n_kv, kv_heads, dk * kv_heads * 2, dk * 2, 0)
+        vv = H.ggml_view_3d(g.ctx, tv, dv, n_kv, kv_heads, dv * kv_heads * 2, dv * 2, 0)
+        r = H.ggml_flash_attn_ext(g.ctx, H.ggml_permute(g.ctx, g.new(L.F32, [dk, heads, n_q], q), 0, 2, 1, 3), kk, vv, g.new(L.F32, [n_kv, mask.shape[0]], mask), scale, 0.0, 0.0)
+        H.ggml_flash_attn_ext_set_prec(r, 10)
+        return r
+
+    got = T.run_case(build, backend)[0].reshape(n_q, heads, dv)
+    for h in range(heads):
+        z = scale * (q[:, h].astype(np.float64) @ k[:, h // (heads // kv_heads)].astype(np.float64).T) + m
+        top = z.max(axis=1, keepdims=True)
+        w = np.where(np.isfinite(z), np.exp(z - np.where(np.isfinite(top), top, 0.0)), 0.0)
+        den = w.sum(axis=1, keepdims=True)
+        ref = np.where(den > 0, w, 0.0) / np.where(den > 0, den, 1.0) @ v[:, h // (heads // kv_heads)].astype(np.float64)
+        # (a weight as two bf16 terms is off by 2^-17, a score of up to 40 in f32 sums by a few 2^-20)
+        assert np.abs(got[:, h] - ref).max() <= 2.0 ** -15 * np.abs(v).max()
