@@ -1334,7 +1334,7 @@ static int try_merge_mm_batch(exec_state & st, int i) {  // returns the number o
             epi_node = -1;
     }
     auto epi_fill = [&](mmq_epi & e, int slot, int role) {  // role: 0 q, 1 k, 2 v
-        e.kind[slot] = role == 0 ? 1 : (role == 1 ? 2 : (epl.a.v_idx ? 4 : 3));
+        e.kind[slot] = role == 0 ? 1 : role == 1 ? (epl.a.k_q8 ? 5 : 2) : epl.a.v_idx ? 4 : epl.a.v_q8 ? 6 : 3;
         e.out[slot] = role == 0 ? epl.a.q_dst : (role == 1 ? epl.a.k_cache : epl.a.v_cache);
         e.nb1[slot] = role == 0 ? epl.a.qd_nb1 : (role == 1 ? epl.a.kc_nb1 : epl.a.vc_nb1);
         e.nb2[slot] = role == 0 ? epl.a.qd_nb2 : 0;
@@ -1530,9 +1530,10 @@ static bool plan_rope_store(const exec_state & st, int i, rope_store_plan & pl) 
     if (rk->type != GGML_TYPE_F32 || ksrc->type != GGML_TYPE_F32 || ksrc->nb[0] != 4 || rk->ne[0] != rq->ne[0] || rk->ne[2] != rq->ne[2] || rk->ne[3] != 1) return false;
     if (use_count(st, rk) != 1 || (rk->flags & GGML_TENSOR_FLAG_OUTPUT)) return false;  // rope(k) lives only in the cache
     const int64_t HD = rq->ne[0], NH = rq->ne[1], NKV = rk->ne[1], T = rq->ne[2];
-    // cache stores: f16 rows of NKV * HD values, one I64 index per token, both stores through the same indices
+    // cache stores: f16 or Q8_0 rows of NKV * HD values, one I64 index per token, both stores through the same indices
+    auto q8_rows = [&](const ggml_tensor * sr) { return sr->type == GGML_TYPE_Q8_0 && (HD % 64) == 0 && rq->op_params[1] == HD && (sr->nb[1] % 2) == 0 && ((uintptr_t) sr->data & 1) == 0; };
     auto store_ok = [&](const ggml_tensor * sr, const ggml_tensor * src) {
-        return sr->type == GGML_TYPE_F16 && sr->nb[0] == 2 && sr->ne[0] == NKV * HD && src->ne[0] == NKV * HD && ggml_abi_nelements(src) == NKV * HD * T &&
+        return ((sr->type == GGML_TYPE_F16 && sr->nb[0] == 2) || q8_rows(sr)) && sr->ne[0] == NKV * HD && src->ne[0] == NKV * HD && ggml_abi_nelements(src) == NKV * HD * T &&
                sr->src[1]->type == GGML_TYPE_I64 && ggml_abi_nelements(sr->src[1]) == T && ggml_abi_is_contiguous(sr->src[1]);
     };
     // ... or, on the non-flash path, V transposed: the projection viewed as rows of ONE element, an index per element
@@ -1555,6 +1556,8 @@ static bool plan_rope_store(const exec_state & st, int i, rope_store_plan & pl) 
     a.kc_nb1 = (int64_t) ks->nb[1]; a.vc_nb1 = (int64_t) vs->nb[1];
     a.idx = (const int64_t *) ks->src[1]->data;
     a.v_idx = v_scatter ? (const int64_t *) vs->src[1]->data : nullptr;
+    a.k_q8 = ks->type == GGML_TYPE_Q8_0;
+    a.v_q8 = vs->type == GGML_TYPE_Q8_0;
     a.pos = (const int32_t *) rq->src[1]->data;
     a.ff = rq->src[2] ? (const float *) rq->src[2]->data : nullptr;
     a.p.n_dims = rq->op_params[1];

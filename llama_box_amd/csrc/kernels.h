@@ -215,9 +215,9 @@ struct mmq_mat_desc { const uint8_t * W; int64_t w_nb1; int N; float * dst; int6
 // Adjacent-pair ("normal") rotation only: both elements of a pair sit in one 32-row tile.
 struct mmq_epi {
     int kind[3];            // per matrix of the launch: 0 plain, 1 ROPE -> f32 rope(q) tensor, 2 ROPE -> f16 cache rows (k), 3 f16 cache rows (v),
-                            // 4 f16 elements of the TRANSPOSED V cache (non-flash path): value n of token t -> element v_idx[t * N + n]
-    char * out[3];          // kind 1: rope(q) data; 2 / 3: cache data
-    int64_t nb1[3], nb2[3]; // kind 1: bytes per head / per token of rope(q); 2 / 3: nb1 = bytes per cache row
+                            // 4 f16 elements of the TRANSPOSED V cache (non-flash path): value n of token t -> element v_idx[t * N + n]; 5 ROPE -> Q8_0 cache rows (k), 6 Q8_0 cache rows (v)
+    char * out[3];          // kind 1: rope(q) data; else cache data
+    int64_t nb1[3], nb2[3]; // kind 1: bytes per head / per token of rope(q); else nb1 = bytes per cache row
     const int32_t * pos;
     const float * ff;
     const int64_t * idx;    // cache row of each token
@@ -330,6 +330,7 @@ struct rope_store_args {
     char * k_cache; char * v_cache;
     int64_t kc_nb1, vc_nb1;
     const int64_t * idx;
+    bool k_q8, v_q8;        // cache rows of Q8_0 blocks instead of f16 (whole heads rotated, head sizes multiples of 64)
     const int64_t * v_idx;  // transposed V cache (non-flash path): one index per ELEMENT, [token][nkv * head_dim]; value j of the token -> f16 element v_idx[..] of v_cache
     const int32_t * pos;
     const float * ff;

@@ -446,13 +446,26 @@ __global__ void __launch_bounds__(SK_NW * 64, 1) k_mmq_skinny(const mmq8_args a)
             const int64_t e_nb2 = mi == 0 ? a.epi.nb2[0] : (mi == 1 ? a.epi.nb2[1] : a.epi.nb2[2]);
             const int head = n / a.epi.head_dim, dd = n - head * a.epi.head_dim;
             float r = v;
-            if (kind < 3 && dd < a.epi.n_dims) {
+            if ((kind < 3 || kind == 5) && dd < a.epi.n_dims) {
                 // (cos, sin) of (token, pair): the table launch_rope_table wrote for this graph run — the chain of multiplies and the accurate
                 // cosf / sinf of rope_cos_sin once per step, not once per layer and element (and no scratch frame in this kernel)
                 const float2 cssn = *(const float2 *) (a.epi.tab + ((size_t) tk * (a.epi.n_dims >> 1) + (dd >> 1)) * 2);
                 const float cs = cssn.x, sn = cssn.y;
                 const float x0 = (dd & 1) ? partner : v, x1 = (dd & 1) ? v : partner;
                 r = (dd & 1) ? x0 * sn + x1 * cs : x0 * cs - x1 * sn;
+            }
+            // the tile's 32 rows of a token are one Q8_0 block of the cache row, a half-wave's lanes (k_set_rows_q8_0's arithmetic).  9 tokens of Llama-3-8B: 12.5 us a layer, where the plain
+            // projections took as long and the sum of their K split, two rotations and two stores 22 us behind them
+            if (kind >= 5) {
+                float amax = fabsf(r);
+#pragma unroll
+                for (int o2 = 1; o2 < 32; o2 <<= 1) amax = fmaxf(amax, __shfl_xor(amax, o2));
+                const float d8 = amax / 127.0f, id8 = d8 != 0.0f ? 1.0f / d8 : 0.0f;
+                if (tok >= a.M) continue;
+                char * const blk = e_out + a.epi.idx[tok] * e_nb1 + (n >> 5) * 34;
+                blk[2 + (n & 31)] = (char) (int) roundf(r * id8);
+                if ((n & 31) == 0) *(uint16_t *) blk = f2h(d8);
+                continue;
             }
             if (tok >= a.M) continue;
             if (kind == 1) *(float *) (e_out + (int64_t) head * e_nb1 + (int64_t) tok * e_nb2 + (int64_t) dd * 4) = r;

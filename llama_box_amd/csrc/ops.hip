@@ -1530,6 +1530,32 @@ void launch_rope_table(hipStream_t s, const int32_t * pos, const float * ff, con
 // made the rope in-place), key heads are rotated and stored as f16 into the cache row the token's index names, value heads
 // are converted.  Arithmetic per element is that of k_rope
 // followed by k_set_rows (f32 result, then one f16 rounding), so fused and unfused graphs agree bit for bit.
+// Q8_0 rows of the cache: one, two or four neighbouring values a lane, a block's 32, 16 or 8 lanes live together; k_set_rows_q8_0's arithmetic
+__device__ __forceinline__ float q8_amax(float m, const int lanes) {
+    for (int o = 1; o < lanes; o <<= 1) m = fmaxf(m, __shfl_xor(m, o));
+    return m;
+}
+__device__ __forceinline__ uint32_t q8_quant(const float v, const float d) { return (uint32_t) ((int) roundf(v * (d != 0.0f ? 1.0f / d : 0.0f)) & 0xFF); }
+__device__ __forceinline__ void q8_store1(char * rowp, const int e, const float v) {
+    const float d = q8_amax(fabsf(v), 32) / 127.0f;
+    char * blk = rowp + (e >> 5) * 34;
+    blk[2 + (e & 31)] = (char) q8_quant(v, d);
+    if ((e & 31) == 0) *(uint16_t *) blk = f2h(d);
+}
+__device__ __forceinline__ void q8_store2(char * rowp, const int e, const float v0, const float v1) {
+    const float d = q8_amax(fmaxf(fabsf(v0), fabsf(v1)), 16) / 127.0f;
+    char * blk = rowp + (e >> 5) * 34;
+    *(uint16_t *) (blk + 2 + (e & 31)) = (uint16_t) (q8_quant(v0, d) | (q8_quant(v1, d) << 8));
+    if ((e & 31) == 0) *(uint16_t *) blk = f2h(d);
+}
+__device__ __forceinline__ void q8_store4(char * rowp, const int e, const float4 v) {
+    const float d = q8_amax(fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))), 8) / 127.0f;
+    char * blk = rowp + (e >> 5) * 34;
+    uint16_t * qs = (uint16_t *) (blk + 2 + (e & 31));
+    qs[0] = (uint16_t) (q8_quant(v.x, d) | (q8_quant(v.y, d) << 8));
+    qs[1] = (uint16_t) (q8_quant(v.z, d) | (q8_quant(v.w, d) << 8));
+    if ((e & 31) == 0) *(uint16_t *) blk = f2h(d);
+}
 __global__ void __launch_bounds__(256) k_rope_qk_store(const rope_store_args a) {
     // one workgroup per token; a thread owns rotation pair (tid & 63) [+ 64, ...] — its (cos, sin) is computed ONCE and serves every
     // head — and the four waves share out the head slots: [0, nh) query heads, [nh, nh + nkv) key heads, then value heads
@@ -1574,6 +1600,14 @@ __global__ void __launch_bounds__(256) k_rope_qk_store(const rope_store_args a) 
                 const float * src = (const float *) (a.k_src + h * a.k_nb1 + t * a.k_nb2);
                 uint16_t * dst = (uint16_t *) (a.k_cache + row * a.kc_nb1) + (int64_t) h * a.head_dim;
                 const float x0 = ld(1, src, h, ia), x1 = ld(1, src, h, ib);
+                if (a.k_q8) {  // (whole heads of 64 values and more: the lanes of a block are live together)
+                    char * rowp = a.k_cache + row * a.kc_nb1;
+                    if (neox) {
+                        q8_store1(rowp, h * a.head_dim + ia, x0 * cs - x1 * sn);
+                        q8_store1(rowp, h * a.head_dim + ib, x0 * sn + x1 * cs);
+                    } else q8_store2(rowp, h * a.head_dim + ia, x0 * cs - x1 * sn, x0 * sn + x1 * cs);
+                    continue;
+                }
                 dst[ia] = f2h(x0 * cs - x1 * sn);
                 dst[ib] = f2h(x0 * sn + x1 * cs);
             }
@@ -1596,6 +1630,8 @@ __global__ void __launch_bounds__(256) k_rope_qk_store(const rope_store_args a) 
             if (a.v_idx) {
                 const int64_t * ix = a.v_idx + ((int64_t) t * a.nkv + h) * a.head_dim;
                 for (int i0 = lane; i0 < a.head_dim; i0 += 64) ((uint16_t *) a.v_cache)[ix[i0]] = f2h(ld(2, src, h, i0));
+            } else if (a.v_q8) {
+                for (int i0 = lane; i0 < a.head_dim; i0 += 64) q8_store1(a.v_cache + row * a.vc_nb1, h * a.head_dim + i0, ld(2, src, h, i0));
             } else {
                 uint16_t * dst = (uint16_t *) (a.v_cache + row * a.vc_nb1) + (int64_t) h * a.head_dim;
                 for (int i0 = lane; i0 < a.head_dim; i0 += 64) dst[i0] = f2h(ld(2, src, h, i0));
@@ -1655,6 +1691,9 @@ __global__ void __launch_bounds__(256) k_rope_qk_store_vec(const rope_store_args
                     float * dst = (float *) (a.q_dst + (int64_t) slot * a.qd_nb1 + t * a.qd_nb2);
                     *(float4 *) (dst + 4 * j) = o0;
                     if (NEOX) *(float4 *) (dst + half + 4 * j) = o1;
+                } else if (a.k_q8) {  // (eight lanes a block)
+                    q8_store4(a.k_cache + row * a.kc_nb1, (slot - a.nh) * hd + 4 * j, o0);
+                    if (NEOX) q8_store4(a.k_cache + row * a.kc_nb1, (slot - a.nh) * hd + half + 4 * j, o1);
                 } else {
                     uint16_t * dst = (uint16_t *) (a.k_cache + row * a.kc_nb1) + (int64_t) (slot - a.nh) * hd;
                     *(uint2 *) (dst + 4 * j) = make_uint2((uint32_t) f2h(o0.x) | ((uint32_t) f2h(o0.y) << 16), (uint32_t) f2h(o0.z) | ((uint32_t) f2h(o0.w) << 16));
@@ -1670,6 +1709,8 @@ __global__ void __launch_bounds__(256) k_rope_qk_store_vec(const rope_store_args
                     vc[i1] = f2h(lo[k].y);
                     vc[i2] = f2h(lo[k].z);
                     vc[i3] = f2h(lo[k].w);
+                } else if (a.v_q8) {
+                    q8_store4(a.v_cache + row * a.vc_nb1, h * hd + 4 * j, lo[k]);
                 } else {
                     uint16_t * dst = (uint16_t *) (a.v_cache + row * a.vc_nb1) + (int64_t) h * hd;
                     *(uint2 *) (dst + 4 * j) = make_uint2((uint32_t) f2h(lo[k].x) | ((uint32_t) f2h(lo[k].y) << 16), (uint32_t) f2h(lo[k].z) | ((uint32_t) f2h(lo[k].w) << 16));
@@ -1683,10 +1724,10 @@ bool rope_qk_store_vec_ok(const rope_store_args & a, int n_tokens) {
     if (!on || n_tokens < 33 || a.ks > 1 || a.sk[0].part || a.sk[1].part || a.sk[2].part) return false;
     if ((a.p.mode & ~GGML_ROPE_TYPE_NEOX) != 0 || a.p.n_dims != a.head_dim || (a.head_dim % 8) != 0) return false;
     auto al16 = [](const void * p) { return (((uintptr_t) p) & 15) == 0; };
-    if (!al16(a.q_src) || !al16(a.q_dst) || !al16(a.k_src) || !al16(a.v_src) || !al16(a.k_cache) || !al16(a.v_cache)) return false;
+    if (!al16(a.q_src) || !al16(a.q_dst) || !al16(a.k_src) || !al16(a.v_src) || (!a.k_q8 && !al16(a.k_cache)) || (!a.v_q8 && !al16(a.v_cache))) return false;
     for (int64_t v : {a.q_nb1, a.q_nb2, a.qd_nb1, a.qd_nb2, a.k_nb1, a.k_nb2, a.v_nb1, a.v_nb2})
         if (v % 16) return false;
-    return (a.kc_nb1 % 8) == 0 && (a.v_idx != nullptr || (a.vc_nb1 % 8) == 0);
+    return (a.k_q8 || (a.kc_nb1 % 8) == 0) && (a.v_idx != nullptr || a.v_q8 || (a.vc_nb1 % 8) == 0);
 }
 void launch_rope_qk_store_vec(hipStream_t s, const rope_store_args & a, int n_tokens, const float * tab) {
     if (a.p.mode & GGML_ROPE_TYPE_NEOX) hipLaunchKernelGGL(k_rope_qk_store_vec<true>, dim3((unsigned) n_tokens), dim3(256), 0, s, a, tab);

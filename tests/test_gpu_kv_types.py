@@ -468,3 +468,42 @@ def test_model_logits_without_flash_attention_and_a_k_cache_in_kv_types(backend,
     finally:
         for o in (cc, cg, mc, mg):
             o.free()
+
+
+# ROPE(q), ROPE(k) and both cache stores of a batch, rows of Q8_0 blocks (or of one type each): in the projections' epilogue (2 .. 32 tokens, adjacent pairs), in one launch (fewer than 33 tokens;
+# split-K sums read there), in its vectorised form (33 and up); heads of 64 and 128 values
+@pytest.mark.parametrize("kt,vt", [(L.Q8_0, L.Q8_0), (L.Q8_0, L.F16), (L.F16, L.Q8_0)])
+@pytest.mark.parametrize("mode,HD,M,project", [(0, 128, 2, True), (0, 128, 9, True), (0, 64, 32, True), (0, 64, 3, False), (L.ROPE_NEOX, 128, 5, False), (L.ROPE_NEOX, 64, 20, True), (0, 128, 33, False),
+                                               (L.ROPE_NEOX, 64, 40, False), (L.ROPE_NEOX, 128, 130, False)])
+def test_batch_rope_and_stores_into_q8_0_rows(backend, H, kt, vt, mode, HD, M, project):
+    rng = np.random.default_rng(M + HD + kt + 3 * vt)
+    E, NH, NKV, NCTX = 512, 8, 2, 300
+    x = rng.standard_normal((M, E)).astype(np.float32)
+    ws = [T.rand_weight(L.Q4_K, E, n * HD, rng) for n in (NH, NKV, NKV)]
+    direct = [(rng.standard_normal((M, n * HD)) * rng.uniform(0.0, 3.0, (M, 1))).astype(np.float32) for n in (NH, NKV, NKV)]
+    direct[1][0] = 0.0  # (a block of zeros)
+    pos, rows = rng.integers(0, 5000, M).astype(np.int32), rng.permutation(NCTX)[:M].astype(np.int64)
+
+    def build(g):
+        cur = g.new(L.F32, [E, M], x)
+        if project:
+            q, k, v = (H.ggml_mul_mat(g.ctx, g.new(L.Q4_K, [E, n * HD], w), cur) for n, w in zip((NH, NKV, NKV), ws))
+        else:
+            q, k, v = (g.new(L.F32, [n * HD, M], d) for n, d in zip((NH, NKV, NKV), direct))
+        tp, idx = g.new(L.I32, [M], pos), g.new(L.I64, [M], rows)
+        q, k = (H.ggml_rope_ext(g.ctx, H.ggml_reshape_3d(g.ctx, t, HD, n, M), tp, None, HD, mode, 8192, 500000.0, 1.0, 0.0, 1.0, 32.0, 1.0) for t, n in ((q, NH), (k, NKV)))
+        return [q, H.ggml_set_rows(g.ctx, g.new(kt, [NKV * HD, NCTX]), H.ggml_reshape_2d(g.ctx, k, NKV * HD, M), idx), H.ggml_set_rows(g.ctx, g.new(vt, [NKV * HD, NCTX]), v, idx)]
+
+    n0, k0 = backend.stat("fused_nodes"), backend.stat("kernel_launches")
+    got = T.run_case(build, backend)
+    fused, launches = backend.stat("fused_nodes") - n0, backend.stat("kernel_launches") - k0
+    backend.set_option("fusion", 0)
+    try:
+        k0 = backend.stat("kernel_launches")
+        plain = T.run_case(build, backend)
+        apart = backend.stat("kernel_launches") - k0
+    finally:
+        backend.set_option("fusion", 1)
+    assert fused >= 3 and launches <= apart - 2, (fused, launches, apart)
+    for name, a, b in zip(("q", "k cache", "v cache"), got, plain):
+        assert np.array_equal(np.asarray(a).view(np.uint8), np.asarray(b).view(np.uint8)), name
