@@ -1004,7 +1004,9 @@ template <int D, bool Q8OUT = false> __global__ void __launch_bounds__(Q8OUT ? 2
 // The arithmetic is k_fattn_combine's: coefficients exp(m_s - max), values selected (not multiplied) where the coefficient is 0, sum in split order.
 // Q8OUT: the rows' only readers are quantised mat-muls (wo): a wave holds two adjacent heads of a token = one Q8_K block, lane l its values
 // 4 l .. 4 l + 3 — the block is quantised in registers (wave_quantize_q8_K, the arithmetic of k_quantize_q8_K) and no f32 row is written.
-template <int D, int S, bool Q8OUT = false>
+// OUT = 2 (head_dim 64): ... by Q8_0 mat-muls on the matrix cores: eight threads hold a Q8_0 block and leave it in panel order (k_quantize_q8_0's arithmetic).  32 heads of 64: 512 tokens 9.1 us and
+// 4.9 for the quantiser behind it -> 6.6; 16 tokens 3.8 and 2.7 -> 4.0.
+template <int D, int S, int OUT = 0>
 __global__ void __launch_bounds__(256) k_fattn_combine_rows(const float * __restrict__ ws, const tdesc dst, const fa_geom geo, const int n_rows, q8k_dev * __restrict__ q8 = nullptr) {
     constexpr int CPR = D / 4;            // chunks (threads) per row
     constexpr int RPB = 256 / CPR;        // rows per workgroup
@@ -1038,7 +1040,21 @@ __global__ void __launch_bounds__(256) k_fattn_combine_rows(const float * __rest
         a.w += c != 0.0f ? v[u].w * c : 0.0f;
     }
     const float inv = 1.0f / lt;
-    if constexpr (Q8OUT) {
+    if constexpr (OUT == 2) {
+        const float t[4] = {a.x * inv, a.y * inv, a.z * inv, a.w * inv};
+        float amax = fmaxf(fmaxf(fabsf(t[0]), fabsf(t[1])), fmaxf(fabsf(t[2]), fabsf(t[3])));
+        amax = fmaxf(amax, __shfl_xor(amax, 1, 64));
+        amax = fmaxf(amax, __shfl_xor(amax, 2, 64));
+        amax = fmaxf(amax, __shfl_xor(amax, 4, 64));
+        const float d = amax / 127.0f, id = d != 0.0f ? 1.0f / d : 0.0f;
+        uint32_t packed = 0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) packed |= (uint32_t) ((int) roundf(t[k] * id) & 0xFF) << (8 * k);
+        const int e0 = h * D + 4 * j, w8 = j & 7, col = bat * geo.n_q + tok;
+        char * tile = (char *) q8 + ((size_t) (col >> 5) * (size_t) (geo.n_head * D / 32) + (size_t) (e0 >> 5)) * 1152;
+        *(uint32_t *) (tile + (w8 >> 2) * 512 + (col & 31) * 16 + (w8 & 3) * 4) = packed;
+        if (w8 == 0) *(float *) (tile + 1024 + (col & 31) * 4) = h2f(f2h(d));
+    } else if constexpr (OUT == 1) {
         static_assert(D == 128, "two heads of 128 = one block");
         const float t[4] = {a.x * inv, a.y * inv, a.z * inv, a.w * inv};
         wave_quantize_q8_K(t, (int) threadIdx.x & 63, q8 + (r >> 1));  // (n_head and n_rows are even: the launcher checked)
@@ -1054,7 +1070,7 @@ bool fattn_combine_rows_applies(int D, int64_t n_q, int64_t n_head, int64_t n_ba
     const int64_t n_rows = n_batch * n_q * n_head;
     return rows_on && !sinks && D == 128 && n_splits >= 2 && n_splits <= 8 && n_rows >= 2048 && n_rows < (1 << 30);
 }
-void launch_flash_attn_combine(hipStream_t s, int D, const float * ws, const float * sinks, const tdesc & dst, int n_q, int n_head, int n_batch, int n_splits, void * q8_out) {
+void launch_flash_attn_combine(hipStream_t s, int D, const float * ws, const float * sinks, const tdesc & dst, int n_q, int n_head, int n_batch, int n_splits, void * q8_out, void * q80_out) {
     fa_geom geo{};
     geo.n_q = n_q;
     geo.n_head = n_head;
@@ -1064,12 +1080,18 @@ void launch_flash_attn_combine(hipStream_t s, int D, const float * ws, const flo
         (q8_out ? (n_head % 2) == 0 : ((dst.nb[1] % 16) == 0 && (dst.nb[2] % 16) == 0 && (dst.nb[3] % 16) == 0 && (((uintptr_t) dst.data) & 15) == 0))) {
         const unsigned blocks = (unsigned) ((n_rows + 7) / 8);
         if (q8_out) {
-            if (n_splits <= 4) hipLaunchKernelGGL((k_fattn_combine_rows<128, 4, true>), dim3(blocks), dim3(256), 0, s, ws, dst, geo, (int) n_rows, (q8k_dev *) q8_out);
-            else hipLaunchKernelGGL((k_fattn_combine_rows<128, 8, true>), dim3(blocks), dim3(256), 0, s, ws, dst, geo, (int) n_rows, (q8k_dev *) q8_out);
+            if (n_splits <= 4) hipLaunchKernelGGL((k_fattn_combine_rows<128, 4, 1>), dim3(blocks), dim3(256), 0, s, ws, dst, geo, (int) n_rows, (q8k_dev *) q8_out);
+            else hipLaunchKernelGGL((k_fattn_combine_rows<128, 8, 1>), dim3(blocks), dim3(256), 0, s, ws, dst, geo, (int) n_rows, (q8k_dev *) q8_out);
         } else {
             if (n_splits <= 4) hipLaunchKernelGGL((k_fattn_combine_rows<128, 4>), dim3(blocks), dim3(256), 0, s, ws, dst, geo, (int) n_rows, (q8k_dev *) nullptr);
             else hipLaunchKernelGGL((k_fattn_combine_rows<128, 8>), dim3(blocks), dim3(256), 0, s, ws, dst, geo, (int) n_rows, (q8k_dev *) nullptr);
         }
+        return;
+    }
+    if (q80_out) {  // (only where fattn_q80_out_ok said so)
+        const unsigned blocks = (unsigned) ((n_rows + 15) / 16);
+        if (n_splits <= 4) hipLaunchKernelGGL((k_fattn_combine_rows<64, 4, 2>), dim3(blocks), dim3(256), 0, s, ws, dst, geo, (int) n_rows, (q8k_dev *) q80_out);
+        else hipLaunchKernelGGL((k_fattn_combine_rows<64, 8, 2>), dim3(blocks), dim3(256), 0, s, ws, dst, geo, (int) n_rows, (q8k_dev *) q80_out);
         return;
     }
     dim3 g2((unsigned) n_head, (unsigned) n_q, (unsigned) n_batch);
@@ -1264,6 +1286,19 @@ bool fattn_q8_out_ok(const tdesc & q, const tdesc & k, const tdesc * mask, const
     if (p.n_splits == 1 && ((G & 1) || p.fat || flash_attn_mma_applies(q, k, mask, sinks, dst, p))) return false;  // one pass: the lane-parallel kernel quantises whole head pairs of a kv group
     return p.logit_softcap == 0.0f && p.max_bias == 0.0f && fa_g_ok(G) && (q.nb[1] % 16) == 0 && (q.nb[2] % 16) == 0 && ((uintptr_t) q.data & 15) == 0;
 }
+// the head_dim-64 forms that take p.lists (see launch_flash_attn)
+static bool dec64_applies(const tdesc & q, const tdesc & k, const tdesc & v, const fattn_params & p) {
+    static const bool on = !getenv("GGML_MI355X_FA_DEC64") || atoi(getenv("GGML_MI355X_FA_DEC64")) != 0;
+    return on && k.ne[0] == 64 && k.type == GGML_TYPE_F16 && v.type == GGML_TYPE_F16 && (q.ne[1] == 1 || (p.lists && q.ne[3] == 1)) && p.logit_softcap == 0.0f && p.max_bias == 0.0f && fa_g_ok((int) (q.ne[2] / k.ne[2])) &&
+           (q.nb[1] % 16) == 0 && (q.nb[2] % 16) == 0 && ((uintptr_t) q.data & 15) == 0 && (k.nb[1] % 16) == 0 && (v.nb[1] % 16) == 0 && (k.nb[2] % 16) == 0 && (v.nb[2] % 16) == 0 &&
+           ((uintptr_t) k.data & 15) == 0 && ((uintptr_t) v.data & 15) == 0 && p.q8_out == nullptr;
+}
+// will launch_flash_attn end in the combine pass that leaves Q8_0 panel blocks? (mirrors its dispatch)
+bool fattn_q80_out_ok(const tdesc & q, const tdesc & k, const tdesc & v, const tdesc * mask, const float * sinks, const tdesc & dst, const fattn_params & p) {
+    if (k.ne[0] != 64 || k.ne[2] <= 0 || q.ne[2] % k.ne[2] != 0 || sinks || p.n_splits < 2 || p.n_splits > 8 || q.ne[3] != 1 || p.kv_type != GGML_TYPE_F16 || p.dq || p.fat) return false;
+    if (!p.lists && flash_attn_mma_applies(q, k, mask, sinks, dst, p)) return true;
+    return p.lists && dec64_applies(q, k, v, p);
+}
 void launch_flash_attn(hipStream_t s, const tdesc & q, const tdesc & k, const tdesc & v, const tdesc * mask, const float * sinks, const tdesc & dst,
                        const fattn_params & p, void * workspace) {
     const bool q8 = p.kv_type == GGML_TYPE_Q8_0;
@@ -1408,10 +1443,7 @@ void launch_flash_attn(hipStream_t s, const tdesc & q, const tdesc & k, const td
     }
     // one decode token at head_dim 64 over an f16 cache (round 6): the lane-parallel kernel in its eight-lane-row form, records + combine pass
     // (generic kernel: 14.9 us per layer for TinyLlama at a 600-cell context; profiles/r06_secondary_kernel_stats.txt)
-    static const bool dec64_on = !getenv("GGML_MI355X_FA_DEC64") || atoi(getenv("GGML_MI355X_FA_DEC64")) != 0;
-    if (dec64_on && D == 64 && k.type == GGML_TYPE_F16 && v.type == GGML_TYPE_F16 && (geo.n_q == 1 || (p.lists && q.ne[3] == 1)) && p.logit_softcap == 0.0f && p.max_bias == 0.0f && fa_g_ok(G) &&
-        (q.nb[1] % 16) == 0 && (q.nb[2] % 16) == 0 && ((uintptr_t) q.data & 15) == 0 && (k.nb[1] % 16) == 0 && (v.nb[1] % 16) == 0 && (k.nb[2] % 16) == 0 && (v.nb[2] % 16) == 0 &&
-        ((uintptr_t) k.data & 15) == 0 && ((uintptr_t) v.data & 15) == 0 && p.q8_out == nullptr) {
+    if (dec64_applies(q, k, v, p)) {
         geo.arrive = nullptr;
         geo.merge2 = 0;
         geo.q8 = nullptr;
@@ -1444,7 +1476,7 @@ void launch_flash_attn(hipStream_t s, const tdesc & q, const tdesc & k, const td
                 else hipLaunchKernelGGL((k_fattn_dec128<8, 0, false, 4, 0, 64>), grid, dim3(256), 0, s, qb, kb, vb, mb, sinks, db, geo, wsb, G, nullptr, 0);
             }
         }
-        if (geo.n_splits > 1) launch_flash_attn_combine(s, 64, ws, sinks, dst, geo.n_q, geo.n_head, (int) q.ne[3], geo.n_splits, nullptr);
+        if (geo.n_splits > 1) launch_flash_attn_combine(s, 64, ws, sinks, dst, geo.n_q, geo.n_head, (int) q.ne[3], geo.n_splits, nullptr, p.q80_out);
         return;
     }
 #define FA_CASE(DD, GG) \

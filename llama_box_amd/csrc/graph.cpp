@@ -3562,9 +3562,21 @@ static int run_node(exec_state & st, int i) {
                 }
             }
             if (q8_reader) p.q8_out = (char *) c->ws + st.act_off;
+            // ... and the same for a Q8_0 wo on the matrix cores behind heads of 64
+            const ggml_tensor * q80_reader = nullptr;
+            const float * const sk = n->src[4] ? (const float *) n->src[4]->data : nullptr;
+            if (!q8_reader && fuse && c->opt.prologue && a->ne[1] > 8 && use_count(st, n) == 1 && !(n->flags & GGML_TENSOR_FLAG_OUTPUT) && ggml_abi_is_contiguous(n) && fattn_q80_out_ok(qd, kd, vd, m ? &md : nullptr, sk, TD(n), p)) {
+                for (int k = i + 1; k < std::min(g->n_nodes, i + 4) && !q80_reader; ++k) {
+                    const ggml_tensor * t = g->nodes[k];
+                    if ((t->op == GGML_OP_RESHAPE || t->op == GGML_OP_VIEW) && t->src[0] == n && t->data == n->data && ggml_abi_is_contiguous(t) && t->ne[0] == n->ne[0] * n->ne[1] &&
+                        t->ne[1] == n->ne[2] && q80_panel_consumers_only(st, k, t))
+                        q80_reader = t;
+                }
+            }
+            if (q80_reader) p.q80_out = (char *) c->ws + st.act_off;
             launch_flash_attn(s, qd, kd, vd, m ? &md : nullptr, n->src[4] ? (const float *) n->src[4]->data : nullptr, TD(n), p, (char *) c->ws + st.aux_off);
-            if (q8_reader) {
-                mark_q8_cache(st, q8_reader);
+            if (q8_reader || q80_reader) {
+                mark_q8_cache(st, q8_reader ? q8_reader : q80_reader, q8_reader ? GGML_TYPE_Q8_K : MI_ACT_Q80_PANEL);
                 c->st.fused_nodes++;
             }
             c->st.kernel_launches += p.n_splits > 1 ? 2 : 1;

@@ -364,6 +364,7 @@ struct fattn_params {
     const int * lists = nullptr;  // per-token lists of visible cache positions (launch_fattn_tile_scan), or nullptr
     void * q8_out = nullptr;  // the result's only readers are quantised mat-muls (wo of a batch): leave it as Q8_K blocks here — honoured by
                               // the combine pass of the head_dim-128 kernels (n_splits > 1), see fattn_q8_out_ok()
+    void * q80_out = nullptr; // ... by Q8_0 mat-muls of 9 columns and up: as Q8_0 blocks in panel order, by the combine pass of the head_dim-64 kernels, see fattn_q80_out_ok()
     unsigned * arrive = nullptr;  // zeroed counters (arrive_slots of them): lets the split kernel of the head_dim-128 decode path merge its own
     int arrive_slots = 0;         // partial records (last workgroup to arrive) instead of a second launch; the kernel leaves them at zero
     const uint8_t * tile_vis = nullptr;  // matrix-core kernel: [q tile of 32][kv tile of 64] visibility bytes (launch_fattn_vis_scan), or nullptr
@@ -390,6 +391,7 @@ int fattn_pick_splits(const tdesc & q, const tdesc & k, const tdesc * mask = nul
 // batches of many sequences over a unified cache, llama-box/httpserver.hpp:4042-4069) of up to 256 tokens walks per-token position lists instead
 bool fattn_prefers_lists(const tdesc & q, const tdesc * mask, int mask_sparse);
 int fattn_fat_splits(const tdesc & q, const tdesc & k, const tdesc * mask, const float * sinks, const fattn_params & p);  // 0 = the fat-split form does not apply
+bool fattn_q80_out_ok(const tdesc & q, const tdesc & k, const tdesc & v, const tdesc * mask, const float * sinks, const tdesc & dst, const fattn_params & p);
 bool fattn_q8_out_ok(const tdesc & q, const tdesc & k, const tdesc * mask, const float * sinks, const tdesc & dst, const fattn_params & p);  // will this launch end in the quantising combine?
 void launch_flash_attn(hipStream_t s, const tdesc & q, const tdesc & k, const tdesc & v, const tdesc * mask, const float * sinks,
                        const tdesc & dst, const fattn_params & p, void * workspace);
@@ -397,7 +399,7 @@ void launch_flash_attn(hipStream_t s, const tdesc & q, const tdesc & k, const td
 bool launch_flash_attn_mma(hipStream_t s, const tdesc & q, const tdesc & k, const tdesc & v, const tdesc * mask, const float * sinks, const tdesc & dst,
                            const fattn_params & p, void * workspace);
 int fattn_mma_pick_splits(const tdesc & q, const tdesc & k);
-void launch_flash_attn_combine(hipStream_t s, int D, const float * ws, const float * sinks, const tdesc & dst, int n_q, int n_head, int n_batch, int n_splits, void * q8_out = nullptr);
+void launch_flash_attn_combine(hipStream_t s, int D, const float * ws, const float * sinks, const tdesc & dst, int n_q, int n_head, int n_batch, int n_splits, void * q8_out = nullptr, void * q80_out = nullptr);
 
 // ---- the decode copy (repack.hip): rows [r0, r0 + n_rows) of a K-quant [K, N] matrix from the block layout at `src` into the plane layout at `dst` (same row stride)
 bool repack_supported(int type, int64_t K, int64_t nb1);

@@ -176,3 +176,37 @@ def test_prompts_over_a_bf16_cache(backend, H, n_q, n_kv, heads, kv_heads, dk, d
         ref = np.where(den > 0, w, 0.0) / np.where(den > 0, den, 1.0) @ v[:, h // (heads // kv_heads)].astype(np.float64)
         # (a weight as two bf16 terms is off by 2^-17, a score of up to 40 in f32 sums by a few 2^-20)
         assert np.abs(got[:, h] - ref).max() <= 2.0 ** -15 * np.abs(v).max()
+
+
+# heads of 64 whose only reader is a Q8_0 product on the matrix cores: the combine pass leaves the product's quantised blocks — tokens on lists (9 .. 32) and prompts, 2 .. 8 records a row
+@pytest.mark.parametrize("T_,n_kv,NH,NKV,splits", [(9, 640, 8, 2, 0), (16, 2560, 32, 4, 0), (32, 512, 8, 8, 8), (40, 512, 16, 4, 0), (130, 700, 8, 4, 5), (512, 1024, 16, 2, 0)])
+def test_heads_of_64_leave_quantised_rows(backend, H, T_, n_kv, NH, NKV, splits):
+    rng = np.random.default_rng(T_ + n_kv)
+    q, k, v = (rng.standard_normal(s).astype(np.float32) for s in ((NH, T_, 64), (NKV, n_kv, 64), (NKV, n_kv, 64)))
+    w = T.rand_weight(L.Q8_0, NH * 64, 256, rng)
+    mask = np.full(((T_ + 63) // 64 * 64, n_kv), -np.inf, np.float16)
+    for t in range(T_):
+        mask[t, : n_kv - T_ + t + 1] = 0
+
+    def build(also):
+        def f(g):
+            tq, tk, tv = g.new(L.F32, [64, T_, NH], q), g.new(L.F16, [64, n_kv, NKV], k.astype(np.float16)), g.new(L.F16, [64, n_kv, NKV], v.astype(np.float16))
+            a = H.ggml_flash_attn_ext(g.ctx, tq, tk, tv, g.new(L.F16, [n_kv, mask.shape[0]], mask), 0.125, 0.0, 0.0)
+            H.ggml_flash_attn_ext_set_prec(a, 10)
+            r = H.ggml_mul_mat(g.ctx, g.new(L.Q8_0, [NH * 64, 256], w), H.ggml_reshape_2d(g.ctx, a, NH * 64, T_))
+            return [r, a] if also else [r]
+        return f
+
+    backend.set_option("fa_splits", splits)
+    try:
+        n = []
+        out = []
+        for also in (False, True):  # (an attention result that is an output itself exists in f32, with a quantiser behind it)
+            k0 = backend.stat("kernel_launches")
+            out.append(np.asarray(T.run_case(build(also), backend)[0], np.float32))
+            n.append(backend.stat("kernel_launches") - k0)
+    finally:
+        backend.set_option("fa_splits", 0)
+    assert n[0] == n[1] - 1, n
+    # (the two combine passes sum the records' weights in another order: a value next to a rounding boundary moves by 1 / 127 of its block's largest, few of them)
+    assert T.nmse(out[0], out[1]) <= 1e-6
