@@ -1423,7 +1423,7 @@ static int try_merge_mm_batch(exec_state & st, int i) {  // returns the number o
 
 // Q8_0 weights, 9 columns and up: wq / wk / wv (and gate / up) of a batch multiply the same activations — one launch of the matrix-core
 // kernel over the concatenated 32-row panels (mmq_q80.hip), bias ADDs folded into the store.  The member search is try_merge_mm_batch's (same dependence rules);
-// no K split, no epilogues: with the K / V projections out of the way the ropes and cache stores that follow fuse as they do for the K-quants (try_fuse_rope_store).
+// no K split.  Up to 32 tokens the ropes and cache stores that follow join the launch, beyond that they fuse as they do for the K-quants (try_fuse_rope_store).
 static int try_merge_q80_skinny(exec_state & st, int i) {  // returns the number of nodes consumed at position i (0: not merged)
     backend_ctx * c = st.c;
     ggml_cgraph * g = st.g;
@@ -1480,12 +1480,64 @@ static int try_merge_q80_skinny(exec_state & st, int i) {  // returns the number
         wbytes += (double) ggml_abi_row_size(w->type, K) * (double) w->ne[1];
     }
     if (with_copy != 0 && with_copy != (int) ms.size()) return 0;  // (one template form per launch: all from their panel copies, or none)
+    // wq / wk / wv of up to 32 tokens with ROPE(q), ROPE(k) and both cache stores behind them (the window plan_rope_store recognises): the launch rotates and stores in its epilogue
+    rope_store_plan epl;
+    mmq_epi epi{};
+    int epi_node = -1;
+    if (c->opt.fusion && c->opt.skinny_rope && M <= 32 && ms.size() == 3 && st.rs_sk.node < 0) {
+        auto member_node = [&](int k) {
+            for (auto & o : ms)
+                if (k == o.k || (o.n_nodes == 2 && k == o.k + 1)) return true;
+            return false;
+        };
+        int jn = -1;
+        for (int k = i + ms[0].n_nodes; k < std::min(g->n_nodes, i + 24) && jn < 0; ++k)
+            if (!st.done[k] && !is_view_op(g->nodes[k]) && !member_node(k)) jn = k;
+        if (jn >= 0 && g->nodes[jn]->op == GGML_OP_ROPE) {
+            std::vector<int> flagged;  // (the members behind node i are flagged done below; the plan's window walk must already see them that way)
+            for (size_t q = 1; q < ms.size(); ++q)
+                for (int d = 0; d < ms[q].n_nodes; ++d)
+                    if (!st.done[ms[q].k + d]) { st.done[ms[q].k + d] = true; flagged.push_back(ms[q].k + d); }
+            bool ok = plan_rope_store(st, jn, epl);
+            for (int f : flagged) st.done[f] = false;
+            ok = ok && epl.a.p.mode == 0 && (epl.a.head_dim % 2) == 0;
+            int seen = 0;
+            for (size_t q = 0; q < ms.size() && ok; ++q) {
+                int r = -1;
+                for (int sidx = 0; sidx < 3; ++sidx)
+                    if (through_views(epl.src[sidx]) == ms[q].dst) r = sidx;
+                const int64_t arows = ms[q].add ? ms[q].add->ne[1] * ms[q].add->ne[2] * ms[q].add->ne[3] : 0, N = mats[q].N;
+                ok = r >= 0 && !(seen & (1 << r)) && use_count(st, ms[q].dst) == 1 && !(ms[q].dst->flags & GGML_TENSOR_FLAG_OUTPUT) && (!ms[q].add || arows == 1) && (N % 32) == 0 &&
+                     N == (r == 0 ? (int64_t) epl.a.nh : (int64_t) epl.a.nkv) * epl.a.head_dim;
+                if (!ok) break;
+                seen |= 1 << r;
+                epi.kind[q] = r == 0 ? 1 : r == 1 ? (epl.a.k_q8 ? 5 : 2) : epl.a.v_idx ? 4 : epl.a.v_q8 ? 6 : 3;
+                epi.out[q] = r == 0 ? epl.a.q_dst : (r == 1 ? epl.a.k_cache : epl.a.v_cache);
+                epi.nb1[q] = r == 0 ? epl.a.qd_nb1 : (r == 1 ? epl.a.kc_nb1 : epl.a.vc_nb1);
+                epi.nb2[q] = r == 0 ? epl.a.qd_nb2 : 0;
+            }
+            if (ok) epi.tab = ensure_rope_table(st, epl.a.pos, epl.a.ff, epl.a.p, (int) M);
+            if (ok && epi.tab) {
+                epi.idx = epl.a.idx;
+                epi.v_idx = epl.a.v_idx;
+                epi.head_dim = epl.a.head_dim;
+                epi.n_dims = epl.a.p.n_dims;
+                epi_node = jn;
+            }
+        }
+    }
     const void * act = quantized_src1(st, X, MI_ACT_Q80_PANEL);
     for (size_t q = 1; q < ms.size(); ++q)
         for (int d = 0; d < ms[q].n_nodes; ++d) { mark_done(st, ms[q].k + d); c->st.fused_nodes++; }
     {
         timed_scope ts(c, (std::string(M <= 32 ? "mmq_q8_0_skinny" : "mmq_q8_0") + (ms.size() == 3 ? "_x3" : "_x2") + "_n" + std::to_string(n_total) + "_k" + std::to_string(K)).c_str(), wbytes, true);
-        c->st.kernel_launches += launch_mmq_q80_multi(c->stream, (int) ms.size(), mats, (int) K, (int) M, act);
+        c->st.kernel_launches += launch_mmq_q80_multi(c->stream, (int) ms.size(), mats, (int) K, (int) M, act, epi_node >= 0 ? &epi : nullptr);
+    }
+    if (epi_node >= 0) {
+        mark_done(st, epi_node);
+        for (int k : epl.nodes) mark_done(st, k);
+        c->st.fused_nodes += 4;
+        c->st.rope_epilogues++;
     }
     c->st.decode_copy_launches += with_copy != 0;
     c->st.skinny_launches++;

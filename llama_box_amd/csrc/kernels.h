@@ -245,7 +245,7 @@ int mmq_skinny_ksplit(int64_t K, int64_t n_total);
 // 9 columns and up: up to 32 with the weights streamed once, above in tiles of 32 rows x 64 columns, or of 128 x 128 where that is faster; activations in panel order
 bool mmq_q80_batch_supported(int type, int64_t K, int64_t N, int64_t M);
 struct mmq80s_desc { const uint8_t * W; const uint8_t * W_panels; int64_t w_nb1; int N; float * dst; int64_t dst_stride; const float * add; int64_t add_stride; };
-int launch_mmq_q80_multi(hipStream_t s, int n, const mmq80s_desc * mats, int K, int M, const void * act_q80_panel);  // up to three matrices over the same activations; returns the launches it took
+int launch_mmq_q80_multi(hipStream_t s, int n, const mmq80s_desc * mats, int K, int M, const void * act_q80_panel, const mmq_epi * epi = nullptr /* 9 .. 32 columns, three matrices */);  // up to three matrices over the same activations; returns the launches it took
 void launch_mmq_q80(hipStream_t s, const uint8_t * W, const uint8_t * W_panels, int64_t w_nb1, int K, int N, int M, const void * act_q80_panel, float * dst, int64_t dst_stride, const float * add, int64_t add_stride);
 void launch_mmq(hipStream_t s, int type, const uint8_t * W, int64_t w_nb1, int K, int N, int M, const void * act_q8k, float * dst, int64_t dst_stride, int ksplit, float * part);
 

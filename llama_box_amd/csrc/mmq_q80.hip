@@ -51,10 +51,12 @@ typedef uint32_t __attribute__((ext_vector_type(4), aligned(2))) q80s_u32x4_a2;
 typedef uint32_t __attribute__((ext_vector_type(4), aligned(4))) q80s_u32x4_a4;
 
 constexpr int Q80S_WV = 8;
-template <bool WP> __global__ void __launch_bounds__(Q80S_WV * 64, 2) k_mmq_q80_skinny(const mmq80s_args a) {
+// EPI: wq / wk / wv of a batch whose rotation and cache stores follow — done here, as in the K-quants' epilogue (mmq_skinny.hip; the arithmetic of k_rope_qk_store).  16 tokens of TinyLlama: the
+// launch of its own cost 5.8 us a layer.
+template <bool WP, bool EPI> __global__ void __launch_bounds__(Q80S_WV * 64, 2) k_mmq_q80_skinny(const mmq80s_args a, const mmq_epi epi) {
     constexpr bool PF = true;
     __shared__ float dwl[Q80S_WV][4][32];       // a chunk's row scales, per wave
-    __shared__ float red[Q80S_WV][16][64];      // the waves' partial tiles
+    __shared__ float red[Q80S_WV][16][65];      // the waves' partial tiles
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int fr = lane & 31, kg = lane >> 5;
     const int mi = (int) blockIdx.x < a.m[0].panel_end ? 0 : ((int) blockIdx.x < a.m[1].panel_end ? 1 : 2);  // (uniform)
@@ -131,14 +133,38 @@ template <bool WP> __global__ void __launch_bounds__(Q80S_WV * 64, 2) k_mmq_q80_
     for (int r = 0; r < 16; ++r) red[wave][r][lane] = C[r];
     __syncthreads();
     for (int e = tid; e < 16 * 64; e += Q80S_WV * 64) {
-        const int r = e >> 6, l = e & 63;
+        const int m = e >> 5, i = e & 31, r = (i >> 3) * 4 + (i & 3), l = m + 32 * ((i >> 2) & 1), n = n0 + i;  // (32 lanes: the 32 rows of one column)
         float v = red[0][r][l];
 #pragma unroll
         for (int w = 1; w < Q80S_WV; ++w) v += red[w][r][l];
-        const int m = l & 31, n = n0 + 8 * (r >> 2) + 4 * (l >> 5) + (r & 3);
-        if (m < a.M && n < mt.N) {
-            if (mt.add) v += mt.add[(size_t) m * mt.add_stride + n];
-            mt.dst[(size_t) m * mt.dst_stride + n] = v;
+        if (!EPI && (m >= a.M || n >= mt.N)) continue;
+        const int tk = min(m, a.M - 1);
+        if (mt.add) v += mt.add[(size_t) tk * mt.add_stride + n];
+        if constexpr (!EPI) mt.dst[(size_t) m * mt.dst_stride + n] = v;
+        else {
+            const float partner = __shfl_xor(v, 1);  // the other element of the rotation pair
+            const int kind = epi.kind[mi], head = n / epi.head_dim, dd = n - head * epi.head_dim;
+            char * const out = epi.out[mi];
+            float x = v;
+            if ((kind < 3 || kind == 5) && dd < epi.n_dims) {
+                const float2 t = *(const float2 *) (epi.tab + ((size_t) tk * (epi.n_dims >> 1) + (dd >> 1)) * 2);
+                const float x0 = (dd & 1) ? partner : v, x1 = (dd & 1) ? v : partner;
+                x = (dd & 1) ? x0 * t.y + x1 * t.x : x0 * t.x - x1 * t.y;
+            }
+            float amax = fabsf(x);
+            if (kind >= 5) {  // (uniform) the 32 rows are one Q8_0 block of the cache row
+#pragma unroll
+                for (int o = 1; o < 32; o <<= 1) amax = fmaxf(amax, __shfl_xor(amax, o));
+            }
+            if (m >= a.M) continue;
+            if (kind == 1) *(float *) (out + (int64_t) head * epi.nb1[mi] + (int64_t) m * epi.nb2[mi] + (int64_t) dd * 4) = x;
+            else if (kind == 4) ((uint16_t *) out)[epi.v_idx[(int64_t) m * mt.N + n]] = f2h(x);
+            else if (kind >= 5) {
+                const float d8 = amax / 127.0f, id8 = d8 != 0.0f ? 1.0f / d8 : 0.0f;
+                char * const blk = out + epi.idx[m] * epi.nb1[mi] + (n >> 5) * 34;
+                blk[2 + i] = (char) (int) roundf(x * id8);
+                if (i == 0) *(uint16_t *) blk = f2h(d8);
+            } else ((uint16_t *) (out + epi.idx[m] * epi.nb1[mi]))[n] = f2h(x);
         }
     }
 }
@@ -414,7 +440,7 @@ static bool q80_tile_pays(int64_t K, int64_t N, int64_t M, bool panels) {
     return K <= 512 && M <= 512 && N * M >= ((int64_t) 7 << 20);
 }
 // n matrices (1 .. 3) over the same activations; returns the launches; panels[q] != nullptr for ALL of them or for none (the template form is per launch)
-int launch_mmq_q80_multi(hipStream_t s, int n, const mmq80s_desc * mats, int K, int M, const void * act_q80) {
+int launch_mmq_q80_multi(hipStream_t s, int n, const mmq80s_desc * mats, int K, int M, const void * act_q80, const mmq_epi * epi) {
     mmq80s_args a;
     int pe = 0;
     const bool wp = mats[0].W_panels != nullptr;
@@ -427,8 +453,10 @@ int launch_mmq_q80_multi(hipStream_t s, int n, const mmq80s_desc * mats, int K, 
     a.M = M;
     a.act = (const char *) act_q80;
     if (M <= 32) {
-        if (wp) hipLaunchKernelGGL(k_mmq_q80_skinny<true>, dim3((unsigned) pe), dim3(Q80S_WV * 64), 0, s, a);
-        else hipLaunchKernelGGL(k_mmq_q80_skinny<false>, dim3((unsigned) pe), dim3(Q80S_WV * 64), 0, s, a);
+        const mmq_epi none{};
+        const dim3 grid((unsigned) pe), block(Q80S_WV * 64);
+        if (epi) { if (wp) hipLaunchKernelGGL((k_mmq_q80_skinny<true, true>), grid, block, 0, s, a, *epi); else hipLaunchKernelGGL((k_mmq_q80_skinny<false, true>), grid, block, 0, s, a, *epi); }
+        else { if (wp) hipLaunchKernelGGL((k_mmq_q80_skinny<true, false>), grid, block, 0, s, a, none); else hipLaunchKernelGGL((k_mmq_q80_skinny<false, false>), grid, block, 0, s, a, none); }
         return 1;
     }
     int64_t n_total = 0;

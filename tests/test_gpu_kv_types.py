@@ -470,16 +470,16 @@ def test_model_logits_without_flash_attention_and_a_k_cache_in_kv_types(backend,
             o.free()
 
 
-# ROPE(q), ROPE(k) and both cache stores of a batch, rows of Q8_0 blocks (or of one type each): in the projections' epilogue (2 .. 32 tokens, adjacent pairs), in one launch (fewer than 33 tokens;
+# ROPE(q), ROPE(k) and both cache stores of a batch, rows of Q8_0 blocks (or of one type each): in the epilogue of K-quant and Q8_0 projections (2 / 9 .. 32 tokens, adjacent pairs), in one launch (fewer than 33 tokens;
 # split-K sums read there), in its vectorised form (33 and up); heads of 64 and 128 values
-@pytest.mark.parametrize("kt,vt", [(L.Q8_0, L.Q8_0), (L.Q8_0, L.F16), (L.F16, L.Q8_0)])
-@pytest.mark.parametrize("mode,HD,M,project", [(0, 128, 2, True), (0, 128, 9, True), (0, 64, 32, True), (0, 64, 3, False), (L.ROPE_NEOX, 128, 5, False), (L.ROPE_NEOX, 64, 20, True), (0, 128, 33, False),
+@pytest.mark.parametrize("kt,vt", [(L.Q8_0, L.Q8_0), (L.Q8_0, L.F16), (L.F16, L.Q8_0), (L.F16, L.F16)])
+@pytest.mark.parametrize("mode,HD,M,project", [(0, 128, 2, L.Q4_K), (0, 128, 9, L.Q4_K), (0, 64, 32, L.Q4_K), (0, 64, 9, L.Q8_0), (0, 128, 17, L.Q8_0), (0, 64, 32, L.Q8_0), (L.ROPE_NEOX, 64, 12, L.Q8_0), (0, 64, 3, False), (L.ROPE_NEOX, 128, 5, False), (L.ROPE_NEOX, 64, 20, L.Q4_K), (0, 128, 33, False),
                                                (L.ROPE_NEOX, 64, 40, False), (L.ROPE_NEOX, 128, 130, False)])
 def test_batch_rope_and_stores_into_q8_0_rows(backend, H, kt, vt, mode, HD, M, project):
     rng = np.random.default_rng(M + HD + kt + 3 * vt)
     E, NH, NKV, NCTX = 512, 8, 2, 300
     x = rng.standard_normal((M, E)).astype(np.float32)
-    ws = [T.rand_weight(L.Q4_K, E, n * HD, rng) for n in (NH, NKV, NKV)]
+    ws = [T.rand_weight(project or L.Q4_K, E, n * HD, rng) for n in (NH, NKV, NKV)]
     direct = [(rng.standard_normal((M, n * HD)) * rng.uniform(0.0, 3.0, (M, 1))).astype(np.float32) for n in (NH, NKV, NKV)]
     direct[1][0] = 0.0  # (a block of zeros)
     pos, rows = rng.integers(0, 5000, M).astype(np.int32), rng.permutation(NCTX)[:M].astype(np.int64)
@@ -487,7 +487,7 @@ def test_batch_rope_and_stores_into_q8_0_rows(backend, H, kt, vt, mode, HD, M, p
     def build(g):
         cur = g.new(L.F32, [E, M], x)
         if project:
-            q, k, v = (H.ggml_mul_mat(g.ctx, g.new(L.Q4_K, [E, n * HD], w), cur) for n, w in zip((NH, NKV, NKV), ws))
+            q, k, v = (H.ggml_mul_mat(g.ctx, g.new(project, [E, n * HD], w), cur) for n, w in zip((NH, NKV, NKV), ws))
         else:
             q, k, v = (g.new(L.F32, [n * HD, M], d) for n, d in zip((NH, NKV, NKV), direct))
         tp, idx = g.new(L.I32, [M], pos), g.new(L.I64, [M], rows)
@@ -505,5 +505,7 @@ def test_batch_rope_and_stores_into_q8_0_rows(backend, H, kt, vt, mode, HD, M, p
     finally:
         backend.set_option("fusion", 1)
     assert fused >= 3 and launches <= apart - 2, (fused, launches, apart)
+    if project and mode == 0:
+        assert launches == 3, launches  # the input's quantiser, the (cos, sin) table, the projections
     for name, a, b in zip(("q", "k cache", "v cache"), got, plain):
         assert np.array_equal(np.asarray(a).view(np.uint8), np.asarray(b).view(np.uint8)), name
