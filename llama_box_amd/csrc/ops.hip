@@ -1346,36 +1346,74 @@ __device__ __forceinline__ float yarn_ramp(const float low, const float high, co
     const float y = ((float) (i0 / 2) - low) / fmaxf(0.001f, high - low);
     return 1.0f - fminf(1.0f, fmaxf(0.0f, y));
 }
-template <bool F16IO> __global__ void __launch_bounds__(64) k_rope(const tdesc a, const tdesc pos, const float * __restrict__ ff, const tdesc d, const rope_params p,
-                                                               const float theta_scale, const float corr0, const float corr1) {
-    // grid: (head i1, token i2, batch i3); lanes = rotation pairs, so all loads of a launch are independent
-    const int64_t i1 = blockIdx.x, i2 = blockIdx.y, i3 = blockIdx.z;
-    const int n_pairs = p.n_dims / 2;
-    const float pos_f = (float) *(const int32_t *) (pos.data + i2 * pos.nb[0]);
-    const char * __restrict__ src = a.data + i1 * a.nb[1] + i2 * a.nb[2] + i3 * a.nb[3];
-    char * __restrict__ dst = d.data + i1 * d.nb[1] + i2 * d.nb[2] + i3 * d.nb[3];
+// The heads of one token, wave (wv of nw) by wave: a lane owns a rotation pair — its (cos, sin), a power and two accurate functions or a chain of multiplies, is computed once and serves every
+// head the wave takes (two and more at a time where the pairs are fewer than the lanes), four of them in flight.  With a wave per (token, head) the angles were the launch: 512 tokens, 32 heads
+// of 128, 64 of them rotated 13.5 -> 7.8 us.
+// NH: heads a lane has in flight; the first ones are requested ahead of the angle's chain
+template <int NH, class LD, class ST>
+__device__ __forceinline__ void rope_heads(const rope_params & p, const float pos_f, const float * __restrict__ ff, const rope_consts rc, const int D, const int H, const int wv, const int nw, LD ld, ST st) {
+    const int lane = threadIdx.x & 63, n_pairs = p.n_dims / 2;
     const bool neox = (p.mode & GGML_ROPE_TYPE_NEOX) != 0;
-    for (int ip = threadIdx.x; ip < n_pairs; ip += blockDim.x) {
+    const int lp = NH == 1 || n_pairs > 32 ? 64 : n_pairs > 16 ? 32 : n_pairs > 8 ? 16 : 8, per = 64 / lp;  // lanes for a head's pairs, heads at a time
+    for (int ip0 = 0; ip0 < n_pairs; ip0 += lp) {
+        const int ip = ip0 + (lane & (lp - 1));
+        if (ip >= n_pairs) continue;
         const int ia = neox ? ip : 2 * ip, ib = neox ? ip + n_pairs : 2 * ip + 1;
-        float x0, x1;
-        if (F16IO) { x0 = h2f(((const uint16_t *) src)[ia]); x1 = h2f(((const uint16_t *) src)[ib]); }
-        else { x0 = ((const float *) src)[ia]; x1 = ((const float *) src)[ib]; }
+        float x0[NH], x1[NH];
+        auto request = [&](const int h) {
+#pragma unroll
+            for (int k = 0; k < NH; ++k) {
+                const int hk = min(h + k * nw * per, H - 1);
+                x0[k] = ld(hk, ia);
+                x1[k] = ld(hk, ib);
+            }
+        };
+        int h = wv * per + lane / lp;
+        request(h);
         float cs, sn;
         if (p.exact_freq == 2) rope_cos_sin_table(ip, pos_f, ff, p.attn_factor, cs, sn);
         else if (p.exact_freq) rope_cos_sin_exact(ip, pos_f, p.freq_base, p.n_dims, cs, sn);
-        else rope_cos_sin(ip, pos_f, ff, rope_consts{theta_scale, p.freq_scale, p.ext_factor, p.attn_factor, corr0, corr1}, cs, sn);
-        if (F16IO) {
-            ((uint16_t *) dst)[ia] = f2h(x0 * cs - x1 * sn);
-            ((uint16_t *) dst)[ib] = f2h(x0 * sn + x1 * cs);
-        } else {
-            ((float *) dst)[ia] = x0 * cs - x1 * sn;
-            ((float *) dst)[ib] = x0 * sn + x1 * cs;
+        else rope_cos_sin(ip, pos_f, ff, rc, cs, sn);
+        while (h < H) {
+#pragma unroll
+            for (int k = 0; k < NH; ++k)
+                if (h + k * nw * per < H) {
+                    st(h + k * nw * per, ia, x0[k] * cs - x1[k] * sn);
+                    st(h + k * nw * per, ib, x0[k] * sn + x1[k] * cs);
+                }
+            h += NH * nw * per;
+            if (h < H) request(h);
         }
     }
-    for (int64_t i0 = p.n_dims + threadIdx.x; i0 < a.ne[0]; i0 += blockDim.x) {  // pass-through tail beyond n_dims
-        if (F16IO) ((uint16_t *) dst)[i0] = ((const uint16_t *) src)[i0];
-        else ((float *) dst)[i0] = ((const float *) src)[i0];
-    }
+    for (int h = wv; h < H; h += NH * nw)  // pass-through tail beyond n_dims
+        for (int i0 = p.n_dims + lane; i0 < D; i0 += 64) {
+            float x[NH];
+#pragma unroll
+            for (int k = 0; k < NH; ++k) x[k] = ld(min(h + k * nw, H - 1), i0);
+#pragma unroll
+            for (int k = 0; k < NH; ++k)
+                if (h + k * nw < H) st(h + k * nw, i0, x[k]);
+        }
+}
+// waves for a token's heads: one each (workgroups of one) while the tokens are few, four a token when those alone fill the chip
+static bool rope_many(const int64_t tokens) { return tokens >= 128; }
+static unsigned rope_grid(const int64_t heads, const int64_t tokens) { return rope_many(tokens) ? 1u : (unsigned) heads; }
+template <bool F16IO, int NH> __global__ void __launch_bounds__(256) k_rope(const tdesc a, const tdesc pos, const float * __restrict__ ff, const tdesc d, const rope_params p,
+                                                                const float theta_scale, const float corr0, const float corr1) {
+    // grid: (share of the heads, token i2, batch i3)
+    const int64_t i2 = blockIdx.y, i3 = blockIdx.z;
+    const float pos_f = (float) *(const int32_t *) (pos.data + i2 * pos.nb[0]);
+    const char * src = a.data + i2 * a.nb[2] + i3 * a.nb[3];  // (in place, when the allocator made it so)
+    char * dst = d.data + i2 * d.nb[2] + i3 * d.nb[3];
+    rope_heads<NH>(p, pos_f, ff, rope_consts{theta_scale, p.freq_scale, p.ext_factor, p.attn_factor, corr0, corr1}, F16IO ? p.n_dims : (int) a.ne[0], (int) a.ne[1], (int) (blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)),
+               (int) (gridDim.x * (blockDim.x >> 6)), [&](const int h, const int i) { return F16IO ? h2f(((const uint16_t *) (src + h * a.nb[1]))[i]) : ((const float *) (src + h * a.nb[1]))[i]; },
+               [&](const int h, const int i, const float v) {
+                   if (F16IO) ((uint16_t *) (dst + h * d.nb[1]))[i] = f2h(v);
+                   else ((float *) (dst + h * d.nb[1]))[i] = v;
+               });
+    if (F16IO)
+        for (int64_t h = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6); h < a.ne[1]; h += gridDim.x * (blockDim.x >> 6))
+            for (int64_t i0 = p.n_dims + (threadIdx.x & 63); i0 < a.ne[0]; i0 += 64) ((uint16_t *) (dst + h * d.nb[1]))[i0] = ((const uint16_t *) (src + h * a.nb[1]))[i0];
 }
 // ggml_rope_multi (ggml_mrope_cache_init): four position streams, one per section of the rotation pairs; every stream's angle
 // advances by theta_scale per pair, and in vision mode restarts from its position when its section begins.  A lane replays
@@ -1748,8 +1786,13 @@ void launch_rope(hipStream_t s, const tdesc & a, const tdesc & pos, const float 
         else hipLaunchKernelGGL(k_rope_multi<false>, grid, dim3(64), 0, s, a, (const int32_t *) pos.data, ff, d, p, theta_scale, c0, c1);
         return;
     }
-    if (a.type == GGML_TYPE_F16) hipLaunchKernelGGL(k_rope<true>, grid, dim3(64), 0, s, a, pos, ff, d, p, theta_scale, c0, c1);
-    else hipLaunchKernelGGL(k_rope<false>, grid, dim3(64), 0, s, a, pos, ff, d, p, theta_scale, c0, c1);
+    grid.x = rope_grid(a.ne[1], a.ne[2] * a.ne[3]);
+    const bool many = rope_many(a.ne[2] * a.ne[3]);
+    if (a.type == GGML_TYPE_F16) {
+        if (many) hipLaunchKernelGGL((k_rope<true, 4>), grid, dim3(256), 0, s, a, pos, ff, d, p, theta_scale, c0, c1);
+        else hipLaunchKernelGGL((k_rope<true, 1>), grid, dim3(64), 0, s, a, pos, ff, d, p, theta_scale, c0, c1);
+    } else if (many) hipLaunchKernelGGL((k_rope<false, 4>), grid, dim3(256), 0, s, a, pos, ff, d, p, theta_scale, c0, c1);
+    else hipLaunchKernelGGL((k_rope<false, 1>), grid, dim3(64), 0, s, a, pos, ff, d, p, theta_scale, c0, c1);
 }
 
 // ROPE whose only reader is the SET_ROWS of a cache: the rotated head goes straight into its cache row (k_rope's arithmetic, then ONE rounding to the
@@ -1760,32 +1803,23 @@ __device__ __forceinline__ void store_as(char * __restrict__ row, const int type
     else if (type == GGML_TYPE_BF16) ((uint16_t *) row)[i] = f2bf(v);
     else ((uint16_t *) row)[i] = f2h(v);
 }
-__global__ void __launch_bounds__(64) k_rope_store(const tdesc a, const tdesc pos, const float * __restrict__ ff, const int64_t * __restrict__ idx, char * __restrict__ cache, const int64_t cache_nb1, const int cache_type,
-                                                   const rope_params p, const float theta_scale, const float corr0, const float corr1) {
-    const int64_t i1 = blockIdx.x, i2 = blockIdx.y;
-    const int n_pairs = p.n_dims / 2;
+template <int NH> __global__ void __launch_bounds__(256) k_rope_store(const tdesc a, const tdesc pos, const float * __restrict__ ff, const int64_t * __restrict__ idx, char * __restrict__ cache, const int64_t cache_nb1, const int cache_type,
+                                                    const rope_params p, const float theta_scale, const float corr0, const float corr1) {
+    const int64_t i2 = blockIdx.y;
     const float pos_f = (float) *(const int32_t *) (pos.data + i2 * pos.nb[0]);
-    const float * __restrict__ src = (const float *) (a.data + i1 * a.nb[1] + i2 * a.nb[2]);
-    char * __restrict__ row = cache + idx[i2] * cache_nb1;
-    const int64_t base = i1 * a.ne[0];
-    const bool neox = (p.mode & GGML_ROPE_TYPE_NEOX) != 0;
-    for (int ip = threadIdx.x; ip < n_pairs; ip += blockDim.x) {
-        const int ia = neox ? ip : 2 * ip, ib = neox ? ip + n_pairs : 2 * ip + 1;
-        const float x0 = src[ia], x1 = src[ib];
-        float cs, sn;
-        if (p.exact_freq == 2) rope_cos_sin_table(ip, pos_f, ff, p.attn_factor, cs, sn);
-        else if (p.exact_freq) rope_cos_sin_exact(ip, pos_f, p.freq_base, p.n_dims, cs, sn);
-        else rope_cos_sin(ip, pos_f, nullptr, rope_consts{theta_scale, p.freq_scale, p.ext_factor, p.attn_factor, corr0, corr1}, cs, sn);
-        store_as(row, cache_type, base + ia, x0 * cs - x1 * sn);
-        store_as(row, cache_type, base + ib, x0 * sn + x1 * cs);
-    }
-    for (int64_t i0 = p.n_dims + threadIdx.x; i0 < a.ne[0]; i0 += blockDim.x) store_as(row, cache_type, base + i0, src[i0]);
+    const char * src = a.data + i2 * a.nb[2];
+    char * row = cache + idx[i2] * cache_nb1;
+    rope_heads<NH>(p, pos_f, p.exact_freq == 2 ? ff : nullptr, rope_consts{theta_scale, p.freq_scale, p.ext_factor, p.attn_factor, corr0, corr1}, (int) a.ne[0], (int) a.ne[1], (int) (blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)),
+               (int) (gridDim.x * (blockDim.x >> 6)), [&](const int h, const int i) { return ((const float *) (src + h * a.nb[1]))[i]; },
+               [&](const int h, const int i, const float v) { store_as(row, cache_type, h * a.ne[0] + i, v); });
 }
 void launch_rope_store(hipStream_t s, const tdesc & a, const tdesc & pos, const float * ff, const int64_t * idx, const tdesc & cache, const rope_params & p) {
     if (a.ne[1] * a.ne[2] == 0) return;
     float theta_scale, c0, c1;
     rope_host_consts(p, theta_scale, c0, c1);
-    hipLaunchKernelGGL(k_rope_store, dim3((unsigned) a.ne[1], (unsigned) a.ne[2]), dim3(64), 0, s, a, pos, ff, idx, cache.data, cache.nb[1], cache.type, p, theta_scale, c0, c1);
+    const dim3 grid(rope_grid(a.ne[1], a.ne[2]), (unsigned) a.ne[2]);
+    if (rope_many(a.ne[2])) hipLaunchKernelGGL(k_rope_store<4>, grid, dim3(256), 0, s, a, pos, ff, idx, cache.data, cache.nb[1], cache.type, p, theta_scale, c0, c1);
+    else hipLaunchKernelGGL(k_rope_store<1>, grid, dim3(64), 0, s, a, pos, ff, idx, cache.data, cache.nb[1], cache.type, p, theta_scale, c0, c1);
 }
 // ------------------------------------------------------------------------------------------------ fused steps of models with token shift / latent attention
 // (each one the arithmetic of the unfused nodes it replaces, operation by operation: fused and unfused graphs agree bit for bit)

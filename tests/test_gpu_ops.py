@@ -1562,3 +1562,24 @@ def test_fused_chains_equal_unfused(backend, H, plog, qt, M):
     T.compare(f"ffn chain fused {QNAME[qt]} M={M}", fused[0], ref[0], max_nmse=2e-6, log=plog)
     T.compare(f"ffn chain unfused {QNAME[qt]} M={M}", plain[0], ref[0], max_nmse=2e-6, log=plog)
     T.compare(f"ffn chain fused-vs-unfused {QNAME[qt]} M={M}", fused[0], plain[0], max_nmse=1e-12, log=plog)
+
+
+# 128 tokens and more take another launch shape (a token's heads share their angles): the bits of fewer tokens, for pairs that fill part of a wave, heads that are no whole wave's or group's, a tail
+# behind the rotated part, and one batch of several
+@pytest.mark.parametrize("mode", [0, L.ROPE_NEOX])
+@pytest.mark.parametrize("D,n_dims,heads,T_,batches,t16", [(64, 64, 1, 128, 1, False), (128, 64, 5, 130, 1, False), (128, 128, 33, 129, 1, False), (96, 20, 18, 140, 1, False), (40, 12, 7, 131, 1, True), (160, 160, 9, 64, 2, True)])
+def test_rope_of_many_tokens_has_the_bits_of_few(backend, H, mode, D, n_dims, heads, T_, batches, t16):
+    rng = np.random.default_rng(D + heads)
+    x = rng.standard_normal((batches, T_, heads, D)).astype(np.float16 if t16 else np.float32)
+    pos = rng.integers(0, 3000, T_).astype(np.int32)
+
+    def run(b0, b1, lo, hi):
+        def f(g):
+            t = g.new(L.F16 if t16 else L.F32, [D, heads, hi - lo, b1 - b0], np.ascontiguousarray(x[b0:b1, lo:hi]))
+            return H.ggml_rope_ext(g.ctx, t, g.new(L.I32, [hi - lo], pos[lo:hi]), None, n_dims, mode, 4096, 10000.0, 1.0, 0.0, 1.0, 32.0, 1.0)
+        return np.asarray(T.run_case(f, backend)[0]).reshape(b1 - b0, hi - lo, heads, D)
+
+    whole = run(0, batches, 0, T_)
+    for b in range(batches):
+        for lo, hi in ((0, 60), (60, T_)):
+            assert np.array_equal(whole[b : b + 1, lo:hi], run(b, b + 1, lo, hi)), (b, lo)
