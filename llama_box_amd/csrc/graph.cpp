@@ -466,6 +466,7 @@ struct exec_state {
     std::vector<char> done;  // nodes already executed out of order by a multi-chain fusion
     std::vector<int> ooo;    // ... those flagged during the current run_node call (quantised-activation cache invalidation)
     bool q8_fresh = false;   // the node just executed produced the quantised-activation cache for its own output
+    bool a16_fresh = false;  // ... and the 16-bit one
     // tile lists (fattn.hip) valid for this mask tensor / tile size during this execution of the graph
     const void * fa_list_mask = nullptr;
     int fa_list_tile = 0;
@@ -592,6 +593,28 @@ static const void * rounded_src1(exec_state & st, const ggml_tensor * b, int wty
     }
     c->act16.set(b, kind);
     return dst;
+}
+
+// The producer of `t` (its last node: `at`) may leave that copy itself when the next product of the form reads t, as it is or reshaped; else {}.  The f32 rows are written as before.
+// What it saves is the launch that reads them back (us, producer and launch -> producer alone): 512 rows, norm of 4096 values 7.3 + 5.3 -> 8.1, gate 5.7 + 5.3 -> 7.0, GELU of 14336 12.9 + 7.1 -> 15.1.
+// (`b`, the product's operand, is what the scratch holds from then on: the producer calls left_16 when its kernel has written it.)
+static copy16 copy_16_for(exec_state & st, int at, const ggml_tensor * t, const ggml_tensor ** b) {
+    const int limit = std::min(st.g->n_nodes, at + 28);
+    if (!is_f32_contig(t)) return {};
+    for (int k = at + 1; k < limit; ++k) {
+        const ggml_tensor * n = st.g->nodes[k];
+        if (st.done[k] || (n->op != GGML_OP_MUL_MAT && n->op != GGML_OP_MUL_MAT_ID)) continue;
+        if (n->op == GGML_OP_MUL_MAT_ID ? !mm_id_tile_applies(n) : !mm_tile_applies(n)) continue;
+        const ggml_tensor * x = n->src[1];  // (the first product that reads the scratch decides)
+        if (n->op != GGML_OP_MUL_MAT || x->data != t->data || !is_f32_contig(x) || ggml_abi_nelements(x) != ggml_abi_nelements(t)) return {};
+        *b = x;
+        return {(char *) st.c->ws + st.act16_off, n->src[0]->type};
+    }
+    return {};
+}
+static void left_16(exec_state & st, const ggml_tensor * b, const copy16 & o) {
+    st.c->act16.set(b, MI_ACT_16 + o.type);
+    st.a16_fresh = true;
 }
 
 static const char * type_tag(int t) {
@@ -3033,7 +3056,9 @@ static int run_node(exec_state & st, int i) {
             if (fuse && n->op_params[0] == GGML_UNARY_OP_SIGMOID && gm && gm->op == GGML_OP_MUL && (gm->src[0] == n || gm->src[1] == n) && gm->src[0] != gm->src[1] && single_use(st, n)) {
                 const ggml_tensor * x = gm->src[0] == n ? gm->src[1] : gm->src[0];
                 if (is_f32_contig(x) && is_f32_contig(gm) && same_shape(x, n) && same_shape(gm, n)) {
-                    launch_mul_sigmoid(s, (const float *) x->data, (const float *) a->data, (float *) gm->data, ggml_abi_nelements(gm));
+                    const ggml_tensor * b16 = nullptr;
+                    const copy16 o16 = copy_16_for(st, i + 1, gm, &b16);
+                    if (launch_mul_sigmoid(s, (const float *) x->data, (const float *) a->data, (float *) gm->data, ggml_abi_nelements(gm), o16)) left_16(st, b16, o16);
                     c->st.kernel_launches++;
                     c->st.fused_nodes++;
                     return 2;
@@ -3042,12 +3067,16 @@ static int run_node(exec_state & st, int i) {
             // RELU -> SQR (the squared-ReLU activation): one pass writing the SQR's output
             ggml_tensor * sq = next(1);
             if (fuse && n->op_params[0] == GGML_UNARY_OP_RELU && sq && sq->op == GGML_OP_SQR && sq->src[0] == n && single_use(st, n) && is_f32_contig(sq) && same_shape(sq, n)) {
-                launch_unary(s, MI_UNARY_RELU_SQR, TD(a), TD(sq));
+                const ggml_tensor * b16 = nullptr;
+                const copy16 o16 = copy_16_for(st, i + 1, sq, &b16);
+                if (launch_unary(s, MI_UNARY_RELU_SQR, TD(a), TD(sq), o16)) left_16(st, b16, o16);
                 c->st.kernel_launches++;
                 c->st.fused_nodes++;
                 return 2;
             }
-            launch_unary(s, n->op_params[0], TD(a), TD(n));
+            const ggml_tensor * b16 = nullptr;
+            const copy16 o16 = fuse ? copy_16_for(st, i, n, &b16) : copy16{};
+            if (launch_unary(s, n->op_params[0], TD(a), TD(n), o16)) left_16(st, b16, o16);
             c->st.kernel_launches++;
             return 1;
         }
@@ -3187,20 +3216,27 @@ static int run_node(exec_state & st, int i) {
                             if (w2 && w2->type == GGML_TYPE_F32 && ggml_abi_is_contiguous(w2) && w2->ne[0] == n->ne[0] && ggml_abi_nelements(w2) == w2->ne[0] && !ranges_overlap(m2, ad) &&
                                 !(ranges_overlap(m2, a) && m2->data != a->data) && !ranges_overlap(m2, res)) {  // (a row's second output is written after the last read of that row of `a`: the allocator may hand `a`'s block to it)
                                 timed_scope ts(c, "layer_norm_mul_add_norm_mul", (double) ggml_abi_nbytes(a) * 4);
-                                launch_layer_norm_twice(s, TD(a), TD(ad), ggml_abi_op_param_f32(n, 0), (const float *) w->data, &rd, (const float *) w2->data, ggml_abi_op_param_f32(n2, 0), TD(m2));
+                                const ggml_tensor * b16 = nullptr;
+                                const copy16 o16 = copy_16_for(st, i + 4, m2, &b16);
+                                if (launch_layer_norm_twice(s, TD(a), TD(ad), ggml_abi_op_param_f32(n, 0), (const float *) w->data, &rd, (const float *) w2->data, ggml_abi_op_param_f32(n2, 0), TD(m2), o16))
+                                    left_16(st, b16, o16);
                                 c->st.kernel_launches++;
                                 c->st.fused_nodes += 4;
                                 return 5;
                             }
                         }
                         timed_scope ts(c, "layer_norm_mul_add", (double) ggml_abi_nbytes(a) * 3);
-                        launch_layer_norm(s, TD(a), TD(ad), ggml_abi_op_param_f32(n, 0), (const float *) w->data, &rd);
+                        const ggml_tensor * b16 = nullptr;
+                        const copy16 o16 = copy_16_for(st, i + 2, ad, &b16);
+                        if (launch_layer_norm(s, TD(a), TD(ad), ggml_abi_op_param_f32(n, 0), (const float *) w->data, &rd, o16)) left_16(st, b16, o16);
                         c->st.kernel_launches++;
                         c->st.fused_nodes += 2;
                         return 3;
                     }
                     timed_scope ts(c, "layer_norm_mul", (double) ggml_abi_nbytes(a) * 2);
-                    launch_layer_norm(s, TD(a), TD(m), ggml_abi_op_param_f32(n, 0), (const float *) w->data, nullptr);
+                    const ggml_tensor * b16 = nullptr;
+                    const copy16 o16 = copy_16_for(st, i + 1, m, &b16);
+                    if (launch_layer_norm(s, TD(a), TD(m), ggml_abi_op_param_f32(n, 0), (const float *) w->data, nullptr, o16)) left_16(st, b16, o16);
                     c->st.kernel_launches++;
                     c->st.fused_nodes++;
                     return 2;
@@ -3681,8 +3717,8 @@ static bool run_nodes(backend_ctx * c, ggml_cgraph * g, const ws_plan & wp) {
             return false;
         };
         if (!st.q8_fresh && c->act.src && written(c->act)) c->act.src = nullptr;
-        if (c->act16.src && written(c->act16)) c->act16.src = nullptr;
-        st.q8_fresh = false;
+        if (!st.a16_fresh && c->act16.src && written(c->act16)) c->act16.src = nullptr;
+        st.q8_fresh = st.a16_fresh = false;
         i += used;
     }
     return hipGetLastError() == hipSuccess;

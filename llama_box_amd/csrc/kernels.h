@@ -168,6 +168,11 @@ struct mul_mat_tile_desc { const void * W; int64_t nb1; int64_t N; void * dst; i
 bool mul_mat_tile_ok(int type, int64_t K, int64_t N, int64_t nb0, int64_t nb1, const void * W);
 bool mul_mat_tile_pays(int64_t K, int64_t N, int64_t M);  // ... faster than launch_mul_mat_f for one matrix of N rows, M > 16 columns
 void launch_to_16(hipStream_t s, int type, const char * x, int64_t nb1, int64_t K, int64_t rows, void * out);
+// where a producer leaves that copy of its (dense, f32) output itself: type F16 / BF16; out == nullptr: nowhere
+struct copy16 {
+    void * out = nullptr;
+    int type = 0;
+};
 // the experts' columns (lists: k_moe_group); x16 rows: src1's [n_b, T]
 void launch_mul_mat_id_tile(hipStream_t s, const tdesc & as, int64_t n_b, int64_t n_used, int64_t T, const tdesc & d, const int32_t * cnt, const int32_t * off, const int32_t * list, const void * x16);
 bool mul_mat_id_tile_pays(int64_t K, int64_t N, int64_t even);  // ... faster than mmf.hip's form for `even` columns an expert?
@@ -255,19 +260,19 @@ void launch_mul_act(hipStream_t s, const float * x, const float * g, float * d, 
 void launch_add3(hipStream_t s, const float * x, const float * a, const float * b, float * d, int64_t n); // d = x + (a + b)
 void launch_gate_norm(hipStream_t s, const float * y, const float * z, const float * w, float * d, int64_t D, int64_t parts, int64_t rows, float eps);
 void launch_rms_norm2_blend(hipStream_t s, const float * l, const float * r, const float * wl, const float * wr, float a, float b, float * d, int64_t n, int64_t rows, float eps);
-void launch_layer_norm(hipStream_t s, const tdesc & src, const tdesc & dst, float eps, const float * mul_w /* optional fused weight */, const tdesc * residual /* optional fused ADD */);
-void launch_layer_norm_twice(hipStream_t s, const tdesc & src, const tdesc & dst, float eps, const float * mul_w, const tdesc * residual, const float * w2, float eps2, const tdesc & dst2);  // ... and dst2 = LN(dst) * w2
+bool launch_layer_norm(hipStream_t s, const tdesc & src, const tdesc & dst, float eps, const float * mul_w /* optional fused weight */, const tdesc * residual /* optional fused ADD */, const copy16 & o16 = {});  // (true, here and below: o16 was written)
+bool launch_layer_norm_twice(hipStream_t s, const tdesc & src, const tdesc & dst, float eps, const float * mul_w, const tdesc * residual, const float * w2, float eps2, const tdesc & dst2, const copy16 & o16 = {});  // ... and dst2 = LN(dst) * w2
 void launch_topk_softmax(hipStream_t s, const tdesc & logits /* [n, T] */, const tdesc & ids /* [n, T] i32: the descending permutation */, const tdesc & wts /* [k, T] */, int k);  // k <= 256
 void launch_argsort(hipStream_t s, const tdesc & src, const tdesc & dst, int descending);  // rows of f32 -> i32 permutation (stable)
 // element-wise forms outside ggml's unary enumeration, served by launch_unary: x^2 (SQR) and relu(x)^2 (RELU followed by SQR)
 #define MI_UNARY_SQR 1000
 #define MI_UNARY_RELU_SQR 1001
 void launch_axpby(hipStream_t s, const float * x, float a, const float * y, float b, float * d, int64_t n);  // d = a x + b y (each product rounded, then the sum: SCALE, SCALE, ADD)
-void launch_mul_sigmoid(hipStream_t s, const float * x, const float * g, float * d, int64_t n);          // d = x * sigmoid(g)
+bool launch_mul_sigmoid(hipStream_t s, const float * x, const float * g, float * d, int64_t n, const copy16 & o16 = {});          // d = x * sigmoid(g)
 void launch_weighted_rows_sum(hipStream_t s, const tdesc & rows /* [n, n_used, T] */, const tdesc & w /* [1, n_used, T] */, const tdesc & d /* [n, T] */);
 void launch_binary(hipStream_t s, int op, const tdesc & a, const tdesc & b, const tdesc & dst);
 void launch_scale(hipStream_t s, const tdesc & src, const tdesc & dst, float scale, float bias);
-void launch_unary(hipStream_t s, int uop, const tdesc & src, const tdesc & dst);
+bool launch_unary(hipStream_t s, int uop, const tdesc & src, const tdesc & dst, const copy16 & o16 = {});
 void launch_swiglu(hipStream_t s, const tdesc & a, const tdesc * b, const tdesc & dst, int swapped);
 // producers fused with the Q8_K activation quantisation (quantize.hip): the f32 intermediate is not written
 // the same with the row ASSEMBLED first from split-K partials (+ epilogue add) — and written out as f32, for its other readers

@@ -137,6 +137,17 @@ void launch_rms_norm_mul_q80_panel(hipStream_t s, const tdesc & src, float eps, 
 }
 
 // ------------------------------------------------------------------------------------------------ NORM (layer normalisation)
+// four values in a 16-bit type, nearest even (k_to_16's conversions)
+__device__ __forceinline__ uint2 round4_16(const float4 v, const int type) {
+    typedef __bf16 bf4 __attribute__((ext_vector_type(4)));
+    typedef _Float16 half4 __attribute__((ext_vector_type(4)));
+    if (type == GGML_TYPE_BF16) {
+        const bf4 h = {(__bf16) v.x, (__bf16) v.y, (__bf16) v.z, (__bf16) v.w};
+        return __builtin_bit_cast(uint2, h);
+    }
+    const half4 h = {(_Float16) v.x, (_Float16) v.y, (_Float16) v.z, (_Float16) v.w};
+    return __builtin_bit_cast(uint2, h);
+}
 // y = (x - mean) / sqrt(var + eps) [* w] [+ r], var = mean of the squared deviations (two passes over a row kept in registers / L2; sums in f64
 // like RMS_NORM's).  w: optional weight of the MUL that follows; r: optional residual rows of the ADD behind that (same shape as the output).
 // second stage (w2 != nullptr): the row just written is normalised once more into d2, y2 = LN(y) * w2 — the norm in front of the next sublayer, which reads
@@ -145,9 +156,10 @@ void launch_rms_norm_mul_q80_panel(hipStream_t s, const tdesc & src, float eps, 
 // weights are ALL requested before anything waits, so a row costs one round trip to memory and the barriers of its sums.  With the weights and the residual loaded behind
 // the sums, value by value under the bounds check, each of the sixteen values of a thread waited for its own two loads.  MI355X, us a launch, before / now: 2 rows of 2048
 // with both stages 12.2 / 4.2, 512 rows of 4096 13.8 / 7.2.  Any other row: k_layer_norm.
+// o16: a second, dense copy of the last stage's rows in the type of the 16-bit matrices that multiply them next (k_to_16's rounding)
 template <int R>
 __global__ void __launch_bounds__(256) k_layer_norm_held(const tdesc a, const tdesc d, const float eps, const float * __restrict__ w, const tdesc r, const int has_r,
-                                                         const float * __restrict__ w2, const float eps2, const tdesc d2) {
+                                                         const float * __restrict__ w2, const float eps2, const tdesc d2, const copy16 o16) {
     __shared__ double sh[4][4];
     const int64_t row = blockIdx.x;
     const int64_t i1 = row % a.ne[1], i2 = (row / a.ne[1]) % a.ne[2], i3 = row / (a.ne[1] * a.ne[2]);
@@ -196,7 +208,15 @@ __global__ void __launch_bounds__(256) k_layer_norm_held(const tdesc a, const td
         if (live(u)) y[threadIdx.x + 256 * u] = v;
         xv[u] = v;
     }
-    if (w2 == nullptr) return;
+    uint2 * const y16 = (uint2 *) o16.out + row * n4;
+    if (w2 == nullptr) {
+        if (o16.out) {
+#pragma unroll
+            for (int u = 0; u < R; ++u)
+                if (live(u)) y16[threadIdx.x + 256 * u] = round4_16(xv[u], o16.type);
+        }
+        return;
+    }
     norm(eps2, 1, mean, scale);
     float4 * const y2 = (float4 *) (d2.data + i1 * d2.nb[1] + i2 * d2.nb[2] + i3 * d2.nb[3]);
 #pragma unroll
@@ -204,6 +224,7 @@ __global__ void __launch_bounds__(256) k_layer_norm_held(const tdesc a, const td
         float4 v;
         v.x = (xv[u].x - mean) * scale * w2v[u].x; v.y = (xv[u].y - mean) * scale * w2v[u].y; v.z = (xv[u].z - mean) * scale * w2v[u].z; v.w = (xv[u].w - mean) * scale * w2v[u].w;
         if (live(u)) y2[threadIdx.x + 256 * u] = v;
+        if (o16.out && live(u)) y16[threadIdx.x + 256 * u] = round4_16(v, o16.type);
     }
 }
 // y = (x - mean) / sqrt(var + eps) per row for rows that are longer, odd or not aligned: the row is read again in every pass
@@ -252,23 +273,26 @@ __global__ void __launch_bounds__(256) k_layer_norm(const tdesc a, const tdesc d
     float * y2 = (float *) (d2.data + i1 * d2.nb[1] + i2 * d2.nb[2] + i3 * d2.nb[3]);
     for (int64_t i = threadIdx.x; i < n; i += blockDim.x) y2[i] = (y[i] - mean2) * scale2 * w2[i];
 }
-static void launch_layer_norm_rows(hipStream_t s, const tdesc & src, const tdesc & dst, const float eps, const float * mul_w, const tdesc * residual, const float * w2, const float eps2, const tdesc & dst2) {
+static bool launch_layer_norm_rows(hipStream_t s, const tdesc & src, const tdesc & dst, const float eps, const float * mul_w, const tdesc * residual, const float * w2, const float eps2, const tdesc & dst2,
+                                   const copy16 & o16) {
     const int64_t rows = src.ne[1] * src.ne[2] * src.ne[3], n = src.ne[0];
-    if (rows == 0) return;
+    if (rows == 0) return false;
     const tdesc r = residual ? *residual : src;
     auto al = [](const tdesc & t) { return (((uintptr_t) t.data | (uintptr_t) t.nb[1] | (uintptr_t) t.nb[2] | (uintptr_t) t.nb[3]) & 15) == 0; };
     const bool held = n > 0 && n <= 4096 && (n & 3) == 0 && al(src) && al(dst) && al(r) && al(dst2) && (((uintptr_t) mul_w | (uintptr_t) w2) & 15) == 0;
     const dim3 g((unsigned) rows), b(256);
     if (!held) hipLaunchKernelGGL(k_layer_norm, g, b, 0, s, src, dst, eps, mul_w, r, residual ? 1 : 0, w2, eps2, dst2);
-    else if (n <= 1024) hipLaunchKernelGGL(k_layer_norm_held<1>, g, b, 0, s, src, dst, eps, mul_w, r, residual ? 1 : 0, w2, eps2, dst2);
-    else if (n <= 2048) hipLaunchKernelGGL(k_layer_norm_held<2>, g, b, 0, s, src, dst, eps, mul_w, r, residual ? 1 : 0, w2, eps2, dst2);
-    else hipLaunchKernelGGL(k_layer_norm_held<4>, g, b, 0, s, src, dst, eps, mul_w, r, residual ? 1 : 0, w2, eps2, dst2);
+    else if (n <= 1024) hipLaunchKernelGGL(k_layer_norm_held<1>, g, b, 0, s, src, dst, eps, mul_w, r, residual ? 1 : 0, w2, eps2, dst2, o16);
+    else if (n <= 2048) hipLaunchKernelGGL(k_layer_norm_held<2>, g, b, 0, s, src, dst, eps, mul_w, r, residual ? 1 : 0, w2, eps2, dst2, o16);
+    else hipLaunchKernelGGL(k_layer_norm_held<4>, g, b, 0, s, src, dst, eps, mul_w, r, residual ? 1 : 0, w2, eps2, dst2, o16);
+    return held && o16.out;
 }
-void launch_layer_norm(hipStream_t s, const tdesc & src, const tdesc & dst, float eps, const float * mul_w, const tdesc * residual) {
-    launch_layer_norm_rows(s, src, dst, eps, mul_w, residual, nullptr, 0.0f, dst);
+bool launch_layer_norm(hipStream_t s, const tdesc & src, const tdesc & dst, float eps, const float * mul_w, const tdesc * residual, const copy16 & o16) {
+    return launch_layer_norm_rows(s, src, dst, eps, mul_w, residual, nullptr, 0.0f, dst, o16);
 }
-void launch_layer_norm_twice(hipStream_t s, const tdesc & src, const tdesc & dst, float eps, const float * mul_w, const tdesc * residual, const float * w2, float eps2, const tdesc & dst2) {
-    launch_layer_norm_rows(s, src, dst, eps, mul_w, residual, w2, eps2, dst2);
+bool launch_layer_norm_twice(hipStream_t s, const tdesc & src, const tdesc & dst, float eps, const float * mul_w, const tdesc * residual, const float * w2, float eps2, const tdesc & dst2,
+                             const copy16 & o16) {
+    return launch_layer_norm_rows(s, src, dst, eps, mul_w, residual, w2, eps2, dst2, o16);
 }
 
 // ------------------------------------------------------------------------------------------------ router: top-k and soft-max over the chosen logits
@@ -684,9 +708,24 @@ __global__ void __launch_bounds__(256) k_mul_sigmoid(const float * __restrict__ 
         d[i] = x[i] * sg;
     }
 }
-void launch_mul_sigmoid(hipStream_t s, const float * x, const float * g, float * d, int64_t n) {
-    if (n == 0) return;
+// ... four values a thread, with the copy in the type of the 16-bit matrices that multiply d next (n % 4 == 0, pointers 16-byte aligned)
+__global__ void __launch_bounds__(256) k_mul_sigmoid_16(const float4 * x, const float4 * g, float4 * d, const int64_t n4, const copy16 o16) {
+    const int64_t i = (int64_t) blockIdx.x * 256 + threadIdx.x;
+    if (i >= n4) return;
+    const float4 a = x[i], b = g[i];
+    const float sx = 1.f / (1.f + expf(-b.x)), sy = 1.f / (1.f + expf(-b.y)), sz = 1.f / (1.f + expf(-b.z)), sw = 1.f / (1.f + expf(-b.w));
+    const float4 r = make_float4(a.x * sx, a.y * sy, a.z * sz, a.w * sw);
+    d[i] = r;
+    ((uint2 *) o16.out)[i] = round4_16(r, o16.type);
+}
+bool launch_mul_sigmoid(hipStream_t s, const float * x, const float * g, float * d, int64_t n, const copy16 & o16) {
+    if (n == 0) return false;
+    if (o16.out && (n & 3) == 0 && !(((uintptr_t) x | (uintptr_t) g | (uintptr_t) d) & 15)) {
+        hipLaunchKernelGGL(k_mul_sigmoid_16, dim3((unsigned) ((n / 4 + 255) / 256)), dim3(256), 0, s, (const float4 *) x, (const float4 *) g, (float4 *) d, n / 4, o16);
+        return true;
+    }
     hipLaunchKernelGGL(k_mul_sigmoid, dim3((unsigned) std::min<int64_t>((n + 255) / 256, 2048)), dim3(256), 0, s, x, g, d, n);
+    return false;
 }
 // x * act(g) with act = the tanh form of GELU or SiLU (UNARY -> MUL; k_unary's formulas), and x + (a + b) (two ADDs)
 __global__ void __launch_bounds__(256) k_mul_act(const float * __restrict__ x, const float * __restrict__ g, float * __restrict__ d, const int64_t n, const int uop) {
@@ -991,29 +1030,41 @@ void launch_scale(hipStream_t s, const tdesc & src, const tdesc & dst, float sca
     hipLaunchKernelGGL(k_scale, dim3(grid), dim3(256), 0, s, (const float *) src.data, (float *) dst.data, n, scale, bias);
 }
 
-__global__ void __launch_bounds__(256) k_unary(const int uop, const float * __restrict__ x, float * __restrict__ y, const int64_t n) {
-    for (int64_t i = (int64_t) blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t) gridDim.x * blockDim.x) {
-        const float v = x[i];
-        float r;
-        switch (uop) {
-            case GGML_UNARY_OP_SILU: r = silu_f(v); break;
-            case GGML_UNARY_OP_RELU: r = v > 0.f ? v : 0.f; break;
-            case GGML_UNARY_OP_NEG: r = -v; break;
-            case GGML_UNARY_OP_EXP: r = expf(v); break;
-            case GGML_UNARY_OP_TANH: r = tanhf(v); break;
-            case GGML_UNARY_OP_GELU_ERF: r = 0.5f * v * (1.0f + erff(v * 0.70710678118654752440f)); break;
-            case GGML_UNARY_OP_GELU: r = 0.5f * v * (1.0f + tanhf(0.79788456080286535588f * (v + 0.044715f * v * v * v))); break;
-            case MI_UNARY_SQR: r = v * v; break;
-            case MI_UNARY_RELU_SQR: r = v > 0.f ? v * v : 0.f; break;
-            default: r = 1.f / (1.f + expf(-v)); break;  // SIGMOID
-        }
-        y[i] = r;
+__device__ __forceinline__ float unary_f(const int uop, const float v) {
+    switch (uop) {
+        case GGML_UNARY_OP_SILU: return silu_f(v);
+        case GGML_UNARY_OP_RELU: return v > 0.f ? v : 0.f;
+        case GGML_UNARY_OP_NEG: return -v;
+        case GGML_UNARY_OP_EXP: return expf(v);
+        case GGML_UNARY_OP_TANH: return tanhf(v);
+        case GGML_UNARY_OP_GELU_ERF: return 0.5f * v * (1.0f + erff(v * 0.70710678118654752440f));
+        case GGML_UNARY_OP_GELU: return 0.5f * v * (1.0f + tanhf(0.79788456080286535588f * (v + 0.044715f * v * v * v)));
+        case MI_UNARY_SQR: return v * v;
+        case MI_UNARY_RELU_SQR: return v > 0.f ? v * v : 0.f;
+        default: return 1.f / (1.f + expf(-v));  // SIGMOID
     }
 }
-void launch_unary(hipStream_t s, int uop, const tdesc & src, const tdesc & dst) {
+__global__ void __launch_bounds__(256) k_unary(const int uop, const float * __restrict__ x, float * __restrict__ y, const int64_t n) {
+    for (int64_t i = (int64_t) blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t) gridDim.x * blockDim.x) y[i] = unary_f(uop, x[i]);
+}
+// ... four values a thread, with the copy in the type of the 16-bit matrices that multiply y next (n % 4 == 0, pointers 16-byte aligned)
+__global__ void __launch_bounds__(256) k_unary_16(const int uop, const float4 * x, float4 * y, const int64_t n4, const copy16 o16) {
+    const int64_t i = (int64_t) blockIdx.x * 256 + threadIdx.x;
+    if (i >= n4) return;
+    const float4 v = x[i];
+    const float4 r = make_float4(unary_f(uop, v.x), unary_f(uop, v.y), unary_f(uop, v.z), unary_f(uop, v.w));
+    y[i] = r;
+    ((uint2 *) o16.out)[i] = round4_16(r, o16.type);
+}
+bool launch_unary(hipStream_t s, int uop, const tdesc & src, const tdesc & dst, const copy16 & o16) {
     const int64_t n = src.ne[0] * src.ne[1] * src.ne[2] * src.ne[3];
+    if (o16.out && n > 0 && (n & 3) == 0 && !(((uintptr_t) src.data | (uintptr_t) dst.data) & 15)) {
+        hipLaunchKernelGGL(k_unary_16, dim3((unsigned) ((n / 4 + 255) / 256)), dim3(256), 0, s, uop, (const float4 *) src.data, (float4 *) dst.data, n / 4, o16);
+        return true;
+    }
     const unsigned grid = (unsigned) std::min<int64_t>((n + 255) / 256, 2048);
     hipLaunchKernelGGL(k_unary, dim3(grid), dim3(256), 0, s, uop, (const float *) src.data, (float *) dst.data, n);
+    return false;
 }
 
 // swiglu: y = silu(a) * b (ggml_compute_forward_swiglu_f32); split form (two tensors) or the two halves of one row

@@ -107,6 +107,54 @@ def test_16_bit_siblings_have_the_bits_of_single_launches(backend, H, M):
         assert np.abs(a.reshape(M, -1) - ref).max() <= 6e-8 * np.sqrt(K) * 8
 
 
+# rows of one, two and four pieces a thread, and rows longer than the norm holds (no copy from that one); reshaped and as they are
+@pytest.mark.parametrize("wt", [L.F16, L.BF16])
+@pytest.mark.parametrize("K,M", [(512, 17), (1088, 70), (4096, 40), (4160, 40)])
+@pytest.mark.parametrize("what", ["norm", "norm_add", "norm_twice", "gate", "gate_rows", "gelu", "silu", "relu_sqr"])
+def test_producers_leave_the_16_bit_copy_of_a_product(backend, H, wt, K, M, what):
+    """the operand rounded by the kernel that makes it: no launch for it, and bit for bit what a launch of its own leaves"""
+    rng = np.random.default_rng(K + M)
+    N = 2048
+    w = (rng.standard_normal((N, K)) / np.sqrt(K)).astype(np.float32)
+    x, r = rng.standard_normal((M, K)).astype(np.float32), rng.standard_normal((M, K)).astype(np.float32)
+    g1, g2 = rng.standard_normal(K).astype(np.float32), rng.standard_normal(K).astype(np.float32)
+
+    def build(g):
+        cur, res = g.new(L.F32, [K, M], x), g.new(L.F32, [K, M], r)
+        outs = []
+        if what.startswith("norm"):
+            cur = H.ggml_mul(g.ctx, H.ggml_norm(g.ctx, cur, 1e-5), g.new(L.F32, [K], g1))
+            if what != "norm":
+                cur = H.ggml_add(g.ctx, cur, res)
+            if what == "norm_twice":
+                cur = H.ggml_mul(g.ctx, H.ggml_norm(g.ctx, cur, 1e-5), g.new(L.F32, [K], g2))
+        elif what.startswith("gate"):
+            if what == "gate_rows":
+                cur, res = g.new(L.F32, [8, K // 8, M], x), g.new(L.F32, [8, K // 8, M], r)
+            cur = H.ggml_mul(g.ctx, cur, H.ggml_unary(g.ctx, res, 7))  # GGML_UNARY_OP_SIGMOID
+            if what == "gate_rows":
+                cur = H.ggml_reshape_2d(g.ctx, cur, K, M)
+        else:
+            cur = H.ggml_unary(g.ctx, cur, {"relu_sqr": 6, "gelu": 8, "silu": 10}[what])  # GGML_UNARY_OP_RELU, _GELU, _SILU
+            if what == "relu_sqr":
+                cur = H.ggml_sqr(g.ctx, cur)
+        return [H.ggml_mul_mat(g.ctx, g.new(wt, [K, N], bits16(round16(w, wt), wt)), cur), cur]
+
+    k0 = backend.stat("kernel_launches")
+    got = T.run_case(build, backend)
+    launches = backend.stat("kernel_launches") - k0
+    backend.set_option("fusion", 0)
+    try:
+        plain = T.run_case(build, backend)
+    finally:
+        backend.set_option("fusion", 1)
+    assert launches == (3 if what.startswith("norm") and K > 4096 else 2)
+    for a, b in zip(got, plain):
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+    ref = round16(got[1].reshape(M, K), wt).astype(np.float64) @ round16(w, wt).astype(np.float64).T
+    assert np.abs(got[0].reshape(M, N) - ref).max() <= 6e-8 * np.sqrt(K) * 8 * max(1.0, np.abs(got[1]).max() / 4)  # (the bound above is for operands of up to about 4)
+
+
 # columns of an expert: none, fewer than a tile, several tiles (one expert draws most); both sides of the lines between the tiles (whose input is rounded by a launch of its own) and mmf.hip's form
 @pytest.mark.parametrize("K,N,n_exp,top,T_,tiled", [
     (64, 40, 5, 2, 40, False), (128, 200, 8, 1, 300, False), (192, 130, 3, 3, 70, True), (256, 4160, 6, 2, 100, True), (192, 130, 3, 3, 47, False), (192, 64, 4, 2, 96, True), (256, 70, 4, 1, 92, False),
