@@ -183,11 +183,12 @@ template <int QT, int TQ> __device__ __forceinline__ void sk_unit_k45(const char
 // EPI: the results of the attention projections of a batch are rotated and stored by this launch (mmq_epi) — a separate instantiation,
 // because the accurate cosf / sinf of the rotation bring a scratch frame that every launch of the kernel would otherwise pay for
 // (measured: 4.27 -> 4.45 ms per -np 32 step with the epilogue compiled into the one kernel, used or not)
+// ... and 2, into Q8_0 cache rows, is another (32 columns, Q4_K_M layers over an f16 cache: 11.5 and 16.4 us a launch in one kernel with it, 11.2 and 16.1 apart)
 // MIXED: the matrices of the launch are stored in two formats (wq / wk as Q4_K next to a Q6_K wv: what Q4_K_M does to half the layers) —
 // this pass serves the items whose matrix is stored as QT and walks past the others (k_mmq_skinny_mix runs one pass per format)
 // (the pass is a lambda INSIDE the kernel: as a device function taking the argument block, by value or by reference, it made the compiler
 // copy the block into scratch memory — 408 bytes per lane — and read every pointer of the launch from there)
-template <int QA, int QB, bool EPI, int TQ, bool TILE = false>
+template <int QA, int QB, int EPI, int TQ, bool TILE = false>
 __global__ void __launch_bounds__(SK_NW * 64, 1) k_mmq_skinny(const mmq8_args a) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     constexpr bool MIXED = QA != QB;
@@ -446,7 +447,7 @@ __global__ void __launch_bounds__(SK_NW * 64, 1) k_mmq_skinny(const mmq8_args a)
             const int64_t e_nb2 = mi == 0 ? a.epi.nb2[0] : (mi == 1 ? a.epi.nb2[1] : a.epi.nb2[2]);
             const int head = n / a.epi.head_dim, dd = n - head * a.epi.head_dim;
             float r = v;
-            if ((kind < 3 || kind == 5) && dd < a.epi.n_dims) {
+            if ((kind < 3 || (EPI == 2 && kind == 5)) && dd < a.epi.n_dims) {
                 // (cos, sin) of (token, pair): the table launch_rope_table wrote for this graph run — the chain of multiplies and the accurate
                 // cosf / sinf of rope_cos_sin once per step, not once per layer and element (and no scratch frame in this kernel)
                 const float2 cssn = *(const float2 *) (a.epi.tab + ((size_t) tk * (a.epi.n_dims >> 1) + (dd >> 1)) * 2);
@@ -456,7 +457,7 @@ __global__ void __launch_bounds__(SK_NW * 64, 1) k_mmq_skinny(const mmq8_args a)
             }
             // the tile's 32 rows of a token are one Q8_0 block of the cache row, a half-wave's lanes (k_set_rows_q8_0's arithmetic).  9 tokens of Llama-3-8B: 12.5 us a layer, where the plain
             // projections took as long and the sum of their K split, two rotations and two stores 22 us behind them
-            if (kind >= 5) {
+            if (EPI == 2 && kind >= 5) {
                 float amax = fabsf(r);
 #pragma unroll
                 for (int o2 = 1; o2 < 32; o2 <<= 1) amax = fmaxf(amax, __shfl_xor(amax, o2));
@@ -1610,6 +1611,11 @@ static int skinny_n_cu() {
     return n_cu.load(std::memory_order_relaxed);
 }
 
+// which epilogue: 0 none, 1 rotation and f32 / f16 stores, 2 with Q8_0 cache rows
+static int skinny_epi(const mmq8_args & a) {
+    if (!a.has_epi) return 0;
+    return a.epi.kind[0] >= 5 || a.epi.kind[1] >= 5 || a.epi.kind[2] >= 5 ? 2 : 1;
+}
 template <int QT, int TQ> static void launch_skinny_t(hipStream_t s, mmq8_args a) {
     const int n_cu = skinny_n_cu();
     a.m_tiles = 1;
@@ -1638,10 +1644,10 @@ template <int QT, int TQ> static void launch_skinny_t(hipStream_t s, mmq8_args a
         }
     }
     const size_t lds = (size_t) SK_NW * sk_wave_lds<QT, TQ>();
-    static std::atomic<uint32_t> lds_raised{0}, lds_raised_epi{0};
-    const void * fn_plain = (const void *) k_mmq_skinny<QT, QT, false, TQ>;
-    const void * fn_epi = (const void *) k_mmq_skinny<QT, QT, true, TQ>;
-    (void) ensure_dyn_lds(a.has_epi ? fn_epi : fn_plain, lds, a.has_epi ? lds_raised_epi : lds_raised);
+    static std::atomic<uint32_t> lds_raised[3] = {};
+    const int epi = skinny_epi(a);
+    const void * const fn[3] = {(const void *) k_mmq_skinny<QT, QT, 0, TQ>, (const void *) k_mmq_skinny<QT, QT, 1, TQ>, (const void *) k_mmq_skinny<QT, QT, 2, TQ>};
+    (void) ensure_dyn_lds(fn[epi], lds, lds_raised[epi]);
     a.n_panels = 0;
     for (int i = 0; i < a.n_mat; ++i) {
         a.mat[i].panel0 = a.n_panels;
@@ -1651,22 +1657,24 @@ template <int QT, int TQ> static void launch_skinny_t(hipStream_t s, mmq8_args a
         // a tile per wave where that fills three quarters of the chip's wave slots: no barrier and no sum over the waves (135 us K-parallel, 113 us so: 128256 x 4096 x 3)
         if (!a.has_epi && a.ksplit == 1 && a.n_panels >= 6 * n_cu) {
             static std::atomic<uint32_t> lds_raised_tile{0};
-            (void) ensure_dyn_lds((const void *) k_mmq_skinny<QT, QT, false, TQ, true>, lds, lds_raised_tile);
-            MI_LAUNCH_PROBED((k_mmq_skinny<QT, QT, false, TQ, true>), dim3((unsigned) n_cu), dim3(SK_NW * 64), lds, s, a);
+            (void) ensure_dyn_lds((const void *) k_mmq_skinny<QT, QT, 0, TQ, true>, lds, lds_raised_tile);
+            MI_LAUNCH_PROBED((k_mmq_skinny<QT, QT, 0, TQ, true>), dim3((unsigned) n_cu), dim3(SK_NW * 64), lds, s, a);
             return;
         }
     }
     // one workgroup per CU (its LDS areas fill the CU), walking the (tile, K slice) items with a stride of the grid
     const int items = a.n_panels * a.ksplit;
-    if (a.has_epi) MI_LAUNCH_PROBED((k_mmq_skinny<QT, QT, true, TQ>), dim3((unsigned) std::min(items, n_cu)), dim3(SK_NW * 64), lds, s, a);
-    else MI_LAUNCH_PROBED((k_mmq_skinny<QT, QT, false, TQ>), dim3((unsigned) std::min(items, n_cu)), dim3(SK_NW * 64), lds, s, a);
+    if (epi == 1) MI_LAUNCH_PROBED((k_mmq_skinny<QT, QT, 1, TQ>), dim3((unsigned) std::min(items, n_cu)), dim3(SK_NW * 64), lds, s, a);
+    else if (epi == 2) MI_LAUNCH_PROBED((k_mmq_skinny<QT, QT, 2, TQ>), dim3((unsigned) std::min(items, n_cu)), dim3(SK_NW * 64), lds, s, a);
+    else MI_LAUNCH_PROBED((k_mmq_skinny<QT, QT, 0, TQ>), dim3((unsigned) std::min(items, n_cu)), dim3(SK_NW * 64), lds, s, a);
 }
 
 template <int QA, int QB, int TQ> static void launch_skinny_mix_t(hipStream_t s, mmq8_args a) {
     constexpr size_t lds = (size_t) SK_NW * (size_t) std::max(sk_wave_lds<QA, TQ>(), sk_wave_lds<QB, TQ>());
-    static std::atomic<uint32_t> lds_raised{0}, lds_raised_epi{0};
-    const void * fn = a.has_epi ? (const void *) k_mmq_skinny<QA, QB, true, TQ> : (const void *) k_mmq_skinny<QA, QB, false, TQ>;
-    (void) ensure_dyn_lds(fn, lds, a.has_epi ? lds_raised_epi : lds_raised);
+    static std::atomic<uint32_t> lds_raised[3] = {};
+    const int epi = skinny_epi(a);
+    const void * const fn[3] = {(const void *) k_mmq_skinny<QA, QB, 0, TQ>, (const void *) k_mmq_skinny<QA, QB, 1, TQ>, (const void *) k_mmq_skinny<QA, QB, 2, TQ>};
+    (void) ensure_dyn_lds(fn[epi], lds, lds_raised[epi]);
     a.m_tiles = 1;
     a.n_panels = 0;
     for (int i = 0; i < a.n_mat; ++i) {
@@ -1674,8 +1682,9 @@ template <int QA, int QB, int TQ> static void launch_skinny_mix_t(hipStream_t s,
         a.n_panels += a.mat[i].N / 32;
     }
     const int items = a.n_panels * a.ksplit;
-    if (a.has_epi) MI_LAUNCH_PROBED((k_mmq_skinny<QA, QB, true, TQ>), dim3((unsigned) std::min(items, skinny_n_cu())), dim3(SK_NW * 64), lds, s, a);
-    else MI_LAUNCH_PROBED((k_mmq_skinny<QA, QB, false, TQ>), dim3((unsigned) std::min(items, skinny_n_cu())), dim3(SK_NW * 64), lds, s, a);
+    if (epi == 1) MI_LAUNCH_PROBED((k_mmq_skinny<QA, QB, 1, TQ>), dim3((unsigned) std::min(items, skinny_n_cu())), dim3(SK_NW * 64), lds, s, a);
+    else if (epi == 2) MI_LAUNCH_PROBED((k_mmq_skinny<QA, QB, 2, TQ>), dim3((unsigned) std::min(items, skinny_n_cu())), dim3(SK_NW * 64), lds, s, a);
+    else MI_LAUNCH_PROBED((k_mmq_skinny<QA, QB, 0, TQ>), dim3((unsigned) std::min(items, skinny_n_cu())), dim3(SK_NW * 64), lds, s, a);
 }
 // the form for a's columns, in whole groups of eight
 template <int QA, int QB, int TQ> static void launch_skinny_one(hipStream_t s, const mmq8_args & a) {
