@@ -1005,7 +1005,7 @@ template <int D, bool Q8OUT = false> __global__ void __launch_bounds__(Q8OUT ? 2
 // Q8OUT: the rows' only readers are quantised mat-muls (wo): a wave holds two adjacent heads of a token = one Q8_K block, lane l its values
 // 4 l .. 4 l + 3 — the block is quantised in registers (wave_quantize_q8_K, the arithmetic of k_quantize_q8_K) and no f32 row is written.
 // OUT = 2 (head_dim 64): ... by Q8_0 mat-muls on the matrix cores: eight threads hold a Q8_0 block and leave it in panel order (k_quantize_q8_0's arithmetic).  32 heads of 64: 512 tokens 9.1 us and
-// 4.9 for the quantiser behind it -> 6.6; 16 tokens 3.8 and 2.7 -> 4.0.
+// 4.9 for the quantiser behind it -> 6.3; 16 tokens 3.8 and 2.7 -> 4.5.
 template <int D, int S, int OUT = 0>
 __global__ void __launch_bounds__(256) k_fattn_combine_rows(const float * __restrict__ ws, const tdesc dst, const fa_geom geo, const int n_rows, q8k_dev * __restrict__ q8 = nullptr) {
     constexpr int CPR = D / 4;            // chunks (threads) per row
@@ -1119,7 +1119,15 @@ int fattn_pick_splits(const tdesc & q, const tdesc & k, const tdesc * mask, int 
         // few hundred cells per sequence: ONE pass, which also writes the Q8_K blocks the wo mat-mul reads (4.35 -> 4.30 ms per step)
         const int64_t trips = std::max<int64_t>(1, (n_kv / q.ne[1] + 63) / 64);
         const int64_t by_len = (trips + 7) / 8, by_occ = std::min<int64_t>(trips, (256 + groups - 1) / groups);
-        return (int) std::max<int64_t>(1, std::min<int64_t>(16, std::max(by_len, by_occ)));
+        int64_t n = std::max(by_len, by_occ);
+        // ... and with a combine pass anyway, two workgroups a CU (three fit; one with heads of 64), two trips each: the tokens may be drafts of ONE sequence, each of which sees all
+        // n_kv cells (a trip is a round trip to memory, 2 us), and splits a token with fewer cells has no work for cost it next to nothing.  us a step, before / now (splits):
+        // Llama-3-8B, 9 tokens of a sequence of 1500 cells, Q8_0 cache 3157 (3) / 3031 (6), f16 3063 (3) / 2906 (6); 5 of 6000 3340 (7) / 3007 (12); 4 sequences of 1500, 5 tokens
+        // each, 3761 (2) / 3568 (3); a small model with heads of 64, 9 tokens of 1000 1662 (2) / 1430 (7); sequences of their own: 9 of 170 cells 2816 (3) / 2808 (6), 6 of 60
+        // 2524 (2) / 2525 (4) but 2565 (8), 8 of 900 2845 (4) / 2800 (7), small model 16 of 150 1393 (3) / 1393 (4) but 1405 (7).  ONE pass stays one pass: it saves the combine launch.
+        const int64_t full = k.ne[0] == 64 ? 256 : 480;
+        if (n > 1) n = std::max(n, std::min((n_kv + 127) / 128, full / groups));
+        return (int) std::max<int64_t>(1, std::min<int64_t>(16, n));
     }
     if (q.ne[1] > 1) {  // a few tokens, other head sizes: short splits
         const int64_t by_len = (n_kv + 255) / 256;

@@ -210,3 +210,34 @@ def test_heads_of_64_leave_quantised_rows(backend, H, T_, n_kv, NH, NKV, splits)
     assert n[0] == n[1] - 1, n
     # (the two combine passes sum the records' weights in another order: a value next to a rounding boundary moves by 1 / 127 of its block's largest, few of them)
     assert T.nmse(out[0], out[1]) <= 1e-6
+
+
+# tokens of one sequence, which see all cells, and tokens with a few cells each, for which most of a row's splits have none; heads of 128 and 64; a number of cells that no split divides
+@pytest.mark.parametrize("T_,n_kv,NH,NKV,HD,seen", [
+    (9, 1532, 8, 2, 128, 0), (9, 1532, 8, 2, 128, 3), (2, 260, 4, 4, 128, 1), (5, 6000, 16, 2, 128, 0), (20, 1600, 32, 8, 128, 77), (9, 1000, 16, 4, 64, 0), (16, 2432, 32, 4, 64, 2), (31, 4096, 16, 8, 64, 130)])
+def test_splits_of_few_tokens(backend, H, T_, n_kv, NH, NKV, HD, seen):
+    """position lists in more splits than a token may have cells for, against float64 on the f16 query: sums of at most 6000 products in f32"""
+    rng = np.random.default_rng(T_ + n_kv)
+    q, k, v = (rng.standard_normal(s).astype(np.float32) for s in ((NH, T_, HD), (NKV, n_kv, HD), (NKV, n_kv, HD)))
+    k, v = k.astype(np.float16), v.astype(np.float16)
+    mask = np.full(((T_ + 63) // 64 * 64, n_kv), -np.inf, np.float16)
+    for t in range(T_):
+        if seen:
+            mask[t, rng.choice(n_kv, seen, replace=False)] = 0
+        else:
+            mask[t, : n_kv - T_ + t + 1] = 0
+
+    def build(g):
+        a = H.ggml_flash_attn_ext(g.ctx, g.new(L.F32, [HD, T_, NH], q), g.new(L.F16, [HD, n_kv, NKV], k), g.new(L.F16, [HD, n_kv, NKV], v), g.new(L.F16, [n_kv, mask.shape[0]], mask), HD ** -0.5, 0.0, 0.0)
+        H.ggml_flash_attn_ext_set_prec(a, 10)
+        return a
+
+    s0 = backend.stat("fa_list_launches")
+    got = T.run_case(build, backend)[0].reshape(T_, NH, HD)
+    assert backend.stat("fa_list_launches") == s0 + 1
+    for h in range(NH):
+        z = q[h].astype(np.float16).astype(np.float64) @ k[h // (NH // NKV)].astype(np.float64).T * HD ** -0.5 + mask[:T_].astype(np.float64)
+        p = np.exp(z - z.max(1, keepdims=True))
+        ref = (p / p.sum(1, keepdims=True)) @ v[h // (NH // NKV)].astype(np.float64)
+        # (scores are f32 sums over packed f16 products, the probabilities packed f16: 2^-10 of a weight, as the few-token tests above)
+        assert np.abs(got[:, h] - ref).max() <= 2e-3 * np.abs(ref).max() + 1e-5, h
