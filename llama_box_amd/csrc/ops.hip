@@ -1645,6 +1645,8 @@ __device__ __forceinline__ void q8_store4(char * rowp, const int e, const float4
     qs[1] = (uint16_t) (q8_quant(v.z, d) | (q8_quant(v.w, d) << 8));
     if ((e & 31) == 0) *(uint16_t *) blk = f2h(d);
 }
+// Q8: some rows are Q8_0 ones.  (In one kernel with them the stores into f16 rows took 9.5 us a launch of 77 tokens of Llama-3-8B, apart 9.0.)
+template <bool Q8>
 __global__ void __launch_bounds__(256) k_rope_qk_store(const rope_store_args a) {
     // one workgroup per token; a thread owns rotation pair (tid & 63) [+ 64, ...] — its (cos, sin) is computed ONCE and serves every
     // head — and the four waves share out the head slots: [0, nh) query heads, [nh, nh + nkv) key heads, then value heads
@@ -1689,7 +1691,7 @@ __global__ void __launch_bounds__(256) k_rope_qk_store(const rope_store_args a) 
                 const float * src = (const float *) (a.k_src + h * a.k_nb1 + t * a.k_nb2);
                 uint16_t * dst = (uint16_t *) (a.k_cache + row * a.kc_nb1) + (int64_t) h * a.head_dim;
                 const float x0 = ld(1, src, h, ia), x1 = ld(1, src, h, ib);
-                if (a.k_q8) {  // (whole heads of 64 values and more: the lanes of a block are live together)
+                if (Q8 && a.k_q8) {  // (whole heads of 64 values and more: the lanes of a block are live together)
                     char * rowp = a.k_cache + row * a.kc_nb1;
                     if (neox) {
                         q8_store1(rowp, h * a.head_dim + ia, x0 * cs - x1 * sn);
@@ -1719,7 +1721,7 @@ __global__ void __launch_bounds__(256) k_rope_qk_store(const rope_store_args a) 
             if (a.v_idx) {
                 const int64_t * ix = a.v_idx + ((int64_t) t * a.nkv + h) * a.head_dim;
                 for (int i0 = lane; i0 < a.head_dim; i0 += 64) ((uint16_t *) a.v_cache)[ix[i0]] = f2h(ld(2, src, h, i0));
-            } else if (a.v_q8) {
+            } else if (Q8 && a.v_q8) {
                 for (int i0 = lane; i0 < a.head_dim; i0 += 64) q8_store1(a.v_cache + row * a.vc_nb1, h * a.head_dim + i0, ld(2, src, h, i0));
             } else {
                 uint16_t * dst = (uint16_t *) (a.v_cache + row * a.vc_nb1) + (int64_t) h * a.head_dim;
@@ -1734,7 +1736,7 @@ __global__ void __launch_bounds__(256) k_rope_qk_store(const rope_store_args a) 
 // and (cos, sin) come from the per-graph-run table of k_rope_table (the chain of multiplies and the accurate cosf / sinf once per run, not once
 // per layer).  Requires: whole heads rotated (n_dims == head_dim), head_dim % 8 == 0, projections in memory (no split-K partials); the V cache row-major, or transposed with llama.cpp's per-element indices (non-flash path).
 // The arithmetic per element is that of k_rope_qk_store (x0 cs - x1 sn, x0 sn + x1 cs; f2h for the cache rows).
-template <bool NEOX>
+template <bool NEOX, bool Q8>
 __global__ void __launch_bounds__(256) k_rope_qk_store_vec(const rope_store_args a, const float * __restrict__ tab) {
     const int64_t t = blockIdx.x;
     const int tid = threadIdx.x, hd = a.head_dim, half = hd >> 1;
@@ -1780,7 +1782,7 @@ __global__ void __launch_bounds__(256) k_rope_qk_store_vec(const rope_store_args
                     float * dst = (float *) (a.q_dst + (int64_t) slot * a.qd_nb1 + t * a.qd_nb2);
                     *(float4 *) (dst + 4 * j) = o0;
                     if (NEOX) *(float4 *) (dst + half + 4 * j) = o1;
-                } else if (a.k_q8) {  // (eight lanes a block)
+                } else if (Q8 && a.k_q8) {  // (eight lanes a block)
                     q8_store4(a.k_cache + row * a.kc_nb1, (slot - a.nh) * hd + 4 * j, o0);
                     if (NEOX) q8_store4(a.k_cache + row * a.kc_nb1, (slot - a.nh) * hd + half + 4 * j, o1);
                 } else {
@@ -1798,7 +1800,7 @@ __global__ void __launch_bounds__(256) k_rope_qk_store_vec(const rope_store_args
                     vc[i1] = f2h(lo[k].y);
                     vc[i2] = f2h(lo[k].z);
                     vc[i3] = f2h(lo[k].w);
-                } else if (a.v_q8) {
+                } else if (Q8 && a.v_q8) {
                     q8_store4(a.v_cache + row * a.vc_nb1, h * hd + 4 * j, lo[k]);
                 } else {
                     uint16_t * dst = (uint16_t *) (a.v_cache + row * a.vc_nb1) + (int64_t) h * hd;
@@ -1819,14 +1821,19 @@ bool rope_qk_store_vec_ok(const rope_store_args & a, int n_tokens) {
     return (a.k_q8 || (a.kc_nb1 % 8) == 0) && (a.v_idx != nullptr || a.v_q8 || (a.vc_nb1 % 8) == 0);
 }
 void launch_rope_qk_store_vec(hipStream_t s, const rope_store_args & a, int n_tokens, const float * tab) {
-    if (a.p.mode & GGML_ROPE_TYPE_NEOX) hipLaunchKernelGGL(k_rope_qk_store_vec<true>, dim3((unsigned) n_tokens), dim3(256), 0, s, a, tab);
-    else hipLaunchKernelGGL(k_rope_qk_store_vec<false>, dim3((unsigned) n_tokens), dim3(256), 0, s, a, tab);
+    const bool neox = (a.p.mode & GGML_ROPE_TYPE_NEOX) != 0, q8 = a.k_q8 || a.v_q8;
+    const dim3 grid((unsigned) n_tokens), block(256);
+    if (neox && q8) hipLaunchKernelGGL((k_rope_qk_store_vec<true, true>), grid, block, 0, s, a, tab);
+    else if (neox) hipLaunchKernelGGL((k_rope_qk_store_vec<true, false>), grid, block, 0, s, a, tab);
+    else if (q8) hipLaunchKernelGGL((k_rope_qk_store_vec<false, true>), grid, block, 0, s, a, tab);
+    else hipLaunchKernelGGL((k_rope_qk_store_vec<false, false>), grid, block, 0, s, a, tab);
 }
 void launch_rope_qk_store(hipStream_t s, rope_store_args a, int n_tokens) {
     rope_host_consts(a.p, a.theta_scale, a.corr0, a.corr1);
     const int n_all = a.nh + 2 * a.nkv;
     const int shares = n_tokens >= 256 ? 1 : std::max(1, std::min((n_all + 3) / 4, 1024 / std::max(1, n_tokens)));
-    hipLaunchKernelGGL(k_rope_qk_store, dim3((unsigned) n_tokens, (unsigned) shares), dim3(256), 0, s, a);
+    if (a.k_q8 || a.v_q8) hipLaunchKernelGGL(k_rope_qk_store<true>, dim3((unsigned) n_tokens, (unsigned) shares), dim3(256), 0, s, a);
+    else hipLaunchKernelGGL(k_rope_qk_store<false>, dim3((unsigned) n_tokens, (unsigned) shares), dim3(256), 0, s, a);
 }
 void launch_rope(hipStream_t s, const tdesc & a, const tdesc & pos, const float * ff, const tdesc & d, const rope_params & p) {
     float theta_scale, c0, c1;
