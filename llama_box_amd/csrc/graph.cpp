@@ -847,6 +847,7 @@ static bool quant_consumers_only(const exec_state & st, int at, const ggml_tenso
 static bool q80_panel_consumers_only(const exec_state & st, int at, const ggml_tensor * t) {
     if ((t->flags & GGML_TENSOR_FLAG_OUTPUT) || t->type != GGML_TYPE_F32 || (t->ne[0] % 128) != 0) return false;
     const int64_t M = t->ne[1] * t->ne[2] * t->ne[3];
+    if (M <= st.c->opt.mmvq_max_cols) return false;  // (the mat-vec fusions quantise t themselves, in another order: opt.mmvq_max_cols can reach up here)
     const ggml_cgraph * g = st.g;
     int last = -1, n_cons = 0;
     for (int j = at + 1; j < g->n_nodes; ++j) {

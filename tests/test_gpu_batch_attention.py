@@ -212,6 +212,48 @@ def test_heads_of_64_leave_quantised_rows(backend, H, T_, n_kv, NH, NKV, splits)
     assert T.nmse(out[0], out[1]) <= 1e-6
 
 
+# the option that widens the mat-vec fusions beyond 8 columns: products that take them quantise their f32 input themselves, so its producer (attention, norm, SwiGLU) may not leave panel blocks alone
+@pytest.mark.parametrize("what", ["attention", "norm", "swiglu"])
+@pytest.mark.parametrize("widest", [11, 12, 16])
+def test_mat_vec_fusions_of_many_columns_find_their_input(backend, H, what, widest):
+    T_, n_kv, NH, NKV, N = 12, 640, 8, 2, 256
+    rng = np.random.default_rng(widest)
+    K = NH * 64
+    q, k, v = (rng.standard_normal(s).astype(np.float32) for s in ((NH, T_, 64), (NKV, n_kv, 64), (NKV, n_kv, 64)))
+    x, w0, r1, r2 = (rng.standard_normal(s).astype(np.float32) for s in ((T_, K), (K,), (T_, N), (T_, N)))
+    ws = [T.rand_weight(L.Q8_0, K, n, rng) for n in (N, N, K, K)]
+    mask = np.full((64, n_kv), -np.inf, np.float16)
+    for t in range(T_):
+        mask[t, : n_kv - T_ + t + 1] = 0
+
+    def build(g):
+        def mm(i, y, n):
+            return H.ggml_mul_mat(g.ctx, g.new(L.Q8_0, [K, n], ws[i]), y)
+
+        if what == "attention":
+            y = H.ggml_flash_attn_ext(g.ctx, g.new(L.F32, [64, T_, NH], q), g.new(L.F16, [64, n_kv, NKV], k.astype(np.float16)), g.new(L.F16, [64, n_kv, NKV], v.astype(np.float16)),
+                                      g.new(L.F16, [n_kv, 64], mask), 0.125, 0.0, 0.0)
+            H.ggml_flash_attn_ext_set_prec(y, 10)
+            y = H.ggml_reshape_2d(g.ctx, y, K, T_)
+        else:
+            y = H.ggml_mul(g.ctx, H.ggml_rms_norm(g.ctx, g.new(L.F32, [K, T_], x), 1e-5), g.new(L.F32, [K], w0))
+            if what == "norm":
+                return [H.ggml_swiglu_split(g.ctx, mm(0, y, N), mm(1, y, N))]
+            y = H.ggml_swiglu_split(g.ctx, mm(2, y, K), mm(3, y, K))
+        return [H.ggml_add(g.ctx, H.ggml_add(g.ctx, mm(0, y, N), g.new(L.F32, [N, T_], r1)), g.new(L.F32, [N, T_], r2))]
+
+    backend.set_option("fa_splits", 4)  # (attention ends in the combine pass that can leave blocks)
+    try:
+        ref = T.run_case(build, backend)[0]
+        backend.set_option("mmvq_max_cols", widest)
+        got = T.run_case(build, backend)[0]
+    finally:
+        backend.set_option("mmvq_max_cols", 2)
+        backend.set_option("fa_splits", 0)
+    # (other kernels in front of the quantiser: a value next to a rounding boundary moves by 1 / 127 of its block's largest, few of them)
+    assert T.nmse(got, ref) <= 1e-6
+
+
 # tokens of one sequence, which see all cells, and tokens with a few cells each, for which most of a row's splits have none; heads of 128 and 64; a number of cells that no split divides
 @pytest.mark.parametrize("T_,n_kv,NH,NKV,HD,seen", [
     (9, 1532, 8, 2, 128, 0), (9, 1532, 8, 2, 128, 3), (2, 260, 4, 4, 128, 1), (5, 6000, 16, 2, 128, 0), (20, 1600, 32, 8, 128, 77), (9, 1000, 16, 4, 64, 0), (16, 2432, 32, 4, 64, 2), (31, 4096, 16, 8, 64, 130)])
