@@ -52,9 +52,8 @@ typedef uint32_t __attribute__((ext_vector_type(4), aligned(4))) q80s_u32x4_a4;
 
 constexpr int Q80S_WV = 8;
 // EPI: wq / wk / wv of a batch whose rotation and cache stores follow — done here, as in the K-quants' epilogue (mmq_skinny.hip; the arithmetic of k_rope_qk_store).  16 tokens of TinyLlama: the
-// launch of its own cost 5.8 us a layer.
+// launch of its own cost 5.8 us a layer; this one takes 7.1 us (6.7 without the epilogue; 7.8 with a branch around the next chunk's loads, behind which each product waited for what had just been requested).
 template <bool WP, bool EPI> __global__ void __launch_bounds__(Q80S_WV * 64, 2) k_mmq_q80_skinny(const mmq80s_args a, const mmq_epi epi) {
-    constexpr bool PF = true;
     __shared__ float dwl[Q80S_WV][4][32];       // a chunk's row scales, per wave
     __shared__ float red[Q80S_WV][16][65];      // the waves' partial tiles
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -93,11 +92,7 @@ template <bool WP, bool EPI> __global__ void __launch_bounds__(Q80S_WV * 64, 2) 
             dY[b] = *(const float *) (yt + 1024 + colc * 4);
         }
     };
-    int c = wave;
-    if (c < nchunk) load_chunk(c, fa, fb, dw, dy);
-    for (; c < nchunk; c += Q80S_WV) {
-        const int cn = c + Q80S_WV;
-        if constexpr (PF) { if (cn < nchunk) load_chunk(cn, nfa, nfb, ndw, ndy); }
+    auto multiply = [&]() __attribute__((always_inline)) {
         // the block scales of the 32 rows: written by the row's first lane, read back as the 16 rows of this lane's accumulator registers
         if (kg == 0) {
 #pragma unroll
@@ -120,14 +115,18 @@ template <bool WP, bool EPI> __global__ void __launch_bounds__(Q80S_WV * 64, 2) 
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();  // (the next chunk's scales overwrite the line)
-        if (cn < nchunk) {
-            if constexpr (PF) {
+    };
+    int c = wave;
+    if (c < nchunk) {
+        load_chunk(c, fa, fb, dw, dy);
+        for (; c + Q80S_WV < nchunk; c += Q80S_WV) {  // (no branch around the next chunk's loads: behind a join the products would wait for them)
+            load_chunk(c + Q80S_WV, nfa, nfb, ndw, ndy);
+            multiply();
+            __builtin_amdgcn_sched_barrier(0);  // (... as they would behind copies that move up between them)
 #pragma unroll
-                for (int b = 0; b < 4; ++b) { fa[b] = nfa[b]; fb[b] = nfb[b]; dw[b] = ndw[b]; dy[b] = ndy[b]; }
-            } else {
-                load_chunk(cn, fa, fb, dw, dy);
-            }
+            for (int b = 0; b < 4; ++b) { fa[b] = nfa[b]; fb[b] = nfb[b]; dw[b] = ndw[b]; dy[b] = ndy[b]; }
         }
+        multiply();
     }
 #pragma unroll
     for (int r = 0; r < 16; ++r) red[wave][r][lane] = C[r];

@@ -509,3 +509,36 @@ def test_batch_rope_and_stores_into_q8_0_rows(backend, H, kt, vt, mode, HD, M, p
         assert launches == 3, launches  # the input's quantiser, the (cos, sin) table, the projections
     for name, a, b in zip(("q", "k cache", "v cache"), got, plain):
         assert np.array_equal(np.asarray(a).view(np.uint8), np.asarray(b).view(np.uint8)), name
+
+
+# the same epilogue behind projections with a bias (added ahead of the rotation), and with heads rotated in part, which only f16 rows take there
+@pytest.mark.parametrize("project,kt,vt,HD,ND,M,bias", [
+    (L.Q8_0, L.F16, L.F16, 128, 64, 12, False), (L.Q8_0, L.F16, L.F16, 64, 64, 9, True), (L.Q8_0, L.F16, L.F16, 128, 32, 32, True), (L.Q8_0, L.Q8_0, L.Q8_0, 64, 64, 17, True),
+    (L.Q4_K, L.Q8_0, L.Q8_0, 128, 128, 9, True), (L.Q5_K, L.Q8_0, L.F16, 128, 128, 3, True), (L.Q4_K, L.F16, L.F16, 128, 64, 16, True), (L.Q6_K, L.F16, L.F16, 128, 64, 5, False)])
+def test_batch_rope_and_stores_behind_biases_and_in_part(backend, H, project, kt, vt, HD, ND, M, bias):
+    rng = np.random.default_rng(M + HD + ND + kt + 3 * vt)
+    E, NH, NKV, NCTX = 512, 8, 2, 300
+    x = rng.standard_normal((M, E)).astype(np.float32)
+    ws = [T.rand_weight(project, E, n * HD, rng) for n in (NH, NKV, NKV)]
+    bs = [rng.standard_normal(n * HD).astype(np.float32) for n in (NH, NKV, NKV)]
+    pos, rows = rng.integers(0, 5000, M).astype(np.int32), rng.permutation(NCTX)[:M].astype(np.int64)
+
+    def build(g):
+        cur = g.new(L.F32, [E, M], x)
+        q, k, v = (H.ggml_mul_mat(g.ctx, g.new(project, [E, n * HD], w), cur) for n, w in zip((NH, NKV, NKV), ws))
+        if bias:
+            q, k, v = (H.ggml_add(g.ctx, t, g.new(L.F32, [n * HD], b)) for t, n, b in zip((q, k, v), (NH, NKV, NKV), bs))
+        tp, idx = g.new(L.I32, [M], pos), g.new(L.I64, [M], rows)
+        q, k = (H.ggml_rope_ext(g.ctx, H.ggml_reshape_3d(g.ctx, t, HD, n, M), tp, None, ND, 0, 8192, 500000.0, 1.0, 0.0, 1.0, 32.0, 1.0) for t, n in ((q, NH), (k, NKV)))
+        return [q, H.ggml_set_rows(g.ctx, g.new(kt, [NKV * HD, NCTX]), H.ggml_reshape_2d(g.ctx, k, NKV * HD, M), idx), H.ggml_set_rows(g.ctx, g.new(vt, [NKV * HD, NCTX]), v, idx)]
+
+    e0 = backend.stat("rope_epilogues")
+    got = T.run_case(build, backend)
+    assert backend.stat("rope_epilogues") == e0 + 1
+    backend.set_option("fusion", 0)
+    try:
+        plain = T.run_case(build, backend)
+    finally:
+        backend.set_option("fusion", 1)
+    for name, a, b in zip(("q", "k cache", "v cache"), got, plain):
+        assert np.array_equal(np.asarray(a).view(np.uint8), np.asarray(b).view(np.uint8)), name
