@@ -152,29 +152,44 @@ __device__ __forceinline__ uint2 round4_16(const float4 v, const int type) {
 // like RMS_NORM's).  w: optional weight of the MUL that follows; r: optional residual rows of the ADD behind that (same shape as the output).
 // second stage (w2 != nullptr): the row just written is normalised once more into d2, y2 = LN(y) * w2 — the norm in front of the next sublayer, which reads
 // the residual stream this kernel has just updated (a thread re-reads the elements it wrote itself)
-// Rows of up to 4096 values in whole, aligned pieces of four (k_layer_norm_held, R pieces a thread): the row, its weights, the residual row and the second stage's
-// weights are ALL requested before anything waits, so a row costs one round trip to memory and the barriers of its sums.  With the weights and the residual loaded behind
-// the sums, value by value under the bounds check, each of the sixteen values of a thread waited for its own two loads.  MI355X, us a launch, before / now: 2 rows of 2048
-// with both stages 12.2 / 4.2, 512 rows of 4096 13.8 / 7.2.  Any other row: k_layer_norm.
-// o16: a second, dense copy of the last stage's rows in the type of the 16-bit matrices that multiply them next (k_to_16's rounding)
-template <int R>
+// Rows of up to 4096 values (k_layer_norm_held, R pieces of V values a thread): the row, its weights, the residual row and the second stage's weights are ALL requested before
+// anything waits, so a row costs one round trip to memory and the barriers of its sums.  With the weights and the residual loaded behind the sums, value by value under the bounds
+// check, each of the sixteen values of a thread waited for its own two loads.  Pieces of four where a row is whole ones at aligned addresses, else single values.  MI355X, us a launch,
+// before / now: 2 rows of 2048 with both stages 12.2 / 4.2, 512 rows of 4096 13.8 / 7.2.  Longer rows: k_layer_norm.
+// o16 (V = 4): a second, dense copy of the last stage's rows in the type of the 16-bit matrices that multiply them next (k_to_16's rounding)
+template <int R, int V>
 __global__ void __launch_bounds__(256) k_layer_norm_held(const tdesc a, const tdesc d, const float eps, const float * __restrict__ w, const tdesc r, const int has_r,
                                                          const float * __restrict__ w2, const float eps2, const tdesc d2, const copy16 o16) {
+    static_assert(V == 1 || V == 4, "single values or quads");
     __shared__ double sh[4][4];
     const int64_t row = blockIdx.x;
     const int64_t i1 = row % a.ne[1], i2 = (row / a.ne[1]) % a.ne[2], i3 = row / (a.ne[1] * a.ne[2]);
-    const float4 * const x = (const float4 *) (a.data + i1 * a.nb[1] + i2 * a.nb[2] + i3 * a.nb[3]);
-    const float4 * const rr = (const float4 *) (r.data + i1 * r.nb[1] + i2 * r.nb[2] + i3 * r.nb[3]);
-    const int n4 = (int) (a.ne[0] >> 2);
+    const float * const x = (const float *) (a.data + i1 * a.nb[1] + i2 * a.nb[2] + i3 * a.nb[3]);
+    const float * const rr = (const float *) (r.data + i1 * r.nb[1] + i2 * r.nb[2] + i3 * r.nb[3]);
+    const int np = (int) (a.ne[0] / V);
     const double inv = (double) a.ne[0];
-    float4 xv[R], wv[R], rv[R], w2v[R];
+    auto get = [](const float * p, const int i, float * v) {
+        if constexpr (V == 4) {
+            const float4 t = ((const float4 *) p)[i];
+            v[0] = t.x; v[1] = t.y; v[2] = t.z; v[3] = t.w;
+        } else v[0] = p[i];
+    };
+    auto put = [](float * p, const int i, const float * v) {
+        if constexpr (V == 4) ((float4 *) p)[i] = make_float4(v[0], v[1], v[2], v[3]);
+        else p[i] = v[0];
+    };
+    auto same = [](float * v, const float f) {
+#pragma unroll
+        for (int c = 0; c < V; ++c) v[c] = f;
+    };
+    float xv[R][V], wv[R][V], rv[R][V], w2v[R][V];
 #pragma unroll
     for (int u = 0; u < R; ++u) {  // (lanes beyond the row read its last piece and add nothing)
-        const int i = min((int) threadIdx.x + 256 * u, n4 - 1);
-        xv[u] = x[i];
-        wv[u] = w ? ((const float4 *) w)[i] : make_float4(1.f, 1.f, 1.f, 1.f);
-        rv[u] = has_r ? rr[i] : make_float4(0.f, 0.f, 0.f, 0.f);
-        w2v[u] = w2 ? ((const float4 *) w2)[i] : make_float4(1.f, 1.f, 1.f, 1.f);
+        const int i = min((int) threadIdx.x + 256 * u, np - 1);
+        get(x, i, xv[u]);
+        if (w) get(w, i, wv[u]); else same(wv[u], 1.0f);
+        if (has_r) get(rr, i, rv[u]); else same(rv[u], 0.0f);
+        if (w2) get(w2, i, w2v[u]); else same(w2v[u], 1.0f);
     }
     auto total = [&](const double part, double * const s4) {
         const double v = wave_sum_d(part);
@@ -182,52 +197,68 @@ __global__ void __launch_bounds__(256) k_layer_norm_held(const tdesc a, const td
         __syncthreads();
         return ((s4[0] + s4[1]) + s4[2]) + s4[3];
     };
-    auto live = [&](const int u) { return (int) threadIdx.x + 256 * u < n4; };
+    auto live = [&](const int u) { return (int) threadIdx.x + 256 * u < np; };
     auto norm = [&](const float e, const int stage, float & mean, float & scale) {
         double s = 0.0, q = 0.0;
 #pragma unroll
         for (int u = 0; u < R; ++u)
-            if (live(u)) s += ((double) xv[u].x + (double) xv[u].y) + ((double) xv[u].z + (double) xv[u].w);
+            if (live(u)) {
+                if constexpr (V == 4) s += ((double) xv[u][0] + (double) xv[u][1]) + ((double) xv[u][2] + (double) xv[u][3]);
+                else s += (double) xv[u][0];
+            }
         mean = (float) (total(s, sh[2 * stage]) / inv);
 #pragma unroll
         for (int u = 0; u < R; ++u) {
-            const float dx = xv[u].x - mean, dy = xv[u].y - mean, dz = xv[u].z - mean, dw = xv[u].w - mean;
-            if (live(u)) q += ((double) (dx * dx) + (double) (dy * dy)) + ((double) (dz * dz) + (double) (dw * dw));
+            float t[V];
+#pragma unroll
+            for (int c = 0; c < V; ++c) {
+                const float dv = xv[u][c] - mean;
+                t[c] = dv * dv;
+            }
+            if (live(u)) {
+                if constexpr (V == 4) q += ((double) t[0] + (double) t[1]) + ((double) t[2] + (double) t[3]);
+                else q += (double) t[0];
+            }
         }
         scale = 1.0f / sqrtf((float) (total(q, sh[2 * stage + 1]) / inv) + e);
     };
     float mean, scale;
     norm(eps, 0, mean, scale);
-    float4 * const y = (float4 *) (d.data + i1 * d.nb[1] + i2 * d.nb[2] + i3 * d.nb[3]);
+    float * const y = (float *) (d.data + i1 * d.nb[1] + i2 * d.nb[2] + i3 * d.nb[3]);
 #pragma unroll
     for (int u = 0; u < R; ++u) {
-        float4 v;
-        v.x = (xv[u].x - mean) * scale; v.y = (xv[u].y - mean) * scale; v.z = (xv[u].z - mean) * scale; v.w = (xv[u].w - mean) * scale;
-        if (w) { v.x *= wv[u].x; v.y *= wv[u].y; v.z *= wv[u].z; v.w *= wv[u].w; }
-        if (has_r) { v.x += rv[u].x; v.y += rv[u].y; v.z += rv[u].z; v.w += rv[u].w; }
-        if (live(u)) y[threadIdx.x + 256 * u] = v;
-        xv[u] = v;
-    }
-    uint2 * const y16 = (uint2 *) o16.out + row * n4;
-    if (w2 == nullptr) {
-        if (o16.out) {
 #pragma unroll
-            for (int u = 0; u < R; ++u)
-                if (live(u)) y16[threadIdx.x + 256 * u] = round4_16(xv[u], o16.type);
+        for (int c = 0; c < V; ++c) {
+            float v = (xv[u][c] - mean) * scale;
+            if (w) v *= wv[u][c];
+            if (has_r) v += rv[u][c];
+            xv[u][c] = v;
         }
+        if (live(u)) put(y, threadIdx.x + 256 * u, xv[u]);
+    }
+    uint2 * const y16 = (uint2 *) o16.out + row * np;
+    if (w2 == nullptr) {
+        if constexpr (V == 4)
+            if (o16.out) {
+#pragma unroll
+                for (int u = 0; u < R; ++u)
+                    if (live(u)) y16[threadIdx.x + 256 * u] = round4_16(make_float4(xv[u][0], xv[u][1], xv[u][2], xv[u][3]), o16.type);
+            }
         return;
     }
     norm(eps2, 1, mean, scale);
-    float4 * const y2 = (float4 *) (d2.data + i1 * d2.nb[1] + i2 * d2.nb[2] + i3 * d2.nb[3]);
+    float * const y2 = (float *) (d2.data + i1 * d2.nb[1] + i2 * d2.nb[2] + i3 * d2.nb[3]);
 #pragma unroll
     for (int u = 0; u < R; ++u) {
-        float4 v;
-        v.x = (xv[u].x - mean) * scale * w2v[u].x; v.y = (xv[u].y - mean) * scale * w2v[u].y; v.z = (xv[u].z - mean) * scale * w2v[u].z; v.w = (xv[u].w - mean) * scale * w2v[u].w;
-        if (live(u)) y2[threadIdx.x + 256 * u] = v;
-        if (o16.out && live(u)) y16[threadIdx.x + 256 * u] = round4_16(v, o16.type);
+        float v[V];
+#pragma unroll
+        for (int c = 0; c < V; ++c) v[c] = (xv[u][c] - mean) * scale * w2v[u][c];
+        if (live(u)) put(y2, threadIdx.x + 256 * u, v);
+        if constexpr (V == 4)
+            if (o16.out && live(u)) y16[threadIdx.x + 256 * u] = round4_16(make_float4(v[0], v[1], v[2], v[3]), o16.type);
     }
 }
-// y = (x - mean) / sqrt(var + eps) per row for rows that are longer, odd or not aligned: the row is read again in every pass
+// y = (x - mean) / sqrt(var + eps) per row for rows that are longer: the row is read again in every pass
 __global__ void __launch_bounds__(256) k_layer_norm(const tdesc a, const tdesc d, const float eps, const float * __restrict__ w, const tdesc r, const int has_r,
                                                     const float * __restrict__ w2, const float eps2, const tdesc d2) {
     __shared__ double sh[4];
@@ -279,13 +310,15 @@ static bool launch_layer_norm_rows(hipStream_t s, const tdesc & src, const tdesc
     if (rows == 0) return false;
     const tdesc r = residual ? *residual : src;
     auto al = [](const tdesc & t) { return (((uintptr_t) t.data | (uintptr_t) t.nb[1] | (uintptr_t) t.nb[2] | (uintptr_t) t.nb[3]) & 15) == 0; };
-    const bool held = n > 0 && n <= 4096 && (n & 3) == 0 && al(src) && al(dst) && al(r) && al(dst2) && (((uintptr_t) mul_w | (uintptr_t) w2) & 15) == 0;
+    const bool quads = (n & 3) == 0 && al(src) && al(dst) && al(r) && al(dst2) && (((uintptr_t) mul_w | (uintptr_t) w2) & 15) == 0, held = n > 0 && n <= 4096;
     const dim3 g((unsigned) rows), b(256);
+#define MI_NORM(R_, V_) hipLaunchKernelGGL((k_layer_norm_held<R_, V_>), g, b, 0, s, src, dst, eps, mul_w, r, residual ? 1 : 0, w2, eps2, dst2, o16)
     if (!held) hipLaunchKernelGGL(k_layer_norm, g, b, 0, s, src, dst, eps, mul_w, r, residual ? 1 : 0, w2, eps2, dst2);
-    else if (n <= 1024) hipLaunchKernelGGL(k_layer_norm_held<1>, g, b, 0, s, src, dst, eps, mul_w, r, residual ? 1 : 0, w2, eps2, dst2, o16);
-    else if (n <= 2048) hipLaunchKernelGGL(k_layer_norm_held<2>, g, b, 0, s, src, dst, eps, mul_w, r, residual ? 1 : 0, w2, eps2, dst2, o16);
-    else hipLaunchKernelGGL(k_layer_norm_held<4>, g, b, 0, s, src, dst, eps, mul_w, r, residual ? 1 : 0, w2, eps2, dst2, o16);
-    return held && o16.out;
+    else if (n <= 1024) { if (quads) MI_NORM(1, 4); else MI_NORM(4, 1); }
+    else if (n <= 2048) { if (quads) MI_NORM(2, 4); else MI_NORM(8, 1); }
+    else { if (quads) MI_NORM(4, 4); else MI_NORM(16, 1); }
+#undef MI_NORM
+    return held && quads && o16.out;
 }
 bool launch_layer_norm(hipStream_t s, const tdesc & src, const tdesc & dst, float eps, const float * mul_w, const tdesc * residual, const copy16 & o16) {
     return launch_layer_norm_rows(s, src, dst, eps, mul_w, residual, nullptr, 0.0f, dst, o16);

@@ -327,6 +327,31 @@ def test_layer_norm_two_stages_at_the_edges_of_its_pieces(backend, H, n):
     assert np.abs(got - R.layer_norm(s, w2.astype(np.float64), 1e-6)).max() <= 2e-5
 
 
+# rows of up to 4096 values that start at no multiple of 16 bytes, or whose weights do (single values a thread, 4, 8 or 16 of them)
+@pytest.mark.parametrize("n", [1, 63, 256, 1024, 1025, 2048, 2049, 4095, 4096])
+@pytest.mark.parametrize("shifted", ["rows", "weight"])
+def test_layer_norm_two_stages_of_unaligned_rows(backend, H, n, shifted):
+    rng = np.random.default_rng(n)
+    rows = 3
+    x = (rng.standard_normal((rows, n)) * 3 + 1.5).astype(np.float32)
+    r = rng.standard_normal((rows, n)).astype(np.float32)
+    w, w2 = (rng.standard_normal(n).astype(np.float32) for _ in range(2))
+
+    def behind(g, a, off):  # (a tensor's values behind `off` others)
+        t = g.new(L.F32, [a.size + off], np.concatenate([np.zeros(off, np.float32), a.reshape(-1)]))
+        return H.ggml_view_2d(g.ctx, t, n, a.size // n, n * 4, off * 4)
+
+    def build(g):
+        s = H.ggml_norm(g.ctx, behind(g, x, 1 if shifted == "rows" else 0), 1e-5)
+        s = H.ggml_add(g.ctx, H.ggml_mul(g.ctx, s, behind(g, w, 1 if shifted == "weight" else 0)), g.new(L.F32, [n, rows], r))
+        return [H.ggml_mul(g.ctx, H.ggml_norm(g.ctx, s, 1e-6), g.new(L.F32, [n], w2))]
+
+    got = run(backend, build)[0].reshape(rows, n)
+    s = R.layer_norm(x.astype(np.float64), w.astype(np.float64), 1e-5) + r
+    # (as above; one value has no deviation to divide by: 0 on both sides)
+    assert np.abs(got - R.layer_norm(s, w2.astype(np.float64), 1e-6)).max() <= 2e-5
+
+
 def test_rotary_on_the_leading_pairs(backend, H):
     rng = np.random.default_rng(6)
     x = rng.standard_normal((9, 3, 20)).astype(np.float32)
