@@ -1430,15 +1430,50 @@ __device__ __forceinline__ float yarn_ramp(const float low, const float high, co
     const float y = ((float) (i0 / 2) - low) / fmaxf(0.001f, high - low);
     return 1.0f - fminf(1.0f, fmaxf(0.0f, y));
 }
+__device__ __forceinline__ void rope_angle(const rope_params & p, const int ip, const float pos_f, const float * __restrict__ ff, const rope_consts & rc, float & cs, float & sn) {
+    if (p.exact_freq == 2) rope_cos_sin_table(ip, pos_f, ff, p.attn_factor, cs, sn);
+    else if (p.exact_freq) rope_cos_sin_exact(ip, pos_f, p.freq_base, p.n_dims, cs, sn);
+    else rope_cos_sin(ip, pos_f, ff, rc, cs, sn);
+}
+template <bool F16IO> __global__ void __launch_bounds__(64) k_rope(const tdesc a, const tdesc pos, const float * __restrict__ ff, const tdesc d, const rope_params p,
+                                                               const float theta_scale, const float corr0, const float corr1) {
+    // grid: (head i1, token i2, batch i3); lanes = rotation pairs, so all loads of a launch are independent
+    const int64_t i1 = blockIdx.x, i2 = blockIdx.y, i3 = blockIdx.z;
+    const int n_pairs = p.n_dims / 2;
+    const float pos_f = (float) *(const int32_t *) (pos.data + i2 * pos.nb[0]);
+    const char * src = a.data + i1 * a.nb[1] + i2 * a.nb[2] + i3 * a.nb[3];  // (in place, when the allocator made it so)
+    char * dst = d.data + i1 * d.nb[1] + i2 * d.nb[2] + i3 * d.nb[3];
+    const bool neox = (p.mode & GGML_ROPE_TYPE_NEOX) != 0;
+    for (int ip = threadIdx.x; ip < n_pairs; ip += blockDim.x) {
+        const int ia = neox ? ip : 2 * ip, ib = neox ? ip + n_pairs : 2 * ip + 1;
+        float x0, x1;
+        if (F16IO) { x0 = h2f(((const uint16_t *) src)[ia]); x1 = h2f(((const uint16_t *) src)[ib]); }
+        else { x0 = ((const float *) src)[ia]; x1 = ((const float *) src)[ib]; }
+        float cs, sn;
+        rope_angle(p, ip, pos_f, ff, rope_consts{theta_scale, p.freq_scale, p.ext_factor, p.attn_factor, corr0, corr1}, cs, sn);
+        if (F16IO) {
+            ((uint16_t *) dst)[ia] = f2h(x0 * cs - x1 * sn);
+            ((uint16_t *) dst)[ib] = f2h(x0 * sn + x1 * cs);
+        } else {
+            ((float *) dst)[ia] = x0 * cs - x1 * sn;
+            ((float *) dst)[ib] = x0 * sn + x1 * cs;
+        }
+    }
+    for (int64_t i0 = p.n_dims + threadIdx.x; i0 < a.ne[0]; i0 += blockDim.x) {  // pass-through tail beyond n_dims
+        if (F16IO) ((uint16_t *) dst)[i0] = ((const uint16_t *) src)[i0];
+        else ((float *) dst)[i0] = ((const float *) src)[i0];
+    }
+}
 // The heads of one token, wave (wv of nw) by wave: a lane owns a rotation pair — its (cos, sin), a power and two accurate functions or a chain of multiplies, is computed once and serves every
 // head the wave takes (two and more at a time where the pairs are fewer than the lanes), four of them in flight.  With a wave per (token, head) the angles were the launch: 512 tokens, 32 heads
 // of 128, 64 of them rotated 13.5 -> 7.8 us.
-// NH: heads a lane has in flight; the first ones are requested ahead of the angle's chain
-template <int NH, class LD, class ST>
+// (the first four are requested ahead of the angle's chain)
+template <class LD, class ST>
 __device__ __forceinline__ void rope_heads(const rope_params & p, const float pos_f, const float * __restrict__ ff, const rope_consts rc, const int D, const int H, const int wv, const int nw, LD ld, ST st) {
+    constexpr int NH = 4;
     const int lane = threadIdx.x & 63, n_pairs = p.n_dims / 2;
     const bool neox = (p.mode & GGML_ROPE_TYPE_NEOX) != 0;
-    const int lp = NH == 1 || n_pairs > 32 ? 64 : n_pairs > 16 ? 32 : n_pairs > 8 ? 16 : 8, per = 64 / lp;  // lanes for a head's pairs, heads at a time
+    const int lp = n_pairs > 32 ? 64 : n_pairs > 16 ? 32 : n_pairs > 8 ? 16 : 8, per = 64 / lp;  // lanes for a head's pairs, heads at a time
     for (int ip0 = 0; ip0 < n_pairs; ip0 += lp) {
         const int ip = ip0 + (lane & (lp - 1));
         if (ip >= n_pairs) continue;
@@ -1455,9 +1490,7 @@ __device__ __forceinline__ void rope_heads(const rope_params & p, const float po
         int h = wv * per + lane / lp;
         request(h);
         float cs, sn;
-        if (p.exact_freq == 2) rope_cos_sin_table(ip, pos_f, ff, p.attn_factor, cs, sn);
-        else if (p.exact_freq) rope_cos_sin_exact(ip, pos_f, p.freq_base, p.n_dims, cs, sn);
-        else rope_cos_sin(ip, pos_f, ff, rc, cs, sn);
+        rope_angle(p, ip, pos_f, ff, rc, cs, sn);
         while (h < H) {
 #pragma unroll
             for (int k = 0; k < NH; ++k)
@@ -1479,17 +1512,21 @@ __device__ __forceinline__ void rope_heads(const rope_params & p, const float po
                 if (h + k * nw < H) st(h + k * nw, i0, x[k]);
         }
 }
-// waves for a token's heads: one each (workgroups of one) while the tokens are few, four a token when those alone fill the chip
-static bool rope_many(const int64_t tokens) { return tokens >= 128; }
-static unsigned rope_grid(const int64_t heads, const int64_t tokens) { return rope_many(tokens) ? 1u : (unsigned) heads; }
-template <bool F16IO, int NH> __global__ void __launch_bounds__(256) k_rope(const tdesc a, const tdesc pos, const float * __restrict__ ff, const tdesc d, const rope_params p,
+// A token's heads: a workgroup of one wave each (k_rope), or one or two groups of four waves a token, whose lanes keep an angle for several heads (k_rope_heads).  The first have the shorter chain and win
+// while the chip holds them at once, up to about 5000; below six heads the groups leave waves without work.  Two groups pay while all of them run at once.  us, launches in a row, heads of 128, 64
+// rotated (a wave a head / one group a token / two): 32 heads x 128 tokens 5.8 / 6.5 / 5.9, x 192 7.7 / 6.7 / 6.4, x 512 13.5 / 8.0 / 8.0, x 1024 23.9 / 12.3 / 14.4, 64 x 512 23.7 / 13.9 / 12.1, 24 x 192
+// 6.2 / 6.3 / 6.1, x 256 7.8 / 6.5 / 6.3, 16 x 192 5.1 / 5.5 / 5.7, x 256 5.8 / 5.8 / 6.1, x 384 7.8 / 6.2 / 6.6, 8 x 128 4.3 / 4.8 / 4.8, x 512 6.3 / 6.0 / 6.9, 4 x 1024 6.3 / 7.0, 1 x 512 4.1 / 5.0; into
+// cache rows, whose stores wait longer: 32 x 160 6.6 / 7.9 / 7.0, x 192 8.2 / 7.9 / 7.1, 16 x 256 6.0 / 6.5 / 6.5, x 384 8.2 / 7.0 / 7.2, 8 x 512 6.6 / 6.4 / 7.4.
+static bool rope_many(const int64_t heads, const int64_t tokens, const bool store) { return heads >= 6 && tokens >= 128 && (store ? heads * tokens > 5120 : heads * tokens >= 4096); }
+static unsigned rope_groups(const int64_t heads, const int64_t tokens) { return heads >= 24 && tokens <= 512 ? 2u : 1u; }
+template <bool F16IO> __global__ void __launch_bounds__(256) k_rope_heads(const tdesc a, const tdesc pos, const float * __restrict__ ff, const tdesc d, const rope_params p,
                                                                 const float theta_scale, const float corr0, const float corr1) {
     // grid: (share of the heads, token i2, batch i3)
     const int64_t i2 = blockIdx.y, i3 = blockIdx.z;
     const float pos_f = (float) *(const int32_t *) (pos.data + i2 * pos.nb[0]);
     const char * src = a.data + i2 * a.nb[2] + i3 * a.nb[3];  // (in place, when the allocator made it so)
     char * dst = d.data + i2 * d.nb[2] + i3 * d.nb[3];
-    rope_heads<NH>(p, pos_f, ff, rope_consts{theta_scale, p.freq_scale, p.ext_factor, p.attn_factor, corr0, corr1}, F16IO ? p.n_dims : (int) a.ne[0], (int) a.ne[1], (int) (blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)),
+    rope_heads(p, pos_f, ff, rope_consts{theta_scale, p.freq_scale, p.ext_factor, p.attn_factor, corr0, corr1}, F16IO ? p.n_dims : (int) a.ne[0], (int) a.ne[1], (int) (blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)),
                (int) (gridDim.x * (blockDim.x >> 6)), [&](const int h, const int i) { return F16IO ? h2f(((const uint16_t *) (src + h * a.nb[1]))[i]) : ((const float *) (src + h * a.nb[1]))[i]; },
                [&](const int h, const int i, const float v) {
                    if (F16IO) ((uint16_t *) (dst + h * d.nb[1]))[i] = f2h(v);
@@ -1877,13 +1914,13 @@ void launch_rope(hipStream_t s, const tdesc & a, const tdesc & pos, const float 
         else hipLaunchKernelGGL(k_rope_multi<false>, grid, dim3(64), 0, s, a, (const int32_t *) pos.data, ff, d, p, theta_scale, c0, c1);
         return;
     }
-    grid.x = rope_grid(a.ne[1], a.ne[2] * a.ne[3]);
-    const bool many = rope_many(a.ne[2] * a.ne[3]);
+    const bool many = rope_many(a.ne[1], a.ne[2] * a.ne[3], false);
+    if (many) grid.x = rope_groups(a.ne[1], a.ne[2] * a.ne[3]);
     if (a.type == GGML_TYPE_F16) {
-        if (many) hipLaunchKernelGGL((k_rope<true, 4>), grid, dim3(256), 0, s, a, pos, ff, d, p, theta_scale, c0, c1);
-        else hipLaunchKernelGGL((k_rope<true, 1>), grid, dim3(64), 0, s, a, pos, ff, d, p, theta_scale, c0, c1);
-    } else if (many) hipLaunchKernelGGL((k_rope<false, 4>), grid, dim3(256), 0, s, a, pos, ff, d, p, theta_scale, c0, c1);
-    else hipLaunchKernelGGL((k_rope<false, 1>), grid, dim3(64), 0, s, a, pos, ff, d, p, theta_scale, c0, c1);
+        if (many) hipLaunchKernelGGL(k_rope_heads<true>, grid, dim3(256), 0, s, a, pos, ff, d, p, theta_scale, c0, c1);
+        else hipLaunchKernelGGL(k_rope<true>, grid, dim3(64), 0, s, a, pos, ff, d, p, theta_scale, c0, c1);
+    } else if (many) hipLaunchKernelGGL(k_rope_heads<false>, grid, dim3(256), 0, s, a, pos, ff, d, p, theta_scale, c0, c1);
+    else hipLaunchKernelGGL(k_rope<false>, grid, dim3(64), 0, s, a, pos, ff, d, p, theta_scale, c0, c1);
 }
 
 // ROPE whose only reader is the SET_ROWS of a cache: the rotated head goes straight into its cache row (k_rope's arithmetic, then ONE rounding to the
@@ -1894,13 +1931,33 @@ __device__ __forceinline__ void store_as(char * __restrict__ row, const int type
     else if (type == GGML_TYPE_BF16) ((uint16_t *) row)[i] = f2bf(v);
     else ((uint16_t *) row)[i] = f2h(v);
 }
-template <int NH> __global__ void __launch_bounds__(256) k_rope_store(const tdesc a, const tdesc pos, const float * __restrict__ ff, const int64_t * __restrict__ idx, char * __restrict__ cache, const int64_t cache_nb1, const int cache_type,
+__global__ void __launch_bounds__(64) k_rope_store(const tdesc a, const tdesc pos, const float * __restrict__ ff, const int64_t * __restrict__ idx, char * __restrict__ cache, const int64_t cache_nb1, const int cache_type,
+                                                   const rope_params p, const float theta_scale, const float corr0, const float corr1) {
+    const int64_t i1 = blockIdx.x, i2 = blockIdx.y;
+    const int n_pairs = p.n_dims / 2;
+    const float pos_f = (float) *(const int32_t *) (pos.data + i2 * pos.nb[0]);
+    const float * __restrict__ src = (const float *) (a.data + i1 * a.nb[1] + i2 * a.nb[2]);
+    char * __restrict__ row = cache + idx[i2] * cache_nb1;
+    const int64_t base = i1 * a.ne[0];
+    const bool neox = (p.mode & GGML_ROPE_TYPE_NEOX) != 0;
+    for (int ip = threadIdx.x; ip < n_pairs; ip += blockDim.x) {
+        const int ia = neox ? ip : 2 * ip, ib = neox ? ip + n_pairs : 2 * ip + 1;
+        const float x0 = src[ia], x1 = src[ib];
+        float cs, sn;
+        rope_angle(p, ip, pos_f, p.exact_freq == 2 ? ff : nullptr, rope_consts{theta_scale, p.freq_scale, p.ext_factor, p.attn_factor, corr0, corr1}, cs, sn);
+        store_as(row, cache_type, base + ia, x0 * cs - x1 * sn);
+        store_as(row, cache_type, base + ib, x0 * sn + x1 * cs);
+    }
+    for (int64_t i0 = p.n_dims + threadIdx.x; i0 < a.ne[0]; i0 += blockDim.x) store_as(row, cache_type, base + i0, src[i0]);
+}
+// ... for more tokens, by groups of four waves a token (rope_many)
+__global__ void __launch_bounds__(256) k_rope_heads_store(const tdesc a, const tdesc pos, const float * __restrict__ ff, const int64_t * __restrict__ idx, char * __restrict__ cache, const int64_t cache_nb1, const int cache_type,
                                                     const rope_params p, const float theta_scale, const float corr0, const float corr1) {
     const int64_t i2 = blockIdx.y;
     const float pos_f = (float) *(const int32_t *) (pos.data + i2 * pos.nb[0]);
     const char * src = a.data + i2 * a.nb[2];
     char * row = cache + idx[i2] * cache_nb1;
-    rope_heads<NH>(p, pos_f, p.exact_freq == 2 ? ff : nullptr, rope_consts{theta_scale, p.freq_scale, p.ext_factor, p.attn_factor, corr0, corr1}, (int) a.ne[0], (int) a.ne[1], (int) (blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)),
+    rope_heads(p, pos_f, p.exact_freq == 2 ? ff : nullptr, rope_consts{theta_scale, p.freq_scale, p.ext_factor, p.attn_factor, corr0, corr1}, (int) a.ne[0], (int) a.ne[1], (int) (blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)),
                (int) (gridDim.x * (blockDim.x >> 6)), [&](const int h, const int i) { return ((const float *) (src + h * a.nb[1]))[i]; },
                [&](const int h, const int i, const float v) { store_as(row, cache_type, h * a.ne[0] + i, v); });
 }
@@ -1908,9 +1965,10 @@ void launch_rope_store(hipStream_t s, const tdesc & a, const tdesc & pos, const 
     if (a.ne[1] * a.ne[2] == 0) return;
     float theta_scale, c0, c1;
     rope_host_consts(p, theta_scale, c0, c1);
-    const dim3 grid(rope_grid(a.ne[1], a.ne[2]), (unsigned) a.ne[2]);
-    if (rope_many(a.ne[2])) hipLaunchKernelGGL(k_rope_store<4>, grid, dim3(256), 0, s, a, pos, ff, idx, cache.data, cache.nb[1], cache.type, p, theta_scale, c0, c1);
-    else hipLaunchKernelGGL(k_rope_store<1>, grid, dim3(64), 0, s, a, pos, ff, idx, cache.data, cache.nb[1], cache.type, p, theta_scale, c0, c1);
+    const bool many = rope_many(a.ne[1], a.ne[2], true);
+    const dim3 grid(many ? rope_groups(a.ne[1], a.ne[2]) : (unsigned) a.ne[1], (unsigned) a.ne[2]);
+    if (many) hipLaunchKernelGGL(k_rope_heads_store, grid, dim3(256), 0, s, a, pos, ff, idx, cache.data, cache.nb[1], cache.type, p, theta_scale, c0, c1);
+    else hipLaunchKernelGGL(k_rope_store, grid, dim3(64), 0, s, a, pos, ff, idx, cache.data, cache.nb[1], cache.type, p, theta_scale, c0, c1);
 }
 // ------------------------------------------------------------------------------------------------ fused steps of models with token shift / latent attention
 // (each one the arithmetic of the unfused nodes it replaces, operation by operation: fused and unfused graphs agree bit for bit)

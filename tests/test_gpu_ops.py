@@ -1583,3 +1583,54 @@ def test_rope_of_many_tokens_has_the_bits_of_few(backend, H, mode, D, n_dims, he
     for b in range(batches):
         for lo, hi in ((0, 60), (60, T_)):
             assert np.array_equal(whole[b : b + 1, lo:hi], run(b, b + 1, lo, hi)), (b, lo)
+
+
+# ... heads x tokens at which a token gets one or two groups of four waves: heads that are no whole share of them, a tail, several batches in one
+@pytest.mark.parametrize("mode", [0, L.ROPE_NEOX])
+@pytest.mark.parametrize("D,n_dims,heads,T_,batches,t16", [(64, 64, 8, 512, 1, False), (128, 64, 9, 229, 1, False), (96, 20, 18, 150, 1, True), (128, 128, 24, 180, 1, False), (40, 12, 31, 140, 1, False), (160, 160, 33, 64, 2, True)])
+def test_rope_in_groups_of_four_waves_has_the_bits_of_one(backend, H, mode, D, n_dims, heads, T_, batches, t16):
+    rng = np.random.default_rng(D + heads)
+    x = rng.standard_normal((batches, T_, heads, D)).astype(np.float16 if t16 else np.float32)
+    pos = rng.integers(0, 3000, T_).astype(np.int32)
+
+    def run(b0, b1, lo, hi):
+        def f(g):
+            t = g.new(L.F16 if t16 else L.F32, [D, heads, hi - lo, b1 - b0], np.ascontiguousarray(x[b0:b1, lo:hi]))
+            return H.ggml_rope_ext(g.ctx, t, g.new(L.I32, [hi - lo], pos[lo:hi]), None, n_dims, mode, 4096, 10000.0, 1.0, 0.0, 1.0, 32.0, 1.0)
+        return np.asarray(T.run_case(f, backend)[0]).reshape(b1 - b0, hi - lo, heads, D)
+
+    whole = run(0, batches, 0, T_)
+    for b in range(batches):
+        for lo in range(0, T_, 100):  # (fewer than 128 tokens: a wave a head)
+            hi = min(lo + 100, T_)
+            assert np.array_equal(whole[b : b + 1, lo:hi], run(b, b + 1, lo, hi)), (b, lo)
+
+
+# ... and the same straight into cache rows (a rotated head whose only reader is the store), beside the store as a launch of its own
+@pytest.mark.parametrize("mode", [0, L.ROPE_NEOX])
+@pytest.mark.parametrize("t", [L.BF16, L.F32])
+@pytest.mark.parametrize("D,n_dims,heads,T_,exact", [(128, 64, 8, 512, 1), (128, 64, 33, 130, 1), (96, 20, 18, 240, 0), (64, 64, 9, 460, 0), (128, 128, 24, 180, 1), (128, 64, 4, 200, 1)])
+def test_rope_in_groups_of_four_waves_into_cache_rows_has_the_bits_of_one(backend, H, mode, t, D, n_dims, heads, T_, exact):
+    rng = np.random.default_rng(D + heads)
+    x = rng.standard_normal((T_, heads, D)).astype(np.float32)
+    pos, rows = rng.integers(0, 3000, T_).astype(np.int32), rng.permutation(T_ + 20)[:T_].astype(np.int64)
+    size = 4 if t == L.F32 else 2
+
+    def run(lo, hi):
+        def f(g):
+            y = H.ggml_rope_ext(g.ctx, g.new(L.F32, [D, heads, hi - lo], np.ascontiguousarray(x[lo:hi])), g.new(L.I32, [hi - lo], pos[lo:hi]), None, n_dims, mode, 4096, 10000.0, 1.0, 0.0, 1.0, 32.0, 1.0)
+            y.contents.op_params[3] = exact
+            return H.ggml_set_rows(g.ctx, g.new(t, [D * heads, T_ + 20]), H.ggml_reshape_2d(g.ctx, y, D * heads, hi - lo), g.new(L.I64, [hi - lo], rows[lo:hi]))
+        return np.ascontiguousarray(T.run_case(f, backend)[0]).view(np.uint8).reshape(T_ + 20, D * heads * size)
+
+    n0 = backend.stat("fused_nodes")
+    whole = run(0, T_)
+    assert backend.stat("fused_nodes") == n0 + 1
+    for lo in range(0, T_, 100):  # (fewer than 128 tokens: a wave a head)
+        hi = min(lo + 100, T_)
+        assert np.array_equal(whole[rows[lo:hi]], run(lo, hi)[rows[lo:hi]]), lo
+    backend.set_option("fusion", 0)
+    try:
+        assert np.array_equal(whole, run(0, T_))
+    finally:
+        backend.set_option("fusion", 1)
