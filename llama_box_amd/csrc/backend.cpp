@@ -915,6 +915,7 @@ static int64_t api_get_stat(ggml_backend_t be, const char * key) {
     if (k == "skinny_launches") return c->st.skinny_launches;
     if (k == "wide_launches") return c->st.wide_launches;
     if (k == "wide_few_launches") return c->st.wide_few_launches;
+    if (k == "mm_tile") return c->st.mm_tile;
     if (k == "tiled_launches") return c->st.tiled_launches;
     if (k == "rope_epilogues") return c->st.rope_epilogues;
     if (k.rfind("ip_", 0) == 0) return ip_stat(c, key);

@@ -148,6 +148,7 @@ struct stats {
     int64_t wide_launches = 0;         // prompt-batch mat-muls served by its wide forms (k_mmq_wide, k_mmq_wide_few)
     int64_t wide_few_launches = 0;     // ... by k_mmq_wide_few (few columns: K slices, Q6_K too)
     int64_t tiled_launches = 0;        // batch mat-muls served by the LDS-tiled int8 GEMM (mmq_i8.hip)
+    int64_t mm_tile = 0;               // form of the last 16-bit matrix product on mmf_tile.hip: stages * 10^6 + columns * 1000 + rows
     int64_t nf_mma_chains = 0;         // non-flash K.q -> SOFT_MAX -> V^T.p chains of a prompt micro-batch served by the two-pass matrix-core kernel (round 4)
     int64_t fa_list_launches = 0;      // FLASH_ATTN_EXT nodes served over per-token position lists (2..32 tokens; 33..256 when the mask is known to be sparse)
     int64_t rope_epilogues = 0;        // batches whose rope + KV-cache stores rode in the skinny QKV launches

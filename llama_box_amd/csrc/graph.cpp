@@ -1949,7 +1949,7 @@ static bool try_merge_mm_16(exec_state & st, int i) {
             bytes += (double) ggml_abi_nbytes(w);
         }
         timed_scope ts(c, "mul_mat_f_siblings", bytes);
-        launch_mul_mat_tile(c->stream, n0->src[0]->type, m, (int) ms.size(), K, M, x16);
+        c->st.mm_tile = launch_mul_mat_tile(c->stream, n0->src[0]->type, m, (int) ms.size(), K, M, x16);
         c->st.kernel_launches++;
         for (size_t q = 1; q < ms.size(); ++q) { mark_done(st, ms[q]); c->st.fused_nodes++; }
         return true;
@@ -2825,7 +2825,7 @@ static int run_node(exec_state & st, int i) {
                 const void * x16 = rounded_src1(st, b, a->type);
                 const mul_mat_tile_desc m{a->data, (int64_t) a->nb[1], a->ne[1], n->data, (int64_t) n->nb[1]};
                 timed_scope ts(c, "mul_mat_f", (double) ggml_abi_nbytes(a));
-                launch_mul_mat_tile(s, a->type, &m, 1, a->ne[0], b->ne[1], x16);
+                c->st.mm_tile = launch_mul_mat_tile(s, a->type, &m, 1, a->ne[0], b->ne[1], x16);
                 c->st.kernel_launches++;
                 return 1;
             }

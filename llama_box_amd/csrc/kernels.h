@@ -177,7 +177,7 @@ struct copy16 {
 void launch_mul_mat_id_tile(hipStream_t s, const tdesc & as, int64_t n_b, int64_t n_used, int64_t T, const tdesc & d, const int32_t * cnt, const int32_t * off, const int32_t * list, const void * x16);
 bool mul_mat_id_tile_pays(int64_t K, int64_t N, int64_t even);  // ... faster than mmf.hip's form for `even` columns an expert?
 bool mul_mat_id_batched(const tdesc & as, const tdesc & b, const tdesc & ids);  // does launch_mul_mat_id group the columns by expert?
-void launch_mul_mat_tile(hipStream_t s, int type, const mul_mat_tile_desc * m, int n, int64_t K, int64_t M, const void * x16);
+int launch_mul_mat_tile(hipStream_t s, int type, const mul_mat_tile_desc * m, int n, int64_t K, int64_t M, const void * x16);  // returns the form it chose: stages * 10^6 + columns * 1000 + rows
 struct matvec_multi { const char * W[4]; int64_t nb1[4]; int64_t N[4]; float * dst[4]; int blk0[5]; int n; };
 void launch_matvec_bf16_multi(hipStream_t s, matvec_multi mm, const float * x, int64_t K);
 bool mul_mat_bf16_multi_ok(int64_t N, int64_t K, int64_t M);  // one column, or the columns launch_mul_mat_f gives the kernel whose sums the launch below repeats

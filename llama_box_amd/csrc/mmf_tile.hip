@@ -74,7 +74,7 @@ struct mt_args {
 template <bool BF, int TM, int TN, int S, bool ID> __global__ void __launch_bounds__(256, 1) k_mul_mat_tile(const mt_args a) {
     constexpr int MT = TM / 64, NT = TN / 64;
     constexpr int STAGE = (TM + TN) * 128, L = (TM + TN) / 32, Q = L / 4;  // bytes of a stage, DMA instructions per wave and stage, of which the first quarter
-    static_assert(S >= 3 && (S - 1) * L <= 63, "ring");
+    static_assert(S >= 2 && S <= 5 && (S - 1) * L <= 63, "ring");
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int fr = lane & 31, g = lane >> 5;
@@ -146,8 +146,15 @@ template <bool BF, int TM, int TN, int S, bool ID> __global__ void __launch_boun
             if (s < steps)
 #pragma unroll
                 for (int j = 0; j < (s < S - 1 ? L : Q); ++j) issue(s, j);
-        if (steps >= S) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((S - 2) * L + Q) : "memory");
-        else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+        auto landed = [&](const int later) __attribute__((always_inline)) {  // a step's pieces are there once no more than those of the `later` steps behind it may fly (0 .. S - 2 of them)
+            if (later == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            else if (later == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(L) : "memory");
+            else if (later == 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * L) : "memory");
+            else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(3 * L) : "memory");
+        };
+        if (steps >= S) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 2) * L + Q) : "memory");
+        else landed(steps - 1);
+        asm volatile("s_barrier" ::: "memory");
         uint4 xa[2][MT], wb[2][NT];
         auto frags = [&](const int s, const int ks, const int set) __attribute__((always_inline)) {
             const int bo = (s % S) * STAGE + (((2 * ks + g) ^ swz) << 4);
@@ -194,10 +201,12 @@ template <bool BF, int TM, int TN, int S, bool ID> __global__ void __launch_boun
 #pragma unroll
             for (int ks = 0; ks < 4; ++ks) {
                 if (ks < 3) frags(s, ks + 1, (ks + 1) & 1);
+                __builtin_amdgcn_sched_barrier(0);
                 products(ks & 1, 0, 0, 0);
             }
             if (++s >= steps) break;
-            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            landed(steps - 1 - s);
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
             frags(s, 0, 0);
         }
         // lane: src0 row; register i: src1 column (i & 3) + 8 (i >> 2) + 4 g — 32 lanes store a whole 128-byte line
@@ -225,13 +234,20 @@ template <bool BF, int TM, int TN, int S, bool ID> __global__ void __launch_boun
 }
 
 // The tile and its ring: the form whose rounds over the 256 CUs take least.  A round of a form costs the same whatever the shape, in proportion to K (us for K = 4096, weights from
-// memory): 256 x 128 in three stages 66, 128 x 128 in four 43, 128 x 64 in five 33, 64 x 64 in four 23 with one workgroup per CU and 38 with two.  Measured (us; bf16, 512 columns unless
+// memory): 256 x 128 in three stages 66, 128 x 128 in four 43, 128 x 64 and 64 x 128 in five 33, 64 x 64 in four 23 with one workgroup per CU and 38 with two.  Measured (us; bf16, 512 columns unless
 // stated; 256 x 128 / 128 x 128 / 128 x 64 / 64 x 64; before, where a step's first operands were read behind its barrier: 128 x 128 in two stages, 64 x 128 in five or 64 x 64):
 // K 4096 N 14336: 70 / 87 / 117 / 116 (84), N 28672: 139 / 173 / 208 / 227 (161), N 10240: 66 / 85 / 88 / 85 (78), N 6144: 63 / 43 / 59 / 53 (63), N 4096: 62 / 42 / 33 / 38 (34);
 // K 14336 N 4096: 192 / 130 / 96 / 119 (107); K 8192 N 2048: 107 / 71 / 51 / 39 (56); K 2048 N 8192: 40 / 28 / 39 / 39 (39), N 2048: 33 / 19 / 14 / 11 (17); 256 columns, K 4096 N 14336:
 // 69 / 50 / 63 / 69 (65); 128 columns, N 14336: 60 / 49 / 38 / 42 (39), N 4096: 56 / 42 / 31 / 23 (23).  What bounds a round: from memory a CU fetches at most 50 KB per us however deep
 // the ring (142 from L2), so a tile's share of src0 is 0.3 us a step whatever its columns.
-static void mt_pick(const mul_mat_tile_desc * m, int n, int64_t M, int * tm, int * tn) {
+// Rows of fewer than 1024 values (MT_SHORT): a round is its latencies and the stores behind it, which only other workgroups of the CU hide, so more of them take turns: 64 x 64 in four stages while the CUs
+// have two each, in three (three each) beyond, and 128 x 128 in two stages (two each) where its rounds, 1.9 times as long, are that much fewer.  Measured (us with the rounding; 64 x 64 in
+// four / in three / 128 x 128 in two / the form the rounds above would choose): K 128, 6000 x 190 7.7 / 7.8 / 11.4 / 9.1, 12081 x 330 18.1 / 15.8 / 16.4 / 20.4, 24000 x 190 15.9 / 13.9 / 15.6 / 20.0,
+// 24000 x 512 30.9 / 27.2 / 23.8 / 29.7; K 448, 2638 x 512 10.5 / 10.5 / 15.6 / 11.5, 24000 x 330 33.1 / 30.1 / 33.4 / 38.2, 24000 x 512 47.1 / 41.2 / 37.2 / 42.2; K 960, 24000 x 330 48.4 / 47.6 /
+// 50.8 / 53.1, 12081 x 190 23.4 / 22.5 / 26.7 / 21.2; K 1536 the other way: 12081 x 190 30.6 / 30.4 / 35.9 / 26.8.
+constexpr int64_t MT_SHORT = 1024;
+struct mt_form { int tm, tn, stages; };
+static mt_form mt_pick(const mul_mat_tile_desc * m, int n, int64_t K, int64_t M) {
     auto count = [&](int64_t TM, int64_t TN) {
         int64_t t = 0;
         for (int q = 0; q < n; ++q) t += (m[q].N + TN - 1) / TN;
@@ -239,15 +255,19 @@ static void mt_pick(const mul_mat_tile_desc * m, int n, int64_t M, int * tm, int
     };
     auto rounds = [](int64_t c, int64_t at_once) { return (c + at_once - 1) / at_once; };
     const int64_t small = count(64, 64);
-    int64_t best = small <= 256 ? 23 : 38 * rounds(small, 512);
-    *tm = 64;
-    *tn = 64;
-    if (M <= 64) return;  // (wider tiles would be half empty)
-    const struct { int tm, tn, cost; } forms[3] = {{128, 64, 33}, {128, 128, 43}, {256, 128, 66}};
-    for (const auto & f : forms) {
-        const int64_t cost = f.cost * rounds(count(f.tm, f.tn), 256);
-        if (cost < best) { best = cost; *tm = f.tm; *tn = f.tn; }
+    mt_form best = {64, 64, 4};
+    if (M <= 64) return best;  // (wider tiles would be half empty)
+    if (K < MT_SHORT) {
+        if (small > 512) best = rounds(count(128, 128), 512) * 1460 <= small ? mt_form{128, 128, 2} : mt_form{64, 64, 3};  // (1460 = 1.9 x 768)
+        return best;
     }
+    int64_t least = small <= 256 ? 23 : 38 * rounds(small, 512);
+    const struct { mt_form f; int cost; } forms[4] = {{{128, 64, 5}, 33}, {{128, 128, 4}, 43}, {{256, 128, 3}, 66}, {{64, 128, 5}, 33}};
+    for (const auto & o : forms) {
+        const int64_t cost = o.cost * rounds(count(o.f.tm, o.f.tn), 256);
+        if (cost < least) { least = cost; best = o.f; }
+    }
+    return best;
 }
 template <bool BF, int TM, int TN, int S, bool ID> static void mt_launch_t(hipStream_t s, const dim3 grid, const mt_args & a) {
     const size_t lds = (size_t) S * (TM + TN) * 128;
@@ -277,7 +297,8 @@ bool mul_mat_tile_pays(int64_t K, int64_t N, int64_t M) {
 // few columns hardly fill.  The longer K, the earlier the tiles win.  Measured at 1592 shapes of 4 .. 128 experts of 32 .. 4096 rows (us, mmf.hip / tiles): K 64, 64 x 2048 x 16 columns 17.7 / 41.5
 // (every workgroup of 64 x 128 waits for its first stage); K 128 within 10 % from 64 columns on, 1.1 .. 1.5 times as long below; K 192, 128 rows x 32 1.03 times, x 64 0.97; K 256, 8 x 2048 x
 // 16 columns 11.8 / 12.1, x 32 17.0 / 13.5, 64 x 2048 x 2 22.3 / 33.7; K 384, 512 rows x 16 1.0 .. 1.08 times, 1408 rows 0.76 .. 0.94; K 512 at most 1.05 times, 0.4 .. 0.9 mostly; up to 32 rows, which
-// leave half a tile empty, K 512 x 16 1.05 times, x 32 0.94 .. 1.02, K 768 0.95.
+// leave half a tile empty, K 512 x 16 1.05 times, x 32 0.94 .. 1.02, K 768 0.95.  (Drawn with the tiles as they were before their fragments ran ahead of the products; 105 shapes since: 0.99 of that time,
+// 0.91 .. 1.02.)
 bool mul_mat_id_tile_pays(int64_t K, int64_t N, int64_t even) {
     if (N < 64) return K >= 768 || (K >= 512 && even >= 32);
     if (K >= 512) return true;
@@ -290,10 +311,10 @@ void launch_to_16(hipStream_t s, int type, const char * x, int64_t nb1, int64_t 
     if (type == GGML_TYPE_BF16) hipLaunchKernelGGL(k_to_16<true>, grid, dim3(256), 0, s, x, nb1, K / 8, total, (uint4 *) out);
     else hipLaunchKernelGGL(k_to_16<false>, grid, dim3(256), 0, s, x, nb1, K / 8, total, (uint4 *) out);
 }
-void launch_mul_mat_tile(hipStream_t s, int type, const mul_mat_tile_desc * m, int n, int64_t K, int64_t M, const void * x16) {
+int launch_mul_mat_tile(hipStream_t s, int type, const mul_mat_tile_desc * m, int n, int64_t K, int64_t M, const void * x16) {
     mt_args a{};
-    int tm, tn;
-    mt_pick(m, n, M, &tm, &tn);
+    const mt_form f = mt_pick(m, n, K, M);
+    const int tm = f.tm, tn = f.tn;
     int64_t t = 0;
     for (int q = 0; q < 4; ++q) {
         const mul_mat_tile_desc & d = m[q < n ? q : n - 1];
@@ -309,10 +330,13 @@ void launch_mul_mat_tile(hipStream_t s, int type, const mul_mat_tile_desc * m, i
     const bool bf = type == GGML_TYPE_BF16;
 #define MT(TM_, TN_, S_) { if (bf) mt_launch_t<true, TM_, TN_, S_, false>(s, grid, a); else mt_launch_t<false, TM_, TN_, S_, false>(s, grid, a); }
     if (tm == 256) MT(256, 128, 3)
-    else if (tn == 128) MT(128, 128, 4)
+    else if (tm == 128 && tn == 128) { if (f.stages == 2) MT(128, 128, 2) else MT(128, 128, 4) }
+    else if (tn == 128) MT(64, 128, 5)
     else if (tm == 128) MT(128, 64, 5)
+    else if (f.stages == 3) MT(64, 64, 3)
     else MT(64, 64, 4)
 #undef MT
+    return f.stages * 1000000 + tm * 1000 + tn;
 }
 
 void launch_mul_mat_id_tile(hipStream_t s, const tdesc & as, int64_t n_b, int64_t n_used, int64_t T, const tdesc & d, const int32_t * cnt, const int32_t * off, const int32_t * list, const void * x16) {

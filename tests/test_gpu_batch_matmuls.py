@@ -67,15 +67,22 @@ def test_16_bit_matrices_with_batches(backend, H, wt, K, N, M):
     assert np.abs(got - ref).max() <= 6e-8 * np.sqrt(K) * 8
 
 
-# every tile of mmf_tile.hip (256 x 128, 128 x 128, 128 x 64, 64 x 64 columns x rows) with fewer steps of K than its ring has stages, as many, one and two more, and remainders on both sides
-@pytest.mark.parametrize("N,M,stages", [(14401, 500, 3), (9000, 190, 4), (4100, 330, 5), (130, 70, 4)])
-@pytest.mark.parametrize("more", [-1, 0, 1, 2])
-def test_16_bit_tiles_and_their_rings(backend, H, N, M, stages, more):
-    rng = np.random.default_rng(N + M + more)
-    K = 64 * (stages + more)
+# every form of mmf_tile.hip (stages of its ring, tile of columns x rows) with fewer steps of K than its ring has stages, as many, one and two more, and enough for the ring to go round several
+# times, on both sides of the line for short rows; remainders on both sides of the tiles
+@pytest.mark.parametrize("stages,tm,tn,N,M,steps", [(3, 256, 128, 14401, 500, (16, 17, 18, 31)), (4, 128, 128, 9000, 330, (16, 17, 18, 31)), (5, 128, 64, 4100, 330, (16, 17, 18, 31)), (5, 64, 128, 9000, 190, (16, 17, 18, 31)),
+                                                    (4, 64, 64, 2000, 70, (3, 4, 5, 6, 15, 16, 17, 31)), (3, 64, 64, 4161, 520, (2, 3, 4, 5, 15)), (2, 128, 128, 12101, 500, (1, 2, 3, 4, 15))])
+def test_16_bit_tiles_and_their_rings(backend, H, stages, tm, tn, N, M, steps):
+    for n_steps in steps:
+        one_ring(backend, H, stages, tm, tn, N, M, n_steps)
+
+
+def one_ring(backend, H, stages, tm, tn, N, M, steps):
+    rng = np.random.default_rng(N + M + steps)
+    K = 64 * steps
     w = round16((rng.standard_normal((N, K)) / np.sqrt(K)).astype(np.float32), L.BF16)
     x = rng.standard_normal((M, K)).astype(np.float32)
     got = T.run_case(lambda g: H.ggml_mul_mat(g.ctx, g.new(L.BF16, [K, N], bits16(w, L.BF16)), g.new(L.F32, [K, M], x)), backend)[0].reshape(M, N)
+    assert backend.stat("mm_tile") == stages * 1000000 + tm * 1000 + tn
     ref = round16(x, L.BF16).astype(np.float64) @ w.astype(np.float64).T
     assert np.abs(got - ref).max() <= 6e-8 * np.sqrt(K) * 8  # (as above)
 
