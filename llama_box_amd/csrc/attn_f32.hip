@@ -387,9 +387,10 @@ __global__ void __launch_bounds__(256) k_attn_f32_tile(const tdesc q, const tdes
 // K and V rows reach the wave's own LDS by LDS-DMA as they lie (a lane-per-row load of K touches 32 lines an instruction), V is transposed by ds_read_b64_tr_b16 on the way out; a wave needs
 // no barrier: the next block's K is requested when this one's has left LDS, its V when the second product has read this one's.  First the mask of the 32 queries is scanned, row by row, for
 // the blocks that any of them sees, and for those where its terms are not all zero: only these read it again.  Head sizes: multiples of 8 up to 16 DK16 / 32 DVT.
-// What bounds it: the vector ALU, about 350 instructions a block beside 24 matrix ones, with two waves a SIMD.  512 queries x 32 heads of 128 on 8 key heads, the last of n cells (us; before:
-// 32 queries a wave, all cells, V^T staged by the workgroup): n = 512 20.9 (44.5), 1024 33.5 (79.7), 2048 60 (150), 8192 210 (545); 16 heads on 4, n = 2048 52 (143); 2048 queries x 64 heads
-// 319 (525); 64 queries x 16 heads, n = 512 17 (41).
+// What bounds it: the vector ALU, about 350 instructions a block beside 24 matrix ones, with two waves a SIMD; with few cells its chain of round trips (queries and mask, rows, sums), so that each
+// requests all it needs before anything waits.  512 queries x 32 heads of 128 on 8 key heads, the last of n cells (us, launches in a row; in brackets with 32 queries a wave, all cells, V^T staged
+// by the workgroup): n = 512 22.3 (45.8), 1024 35.0 (80.0), 2048 58.3 (147), 8192 205 (569); 16 heads on 4, n = 2048 49.7 (147); 2048 queries x 64 heads 313 (525); 64 queries x 16 heads, n = 512
+// 18.6 (44.8); a first prompt of 128 tokens, 256 cells, 12.0 (19.9), of 32, which see one block, 9.9 (10.0; 11.1 with the four waves meeting and the queries waited for piece by piece).
 typedef __bf16 att_bf8 __attribute__((ext_vector_type(8)));
 typedef float att_f16v __attribute__((ext_vector_type(16)));
 __device__ __forceinline__ uint32_t att_bf16_bits(const float f) {
@@ -462,53 +463,44 @@ __global__ void __launch_bounds__(256, 2) k_attn_mma_bf16(const tdesc q, const t
             }
         }
     };
-    for (int i = threadIdx.x; i < (n_scan + 31) / 32; i += blockDim.x) {
-        bits[i] = 0;
-        mixed[i] = 0;
-    }
-    // the queries as second operands: element group (16 s + 8 g .. + 7) of query n
-    uint4 qf[DK16];
-    {
-        const float * qrow = (const float *) (q.data + (q_live ? tq : 0) * q.nb[1] + h * q.nb[2]);
-        const bool quads = PLAIN && (((uintptr_t) q.data | (uintptr_t) q.nb[1] | (uintptr_t) q.nb[2]) & 15) == 0;  // (uniform)
+    for (int i = threadIdx.x; i < (n_scan + 31) / 32; i += blockDim.x) bits[i] = mixed[i] = n_blk == 1 ? 1 : 0;  // (a lone block is not looked at)
+    // the queries as second operands: element group (16 s + 8 g .. + 7) of query n; all of a row requested ahead of the mask's scan, rounded behind it
+    const float * const qrow = (const float *) (q.data + (q_live ? tq : 0) * q.nb[1] + h * q.nb[2]);
+    float qx[PLAIN ? DK16 : 1][8];
+    if constexpr (PLAIN) {
+        if ((((uintptr_t) q.data | (uintptr_t) q.nb[1] | (uintptr_t) q.nb[2]) & 15) == 0) {  // (uniform)
 #pragma unroll
-        for (int s = 0; s < DK16; ++s) {
-            const int i0 = 16 * s + 8 * g;
-            uint32_t b[4];
-            if (quads) {
-                float4 x = *(const float4 *) (qrow + i0), y = *(const float4 *) (qrow + i0 + 4);
-                if (!q_live) x = y = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                b[0] = att_bf16_pack(x.x, x.y); b[1] = att_bf16_pack(x.z, x.w); b[2] = att_bf16_pack(y.x, y.y); b[3] = att_bf16_pack(y.z, y.w);
-            } else {
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float x = (q_live && i0 + 2 * e < DK) ? qrow[i0 + 2 * e] : 0.0f, y = (q_live && i0 + 2 * e + 1 < DK) ? qrow[i0 + 2 * e + 1] : 0.0f;
-                    b[e] = att_bf16_pack(x, y);
-                }
+            for (int s = 0; s < DK16; ++s) {
+                const float4 x = *(const float4 *) (qrow + 16 * s + 8 * g), y = *(const float4 *) (qrow + 16 * s + 8 * g + 4);
+                qx[s][0] = x.x; qx[s][1] = x.y; qx[s][2] = x.z; qx[s][3] = x.w;
+                qx[s][4] = y.x; qx[s][5] = y.y; qx[s][6] = y.z; qx[s][7] = y.w;
             }
-            qf[s] = make_uint4(b[0], b[1], b[2], b[3]);
+        } else {
+#pragma unroll
+            for (int s = 0; s < DK16; ++s)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) qx[s][e] = qrow[16 * s + 8 * g + e];
         }
     }
-    __syncthreads();
-    {  // a wave reads eight of the 32 rows, 256 cells at a time
+    __syncthreads();  // (bits and mixed are clear)
+    {  // a wave reads eight of the 32 rows, 256 cells at a time; cells behind the last whole four of a row count as seen, with a bias
         const char * const m0 = mask.data + (int64_t) qt * 32 * mask.nb[1];
         const int rows = (int) std::min<int64_t>(32, n_q - (int64_t) qt * 32) - 1;
-        for (int c = 0; c < n_scan; c += 8) {
+        const int64_t n4 = n_kv & ~(int64_t) 3;
+        for (int c = 0; n_blk > 1 && c < n_scan; c += 8) {
             const int64_t j = (int64_t) c * 32 + 4 * lane;
-            float4 t[8];
-#pragma unroll
-            for (int r = 0; r < 8; ++r) {
-                const float * p = (const float *) (m0 + (int64_t) std::min(8 * wave + r, rows) * mask.nb[1]);
-                if (j + 4 <= n_kv) t[r] = *(const float4 *) (p + j);
-                else t[r] = make_float4(j < n_kv ? p[j] : -INFINITY, j + 1 < n_kv ? p[j + 1] : -INFINITY, j + 2 < n_kv ? p[j + 2] : -INFINITY, -INFINITY);
-            }
             bool any = false, odd = false;
+            float4 t[8];  // (no branch between the eight loads: lanes past the end read the row's last four)
+#pragma unroll
+            for (int r = 0; r < 8; ++r) t[r] = *(const float4 *) (m0 + (int64_t) std::min(8 * wave + r, rows) * mask.nb[1] + std::min(j, n4 - 4) * 4);
 #pragma unroll
             for (int r = 0; r < 8; ++r) {
                 any |= t[r].x > -INFINITY || t[r].y > -INFINITY || t[r].z > -INFINITY || t[r].w > -INFINITY;
                 odd |= t[r].x != 0.0f || t[r].y != 0.0f || t[r].z != 0.0f || t[r].w != 0.0f;
             }
-            uint64_t va = __ballot(any), vo = __ballot(odd);  // eight lanes a block
+            any = j < n4 ? any : j < n_kv;
+            odd |= j >= n4;
+            const uint64_t va = __ballot(any), vo = __ballot(odd);  // eight lanes a block
             uint32_t wa = 0, wo = 0;
 #pragma unroll
             for (int b = 0; b < 8; ++b) {
@@ -522,10 +514,32 @@ __global__ void __launch_bounds__(256, 2) k_attn_mma_bf16(const tdesc q, const t
             }
         }
     }
+    uint4 qf[DK16];
+    {
+        const uint32_t keep = q_live ? 0xFFFFFFFFu : 0u;
+#pragma unroll
+        for (int s = 0; s < DK16; ++s) {
+            const int i0 = 16 * s + 8 * g;
+            uint32_t b[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                if constexpr (PLAIN) b[e] = att_bf16_pack(qx[s][2 * e], qx[s][2 * e + 1]) & keep;
+                else {
+                    const float x = (q_live && i0 + 2 * e < DK) ? qrow[i0 + 2 * e] : 0.0f, y = (q_live && i0 + 2 * e + 1 < DK) ? qrow[i0 + 2 * e + 1] : 0.0f;
+                    b[e] = att_bf16_pack(x, y);
+                }
+            }
+            qf[s] = make_uint4(b[0], b[1], b[2], b[3]);
+        }
+    }
     __syncthreads();
+    // ONE visible block is the first wave's alone, which stores the result itself (uniform)
+    const bool alone = n_blk <= 64 && __builtin_amdgcn_readfirstlane(__builtin_popcount(bits[0]) + (n_blk > 32 ? __builtin_popcount(bits[1]) : 0)) <= 1;
+    if (alone && wave != 0) return;
+    const uint32_t mine = alone ? 0xFFFFFFFFu : 0x11111111u << wave;
     auto next_block = [&](int blk) {  // this wave's first visible block from blk on (n_blk: none); uniform
         while (blk < n_scan) {
-            const uint32_t w = (uint32_t) __builtin_amdgcn_readfirstlane((int) (bits[blk >> 5] & (0x11111111u << wave))) >> (blk & 31);
+            const uint32_t w = (uint32_t) __builtin_amdgcn_readfirstlane((int) (bits[blk >> 5] & mine)) >> (blk & 31);
             if (w) { blk += __builtin_ctz(w); break; }
             blk = (blk | 31) + 1;
         }
@@ -687,6 +701,23 @@ __global__ void __launch_bounds__(256, 2) k_attn_mma_bf16(const tdesc q, const t
         }
         if (blk < n_blk) dma_v(blk);
     }
+    float * out = (float *) (dst.data + h * dst.nb[1] + (q_live ? tq : 0) * dst.nb[2]);
+    auto store = [&](const int d0, const float4 v) {
+        if (PLAIN || d0 + 3 < DV) *(float4 *) (out + d0) = v;
+        else {
+            const float e[4] = {v.x, v.y, v.z, v.w};
+            for (int r = 0; r < 4; ++r) if (d0 + r < DV) out[d0 + r] = e[r];
+        }
+    };
+    if (alone) {
+        if (!q_live) return;
+        const float inv = sgm ? 1.0f : (l > 0.0f ? 1.0f / l : 0.0f);
+#pragma unroll
+        for (int dt = 0; dt < DVT; ++dt)
+#pragma unroll
+            for (int b = 0; b < 4; ++b) store(32 * dt + 8 * b + 4 * g, make_float4(O[dt][4 * b] * inv, O[dt][4 * b + 1] * inv, O[dt][4 * b + 2] * inv, O[dt][4 * b + 3] * inv));
+        return;
+    }
     // the waves' sums, relative to the largest of their references, added in the waves' order; a wave stores DVT of the 4 DVT groups of 8 entries
     if (g == 0) {
         meet[wave][0][n] = m;
@@ -708,18 +739,14 @@ __global__ void __launch_bounds__(256, 2) k_attn_mma_bf16(const tdesc q, const t
     __syncthreads();
     if (!q_live) return;
     const float inv = sgm ? 1.0f : (l > 0.0f ? 1.0f / l : 0.0f);
-    float * out = (float *) (dst.data + h * dst.nb[1] + tq * dst.nb[2]);
 #pragma unroll
     for (int i = 0; i < DVT; ++i) {
         const int gi = wave * DVT + i, d0 = 32 * (gi >> 2) + 8 * (gi & 3) + 4 * g;
         float4 p[W];
 #pragma unroll
         for (int w = 0; w < W; ++w) p[w] = sums[(w * DVT * 4 + gi) * 64 + lane];
-        const float v[4] = {((p[0].x + p[1].x) + (p[2].x + p[3].x)) * inv, ((p[0].y + p[1].y) + (p[2].y + p[3].y)) * inv, ((p[0].z + p[1].z) + (p[2].z + p[3].z)) * inv,
-                            ((p[0].w + p[1].w) + (p[2].w + p[3].w)) * inv};
-        if (PLAIN || d0 + 3 < DV) *(float4 *) (out + d0) = make_float4(v[0], v[1], v[2], v[3]);
-        else
-            for (int r = 0; r < 4; ++r) if (d0 + r < DV) out[d0 + r] = v[r];
+        store(d0, make_float4(((p[0].x + p[1].x) + (p[2].x + p[3].x)) * inv, ((p[0].y + p[1].y) + (p[2].y + p[3].y)) * inv, ((p[0].z + p[1].z) + (p[2].z + p[3].z)) * inv,
+                              ((p[0].w + p[1].w) + (p[2].w + p[3].w)) * inv));
     }
 }
 

@@ -178,6 +178,40 @@ def test_prompts_over_a_bf16_cache(backend, H, n_q, n_kv, heads, kv_heads, dk, d
         assert np.abs(got[:, h] - ref).max() <= 2.0 ** -15 * np.abs(v).max()
 
 
+# up to three visible blocks of 32 cells, near the start and the end of a cache of one block, of up to 64 and of more (a wave alone, or four that meet), rows that are no whole fours, with and without sinks
+@pytest.mark.parametrize("n_kv", [3, 31, 32, 35, 256, 1026, 2048, 2080])
+@pytest.mark.parametrize("blocks", [0, 1, 2, 3])
+@pytest.mark.parametrize("sinks", [False, True])
+def test_prompts_that_see_few_blocks_of_a_bf16_cache(backend, H, n_kv, blocks, sinks):
+    n_q, heads, kv_heads, d = 37, 8, 2, 64
+    rng = np.random.default_rng(n_kv + blocks)
+    r16 = lambda a: (np.ascontiguousarray(a, np.float32).view(np.uint32) & 0xFFFF0000).view(np.float32)
+    bits = lambda a: (np.ascontiguousarray(a, np.float32).view(np.uint32) >> 16).astype(np.uint16)
+    q, k, v = (r16(rng.standard_normal(s) * f) for s, f in (((n_q, heads, d), 2.0), ((n_kv, kv_heads, d), 1.0), ((n_kv, kv_heads, d), 1.0)))
+    sk = rng.standard_normal(heads).astype(np.float32)
+    m = np.full((64, n_kv), -np.inf, np.float32)
+    for b in [b for b in (1, (n_kv - 1) // 32, 4)[:blocks] if 32 * b < n_kv]:
+        m[:n_q, 32 * b : 32 * b + 32] = np.where(rng.random((n_q, min(32, n_kv - 32 * b))) < 0.5, 0.0, -np.inf)
+
+    def build(g):
+        tk, tv = (g.new(L.BF16, [d * kv_heads, n_kv], bits(x)) for x in (k, v))
+        kk, vv = (H.ggml_view_3d(g.ctx, t, d, n_kv, kv_heads, d * kv_heads * 2, d * 2, 0) for t in (tk, tv))
+        r = H.ggml_flash_attn_ext(g.ctx, H.ggml_permute(g.ctx, g.new(L.F32, [d, heads, n_q], q), 0, 2, 1, 3), kk, vv, g.new(L.F32, [n_kv, 64], m), 0.125, 0.0, 0.0)
+        H.ggml_flash_attn_ext_set_prec(r, 10)
+        if sinks:
+            H.ggml_flash_attn_ext_add_sinks(r, g.new(L.F32, [heads], sk))
+        return r
+
+    got = T.run_case(build, backend)[0].reshape(n_q, heads, d)
+    for h in range(heads):
+        z = 0.125 * (q[:, h].astype(np.float64) @ k[:, h // 4].astype(np.float64).T) + m[:n_q]
+        top = np.maximum(z.max(axis=1, keepdims=True), sk[h] if sinks else -1e300)
+        w = np.exp(z - top)
+        den = w.sum(axis=1, keepdims=True) + (np.exp(sk[h] - top) if sinks else 0.0)
+        ref = np.where(den > 0, w, 0.0) / np.where(den > 0, den, 1.0) @ v[:, h // 4].astype(np.float64)
+        assert np.abs(got[:, h] - ref).max() <= 2.0 ** -15 * np.abs(v).max()  # (as above)
+
+
 # heads of 64 whose only reader is a Q8_0 product on the matrix cores: the combine pass leaves the product's quantised blocks — tokens on lists (9 .. 32) and prompts, 2 .. 8 records a row
 @pytest.mark.parametrize("T_,n_kv,NH,NKV,splits", [(9, 640, 8, 2, 0), (16, 2560, 32, 4, 0), (32, 512, 8, 8, 8), (40, 512, 16, 4, 0), (130, 700, 8, 4, 5), (512, 1024, 16, 2, 0)])
 def test_heads_of_64_leave_quantised_rows(backend, H, T_, n_kv, NH, NKV, splits):
