@@ -432,14 +432,17 @@ __global__ void __launch_bounds__(WV * 64) k_fattn_dec128(const tdesc q, const t
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int sub = lane / LPR, sl = lane & (LPR - 1);
     const int ul = sl / G, gl = sl % G;  // the (row group, head) pair this lane owns in the lane-parallel part
-    const int split = blockIdx.x, kvh = blockIdx.y;
+    // (LIST: splits slowest — workgroups go to the XCDs in turn and in this order, and a token with few cells has trips in its first splits only, which come first and on all XCDs this way; with the
+    // splits fastest, those of four splits shared two XCDs and of eight one: Llama-3-8B, us a step, 6 sequences of 130 cells in 8 splits 2587 -> 2540, 15 of 60 in 4 2815 -> 2775, a small model's 24 of
+    // 400 1665 -> 1605.  Drafts of one sequence share its cells and gain nothing; 9 of 6000 3605 -> 3680)
+    const int split = LIST ? blockIdx.z : blockIdx.x, kvh = LIST ? blockIdx.x : blockIdx.y;
     // SKIP (a few query tokens, each seeing its own part of a unified cache): the workgroup first asks the mask whether its
     // token can see anything in its split — one 8-byte load per lane covers 256 positions — and leaves an empty record
     // if not: of the 64 x 32 (split, token) pairs of a -np 32 decode step only ~1/16 touch K/V at all
     // (no batch index, no division: the launcher issues one launch per q.ne[3] slice with the descriptors, the records, the counters and the Q8_K area moved
     // to that slice, and passes the cells per split — the preamble used to fetch its kernel arguments in four dependent rounds around emulated divisions,
     // ~1.9 us between a workgroup's entry and its first K / V request: profiles/r06_fa_stamps.txt)
-    const int tok = (int) blockIdx.z;
+    const int tok = LIST ? (int) blockIdx.y : (int) blockIdx.z;
     constexpr int bat = 0;
     const int per = geo.per;
     const int kv0 = LIST ? 0 : min(split * per, geo.n_kv);
@@ -1121,12 +1124,13 @@ int fattn_pick_splits(const tdesc & q, const tdesc & k, const tdesc * mask, int 
         const int64_t by_len = (trips + 7) / 8, by_occ = std::min<int64_t>(trips, (256 + groups - 1) / groups);
         int64_t n = std::max(by_len, by_occ);
         // ... and with a combine pass anyway, two workgroups a CU (three fit; one with heads of 64), two trips each: the tokens may be drafts of ONE sequence, each of which sees all
-        // n_kv cells (a trip is a round trip to memory, 2 us), and splits a token with fewer cells has no work for cost it next to nothing.  us a step, before / now (splits):
-        // Llama-3-8B, 9 tokens of a sequence of 1500 cells, Q8_0 cache 3157 (3) / 3031 (6), f16 3063 (3) / 2906 (6); 5 of 6000 3340 (7) / 3007 (12); 4 sequences of 1500, 5 tokens
-        // each, 3761 (2) / 3568 (3); a small model with heads of 64, 9 tokens of 1000 1662 (2) / 1430 (7); sequences of their own: 9 of 170 cells 2816 (3) / 2808 (6), 6 of 60
-        // 2524 (2) / 2525 (4) but 2565 (8), 8 of 900 2845 (4) / 2800 (7), small model 16 of 150 1393 (3) / 1393 (4) but 1405 (7).  ONE pass stays one pass: it saves the combine launch.
+        // n_kv cells (a trip is a round trip to memory, 2 us), and splits a token with fewer cells has no work for cost it little, as they come last (k_fattn_dec128: LIST).  us a step,
+        // before / now (splits): Llama-3-8B, 9 tokens of a sequence of 1500 cells, Q8_0 cache 3773 (3) / 3070 (6, rows stored by the projections too), f16 3064 (3) / 2922 (6); 5 of 6000 3328 (7) /
+        // 3045 (12); 4 sequences of 1500, 5 tokens each, 3736 (2) / 3565 (3); 3 of 1000, 7 each, 3499 (2) / 3428 (3); sequences of their own: 6 of 130 cells 2544 (3) / 2546 (8), 13 of 60 2766 (2) /
+        // 2775 (4), 15 of 60 2773 / 2778, 4 of 300 2525 (6) / 2521 (15), 8 of 300 2652 (4) / 2629 (7), 18 of 130 3120 (2) / 3070 (3), 31 of 60 3290 (2) / 3264 (3).  ONE pass stays one pass: it saves
+        // the combine launch.
         const int64_t full = k.ne[0] == 64 ? 256 : 480;
-        if (n > 1) n = std::max(n, std::min((n_kv + 127) / 128, full / groups));
+        if (n > 1) n = std::max({n, std::min((n_kv + 127) / 128, full / groups), (int64_t) (k.ne[0] == 64 ? 2 : 3)});
         return (int) std::max<int64_t>(1, std::min<int64_t>(16, n));
     }
     if (q.ne[1] > 1) {  // a few tokens, other head sizes: short splits
@@ -1420,7 +1424,7 @@ void launch_flash_attn(hipStream_t s, const tdesc & q, const tdesc & k, const td
             const fa_geom geo0 = geo;
             float * const ws0 = ws;
             const int64_t nb_ = q0.ne[3];
-            const dim3 grid((unsigned) geo0.n_splits, (unsigned) geo0.n_kv_head, (unsigned) geo0.n_q);
+            const dim3 grid = list ? dim3((unsigned) geo0.n_kv_head, (unsigned) geo0.n_q, (unsigned) geo0.n_splits) : dim3((unsigned) geo0.n_splits, (unsigned) geo0.n_kv_head, (unsigned) geo0.n_q);
             for (int64_t b = 0; b < nb_; ++b) {
                 tdesc q = q0, k = k0, v = v0, mk = mk0, dst = dst0;
                 fa_geom geo = geo0;
@@ -1457,8 +1461,8 @@ void launch_flash_attn(hipStream_t s, const tdesc & q, const tdesc & k, const td
         geo.q8 = nullptr;
         geo.per = (geo.n_kv + geo.n_splits - 1) / geo.n_splits;
         const tdesc q0 = q, k0 = k, v0 = v, mk0 = mk, dst0 = dst;
-        const dim3 grid((unsigned) geo.n_splits, (unsigned) geo.n_kv_head, (unsigned) geo.n_q);
         const bool list = p.lists != nullptr;  // (2 .. 32 tokens of a -np decode step: each walks the list of its own visible cells, as at head_dim 128)
+        const dim3 grid = list ? dim3((unsigned) geo.n_kv_head, (unsigned) geo.n_q, (unsigned) geo.n_splits) : dim3((unsigned) geo.n_splits, (unsigned) geo.n_kv_head, (unsigned) geo.n_q);
         const int lstride = geo.n_kv + 1;
         const bool wide = !list && geo.n_splits > 1;  // (eight waves: a trip covers 64 / 128 cells)
         for (int64_t b = 0; b < q0.ne[3]; ++b) {  // one launch per batch slice: the kernel has no batch arithmetic
