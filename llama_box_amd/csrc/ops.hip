@@ -1513,12 +1513,14 @@ __device__ __forceinline__ void rope_heads(const rope_params & p, const float po
         }
 }
 // A token's heads: a workgroup of one wave each (k_rope), or one or two groups of four waves a token, whose lanes keep an angle for several heads (k_rope_heads).  The first have the shorter chain and win
-// while the chip holds them at once, up to about 5000; below six heads the groups leave waves without work.  Two groups pay while all of them run at once.  us, launches in a row, heads of 128, 64
-// rotated (a wave a head / one group a token / two): 32 heads x 128 tokens 5.8 / 6.5 / 5.9, x 192 7.7 / 6.7 / 6.4, x 512 13.5 / 8.0 / 8.0, x 1024 23.9 / 12.3 / 14.4, 64 x 512 23.7 / 13.9 / 12.1, 24 x 192
+// while the chip holds them at once, up to about 5000; below six heads the groups leave waves without work.  Two groups pay while the tokens are few.  us, launches in a row, heads of 128, 64
+// rotated (a wave a head / one group a token / two): 32 heads x 128 tokens 5.8 / 6.5 / 5.9, x 192 7.7 / 6.7 / 6.4, x 384 11.1 / 7.6 / 7.3, x 512 13.5 / 8.0 / 8.0 (between other launches of a model 7.9 / 8.3), x 1024 23.9 / 12.3 / 14.4, 24 x 192
 // 6.2 / 6.3 / 6.1, x 256 7.8 / 6.5 / 6.3, 16 x 192 5.1 / 5.5 / 5.7, x 256 5.8 / 5.8 / 6.1, x 384 7.8 / 6.2 / 6.6, 8 x 128 4.3 / 4.8 / 4.8, x 512 6.3 / 6.0 / 6.9, 4 x 1024 6.3 / 7.0, 1 x 512 4.1 / 5.0; into
-// cache rows, whose stores wait longer: 32 x 160 6.6 / 7.9 / 7.0, x 192 8.2 / 7.9 / 7.1, 16 x 256 6.0 / 6.5 / 6.5, x 384 8.2 / 7.0 / 7.2, 8 x 512 6.6 / 6.4 / 7.4.
-static bool rope_many(const int64_t heads, const int64_t tokens, const bool store) { return heads >= 6 && tokens >= 128 && (store ? heads * tokens > 5120 : heads * tokens >= 4096); }
-static unsigned rope_groups(const int64_t heads, const int64_t tokens) { return heads >= 24 && tokens <= 512 ? 2u : 1u; }
+// cache rows, whose stores wait longer: 32 x 160 6.6 / 7.9 / 7.0, x 192 8.2 / 7.9 / 7.1, 16 x 256 6.0 / 6.5 / 6.5, x 384 8.2 / 7.0 / 7.2, 8 x 512 6.6 / 6.4 / 7.4 (in a model 6.6 / 6.2).
+static bool rope_many(const int64_t heads, const int64_t tokens, const bool store) {
+    return heads >= 6 && tokens >= 128 && heads * tokens >= 4096 && (!store || tokens >= 512 || heads * tokens > 5120);
+}
+static unsigned rope_groups(const int64_t heads, const int64_t tokens) { return heads >= 24 && tokens < 512 ? 2u : 1u; }
 template <bool F16IO> __global__ void __launch_bounds__(256) k_rope_heads(const tdesc a, const tdesc pos, const float * __restrict__ ff, const tdesc d, const rope_params p,
                                                                 const float theta_scale, const float corr0, const float corr1) {
     // grid: (share of the heads, token i2, batch i3)
