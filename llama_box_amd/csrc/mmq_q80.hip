@@ -173,7 +173,8 @@ template <bool WP, bool EPI> __global__ void __launch_bounds__(Q80S_WV * 64, 2) 
 // blocks and make one partial sum each, added in wave order: an output has the same bits whatever matrices and columns share the launch.  Per two blocks and 32
 // columns: two v_mfma_i32_32x32x32_i8 for the integer block sums, and ONE v_mfma_f32_32x32x1 (two outer products) for the factors d_w * d_x of all 2 x 1024 outputs —
 // the multiplication that would be a third VALU instruction per output and block, and the row scales need no way through LDS to the accumulator's rows.  Two VALU
-// are left (convert, fused multiply-add): 128 issue cycles per block beside the matrix core's 64, 1.26 POP/s for the chip.  The next step of two blocks is in flight
+// are left (convert, fused multiply-add): 128 issue cycles per block beside the matrix core's 64, which would be 1.26 POP/s for the chip.  The tighter bound is the operands' way: a wave fetches 3 KB
+// for the 2048 outputs of a block, four SIMDs 96 bytes a clock where a CU's L1 gives 64, 0.84 POP/s.  The next step of two blocks is in flight
 // while one is multiplied, three waves per SIMD (160 registers; three steps in flight at two waves per SIMD: 55 us below).  Workgroups that read the same weights
 // (the column tiles of a panel) follow one another on one XCD, so the weights cross HBM once per 1024 columns: an XCD runs about 96 workgroups at once, and 6 panels x 16 tiles draw
 // fewer different operands than 3 x 32 (2048 columns in two groups / in one, 128 x 128 tiles: 14336 x 4096 385 / 571 / 473 us, 4096 x 4096 124 / 175 / 149).
