@@ -82,7 +82,7 @@ static void decode_copy_drop(ggml_backend_buffer_t b, const ggml_tensor * t, siz
     buffer_ctx * c = (buffer_ctx *) b->context;
     if (c->shadow != nullptr && t->data != nullptr) decode_copy_drop(c, (size_t) ((const char *) t->data - (const char *) c->base) + offset, size);
 }
-// (q80_panels: the OTHER second copy — Q8_0 matrices regrouped into the 32-row x 4-block tiles the 9 .. 32-column matrix-core kernel loads with whole-line
+// (q80_panels: the OTHER second copy — Q8_0 matrices regrouped into the 32-row x 4-block tiles the matrix-core kernels load with whole-line
 // wave-instructions, repack.hip: k_repack_q80_panels.  A tensor has one kind of copy: the K-quants planes, Q8_0 panels; same shadow allocation, same invalidation)
 static const uint8_t * second_copy(backend_ctx * c, const ggml_tensor * w, const bool q80_panels) {
     if (!c->opt.decode_copy || w == nullptr || w->view_src != nullptr || w->data == nullptr || w->ne[2] != 1 || w->ne[3] != 1) return nullptr;

@@ -26,6 +26,10 @@ static inline int mmq_min_cols_for(const backend_ctx * c, int wtype) {
     if (c->opt.mmq_min_cols != 3) return c->opt.mmq_min_cols;
     return (wtype == GGML_TYPE_Q4_K || (wtype == GGML_TYPE_Q6_K && !c->mm_q5_major)) ? 2 : 3;
 }
+// Does a batch of M columns take the mat-vec fusions (gate/up/SwiGLU, bias and residual in one launch)?  Left at its default, the option leaves Q8_0 batches to the matrix-core kernel.
+static bool mat_vec_fusions(const backend_ctx * c, const ggml_tensor * w, int64_t M) {
+    return M <= c->opt.mmvq_max_cols && !(c->opt.mmvq_max_cols == 2 && mmq_q80_batch_supported(w->type, w->ne[0], w->ne[1], M));
+}
 static int act_kind(int wtype) { return wtype == GGML_TYPE_Q8_0 ? GGML_TYPE_Q8_0 : GGML_TYPE_Q8_K; }
 static bool is_f32_contig(const ggml_tensor * t) { return t->type == GGML_TYPE_F32 && ggml_abi_is_contiguous(t); }
 static bool rows_contig(const ggml_tensor * t) { return t->nb[0] == ggml_abi_type_size(t->type); }
@@ -549,7 +553,7 @@ static bool single_use(const exec_state & st, const ggml_tensor * t) { return us
 
 // returns the device pointer of src1 quantised for weight type `wtype`, quantising only if the scratch does not
 // already hold exactly this tensor (Q/K/V and gate/up share their input)
-static const void * quantized_src1(exec_state & st, const ggml_tensor * b, int wtype) {  // (wtype MI_ACT_Q80_PANEL: Q8_0 blocks in the panel order of the 9 .. 32-column kernel)
+static const void * quantized_src1(exec_state & st, const ggml_tensor * b, int wtype) {  // (wtype MI_ACT_Q80_PANEL: Q8_0 blocks in the panel order of mmq_q80.hip)
     backend_ctx * c = st.c;
     const int kind = wtype == MI_ACT_Q80_PANEL ? MI_ACT_Q80_PANEL : act_kind(wtype);
     void * dst = (char *) c->ws + st.act_off;
@@ -842,12 +846,11 @@ static bool quant_consumers_only(const exec_state & st, int at, const ggml_tenso
     }
     return true;
 }
-// ... and the same question for Q8_0 weights (round 6): every reader of t is a Q8_0 mat-mul that takes a matrix-core kernel (9 columns and up) (its activations in panel
+// ... and the same question for Q8_0 weights (round 6): every reader of t is a Q8_0 mat-mul that takes a matrix-core kernel (2 columns and up) (its activations in panel
 // order), so a producer may leave Q8_0 panel blocks instead of f32
 static bool q80_panel_consumers_only(const exec_state & st, int at, const ggml_tensor * t) {
     if ((t->flags & GGML_TENSOR_FLAG_OUTPUT) || t->type != GGML_TYPE_F32 || (t->ne[0] % 128) != 0) return false;
     const int64_t M = t->ne[1] * t->ne[2] * t->ne[3];
-    if (M <= st.c->opt.mmvq_max_cols) return false;  // (the mat-vec fusions quantise t themselves, in another order: opt.mmvq_max_cols can reach up here)
     const ggml_cgraph * g = st.g;
     int last = -1, n_cons = 0;
     for (int j = at + 1; j < g->n_nodes; ++j) {
@@ -858,6 +861,7 @@ static bool q80_panel_consumers_only(const exec_state & st, int at, const ggml_t
             if (!(u->op == GGML_OP_MUL_MAT && s == 1 && wt->type == GGML_TYPE_Q8_0 && wt->ne[2] == 1 && wt->ne[3] == 1 && rows_contig(wt) && !buffer_is_split(wt->buffer) &&
                   mmq_q80_batch_supported(wt->type, wt->ne[0], wt->ne[1], M) && u->type == GGML_TYPE_F32 && ggml_abi_is_contiguous(u)))
                 return false;
+            if (mat_vec_fusions(st.c, wt, M)) return false;  // (those quantise t themselves, in another order)
             if (tp_active(st.c) && buffer_is_rowpar(wt->view_src ? wt->view_src->buffer : wt->buffer)) return false;
             last = j;
             n_cons++;
@@ -1445,7 +1449,7 @@ static int try_merge_mm_batch(exec_state & st, int i) {  // returns the number o
     return ms[0].n_nodes;
 }
 
-// Q8_0 weights, 9 columns and up: wq / wk / wv (and gate / up) of a batch multiply the same activations — one launch of the matrix-core
+// Q8_0 weights, 2 columns and up: wq / wk / wv (and gate / up) of a batch multiply the same activations — one launch of the matrix-core
 // kernel over the concatenated 32-row panels (mmq_q80.hip), bias ADDs folded into the store.  The member search is try_merge_mm_batch's (same dependence rules);
 // no K split.  Up to 32 tokens the ropes and cache stores that follow join the launch, beyond that they fuse as they do for the K-quants (try_fuse_rope_store).
 static int try_merge_q80_skinny(exec_state & st, int i) {  // returns the number of nodes consumed at position i (0: not merged)
@@ -2768,7 +2772,7 @@ static int run_node(exec_state & st, int i) {
                         return 2;
                     }
                     static const bool q80_producers = !getenv("GGML_MI355X_Q80_PRODUCERS") || atoi(getenv("GGML_MI355X_Q80_PRODUCERS")) != 0;
-                    if (q80_producers && c->opt.prologue && ggml_abi_nrows(m) >= 9 && st.sk_dst != a && rms_norm_q80_panel_ok(TD(a), (const float *) w->data) && q80_panel_consumers_only(st, i + 1, m)) {
+                    if (q80_producers && c->opt.prologue && ggml_abi_nrows(m) >= 2 && st.sk_dst != a && rms_norm_q80_panel_ok(TD(a), (const float *) w->data) && q80_panel_consumers_only(st, i + 1, m)) {
                         timed_scope ts(c, "rms_norm_mul_quantize_q8_0", (double) ggml_abi_nbytes(a));
                         launch_rms_norm_mul_q80_panel(s, TD(a), ggml_abi_op_param_f32(n, 0), (const float *) w->data, (char *) c->ws + st.act_off);
                         mark_q8_cache(st, m, MI_ACT_Q80_PANEL);
@@ -2872,7 +2876,7 @@ static int run_node(exec_state & st, int i) {
             const bool rowpar = tp_active(c) && buffer_is_rowpar(a->view_src ? a->view_src->buffer : a->buffer);
             const int64_t M = b->ne[1] * b->ne[2] * b->ne[3];
             if (fuse && c->opt.qkv && !rowpar && M == 1 && try_fuse_qkv(st, i)) return 1;
-            if (fuse && !rowpar && M <= c->opt.mmvq_max_cols) {
+            if (fuse && !rowpar && mat_vec_fusions(c, a, M)) {
                 // gate/up/SwiGLU: MUL_MAT(Wg,x) MUL_MAT(Wu,x) GLU(g,u)
                 ggml_tensor * n2 = next(1);
                 ggml_tensor * n3 = next(2);
@@ -3282,7 +3286,7 @@ static int run_node(exec_state & st, int i) {
                 return 1;
             }
             static const bool q80_producers = !getenv("GGML_MI355X_Q80_PRODUCERS") || atoi(getenv("GGML_MI355X_Q80_PRODUCERS")) != 0;
-            if (q80_producers && fuse && c->opt.prologue && ggml_abi_nrows(n) >= 9 && swiglu_q80_panel_ok(TD(a), b ? &bd : nullptr, n->ne[0], n->op_params[1]) && q80_panel_consumers_only(st, i, n)) {
+            if (q80_producers && fuse && c->opt.prologue && ggml_abi_nrows(n) >= 2 && swiglu_q80_panel_ok(TD(a), b ? &bd : nullptr, n->ne[0], n->op_params[1]) && q80_panel_consumers_only(st, i, n)) {
                 timed_scope ts(c, "swiglu_quantize_q8_0", (double) ggml_abi_nbytes(n) * 2);
                 launch_swiglu_q80_panel(s, TD(a), b ? &bd : nullptr, n->ne[0], n->op_params[1], (char *) c->ws + st.act_off);
                 mark_q8_cache(st, n, MI_ACT_Q80_PANEL);
@@ -3654,7 +3658,7 @@ static int run_node(exec_state & st, int i) {
             // ... and the same for a Q8_0 wo on the matrix cores behind heads of 64
             const ggml_tensor * q80_reader = nullptr;
             const float * const sk = n->src[4] ? (const float *) n->src[4]->data : nullptr;
-            if (!q8_reader && fuse && c->opt.prologue && a->ne[1] > 8 && use_count(st, n) == 1 && !(n->flags & GGML_TENSOR_FLAG_OUTPUT) && ggml_abi_is_contiguous(n) && fattn_q80_out_ok(qd, kd, vd, m ? &md : nullptr, sk, TD(n), p)) {
+            if (!q8_reader && fuse && c->opt.prologue && a->ne[1] > 1 && use_count(st, n) == 1 && !(n->flags & GGML_TENSOR_FLAG_OUTPUT) && ggml_abi_is_contiguous(n) && fattn_q80_out_ok(qd, kd, vd, m ? &md : nullptr, sk, TD(n), p)) {
                 for (int k = i + 1; k < std::min(g->n_nodes, i + 4) && !q80_reader; ++k) {
                     const ggml_tensor * t = g->nodes[k];
                     if ((t->op == GGML_OP_RESHAPE || t->op == GGML_OP_VIEW) && t->src[0] == n && t->data == n->data && ggml_abi_is_contiguous(t) && t->ne[0] == n->ne[0] * n->ne[1] &&

@@ -247,10 +247,10 @@ int launch_mmq_i8(hipStream_t s, int type, const uint8_t * W, int64_t w_nb1, int
 bool mmq_skinny_supported(int type, int64_t K, int64_t N, int64_t M, int64_t w_nb1);
 int mmq_skinny_ksplit(int64_t K, int64_t n_total);
 // Q8_0 weights x Q8_0 activations, one int8 MFMA per 32-value block + immediate f32 scale-accumulate (mmq_q80.hip)
-// 9 columns and up: up to 32 with the weights streamed once, above in tiles of 32 rows x 64 columns, or of 128 x 128 where that is faster; activations in panel order
+// 2 columns and up: up to 32 with the weights streamed once, above in tiles of 32 rows x 64 columns, or of 128 x 128 where that is faster; activations in panel order
 bool mmq_q80_batch_supported(int type, int64_t K, int64_t N, int64_t M);
 struct mmq80s_desc { const uint8_t * W; const uint8_t * W_panels; int64_t w_nb1; int N; float * dst; int64_t dst_stride; const float * add; int64_t add_stride; };
-int launch_mmq_q80_multi(hipStream_t s, int n, const mmq80s_desc * mats, int K, int M, const void * act_q80_panel, const mmq_epi * epi = nullptr /* 9 .. 32 columns, three matrices */);  // up to three matrices over the same activations; returns the launches it took
+int launch_mmq_q80_multi(hipStream_t s, int n, const mmq80s_desc * mats, int K, int M, const void * act_q80_panel, const mmq_epi * epi = nullptr /* 2 .. 32 columns, three matrices */);  // up to three matrices over the same activations; returns the launches it took
 void launch_mmq_q80(hipStream_t s, const uint8_t * W, const uint8_t * W_panels, int64_t w_nb1, int K, int N, int M, const void * act_q80_panel, float * dst, int64_t dst_stride, const float * add, int64_t add_stride);
 void launch_mmq(hipStream_t s, int type, const uint8_t * W, int64_t w_nb1, int K, int N, int M, const void * act_q8k, float * dst, int64_t dst_stride, int ksplit, float * part);
 
@@ -369,7 +369,7 @@ struct fattn_params {
     const int * lists = nullptr;  // per-token lists of visible cache positions (launch_fattn_tile_scan), or nullptr
     void * q8_out = nullptr;  // the result's only readers are quantised mat-muls (wo of a batch): leave it as Q8_K blocks here — honoured by
                               // the combine pass of the head_dim-128 kernels (n_splits > 1), see fattn_q8_out_ok()
-    void * q80_out = nullptr; // ... by Q8_0 mat-muls of 9 columns and up: as Q8_0 blocks in panel order, by the combine pass of the head_dim-64 kernels, see fattn_q80_out_ok()
+    void * q80_out = nullptr; // ... by Q8_0 mat-muls of 2 columns and up: as Q8_0 blocks in panel order, by the combine pass of the head_dim-64 kernels, see fattn_q80_out_ok()
     unsigned * arrive = nullptr;  // zeroed counters (arrive_slots of them): lets the split kernel of the head_dim-128 decode path merge its own
     int arrive_slots = 0;         // partial records (last workgroup to arrive) instead of a second launch; the kernel leaves them at zero
     const uint8_t * tile_vis = nullptr;  // matrix-core kernel: [q tile of 32][kv tile of 64] visibility bytes (launch_fattn_vis_scan), or nullptr
@@ -409,7 +409,7 @@ void launch_flash_attn_combine(hipStream_t s, int D, const float * ws, const flo
 // ---- the decode copy (repack.hip): rows [r0, r0 + n_rows) of a K-quant [K, N] matrix from the block layout at `src` into the plane layout at `dst` (same row stride)
 bool repack_supported(int type, int64_t K, int64_t nb1);
 void launch_repack_planes(hipStream_t s, int type, const void * src, void * dst, int64_t K, int64_t nb1, int64_t r0, int64_t n_rows);
-bool repack_q80_supported(int type, int64_t K, int64_t N, int64_t nb1);  // Q8_0: the panel copy of the 9 .. 32-column matrix-core kernel (repack.hip)
+bool repack_q80_supported(int type, int64_t K, int64_t N, int64_t nb1);  // Q8_0: the panel copy of the matrix-core kernels (repack.hip)
 void launch_repack_q80_panels(hipStream_t s, const void * src, void * dst, int64_t K, int64_t N, int64_t nb1);
 
 // ---- layers with state per sequence (seq.hip): short convolutions over a sequence's history and three recurrences over a matrix state per head

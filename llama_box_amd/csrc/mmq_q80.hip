@@ -1,4 +1,4 @@
-// mmq_q80.hip — batched mat-mul (9 columns and up) for Q8_0 weights on the gfx950 INTEGER matrix cores.
+// mmq_q80.hip — batched mat-mul (2 columns and up) for Q8_0 weights on the gfx950 INTEGER matrix cores.
 //
 // ggml-cpu's ggml_vec_dot_q8_0_q8_0 quantises the activations to Q8_0 as well and sums,
 // per 32-value block, sumi * (d_w * d_x) in f32.  A block is exactly the K extent of v_mfma_i32_32x32x32_i8, so one MFMA
@@ -25,7 +25,9 @@ typedef int int4q __attribute__((ext_vector_type(4)));
 typedef int int16q __attribute__((ext_vector_type(16)));
 typedef float float32q __attribute__((ext_vector_type(32)));
 
-// ------------------------------------------------------------------------------------------------ 9 .. 32 columns
+// ------------------------------------------------------------------------------------------------ 2 .. 32 columns
+// (Two to eight took 2-, 4- and 8-column mat-vec passes, with launches of their own for norm, quantiser, SwiGLU, rotation and stores.  A step of TinyLlama, 2 / 4 / 8 sequences of 200 tokens:
+// 1706 / 2265 / 2832 us; on this kernel, fused as the wider batches are, 1251 / 1253 / 1303; with 16 rows a workgroup where that is faster, below, 1117 / 1114 / 1158.)
 // A -np decode step of a Q8_0 model (as 8-column mat-vec passes the weights streamed once per pass: 61 us per matrix of Llama-3-8B Q8_0 at 32 columns, a 16 ms
 // step).  Here the WEIGHTS stream once: a workgroup owns 32 weight rows, its eight waves take the K range in interleaved chunks of four blocks (128 values:
 // one cache line of every row), one v_mfma_i32_32x32x32_i8 per block gives the 32 x 32 integer block sums, and the f32 scale-accumulate follows
@@ -49,6 +51,40 @@ struct mmq80s_args {    // up to three matrices over the same activations in one
 };
 typedef uint32_t __attribute__((ext_vector_type(4), aligned(2))) q80s_u32x4_a2;
 typedef uint32_t __attribute__((ext_vector_type(4), aligned(4))) q80s_u32x4_a4;
+
+// the sum v of column m and row n (of matrix mi), a row a lane: into the result, or (EPI) through the rotation into where its kind goes.  Every lane of a wave comes here.
+// Q8: kinds 5 and 6 are among them; 32 lanes hold the rows of a block
+template <bool EPI, bool Q8> __device__ __forceinline__ void q80s_result(const mmq80s_args & a, const mmq80s_mat & mt, const mmq_epi & epi, const int mi, const int m, const int n, float v) {
+    if (!EPI && (m >= a.M || n >= mt.N)) return;
+    const int tk = min(m, a.M - 1);
+    if (mt.add) v += mt.add[(size_t) tk * mt.add_stride + n];
+    if constexpr (!EPI) mt.dst[(size_t) m * mt.dst_stride + n] = v;
+    else {
+        const float partner = __shfl_xor(v, 1);  // the other element of the rotation pair
+        const int kind = epi.kind[mi], head = n / epi.head_dim, dd = n - head * epi.head_dim;
+        char * const out = epi.out[mi];
+        float x = v;
+        if ((kind < 3 || kind == 5) && dd < epi.n_dims) {
+            const float2 t = *(const float2 *) (epi.tab + ((size_t) tk * (epi.n_dims >> 1) + (dd >> 1)) * 2);
+            const float x0 = (dd & 1) ? partner : v, x1 = (dd & 1) ? v : partner;
+            x = (dd & 1) ? x0 * t.y + x1 * t.x : x0 * t.x - x1 * t.y;
+        }
+        float amax = fabsf(x);
+        if (Q8 && kind >= 5) {  // (uniform) the 32 rows are one Q8_0 block of the cache row
+#pragma unroll
+            for (int o = 1; o < 32; o <<= 1) amax = fmaxf(amax, __shfl_xor(amax, o));
+        }
+        if (m >= a.M) return;
+        if (kind == 1) *(float *) (out + (int64_t) head * epi.nb1[mi] + (int64_t) m * epi.nb2[mi] + (int64_t) dd * 4) = x;
+        else if (kind == 4) ((uint16_t *) out)[epi.v_idx[(int64_t) m * mt.N + n]] = f2h(x);
+        else if (Q8 && kind >= 5) {
+            const float d8 = amax / 127.0f, id8 = d8 != 0.0f ? 1.0f / d8 : 0.0f;
+            char * const blk = out + epi.idx[m] * epi.nb1[mi] + (n >> 5) * 34;
+            blk[2 + (n & 31)] = (char) (int) roundf(x * id8);
+            if ((n & 31) == 0) *(uint16_t *) blk = f2h(d8);
+        } else ((uint16_t *) (out + epi.idx[m] * epi.nb1[mi]))[n] = f2h(x);
+    }
+}
 
 constexpr int Q80S_WV = 8;
 // EPI: wq / wk / wv of a batch whose rotation and cache stores follow — done here, as in the K-quants' epilogue (mmq_skinny.hip; the arithmetic of k_rope_qk_store).  16 tokens of TinyLlama: the
@@ -136,35 +172,114 @@ template <bool WP, bool EPI> __global__ void __launch_bounds__(Q80S_WV * 64, 2) 
         float v = red[0][r][l];
 #pragma unroll
         for (int w = 1; w < Q80S_WV; ++w) v += red[w][r][l];
-        if (!EPI && (m >= a.M || n >= mt.N)) continue;
-        const int tk = min(m, a.M - 1);
-        if (mt.add) v += mt.add[(size_t) tk * mt.add_stride + n];
-        if constexpr (!EPI) mt.dst[(size_t) m * mt.dst_stride + n] = v;
-        else {
-            const float partner = __shfl_xor(v, 1);  // the other element of the rotation pair
-            const int kind = epi.kind[mi], head = n / epi.head_dim, dd = n - head * epi.head_dim;
-            char * const out = epi.out[mi];
-            float x = v;
-            if ((kind < 3 || kind == 5) && dd < epi.n_dims) {
-                const float2 t = *(const float2 *) (epi.tab + ((size_t) tk * (epi.n_dims >> 1) + (dd >> 1)) * 2);
-                const float x0 = (dd & 1) ? partner : v, x1 = (dd & 1) ? v : partner;
-                x = (dd & 1) ? x0 * t.y + x1 * t.x : x0 * t.x - x1 * t.y;
-            }
-            float amax = fabsf(x);
-            if (kind >= 5) {  // (uniform) the 32 rows are one Q8_0 block of the cache row
+        q80s_result<EPI, true>(a, mt, epi, mi, m, n, v);
+    }
+}
+
+// ------------------------------------------------------------------------------------------------ 2 .. 32 columns, few rows
+// The same product where 32 rows a workgroup leave CUs idle or each wave a chain of dependent round trips: 16 rows and 16 columns (CT: times two) a workgroup on v_mfma_i32_16x16x32_i8, four
+// chunks of a wave in flight at once (18 registers each: 32-row tiles hold one ahead).  A lane fetches 16 bytes of one half of a block for two blocks at a time, 256 consecutive bytes per 16
+// lanes, and v_permlane32_swap turns them into the operands of the two blocks (the K order inside a block is the same on both sides, so the integer sums are).  One v_mfma_f32_16x16x1 (four outer
+// products) gives d_w * d_x of a chunk's four blocks.  The chunks go to the eight sums, and these are added, as above: the same bits.
+template <int CT, bool EPI> __global__ void __launch_bounds__(Q80S_WV * 64, 2) k_mmq_q80_rows16(const mmq80s_args a, const mmq_epi epi) {
+    constexpr int DEPTH = 4;
+    __shared__ float red[Q80S_WV][4 * CT][64];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int fr = lane & 15, q = lane >> 4;
+    const int gp = (int) blockIdx.x >> 1;
+    const int mi = gp < a.m[0].panel_end ? 0 : (gp < a.m[1].panel_end ? 1 : 2);  // (uniform)
+    const mmq80s_mat & mt = a.m[mi];
+    const int panel = gp - (mi ? a.m[mi - 1].panel_end : 0), r0 = 16 * ((int) blockIdx.x & 1);
+    const int nchunk = a.K / 128;
+    const uint8_t * const wp = mt.W + (size_t) panel * nchunk * 4352;
+    const int w_off = (q >> 1) * 1024 + (q & 1) * 512 + (r0 + fr) * 16, dw_off = 4096 + q * 64 + (r0 + fr) * 2;
+    int y_off[CT], dy_off[CT];
 #pragma unroll
-                for (int o = 1; o < 32; o <<= 1) amax = fmaxf(amax, __shfl_xor(amax, o));
-            }
-            if (m >= a.M) continue;
-            if (kind == 1) *(float *) (out + (int64_t) head * epi.nb1[mi] + (int64_t) m * epi.nb2[mi] + (int64_t) dd * 4) = x;
-            else if (kind == 4) ((uint16_t *) out)[epi.v_idx[(int64_t) m * mt.N + n]] = f2h(x);
-            else if (kind >= 5) {
-                const float d8 = amax / 127.0f, id8 = d8 != 0.0f ? 1.0f / d8 : 0.0f;
-                char * const blk = out + epi.idx[m] * epi.nb1[mi] + (n >> 5) * 34;
-                blk[2 + i] = (char) (int) roundf(x * id8);
-                if (i == 0) *(uint16_t *) blk = f2h(d8);
-            } else ((uint16_t *) (out + epi.idx[m] * epi.nb1[mi]))[n] = f2h(x);
+    for (int t = 0; t < CT; ++t) {
+        const int col = min(16 * t + fr, a.M - 1);
+        y_off[t] = (q >> 1) * 1152 + (q & 1) * 512 + col * 16;
+        dy_off[t] = q * 1152 + 1024 + col * 4;
+    }
+    struct chunk { int4q w[2], y[CT][2]; uint32_t dw; float dy[CT]; };
+    auto fetch = [&](const int c, chunk & o) __attribute__((always_inline)) {
+        const uint8_t * const t = wp + (size_t) c * 4352;
+        const char * const yt = a.act + (size_t) c * 4608;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) o.w[u] = *(const int4q *) (t + w_off + u * 2048);
+        o.dw = *(const uint16_t *) (t + dw_off);
+#pragma unroll
+        for (int k = 0; k < CT; ++k) {
+#pragma unroll
+            for (int u = 0; u < 2; ++u) o.y[k][u] = *(const int4q *) (yt + y_off[k] + u * 2304);
+            o.dy[k] = *(const float *) (yt + dy_off[k]);
         }
+    };
+    float C[CT][4];
+#pragma unroll
+    for (int k = 0; k < CT; ++k)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) C[k][r] = 0.0f;
+    const int4q zi = {0, 0, 0, 0};
+    float16q zf;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) zf[r] = 0.0f;
+    auto blocks = [](const int4q v, long & b0, long & b1) __attribute__((always_inline)) {  // lanes 0 .. 31 hold the first block's halves, lanes 32 .. 63 the second's -> 8 bytes of each for every lane
+        const auto x = __builtin_amdgcn_permlane32_swap((unsigned) v[0], (unsigned) v[2], false, false);
+        const auto y = __builtin_amdgcn_permlane32_swap((unsigned) v[1], (unsigned) v[3], false, false);
+        b0 = (long) (((unsigned long) y[0] << 32) | x[0]);
+        b1 = (long) (((unsigned long) y[1] << 32) | x[1]);
+    };
+    auto multiply = [&](const chunk & o) __attribute__((always_inline)) {
+        long w[4];
+        blocks(o.w[0], w[0], w[1]);
+        blocks(o.w[1], w[2], w[3]);
+        const float dw = h2f((uint16_t) o.dw);
+#pragma unroll
+        for (int k = 0; k < CT; ++k) {
+            long y[4];
+            blocks(o.y[k][0], y[0], y[1]);
+            blocks(o.y[k][1], y[2], y[3]);
+            const float16q p = __builtin_amdgcn_mfma_f32_16x16x1f32(o.dy[k], dw, zf, 0, 0, 0);
+#pragma unroll
+            for (int b = 0; b < 4; ++b) {
+                const int4q s = __builtin_amdgcn_mfma_i32_16x16x32_i8(y[b], w[b], zi, 0, 0, 0);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) C[k][r] = __builtin_fmaf((float) s[r], p[4 * b + r], C[k][r]);
+            }
+        }
+    };
+    const int mine = wave < nchunk ? (nchunk - wave + Q80S_WV - 1) / Q80S_WV : 0;  // chunks wave, wave + 8, ..
+    if (mine) {
+        auto at = [&](const int i) { return wave + Q80S_WV * min(i, mine - 1); };  // (past the last: that one again, read and not used)
+        chunk o[DEPTH];
+#pragma unroll
+        for (int d = 0; d < DEPTH; ++d) fetch(at(d), o[d]);
+        __builtin_amdgcn_sched_barrier(0);
+        int i = 0;
+        for (; i + DEPTH < mine; i += DEPTH) {
+#pragma unroll
+            for (int d = 0; d < DEPTH; ++d) {
+                multiply(o[d]);
+                __builtin_amdgcn_sched_barrier(0);  // (the next loads into these registers, and not further down)
+                fetch(at(i + DEPTH + d), o[d]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+#pragma unroll
+        for (int d = 0; d < DEPTH; ++d)
+            if (i + d < mine) multiply(o[d]);
+    }
+#pragma unroll
+    for (int k = 0; k < CT; ++k)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) red[wave][4 * k + r][lane] = C[k][r];
+    __syncthreads();
+    for (int e = tid; e < 256 * CT; e += Q80S_WV * 64) {  // (16 lanes: the 16 rows of one column)
+        const int m = e >> 4, i = e & 15, r = (m >> 4) * 4 + (m & 3), l = ((m >> 2) & 3) * 16 + i;
+        float v = red[0][r][l];
+#pragma unroll
+        for (int w = 1; w < Q80S_WV; ++w) v += red[w][r][l];
+        q80s_result<EPI, false>(a, mt, epi, mi, m, panel * 32 + r0 + i, v);
     }
 }
 
@@ -427,7 +542,7 @@ template <bool WP> __global__ void __launch_bounds__(512, 1) k_mmq_q80_tile(cons
 
 bool mmq_q80_batch_supported(int type, int64_t K, int64_t N, int64_t M) {
     static const bool on = !getenv("GGML_MI355X_Q80_SKINNY") || atoi(getenv("GGML_MI355X_Q80_SKINNY")) != 0;
-    return (on || M > 32) && type == GGML_TYPE_Q8_0 && (K % 128) == 0 && N >= 1 && M >= 9;  // (off: the mat-vec passes up to 32 columns)
+    return (on || M > 32) && type == GGML_TYPE_Q8_0 && (K % 128) == 0 && N >= 1 && M >= 2;  // (off: the mat-vec passes up to 32 columns)
 }
 // Tiles of 128 x 128 instead of the column kernel (N: rows of all matrices of the launch)?  Measured (us, one product with its quantiser, tiles / columns):
 // - K of one or two chunks: from about two million outputs on.  K 128, 5632 x 256 10.8 / 9.2, 4096 x 512 10.6 / 12.5, 14336 x 512 19.9 / 27.4; K 256, 4096 x 384 12.9 / 10.5,
@@ -438,6 +553,17 @@ static bool q80_tile_pays(int64_t K, int64_t N, int64_t M, bool panels) {
     if (K <= 256) return N * M >= ((int64_t) 15 << 17);
     if (!panels) return N * M >= ((int64_t) 5 << 19);
     return K <= 512 && M <= 512 && N * M >= ((int64_t) 7 << 20);
+}
+// 16 rows a workgroup instead of 32 (panels: groups of 32 rows of all matrices of the launch; over panel copies)?  Measured at 16 .. 1000 panels, K 1024 .. 14336, one product with its quantiser
+// (us, 32 rows / 16 rows):
+// - up to 128 panels the 32-row tiles leave half of the CUs idle.  16 columns: K 2048, 64 panels 8.4 / 7.4, K 5632 12.8 / 10.6, K 14336, 128 panels 27.5 / 21.3; K 1024 6.5 / 6.2; 32 columns: K 2048,
+//   64 panels 9.1 / 8.7, K 14336, 128 panels 29.5 / 26.2, but K 1024 6.7 / 7.1.
+// - 129 to 256: one 32-row workgroup a CU against two that share it: K 1024, 160 panels 7.4 / 8.5, K 14336 28.8 / 30.8 (K 4096 13.1 / 12.3).
+// - beyond, up to 16 columns, four chunks in flight a wave against one: K 2048, 352 panels 13.8 / 12.6, K 4096, 448 22.0 / 20.6, 1000 42.4 / 36.5, K 14336, 300 46.5 / 45.0; K 1024, 700 14.1 / 15.3; and at
+//   449 to 512, where the 32-row tiles fill the chip twice, only up to 8 columns: K 8192, 512 panels x 4 36.3 / 34.2, x 16 37.3 / 38.5.  32 columns the other way: K 4096, 352 21.9 / 23.8.
+static bool q80_rows16_pays(int64_t K, int panels, int64_t M) {
+    if (panels <= 128) return M <= 16 || K >= 2048;
+    return panels > 256 && K >= 2048 && M <= (panels > 448 && panels <= 512 ? 8 : 16);
 }
 // n matrices (1 .. 3) over the same activations; returns the launches; panels[q] != nullptr for ALL of them or for none (the template form is per launch)
 int launch_mmq_q80_multi(hipStream_t s, int n, const mmq80s_desc * mats, int K, int M, const void * act_q80, const mmq_epi * epi) {
@@ -455,6 +581,12 @@ int launch_mmq_q80_multi(hipStream_t s, int n, const mmq80s_desc * mats, int K, 
     if (M <= 32) {
         const mmq_epi none{};
         const dim3 grid((unsigned) pe), block(Q80S_WV * 64);
+        if (wp && q80_rows16_pays(K, pe, M) && !(epi && (epi->kind[0] >= 5 || epi->kind[1] >= 5 || epi->kind[2] >= 5))) {
+            const dim3 grid16(2 * (unsigned) pe);
+            if (M <= 16) { if (epi) hipLaunchKernelGGL((k_mmq_q80_rows16<1, true>), grid16, block, 0, s, a, *epi); else hipLaunchKernelGGL((k_mmq_q80_rows16<1, false>), grid16, block, 0, s, a, none); }
+            else { if (epi) hipLaunchKernelGGL((k_mmq_q80_rows16<2, true>), grid16, block, 0, s, a, *epi); else hipLaunchKernelGGL((k_mmq_q80_rows16<2, false>), grid16, block, 0, s, a, none); }
+            return 1;
+        }
         if (epi) { if (wp) hipLaunchKernelGGL((k_mmq_q80_skinny<true, true>), grid, block, 0, s, a, *epi); else hipLaunchKernelGGL((k_mmq_q80_skinny<false, true>), grid, block, 0, s, a, *epi); }
         else { if (wp) hipLaunchKernelGGL((k_mmq_q80_skinny<true, false>), grid, block, 0, s, a, none); else hipLaunchKernelGGL((k_mmq_q80_skinny<false, false>), grid, block, 0, s, a, none); }
         return 1;

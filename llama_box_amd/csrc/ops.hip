@@ -57,7 +57,7 @@ __device__ __forceinline__ void q80_panel_store(const float r0, const float r1, 
     *(uint32_t *) (tile + (w8 >> 2) * 512 + cr * 16 + (w8 & 3) * 4) = packed;
     if (w8 == 0) *(float *) (tile + 1024 + cr * 4) = h2f(f2h(d));
 }
-// Q80P (round 6): the row leaves as Q8_0 blocks in panel order instead of f32 — every reader is a Q8_0 mat-mul of 9 columns and up (graph.cpp: q80_panel_consumers_only);
+// Q80P (round 6): the row leaves as Q8_0 blocks in panel order instead of f32 — every reader is a Q8_0 mat-mul of 2 columns and up (graph.cpp: q80_panel_consumers_only);
 // the vector path only (the launcher checks), same arithmetic as the two kernels it replaces
 template <bool Q80P>
 __global__ void __launch_bounds__(256) k_rms_norm(const tdesc a, const tdesc d, const float eps, const float * __restrict__ w, char * __restrict__ q80 = nullptr,

@@ -82,7 +82,7 @@ void launch_repack_planes(hipStream_t s, int type, const void * src, void * dst,
     }
 }
 
-// ---- Q8_0: the PANEL copy read by the 9 .. 32-column matrix-core kernel (mmq_q80.hip: k_mmq_q80_skinny).  Same bytes as the tensor (N x K / 32 x 34), regrouped per
+// ---- Q8_0: the PANEL copy read by the matrix-core kernels (mmq_q80.hip).  Same bytes as the tensor (N x K / 32 x 34), regrouped per
 // (panel of 32 rows, chunk of 4 blocks) into a tile of 4352 bytes: [block 0 .. 3][K half 0 / 1][row 0 .. 31][16 quants] (4 KB: a wave-instruction's operand load is
 // 1 KB of consecutive bytes) + [block][row] f16 scales (256 B).  Rows a multiple of 32, K a multiple of 128, rows densely packed.
 __global__ void __launch_bounds__(256) k_repack_q80_panels(const uint8_t * __restrict__ src, uint8_t * __restrict__ dst, const int nchunk, const int64_t nb1) {

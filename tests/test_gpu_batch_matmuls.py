@@ -435,8 +435,35 @@ def test_q8_0_batches_with_and_without_the_panel_copy(backend, H, panels, K, N, 
     assert T.nmse(got[:, rows], ref) <= 1e-10
 
 
+# 16 rows a workgroup over panel copies: one panel, 128 and 129 of them, 257; K of fewer chunks than waves, of a whole ring of four chunks a wave and of one more, of a last ring in part
+@pytest.mark.parametrize("M", [2, 3, 15, 16, 17, 32])
+@pytest.mark.parametrize("K,N", [(640, 2560), (128, 32), (1152, 4096), (2048, 4128), (2048, 8224), (4096, 64), (4224, 512), (5632, 96)])
+def test_q8_0_batches_of_few_columns(backend, H, K, N, M):
+    """mmq_q80.hip up to 32 columns: the same bits from the blocks (32 rows a workgroup) and from the panel copy, and the oracle's values."""
+    rng = np.random.default_rng(K + N + M)
+    w = T.rand_weight(L.Q8_0, K, N, rng)
+    x = (rng.standard_normal((M, K)) * rng.uniform(0.2, 3.0, (M, 1))).astype(np.float32)
+    b = rng.standard_normal(N).astype(np.float32)
+    g = T.G(backend)
+    try:
+        out = H.ggml_add(g.ctx, H.ggml_mul_mat(g.ctx, g.new(L.Q8_0, [K, N], w), g.new(L.F32, [K, M], x)), g.new(L.F32, [N], b))
+        s0 = backend.stat("skinny_launches")
+        blocks = g.compute([out])[0].reshape(M, N)
+        p0 = backend.stat("decode_copy_launches")
+        H.ggml_backend_buffer_set_usage(g.buf, 1)
+        assert H.ggml_backend_graph_compute(backend.backend, g.gf) == 0
+        assert backend.stat("decode_copy_launches") == p0 + 1 and backend.stat("skinny_launches") == s0 + 2
+        panels = g.read(out).reshape(M, N)
+    finally:
+        g.free()
+    assert np.array_equal(panels.view(np.uint32), blocks.view(np.uint32))
+    rows = np.unique(np.concatenate([np.arange(32), np.arange(N - 32, N)]))
+    ref = T.run_case(lambda g: H.ggml_add(g.ctx, H.ggml_mul_mat(g.ctx, g.new(L.Q8_0, [K, len(rows)], np.ascontiguousarray(w[rows])), g.new(L.F32, [K, M], x)), g.new(L.F32, [len(rows)], b[rows])), "oracle")[0].reshape(M, -1)
+    assert T.nmse(panels[:, rows], ref) <= 1e-10
+
+
 def test_q8_0_batches_without_the_skinny_kernel(built):
-    """GGML_MI355X_Q80_SKINNY=0 turns off the kernel of 9 .. 32 columns; 33 and more stay on the matrix cores."""
+    """GGML_MI355X_Q80_SKINNY=0 turns off the kernels of 2 .. 32 columns; 33 and more stay on the matrix cores."""
     code = """if 1:
         import numpy as np, harness as T, llama_box_amd as L
         be, H, rng = L.Backend(0), L.host(), np.random.default_rng(1)
