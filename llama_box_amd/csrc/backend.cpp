@@ -68,10 +68,11 @@ static std::atomic<uint64_t> g_decode_epoch{1};
 uint64_t decode_copy_epoch() { return g_decode_epoch.load(std::memory_order_acquire); }
 // bytes [off, off + n) of the buffer are about to change: the copies of tensors in that range are stale from now on
 static void decode_copy_drop(buffer_ctx * c, size_t off, size_t n) {
-    if (c->shadow == nullptr) return;
+    if (!c->has_copies) return;
     std::lock_guard<std::mutex> lk(c->sh_mtx);
-    if (c->sh_valid.empty()) return;
     bool any = false;
+    for (auto & p : c->panels)
+        if (p.second.valid && p.first < off + n && off < p.first + p.second.bytes) { p.second.valid = false; any = true; }
     for (auto it = c->sh_valid.begin(); it != c->sh_valid.end();) {
         if (it->first < off + n && off < it->first + it->second) { it = c->sh_valid.erase(it); any = true; }
         else ++it;
@@ -80,19 +81,28 @@ static void decode_copy_drop(buffer_ctx * c, size_t off, size_t n) {
 }
 static void decode_copy_drop(ggml_backend_buffer_t b, const ggml_tensor * t, size_t offset, size_t size) {
     buffer_ctx * c = (buffer_ctx *) b->context;
-    if (c->shadow != nullptr && t->data != nullptr) decode_copy_drop(c, (size_t) ((const char *) t->data - (const char *) c->base) + offset, size);
+    if (c->has_copies && t->data != nullptr) decode_copy_drop(c, (size_t) ((const char *) t->data - (const char *) c->base) + offset, size);
 }
 // (q80_panels: the OTHER second copy — Q8_0 matrices regrouped into the 32-row x 4-block tiles the matrix-core kernels load with whole-line
-// wave-instructions, repack.hip: k_repack_q80_panels.  A tensor has one kind of copy: the K-quants planes, Q8_0 panels; same shadow allocation, same invalidation)
-static const uint8_t * second_copy(backend_ctx * c, const ggml_tensor * w, const bool q80_panels) {
+// wave-instructions, repack.hip: k_repack_q80_panels.  A tensor has one kind of copy in the shadow: the K-quants planes, Q8_0 panels; same invalidation)
+static buffer_ctx * copyable(backend_ctx * c, const ggml_tensor * w) {  // the buffer of a weight matrix that may have a second copy
     if (!c->opt.decode_copy || w == nullptr || w->view_src != nullptr || w->data == nullptr || w->ne[2] != 1 || w->ne[3] != 1) return nullptr;
     ggml_backend_buffer_t b = w->buffer;
     if (b == nullptr || !buffer_is_ours(b) || b->usage != GGML_BACKEND_BUFFER_USAGE_WEIGHTS || buffer_is_split(b) || buffer_is_rowpar(b)) return nullptr;
-    if (q80_panels ? !repack_q80_supported(w->type, w->ne[0], w->ne[1], (int64_t) w->nb[1]) : !repack_supported(w->type, w->ne[0], (int64_t) w->nb[1])) return nullptr;
     buffer_ctx * bc = (buffer_ctx *) b->context;
-    if (bc->device != c->device || bc->shadow_failed) return nullptr;
     const size_t off = (size_t) ((const char *) w->data - (const char *) bc->base), bytes = (size_t) w->nb[1] * (size_t) w->ne[1];
-    if (off + bytes > bc->size) return nullptr;
+    return bc->device == c->device && off + bytes <= bc->size ? bc : nullptr;
+}
+static bool room_for_copy(const backend_ctx * c, size_t bytes) {
+    size_t free_b = 0, total_b = 0;
+    return hipMemGetInfo(&free_b, &total_b) == hipSuccess && free_b >= bytes + ((size_t) std::max(0, c->opt.decode_copy_headroom_gib) << 30);
+}
+static const uint8_t * second_copy(backend_ctx * c, const ggml_tensor * w, const bool q80_panels) {
+    buffer_ctx * const bc = copyable(c, w);
+    if (bc == nullptr) return nullptr;
+    if (q80_panels ? !repack_q80_supported(w->type, w->ne[0], w->ne[1], (int64_t) w->nb[1]) : !repack_supported(w->type, w->ne[0], (int64_t) w->nb[1])) return nullptr;
+    if (bc->shadow_failed) return nullptr;
+    const size_t off = (size_t) ((const char *) w->data - (const char *) bc->base), bytes = (size_t) w->nb[1] * (size_t) w->ne[1];
     std::lock_guard<std::mutex> lk(bc->sh_mtx);
     auto it = bc->sh_valid.find(off);
     if (it != bc->sh_valid.end() && it->second == bytes) return (const uint8_t *) bc->shadow + off;
@@ -100,14 +110,14 @@ static const uint8_t * second_copy(backend_ctx * c, const ggml_tensor * w, const
     if (bc->shadow == nullptr) {
         // 288 GB of HBM: a second copy of the weights one GPU serves always fits beside the first — unless the user filled the device on purpose; then the
         // mat-vecs keep reading the block layout, as before round 6
-        size_t free_b = 0, total_b = 0;
-        if (hipMemGetInfo(&free_b, &total_b) != hipSuccess || free_b < bc->size + ((size_t) std::max(0, c->opt.decode_copy_headroom_gib) << 30) || hipMalloc(&bc->shadow, bc->size) != hipSuccess) {
+        if (!room_for_copy(c, bc->size) || hipMalloc(&bc->shadow, bc->size) != hipSuccess) {
             (void) hipGetLastError();
             bc->shadow = nullptr;
             bc->shadow_failed = true;
             MI_INFO("decode copy: no room for a second copy of a %.1f GiB weights buffer on device %d — the mat-vec kernels read the block layout", (double) bc->size / (1 << 30), bc->device);
             return nullptr;
         }
+        bc->has_copies = true;
     }
     if (q80_panels) launch_repack_q80_panels(c->stream, w->data, (char *) bc->shadow + off, w->ne[0], w->ne[1], (int64_t) w->nb[1]);
     else launch_repack_planes(c->stream, w->type, w->data, (char *) bc->shadow + off, w->ne[0], (int64_t) w->nb[1], 0, w->ne[1]);
@@ -120,14 +130,66 @@ static const uint8_t * second_copy(backend_ctx * c, const ggml_tensor * w, const
 }
 const uint8_t * decode_copy(backend_ctx * c, const ggml_tensor * w) { return second_copy(c, w, false); }
 const uint8_t * q80_panel_copy(backend_ctx * c, const ggml_tensor * w) { return second_copy(c, w, true); }
+const uint8_t * k_panel_copy(backend_ctx * c, const ggml_tensor * w) {
+    buffer_ctx * const bc = copyable(c, w);
+    if (bc == nullptr || !repack_supported(w->type, w->ne[0], (int64_t) w->nb[1]) || (w->ne[1] % 16) != 0) return nullptr;
+    const size_t off = (size_t) ((const char *) w->data - (const char *) bc->base), bytes = (size_t) w->nb[1] * (size_t) w->ne[1];
+    std::lock_guard<std::mutex> lk(bc->sh_mtx);
+    auto it = bc->panels.find(off);
+    if (it != bc->panels.end()) {
+        buffer_ctx::panel_mem & p = it->second;
+        if (p.bytes != bytes) return nullptr;  // (another tensor was laid out at this offset before)
+        if (p.valid && p.maker != nullptr && p.maker != c) {  // (the maker may be gone by now, the event is the buffer's)
+            if (c->capturing || hipEventSynchronize(p.made) != hipSuccess) { (void) hipGetLastError(); return nullptr; }
+            p.maker = nullptr;
+        }
+        if (p.valid) return (const uint8_t *) p.mem;
+    }
+    if (c->capturing || bc->panels_failed) return nullptr;
+    if (it == bc->panels.end()) {
+        constexpr size_t CHUNK = (size_t) 256 << 20;
+        const size_t need = (bytes + 255) & ~(size_t) 255;
+        auto ch = std::find_if(bc->panel_chunks.begin(), bc->panel_chunks.end(), [&](const buffer_ctx::panel_chunk & k) { return k.size - k.used >= need; });
+        hipEvent_t made = nullptr;
+        bool ok = hipEventCreateWithFlags(&made, hipEventDisableTiming) == hipSuccess;
+        if (ok && ch == bc->panel_chunks.end()) {
+            buffer_ctx::panel_chunk k{nullptr, std::max(need, std::min(CHUNK, bc->size)), 0};
+            ok = room_for_copy(c, k.size) && hipMalloc(&k.mem, k.size) == hipSuccess;
+            if (ok) {
+                bc->panel_chunks.push_back(k);
+                ch = bc->panel_chunks.end() - 1;
+                bc->has_copies = true;
+            }
+        }
+        if (!ok) {
+            (void) hipGetLastError();
+            if (made) (void) hipEventDestroy(made);
+            bc->panels_failed = true;
+            MI_INFO("panel copies: no room for %.2f GiB on device %d — batches of a few columns read the block layout", (double) bytes / (1 << 30), bc->device);
+            return nullptr;
+        }
+        it = bc->panels.emplace(off, buffer_ctx::panel_mem{(char *) ch->mem + ch->used, bytes, false, nullptr, made}).first;
+        ch->used += need;
+    }
+    buffer_ctx::panel_mem & p = it->second;
+    launch_repack_k_panels(c->stream, w->type, w->data, p.mem, w->ne[0], w->ne[1], (int64_t) w->nb[1]);
+    if (hipEventRecord(p.made, c->stream) != hipSuccess) { (void) hipGetLastError(); return nullptr; }
+    p.maker = c;
+    p.valid = true;
+    c->st.decode_copy_tensors++;
+    c->st.decode_copy_bytes += (int64_t) bytes;
+    return (const uint8_t *) p.mem;
+}
 static void buf_free(ggml_backend_buffer_t b) {
     buffer_ctx * c = (buffer_ctx *) b->context;
     if (ip_any()) ip_host_buffer_freed(b);  // (tp_inproc.cpp mirrors host buffers on the other devices)
     HIP_SOFT(hipSetDevice(c->device));
     uploader_drain(c->device);  // a staged upload may still be writing into this arena
-    if (c->shadow) {  // (graphs captured over it must never be replayed: a new buffer may get the same addresses)
+    if (c->has_copies) {  // (graphs captured over it must never be replayed: a new buffer may get the same addresses)
         HIP_SOFT(hipDeviceSynchronize());
-        HIP_NOTE(hipFree(c->shadow));
+        if (c->shadow) HIP_NOTE(hipFree(c->shadow));
+        for (auto & p : c->panels) HIP_NOTE(hipEventDestroy(p.second.made));
+        for (auto & k : c->panel_chunks) HIP_NOTE(hipFree(k.mem));
         g_decode_epoch.fetch_add(1, std::memory_order_acq_rel);
     }
     HIP_NOTE(hipFree(c->base));
@@ -560,7 +622,7 @@ static void be_set_tensor_async(ggml_backend_t be, ggml_tensor * t, const void *
     note_mask_upload(t, data, offset, size);
     {
         ggml_backend_buffer_t tb = t->view_src ? t->view_src->buffer : t->buffer;
-        if (tb && buffer_is_ours(tb) && ((buffer_ctx *) tb->context)->shadow) decode_copy_drop(tb, t, offset, size);
+        if (tb && buffer_is_ours(tb) && ((buffer_ctx *) tb->context)->has_copies) decode_copy_drop(tb, t, offset, size);
     }
     constexpr size_t SMALL = 64 * 1024, RING = 4u << 20;
     if (size > 0 && size <= SMALL && c->opt.small_uploads) {
@@ -614,7 +676,7 @@ static bool be_cpy_tensor_async(ggml_backend_t be_src, ggml_backend_t be_dst, co
     if (cd != cs) flush_uploads(cd);
     const size_t n = ggml_abi_nbytes(src);
     copy_mask_stats(src, dst, n);
-    if (((buffer_ctx *) db->context)->shadow) decode_copy_drop(db, dst, 0, n);
+    if (((buffer_ctx *) db->context)->has_copies) decode_copy_drop(db, dst, 0, n);
     if (ip_any()) { ip_host_access(sb, false); ip_host_access(db, true); }
     uploader_join(cs->device, cs->stream);
     if (cd->device != cs->device) uploader_drain(cd->device);

@@ -233,7 +233,6 @@ struct backend_ctx {
     uint64_t tick = 0;
     uint64_t decode_epoch = 0;  // decode_copy_epoch() the cached graphs were captured under
     bool capturing = false;
-    bool mm_q5_major = false;  // the graph being planned / run holds more Q5_K than Q4_K weight bytes (graph.cpp: mmq_min_cols_for)
     // tensor parallel
     tp_state * tp = nullptr;
     ip_engine * ip = nullptr;  // -sm row served as in-process tensor parallelism (tp_inproc.cpp); owned by the main device's backend
@@ -291,10 +290,19 @@ struct buffer_ctx {
     bool shadow_failed = false;
     std::mutex sh_mtx;
     std::unordered_map<size_t, size_t> sh_valid;  // offset of a repacked tensor -> its bytes
+    // ... and the K-quant matrices that batches of a few columns multiply over panels (mmq_panel.hip): those only, in chunks that hold several; made, dropped and freed as above.  The step that first
+    // uses a copy makes it on its own stream and goes on; another backend instance waits for `made` first
+    struct panel_mem { void * mem; size_t bytes; bool valid; const backend_ctx * maker; hipEvent_t made; };
+    struct panel_chunk { void * mem; size_t size, used; };
+    std::unordered_map<size_t, panel_mem> panels;  // offset of the tensor -> its panel copy
+    std::vector<panel_chunk> panel_chunks;
+    bool panels_failed = false;
+    std::atomic<bool> has_copies{false};           // any copy was ever made
 };
 // the plane-layout copy of weight matrix w for the batch-1 mat-vec kernels, or nullptr (no copy: views, split / row-parallel buffers, option off,
 // allocation failed, or asked during a capture for a tensor not yet repacked)
 const uint8_t * decode_copy(backend_ctx * c, const ggml_tensor * w);
+const uint8_t * k_panel_copy(backend_ctx * c, const ggml_tensor * w);    // a K-quant matrix's panel copy (mmq_panel.hip), or nullptr
 const uint8_t * q80_panel_copy(backend_ctx * c, const ggml_tensor * w);  // a Q8_0 matrix's panel copy (mmq_q80.hip), or nullptr
 uint64_t decode_copy_epoch();  // bumped whenever a copy was dropped: graphs captured before hold pointers to it
 bool buffer_is_ours(ggml_backend_buffer_t b);

@@ -17,18 +17,18 @@
 namespace mi355x {
 
 static bool is_quant(int t) { return t == GGML_TYPE_Q4_K || t == GGML_TYPE_Q5_K || t == GGML_TYPE_Q6_K || t == GGML_TYPE_Q8_0; }
-// batches at least this wide run on the matrix cores.  The option's default (3) is per weight type since round 6: Q4_K / Q6_K matrices take the weight-streaming
-// kernel from TWO columns on (a 2-sequence step of Llama-3-8B Q4_K_M: 2.89-3.03 -> 2.78 ms — the multi-column mat-vec path has none of the batch path's fusions,
-// 17 launches a layer), Q5_K stays at 3 (its skinny unit is slower: Qwen2-7B Q5_K_M 3.13 -> 3.79 ms with 2; profiles/r06_np2_min_cols.txt)
-// (Q6_K follows the model: with 2 where Q4_K carries the graph's weight bytes — Q4_K_M; 3 in a Q5_K_M model, whose Q6_K matrices measured slower on the unit at 2
-// columns: Qwen2 3.13 -> 3.30 ms when only they moved.  plan_ws counts the bytes.)
-static inline int mmq_min_cols_for(const backend_ctx * c, int wtype) {
-    if (c->opt.mmq_min_cols != 3) return c->opt.mmq_min_cols;
-    return (wtype == GGML_TYPE_Q4_K || (wtype == GGML_TYPE_Q6_K && !c->mm_q5_major)) ? 2 : 3;
+// batches at least this wide run on the matrix cores; the option's default (3) means two columns.  (The multi-column mat-vec has none of the batch path's fusions.  Two sequences of 200 tokens, us a
+// step, from three columns on / from two: Llama-3-8B Q4_K_M 2586 / 2458, Qwen2-7B Q5_K_M 3134 / 2767 with its gate/up pair over panels.)
+static inline int mmq_min_cols_for(const backend_ctx * c) { return c->opt.mmq_min_cols != 3 ? c->opt.mmq_min_cols : 2; }
+// the panel copy of a K-quant matrix where M columns are multiplied over it (mmq_panel.hip) in a launch of n_total rows, else nullptr
+static const uint8_t * k_panels(backend_ctx * c, const ggml_tensor * w, int64_t n_total, int64_t M) {
+    return c->opt.mmq_i8 && c->opt.mmq_skinny && M >= mmq_min_cols_for(c) && mmq_panel_applies(w->type, w->ne[0], n_total, M) ? k_panel_copy(c, w) : nullptr;
 }
-// Does a batch of M columns take the mat-vec fusions (gate/up/SwiGLU, bias and residual in one launch)?  Left at its default, the option leaves Q8_0 batches to the matrix-core kernel.
+// Does a batch of M columns take the mat-vec fusions (gate/up/SwiGLU, bias and residual in one launch)?  Left at its default, the option leaves batches to the matrix-core kernels that serve 2 columns.
 static bool mat_vec_fusions(const backend_ctx * c, const ggml_tensor * w, int64_t M) {
-    return M <= c->opt.mmvq_max_cols && !(c->opt.mmvq_max_cols == 2 && mmq_q80_batch_supported(w->type, w->ne[0], w->ne[1], M));
+    if (M > c->opt.mmvq_max_cols) return false;
+    return M < 2 || c->opt.mmvq_max_cols != 2 ||
+           !(mmq_q80_batch_supported(w->type, w->ne[0], w->ne[1], M) || (c->opt.mmq_i8 && M >= mmq_min_cols_for(c) && mmq_i8_supported(w->type, w->ne[0], w->ne[1], M)));
 }
 static int act_kind(int wtype) { return wtype == GGML_TYPE_Q8_0 ? GGML_TYPE_Q8_0 : GGML_TYPE_Q8_K; }
 static bool is_f32_contig(const ggml_tensor * t) { return t->type == GGML_TYPE_F32 && ggml_abi_is_contiguous(t); }
@@ -335,16 +335,6 @@ static bool mm_id_tile_applies(const ggml_tensor * n);
 static size_t fa_image_offset(const tdesc & q, const tdesc & k, const tdesc & v) { return (fattn_workspace_bytes(q, k, v, 64, GGML_TYPE_F16) + 255) & ~(size_t) 255; }
 static ws_plan plan_ws(backend_ctx * c, const ggml_cgraph * g) {
     ws_plan p;
-    {   // which K-quant carries this graph's weight bytes (mmq_min_cols_for)
-        size_t q4 = 0, q5 = 0;
-        for (int i = 0; i < g->n_nodes; ++i) {
-            const ggml_tensor * n = g->nodes[i];
-            if (n->op != GGML_OP_MUL_MAT || !n->src[0]) continue;
-            if (n->src[0]->type == GGML_TYPE_Q4_K) q4 += ggml_abi_nbytes(n->src[0]);
-            else if (n->src[0]->type == GGML_TYPE_Q5_K) q5 += ggml_abi_nbytes(n->src[0]);
-        }
-        c->mm_q5_major = q5 > q4;
-    }
     for (int i = 0; i < g->n_nodes; ++i) {
         const ggml_tensor * n = g->nodes[i];
         // (besides what follows: K.q of one head on one key head has this form, and the attention chain that may start at it has its own scratch)
@@ -355,7 +345,7 @@ static ws_plan plan_ws(backend_ctx * c, const ggml_cgraph * g) {
             // (2..32 columns: the skinny matrix-core kernel fetches 32 columns' worth of activation bytes whatever M is)
             // (and the wide form of the same unit fetches whole groups of 128 columns of a prompt batch)
             p.act_bytes = std::max(p.act_bytes, quantized_act_bytes(act_kind(n->src[0]->type), b->ne[0], (Mc >= 2 && Mc < 32) ? 32 : (Mc >= 33 ? (Mc + 127) / 128 * 128 : Mc)));
-            if (Mc >= mmq_min_cols_for(c, n->src[0]->type) && (n->ne[0] % 4) == 0) p.aux_bytes = std::max(p.aux_bytes, 3 * mmq_workspace_bytes(n->src[0]->type, b->ne[0], n->src[0]->ne[1], Mc, c->opt.mmq_skinny));  // (x3: up to three sibling matrices share a launch)
+            if (Mc >= mmq_min_cols_for(c) && (n->ne[0] % 4) == 0) p.aux_bytes = std::max(p.aux_bytes, 3 * mmq_workspace_bytes(n->src[0]->type, b->ne[0], n->src[0]->ne[1], Mc, c->opt.mmq_skinny));  // (x3: up to three sibling matrices share a launch)
         } else if (n->op == GGML_OP_MUL_MAT && mm_cache_image_ok(n) && !buffer_is_split(n->src[0]->buffer)) {
             const tdesc a16 = kv_image_desc(TD(n->src[0]), nullptr);
             p.aux_bytes = std::max(p.aux_bytes, ((mul_mat_f_workspace_bytes(a16, TD(n->src[1])) + 255) & ~(size_t) 255) + kv_image_bytes(a16));
@@ -723,9 +713,10 @@ static bool run_mul_mat_q(exec_state & st, const ggml_tensor * w, const ggml_ten
         return true;
     }
     const bool i8 = c->opt.mmq_i8 && mmq_i8_supported(w->type, K, N, M);
-    if (M >= mmq_min_cols_for(c, w->type) && !w2 && !add2 && (!add || i8) && (i8 || mmq_supported(w->type, K, N, M))) {
+    const uint8_t * const panels = i8 && !w2 && !add2 && st.epi_dst != dst ? k_panels(c, w, N, M) : nullptr;
+    if (M >= mmq_min_cols_for(c) && !w2 && !add2 && (!add || i8) && (i8 || mmq_supported(w->type, K, N, M))) {
         timed_scope ts(c, (std::string("mmq_") + type_tag(w->type) + "_n" + std::to_string(N) + "_k" + std::to_string(K)).c_str(), wbytes, i8);
-        const int ks = st.epi_dst == dst ? 1 : ((N % 4) == 0 && (dst->nb[1] % 16) == 0 ? mmq_pick_ksplit(K, N, M, c->opt.mmq_skinny, w->type) : 1);
+        const int ks = panels || st.epi_dst == dst ? 1 : ((N % 4) == 0 && (dst->nb[1] % 16) == 0 ? mmq_pick_ksplit(K, N, M, c->opt.mmq_skinny, w->type) : 1);
         float * part = (float *) ((char *) c->ws + st.aux_off);
         if (i8) {
             const int64_t arows = add ? add->ne[1] * add->ne[2] * add->ne[3] : 0;
@@ -748,7 +739,12 @@ static bool run_mul_mat_q(exec_state & st, const ggml_tensor * w, const ggml_ten
                 }
             }
             const mmq_epi * epi = st.epi_dst == dst ? &st.epi : nullptr;
-            const int served = launch_mmq_i8(c->stream, w->type, (const uint8_t *) w->data, (int64_t) w->nb[1], (int) K, (int) N, (int) M, act, (float *) dst->data, (int64_t) (dst->nb[1] / 4), c->opt.mmq_bn, epi ? 1 : ks, part,
+            if (panels) {
+                const mmqp_mat mt{panels, (int) N, 0, (float *) dst->data, (int64_t) (dst->nb[1] / 4), add ? (const float *) add->data : nullptr, add_stride};
+                launch_mmq_panel(c->stream, w->type, 1, &mt, (int) K, (int) M, act);
+                c->st.decode_copy_launches++;
+            }
+            const int served = panels ? 1 : launch_mmq_i8(c->stream, w->type, (const uint8_t *) w->data, (int64_t) w->nb[1], (int) K, (int) N, (int) M, act, (float *) dst->data, (int64_t) (dst->nb[1] / 4), c->opt.mmq_bn, epi ? 1 : ks, part,
                                              add ? (const float *) add->data : nullptr, add_stride, !defer, c->opt.mmq_skinny, epi);
             c->st.skinny_launches += served == 1;
             c->st.wide_launches += served >= 2;
@@ -1367,6 +1363,10 @@ static int try_merge_mm_batch(exec_state & st, int i) {  // returns the number o
         e.nb1[slot] = role == 0 ? epl.a.qd_nb1 : (role == 1 ? epl.a.kc_nb1 : epl.a.vc_nb1);
         e.nb2[slot] = role == 0 ? epl.a.qd_nb2 : 0;
     };
+    const uint8_t * panels[3] = {nullptr, nullptr, nullptr};
+    bool over_panels = epi_node < 0 && !mixed;
+    for (size_t q = 0; q < ms.size() && over_panels; ++q) over_panels = (panels[q] = k_panels(c, g->nodes[ms[q].k]->src[0], n_total, M)) != nullptr;
+    if (over_panels) ks = 1;
     if ((size_t) ks * (size_t) M * (size_t) n_total * sizeof(float) > c->ws_size - st.aux_off && ks > 1) return 0;
     const void * act = quantized_src1(st, X, type);
     for (size_t q = 1; q < ms.size(); ++q)
@@ -1405,7 +1405,13 @@ static int try_merge_mm_batch(exec_state & st, int i) {  // returns the number o
             };
             for (size_t q = 0; q < ms.size(); ++q) epi_fill(epi, (int) q, role_of2(ms[q]));
         }
-        const int served = launch_mmq_i8_multi(c->stream, type, (int) ms.size(), mats, (int) K, (int) M, act, c->opt.mmq_bn, ks, part, !defer, c->opt.mmq_skinny, epi_node >= 0 ? &epi : nullptr);
+        if (over_panels) {
+            mmqp_mat pm[3];
+            for (size_t q = 0; q < ms.size(); ++q) pm[q] = {panels[q], mats[q].N, 0, mats[q].dst, mats[q].dst_stride, mats[q].add, mats[q].add_stride};
+            launch_mmq_panel(c->stream, type, (int) ms.size(), pm, (int) K, (int) M, act);
+            c->st.decode_copy_launches++;
+        }
+        const int served = over_panels ? 1 : launch_mmq_i8_multi(c->stream, type, (int) ms.size(), mats, (int) K, (int) M, act, c->opt.mmq_bn, ks, part, !defer, c->opt.mmq_skinny, epi_node >= 0 ? &epi : nullptr);
         c->st.skinny_launches += served == 1;
         c->st.wide_launches += served >= 2;
         c->st.wide_few_launches += served == 3;
@@ -2907,11 +2913,11 @@ static int run_node(exec_state & st, int i) {
                 const int used = try_merge_q80_skinny(st, i);
                 if (used != 0) return used;
             }
-            if (fuse && !rowpar && c->opt.mm_merge && M >= mmq_min_cols_for(c, a->type) && c->opt.mmq_i8 && mmq_i8_supported(a->type, a->ne[0], a->ne[1], M)) {
+            if (fuse && !rowpar && c->opt.mm_merge && M >= mmq_min_cols_for(c) && c->opt.mmq_i8 && mmq_i8_supported(a->type, a->ne[0], a->ne[1], M)) {
                 const int used = try_merge_mm_batch(st, i);
                 if (used != 0) return used;
             }
-            if (fuse && !rowpar && ((M >= mmq_min_cols_for(c, a->type) && c->opt.mmq_i8 && mmq_i8_supported(a->type, a->ne[0], a->ne[1], M)) ||
+            if (fuse && !rowpar && ((M >= mmq_min_cols_for(c) && c->opt.mmq_i8 && mmq_i8_supported(a->type, a->ne[0], a->ne[1], M)) ||
                                     mmq_q80_batch_supported(a->type, a->ne[0], a->ne[1], M))) {
                 // batches: MUL_MAT -> ADD (bias row or residual) rides in the GEMM's store
                 ggml_tensor * a1 = next(1);

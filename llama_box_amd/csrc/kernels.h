@@ -249,6 +249,16 @@ int mmq_skinny_ksplit(int64_t K, int64_t n_total);
 // Q8_0 weights x Q8_0 activations, one int8 MFMA per 32-value block + immediate f32 scale-accumulate (mmq_q80.hip)
 // 2 columns and up: up to 32 with the weights streamed once, above in tiles of 32 rows x 64 columns, or of 128 x 128 where that is faster; activations in panel order
 bool mmq_q80_batch_supported(int type, int64_t K, int64_t N, int64_t M);
+// K-quants x 2 .. 32 columns over panel copies (mmq_panel.hip)
+struct mmqp_mat { const uint8_t * W; int N, tile_end; float * dst; int64_t dst_stride; const float * add; int64_t add_stride; };  // W: the panel copy; tile_end: set by the launcher
+struct mmqp_args {
+    mmqp_mat m[3];
+    int n_tiles, K, M;
+    int split, red_off;     // set by the launcher: waves that share the super-blocks of a tile, LDS offset of their partial sums (0: one round, in the activations' place)
+    const q8k_dev * act;    // [M][K / 256]
+};
+bool mmq_panel_applies(int type, int64_t K, int64_t n_total, int64_t M);  // n_total: rows of all matrices of the launch
+void launch_mmq_panel(hipStream_t s, int type, int n, const mmqp_mat * mats, int K, int M, const void * act_q8k);
 struct mmq80s_desc { const uint8_t * W; const uint8_t * W_panels; int64_t w_nb1; int N; float * dst; int64_t dst_stride; const float * add; int64_t add_stride; };
 int launch_mmq_q80_multi(hipStream_t s, int n, const mmq80s_desc * mats, int K, int M, const void * act_q80_panel, const mmq_epi * epi = nullptr /* 2 .. 32 columns, three matrices */);  // up to three matrices over the same activations; returns the launches it took
 void launch_mmq_q80(hipStream_t s, const uint8_t * W, const uint8_t * W_panels, int64_t w_nb1, int K, int N, int M, const void * act_q80_panel, float * dst, int64_t dst_stride, const float * add, int64_t add_stride);
@@ -410,6 +420,7 @@ void launch_flash_attn_combine(hipStream_t s, int D, const float * ws, const flo
 bool repack_supported(int type, int64_t K, int64_t nb1);
 void launch_repack_planes(hipStream_t s, int type, const void * src, void * dst, int64_t K, int64_t nb1, int64_t r0, int64_t n_rows);
 bool repack_q80_supported(int type, int64_t K, int64_t N, int64_t nb1);  // Q8_0: the panel copy of the matrix-core kernels (repack.hip)
+void launch_repack_k_panels(hipStream_t s, int type, const void * src, void * dst, int64_t K, int64_t N, int64_t nb1);
 void launch_repack_q80_panels(hipStream_t s, const void * src, void * dst, int64_t K, int64_t N, int64_t nb1);
 
 // ---- layers with state per sequence (seq.hip): short convolutions over a sequence's history and three recurrences over a matrix state per head
@@ -513,6 +524,7 @@ void tu_touch_mmq(hipStream_t s);
 void tu_touch_mmq_i8(hipStream_t s);
 void tu_touch_mmq_skinny(hipStream_t s);
 void tu_touch_mmq_q80(hipStream_t s);
+void tu_touch_mmq_panel(hipStream_t s);
 void tu_touch_ops(hipStream_t s);
 void tu_touch_fattn(hipStream_t s);
 void tu_touch_attn_f32(hipStream_t s);
@@ -535,6 +547,7 @@ inline void preload_kernel_files(hipStream_t s) {
     tu_touch_mmq_i8(s);
     tu_touch_mmq_skinny(s);
     tu_touch_mmq_q80(s);
+    tu_touch_mmq_panel(s);
     tu_touch_ops(s);
     tu_touch_fattn(s);
     tu_touch_attn_f32(s);

@@ -106,6 +106,62 @@ void launch_repack_q80_panels(hipStream_t s, const void * src, void * dst, int64
     }
 }
 
+// ---- K-quants: the PANEL copy read by mmq_panel.hip.  Same bytes as the tensor, regrouped per (16 rows, super-block) into a unit whose operand loads are 1 KB of consecutive bytes:
+//   Q4_K (2304 B): [row][16 B header] [lane][qs bytes o .. o + 7 of values 0 .. 63 | of 64 .. 127] [lane][of 128 .. 191 | of 192 .. 255], lane = row + 16 q, o = 8 (q >> 1) + 16 (q & 1)
+//   Q5_K (2816 B): [row][header] [lane][qh bytes o .. o + 7] and the quants as Q4_K
+//   Q6_K (3328 B): [lane][ql o .. o + 7 | ql 32 + o ..] [lane][ql 64 + o .. | ql 96 + o ..] [lane][qh o .. | qh 32 + o ..] [row][16 scales]; the d's (32 B a unit) behind the tile's units
+// One thread a 16-byte piece of the unit; rows a multiple of 16.
+template <int QT> __global__ void __launch_bounds__(256) k_repack_k_panels(const uint8_t * __restrict__ src, uint8_t * __restrict__ dst, const int nblk, const int64_t nb1) {
+    constexpr int BYTES = QT == 4 ? 144 : QT == 5 ? 176 : 210, UNIT = QT == 6 ? 3328 : 16 * BYTES;
+    const int p = threadIdx.x, sb = blockIdx.x;
+    const uint8_t * const rows = src + (size_t) blockIdx.y * 16 * nb1 + (size_t) sb * BYTES;
+    uint8_t * const tile = dst + (size_t) blockIdx.y * 16 * BYTES * nblk;
+    uint8_t * const unit = tile + (size_t) sb * UNIT;
+    if (p >= UNIT / 16) return;
+    constexpr int FIRST = QT == 6 ? 0 : QT == 5 ? 48 : 16;  // pieces ahead of the quants
+    auto two = [&](const uint8_t * x, const uint8_t * y) {  // 8 bytes of each
+        piece16 v;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) { v.h[i] = *(const uint16_t *) (x + 2 * i); v.h[4 + i] = *(const uint16_t *) (y + 2 * i); }
+        st_piece_a2(unit + 16 * p, v);
+    };
+    if (QT != 6 && p < 16) {
+        st_piece_a2(unit + 16 * p, ld_piece_a2(rows + (size_t) p * nb1));
+        return;
+    }
+    if (QT == 5 && p < 48) {  // two lanes' qh bytes
+        const int l = 2 * (p - 16), row = l & 15, q = l >> 4, o = 8 * (q >> 1) + 16 * (q & 1);
+        two(rows + (size_t) row * nb1 + 16 + o, rows + (size_t) (row + 1) * nb1 + 16 + o);
+        return;
+    }
+    if (QT == 6 && p >= 192) {
+        const uint8_t * blk = rows + (size_t) (p - 192) * nb1;
+        st_piece_a2(unit + 16 * p, ld_piece_a2(blk + 192));
+        *(uint16_t *) (tile + (size_t) nblk * UNIT + (size_t) sb * 32 + 2 * (p - 192)) = *(const uint16_t *) (blk + 208);
+        return;
+    }
+    const int u = (p - FIRST) >> 6, l = (p - FIRST) & 63, row = l & 15, q = l >> 4, o = 8 * (q >> 1) + 16 * (q & 1);
+    const uint8_t * blk = rows + (size_t) row * nb1;
+    if constexpr (QT == 6) {
+        if (u < 2) two(blk + 64 * u + o, blk + 64 * u + 32 + o);
+        else two(blk + 128 + o, blk + 160 + o);
+    } else {
+        const uint8_t * qs = blk + BYTES - 128 + 64 * u + o;
+        two(qs, qs + 32);
+    }
+}
+void launch_repack_k_panels(hipStream_t s, int type, const void * src, void * dst, int64_t K, int64_t N, int64_t nb1) {
+    const int nblk = (int) (K / 256);
+    for (int64_t t0 = 0; t0 < N / 16; t0 += 32768) {  // (grid.y limit)
+        const dim3 grid((unsigned) nblk, (unsigned) std::min<int64_t>(32768, N / 16 - t0));
+        const uint8_t * s1 = (const uint8_t *) src + (size_t) t0 * 16 * nb1;
+        uint8_t * d1 = (uint8_t *) dst + (size_t) t0 * 16 * nb1;  // (a tile has the bytes of its 16 rows)
+        if (type == GGML_TYPE_Q4_K) hipLaunchKernelGGL(k_repack_k_panels<4>, grid, dim3(256), 0, s, s1, d1, nblk, nb1);
+        else if (type == GGML_TYPE_Q5_K) hipLaunchKernelGGL(k_repack_k_panels<5>, grid, dim3(256), 0, s, s1, d1, nblk, nb1);
+        else hipLaunchKernelGGL(k_repack_k_panels<6>, grid, dim3(256), 0, s, s1, d1, nblk, nb1);
+    }
+}
+
 MI_TU_TOUCH(repack)
 
 }  // namespace mi355x

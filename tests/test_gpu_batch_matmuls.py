@@ -477,3 +477,42 @@ def test_q8_0_batches_without_the_skinny_kernel(built):
     env = dict(os.environ, GGML_MI355X_Q80_SKINNY="0", PYTHONPATH=os.pathsep.join([T.REPO, os.path.join(T.REPO, "tests")]))
     r = subprocess.run([sys.executable, "-c", code], env=env, capture_output=True, text=True, timeout=100)
     assert r.returncode == 0 and r.stdout.split() == ["0", "True", "1", "True"], (r.stdout, r.stderr[-1000:])
+
+
+# K-quants over panel copies: 576 and 577 tiles of 16 rows, rounds of one to several tiles a wave, a wave without a unit (3 super-blocks), one and two matrices a launch, both sides of 16 columns
+@pytest.mark.parametrize("M", [2, 7, 8, 9, 16, 17, 32])
+@pytest.mark.parametrize("wt,K,Ns,widest,narrowest", [  # (the columns for which panels are used)
+    (L.Q4_K, 4096, (4608, 4608), 16, 2), (L.Q4_K, 4352, (9232,), 16, 2), (L.Q4_K, 2048, (9216,), 16, 9), (L.Q4_K, 4096, (33792,), 16, 2), (L.Q4_K, 4096, (9200,), 0, 0), (L.Q5_K, 1024, (9232,), 16, 2),
+    (L.Q5_K, 2560, (4624, 4608), 32, 2), (L.Q5_K, 4352, (12288,), 32, 2), (L.Q5_K, 4608, (12288,), 16, 2), (L.Q5_K, 2048, (38400,), 32, 2), (L.Q6_K, 1024, (9216,), 16, 2), (L.Q6_K, 1280, (32784,), 16, 2),
+    (L.Q6_K, 2304, (16384, 16384), 32, 2), (L.Q6_K, 3584, (32768,), 32, 2), (L.Q6_K, 8704, (9216,), 16, 2)])
+def test_k_quants_over_panels(backend, H, wt, K, Ns, widest, narrowest, M):
+    """mmq_panel.hip: the values of the block layout's kernels and of the oracle, with an addend."""
+    rng = np.random.default_rng(K + sum(Ns) + M)
+    ws = [T.rand_weight(wt, K, N, rng) for N in Ns]
+    x = (rng.standard_normal((M, K)) * rng.uniform(0.2, 3.0, (M, 1))).astype(np.float32)
+    bs = [rng.standard_normal(N).astype(np.float32) for N in Ns]
+
+    def outs(g, rows=None):
+        cur = g.new(L.F32, [K, M], x)
+        sel = [(w, b) if rows is None else (np.ascontiguousarray(w[r]), b[r]) for w, b, r in zip(ws, bs, rows or Ns)]
+        return [H.ggml_add(g.ctx, H.ggml_mul_mat(g.ctx, g.new(wt, [K, len(b)], w), cur), g.new(L.F32, [len(b)], b)) for w, b in sel]
+
+    g = T.G(backend)
+    try:
+        os_ = outs(g)
+        blocks = [r.copy() for r in g.compute(os_)]
+        k0, p0 = backend.stat("kernel_launches"), backend.stat("decode_copy_launches")
+        H.ggml_backend_buffer_set_usage(g.buf, 1)
+        assert H.ggml_backend_graph_compute(backend.backend, g.gf) == 0
+        panels = [g.read(o) for o in os_]
+        over = narrowest <= M <= widest
+        assert backend.stat("decode_copy_launches") == p0 + over
+        if over:
+            assert backend.stat("kernel_launches") == k0 + 2  # (the quantiser and one launch)
+    finally:
+        g.free()
+    rows = [np.unique(np.concatenate([np.arange(16), np.arange(N - 16, N)])) for N in Ns]
+    ref = T.run_case(lambda g: outs(g, rows), "oracle")
+    for q, N in enumerate(Ns):
+        assert T.nmse(panels[q], blocks[q]) <= 1e-12
+        assert T.nmse(panels[q].reshape(M, N)[:, rows[q]], ref[q].reshape(M, -1)) <= 1e-10
