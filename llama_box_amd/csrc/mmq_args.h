@@ -37,7 +37,10 @@ bool launch_mmq_skinny_mixed(hipStream_t s, const mmq8_args & a);
 // prompt batches on the same unit (mmq_skinny.hip): 0 = not there, 1 = k_mmq_wide (no K split), 2 / 3 = k_mmq_wide_few with that many token tiles a workgroup
 int mmq_wide_form(int type, int64_t K, const int64_t * N, int n_mat, int64_t M, int64_t w_nb1);
 int mmq_wide_ksplit(int type, int64_t K, int64_t N, int64_t M);  // K slices of such a launch (0: it does not apply)
-int mmq_tiled_ksplit(int64_t K, int64_t N, int64_t M);  // K slices of the tiled GEMM (mmq_i8.hip)
+int mmq_tiled_ksplit(int64_t K, int64_t N, int64_t M);  // K slices of the tiled GEMM (mmq_i8.hip; Q6_K of more than 64 columns: mmq_q6_tile)
+struct q6_tile { int bn, ks; double us; };  // its panel rows, K slices and expected time for a Q6_K product of more than 64 columns
+q6_tile mmq_q6_tile(int64_t K, int64_t N, int64_t M);
+double q6_slices_us(int64_t N, int64_t M, int64_t ks);  // ... the part of that time that its slices cost
 void launch_mmq_wide(hipStream_t s, int type, int form, const mmq8_args & a);  // mmq_skinny.hip; a.mat[].panel0 / n_panels are set by the launcher
 
 }  // namespace mi355x

@@ -421,14 +421,38 @@ template <int QT, int BN, int BM = 128> static void launch_mmq8_t(hipStream_t s,
     MI_LAUNCH_PROBED((k_mmq_i8<QT, BN, BM>), dim3(grid, (unsigned) a.ksplit), dim3(BN * 4), lds, s, a);
 }
 
+double q6_slices_us(int64_t N, int64_t M, int64_t ks) { return 2.6 + 2.3e-6 * (double) (ks * N * M); }  // the launch that sums them, and their bytes
+// Time of a Q6_K product of more than 64 columns on panels of bn rows with the K range in ks slices, us without the quantisation of the activations.  A CU holds one workgroup of 128
+// rows or two of 64; panels are dealt out in eights, one XCD each, and so a round of 256 CUs counts whole eights: 28 panels of 128 rows occupy as many rounds as 32.  A workgroup's
+// steps (super-blocks of its slice) follow one another: 3.15 us for 128 rows, 2.39 for 64 rows alone on a CU and 3.57 for two of these beside each other - latencies of a step's
+// weights, barriers and matrix instructions, all of them there with 12 columns of a tile as with 128.  So a tile that leaves CUs idle is split in K until it does not, and the sum of the slices
+// (2.6 us and their bytes) is what that costs.  Fitted to 1440 products (512 x 3584 .. 8192 x 28672, 70 .. 512 columns, 1 .. 8 slices, weights from memory): 5.5 % rms; the pair that it picks
+// is at most 4 % slower than the fastest one, but for 4096 x 4096 x 100 (6 %).
+static double q6_tile_us(int64_t K, int64_t N, int64_t M, int bn, int64_t ks) {
+    const int64_t nb = (K / 256 + ks - 1) / ks, panels = (N + bn - 1) / bn, rounds = ((panels + 7) / 8 * 8 * ((M + 127) / 128) * ks + 255) / 256;
+    const double us = 4.5 + (bn == 128 ? rounds * (3.15 * nb - 1.8) : (rounds / 2) * (3.57 * nb - 4.0) + (rounds % 2) * (2.39 * nb - 2.0));
+    return us + (ks > 1 ? q6_slices_us(N, M, ks) : 0.0);
+}
+// Panel rows and K slices of such a product.  One launch and the sum of its slices, us, by the rule for the other formats below / by this one: 4096 x 14336 at 140 columns 77 / 66 (128 rows, 4 slices),
+// 300: 134 / 102, 512: 121 / 119 (128, 2); 3584 x 18944 at 200: 101 / 84, 300: 173 / 113 (64, 3), 512: 191 / 145 (128, 2); 1024 x 4096 at 128: 20.3 / 18.3 (64, 8); 14336 x 4096 at 512: 128 / 122.
+q6_tile mmq_q6_tile(int64_t K, int64_t N, int64_t M) {
+    q6_tile best{64, 1, 0.0};
+    for (int bn = 64; bn <= 128; bn += 64)
+        for (const int ks : {1, 2, 3, 4, 6, 8}) {
+            if (ks > K / 256) break;
+            const double us = q6_tile_us(K, N, M, bn, ks);
+            if (best.us == 0.0 || us < best.us) best = {bn, ks, us};
+        }
+    return best;
+}
 // few activation columns (continuous-batching decode, M <= 64) leave N/64 x 1 workgroups — far fewer than 256 CUs — so
 // the K range is split over blockIdx.y and the partial products are summed in a fixed order by a second tiny kernel
 int mmq_tiled_ksplit(int64_t K, int64_t N, int64_t M) {
     const int64_t wgs = ((N + 63) / 64) * ((M + 127) / 128), nblk = K / 256;
     static const int ks_target = getenv("GGML_MI355X_MMQ_KS_TARGET") ? atoi(getenv("GGML_MI355X_MMQ_KS_TARGET")) : 512;
     if (M <= 64) return (int) std::max<int64_t>(1, std::min<int64_t>(nblk, ks_target / std::max<int64_t>(1, wgs)));
-    // wide batches (prefill micro-batches): only when the output is too small to occupy the chip (wk/wv: 64 workgroups at
-    // M = 512), or when a long K leaves exactly one workgroup per CU (ffn_down): measured 36 -> 19 us and 134 -> 117 us
+    // wide batches (prefill micro-batches) of the other formats (Q6_K: mmq_q6_tile): only when the output is too small to occupy the chip (wk/wv: 64 workgroups at
+    // M = 512), or when a long K leaves exactly one workgroup per CU: measured 36 -> 19 us and 134 -> 117 us
     if (wgs < 256) return (int) std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(4, nblk / 4), 256 / wgs));
     if (wgs == 256 && nblk >= 32) return 2;
     return 1;
@@ -437,7 +461,7 @@ int mmq_pick_ksplit(int64_t K, int64_t N, int64_t M, bool skinny, int type) {
     if (skinny && M >= 2 && M <= 32 && (N % 32) == 0) return mmq_skinny_ksplit(K, N);
     // prompt batches on the wide forms of mmq_skinny.hip: without a K split where the grid fills the chip by token-tile groups, with their own slices otherwise
     if (const int ks = skinny ? mmq_wide_ksplit(type, K, N, M) : 0) return ks;
-    return mmq_tiled_ksplit(K, N, M);
+    return type == GGML_TYPE_Q6_K && M > 64 ? mmq_q6_tile(K, N, M).ks : mmq_tiled_ksplit(K, N, M);
 }
 // can matrices of these K-quant types (same K, same activations) share one launch of 2..32 columns?
 bool mmq_skinny_mix_ok(const int * types, const int64_t * N, const int64_t * w_nb1, int n, int64_t K, int64_t M) {
@@ -511,7 +535,7 @@ int launch_mmq_i8_multi(hipStream_t s, int type, int n_mat, const mmq_mat_desc *
     a.M = M;
     a.act = (const q8k_dev *) act_q8k;
     a.ksplit = std::max(1, ksplit);
-    int64_t panels128 = 0;
+    int64_t panels128 = 0, n_rows = 0;
     const bool skinny_opt = skinny;
     bool mixed = false;
     float * pp = part;
@@ -526,6 +550,7 @@ int launch_mmq_i8_multi(hipStream_t s, int type, int n_mat, const mmq_mat_desc *
         a.mat[i].part = pp;
         pp += (size_t) a.ksplit * M * mats[i].N;
         panels128 += (mats[i].N + 127) / 128;
+        n_rows += mats[i].N;
         const int ti = mats[i].type ? mats[i].type : type;
         mixed = mixed || ti != type;
         a.mat[i].qt = ti == GGML_TYPE_Q4_K ? 4 : (ti == GGML_TYPE_Q5_K ? 5 : 6);
@@ -572,13 +597,15 @@ int launch_mmq_i8_multi(hipStream_t s, int type, int n_mat, const mmq_mat_desc *
     // continuous-batching decode steps: column tiles of 32 / 64 (always on 64-row panels — the output matrix included)
     static const int force_bm = getenv("GGML_MI355X_MMQ_BM") ? atoi(getenv("GGML_MI355X_MMQ_BM")) : 0;
     const int bm = force_bm ? force_bm : (M <= 32 ? 32 : (M <= 64 ? 64 : 128));
-    // 128-row panels (one 8-wave workgroup per CU) when they still fill the chip — except for Q4_K / Q6_K at K < 8192, where 64-row
-    // panels (two independent 4-wave workgroups per CU, not behind one barrier) measure 2-3 % ahead on every prompt shape of the 8B
-    // model; Q5_K (three pieces: the 64-row variant spills) and the 70B shapes measure 4-30 % ahead with 128
-    const bool prefer128 = type == GGML_TYPE_Q5_K || K >= 8192;
-    // (with the K range split — ffn_down of a prompt micro-batch: 32 panels x 4 column tiles x 2 K halves — the splits count as workgroups too:
-    // Q6_K 14336 -> 4096 x 512 measures 102 -> 93-98 us on 128-row panels, round 4)
-    const int bn = force_bn ? force_bn : (bm == 128 && wg128 * std::max(1, a.ksplit) >= 256 && prefer128 ? 128 : 64);
+    // Q6_K: the faster panel height for the slices that the caller chose (q6_tile_us).  Q4_K / Q5_K: 128-row panels (one 8-wave workgroup per CU) when they still fill the chip, K slices
+    // counting as workgroups too - except for Q4_K at K < 8192, where 64-row panels (two independent 4-wave workgroups per CU, not behind one barrier) measure 2-3 % ahead on every prompt
+    // shape of the 8B model; Q5_K (three pieces: the 64-row variant spills) and the 70B shapes measure 4-30 % ahead with 128
+    const auto auto_bn = [&] {
+        if (bm < 128) return 64;
+        if (type == GGML_TYPE_Q6_K) return q6_tile_us(K, n_rows, M, 128, a.ksplit) < q6_tile_us(K, n_rows, M, 64, a.ksplit) ? 128 : 64;
+        return wg128 * a.ksplit >= 256 && (type == GGML_TYPE_Q5_K || K >= 8192) ? 128 : 64;
+    };
+    const int bn = force_bn ? force_bn : auto_bn();
     if (bm < 128 && bn == 64) {
 #define MMQ_SKINNY(QT)                                   \
     {                                                    \

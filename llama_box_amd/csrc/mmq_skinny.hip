@@ -1498,7 +1498,11 @@ static bool wide_fills(int type, int64_t g128, int64_t M) { return type != GGML_
 // (2.4 us): more often than not the next kernel makes it.  The pick is the slower one by more than 5 % at 74 of the points, by 15 % at most; what it decides, other kernel / this one:
 // - Against k_mmq_wide: Q4_K, 77 columns, 28672 x 4096 53.8 / 38.8 (one round of three tiles for two of two), 14336 x 2048 17.5 / 16.5 and the sum of two slices.
 // - Against the tiled GEMM, whose workgroups share a CU and whose own K slices are at most four from 65 columns on: Q4_K, 77 columns, 5120 x 4096 18.8 / 15.1, 1024 x 2048 12.6 / 10.0,
-//   4096 x 512 8.1 / 9.8; Q6_K, 160 columns, 5120 x 4096 43.4 / 26.3, 14336 x 4096 66.1 / 81.4; up to 64 columns it slices as finely as this one: Q6_K, 128 x 5120 x 64 6.2 / 12.6.
+//   4096 x 512 8.1 / 9.8; up to 64 columns it slices as finely as this one: Q6_K, 128 x 5120 x 64 6.2 / 12.6.
+// - Against the tiled GEMM on Q6_K beyond 64 columns as mmq_q6_tile slices it (finer than the line above supposes): it has what it takes from this kernel by more than 20 us, which is where
+//   two tiles of 32 columns are a second round or K slices are missing.  One product and the sum of its slices, us, this one / tiled: 3584 x 18944 at 200 columns 101 / 84, at 300 173 / 113,
+//   4096 x 14336 at 384 136 / 107, 5120 x 13824 at 200 128 / 82.  Below that the estimates are off by as much as they promise: 8192 x 8192 at 257 96 / 109, 4096 x 14336 at 257 92 / 100,
+//   at 140 77 / 66.
 static bool few_pays(int type, int64_t K, int64_t n, int64_t M) {
     const int64_t cu = skinny_n_cu(), nblk = K / 256, tt = few_tiles(type, M), items = dealt_items(n, M, tt), ks = few_slices(K, items);
     const int f = type == GGML_TYPE_Q4_K ? 0 : type == GGML_TYPE_Q5_K ? 1 : 2;
@@ -1518,7 +1522,11 @@ static bool few_pays(int type, int64_t K, int64_t n, int64_t M) {
     const int64_t tks = mmq_tiled_ksplit(K, n, M);
     const tile & t = M <= 64 ? TILE64[f] : TILE128[f];
     const double r = up((n + 63) / 64 * ((M + 127) / 128) * tks, cu);
-    return few < t.start + t.per_wg * r + (t.step + t.shared * r) * up(nblk, tks) + (tks > 1 ? slices_sum : 0);
+    const bool pays = few < t.start + t.per_wg * r + (t.step + t.shared * r) * up(nblk, tks) + (tks > 1 ? slices_sum : 0);
+    if (type != GGML_TYPE_Q6_K || M <= 64 || !pays) return pays;
+    static const form Q6[2] = {{4.6, 2.25, 2.1}, {5.0, 2.71, 2.2}};  // two / three tiles, fitted together with q6_tile_us (40 points, 5.4 % rms)
+    const form & q = Q6[tt - 2];
+    return q.start + q.step * up(nblk, ks) * rounds + q.round * (rounds - 1) + (ks > 1 ? q6_slices_us(n, M, ks) : 0.0) < mmq_q6_tile(K, n, M).us + 20.0;
 }
 int mmq_wide_form(int type, int64_t K, const int64_t * N, int n_mat, int64_t M, int64_t w_nb1) {
     static const bool on = !getenv("GGML_MI355X_MMQ_WIDE") || atoi(getenv("GGML_MI355X_MMQ_WIDE")) != 0;

@@ -516,3 +516,25 @@ def test_k_quants_over_panels(backend, H, wt, K, Ns, widest, narrowest, M):
     for q, N in enumerate(Ns):
         assert T.nmse(panels[q], blocks[q]) <= 1e-12
         assert T.nmse(panels[q].reshape(M, N)[:, rows[q]], ref[q].reshape(M, -1)) <= 1e-10
+
+
+# Q6_K beyond 64 columns on the tiled GEMM: panels of 64 and 128 rows in 1, 2, 3, 4, 6 and 8 slices, slices of unequal lengths, fewer super-blocks than slices, ragged last panels and column
+# tiles, rows that are no multiple of four (no slices); tiled: also where k_mmq_wide_few could run
+@pytest.mark.parametrize("K,N,M,tiled", [
+    (256, 300, 65, True), (768, 70, 129, True), (1280, 1000, 140, True), (2304, 999, 300, True), (4096, 4096, 385, True), (4096, 14336, 257, True), (8192, 2044, 257, True), (8448, 8192, 100, True),
+    (14336, 4096, 300, True), (14336, 4096, 160, False), (18944, 3584, 140, True), (18944, 3584, 257, False), (18944, 3580, 300, True), (18944, 3584, 400, True), (13824, 5120, 200, True)])
+def test_q6_k_panels_and_slices(backend, H, K, N, M, tiled):
+    """mmq_i8.hip: what mmq_q6_tile picks gives the oracle's values (exact integer block sums, f32 sums over K / 256 terms in another order)."""
+    rng = np.random.default_rng(K + N + M)
+    w = T.rand_weight(L.Q6_K, K, N, rng).reshape(N, -1)
+    x = (rng.standard_normal((M, K)) * rng.uniform(0.2, 3.0, (M, 1))).astype(np.float32)
+    b = rng.standard_normal((M, N)).astype(np.float32)
+
+    def run(where, ww, bb):
+        return T.run_case(lambda g: H.ggml_add(g.ctx, H.ggml_mul_mat(g.ctx, g.new(L.Q6_K, [K, ww.shape[0]], ww), g.new(L.F32, [K, M], x)), g.new(L.F32, [ww.shape[0], M], bb)), where)[0].reshape(M, -1)
+
+    c0 = backend.stat("tiled_launches")
+    got = run(backend, w, b)
+    assert backend.stat("tiled_launches") == c0 + tiled
+    rows = np.unique(np.concatenate([np.arange(min(N, 20)), np.arange(max(0, N - 20), N)]))
+    assert T.nmse(got[:, rows], run("oracle", np.ascontiguousarray(w[rows]), np.ascontiguousarray(b[:, rows]))) <= 1e-10
