@@ -7,13 +7,13 @@
 // -inf, expf gives 0, the running max and the double sum are unchanged, and 0 x V adds 0 — so walking the token's list of VISIBLE
 // positions (k_fattn_pos_scan, once per graph run: the mask is the same tensor in every layer) computes the same numbers:
 //   1. logits of the listed cells for the G query heads of a KV head (K rows are gathered, 256 B each; q rounded to f16 as
-//      from_float does; f32 accumulation), kept compactly in scratch;
+//      from_float does; f32 accumulation: on the matrix cores up to NF_CAP cells), kept in LDS or, of longer lists, in scratch;
 //   2. ggml_compute_forward_soft_max_f32 over them: w = s scale + mask, max, e = expf(w - max), sum in double, llama-box's zero-sum
 //      guard (ggml-cpu.patch:5-15), p = e (1 / sum), rounded to f16 where the CPU's second MUL_MAT rounds its src1;
 //   3. V^T.p: a wave takes rows of the TRANSPOSED cache (one per head dimension), lanes take listed cells — the prompt's cells are
 //      contiguous in a row, the decode cells of 32 interleaved sequences are 64 B apart — and the G sums are wave-reduced.
 // A workgroup is (token, KV head, slice of the head dimensions); slices exist so that a handful of tokens still fill the chip, and
-// each repeats steps 1-2 for itself (cheap next to step 3).  Sums run in another order than the dense kernels' (and the CPU's).
+// each repeats steps 1-2 for itself.  Sums run in another order than the dense kernels' (and the CPU's).
 #include <algorithm>
 #include <type_traits>
 
@@ -23,6 +23,8 @@
 namespace mi355x {
 
 #define NF_CAP 1024  // visible cells per token served from registers and LDS
+typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 struct __attribute__((aligned(4))) u32x4a { uint32_t x, y, z, w; };  // a 16-byte load that only promises dword alignment
 template <int G, int NW>
 __global__ void __launch_bounds__(NW * 64) k_attn_nf_list(const tdesc q, const tdesc k, const tdesc v, const tdesc mask, const tdesc dst, const int * __restrict__ lists,
@@ -34,12 +36,33 @@ __global__ void __launch_bounds__(NW * 64) k_attn_nf_list(const tdesc q, const t
     extern __shared__ __attribute__((aligned(16))) float nf_smem[];  // q [G][128] | positions [NF_CAP] | probabilities [G][NF_CAP]
     __shared__ float shf[NW];
     __shared__ double shd[NW];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int tok = blockIdx.x, kvh = blockIdx.y, dq = blockIdx.z;
     const int n_kv = (int) k.ne[1], nkv_heads = (int) k.ne[2];
     const int * lt = lists + (int64_t) tok * list_stride;
-    const int cnt = lt[0];
     const int * pos = lt + 1;
+    // What does not depend on the count is requested with it: the cells of this wave's first tiles, with eight waves a lane's cells of step 3 (within the list's row; what lies beyond the count is
+    // not used), the queries as f16
+    constexpr int U = 4;  // tiles of 16 cells a wave has in flight (512 or 256 cells a trip; six: the same time, and spills)
+    const int col = lane & 15, quad = lane >> 4;
+    int pk[U], pv[NW == 8 ? NF_CAP / 64 : 1];
+#pragma unroll
+    for (int u = 0; u < U; ++u) pk[u] = pos[min(16 * (wave + u * NW) + col, n_kv - 1)];
+    if constexpr (NW == 8) {
+#pragma unroll
+        for (int j = 0; j < NF_CAP / 64; ++j) pv[j] = pos[min(64 * j + lane, n_kv - 1)];
+    }
+    half8 qa[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+        qa[s] = half8{};
+        if (col < G) {
+            const float * qr = (const float *) (q.data + (int64_t) tok * q.nb[1] + (int64_t) (kvh * G + col) * q.nb[2]) + 32 * s + 8 * quad;
+            const float4 x = *(const float4 *) qr, y = *(const float4 *) (qr + 4);
+            qa[s] = (half8){(_Float16) x.x, (_Float16) x.y, (_Float16) x.z, (_Float16) x.w, (_Float16) y.x, (_Float16) y.y, (_Float16) y.z, (_Float16) y.w};
+        }
+    }
+    const int cnt = lt[0];
     float * sc = scratch + (((int64_t) tok * nkv_heads + kvh) * dq_n + dq) * (int64_t) G * n_kv;  // [G][n_kv], the first cnt of each row in use
     const int rows_per = D / dq_n, d0 = dq * rows_per;
     auto out_ptr = [&](const int g, const int d) { return (float *) (dst.data + (int64_t) d * dst.nb[0] + (int64_t) tok * dst.nb[1] + (int64_t) (kvh * G + g) * dst.nb[2]); };
@@ -64,101 +87,155 @@ __global__ void __launch_bounds__(NW * 64) k_attn_nf_list(const tdesc q, const t
     const char * mrow = mask.data + (int64_t) tok * mask.nb[1];
     const bool m16 = mask.type == GGML_TYPE_F16;
     const char * vbase = v.data + (int64_t) kvh * v.nb[2];
-    // ---- up to NF_CAP visible cells (every -np decode step): everything stays on chip.  A thread owns cells tid, tid + NT, ..: it reads
-    // their K rows whole (16 independent 16-byte loads, the q rows come from LDS by broadcast), so a logit needs no cross-lane sum and
-    // the soft-max runs on registers; probabilities and positions go to LDS for step 3.  (The first version walked the list with one
-    // dependent load pair per trip in every phase: 102 us per launch, all of it memory latency.)
+    // ---- up to NF_CAP visible cells (every -np decode step): everything stays on chip.
     if (cnt <= NF_CAP) {
-        float * qs = nf_smem;                       // [G][128] q rounded to f16
         int * pos_s = (int *) (nf_smem + G * D);    // [NF_CAP]
         float * p_s = nf_smem + G * D + NF_CAP;     // [G][NF_CAP]
-        for (int e = tid; e < G * D; e += NT) {
-            const int g = e / D, i = e % D;
-            qs[e] = h2f(f2h(*((const float *) (q.data + (int64_t) tok * q.nb[1] + (int64_t) (kvh * G + g) * q.nb[2]) + i)));
-        }
-        for (int c = tid; c < cnt; c += NT) pos_s[c] = pos[c];
-        __syncthreads();
-        float mx[G];
-#pragma unroll
-        for (int g = 0; g < G; ++g) mx[g] = -INFINITY;
-        const char * kbase = k.data + (int64_t) kvh * k.nb[2];
+        if (NW == 4)
+            for (int c = tid; c < cnt; c += NT) pos_s[c] = pos[c];
+        // 1. The logits on the matrix cores: tiles of 16 cells (columns) against the heads (rows, the first G of 16), K = 128 in four instructions whose operands lie in memory as a lane needs them:
+        // 16 bytes of a K row.  f16 products, f32 sums.  U tiles of a wave are requested before the first is used; then `requested` issues what else has to be on its way meanwhile.
+        auto logits = [&](auto && requested) {
+            if (16 * wave >= cnt) {
+                requested();
+                return;
+            }
+            const char * kbase = k.data + (int64_t) kvh * k.nb[2];
+            const uint32_t knb = (uint32_t) k.nb[1];  // (the launch checks that offsets fit 32 bits: half the registers for addresses)
 #pragma unroll 1
-        for (int c = tid; c < cnt; c += NT) {
-            const int pc = pos_s[c];
-            const uint4 * kr = (const uint4 *) (kbase + (int64_t) pc * k.nb[1]);
-            uint4 kv[16];  // the K row: 128 halves, all 16 loads in flight
+            for (int t0 = wave; 16 * t0 < cnt; t0 += NW * U) {
+                half8 kf[U][4];
+                float mv[U];
 #pragma unroll
-            for (int u = 0; u < 16; ++u) kv[u] = kr[u];
-            const float mv = m16 ? h2f(((const uint16_t *) mrow)[pc]) : ((const float *) mrow)[pc];
-            // one head at a time (a real loop: unrolled over G, the scheduler reads all 128 G values of q ahead — 512 registers and spills
-            // at G = 4); the logit goes straight to its LDS slot
-#pragma unroll 1
-            for (int g = 0; g < G; ++g) {
-                const float * qg = qs + g * D;
-                float s0 = 0.0f, s1 = 0.0f;
+                for (int u = 0; u < U; ++u) {
+                    const int c = 16 * (t0 + u * NW) + col;
+                    if (16 * (t0 + u * NW) < cnt) {
+                        const uint32_t pc = c >= cnt ? 0 : (t0 == wave ? pk[u] : pos[c]);  // (beyond the list: cell 0, whose logit is not stored)
 #pragma unroll
-                for (int u = 0; u < 16; ++u) {
-                    const uint32_t uu[4] = {kv[u].x, kv[u].y, kv[u].z, kv[u].w};
-                    const float4 q0 = *(const float4 *) (qg + 8 * u), q1 = *(const float4 *) (qg + 8 * u + 4);
-                    s0 = fmaf(h2f((uint16_t) (uu[0] & 0xFFFF)), q0.x, s0); s1 = fmaf(h2f((uint16_t) (uu[0] >> 16)), q0.y, s1);
-                    s0 = fmaf(h2f((uint16_t) (uu[1] & 0xFFFF)), q0.z, s0); s1 = fmaf(h2f((uint16_t) (uu[1] >> 16)), q0.w, s1);
-                    s0 = fmaf(h2f((uint16_t) (uu[2] & 0xFFFF)), q1.x, s0); s1 = fmaf(h2f((uint16_t) (uu[2] >> 16)), q1.y, s1);
-                    s0 = fmaf(h2f((uint16_t) (uu[3] & 0xFFFF)), q1.z, s0); s1 = fmaf(h2f((uint16_t) (uu[3] >> 16)), q1.w, s1);
+                        for (int s = 0; s < 4; ++s) kf[u][s] = *(const half8 *) (kbase + (pc * knb + 64u * s + 16u * quad));
+                        mv[u] = m16 ? h2f(((const uint16_t *) mrow)[pc]) : ((const float *) mrow)[pc];
+                    }
                 }
-                float t = (s0 + s1) * scale;
-                t += mv;
-                p_s[g * NF_CAP + c] = t;  // (this thread's own slot until the probabilities are published below)
+                if (t0 == wave) requested();
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const int c = 16 * (t0 + u * NW) + col;
+                    if (16 * (t0 + u * NW) < cnt) {
+                        f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                        for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(qa[s], kf[u][s], acc, 0, 0, 0);
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+                            if (4 * quad + r < G && c < cnt) p_s[(4 * quad + r) * NF_CAP + c] = acc[r] * scale + mv[u];
+                    }
+                }
             }
-        }
-        for (int c = tid; c < cnt; c += NT) {
+        };
+        // 2. The soft-max, a head a wave: its logits (at most 16 a lane) stay in registers from the maximum to the probabilities.
+        auto soft_max = [&]() {
+            __syncthreads();
+#pragma unroll 1
+            for (int g = wave; g < G; g += NW) {
+                float * row = p_s + g * NF_CAP + lane;
+                float e[NF_CAP / 64];
+                float mx = -INFINITY;
 #pragma unroll
-            for (int g = 0; g < G; ++g) mx[g] = fmaxf(mx[g], p_s[g * NF_CAP + c]);
-        }
-        __shared__ float shm[NW][G];
-        __shared__ double shs[NW][G];
+                for (int jj = 0; jj < NF_CAP / 64; jj += 4)
+                    if (64 * jj < cnt) {
 #pragma unroll
-        for (int g = 0; g < G; ++g) {
-            const float t = wave_max(mx[g]);
-            if (lane == 0) shm[wave][g] = t;
-        }
-        __syncthreads();
-        double sum[G];
+                        for (int j = jj; j < jj + 4; ++j) {
+                            e[j] = 64 * j + lane < cnt ? row[64 * j] : -INFINITY;
+                            mx = fmaxf(mx, e[j]);
+                        }
+                    }
+                mx = wave_max(mx);
+                double sum = 0.0;
 #pragma unroll
-        for (int g = 0; g < G; ++g) {
-            mx[g] = shm[0][g];
+                for (int jj = 0; jj < NF_CAP / 64; jj += 4)
+                    if (64 * jj < cnt) {
 #pragma unroll
-            for (int w = 1; w < NW; ++w) mx[g] = fmaxf(mx[g], shm[w][g]);
-            sum[g] = 0.0;
-        }
-        for (int c = tid; c < cnt; c += NT) {
+                        for (int j = jj; j < jj + 4; ++j) e[j] = 64 * j + lane < cnt ? expf(e[j] - mx) : 0.0f;
+                        sum += ((double) e[jj] + (double) e[jj + 1]) + ((double) e[jj + 2] + (double) e[jj + 3]);
+                    }
+                sum = wave_sum_d(sum);
+                if (isnan(sum) || sum == 0.0) sum = -INFINITY;
+                const float inv = (float) (1.0 / sum);
 #pragma unroll
-            for (int g = 0; g < G; ++g) {
-                const float e = expf(p_s[g * NF_CAP + c] - mx[g]);
-                p_s[g * NF_CAP + c] = e;
-                sum[g] += (double) e;
+                for (int jj = 0; jj < NF_CAP / 64; jj += 4)
+                    if (64 * jj < cnt) {
+#pragma unroll
+                        for (int j = jj; j < jj + 4; ++j) row[64 * j] = 64 * j + lane < cnt ? h2f(f2h(e[j] * inv)) : 0.0f;  // (zeros to the end of a 256-cell group: step 3 reads whole ones)
+                    }
             }
-        }
+            __syncthreads();
+        };
+        // 3. V^T.p with eight waves (two slices and more: 64 rows at the most, two to eight a wave), lanes take cells: the first 32 loads of a lane, 1024 to 256 cells, are requested with the K rows and arrive during the soft-max.
+        auto vtp8 = [&](auto rb_tag) {
+            constexpr int RB = decltype(rb_tag)::value, J = 32 / RB;
+            const char * vr0 = vbase + (int64_t) (d0 + wave * RB) * v.nb[1];
+            const int p0 = __builtin_amdgcn_readfirstlane(pv[0]);
+            uint16_t xv[RB][J];
+            auto request = [&](const int c0) {  // (lanes beyond the list: its first cell, times a probability of 0)
 #pragma unroll
-        for (int g = 0; g < G; ++g) {
-            const double t = wave_sum_d(sum[g]);
-            if (lane == 0) shs[wave][g] = t;
-        }
-        __syncthreads();
+                for (int jj = 0; jj < J; jj += 4)
+                    if (c0 + 64 * jj < cnt) {
 #pragma unroll
-        for (int g = 0; g < G; ++g) {
-            double t = shs[0][g];
+                        for (int j = jj; j < jj + 4; ++j) {
+                            const uint32_t pc = c0 + 64 * j + lane < cnt ? pv[c0 / 64 + j] : p0;
 #pragma unroll
-            for (int w = 1; w < NW; ++w) t += shs[w][g];
-            if (isnan(t) || t == 0.0) t = -INFINITY;
-            const float inv = (float) (1.0 / t);
-            for (int c = tid; c < cnt; c += NT) p_s[g * NF_CAP + c] = h2f(f2h(p_s[g * NF_CAP + c] * inv));
+                            for (int r = 0; r < RB; ++r) xv[r][j] = *(const uint16_t *) ((vr0 + (int64_t) r * v.nb[1]) + 2u * pc);
+                        }
+                    }
+            };
+            logits([&] { request(0); });
+            soft_max();
+            float acc[RB][G];
+#pragma unroll
+            for (int r = 0; r < RB; ++r)
+#pragma unroll
+                for (int g = 0; g < G; ++g) acc[r][g] = 0.0f;
+#pragma unroll
+            for (int c0 = 0; c0 < NF_CAP; c0 += 64 * J) {
+                if (c0) request(c0);
+#pragma unroll
+                for (int jj = 0; jj < J; jj += 4)
+                    if (c0 + 64 * jj < cnt) {
+#pragma unroll
+                        for (int j = jj; j < jj + 4; ++j) {
+                            float pp[G];
+#pragma unroll
+                            for (int g = 0; g < G; ++g) pp[g] = p_s[g * NF_CAP + c0 + 64 * j + lane];
+#pragma unroll
+                            for (int r = 0; r < RB; ++r) {
+                                const float x = h2f(xv[r][j]);
+#pragma unroll
+                                for (int g = 0; g < G; ++g) acc[r][g] = fmaf(x, pp[g], acc[r][g]);
+                            }
+                        }
+                    }
+            }
+#pragma unroll
+            for (int r = 0; r < RB; ++r)
+#pragma unroll
+                for (int g = 0; g < G; ++g) {
+                    const float t = wave_sum(acc[r][g]);
+                    if (lane == 0) put(g, d0 + wave * RB + r, t);
+                }
+        };
+        if constexpr (NW == 8) {
+            if (rows_per == 64) vtp8(std::integral_constant<int, 8>{});
+            else if (rows_per == 32) vtp8(std::integral_constant<int, 4>{});
+            else vtp8(std::integral_constant<int, 2>{});
+            finish();
+            return;
         }
-        __syncthreads();
+        logits([] {});
+        soft_max();
         // 3. V^T.p: lanes take cells (4 per lane and group of 256), a wave takes RB rows of the transposed cache at a time — all RB x 4 two-byte
         // loads of a block are requested before the first is used (one row pair at a time, each trip waited for its own loads: 16 round
         // trips per wave were 30 of the launch's 52 us)
         auto vtp = [&](auto rb_tag) {
-        constexpr int RB = decltype(rb_tag)::value, J = NW == 4 ? 4 : 16 / RB;  // cells a lane takes per trip
+        constexpr int RB = decltype(rb_tag)::value, J = 4;  // cells a lane takes per trip
         for (int r0 = wave * RB; r0 < rows_per; r0 += NW * RB) {
             float acc[RB][G];
 #pragma unroll
@@ -287,11 +364,7 @@ __global__ void __launch_bounds__(NW * 64) k_attn_nf_list(const tdesc q, const t
             finish();
             return;
         }
-        if constexpr (NW == 8) {  // (two slices and more: 64 rows at the most, two to eight a wave, sixteen loads a row group in flight)
-            if (rows_per >= 64) vtp(std::integral_constant<int, 8>{});
-            else if (rows_per >= 32) vtp(std::integral_constant<int, 4>{});
-            else vtp(std::integral_constant<int, 2>{});
-        } else if (G <= 4 && rows_per >= 64) vtp(std::integral_constant<int, 16>{});
+        if (G <= 4 && rows_per >= 64) vtp(std::integral_constant<int, 16>{});
         else if (rows_per >= 32) vtp(std::integral_constant<int, 8>{});
         else vtp(std::integral_constant<int, 4>{});
         finish();
@@ -402,8 +475,14 @@ size_t attn_nf_list_scratch_bytes(const tdesc & q, const tdesc & k, int * dq_out
     // when the cache holds at most NF_CAP cells per token of the batch — the decode steps of many sequences — and a few tokens over
     // long contexts stay on the dense kernels.
     if (n_kv > (int64_t) NF_CAP * T) return 0;
+    // Slices of the head dimensions: enough workgroups for the chip when the tokens are few.  But each slice fetches all the K rows again, and only whole rows leave as Q8_K blocks: from 80
+    // (token, KV head) pairs on whole rows are faster while a token sees 256 cells at the most (512 from 160 pairs on).  A step of Llama-3-8B, us, slices / whole rows: 12 sequences of 160 cells
+    // 2957 / 2816, 16 of 160 3017 / 2882, of 300 3074 / 3110, 20 of 380 3610 / 3517, 8 of 150 2703 / 2729; Qwen2-7B, 30 of 100 4036 / 3846.  Measured with four and seven heads on a KV head and
+    // from 64 cells a token on; others keep their slices.
     int dq = 1;
-    while (dq < 8 && T * NKV * dq < 192) dq *= 2;  // slices of the head dimensions: enough workgroups for the chip when the tokens are few
+    const int64_t pairs = T * NKV;
+    const bool whole = G >= 4 && pairs >= 80 && n_kv >= 64 * T && n_kv <= (pairs >= 160 ? 512 : 256) * T;
+    while (!whole && dq < 8 && pairs * dq < 192) dq *= 2;
     if (dq_out) *dq_out = dq;
     return (size_t) (T * NKV * dq * G * n_kv) * sizeof(float);
 }
@@ -418,16 +497,21 @@ bool launch_attn_nf_list(hipStream_t s, const tdesc & q, const tdesc & k, const 
     if (v.ne[0] != k.ne[1] || v.ne[1] != 128 || v.ne[2] != k.ne[2] || v.ne[3] != 1) return false;
     if ((k.nb[1] % 16) || (k.nb[2] % 16) || (((uintptr_t) k.data) & 15) || (q.nb[1] % 16) || (q.nb[2] % 16) || (((uintptr_t) q.data) & 15)) return false;
     if ((mask.type != GGML_TYPE_F16 && mask.type != GGML_TYPE_F32) || mask.ne[0] < k.ne[1] || mask.ne[1] < q.ne[1] || mask.ne[2] != 1 || mask.ne[3] != 1) return false;
+    if (k.ne[1] * k.nb[1] > INT32_MAX) return false;  // (32-bit offsets)
     const int G = (int) (q.ne[2] / k.ne[2]);
     if (q8_out && (dq != 1 || (G & 1))) return false;  // Q8_K blocks are head pairs of whole rows
     static const int groups_on = !getenv("GGML_MI355X_NF_GROUPS") || atoi(getenv("GGML_MI355X_NF_GROUPS")) != 0;
     dim3 grid((unsigned) q.ne[1], (unsigned) k.ne[2], (unsigned) dq);
-    // Few tokens: every slice of the head dimensions computes ALL the logits of its heads, one wave a SIMD, and that is most of the launch.  While the grid is no more than
-    // one workgroup a CU, eight waves share the logits and the gathers (3 tokens x 700 cells of Llama-3-8B: 26.5 -> 19.5 us a launch; with sixteen waves, 128 registers
-    // and spills, 29.2); more workgroups than that already have the company of another (20 tokens: a step of 3.9 ms with four waves, 4.0 with eight).
+    // Few tokens: every slice of the head dimensions computes all the logits of its heads.  While the grid is no more than one workgroup a CU, eight waves share the fetches (3 tokens x 700 cells of
+    // Llama-3-8B, a launch: 26.5 us with four waves, 19.5 with eight; with the logits on the matrix cores, V^T requested ahead and a head's soft-max in one wave's registers 13.5: of these 6
+    // wait for the 200 KB a workgroup fetches, whatever its mapping to XCDs or the shape of its loads); more workgroups than that already have the company of another.
     const bool few = dq > 1 && q.ne[1] * k.ne[2] * dq <= 256;
-#define NF_GO(G_, W_) hipLaunchKernelGGL((k_attn_nf_list<G_, W_>), grid, dim3(W_ * 64), (size_t) (G_ * 128 + NF_CAP + G_ * NF_CAP) * 4, s, q, k, v, mask, dst, lists, list_stride, scratch, scale, dq, (q8k_dev *) q8_out, groups_on)
-#define NF(G_) case G_: if (few) NF_GO(G_, 8); else NF_GO(G_, 4); return true;
+#define NF_GO(G_, W_)                                                                                                                                                              \
+    {                                                                                                                                                                              \
+        constexpr size_t lds = (size_t) (G_ * 128 + NF_CAP + G_ * NF_CAP) * 4;                                                                                   \
+        hipLaunchKernelGGL((k_attn_nf_list<G_, W_>), grid, dim3(W_ * 64), lds, s, q, k, v, mask, dst, lists, list_stride, scratch, scale, dq, (q8k_dev *) q8_out, groups_on);      \
+    }
+#define NF(G_) case G_: if (few) NF_GO(G_, 8) else NF_GO(G_, 4) return true;
     switch (G) { NF(1) NF(2) NF(3) NF(4) NF(5) NF(6) NF(7) NF(8) default: break; }
 #undef NF
 #undef NF_GO

@@ -317,3 +317,47 @@ def test_splits_of_few_tokens(backend, H, T_, n_kv, NH, NKV, HD, seen):
         ref = (p / p.sum(1, keepdims=True)) @ v[h // (NH // NKV)].astype(np.float64)
         # (scores are f32 sums over packed f16 products, the probabilities packed f16: 2^-10 of a weight, as the few-token tests above)
         assert np.abs(got[:, h] - ref).max() <= 2e-3 * np.abs(ref).max() + 1e-5, h
+
+
+# trips of 512 cells with eight waves (16, 32 and 64 rows of V^T a workgroup) and of 256 with four, the last tile and the last trip in part, waves without a tile; whole rows from 80 pairs of
+# a token and a key head and 64 cells a token on (their 256- and 512-cell limits on both sides)
+@pytest.mark.parametrize("T_,NKV,G,per", [
+    (2, 8, 4, 17), (3, 8, 5, 513), (4, 8, 4, 1024), (6, 8, 3, 129), (6, 8, 8, 1000), (12, 8, 1, 1023), (14, 8, 6, 257), (10, 8, 4, 64), (10, 8, 7, 250), (10, 8, 4, 260), (20, 8, 4, 500), (20, 8, 5, 520), (9, 8, 4, 100)])
+def test_few_tokens_on_matrix_cores(backend, H, T_, NKV, G, per):
+    """attn_nf.hip; infinities and NaN in cells that a token does not see stay out of its result"""
+    rng = np.random.default_rng(T_ + 31 * per + G)
+    HD, NH = 128, NKV * G
+    n_kv = max(256, (T_ * per + 255) // 256 * 256)
+    k = rng.standard_normal((n_kv, NKV, HD)).astype(np.float16)
+    v = rng.standard_normal((NKV, HD, n_kv)).astype(np.float16)
+    q = (3 * rng.standard_normal((T_, NH, HD))).astype(np.float32)
+    mask = np.full((T_, n_kv), -np.inf, np.float32)
+    cells = rng.permutation(n_kv)[:T_ * per - 4]
+    for t in range(T_):
+        own = cells[t::T_]
+        mask[t, own] = np.where(np.arange(len(own)) % 3, 0, -0.5)
+    hidden = np.setdiff1d(np.arange(n_kv), cells)
+    k[hidden], v[:, :, hidden] = np.inf, np.nan
+
+    def build(g):
+        kc, vc = g.new(L.F16, [NKV * HD, n_kv], k.reshape(n_kv, -1)), g.new(L.F16, [n_kv, NKV * HD], v.reshape(-1, n_kv))
+        qp = H.ggml_permute(g.ctx, g.new(L.F32, [HD, NH, T_], q), 0, 2, 1, 3)
+        kv = H.ggml_view_3d(g.ctx, kc, HD, n_kv, NKV, NKV * HD * 2, HD * 2, 0)
+        vv = H.ggml_view_3d(g.ctx, vc, n_kv, HD, NKV, n_kv * 2, n_kv * 2 * HD, 0)
+        p = H.ggml_soft_max_ext(g.ctx, H.ggml_mul_mat(g.ctx, kv, qp), g.new(L.F32, [n_kv, T_], mask), HD ** -0.5, 0.0)
+        return H.ggml_mul_mat(g.ctx, vv, p)
+
+    s0 = backend.stat("kernel_launches")
+    got = T.run_case(build, backend)[0].reshape(NH, T_, HD)
+    assert backend.stat("kernel_launches") - s0 <= 2
+    qh = q.astype(np.float16).astype(np.float64)
+    for t in range(T_):
+        see = np.flatnonzero(mask[t] > -1)
+        kt, vt = k[see].astype(np.float64), v[:, :, see].astype(np.float64)
+        for h in range(NH):
+            s = kt[:, h // G] @ qh[t, h] * HD ** -0.5 + mask[t, see]
+            p = np.exp(s - s.max())
+            p = (p / p.sum()).astype(np.float16).astype(np.float64)
+            ref = vt[h // G] @ p
+            # f32 sums; a probability next to a rounding boundary may round the other way: 2^-11 of it
+            assert np.abs(got[h, t] - ref).max() <= 2e-3 * np.abs(ref).max() + 1e-5, (t, h)
