@@ -159,6 +159,7 @@ struct stats {
     int64_t kv_native_nodes = 0;       // ... and those whose K / V in such a type were read in place by the lane-parallel kernel's DQ form
     int64_t attn_f32_nodes = 0;        // FLASH_ATTN_EXT nodes served by the 32-bit kernel over f32 / bf16 / f16 rows read in place (attn_f32.hip)
     int64_t kv_image_nodes = 0;        // FLASH_ATTN_EXT nodes whose K / V (kept in q4_0, q4_1, q5_0, q5_1, iq4_nl, bf16, f32 ...) were read through an f16 image
+    int64_t staged_uploads = 0;        // set_tensor_async calls whose copy over the link ran beside a graph (backend.cpp: stage_upload)
     int64_t kernel_downloads = 0;      // get_tensor_async calls served by a copy kernel writing mapped pinned memory
     int64_t graph_early_captures = 0;  // graphs captured at their FIRST sighting (same step as the one replayed last, over a grown cache)
     int64_t graph_shadow_captures = 0; // ... of which the capture ran behind the step's own eager launches (the GPU busy meanwhile) and serves the NEXT step
@@ -243,6 +244,15 @@ struct backend_ctx {
     // tiny kernel — a blit through hipMemcpyAsync costs ~25 us of stream time per copy, five of them per decode step
     char * up_ring = nullptr;
     size_t up_cap = 0, up_head = 0;
+    // larger uploads while the stream is busy (backend.cpp: stage_upload): a copy stream of its own and device buffers that the copies wait in
+    struct up_slot { char * buf = nullptr; size_t cap = 0; hipEvent_t filled = nullptr; };
+    static constexpr int UP_SLOTS = 8;
+    hipStream_t up_stream = nullptr;
+    up_slot up_slots[UP_SLOTS];
+    hipEvent_t up_round = nullptr;
+    int up_used = 0;       // slots whose contents may not have been taken yet: since the last synchronize, or the last wait of up_stream for the stream
+    bool up_behind = false;  // a graph entered the stream since the last synchronize
+    bool up_off = false;     // (could not be set up)
     upload_batch up_pending{};  // staged in the ring, not yet launched: flushed as ONE kernel before anything else enters the stream
     // attention over a unified cache with a few query tokens: per-token lists of visible tiles (fattn.hip, k_fattn_tile_scan),
     // built once per graph execution and shared by the attention nodes of all layers

@@ -2375,8 +2375,15 @@ struct llm_context {
     int pin_out_rows = 0;
     // micro-batches without outputs are not waited for (as llama.cpp: the wait happens when results are fetched); each
     // in-flight micro-batch keeps its own input slot, so the host builds and stages batch i+1 while the GPU runs batch i
+    // (only the slot's own micro-batch is waited for, on its event: a full wait before the fourth of four micro-batches left the GPU idle while the host filled its masks, 213 of 2950 us)
     static constexpr int PIN_SLOTS = 4;
     int pin_slot = 0, in_flight = 0;
+    ggml_backend_event_t pin_ev[PIN_SLOTS] = {};  // recorded behind the slot's micro-batch where the same call comes round to the slot again (a record costs the stream some 10 us)
+    bool pin_busy[PIN_SLOTS] = {}, pin_recorded[PIN_SLOTS] = {};
+    void all_done() {  // after a full wait
+        in_flight = 0;
+        for (bool & b : pin_busy) b = false;
+    }
     // -sm layer (llm_context_new_layer_split): one graph segment per device, driven the way ggml_backend_sched drives the splits of a
     // layer-split model — input copies in LS_COPIES slots per device, cpy_tensor_async of the residual stream between neighbouring
     // devices, one event per (device, slot) recorded after the segment's graph and waited for before the slot is overwritten
@@ -3389,6 +3396,7 @@ extern "C" struct llm_context * llm_context_new(struct llm_model * m, ggml_backe
             if (c->buf_pin) {
                 c->pin = (char *) ggml_backend_buffer_get_base(c->buf_pin);
                 c->pin_in_bytes = in_bytes;
+                for (ggml_backend_event_t & e : c->pin_ev) e = ggml_backend_event_new(backend->device);
             }
         }
     }
@@ -3411,6 +3419,8 @@ extern "C" void llm_context_free(struct llm_context * c) {
     }
     if (c->ctx_compute) ggml_free(c->ctx_compute);
     if (c->galloc) ggml_gallocr_free(c->galloc);
+    for (ggml_backend_event_t e : c->pin_ev)
+        if (e) ggml_backend_event_free(e);
     if (c->buf_pin) ggml_backend_buffer_free(c->buf_pin);
     if (c->buf_kv) ggml_backend_buffer_free(c->buf_kv);
     if (c->ctx_kv) ggml_free(c->ctx_kv);
@@ -3438,7 +3448,7 @@ static int kv_apply_shift(llm_context * c, const std::vector<int32_t> & delta) {
     llm_model * m = c->model;
     const llm_hparams & hp = m->hp;
     const int64_t HD = hp.n_embd_head, NKV = m->n_head_kv_l, n_ctx = c->p.n_ctx;
-    if (c->backend && c->in_flight) { ggml_backend_synchronize(c->backend); c->in_flight = 0; }
+    if (c->backend && c->in_flight) { ggml_backend_synchronize(c->backend); c->all_done(); }
     ggml_context * ctx = ggml_init({0, nullptr, true});
     ggml_cgraph * gf = ggml_new_graph_custom(ctx, 1024, false);
     ggml_tensor * shift = ggml_new_tensor_1d(ctx, GGML_TYPE_I32, n_ctx);
@@ -3666,7 +3676,7 @@ static int decode_ubatch_ls(llm_context * c, int n_tokens, const int32_t * token
 }
 
 static int decode_ubatch(llm_context * c, int n_tokens, const int32_t * tokens, const int32_t * pos, const int32_t * seq_id, const int8_t * want, float * logits_out, int * n_out_acc,
-                         bool defer_sync) {
+                         bool defer_sync, bool slot_again) {
     llm_model * m = c->model;
     const llm_hparams & hp = m->hp;
     const int n_ctx = c->p.n_ctx;
@@ -3777,11 +3787,17 @@ static int decode_ubatch(llm_context * c, int n_tokens, const int32_t * tokens, 
     // inputs: filled straight into the pinned staging area and uploaded asynchronously on the backend's stream (the copies
     // and the graph are stream-ordered); without a device backend (CPU oracle) the plain blocking setter is used
     const bool async_io = c->backend != nullptr && c->pin != nullptr;
-    if (async_io && c->in_flight >= llm_context::PIN_SLOTS - 1) {  // the slot about to be re-used may still be in flight
-        ggml_backend_synchronize(c->backend);
-        c->in_flight = 0;
+    const int slot = c->pin_slot;
+    if (async_io && c->pin_busy[slot]) {  // its last micro-batch may still be in flight
+        if (c->pin_recorded[slot]) {
+            ggml_backend_event_synchronize(c->pin_ev[slot]);
+            c->pin_busy[slot] = false;
+        } else {
+            ggml_backend_synchronize(c->backend);
+            c->all_done();
+        }
     }
-    char * const pin_in = c->pin ? c->pin + (size_t) c->pin_slot * c->pin_in_bytes : nullptr;
+    char * const pin_in = c->pin ? c->pin + (size_t) slot * c->pin_in_bytes : nullptr;
     char * const pin_out = c->pin ? c->pin + (size_t) llm_context::PIN_SLOTS * c->pin_in_bytes : nullptr;
     c->pin_slot = (c->pin_slot + 1) % llm_context::PIN_SLOTS;
     size_t pin_at = 0;
@@ -3877,9 +3893,12 @@ static int decode_ubatch(llm_context * c, int n_tokens, const int32_t * tokens, 
         if (st == GGML_STATUS_SUCCESS && async_out) ggml_backend_tensor_get_async(c->backend, c->t_logits, direct_out ? (void *) logits_out : (void *) pin_out, 0, logit_bytes);
         if (n_outputs > 0 || st != GGML_STATUS_SUCCESS || !defer_sync) {
             ggml_backend_synchronize(c->backend);
-            c->in_flight = 0;
+            c->all_done();
         } else {
             c->in_flight++;
+            c->pin_busy[slot] = true;
+            c->pin_recorded[slot] = slot_again && c->pin_ev[slot];
+            if (c->pin_recorded[slot]) ggml_backend_event_record(c->pin_ev[slot], c->backend);
         }
     } else {
         st = c->backend ? ggml_backend_graph_compute(c->backend, c->gf) : c->compute(c->gf, c->p.n_threads);
@@ -3929,9 +3948,9 @@ extern "C" int llm_decode(struct llm_context * c, int n_tokens, const int32_t * 
     for (int i0 = 0; i0 < n_tokens; i0 += c->p.n_ubatch) {
         const int n = std::min(c->p.n_ubatch, n_tokens - i0);
         int rc = decode_ubatch(c, n, tokens + i0, pos + i0, seq_id ? seq_id + i0 : nullptr, want_logits ? want_logits + i0 : nullptr,
-                               c->logits_base + (size_t) c->n_outputs * c->model->n_vocab_l, &c->n_outputs, /*defer_sync=*/i0 + n < n_tokens);
+                               c->logits_base + (size_t) c->n_outputs * c->model->n_vocab_l, &c->n_outputs, /*defer_sync=*/i0 + n < n_tokens, /*slot_again=*/n_tokens - i0 > llm_context::PIN_SLOTS * c->p.n_ubatch);
         if (rc != 0) {
-            if (c->backend && c->in_flight) { ggml_backend_synchronize(c->backend); c->in_flight = 0; }
+            if (c->backend && c->in_flight) { ggml_backend_synchronize(c->backend); c->all_done(); }
             if (!c->ls.empty()) ls_sync_all(c);
             return rc;
         }
@@ -3939,7 +3958,7 @@ extern "C" int llm_decode(struct llm_context * c, int n_tokens, const int32_t * 
     if (!c->ls.empty() && c->in_flight) ls_sync_all(c);
     if (c->backend && c->in_flight) {  // the call returns with everything finished
         ggml_backend_synchronize(c->backend);
-        c->in_flight = 0;
+        c->all_done();
     }
     return 0;
 }

@@ -930,3 +930,36 @@ def test_no_room_for_a_decode_copy_keeps_the_block_layout(backend, H, plog):
     plog(f"decode copy with / without room: {outs['room'][1]} / {outs['no room'][1]}")
     assert outs["room"][1]["decode_copy_tensors"] > 0 and outs["no room"][1]["decode_copy_tensors"] == 0 and outs["no room"][1]["decode_copy_launches"] == 0
     assert np.array_equal(outs["room"][0].view(np.uint32), outs["no room"][0].view(np.uint32))
+
+
+@pytest.mark.parametrize("fa,n", [(1, 5000), (0, 1800)])
+def test_micro_batches_back_to_back(backend, H, fa, n):
+    """A prompt of more micro-batches than the host has input slots and the backend has buffers for uploads (masks of 1 to 10 MB copied beside the graph before), against the same micro-batches
+    decoded one call after the other (nothing in flight): the same bits, also of a second prompt and of a token behind it."""
+    m = Model(preset("test-llama", n_ctx_train=8192), 5, backend.buft)
+    rng = np.random.default_rng(n)
+    c1, c2 = (Context(m, backend=backend, n_ctx=5632, flash_attn=fa) for _ in range(2))
+    try:
+        for _ in range(2):
+            toks = [int(t) for t in rng.integers(0, 500, n)]
+            s0 = backend.stat("staged_uploads")
+            rc, together = c1.decode(toks, range(n), want=[0] * (n - 1) + [1])
+            assert rc == 0
+            staged = backend.stat("staged_uploads") - s0
+            assert staged <= (n - 1) // 512
+            s0 = backend.stat("staged_uploads")
+            for i in range(0, n, 512):
+                part = toks[i:i + 512]
+                rc, single = c2.decode(part, range(i, i + len(part)), want=[0] * (len(part) - 1) + [1 if i + 512 >= n else 0])
+                assert rc == 0
+            assert backend.stat("staged_uploads") == s0
+            assert np.array_equal(together.view(np.uint32), single.view(np.uint32))
+            (_, a), (_, b) = (c.decode([7], [n]) for c in (c1, c2))
+            assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+            c1.clear()
+            c2.clear()
+        assert staged > 0
+    finally:
+        c1.free()
+        c2.free()
+        m.free()
