@@ -512,7 +512,7 @@ __global__ void __launch_bounds__(WV * 64) k_fattn_dec128(const tdesc q, const t
 
     // a trip covers NG*16 consecutive positions: position of (u, wave, sub) = p0 + u*16 + wave*4 + sub
     uint4 kraw[NG], vraw[NG];
-    float mvl = 0.0f;   // mask value / validity of THIS lane's pair (ul, sub)
+    uint16_t mvl = 0;   // mask value / validity of THIS lane's pair (ul, sub): as loaded - converted here, it was waited for on the spot, and with it everything that the trip had requested
     bool okl = false;
     int p0 = LIST ? ti * TRIP : kv0;
 #define FA_LOAD_TRIP()                                                                  \
@@ -525,9 +525,9 @@ __global__ void __launch_bounds__(WV * 64) k_fattn_dec128(const tdesc q, const t
             if constexpr (DQ) {  /* the raw octet of this lane's block, whatever the type */ \
                 kraw[u] = kv_load_octet_raw_t<KVT>(kp_, sl & 3);                        \
                 vraw[u] = kv_load_octet_raw_t<KVT>(vp_, sl & 3);                        \
-            } else if constexpr (Q8) {  /* 8 quants (2-byte aligned) + the block's f16 scale */  \
-                kraw[u] = make_uint4(ld32_a2(kp_), ld32_a2(kp_ + 4), (uint32_t) ld16(kp_ - 2 - (sl & 3) * 8), 0u);  \
-                vraw[u] = make_uint4(ld32_a2(vp_), ld32_a2(vp_ + 4), (uint32_t) ld16(vp_ - 2 - (sl & 3) * 8), 0u);  \
+            } else if constexpr (Q8) {  /* 8 quants (2-byte aligned) + the block's f16 scale: as the dword it begins, since a halfword would be widened, and waited for, here */  \
+                kraw[u] = make_uint4(ld32_a2(kp_), ld32_a2(kp_ + 4), ld32_a2(kp_ - 2 - (sl & 3) * 8), 0u);  \
+                vraw[u] = make_uint4(ld32_a2(vp_), ld32_a2(vp_ + 4), ld32_a2(vp_ - 2 - (sl & 3) * 8), 0u);  \
             } else {                                                                    \
                 kraw[u] = *(const uint4 *) kp_;                                         \
                 vraw[u] = *(const uint4 *) vp_;                                         \
@@ -541,7 +541,7 @@ __global__ void __launch_bounds__(WV * 64) k_fattn_dec128(const tdesc q, const t
             _Pragma("unroll") for (int u = 1; u < NG; ++u) plc_ = ul == u ? nidx[u] : plc_; \
             plc_ = okl ? plc_ : first;                                                  \
         }                                                                               \
-        mvl = mp ? h2f(mp[plc_]) : 0.0f;                                                \
+        mvl = mp ? mp[plc_] : (uint16_t) 0;                                             \
         if constexpr (LIST) FA_LIST_AHEAD(p0 + TRIP)                                    \
     }
     uint32_t vis = 0xFFFFFFFFu;  // bit i: trip i has a position this wave can see
@@ -722,7 +722,7 @@ __global__ void __launch_bounds__(WV * 64) k_fattn_dec128(const tdesc q, const t
         if (trip == 0) { asm volatile("" :: "v"(t[0]), "v"(t[15])); FA_STAMP_AT(3) }  // the first trip's K has arrived and its dot products are done
 #endif
         const bool more = p_next < kv1 && (!SKIP || ((vis >> (trip + 1)) & 1u));
-        const float mv_cur = mvl;
+        const uint16_t mv_raw = mvl;
         const bool ok_cur = okl;
         p0 = p_next;  // (nothing below uses the current trip's position)
         if (more) FA_LOAD_TRIP()  // long splits: the next trip's loads go out before the reductions
@@ -753,6 +753,7 @@ __global__ void __launch_bounds__(WV * 64) k_fattn_dec128(const tdesc q, const t
             sv = keep + dpp_f32<MI_DPP_QUAD_XOR1>(send);
         }
         // ---- softmax bookkeeping, once per lane for its own pair
+        const float mv_cur = h2f(mv_raw);
         sv = (ok_cur && !(mv_cur == -INFINITY)) ? fmaf(sv, sc2, mv_cur * LOG2E) : -INFINITY;
         float mx = sv;
         if constexpr (G <= 2) mx = fmaxf(mx, dpp_f32<MI_DPP_ROR2>(mx));
