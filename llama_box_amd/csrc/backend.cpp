@@ -605,9 +605,10 @@ static void be_free(ggml_backend_t be) {
         HIP_NOTE(hipStreamDestroy(c->up_stream));
     }
     for (backend_ctx::up_slot & u : c->up_slots) {
-        if (u.buf) HIP_NOTE(hipFree(u.buf));
+        if (u.cap > backend_ctx::UP_FIRST) HIP_NOTE(hipFree(u.buf));
         if (u.filled) HIP_NOTE(hipEventDestroy(u.filled));
     }
+    if (c->up_block) HIP_NOTE(hipFree(c->up_block));
     if (c->up_round) HIP_NOTE(hipEventDestroy(c->up_round));
     if (c->fa_lists) HIP_NOTE(hipFree(c->fa_lists));
     if (c->rope_tab) HIP_NOTE(hipFree(c->rope_tab));
@@ -640,35 +641,34 @@ static bool stage_upload(backend_ctx * c, char * dst, const void * data, size_t 
         c->up_off = true;
         return false;
     };
-    if (!c->up_stream && hipStreamCreateWithFlags(&c->up_stream, hipStreamNonBlocking) != hipSuccess) {
-        c->up_stream = nullptr;
-        return off();
+    if (!c->up_block) {
+        if (hipMalloc((void **) &c->up_block, backend_ctx::UP_SLOTS * backend_ctx::UP_FIRST) != hipSuccess) {
+            c->up_block = nullptr;
+            return off();
+        }
+        for (int i = 0; i < backend_ctx::UP_SLOTS; ++i) {
+            c->up_slots[i].buf = c->up_block + i * backend_ctx::UP_FIRST;
+            c->up_slots[i].cap = backend_ctx::UP_FIRST;
+        }
     }
     if (c->up_used == backend_ctx::UP_SLOTS) {  // all of them since the last synchronize: the copies wait for what the stream holds now, this once
-        if ((!c->up_round && hipEventCreateWithFlags(&c->up_round, hipEventDisableTiming) != hipSuccess) || hipEventRecord(c->up_round, c->stream) != hipSuccess ||
-            hipStreamWaitEvent(c->up_stream, c->up_round, 0) != hipSuccess)
-            return off();
+        if (hipEventRecord(c->up_round, c->stream) != hipSuccess || hipStreamWaitEvent(c->up_stream, c->up_round, 0) != hipSuccess) return off();
         c->up_used = 0;
     }
     backend_ctx::up_slot & u = c->up_slots[c->up_used];
-    if (!u.filled && hipEventCreateWithFlags(&u.filled, hipEventDisableTiming) != hipSuccess) {
-        u.filled = nullptr;
-        return off();
-    }
     if (u.cap < size) {
-        if (u.buf) {
-            HIP_SOFT(hipStreamSynchronize(c->stream));  // (its last copy out may be there)
-            HIP_NOTE(hipFree(u.buf));
-        }
-        u.buf = nullptr;
-        u.cap = 0;
-        size_t cap = (size_t) 4 << 20;  // (powers of two: a growing context does not replace its buffers at every micro-batch)
+        size_t cap = u.cap;  // (powers of two: a growing context does not replace its buffers at every micro-batch)
         while (cap < size) cap *= 2;
-        if (hipMalloc((void **) &u.buf, cap) != hipSuccess) {
-            u.buf = nullptr;
+        char * buf = nullptr;
+        if (hipMalloc((void **) &buf, cap) != hipSuccess) {
             (void) hipGetLastError();
             return false;
         }
+        if (u.cap > backend_ctx::UP_FIRST) {  // (not a part of the block)
+            HIP_SOFT(hipStreamSynchronize(c->stream));  // (its last copy out may be there)
+            HIP_NOTE(hipFree(u.buf));
+        }
+        u.buf = buf;
         u.cap = cap;
     }
     if (hipMemcpyAsync(u.buf, data, size, hipMemcpyHostToDevice, c->up_stream) != hipSuccess || hipEventRecord(u.filled, c->up_stream) != hipSuccess || hipStreamWaitEvent(c->stream, u.filled, 0) != hipSuccess)
@@ -832,6 +832,14 @@ static ggml_backend_t dev_init_backend(ggml_backend_dev_t dev, const char *) {
         MI_ERR("init_backend: no stream on device %d", d->device);
         delete c;
         return nullptr;
+    }
+    {   // the copy stream of stage_upload and its events: a stream's first use takes longer than the prompt that would find it missing
+        bool ok = hipStreamCreateWithFlags(&c->up_stream, hipStreamNonBlocking) == hipSuccess;
+        if (!ok) c->up_stream = nullptr;
+        ok = ok && hipEventCreateWithFlags(&c->up_round, hipEventDisableTiming) == hipSuccess;
+        for (backend_ctx::up_slot & u : c->up_slots) ok = ok && hipEventCreateWithFlags(&u.filled, hipEventDisableTiming) == hipSuccess;
+        if (!ok) (void) hipGetLastError();
+        c->up_off = !ok;
     }
     {   // every kernel file's code object onto this device now, not in front of the first prompt (kernels.h: MI_TU_TOUCH)
         static const bool preload = !getenv("GGML_MI355X_PRELOAD") || atoi(getenv("GGML_MI355X_PRELOAD")) != 0;

@@ -111,9 +111,9 @@ struct options {
     bool fusion = true;        // node fusion (norm+mul, mul_mat+add, ...)
     bool prologue = true;      // fold RMS_NORM / activation quantisation into the mat-vec prologue
     bool qkv = true;           // fused Q/K/V + rope + cache store launch
-    int mmvq_max_cols = 2;     // widest batch that takes the mat-vec fusions (gate/up/SwiGLU, +bias +residual in one launch); from three columns on the
-                               // skinny matrix-core kernel + its separate SwiGLU launch is faster (-np 8 step 4.06 -> 3.45 ms, -np 3 3.77 -> 3.35)
-    int mmq_min_cols = 3;      // batches at least this wide run on the matrix cores (measured, ms/step matrix cores vs multi-column mat-vec: 3 columns 4.1 / 4.4, 4: 3.9 / 4.2, 8: 4.4 / 5.7; 2 columns: 3.6 / 3.1)
+    int mmvq_max_cols = 2;     // widest batch that takes the mat-vec fusions (gate/up/SwiGLU, +bias +residual in one launch).  2, the default: only matrices that the matrix-core kernels do not
+                               // serve at two columns (graph.cpp: mat_vec_fusions); other values are taken as they are
+    int mmq_min_cols = 3;      // batches at least this wide run on the matrix cores.  3, the default: two columns (graph.cpp: mmq_min_cols_for); other values are taken as they are
     bool mmq_i8 = true;        // Q4_K/Q5_K batches on the int8 matrix cores (mmq_i8.hip) instead of the f16 variant (mmq.hip)
     bool mm_merge = true;      // batches: sibling mat-muls over the same activations (wq/wk/wv, gate/up) as one launch
     bool ss_partials = true;    // residual-stream mat-vecs leave the sum of squares of their result for the next RMS_NORM prologue (GGML_MI355X_SS_PARTIALS=0: off)
@@ -249,6 +249,8 @@ struct backend_ctx {
     static constexpr int UP_SLOTS = 8;
     hipStream_t up_stream = nullptr;
     up_slot up_slots[UP_SLOTS];
+    char * up_block = nullptr;  // their first buffers, one allocation of UP_SLOTS x UP_FIRST bytes at the first use
+    static constexpr size_t UP_FIRST = (size_t) 4 << 20;
     hipEvent_t up_round = nullptr;
     int up_used = 0;       // slots whose contents may not have been taken yet: since the last synchronize, or the last wait of up_stream for the stream
     bool up_behind = false;  // a graph entered the stream since the last synchronize
