@@ -503,7 +503,7 @@ bool launch_attn_nf_list(hipStream_t s, const tdesc & q, const tdesc & k, const 
     static const int groups_on = !getenv("GGML_MI355X_NF_GROUPS") || atoi(getenv("GGML_MI355X_NF_GROUPS")) != 0;
     dim3 grid((unsigned) q.ne[1], (unsigned) k.ne[2], (unsigned) dq);
     // Few tokens: every slice of the head dimensions computes all the logits of its heads.  While the grid is no more than one workgroup a CU, eight waves share the fetches (3 tokens x 700 cells of
-    // Llama-3-8B, a launch: 26.5 us with four waves, 19.5 with eight; with the logits on the matrix cores, V^T requested ahead and a head's soft-max in one wave's registers 13.5: of these 6
+    // Llama-3-8B, a launch: 26.5 us with four waves, 19.5 with eight; with the logits on the matrix cores, V^T requested ahead and a head's soft-max in one wave's registers 14.2: of these 6
     // wait for the 200 KB a workgroup fetches, whatever its mapping to XCDs or the shape of its loads); more workgroups than that already have the company of another.
     const bool few = dq > 1 && q.ne[1] * k.ne[2] * dq <= 256;
 #define NF_GO(G_, W_)                                                                                                                                                              \
