@@ -512,7 +512,9 @@ __global__ void __launch_bounds__(WV * 64) k_fattn_dec128(const tdesc q, const t
 
     // a trip covers NG*16 consecutive positions: position of (u, wave, sub) = p0 + u*16 + wave*4 + sub
     uint4 kraw[NG], vraw[NG];
-    uint16_t mvl = 0;   // mask value / validity of THIS lane's pair (ul, sub): as loaded - converted here, it was waited for on the spot, and with it everything that the trip had requested
+    // mask value / validity of THIS lane's pair (ul, sub).  The mask as loaded: converted with the loads, it was waited for on the spot, and with it (loads come back in order) everything that the trip had
+    // requested - no reduction ran beside the next trip's rows.  Llama-3-8B, a launch: 32 sequences of 160 cells 11.5 -> 9.5 us, 9 drafts of 1500 Q8_0 cells 16.7 -> 15.9
+    uint16_t mvl = 0;
     bool okl = false;
     int p0 = LIST ? ti * TRIP : kv0;
 #define FA_LOAD_TRIP()                                                                  \
