@@ -958,6 +958,9 @@ static int api_graph_key_probe(const ggml_cgraph * a, const ggml_cgraph * b, int
     if (n_words) *n_words = (int64_t) key.size();
     return graph_key_equals(b, key) ? 1 : 0;
 }
+// ... and what decides whether K slices fit the scratch: the bytes set aside for a graph, the slices that a product of n_rows rows (of all matrices of its launch) and M columns takes
+static int64_t api_scratch_probe(const ggml_cgraph * g) { return partials_reserved(g); }
+static int api_k_slices(int type, int64_t K, int64_t n_rows, int64_t M) { return mmq_pick_ksplit(K, n_rows, M, options().mmq_skinny, type); }
 // tests: the decode copy of weight matrix t (repacking it first if need be) into `out`; returns its bytes, 0 when the tensor has / gets no copy, -1 on error
 static int64_t api_decode_copy_read(ggml_backend_t be, const ggml_tensor * t, void * out, size_t size) {
     if (!be_is_ours(be) || t == nullptr) return -1;
@@ -1107,6 +1110,8 @@ static void * reg_get_proc_address(ggml_backend_reg_t, const char * name) {
     if (n == "ggml_backend_split_buffer_type") return (void *) api_split_buffer_type;  // -sm row (split.cpp)
     if (n == "ggml_backend_mi355x_split_rows") return (void *) api_split_rows;
     if (n == "ggml_backend_mi355x_graph_key_probe") return (void *) api_graph_key_probe;
+    if (n == "ggml_backend_mi355x_scratch_probe") return (void *) api_scratch_probe;
+    if (n == "ggml_backend_mi355x_k_slices") return (void *) api_k_slices;
     return nullptr;
 }
 static const ggml_backend_reg_i k_reg_iface = {reg_get_name, reg_get_device_count, reg_get_device, reg_get_proc_address};

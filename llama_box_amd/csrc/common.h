@@ -355,6 +355,7 @@ bool supports_op(const ggml_tensor * op);
 enum ggml_status graph_compute(backend_ctx * ctx, ggml_cgraph * g);
 void free_graph_cache(backend_ctx * ctx);
 bool graph_key_equals(const ggml_cgraph * g, const std::vector<uint64_t> & key);  // the graph-key words (graph.cpp: walk_key), compared in place ...
+int64_t partials_reserved(const ggml_cgraph * g);  // bytes of scratch behind the activations that a backend with the default options sets aside for the graph
 void graph_key_build(const ggml_cgraph * g, std::vector<uint64_t> & key);         // ... or materialised
 
 // ---- in-process tensor parallel over the devices of a row-split model, -sm row (tp_inproc.cpp) ----

@@ -333,6 +333,28 @@ struct ws_plan {
 static bool mm_tile_form(const ggml_tensor * n);
 static bool mm_id_tile_applies(const ggml_tensor * n);
 static size_t fa_image_offset(const tdesc & q, const tdesc & k, const tdesc & v) { return (fattn_workspace_bytes(q, k, v, 64, GGML_TYPE_F16) + 255) & ~(size_t) 255; }
+// Bytes of partial products where the K-quant product of node i is the first of a launch of several (try_merge_mm_batch): any of the siblings may be in it, a larger launch need not have fewer K slices
+// than each of its matrices (mmq_q6_tile), and siblings of another format may run while its partial products wait for the rotation, behind these.
+static size_t merged_partials(const backend_ctx * c, const ggml_cgraph * g, int i, int64_t M) {
+    const ggml_tensor * n0 = g->nodes[i];
+    const int type = n0->src[0]->type;
+    const int64_t K = n0->src[0]->ne[0];
+    auto need = [&](int t, int64_t rows) { return mmq_workspace_bytes(t, K, rows, M, c->opt.mmq_skinny); };
+    size_t most = 0, behind = 0;
+    std::vector<int64_t> same;  // rows of the siblings that may share the launch
+    for (int k = i + 1; k < std::min(g->n_nodes, i + 24); ++k) {
+        const ggml_tensor * t = g->nodes[k];
+        if (t->op != GGML_OP_MUL_MAT || t->src[1] != n0->src[1] || t->src[0]->ne[0] != K || !mmq_i8_supported(t->src[0]->type, K, t->src[0]->ne[1], M)) continue;
+        const int64_t rows = t->src[0]->ne[1];
+        if (t->src[0]->type != type) behind = std::max(behind, need(t->src[0]->type, rows));
+        if (t->src[0]->type == type || M <= 32) same.push_back(rows);  // (up to 32 columns two formats share a launch)
+    }
+    for (size_t a = 0; a < same.size(); ++a) {
+        most = std::max(most, need(type, n0->src[0]->ne[1] + same[a]));
+        for (size_t b = a + 1; b < same.size(); ++b) most = std::max(most, need(type, n0->src[0]->ne[1] + same[a] + same[b]));
+    }
+    return most ? ((most + 255) & ~(size_t) 255) + behind : 0;
+}
 static ws_plan plan_ws(backend_ctx * c, const ggml_cgraph * g) {
     ws_plan p;
     for (int i = 0; i < g->n_nodes; ++i) {
@@ -345,7 +367,10 @@ static ws_plan plan_ws(backend_ctx * c, const ggml_cgraph * g) {
             // (2..32 columns: the skinny matrix-core kernel fetches 32 columns' worth of activation bytes whatever M is)
             // (and the wide form of the same unit fetches whole groups of 128 columns of a prompt batch)
             p.act_bytes = std::max(p.act_bytes, quantized_act_bytes(act_kind(n->src[0]->type), b->ne[0], (Mc >= 2 && Mc < 32) ? 32 : (Mc >= 33 ? (Mc + 127) / 128 * 128 : Mc)));
-            if (Mc >= mmq_min_cols_for(c) && (n->ne[0] % 4) == 0) p.aux_bytes = std::max(p.aux_bytes, 3 * mmq_workspace_bytes(n->src[0]->type, b->ne[0], n->src[0]->ne[1], Mc, c->opt.mmq_skinny));  // (x3: up to three sibling matrices share a launch)
+            if (Mc >= mmq_min_cols_for(c) && (n->ne[0] % 4) == 0) {
+                p.aux_bytes = std::max(p.aux_bytes, 3 * mmq_workspace_bytes(n->src[0]->type, b->ne[0], n->src[0]->ne[1], Mc, c->opt.mmq_skinny));  // (x3: up to three sibling matrices share a launch)
+                if (c->opt.mm_merge && c->opt.mmq_i8 && mmq_i8_supported(n->src[0]->type, b->ne[0], n->src[0]->ne[1], Mc)) p.aux_bytes = std::max(p.aux_bytes, merged_partials(c, g, i, Mc));
+            }
         } else if (n->op == GGML_OP_MUL_MAT && mm_cache_image_ok(n) && !buffer_is_split(n->src[0]->buffer)) {
             const tdesc a16 = kv_image_desc(TD(n->src[0]), nullptr);
             p.aux_bytes = std::max(p.aux_bytes, ((mul_mat_f_workspace_bytes(a16, TD(n->src[1])) + 255) & ~(size_t) 255) + kv_image_bytes(a16));
@@ -379,6 +404,11 @@ static ws_plan plan_ws(backend_ctx * c, const ggml_cgraph * g) {
     p.act_bytes = (p.act_bytes + 255) & ~(size_t) 255;
     p.act16_bytes = (p.act16_bytes + 255) & ~(size_t) 255;
     return p;
+}
+
+int64_t partials_reserved(const ggml_cgraph * g) {
+    backend_ctx c;  // (its options only)
+    return (int64_t) plan_ws(&c, g).aux_bytes;
 }
 
 // ------------------------------------------------------------------------------------------------ attention-mask content hints
@@ -716,7 +746,8 @@ static bool run_mul_mat_q(exec_state & st, const ggml_tensor * w, const ggml_ten
     const uint8_t * const panels = i8 && !w2 && !add2 && st.epi_dst != dst ? k_panels(c, w, N, M) : nullptr;
     if (M >= mmq_min_cols_for(c) && !w2 && !add2 && (!add || i8) && (i8 || mmq_supported(w->type, K, N, M))) {
         timed_scope ts(c, (std::string("mmq_") + type_tag(w->type) + "_n" + std::to_string(N) + "_k" + std::to_string(K)).c_str(), wbytes, i8);
-        const int ks = panels || st.epi_dst == dst ? 1 : ((N % 4) == 0 && (dst->nb[1] % 16) == 0 ? mmq_pick_ksplit(K, N, M, c->opt.mmq_skinny, w->type) : 1);
+        int ks = panels || st.epi_dst == dst ? 1 : ((N % 4) == 0 && (dst->nb[1] % 16) == 0 ? mmq_pick_ksplit(K, N, M, c->opt.mmq_skinny, w->type) : 1);
+        if ((size_t) ks * (size_t) M * (size_t) N * sizeof(float) > c->ws_size - st.aux_off) ks = 1;  // (no room behind partial products that wait for their reader)
         float * part = (float *) ((char *) c->ws + st.aux_off);
         if (i8) {
             const int64_t arows = add ? add->ne[1] * add->ne[2] * add->ne[3] : 0;

@@ -463,3 +463,52 @@ def test_graph_key_decides_what_a_captured_graph_stands_for():
     assert probe(g0, build(swap=True), None) == 0                                     # another source tensor in one slot
     for ctx in keep:
         H.ggml_free(ctx)
+
+
+def test_scratch_holds_the_slices_of_merged_launches():
+    """graph.cpp: plan_ws sets aside what the products of a layer write as partial products: those of up to three sibling matrices of one format in one launch (whose K slices need
+    not be fewer than a single matrix's), and behind them, where they wait for the rotation, those of a sibling in another format."""
+    import ctypes as C
+    import itertools
+
+    import llama_box_amd as L
+
+    H = L.host()
+    lib = C.CDLL(L.BACKEND_SO)
+    lib.ggml_backend_mi355x_reg.restype = C.c_void_p
+    reg = lib.ggml_backend_mi355x_reg()
+
+    def proc(name, res, *args):
+        return C.CFUNCTYPE(res, *args)(H.ggml_backend_reg_get_proc_address(reg, name))
+
+    reserved = proc(b"ggml_backend_mi355x_scratch_probe", C.c_int64, C.POINTER(L.CGraph))
+    slices = proc(b"ggml_backend_mi355x_k_slices", C.c_int, C.c_int, C.c_int64, C.c_int64, C.c_int64)
+
+    def part(t, K, n, M):
+        ks = slices(t, K, n, M)
+        return ks * M * n * 4 if ks > 1 else 0
+
+    short = []
+    for (K, nq, nkv, ff), M in itertools.product([(4096, 4096, 1024, 14336), (3584, 3584, 512, 18944), (5120, 5120, 1024, 13824), (6144, 6144, 1024, 16384), (2048, 2048, 256, 5632)],
+                                                 [2, 9, 31, 33, 48, 64, 65, 100, 128, 129, 200, 257, 290, 322, 400, 512]):
+        for types in itertools.product([L.Q4_K, L.Q5_K, L.Q6_K], repeat=3):
+            ctx = H.ggml_init(L.InitParams(0, None, True))
+            gf = H.ggml_new_graph_custom(ctx, 32, False)
+            x = H.ggml_new_tensor_4d(ctx, L.F32, K, M, 1, 1)
+            for t, n in zip(types, (nq, nkv, nkv)):
+                H.ggml_build_forward_expand(gf, H.ggml_mul_mat(ctx, H.ggml_new_tensor_4d(ctx, t, K, n, 1, 1), x))
+            got = reserved(gf)
+            qkv = list(zip(types, (nq, nkv, nkv)))
+            need = max(part(t, K, n, M) for t, n in qkv)
+            for first in range(2):  # a launch of several matrices starts at any of them; the others behind its partial products
+                later = range(first + 1, 3)
+                rest = max((part(types[q], K, qkv[q][1], M) for q in later if types[q] != types[first]), default=0)
+                for g in itertools.chain(itertools.combinations(later, 1), itertools.combinations(later, 2)):
+                    if all(types[q] == types[first] for q in g):
+                        need = max(need, part(types[first], K, qkv[first][1] + sum(qkv[q][1] for q in g), M) + rest)
+            if M <= 32 and len(set(types)) == 2:  # two formats in one launch
+                need = max(need, part(types[0], K, nq + 2 * nkv, M))
+            if need > got:
+                short.append((K, nq, nkv, M, types, need, got))
+            H.ggml_free(ctx)
+    assert not short, (len(short), short[:5])
