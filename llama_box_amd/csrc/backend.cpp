@@ -368,7 +368,7 @@ void note_mask_upload(const ggml_tensor * t, const void * host, size_t offset, s
     // (16 MiB: a 160-token draft batch — 192 rows with padding — over a 40 k-cell cache; the 2 MiB of round 4's first cut lost the 10 k-cell cache of the
     // bench's own `--np 32 --draft 4` line: 10.3 -> 12.1 ms per step on the dense kernel.  A sparse mask is read in full, ~0.1 ms per MiB on one host
     // core; a dense one is given up as soon as a quarter of its cells have been seen visible)
-    if (!named || !whole || t->ne[1] < 2 || t->ne[1] > 256 || size > ((size_t) 16 << 20)) { forget(); return; }
+    if (!named || !whole || host == nullptr || t->ne[1] < 2 || t->ne[1] > 256 || size > ((size_t) 16 << 20)) { forget(); return; }
     const int64_t n = t->ne[0], rows = (int64_t) (size / (size_t) t->nb[1]);
     if (rows < 2) { forget(); return; }
     mask_stats st;
@@ -551,6 +551,35 @@ static const ggml_backend_buffer_type_i k_buft_iface = {buft_get_name, buft_allo
 // it — get_tensor_async uses that for the logits rows of a decode step (be_get_tensor_async).
 static std::mutex g_pinned_mtx;
 static std::vector<std::pair<const char *, size_t>> g_pinned;
+// host memory that a download (get_tensor_async) of a backend may still be about to write: an upload from it has to take its turn in the stream
+struct open_download { const char * p; size_t n; const backend_ctx * c; };
+static std::vector<open_download> g_downloads;  // under g_pinned_mtx; a backend's entries go with its next synchronize
+static void note_download(backend_ctx * c, const void * p, size_t n) {
+    std::lock_guard<std::mutex> lock(g_pinned_mtx);
+    open_download * last = nullptr;
+    int own = 0;
+    for (auto & d : g_downloads)
+        if (d.c == c) { last = &d; own++; }
+    if (own >= 32) {  // (a host that never synchronises: one range around the rest)
+        const char * lo = std::min(last->p, (const char *) p), * hi = std::max(last->p + last->n, (const char *) p + n);
+        last->p = lo;
+        last->n = (size_t) (hi - lo);
+    } else
+        g_downloads.push_back({(const char *) p, n, c});
+    c->downloads_open = true;
+}
+static bool download_open(const void * p, size_t n) {
+    std::lock_guard<std::mutex> lock(g_pinned_mtx);
+    for (const auto & d : g_downloads)
+        if ((const char *) p < d.p + d.n && d.p < (const char *) p + n) return true;
+    return false;
+}
+static void downloads_done(backend_ctx * c) {  // its stream has been waited for
+    if (!c->downloads_open) return;
+    std::lock_guard<std::mutex> lock(g_pinned_mtx);
+    g_downloads.erase(std::remove_if(g_downloads.begin(), g_downloads.end(), [&](const open_download & d) { return d.c == c; }), g_downloads.end());
+    c->downloads_open = false;
+}
 static bool is_pinned_range(const void * p, size_t n) {
     std::lock_guard<std::mutex> lock(g_pinned_mtx);
     for (const auto & r : g_pinned)
@@ -594,6 +623,7 @@ static void be_free(ggml_backend_t be) {
     backend_ctx * c = (backend_ctx *) be->context;
     HIP_SOFT(hipSetDevice(c->device));
     HIP_SOFT(hipStreamSynchronize(c->stream));
+    downloads_done(c);
     free_graph_cache(c);
     ip_free(c);
     tp_free(c);
@@ -629,7 +659,8 @@ void flush_uploads(backend_ctx * c) {
 // own, into a device buffer that the backend keeps, and reaches the tensor by a copy on the device in the stream's order.  Waiting for the stream first left the GPU idle
 // for the link's 40 .. 80 us in front of every micro-batch.  A 4-layer model's prompt of 2000 tokens with two masks, us: 2815 / 2690; below 1 MB the streams' waits for each other cost more than
 // the link (the same model's 700 tokens 1262 / 1280).  Sources are pinned memory of our host buffer type only (a copy from other memory is not asynchronous), and as with a plain asynchronous
-// copy they are the caller's again after a synchronize: the stream waits for the copy, so a wait for the stream covers both.
+// copy they are the caller's again after a synchronize: the stream waits for the copy, so a wait for the stream covers both.  What they hold has to be there when the call is made: memory that a
+// download still has to fill (of this backend, or of one that its stream has been told to wait for) goes the plain way (be_set_tensor_async).
 static bool stage_upload(backend_ctx * c, char * dst, const void * data, size_t size) {
     constexpr size_t LEAST = (size_t) 1 << 20, MOST = (size_t) 16 << 20;
     if (!c->up_behind || c->up_off || size < LEAST || size > MOST || ip_any() || !is_pinned_range(data, size)) return false;
@@ -682,13 +713,14 @@ static void be_set_tensor_async(ggml_backend_t be, ggml_tensor * t, const void *
     backend_ctx * c = (backend_ctx *) be->context;
     if (ip_any()) ip_host_access(t->view_src ? t->view_src->buffer : t->buffer, true);
     HIP_SOFT(hipSetDevice(c->device));
-    note_mask_upload(t, data, offset, size);
+    const bool at_once = !download_open(data, size);  // may the source be read now, before the stream gets here?
+    note_mask_upload(t, at_once ? data : nullptr, offset, size);
     {
         ggml_backend_buffer_t tb = t->view_src ? t->view_src->buffer : t->buffer;
         if (tb && buffer_is_ours(tb) && ((buffer_ctx *) tb->context)->has_copies) decode_copy_drop(tb, t, offset, size);
     }
     constexpr size_t SMALL = 64 * 1024, RING = 4u << 20;
-    if (size > 0 && size <= SMALL && c->opt.small_uploads) {
+    if (size > 0 && size <= SMALL && c->opt.small_uploads && at_once) {
         if (!c->up_ring) {
             if (hipHostMalloc((void **) &c->up_ring, RING, hipHostMallocDefault) == hipSuccess) c->up_cap = RING;
             else { (void) hipGetLastError(); c->up_ring = nullptr; c->opt.small_uploads = false; }
@@ -709,7 +741,7 @@ static void be_set_tensor_async(ggml_backend_t be, ggml_tensor * t, const void *
     }
     flush_uploads(c);
     uploader_join(c->device, c->stream);
-    if (stage_upload(c, (char *) t->data + offset, data, size)) return;
+    if (at_once && stage_upload(c, (char *) t->data + offset, data, size)) return;
     HIP_SOFT(hipMemcpyAsync((char *) t->data + offset, data, size, hipMemcpyHostToDevice, c->stream));
 }
 static void be_get_tensor_async(ggml_backend_t be, const ggml_tensor * t, void * data, size_t offset, size_t size) {
@@ -718,6 +750,7 @@ static void be_get_tensor_async(ggml_backend_t be, const ggml_tensor * t, void *
     HIP_SOFT(hipSetDevice(c->device));
     flush_uploads(c);
     uploader_join(c->device, c->stream);
+    note_download(c, data, size);
     // The logits of a decode step (513 KB per sequence, llama.cpp's pinned output buffer): a blit through hipMemcpyAsync starts ~20 us after
     // the graph's last kernel and takes 10 us (profiles/r05_decode_gaps_*.txt); a copy kernel writing the mapped pinned memory is an ordinary
     // launch behind that kernel.  Only into memory of OUR host buffer type (known to be device-mapped), up to 8 MiB.
@@ -767,6 +800,7 @@ static void be_synchronize(ggml_backend_t be) {
     flush_uploads(c);
     uploader_drain(c->device);
     HIP_SOFT(hipStreamSynchronize(c->stream));
+    downloads_done(c);
     c->up_used = 0;
     c->up_behind = false;
 }

@@ -255,6 +255,7 @@ struct backend_ctx {
     int up_used = 0;       // slots whose contents may not have been taken yet: since the last synchronize, or the last wait of up_stream for the stream
     bool up_behind = false;  // a graph entered the stream since the last synchronize
     bool up_off = false;     // (could not be set up)
+    bool downloads_open = false;  // get_tensor_async calls since the last synchronize (backend.cpp: note_download)
     upload_batch up_pending{};  // staged in the ring, not yet launched: flushed as ONE kernel before anything else enters the stream
     // attention over a unified cache with a few query tokens: per-token lists of visible tiles (fattn.hip, k_fattn_tile_scan),
     // built once per graph execution and shared by the attention nodes of all layers

@@ -963,3 +963,62 @@ def test_micro_batches_back_to_back(backend, H, fa, n):
         c1.free()
         c2.free()
         m.free()
+
+
+@pytest.mark.parametrize("two", [False, True])
+@pytest.mark.parametrize("nbytes", [4096, 2 << 20, 20 << 20])
+def test_uploads_wait_for_the_download_that_fills_their_source(backend, H, nbytes, two):
+    """set_tensor_async from pinned memory that a get_tensor_async before it still has to fill behind a running graph: of the same backend, or of another one that it waits for by an event."""
+    P, SZ = C.c_void_p, C.c_size_t
+    H.ggml_backend_tensor_set_async.argtypes = [P, L.TP, P, SZ, SZ]
+    H.ggml_backend_tensor_get_async.argtypes = [P, L.TP, P, SZ, SZ]
+    H.ggml_backend_graph_compute_async.argtypes = [P, C.POINTER(L.CGraph)]
+    H.ggml_backend_event_new.argtypes, H.ggml_backend_event_new.restype = [P], P
+    for f, a in (("record", [P, P]), ("wait", [P, P]), ("free", [P])):
+        getattr(H, "ggml_backend_event_" + f).argtypes = a
+    rng = np.random.default_rng(nbytes)
+    a_data = rng.integers(0, 256, nbytes, dtype=np.uint8)
+    other = L.Backend(0) if two else backend
+    K, M, n = 8192, 512, 40
+    gs = []
+    pin = None
+    ev = None
+    try:
+        for be in {id(b): b for b in (other, backend)}.values():  # each with some milliseconds of products, and a tensor
+            g = T.G(be)
+            gs.append((be, g))
+            w = g.new(L.Q8_0, [K, K], T.rand_weight(L.Q8_0, K, K, rng))
+            cur = g.new(L.F32, [K, M], rng.standard_normal((M, K)).astype(np.float32))
+            for _ in range(n):
+                cur = H.ggml_mul_mat(g.ctx, w, cur)
+            g.t = g.new(L.F32, [nbytes // 4], a_data if be is other else np.zeros(nbytes, np.uint8))
+            if not two:
+                g.u = g.new(L.F32, [nbytes // 4], np.zeros(nbytes, np.uint8))
+            g.compute([cur])
+        (src_be, src), (dst_be, dst) = gs[0], gs[-1]
+        b = dst.t if two else dst.u
+        pin = H.ggml_backend_buft_alloc_buffer(H.ggml_backend_dev_host_buffer_type(backend.dev), nbytes)
+        base = H.ggml_backend_buffer_get_base(pin)
+        for _ in range(2):
+            C.memset(base, 0x55, nbytes)
+            H.ggml_backend_tensor_set(b, np.zeros(nbytes, np.uint8).ctypes.data_as(P), 0, nbytes)
+            for be, g in gs:
+                assert H.ggml_backend_graph_compute_async(be.backend, g.gf) == 0
+            H.ggml_backend_tensor_get_async(src_be.backend, src.t, base, 0, nbytes)
+            if two:
+                ev = ev or H.ggml_backend_event_new(backend.dev)
+                H.ggml_backend_event_record(ev, src_be.backend)
+                H.ggml_backend_event_wait(dst_be.backend, ev)
+            H.ggml_backend_tensor_set_async(dst_be.backend, b, base, 0, nbytes)
+            H.ggml_backend_synchronize(dst_be.backend)
+            H.ggml_backend_synchronize(src_be.backend)
+            assert np.array_equal(dst.read(b).view(np.uint8).ravel(), a_data)
+    finally:
+        if ev:
+            H.ggml_backend_event_free(ev)
+        if pin:
+            H.ggml_backend_buffer_free(pin)
+        for _, g in gs:
+            g.free()
+        if two:
+            other.close()
