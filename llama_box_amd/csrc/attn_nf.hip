@@ -101,7 +101,6 @@ __global__ void __launch_bounds__(NW * 64) k_attn_nf_list(const tdesc q, const t
                 return;
             }
             const char * kbase = k.data + (int64_t) kvh * k.nb[2];
-            const uint32_t knb = (uint32_t) k.nb[1];  // (the launch checks that offsets fit 32 bits: half the registers for addresses)
 #pragma unroll 1
             for (int t0 = wave; 16 * t0 < cnt; t0 += NW * U) {
                 half8 kf[U][4];
@@ -111,8 +110,9 @@ __global__ void __launch_bounds__(NW * 64) k_attn_nf_list(const tdesc q, const t
                     const int c = 16 * (t0 + u * NW) + col;
                     if (16 * (t0 + u * NW) < cnt) {
                         const uint32_t pc = c >= cnt ? 0 : (t0 == wave ? pk[u] : pos[c]);  // (beyond the list: cell 0, whose logit is not stored)
+                        const char * const kr = kbase + ((int64_t) pc * k.nb[1] + 16 * quad);
 #pragma unroll
-                        for (int s = 0; s < 4; ++s) kf[u][s] = *(const half8 *) (kbase + (pc * knb + 64u * s + 16u * quad));
+                        for (int s = 0; s < 4; ++s) kf[u][s] = *(const half8 *) (kr + 64 * s);
                         mv[u] = m16 ? h2f(((const uint16_t *) mrow)[pc]) : ((const float *) mrow)[pc];
                     }
                 }
@@ -497,7 +497,6 @@ bool launch_attn_nf_list(hipStream_t s, const tdesc & q, const tdesc & k, const 
     if (v.ne[0] != k.ne[1] || v.ne[1] != 128 || v.ne[2] != k.ne[2] || v.ne[3] != 1) return false;
     if ((k.nb[1] % 16) || (k.nb[2] % 16) || (((uintptr_t) k.data) & 15) || (q.nb[1] % 16) || (q.nb[2] % 16) || (((uintptr_t) q.data) & 15)) return false;
     if ((mask.type != GGML_TYPE_F16 && mask.type != GGML_TYPE_F32) || mask.ne[0] < k.ne[1] || mask.ne[1] < q.ne[1] || mask.ne[2] != 1 || mask.ne[3] != 1) return false;
-    if (k.ne[1] * k.nb[1] > INT32_MAX) return false;  // (32-bit offsets)
     const int G = (int) (q.ne[2] / k.ne[2]);
     if (q8_out && (dq != 1 || (G & 1))) return false;  // Q8_K blocks are head pairs of whole rows
     static const int groups_on = !getenv("GGML_MI355X_NF_GROUPS") || atoi(getenv("GGML_MI355X_NF_GROUPS")) != 0;

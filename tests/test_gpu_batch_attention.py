@@ -361,3 +361,44 @@ def test_few_tokens_on_matrix_cores(backend, H, T_, NKV, G, per):
             ref = vt[h // G] @ p
             # f32 sums; a probability next to a rounding boundary may round the other way: 2^-11 of it
             assert np.abs(got[h, t] - ref).max() <= 2e-3 * np.abs(ref).max() + 1e-5, (t, h)
+
+
+def test_few_tokens_over_a_cache_beyond_32_bit_offsets(backend, H):
+    """attn_nf.hip: cells 4 MiB apart, the last ones more than 2 GiB behind the first: one list and one launch, as of a dense cache."""
+    rng = np.random.default_rng(5)
+    HD, NKV, G, T_, n_kv, far = 128, 2, 4, 2, 768, 4 << 20
+    NH = NKV * G
+    k = rng.standard_normal((n_kv, NKV, HD)).astype(np.float16)
+    v = rng.standard_normal((NKV, HD, n_kv)).astype(np.float16)
+    q = (3 * rng.standard_normal((T_, NH, HD))).astype(np.float32)
+    mask = np.full((T_, n_kv), -np.inf, np.float32)
+    mask[0, ::2] = mask[1, 1::2] = 0
+    g = T.G(backend)
+    try:
+        base = g.new(L.F16, [far // 2, n_kv])
+        vc = g.new(L.F16, [n_kv, NKV * HD], v.reshape(-1, n_kv))
+        qp = H.ggml_permute(g.ctx, g.new(L.F32, [HD, NH, T_], q), 0, 2, 1, 3)
+        kv = H.ggml_view_3d(g.ctx, base, HD, n_kv, NKV, far, HD * 2, 0)
+        vv = H.ggml_view_3d(g.ctx, vc, n_kv, HD, NKV, n_kv * 2, n_kv * 2 * HD, 0)
+        p = H.ggml_soft_max_ext(g.ctx, H.ggml_mul_mat(g.ctx, kv, qp), g.new(L.F32, [n_kv, T_], mask), HD ** -0.5, 0.0)
+        out = H.ggml_mul_mat(g.ctx, vv, p)
+        g.compute([out])
+        for i in range(n_kv):
+            row = np.ascontiguousarray(k[i])
+            H.ggml_backend_tensor_set(base, row.ctypes.data, i * far, row.nbytes)
+        s0 = backend.stat("kernel_launches")
+        assert H.ggml_backend_graph_compute(backend.backend, g.gf) == 0
+        assert backend.stat("kernel_launches") - s0 <= 2
+        got = g.read(out).reshape(NH, T_, HD)
+    finally:
+        g.free()
+    qh = q.astype(np.float16).astype(np.float64)
+    for t in range(T_):
+        see = np.flatnonzero(mask[t] == 0)
+        for h in range(NH):
+            s = k[see, h // G].astype(np.float64) @ qh[t, h] * HD ** -0.5
+            p = np.exp(s - s.max())
+            p = (p / p.sum()).astype(np.float16).astype(np.float64)
+            ref = v[h // G][:, see].astype(np.float64) @ p
+            # (as test_few_tokens_on_matrix_cores)
+            assert np.abs(got[h, t] - ref).max() <= 2e-3 * np.abs(ref).max() + 1e-5, (t, h)
