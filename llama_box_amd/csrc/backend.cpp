@@ -85,7 +85,7 @@ static void decode_copy_drop(ggml_backend_buffer_t b, const ggml_tensor * t, siz
 }
 // (q80_panels: the OTHER second copy — Q8_0 matrices regrouped into the 32-row x 4-block tiles the matrix-core kernels load with whole-line
 // wave-instructions, repack.hip: k_repack_q80_panels.  A tensor has one kind of copy in the shadow: the K-quants planes, Q8_0 panels; same invalidation)
-static buffer_ctx * copyable(backend_ctx * c, const ggml_tensor * w) {  // the buffer of a weight matrix that may have a second copy
+static buffer_ctx * copyable(const backend_ctx * c, const ggml_tensor * w) {  // the buffer of a weight matrix that may have a second copy
     if (!c->opt.decode_copy || w == nullptr || w->view_src != nullptr || w->data == nullptr || w->ne[2] != 1 || w->ne[3] != 1) return nullptr;
     ggml_backend_buffer_t b = w->buffer;
     if (b == nullptr || !buffer_is_ours(b) || b->usage != GGML_BACKEND_BUFFER_USAGE_WEIGHTS || buffer_is_split(b) || buffer_is_rowpar(b)) return nullptr;
@@ -130,6 +130,10 @@ static const uint8_t * second_copy(backend_ctx * c, const ggml_tensor * w, const
 }
 const uint8_t * decode_copy(backend_ctx * c, const ggml_tensor * w) { return second_copy(c, w, false); }
 const uint8_t * q80_panel_copy(backend_ctx * c, const ggml_tensor * w) { return second_copy(c, w, true); }
+bool k_panel_possible(const backend_ctx * c, const ggml_tensor * w) {
+    const buffer_ctx * const bc = copyable(c, w);
+    return bc != nullptr && !bc->panels_failed && repack_supported(w->type, w->ne[0], (int64_t) w->nb[1]) && (w->ne[1] % 16) == 0;
+}
 const uint8_t * k_panel_copy(backend_ctx * c, const ggml_tensor * w) {
     buffer_ctx * const bc = copyable(c, w);
     if (bc == nullptr || !repack_supported(w->type, w->ne[0], (int64_t) w->nb[1]) || (w->ne[1] % 16) != 0) return nullptr;

@@ -111,9 +111,9 @@ struct options {
     bool fusion = true;        // node fusion (norm+mul, mul_mat+add, ...)
     bool prologue = true;      // fold RMS_NORM / activation quantisation into the mat-vec prologue
     bool qkv = true;           // fused Q/K/V + rope + cache store launch
-    int mmvq_max_cols = 2;     // widest batch that takes the mat-vec fusions (gate/up/SwiGLU, +bias +residual in one launch).  2, the default: only matrices that the matrix-core kernels do not
-                               // serve at two columns (graph.cpp: mat_vec_fusions); other values are taken as they are
-    int mmq_min_cols = 3;      // batches at least this wide run on the matrix cores.  3, the default: two columns (graph.cpp: mmq_min_cols_for); other values are taken as they are
+    int mmvq_max_cols = 2;     // widest batch that takes the mat-vec fusions (gate/up/SwiGLU, +bias +residual in one launch).  2, the default: two columns only of matrices without a second copy
+                               // for the matrix-core kernels (graph.cpp: mat_vec_fusions); other values are taken as they are
+    int mmq_min_cols = 3;      // batches at least this wide run on the matrix cores.  3, the default: by matrix, two or three columns (graph.cpp: mmq_min_cols_for); other values are taken as they are
     bool mmq_i8 = true;        // Q4_K/Q5_K batches on the int8 matrix cores (mmq_i8.hip) instead of the f16 variant (mmq.hip)
     bool mm_merge = true;      // batches: sibling mat-muls over the same activations (wq/wk/wv, gate/up) as one launch
     bool ss_partials = true;    // residual-stream mat-vecs leave the sum of squares of their result for the next RMS_NORM prologue (GGML_MI355X_SS_PARTIALS=0: off)
@@ -234,6 +234,7 @@ struct backend_ctx {
     uint64_t tick = 0;
     uint64_t decode_epoch = 0;  // decode_copy_epoch() the cached graphs were captured under
     bool capturing = false;
+    bool mm_q5_major = false;  // the graph being planned / run holds more Q5_K than Q4_K weight bytes (graph.cpp: mmq_min_cols_for)
     // tensor parallel
     tp_state * tp = nullptr;
     ip_engine * ip = nullptr;  // -sm row served as in-process tensor parallelism (tp_inproc.cpp); owned by the main device's backend
@@ -309,12 +310,13 @@ struct buffer_ctx {
     struct panel_chunk { void * mem; size_t size, used; };
     std::unordered_map<size_t, panel_mem> panels;  // offset of the tensor -> its panel copy
     std::vector<panel_chunk> panel_chunks;
-    bool panels_failed = false;
+    std::atomic<bool> panels_failed{false};
     std::atomic<bool> has_copies{false};           // any copy was ever made
 };
 // the plane-layout copy of weight matrix w for the batch-1 mat-vec kernels, or nullptr (no copy: views, split / row-parallel buffers, option off,
 // allocation failed, or asked during a capture for a tensor not yet repacked)
 const uint8_t * decode_copy(backend_ctx * c, const ggml_tensor * w);
+bool k_panel_possible(const backend_ctx * c, const ggml_tensor * w);    // does it have a panel copy, or may it get one?
 const uint8_t * k_panel_copy(backend_ctx * c, const ggml_tensor * w);    // a K-quant matrix's panel copy (mmq_panel.hip), or nullptr
 const uint8_t * q80_panel_copy(backend_ctx * c, const ggml_tensor * w);  // a Q8_0 matrix's panel copy (mmq_q80.hip), or nullptr
 uint64_t decode_copy_epoch();  // bumped whenever a copy was dropped: graphs captured before hold pointers to it

@@ -17,18 +17,28 @@
 namespace mi355x {
 
 static bool is_quant(int t) { return t == GGML_TYPE_Q4_K || t == GGML_TYPE_Q5_K || t == GGML_TYPE_Q6_K || t == GGML_TYPE_Q8_0; }
-// batches at least this wide run on the matrix cores; the option's default (3) means two columns.  (The multi-column mat-vec has none of the batch path's fusions.  Two sequences of 200 tokens, us a
-// step, from three columns on / from two: Llama-3-8B Q4_K_M 2586 / 2458, Qwen2-7B Q5_K_M 3134 / 2767 with its gate/up pair over panels.)
-static inline int mmq_min_cols_for(const backend_ctx * c) { return c->opt.mmq_min_cols != 3 ? c->opt.mmq_min_cols : 2; }
+// Batches at least this wide run on the matrix cores.  The option's default (3) means two columns where a panel copy may exist (backend.cpp), which gate / up of most models then take; where none
+// may (no room, GGML_MI355X_DECODE_COPY=0, matrices spread over devices) two columns of Q5_K, and of Q6_K in a model that is mostly Q5_K, stay with the multi-column mat-vec.  Steps of two sequences of
+// 200 tokens, eight layers, mat-vec / matrix cores, us: widths 2048, 3584, 4096, 8192 of Q5_K_M models with the copies 568 / 457, 922 / 807, 819 / 749, 1984 / 1546; without 562 / 487, 920 / 1035,
+// 815 / 835, 1984 / 2047.
+static bool panels_possible(const backend_ctx * c, const ggml_tensor * w) { return c->opt.mmq_i8 && c->opt.mmq_skinny && k_panel_possible(c, w); }
+static int mmq_min_cols_for(const backend_ctx * c, const ggml_tensor * w) {
+    if (c->opt.mmq_min_cols != 3) return c->opt.mmq_min_cols;
+    return panels_possible(c, w) || w->type == GGML_TYPE_Q4_K || (w->type == GGML_TYPE_Q6_K && !c->mm_q5_major) ? 2 : 3;
+}
+// Does a batch of M columns multiply a Q8_0 matrix on the matrix cores (mmq_q80.hip)?
+static bool q80_mm_ok(backend_ctx *, const ggml_tensor * w, int64_t M) { return mmq_q80_batch_supported(w->type, w->ne[0], w->ne[1], M); }
 // the panel copy of a K-quant matrix where M columns are multiplied over it (mmq_panel.hip) in a launch of n_total rows, else nullptr
 static const uint8_t * k_panels(backend_ctx * c, const ggml_tensor * w, int64_t n_total, int64_t M) {
-    return c->opt.mmq_i8 && c->opt.mmq_skinny && M >= mmq_min_cols_for(c) && mmq_panel_applies(w->type, w->ne[0], n_total, M) ? k_panel_copy(c, w) : nullptr;
+    return c->opt.mmq_i8 && c->opt.mmq_skinny && M >= mmq_min_cols_for(c, w) && mmq_panel_applies(w->type, w->ne[0], n_total, M) ? k_panel_copy(c, w) : nullptr;
 }
-// Does a batch of M columns take the mat-vec fusions (gate/up/SwiGLU, bias and residual in one launch)?  Left at its default, the option leaves batches to the matrix-core kernels that serve 2 columns.
-static bool mat_vec_fusions(const backend_ctx * c, const ggml_tensor * w, int64_t M) {
+// Does a batch of M columns take the mat-vec fusions (gate/up/SwiGLU, bias and residual in one launch)?  Left at its default, the option leaves two columns to the matrix cores where copies serve them.
+// Without copies, steps as above, fusions / none: Q4_K_M at width 8192 1429 / 1500, 3584 747 / 757, 4096 684 / 653.
+static bool mat_vec_fusions(backend_ctx * c, const ggml_tensor * w, int64_t M) {
     if (M > c->opt.mmvq_max_cols) return false;
-    return M < 2 || c->opt.mmvq_max_cols != 2 ||
-           !(mmq_q80_batch_supported(w->type, w->ne[0], w->ne[1], M) || (c->opt.mmq_i8 && M >= mmq_min_cols_for(c) && mmq_i8_supported(w->type, w->ne[0], w->ne[1], M)));
+    if (M < 2 || c->opt.mmvq_max_cols != 2) return true;
+    if (w->type == GGML_TYPE_Q8_0) return !q80_mm_ok(c, w, M);
+    return !(panels_possible(c, w) && M >= mmq_min_cols_for(c, w) && mmq_i8_supported(w->type, w->ne[0], w->ne[1], M));
 }
 static int act_kind(int wtype) { return wtype == GGML_TYPE_Q8_0 ? GGML_TYPE_Q8_0 : GGML_TYPE_Q8_K; }
 static bool is_f32_contig(const ggml_tensor * t) { return t->type == GGML_TYPE_F32 && ggml_abi_is_contiguous(t); }
@@ -357,6 +367,16 @@ static size_t merged_partials(const backend_ctx * c, const ggml_cgraph * g, int 
 }
 static ws_plan plan_ws(backend_ctx * c, const ggml_cgraph * g) {
     ws_plan p;
+    {   // which K-quant carries this graph's weight bytes (mmq_min_cols_for)
+        size_t q4 = 0, q5 = 0;
+        for (int i = 0; i < g->n_nodes; ++i) {
+            const ggml_tensor * n = g->nodes[i];
+            if (n->op != GGML_OP_MUL_MAT || !n->src[0]) continue;
+            if (n->src[0]->type == GGML_TYPE_Q4_K) q4 += ggml_abi_nbytes(n->src[0]);
+            else if (n->src[0]->type == GGML_TYPE_Q5_K) q5 += ggml_abi_nbytes(n->src[0]);
+        }
+        c->mm_q5_major = q5 > q4;
+    }
     for (int i = 0; i < g->n_nodes; ++i) {
         const ggml_tensor * n = g->nodes[i];
         // (besides what follows: K.q of one head on one key head has this form, and the attention chain that may start at it has its own scratch)
@@ -367,7 +387,7 @@ static ws_plan plan_ws(backend_ctx * c, const ggml_cgraph * g) {
             // (2..32 columns: the skinny matrix-core kernel fetches 32 columns' worth of activation bytes whatever M is)
             // (and the wide form of the same unit fetches whole groups of 128 columns of a prompt batch)
             p.act_bytes = std::max(p.act_bytes, quantized_act_bytes(act_kind(n->src[0]->type), b->ne[0], (Mc >= 2 && Mc < 32) ? 32 : (Mc >= 33 ? (Mc + 127) / 128 * 128 : Mc)));
-            if (Mc >= mmq_min_cols_for(c) && (n->ne[0] % 4) == 0) {
+            if (Mc >= (c->opt.mmq_min_cols != 3 ? c->opt.mmq_min_cols : 2) && (n->ne[0] % 4) == 0) {
                 p.aux_bytes = std::max(p.aux_bytes, 3 * mmq_workspace_bytes(n->src[0]->type, b->ne[0], n->src[0]->ne[1], Mc, c->opt.mmq_skinny));  // (x3: up to three sibling matrices share a launch)
                 if (c->opt.mm_merge && c->opt.mmq_i8 && mmq_i8_supported(n->src[0]->type, b->ne[0], n->src[0]->ne[1], Mc)) p.aux_bytes = std::max(p.aux_bytes, merged_partials(c, g, i, Mc));
             }
@@ -729,7 +749,7 @@ static bool run_mul_mat_q(exec_state & st, const ggml_tensor * w, const ggml_ten
         c->st.kernel_launches++;
         return true;
     }
-    const bool q80_batch = w->type == GGML_TYPE_Q8_0 && !w2 && !add2 && mmq_q80_batch_supported(w->type, K, N, M);
+    const bool q80_batch = w->type == GGML_TYPE_Q8_0 && !w2 && !add2 && q80_mm_ok(c, w, M);
     const void * act = quantized_src1(st, b, q80_batch ? MI_ACT_Q80_PANEL : w->type);
     if (q80_batch) {  // a -np decode step, a prompt
         const uint8_t * wp = q80_panel_copy(c, w);
@@ -744,7 +764,7 @@ static bool run_mul_mat_q(exec_state & st, const ggml_tensor * w, const ggml_ten
     }
     const bool i8 = c->opt.mmq_i8 && mmq_i8_supported(w->type, K, N, M);
     const uint8_t * const panels = i8 && !w2 && !add2 && st.epi_dst != dst ? k_panels(c, w, N, M) : nullptr;
-    if (M >= mmq_min_cols_for(c) && !w2 && !add2 && (!add || i8) && (i8 || mmq_supported(w->type, K, N, M))) {
+    if (M >= mmq_min_cols_for(c, w) && !w2 && !add2 && (!add || i8) && (i8 || mmq_supported(w->type, K, N, M))) {
         timed_scope ts(c, (std::string("mmq_") + type_tag(w->type) + "_n" + std::to_string(N) + "_k" + std::to_string(K)).c_str(), wbytes, i8);
         int ks = panels || st.epi_dst == dst ? 1 : ((N % 4) == 0 && (dst->nb[1] % 16) == 0 ? mmq_pick_ksplit(K, N, M, c->opt.mmq_skinny, w->type) : 1);
         if ((size_t) ks * (size_t) M * (size_t) N * sizeof(float) > c->ws_size - st.aux_off) ks = 1;  // (no room behind partial products that wait for their reader)
@@ -873,7 +893,7 @@ static bool quant_consumers_only(const exec_state & st, int at, const ggml_tenso
     }
     return true;
 }
-// ... and the same question for Q8_0 weights (round 6): every reader of t is a Q8_0 mat-mul that takes a matrix-core kernel (2 columns and up) (its activations in panel
+// ... and the same question for Q8_0 weights (round 6): every reader of t is a Q8_0 mat-mul that takes a matrix-core kernel (q80_mm_ok) (its activations in panel
 // order), so a producer may leave Q8_0 panel blocks instead of f32
 static bool q80_panel_consumers_only(const exec_state & st, int at, const ggml_tensor * t) {
     if ((t->flags & GGML_TENSOR_FLAG_OUTPUT) || t->type != GGML_TYPE_F32 || (t->ne[0] % 128) != 0) return false;
@@ -886,7 +906,7 @@ static bool q80_panel_consumers_only(const exec_state & st, int at, const ggml_t
             if (u->src[s] != t) continue;
             const ggml_tensor * wt = u->src[0];
             if (!(u->op == GGML_OP_MUL_MAT && s == 1 && wt->type == GGML_TYPE_Q8_0 && wt->ne[2] == 1 && wt->ne[3] == 1 && rows_contig(wt) && !buffer_is_split(wt->buffer) &&
-                  mmq_q80_batch_supported(wt->type, wt->ne[0], wt->ne[1], M) && u->type == GGML_TYPE_F32 && ggml_abi_is_contiguous(u)))
+                  q80_mm_ok(st.c, wt, M) && u->type == GGML_TYPE_F32 && ggml_abi_is_contiguous(u)))
                 return false;
             if (mat_vec_fusions(st.c, wt, M)) return false;  // (those quantise t themselves, in another order)
             if (tp_active(st.c) && buffer_is_rowpar(wt->view_src ? wt->view_src->buffer : wt->buffer)) return false;
@@ -1499,7 +1519,7 @@ static int try_merge_q80_skinny(exec_state & st, int i) {  // returns the number
     auto eligible = [&](const ggml_tensor * t) {
         const ggml_tensor * w = t->src[0];
         return t->op == GGML_OP_MUL_MAT && t->src[1] == X && w->type == GGML_TYPE_Q8_0 && w->ne[0] == K && w->ne[2] == 1 && w->ne[3] == 1 && rows_contig(w) && !buffer_is_split(w->buffer) &&
-               mmq_q80_batch_supported(w->type, K, w->ne[1], M) && t->type == GGML_TYPE_F32 && ggml_abi_is_contiguous(t) && !(tp_active(c) && buffer_is_rowpar(w->view_src ? w->view_src->buffer : w->buffer));
+               q80_mm_ok(c, w, M) && t->type == GGML_TYPE_F32 && ggml_abi_is_contiguous(t) && !(tp_active(c) && buffer_is_rowpar(w->view_src ? w->view_src->buffer : w->buffer));
     };
     auto with_add = [&](int k) {  // member at node k, with the ADD that directly follows it folded in
         ggml_tensor * t = g->nodes[k];
@@ -2940,16 +2960,15 @@ static int run_node(exec_state & st, int i) {
                     return 2;
                 }
             }
-            if (fuse && !rowpar && c->opt.mm_merge && a->type == GGML_TYPE_Q8_0 && mmq_q80_batch_supported(a->type, a->ne[0], a->ne[1], M)) {
+            if (fuse && !rowpar && c->opt.mm_merge && a->type == GGML_TYPE_Q8_0 && q80_mm_ok(c, a, M)) {
                 const int used = try_merge_q80_skinny(st, i);
                 if (used != 0) return used;
             }
-            if (fuse && !rowpar && c->opt.mm_merge && M >= mmq_min_cols_for(c) && c->opt.mmq_i8 && mmq_i8_supported(a->type, a->ne[0], a->ne[1], M)) {
+            if (fuse && !rowpar && c->opt.mm_merge && M >= mmq_min_cols_for(c, a) && c->opt.mmq_i8 && mmq_i8_supported(a->type, a->ne[0], a->ne[1], M)) {
                 const int used = try_merge_mm_batch(st, i);
                 if (used != 0) return used;
             }
-            if (fuse && !rowpar && ((M >= mmq_min_cols_for(c) && c->opt.mmq_i8 && mmq_i8_supported(a->type, a->ne[0], a->ne[1], M)) ||
-                                    mmq_q80_batch_supported(a->type, a->ne[0], a->ne[1], M))) {
+            if (fuse && !rowpar && ((M >= mmq_min_cols_for(c, a) && c->opt.mmq_i8 && mmq_i8_supported(a->type, a->ne[0], a->ne[1], M)) || q80_mm_ok(c, a, M))) {
                 // batches: MUL_MAT -> ADD (bias row or residual) rides in the GEMM's store
                 ggml_tensor * a1 = next(1);
                 const ggml_tensor * o1 = (a1 && single_use(st, n)) ? add_partner(a1, n) : nullptr;

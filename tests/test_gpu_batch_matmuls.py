@@ -538,3 +538,31 @@ def test_q6_k_panels_and_slices(backend, H, K, N, M, tiled):
     assert backend.stat("tiled_launches") == c0 + tiled
     rows = np.unique(np.concatenate([np.arange(min(N, 20)), np.arange(max(0, N - 20), N)]))
     assert T.nmse(got[:, rows], run("oracle", np.ascontiguousarray(w[rows]), np.ascontiguousarray(b[:, rows]))) <= 1e-10
+
+
+@pytest.mark.parametrize("copies", [1, 0])
+@pytest.mark.parametrize("types,M,served", [  # (launches of the matrix-core kernels with / without the copies)
+    ((L.Q5_K,), 2, (1, 0)), ((L.Q5_K,), 3, (1, 1)), ((L.Q5_K, L.Q6_K), 2, (2, 0)), ((L.Q4_K, L.Q6_K), 2, (2, 2)), ((L.Q4_K,), 2, (1, 1))])
+def test_two_columns_with_and_without_second_copies(backend, H, copies, types, M, served):
+    """graph.cpp: mmq_min_cols_for: two columns of a model's weights leave the mat-vec for the matrix cores only where second copies of the matrices may exist."""
+    K, N = 1024, 96
+    rng = np.random.default_rng(M + len(types))
+    ws = [T.rand_weight(t, K, N, rng) for t in types]
+    xs = [(rng.standard_normal((M, K)) * rng.uniform(0.2, 3.0, (M, 1))).astype(np.float32) for _ in types]
+    outs = lambda g: [H.ggml_mul_mat(g.ctx, g.new(t, [K, N], w), g.new(L.F32, [K, M], x)) for t, w, x in zip(types, ws, xs)]  # noqa: E731
+    ref = T.run_case(outs, "oracle")
+    backend.set_option("decode_copy", copies)
+    g = T.G(backend)
+    try:
+        os_ = outs(g)
+        g.compute(os_)
+        H.ggml_backend_buffer_set_usage(g.buf, 1)
+        s0 = backend.stat("skinny_launches")
+        assert H.ggml_backend_graph_compute(backend.backend, g.gf) == 0
+        assert backend.stat("skinny_launches") - s0 == served[0 if copies else 1]
+        got = [g.read(o) for o in os_]
+    finally:
+        g.free()
+        backend.set_option("decode_copy", 1)
+    for a, b in zip(got, ref):
+        assert T.nmse(a, b) <= 1e-10
