@@ -542,9 +542,9 @@ def test_q6_k_panels_and_slices(backend, H, K, N, M, tiled):
 
 @pytest.mark.parametrize("copies", [1, 0])
 @pytest.mark.parametrize("types,M,served", [  # (launches of the matrix-core kernels with / without the copies)
-    ((L.Q5_K,), 2, (1, 0)), ((L.Q5_K,), 3, (1, 1)), ((L.Q5_K, L.Q6_K), 2, (2, 0)), ((L.Q4_K, L.Q6_K), 2, (2, 2)), ((L.Q4_K,), 2, (1, 1))])
+    ((L.Q8_0,), 2, (1, 0)), ((L.Q8_0,), 3, (1, 1)), ((L.Q5_K,), 2, (1, 0)), ((L.Q5_K,), 3, (1, 1)), ((L.Q5_K, L.Q6_K), 2, (2, 0)), ((L.Q4_K, L.Q6_K), 2, (2, 2)), ((L.Q4_K,), 2, (1, 1))])
 def test_two_columns_with_and_without_second_copies(backend, H, copies, types, M, served):
-    """graph.cpp: mmq_min_cols_for: two columns of a model's weights leave the mat-vec for the matrix cores only where second copies of the matrices may exist."""
+    """graph.cpp: q80_mm_ok, mmq_min_cols_for: two columns of a model's weights leave the mat-vec for the matrix cores only where second copies of the matrices may exist."""
     K, N = 1024, 96
     rng = np.random.default_rng(M + len(types))
     ws = [T.rand_weight(t, K, N, rng) for t in types]
