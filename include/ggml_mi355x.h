@@ -55,6 +55,9 @@ ggml_backend_reg_t ggml_backend_mi355x_reg(void);
  *   "ggml_backend_mi355x_tp_p2p_attach"   ggml_backend_mi355x_tp_p2p_attach_t
  *   "ggml_backend_mi355x_tp_all_reduce"   ggml_backend_mi355x_tp_all_reduce_t
  *   "ggml_backend_mi355x_graph_key_probe" ggml_backend_mi355x_graph_key_probe_t   (tests: is graph b the graph a captured hipGraph of a stands for?)
+ *   "ggml_backend_mi355x_scratch_probe"   ggml_backend_mi355x_scratch_probe_t   (tests: the scratch that a graph's partial products and records may take)
+ *   "ggml_backend_mi355x_k_slices"        ggml_backend_mi355x_k_slices_t        (tests: K slices of a K-quant product)
+ *   "ggml_backend_mi355x_prepare_columns" ggml_backend_mi355x_prepare_columns_t
  *   "ggml_backend_mi355x_decode_copy_read" ggml_backend_mi355x_decode_copy_read_t (tests: the plane-layout decode copy of a weight matrix, csrc/repack.hip)
  */
 
@@ -89,6 +92,16 @@ typedef ggml_backend_buffer_type_t (*ggml_backend_mi355x_tp_rowpar_buffer_type_t
  * llama_decode with the one it replayed last: 1 = same captured hipGraph serves both, 0 = not.  *n_words (may be NULL) = 8-byte words of the key.
  * Host arithmetic: works without a device. */
 typedef int (*ggml_backend_mi355x_graph_key_probe_t)(const struct ggml_cgraph * a, const struct ggml_cgraph * b, int64_t * n_words);
+
+/* Bytes behind the activations that a backend with the default options sets aside for graph `g`; the slices of the K range in a launch of n_rows rows (of all its matrices) and
+ * n_cols columns.  Host arithmetic: both work without a device. */
+typedef int64_t (*ggml_backend_mi355x_scratch_probe_t)(const struct ggml_cgraph * g);
+typedef int (*ggml_backend_mi355x_k_slices_t)(int type, int64_t K, int64_t n_rows, int64_t n_cols);
+
+/* Makes the panel copies (csrc/mmq_panel.hip) that batches of from .. to (2 .. 32) columns would read of n weight matrices over the same activations (gate and up, say), in the backend's
+ * stream.  A host that has loaded its weights may call it once per group of matrices, so that the first such batch does not have to make them; copies that exist are kept.  Returns the
+ * number of matrices that have one, -1 on error. */
+typedef int (*ggml_backend_mi355x_prepare_columns_t)(ggml_backend_t backend, const struct ggml_tensor * const * matrices, int n, int64_t from, int64_t to);
 
 /* The decode copy (round 6): K-quant weight matrices of a usage-WEIGHTS buffer are kept a second time in a line-aligned plane layout that the batch-1 mat-vec kernels
  * stream with non-temporal loads (csrc/repack.hip, csrc/mmvq_types.h; option "decode_copy", GGML_MI355X_DECODE_COPY).  The tensor the host uploaded stays as it is:

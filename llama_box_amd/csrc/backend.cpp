@@ -999,6 +999,13 @@ static int api_graph_key_probe(const ggml_cgraph * a, const ggml_cgraph * b, int
 // ... and what decides whether K slices fit the scratch: the bytes set aside for a graph, the slices that a product of n_rows rows (of all matrices of its launch) and M columns takes
 static int64_t api_scratch_probe(const ggml_cgraph * g) { return partials_reserved(g); }
 static int api_k_slices(int type, int64_t K, int64_t n_rows, int64_t M) { return mmq_pick_ksplit(K, n_rows, M, options().mmq_skinny, type); }
+static int api_prepare_columns(ggml_backend_t be, const ggml_tensor * const * w, int n, int64_t from, int64_t to) {
+    if (!be_is_ours(be) || w == nullptr || n < 1 || std::find(w, w + n, nullptr) != w + n) return -1;
+    backend_ctx * c = (backend_ctx *) be->context;
+    HIP_TRY(hipSetDevice(c->device), -1);
+    uploader_join(c->device, c->stream);  // (weights staged by set_tensor are complete before they are read)
+    return prepare_columns(c, w, n, from, to);
+}
 // tests: the decode copy of weight matrix t (repacking it first if need be) into `out`; returns its bytes, 0 when the tensor has / gets no copy, -1 on error
 static int64_t api_decode_copy_read(ggml_backend_t be, const ggml_tensor * t, void * out, size_t size) {
     if (!be_is_ours(be) || t == nullptr) return -1;
@@ -1142,6 +1149,7 @@ static void * reg_get_proc_address(ggml_backend_reg_t, const char * name) {
     if (n == "ggml_backend_mi355x_tp_all_reduce") return (void *) api_tp_all_reduce;
     if (n == "ggml_backend_mi355x_tp_rowpar_buffer_type") return (void *) api_tp_rowpar_buft;
     if (n == "ggml_backend_mi355x_set_option") return (void *) api_set_option;
+    if (n == "ggml_backend_mi355x_prepare_columns") return (void *) api_prepare_columns;
     if (n == "ggml_backend_mi355x_decode_copy_read") return (void *) api_decode_copy_read;
     if (n == "ggml_backend_mi355x_get_stat") return (void *) api_get_stat;
     if (n == "ggml_backend_mi355x_timing_report") return (void *) api_timing_report;

@@ -316,6 +316,7 @@ struct buffer_ctx {
 // the plane-layout copy of weight matrix w for the batch-1 mat-vec kernels, or nullptr (no copy: views, split / row-parallel buffers, option off,
 // allocation failed, or asked during a capture for a tensor not yet repacked)
 const uint8_t * decode_copy(backend_ctx * c, const ggml_tensor * w);
+int prepare_columns(backend_ctx * c, const ggml_tensor * const * w, int n, int64_t from, int64_t to);  // graph.cpp
 bool k_panel_possible(const backend_ctx * c, const ggml_tensor * w);    // does it have a panel copy, or may it get one?
 const uint8_t * k_panel_copy(backend_ctx * c, const ggml_tensor * w);    // a K-quant matrix's panel copy (mmq_panel.hip), or nullptr
 const uint8_t * q80_panel_copy(backend_ctx * c, const ggml_tensor * w);  // a Q8_0 matrix's panel copy (mmq_q80.hip), or nullptr

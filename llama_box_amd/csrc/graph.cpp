@@ -37,6 +37,24 @@ static bool q80_mm_ok(backend_ctx * c, const ggml_tensor * w, int64_t M) {
 static const uint8_t * k_panels(backend_ctx * c, const ggml_tensor * w, int64_t n_total, int64_t M) {
     return c->opt.mmq_i8 && c->opt.mmq_skinny && M >= mmq_min_cols_for(c, w) && mmq_panel_applies(w->type, w->ne[0], n_total, M) ? k_panel_copy(c, w) : nullptr;
 }
+// Panel copies, made now, of n matrices over the same activations that a batch of `from` .. `to` columns would read (as the launch over all of them, or each alone where their formats differ); returns
+// how many have one.  The context's creation asks for them (host/llama_lite.cpp): left to the first batch, they came with its time (k_panel_copy: the first step of three sequences 5.3 ms, not 3.9).
+int prepare_columns(backend_ctx * c, const ggml_tensor * const * w, int n, int64_t from, int64_t to) {
+    bool together = true;
+    int64_t rows = 0;
+    int made = 0;
+    for (int i = 0; i < n; ++i) {
+        together = together && w[i]->type == w[0]->type && w[i]->ne[0] == w[0]->ne[0];
+        rows += w[i]->ne[1];
+    }
+    for (int i = 0; i < n; ++i)
+        for (int64_t M = std::max<int64_t>(2, from); M <= std::min<int64_t>(32, to); ++M)
+            if (k_panels(c, w[i], together ? rows : w[i]->ne[1], M)) {
+                made++;
+                break;
+            }
+    return made;
+}
 // Does a batch of M columns take the mat-vec fusions (gate/up/SwiGLU, bias and residual in one launch)?  Left at its default, the option leaves two columns to the matrix cores where copies serve them.
 // Without copies, steps as above, fusions / none: Q4_K_M at width 8192 1429 / 1500, 3584 747 / 757, 4096 684 / 653.
 static bool mat_vec_fusions(backend_ctx * c, const ggml_tensor * w, int64_t M) {

@@ -3273,6 +3273,29 @@ static void build_graph(llm_context * c, int n_tokens, int n_kv, int n_outputs, 
     c->gf = gf;
 }
 
+// the second copies that the device's kernels for batches of a few columns read are made with the context, not in front of the first such batch
+static void prepare_columns(ggml_backend_t be, int n_ubatch, const std::vector<std::vector<ggml_tensor *>> & groups) {
+    typedef int (*prepare_t)(ggml_backend_t, ggml_tensor * const *, int, int64_t, int64_t);
+    const prepare_t prepare = be->device && be->device->reg ? (prepare_t) ggml_backend_reg_get_proc_address(be->device->reg, "ggml_backend_mi355x_prepare_columns") : nullptr;
+    if (prepare == nullptr || n_ubatch < 2) return;
+    for (auto g : groups) {
+        g.erase(std::remove(g.begin(), g.end(), nullptr), g.end());
+        if (!g.empty()) prepare(be, g.data(), (int) g.size(), 2, n_ubatch);
+    }
+    ggml_backend_synchronize(be);
+}
+static std::vector<std::vector<ggml_tensor *>> column_groups(const llm_model * m, int l0, int l1, bool with_output) {  // matrices that a batch multiplies by the same rows
+    std::vector<std::vector<ggml_tensor *>> groups;
+    for (int il = l0; il < l1; ++il) {
+        const llm_layer & L = m->layers[(size_t) il];
+        groups.push_back({L.ffn_gate, L.ffn_up});
+        groups.push_back({L.ffn_down});
+        groups.push_back({L.wo});
+    }
+    if (with_output) groups.push_back({m->output});
+    return groups;
+}
+
 extern "C" struct llm_context * llm_context_new(struct llm_model * m, ggml_backend_t backend, llm_compute_fn compute, const struct llm_context_params * p) {
     if ((backend == nullptr) == (compute == nullptr)) {
         fprintf(stderr, "llm_context_new: exactly one of backend / compute must be given\n");
@@ -3399,6 +3422,7 @@ extern "C" struct llm_context * llm_context_new(struct llm_model * m, ggml_backe
                 for (ggml_backend_event_t & e : c->pin_ev) e = ggml_backend_event_new(backend->device);
             }
         }
+        prepare_columns(backend, c->p.n_ubatch, column_groups(m, 0, (int) m->layers.size(), true));
     }
     return c;
 }
@@ -3557,6 +3581,7 @@ extern "C" struct llm_context * llm_context_new_layer_split(struct llm_model * m
         const bool ok = ggml_gallocr_reserve(D.galloc, gf);
         ggml_free(tmp);
         if (!ok) { llm_context_free(c); return nullptr; }
+        prepare_columns(D.be, c->p.n_ubatch, column_groups(m, D.l0, D.l1, d == n_dev - 1));
     }
     c->cells.assign((size_t) c->p.n_ctx, kv_cell());
     c->used_max = 0;

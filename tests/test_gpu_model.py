@@ -1022,3 +1022,26 @@ def test_uploads_wait_for_the_download_that_fills_their_source(backend, H, nbyte
             g.free()
         if two:
             other.close()
+
+
+def test_copies_for_batches_are_made_with_the_context(backend, H):
+    """The first step of a few sequences finds the panel copies that it reads (llama_lite.cpp: prepare_columns)."""
+    hp = preset("llama3-8b-q4_k_m")
+    hp.n_layer, hp.n_vocab = 2, 32000
+    m = Model(hp, 3, backend.buft)
+    c = None
+    try:
+        s0 = backend.stat("decode_copy_tensors")
+        c = Context(m, backend=backend, n_ctx=512, flash_attn=1)
+        made = backend.stat("decode_copy_tensors") - s0
+        assert made == 5  # gate and up of two layers, the output matrix
+        n0 = backend.stat("decode_copy_launches")
+        assert c.decode([1, 2, 3], [0, 0, 0], seq=[0, 1, 2])[0] == 0
+        assert backend.stat("decode_copy_launches") > n0 and backend.stat("decode_copy_tensors") - s0 == made
+        c2 = Context(m, backend=backend, n_ctx=512, flash_attn=0)
+        c2.free()
+        assert backend.stat("decode_copy_tensors") - s0 == made
+    finally:
+        if c:
+            c.free()
+        m.free()
