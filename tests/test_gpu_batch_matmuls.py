@@ -1,4 +1,5 @@
 """Mat-muls of prompts and batches at the edges of their kernels' tiles, against the oracle."""
+import ctypes as C
 import os
 import subprocess
 import sys
@@ -566,3 +567,74 @@ def test_two_columns_with_and_without_second_copies(backend, H, copies, types, M
         backend.set_option("decode_copy", 1)
     for a, b in zip(got, ref):
         assert T.nmse(a, b) <= 1e-10
+
+
+@pytest.mark.parametrize("wt", [L.Q4_K, L.Q5_K, L.Q6_K])
+def test_panel_copies_follow_their_weight(backend, H, wt):
+    """backend.cpp: k_panel_copy: eager and captured runs follow a weight that is written again in part; a second backend may use a copy that the first has just been asked to make; without
+    room the blocks are read."""
+    K, N, M = 4096, 9216, 5
+    rng = np.random.default_rng(wt)
+    w = [T.rand_weight(wt, K, N, rng).reshape(N, -1) for _ in range(2)]
+    x = [(rng.standard_normal((M, K)) * rng.uniform(0.2, 3.0, (M, 1))).astype(np.float32) for _ in range(2)]
+    w_mixed = np.concatenate([w[0][:N // 2], w[1][N // 2:]])
+    rows = np.unique(np.concatenate([np.arange(16), np.arange(N // 2 - 16, N // 2 + 16), np.arange(N - 16, N)]))
+
+    def ref(ww, xx):
+        return T.run_case(lambda g: H.ggml_mul_mat(g.ctx, g.new(wt, [K, len(rows)], np.ascontiguousarray(ww[rows])), g.new(L.F32, [K, M], xx)), "oracle")[0].reshape(M, -1)
+
+    H.ggml_backend_graph_compute_async.argtypes = [C.c_void_p, C.POINTER(L.CGraph)]
+    other = L.Backend(0)
+    g = T.G(backend)
+    try:
+        wt_t = g.new(wt, [K, N], w[0])
+        outs, graphs = [], []
+        for xx in x:  # (eight nodes: a repeated graph is captured)
+            cur = g.new(L.F32, [K, M], xx)
+            for _ in range(8):
+                cur = H.ggml_scale(g.ctx, cur, -1.0)
+            outs.append(H.ggml_mul_mat(g.ctx, wt_t, cur))
+        g.compute(outs)
+        H.ggml_backend_buffer_set_usage(g.buf, 1)
+        for o in outs:
+            graphs.append(H.ggml_new_graph_custom(g.ctx, 64, False))
+            H.ggml_build_forward_expand(graphs[-1], o)
+        bes = [backend, other]
+
+        def both():
+            for be, gf in zip(bes, graphs):
+                assert H.ggml_backend_graph_compute_async(be.backend, gf) == 0
+            for be in bes:
+                H.ggml_backend_synchronize(be.backend)
+            return [g.read(o).reshape(M, N)[:, rows] for o in outs]
+
+        for ww in (w[0], w_mixed, w[1]):
+            if ww is w_mixed:
+                part = np.ascontiguousarray(w[1][N // 2:])
+                H.ggml_backend_tensor_set(wt_t, part.ctypes.data, w[0][:N // 2].nbytes, part.nbytes)
+            elif ww is w[1]:
+                H.ggml_backend_tensor_set(wt_t, w[1].ctypes.data, 0, w[1].nbytes)
+            want = [ref(ww, xx) for xx in x]
+            n0, l0 = backend.stat("decode_copy_launches"), backend.stat("graph_launches")
+            for _ in range(4):
+                for a, b in zip(both(), want):
+                    assert T.nmse(a, b) <= 1e-10
+            assert backend.stat("decode_copy_launches") > n0 and backend.stat("graph_launches") > l0
+            bes.reverse()  # (the other backend makes the next copy)
+    finally:
+        g.free()
+        other.close()
+    backend.set_option("decode_copy_headroom_gib", 1 << 20)
+    g = T.G(backend)
+    try:
+        o = H.ggml_mul_mat(g.ctx, g.new(wt, [K, N], w[0]), g.new(L.F32, [K, M], x[0]))
+        blocks = g.compute([o])[0].copy()
+        H.ggml_backend_buffer_set_usage(g.buf, 1)
+        n0 = backend.stat("decode_copy_launches")
+        assert H.ggml_backend_graph_compute(backend.backend, g.gf) == 0
+        assert backend.stat("decode_copy_launches") == n0
+        assert np.array_equal(g.read(o).view(np.uint32), blocks.view(np.uint32))
+        assert T.nmse(blocks.reshape(M, N)[:, rows], ref(w[0], x[0])) <= 1e-10
+    finally:
+        g.free()
+        backend.set_option("decode_copy_headroom_gib", 2)
