@@ -25,7 +25,7 @@ namespace mi355x {
 #define NF_CAP 1024  // visible cells per token served from registers and LDS
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
-struct __attribute__((aligned(4))) u32x4a { uint32_t x, y, z, w; };  // a 16-byte load that only promises dword alignment
+struct __attribute__((packed, aligned(2))) u32x4a { uint32_t x, y, z, w; };  // a 16-byte load from where a value of 16 bits may lie
 template <int G, int NW>
 __global__ void __launch_bounds__(NW * 64) k_attn_nf_list(const tdesc q, const tdesc k, const tdesc v, const tdesc mask, const tdesc dst, const int * __restrict__ lists,
                                                       const int list_stride, float * __restrict__ scratch, const float scale, const int dq_n, q8k_dev * __restrict__ q8, const int nf_groups_on) {
@@ -291,7 +291,7 @@ __global__ void __launch_bounds__(NW * 64) k_attn_nf_list(const tdesc q, const t
             const int ngr = (cnt + 7) / 8, gi_l = lane;
             const bool in = gi_l < ngr;
             const int p_first = pos_s[min(8 * gi_l, cnt - 1)], p_last = pos_s[min(8 * gi_l + 7, cnt - 1)];
-            const bool is_run = in && 8 * gi_l + 7 < cnt && p_last == p_first + 7 && (p_first & 1) == 0;  // ascending list: consecutive; even start: dword-aligned
+            const bool is_run = in && 8 * gi_l + 7 < cnt && p_last == p_first + 7;  // ascending list: consecutive
             const int wv = __builtin_amdgcn_readfirstlane(wave);  // (wave-uniform for the compiler too: the masks and group indices below are scalars)
             const unsigned long long par = (wv >> 1) ? 0xAAAAAAAAAAAAAAAAull : 0x5555555555555555ull;
             unsigned long long m_run = __ballot(is_run) & par, m_sc = __ballot(in && !is_run) & par;
@@ -475,13 +475,15 @@ size_t attn_nf_list_scratch_bytes(const tdesc & q, const tdesc & k, int * dq_out
     // when the cache holds at most NF_CAP cells per token of the batch — the decode steps of many sequences — and a few tokens over
     // long contexts stay on the dense kernels.
     if (n_kv > (int64_t) NF_CAP * T) return 0;
-    // Slices of the head dimensions: enough workgroups for the chip when the tokens are few.  But each slice fetches all the K rows again, and only whole rows leave as Q8_K blocks: from 80
-    // (token, KV head) pairs on whole rows are faster while a token sees 256 cells at the most (512 from 160 pairs on).  A step of Llama-3-8B, us, slices / whole rows: 12 sequences of 160 cells
-    // 2957 / 2816, 16 of 160 3017 / 2882, of 300 3074 / 3110, 20 of 380 3610 / 3517, 8 of 150 2703 / 2729; Qwen2-7B, 30 of 100 4036 / 3846.  Measured with four and seven heads on a KV head and
-    // from 64 cells a token on; others keep their slices.
+    // Slices of the head dimensions: enough workgroups for the chip when the tokens are few.  But each slice fetches all the K rows again, and only whole rows leave as Q8_K blocks (of an even number of
+    // heads): from 80 (token, KV head) pairs on whole rows are faster while a token sees few cells.  Steps of eight layers, 8 KV heads of 128, us, slices / whole rows, sequences x cells:
+    //   4 heads: 10 x 151 776 / 772, 201 781 / 792; 16 x 151 817 / 798, 241 829 / 840; 20 x 151 913 / 871, 241 939 / 927, 401 1010 / 1023;  6: 10 x 151 1025 / 1017, 16 x 241 1091 / 1094,
+    //   20 x 241 1258 / 1223;  7: 10 x 151 1162 / 1164, 16 x 151 1218 / 1192, 241 1234 / 1247, 20 x 241 1402 / 1384;  8: 10 x 151 1241 / 1219, 16 x 151 1314 / 1260, 20 x 401 1616 / 1591;
+    //   5 (no blocks left, and rows of five sums): 10 x 71 937 / 931, 125 950 / 965, 16 x 71 982 / 960, 151 995 / 1001, 20 x 151 1135 / 1106, 401 1237 / 1259.
+    // (Histories of an even number of cells are 1 to 3 % better off with whole rows than these.)  Fewer heads keep their slices.
     int dq = 1;
     const int64_t pairs = T * NKV;
-    const bool whole = G >= 4 && pairs >= 80 && n_kv >= 64 * T && n_kv <= (pairs >= 160 ? 512 : 256) * T;
+    const bool whole = G >= 4 && pairs >= 80 && n_kv >= 64 * T && n_kv <= (pairs >= 160 ? 320 : G == 5 ? 112 : pairs >= 104 ? 208 : 176) * T;
     while (!whole && dq < 8 && pairs * dq < 192) dq *= 2;
     if (dq_out) *dq_out = dq;
     return (size_t) (T * NKV * dq * G * n_kv) * sizeof(float);

@@ -402,3 +402,41 @@ def test_few_tokens_over_a_cache_beyond_32_bit_offsets(backend, H):
             ref = v[h // G][:, see].astype(np.float64) @ p
             # (as test_few_tokens_on_matrix_cores)
             assert np.abs(got[h, t] - ref).max() <= 2e-3 * np.abs(ref).max() + 1e-5, (t, h)
+
+
+@pytest.mark.parametrize("T_,NKV,G,per,first", [(10, 8, 4, 71, 1), (16, 8, 5, 69, 0), (10, 8, 7, 75, 17), (12, 8, 8, 170, 7), (24, 8, 6, 33, 231)])
+def test_few_tokens_over_runs_of_cells(backend, H, T_, NKV, G, per, first):
+    """attn_nf.hip, whole rows: eight consecutive cells are one load wherever they begin, up to the last cell of the cache; a cell out of the row ends a run."""
+    rng = np.random.default_rng(T_ + per + G)
+    HD, NH = 128, NKV * G
+    n_kv = (first + T_ * per + 255) // 256 * 256
+    k = rng.standard_normal((n_kv, NKV, HD)).astype(np.float16)
+    v = rng.standard_normal((NKV, HD, n_kv)).astype(np.float16)
+    q = (3 * rng.standard_normal((T_, NH, HD))).astype(np.float32)
+    mask = np.full((T_, n_kv), -np.inf, np.float32)
+    for t in range(T_):
+        mask[t, first + t * per:first + (t + 1) * per] = 0
+        mask[t, (7 * t) % n_kv] = 0
+    mask[T_ - 1, n_kv - 9:] = 0
+
+    def build(g):
+        kc, vc = g.new(L.F16, [NKV * HD, n_kv], k.reshape(n_kv, -1)), g.new(L.F16, [n_kv, NKV * HD], v.reshape(-1, n_kv))
+        qp = H.ggml_permute(g.ctx, g.new(L.F32, [HD, NH, T_], q), 0, 2, 1, 3)
+        kv = H.ggml_view_3d(g.ctx, kc, HD, n_kv, NKV, NKV * HD * 2, HD * 2, 0)
+        vv = H.ggml_view_3d(g.ctx, vc, n_kv, HD, NKV, n_kv * 2, n_kv * 2 * HD, 0)
+        p = H.ggml_soft_max_ext(g.ctx, H.ggml_mul_mat(g.ctx, kv, qp), g.new(L.F32, [n_kv, T_], mask), HD ** -0.5, 0.0)
+        return H.ggml_mul_mat(g.ctx, vv, p)
+
+    s0 = backend.stat("kernel_launches")
+    got = T.run_case(build, backend)[0].reshape(NH, T_, HD)
+    assert backend.stat("kernel_launches") - s0 <= 2
+    qh = q.astype(np.float16).astype(np.float64)
+    for t in range(T_):
+        see = np.flatnonzero(mask[t] == 0)
+        for h in range(NH):
+            s = k[see, h // G].astype(np.float64) @ qh[t, h] * HD ** -0.5
+            p = np.exp(s - s.max())
+            p = (p / p.sum()).astype(np.float16).astype(np.float64)
+            ref = v[h // G][:, see].astype(np.float64) @ p
+            # (as test_few_tokens_on_matrix_cores)
+            assert np.abs(got[h, t] - ref).max() <= 2e-3 * np.abs(ref).max() + 1e-5, (t, h)
