@@ -72,9 +72,9 @@ static void decode_copy_drop(buffer_ctx * c, size_t off, size_t n) {
     std::lock_guard<std::mutex> lk(c->sh_mtx);
     bool any = false;
     for (auto & p : c->panels)
-        if (p.second.valid && p.first < off + n && off < p.first + p.second.bytes) { p.second.valid = false; any = true; }
+        if (p.second.valid && p.first < off + n && off < p.first + p.second.of.bytes) { p.second.valid = false; any = true; }
     for (auto it = c->sh_valid.begin(); it != c->sh_valid.end();) {
-        if (it->first < off + n && off < it->first + it->second) { it = c->sh_valid.erase(it); any = true; }
+        if (it->first < off + n && off < it->first + it->second.bytes) { it = c->sh_valid.erase(it); any = true; }
         else ++it;
     }
     if (any) g_decode_epoch.fetch_add(1, std::memory_order_acq_rel);
@@ -105,7 +105,7 @@ static const uint8_t * second_copy(backend_ctx * c, const ggml_tensor * w, const
     const size_t off = (size_t) ((const char *) w->data - (const char *) bc->base), bytes = (size_t) w->nb[1] * (size_t) w->ne[1];
     std::lock_guard<std::mutex> lk(bc->sh_mtx);
     auto it = bc->sh_valid.find(off);
-    if (it != bc->sh_valid.end() && it->second == bytes) return (const uint8_t *) bc->shadow + off;
+    if (it != bc->sh_valid.end()) return it->second == buffer_ctx::copy_of{bytes, (int) w->type, w->ne[0]} ? (const uint8_t *) bc->shadow + off : nullptr;  // (another tensor over the same bytes has it)
     if (c->capturing) return nullptr;  // (a capture is the SECOND run of a graph: its weights were repacked by the first; anything else keeps the block layout)
     if (bc->shadow == nullptr) {
         // 288 GB of HBM: a second copy of the weights one GPU serves always fits beside the first — unless the user filled the device on purpose; then the
@@ -123,7 +123,7 @@ static const uint8_t * second_copy(backend_ctx * c, const ggml_tensor * w, const
     else launch_repack_planes(c->stream, w->type, w->data, (char *) bc->shadow + off, w->ne[0], (int64_t) w->nb[1], 0, w->ne[1]);
     // (another backend instance of this device — its own stream — may find the entry valid a moment later: the copy is complete before it is announced)
     if (hipStreamSynchronize(c->stream) != hipSuccess) { (void) hipGetLastError(); return nullptr; }
-    bc->sh_valid[off] = bytes;
+    bc->sh_valid[off] = {bytes, (int) w->type, w->ne[0]};
     c->st.decode_copy_tensors++;
     c->st.decode_copy_bytes += (int64_t) bytes;
     return (const uint8_t *) bc->shadow + off;
@@ -142,7 +142,10 @@ const uint8_t * k_panel_copy(backend_ctx * c, const ggml_tensor * w) {
     auto it = bc->panels.find(off);
     if (it != bc->panels.end()) {
         buffer_ctx::panel_mem & p = it->second;
-        if (p.bytes != bytes) return nullptr;  // (another tensor was laid out at this offset before)
+        if (!(p.of == buffer_ctx::copy_of{bytes, (int) w->type, w->ne[0]})) {
+            if (p.valid || p.of.bytes != bytes) return nullptr;  // (another tensor over the same bytes has it, or had one of another size)
+            p.of = {bytes, (int) w->type, w->ne[0]};
+        }
         if (p.valid && p.maker != nullptr && p.maker != c) {  // (the maker may be gone by now, the event is the buffer's)
             if (c->capturing || hipEventSynchronize(p.made) != hipSuccess) { (void) hipGetLastError(); return nullptr; }
             p.maker = nullptr;
@@ -172,7 +175,7 @@ const uint8_t * k_panel_copy(backend_ctx * c, const ggml_tensor * w) {
             MI_INFO("panel copies: no room for %.2f GiB on device %d — batches of a few columns read the block layout", (double) bytes / (1 << 30), bc->device);
             return nullptr;
         }
-        it = bc->panels.emplace(off, buffer_ctx::panel_mem{(char *) ch->mem + ch->used, bytes, false, nullptr, made}).first;
+        it = bc->panels.emplace(off, buffer_ctx::panel_mem{(char *) ch->mem + ch->used, {bytes, (int) w->type, w->ne[0]}, false, nullptr, made}).first;
         ch->used += need;
     }
     buffer_ctx::panel_mem & p = it->second;

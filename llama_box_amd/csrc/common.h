@@ -303,10 +303,14 @@ struct buffer_ctx {
     void * shadow = nullptr;
     bool shadow_failed = false;
     std::mutex sh_mtx;
-    std::unordered_map<size_t, size_t> sh_valid;  // offset of a repacked tensor -> its bytes
+    struct copy_of {  // what a copy was made of: the same bytes read as rows of another length, or as another format, are another matrix
+        size_t bytes; int type; int64_t K;
+        bool operator==(const copy_of & o) const { return bytes == o.bytes && type == o.type && K == o.K; }
+    };
+    std::unordered_map<size_t, copy_of> sh_valid;  // offset of a repacked tensor -> the tensor
     // ... and the K-quant matrices that batches of a few columns multiply over panels (mmq_panel.hip): those only, in chunks that hold several; made, dropped and freed as above.  The step that first
     // uses a copy makes it on its own stream and goes on; another backend instance waits for `made` first
-    struct panel_mem { void * mem; size_t bytes; bool valid; const backend_ctx * maker; hipEvent_t made; };
+    struct panel_mem { void * mem; copy_of of; bool valid; const backend_ctx * maker; hipEvent_t made; };
     struct panel_chunk { void * mem; size_t size, used; };
     std::unordered_map<size_t, panel_mem> panels;  // offset of the tensor -> its panel copy
     std::vector<panel_chunk> panel_chunks;

@@ -638,3 +638,27 @@ def test_panel_copies_follow_their_weight(backend, H, wt):
     finally:
         g.free()
         backend.set_option("decode_copy_headroom_gib", 2)
+
+
+@pytest.mark.parametrize("wt,K,N,M", [(L.Q5_K, 2048, 18432, 4), (L.Q4_K, 2048, 512, 1), (L.Q8_0, 2048, 512, 4)])
+def test_two_tensors_over_the_same_bytes(backend, H, wt, K, N, M):
+    """backend.cpp: a second copy belongs to a matrix of one row length; another matrix over the same bytes (rows twice as long) does not read it."""
+    rng = np.random.default_rng(K + N + M)
+    w = T.rand_weight(wt, K, N, rng)
+    xs = [rng.standard_normal((M, k)).astype(np.float32) for k in (K, 2 * K)]
+    shapes = [(K, N), (2 * K, N // 2)]
+    ref = [T.run_case(lambda g: H.ggml_mul_mat(g.ctx, g.new(wt, [k, 64], np.ascontiguousarray(w.reshape(n, -1)[:64])), g.new(L.F32, [k, M], x)), "oracle")[0].reshape(M, -1) for (k, n), x in zip(shapes, xs)]
+    g = T.G(backend)
+    try:
+        ws = [g.new(wt, [k, n], w) for k, n in shapes]
+        outs = [H.ggml_mul_mat(g.ctx, t, g.new(L.F32, [k, M], x)) for t, (k, n), x in zip(ws, shapes, xs)]
+        g.compute(outs, same_block=[(ws[1], ws[0])])
+        H.ggml_backend_buffer_set_usage(g.buf, 1)
+        n0 = backend.stat("decode_copy_launches")
+        for _ in range(2):
+            assert H.ggml_backend_graph_compute(backend.backend, g.gf) == 0
+            for o, (k, n), r in zip(outs, shapes, ref):
+                assert T.nmse(g.read(o).reshape(M, n)[:, :64], r) <= 1e-10
+        assert backend.stat("decode_copy_launches") - n0 == 2
+    finally:
+        g.free()
