@@ -874,7 +874,7 @@ static ggml_backend_t dev_init_backend(ggml_backend_dev_t dev, const char *) {
         delete c;
         return nullptr;
     }
-    {   // the copy stream of stage_upload and its events: a stream's first use takes longer than the prompt that would find it missing
+    {   // the copy stream of stage_upload and its events, here and not in front of the first prompt that uses them: the process's first two streams take 5 ms longer to make than one
         bool ok = hipStreamCreateWithFlags(&c->up_stream, hipStreamNonBlocking) == hipSuccess;
         if (!ok) c->up_stream = nullptr;
         ok = ok && hipEventCreateWithFlags(&c->up_round, hipEventDisableTiming) == hipSuccess;

@@ -52,8 +52,8 @@ def test_mul_mat_q(backend, H, plog, qt, K, N, M):
 @pytest.mark.parametrize("qt", QTYPES)
 @pytest.mark.parametrize("K,N,M", [(1024, 48, 3), (512, 64, 4), (512, 20, 5), (768, 32, 8), (4096, 130, 7)])
 def test_mul_mat_q_multi_column_mat_vec(backend, H, plog, qt, K, N, M):
-    """3..8 columns on the multi-column mat-vec kernels (k_mmvq<T, NC>): the route taken when the matrix-core path is switched
-    off (mmq_min_cols above the batch) and, for Q8_0 weights, always below 33 columns."""
+    """3..8 columns on the multi-column mat-vec kernels (k_mmvq<T, NC>): the route of K-quants when the matrix-core path is switched
+    off (mmq_min_cols above the batch).  (Q8_0 rows of whole 128-value chunks take mmq_q80.hip all the same; the others: the next test.)"""
     rng = np.random.default_rng(K + N + M + qt)
     w = T.rand_weight(qt, K, N, rng)
     x = (rng.standard_normal((M, K)) * rng.uniform(0.2, 3.0, (M, 1))).astype(np.float32)
@@ -67,6 +67,18 @@ def test_mul_mat_q_multi_column_mat_vec(backend, H, plog, qt, K, N, M):
     finally:
         backend.set_option("mmq_min_cols", 3)
     T.compare(f"mul_mat multi-column mat-vec {QNAME[qt]} K={K} N={N} M={M}", got[0], ref[0], max_nmse=1e-10, log=plog)
+
+
+@pytest.mark.parametrize("K,N,M", [(1056, 48, 2), (544, 64, 3), (96, 20, 4), (800, 33, 5), (4128, 130, 7), (2080, 32, 8)])
+def test_mul_mat_q8_0_multi_column_mat_vec(backend, H, plog, K, N, M):
+    """2..8 columns of Q8_0 rows that are no whole 128-value chunks: the multi-column mat-vec kernel."""
+    rng = np.random.default_rng(K + N + M)
+    w = T.rand_weight(L.Q8_0, K, N, rng)
+    x = (rng.standard_normal((M, K)) * rng.uniform(0.2, 3.0, (M, 1))).astype(np.float32)
+    s0 = backend.stat("skinny_launches")
+    ref, got = both(lambda g: H.ggml_mul_mat(g.ctx, g.new(L.Q8_0, [K, N], w), g.new(L.F32, [K, M], x)), backend)
+    assert backend.stat("skinny_launches") == s0
+    T.compare(f"mul_mat q8_0 multi-column mat-vec K={K} N={N} M={M}", got[0], ref[0], max_nmse=1e-10, log=plog)
 
 
 @pytest.mark.parametrize("bias", [False, True])
