@@ -134,7 +134,7 @@ bool k_panel_possible(const backend_ctx * c, const ggml_tensor * w) {
     const buffer_ctx * const bc = copyable(c, w);
     return bc != nullptr && !bc->panels_failed && repack_supported(w->type, w->ne[0], (int64_t) w->nb[1]) && (w->ne[1] % 16) == 0;
 }
-const uint8_t * k_panel_copy(backend_ctx * c, const ggml_tensor * w) {
+const uint8_t * k_panel_copy(backend_ctx * c, const ggml_tensor * w, bool ahead) {
     buffer_ctx * const bc = copyable(c, w);
     if (bc == nullptr || !repack_supported(w->type, w->ne[0], (int64_t) w->nb[1]) || (w->ne[1] % 16) != 0) return nullptr;
     const size_t off = (size_t) ((const char *) w->data - (const char *) bc->base), bytes = (size_t) w->nb[1] * (size_t) w->ne[1];
@@ -161,6 +161,11 @@ const uint8_t * k_panel_copy(backend_ctx * c, const ggml_tensor * w) {
         bool ok = hipEventCreateWithFlags(&made, hipEventDisableTiming) == hipSuccess;
         if (ok && ch == bc->panel_chunks.end()) {
             buffer_ctx::panel_chunk k{nullptr, std::max(need, std::min(CHUNK, bc->size)), 0};
+            if (ahead && !room_for_copy(c, k.size + (bc->shadow || bc->shadow_failed ? 0 : bc->size))) {  // (the mat-vecs' copy of the whole buffer goes first)
+                (void) hipGetLastError();
+                (void) hipEventDestroy(made);
+                return nullptr;
+            }
             ok = room_for_copy(c, k.size) && hipMalloc(&k.mem, k.size) == hipSuccess;
             if (ok) {
                 bc->panel_chunks.push_back(k);

@@ -322,7 +322,8 @@ struct buffer_ctx {
 const uint8_t * decode_copy(backend_ctx * c, const ggml_tensor * w);
 int prepare_columns(backend_ctx * c, const ggml_tensor * const * w, int n, int64_t from, int64_t to);  // graph.cpp
 bool k_panel_possible(const backend_ctx * c, const ggml_tensor * w);    // does it have a panel copy, or may it get one?
-const uint8_t * k_panel_copy(backend_ctx * c, const ggml_tensor * w);    // a K-quant matrix's panel copy (mmq_panel.hip), or nullptr
+// a K-quant matrix's panel copy (mmq_panel.hip), or nullptr; ahead: no batch waits for it, so none either where the buffer's decode copy would not fit beside it any more
+const uint8_t * k_panel_copy(backend_ctx * c, const ggml_tensor * w, bool ahead = false);
 const uint8_t * q80_panel_copy(backend_ctx * c, const ggml_tensor * w);  // a Q8_0 matrix's panel copy (mmq_q80.hip), or nullptr
 uint64_t decode_copy_epoch();  // bumped whenever a copy was dropped: graphs captured before hold pointers to it
 bool buffer_is_ours(ggml_backend_buffer_t b);

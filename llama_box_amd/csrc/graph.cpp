@@ -34,8 +34,8 @@ static bool q80_mm_ok(backend_ctx * c, const ggml_tensor * w, int64_t M) {
     return M != 2 || b == nullptr || b->usage != GGML_BACKEND_BUFFER_USAGE_WEIGHTS || q80_panel_copy(c, w) != nullptr;
 }
 // the panel copy of a K-quant matrix where M columns are multiplied over it (mmq_panel.hip) in a launch of n_total rows, else nullptr
-static const uint8_t * k_panels(backend_ctx * c, const ggml_tensor * w, int64_t n_total, int64_t M) {
-    return c->opt.mmq_i8 && c->opt.mmq_skinny && M >= mmq_min_cols_for(c, w) && mmq_panel_applies(w->type, w->ne[0], n_total, M) ? k_panel_copy(c, w) : nullptr;
+static const uint8_t * k_panels(backend_ctx * c, const ggml_tensor * w, int64_t n_total, int64_t M, bool ahead = false) {
+    return c->opt.mmq_i8 && c->opt.mmq_skinny && M >= mmq_min_cols_for(c, w) && mmq_panel_applies(w->type, w->ne[0], n_total, M) ? k_panel_copy(c, w, ahead) : nullptr;
 }
 // Panel copies, made now, of n matrices over the same activations that a batch of `from` .. `to` columns would read (as the launch over all of them, or each alone where their formats differ); returns
 // how many have one.  The context's creation asks for them (host/llama_lite.cpp): left to the first batch, they came with its time (k_panel_copy: the first step of three sequences 5.3 ms, not 3.9).
@@ -49,7 +49,7 @@ int prepare_columns(backend_ctx * c, const ggml_tensor * const * w, int n, int64
     }
     for (int i = 0; i < n; ++i)
         for (int64_t M = std::max<int64_t>(2, from); M <= std::min<int64_t>(32, to); ++M)
-            if (k_panels(c, w[i], together ? rows : w[i]->ne[1], M)) {
+            if (k_panels(c, w[i], together ? rows : w[i]->ne[1], M, /*ahead=*/true)) {
                 made++;
                 break;
             }

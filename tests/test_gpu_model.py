@@ -1045,3 +1045,24 @@ def test_copies_for_batches_are_made_with_the_context(backend, H):
         if c:
             c.free()
         m.free()
+
+
+def test_copies_made_with_the_context_leave_room_for_the_decode_copy(backend, H):
+    """Where the mat-vecs' copy of the weights would not fit beside them, panel copies are not made with the context; the first batch that reads them makes them."""
+    m = Model(preset("llama3-8b-q4_k_m"), 3, backend.buft)
+    c = None
+    try:
+        free, total = C.c_size_t(), C.c_size_t()
+        H.ggml_backend_dev_memory(backend.dev, C.byref(free), C.byref(total))
+        backend.set_option("decode_copy_headroom_gib", (free.value >> 30) - 4)  # (4 GiB to spare, and some; the weights take 4.6)
+        s0 = backend.stat("decode_copy_tensors")
+        c = Context(m, backend=backend, n_ctx=512, flash_attn=1)
+        assert backend.stat("decode_copy_tensors") == s0
+        n0 = backend.stat("decode_copy_launches")
+        assert c.decode([1, 2, 3], [0, 0, 0], seq=[0, 1, 2])[0] == 0
+        assert backend.stat("decode_copy_tensors") > s0 and backend.stat("decode_copy_launches") > n0
+    finally:
+        backend.set_option("decode_copy_headroom_gib", 2)
+        if c:
+            c.free()
+        m.free()
