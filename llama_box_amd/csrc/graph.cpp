@@ -27,7 +27,7 @@ static int mmq_min_cols_for(const backend_ctx * c, const ggml_tensor * w) {
     return panels_possible(c, w) || w->type == GGML_TYPE_Q4_K || (w->type == GGML_TYPE_Q6_K && !c->mm_q5_major) ? 2 : 3;
 }
 // Does a batch of M columns multiply a Q8_0 matrix on the matrix cores (mmq_q80.hip)?  Two columns of a model's weights over their panel copy only.  Steps as above, mat-vec / matrix cores: TinyLlama with the copies 663 / 432,
-// without 678 / 726; width 4096 1076 / 696 and 1076 / 1556; three columns and more without them: TinyLlama x 3 1024 / 733, width 4096 x 4 1604 / 1569, x 8 2076 / 1604.
+// without 678 / 726; width 4096 1076 / 696 and 1076 / 1556 (width 1024 528 / 437 without: not told apart); three columns and more without them: TinyLlama x 3 1024 / 733, width 4096 x 4 1604 / 1569, x 8 2076 / 1604.
 static bool q80_mm_ok(backend_ctx * c, const ggml_tensor * w, int64_t M) {
     if (!mmq_q80_batch_supported(w->type, w->ne[0], w->ne[1], M)) return false;
     const ggml_backend_buffer_t b = w->view_src ? w->view_src->buffer : w->buffer;
