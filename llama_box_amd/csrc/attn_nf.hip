@@ -505,7 +505,7 @@ bool launch_attn_nf_list(hipStream_t s, const tdesc & q, const tdesc & k, const 
     dim3 grid((unsigned) q.ne[1], (unsigned) k.ne[2], (unsigned) dq);
     // Few tokens: every slice of the head dimensions computes all the logits of its heads.  While the grid is no more than one workgroup a CU, eight waves share the fetches (3 tokens x 700 cells of
     // Llama-3-8B, a launch: 26.5 us with four waves, 19.5 with eight; with the logits on the matrix cores, V^T requested ahead and a head's soft-max in one wave's registers 14.2: of these 6
-    // wait for the 200 KB a workgroup fetches, whatever its mapping to XCDs or the shape of its loads; one head on a KV head pays for the longer code where a token sees few cells: 32 KV heads, 2 x 60
+    // wait for the 200 KB a workgroup fetches, whatever its mapping to XCDs or the shape of its loads; one head on a KV head takes longer than before where a token sees few cells: 32 KV heads, 2 x 60
     // cells 5.8 -> 6.4, 2 x 300 9.2 -> 8.7, 4 x 901 22.6 -> 20.5); more workgroups than that already have the company of another.
     const bool few = dq > 1 && q.ne[1] * k.ne[2] * dq <= 256;
 #define NF_GO(G_, W_)                                                                                                                                                              \
