@@ -916,7 +916,7 @@ static bool quant_consumers_only(const exec_state & st, int at, const ggml_tenso
     }
     return true;
 }
-// ... and the same question for Q8_0 weights (round 6): every reader of t is a Q8_0 mat-mul that takes a matrix-core kernel (q80_mm_ok) (its activations in panel
+// ... and the same question for Q8_0 weights: every reader of t is a Q8_0 mat-mul that takes a matrix-core kernel (q80_mm_ok) (its activations in panel
 // order), so a producer may leave Q8_0 panel blocks instead of f32
 static bool q80_panel_consumers_only(const exec_state & st, int at, const ggml_tensor * t) {
     if ((t->flags & GGML_TENSOR_FLAG_OUTPUT) || t->type != GGML_TYPE_F32 || (t->ne[0] % 128) != 0) return false;
