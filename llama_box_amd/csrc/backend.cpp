@@ -385,7 +385,8 @@ void note_mask_upload(const ggml_tensor * t, const void * host, size_t offset, s
     if (rows < 2) { forget(); return; }
     mask_stats st;
     int64_t total = 0;
-    const int64_t dense_at = rows * n / 4 + 1;
+    // (a small mask is read to its end: the longest row decides how a few tokens' attention is split, and 64 KB take a few microseconds)
+    const int64_t dense_at = size <= (size_t) 65536 ? rows * n + 1 : rows * n / 4 + 1;
     for (int64_t r = 0; r < rows; ++r) {
         if (total >= dense_at) {  // dense whatever follows: density > 0.25 is all its readers ask (the longest row so far stands in for the rest)
             st.rows = (int) rows;

@@ -38,6 +38,7 @@ struct fa_geom {
     uint32_t n_head_log2;
     unsigned * arrive;  // != null (lane-parallel decode kernel, n_splits > 1): one counter per (batch, token, kv head); the LAST split workgroup to
                         // arrive merges the partial records itself — no combine launch (the counter is left at zero again)
+    void * q80;         // PART at head_dim 64: leave the result as Q8_0 blocks in panel order here instead of f32 in dst (see fattn_params::q80_out)
     void * q8;          // with `arrive`: leave the merged result as Q8_K blocks here instead of f32 in dst (see fattn_params::q8_out)
     int one_batch;      // q.ne[3] == 1 (every graph llama.cpp builds): the batch index is 0 and the kernels skip its integer divisions — the lane-parallel decode kernel ran
                         // 974 instructions, four emulated 64-bit divisions among them, before it issued its first load (round 6)
@@ -409,9 +410,11 @@ __device__ unsigned long long g_fa_stamps[1024][8];
 // D = 64 (round 6: TinyLlama, Llama-3.2-1B ...; f16 cache, no Q8_K output, records + combine pass): a K / V row is EIGHT lanes, a wave-instruction fetches eight
 // rows, the (row group, head) pairs of a row are 8 = NG * G; everything else is the head_dim-128 kernel — its 16-lane transpose-reduce minus the first stage,
 // probabilities broadcast per 8-lane half of a DPP row, the two halves' accumulators added before the rows meet.
-template <int G, int MODE, bool Q8, int WV = 4, int KVT = 0, int D = 128>
+// PART: one pass, and G query heads a workgroup instead of the KV head's whole group: ceil(g_real / G) workgroups share a (token, KV head).  Fewer heads are more rows a trip (a lane's 16 pairs are G
+// heads of 16 / G rows), and no records, so no combine launch behind it; what it costs is that each part reads the rows for itself.
+template <int G, int MODE, bool Q8, int WV = 4, int KVT = 0, int D = 128, bool PART = false>
 __global__ void __launch_bounds__(WV * 64) k_fattn_dec128(const tdesc q, const tdesc k, const tdesc v, const tdesc mask, const float * __restrict__ sinks,
-                                                      const tdesc dst, const fa_geom geo, float * __restrict__ ws, const int g_real,
+                                                      const tdesc dst, const fa_geom geo, float * __restrict__ ws, const int g_group,
                                                       const int * __restrict__ lists, const int list_stride) {
     constexpr bool SKIP = MODE == 1, LIST = MODE == 2;
     constexpr int LPR = D / 8, RPW = 64 / LPR, NG = LPR / G;  // lanes per K / V row, rows per wave-instruction, row groups per trip
@@ -435,7 +438,9 @@ __global__ void __launch_bounds__(WV * 64) k_fattn_dec128(const tdesc q, const t
     // (LIST: splits slowest — workgroups go to the XCDs in turn and in this order, and a token with few cells has trips in its first splits only, which come first and on all XCDs this way; with the
     // splits fastest, those of four splits shared two XCDs and of eight one: Llama-3-8B, us a step, 6 sequences of 130 cells in 8 splits 2587 -> 2540, 15 of 60 in 4 2815 -> 2775, a small model's 24 of
     // 400 1665 -> 1605.  Drafts of one sequence share its cells and gain nothing; 9 of 6000 3605 -> 3680)
-    const int split = LIST ? blockIdx.z : blockIdx.x, kvh = LIST ? blockIdx.x : blockIdx.y;
+    const int split = PART ? 0 : LIST ? blockIdx.z : blockIdx.x, kvh = LIST ? blockIdx.x : blockIdx.y;
+    const int part = PART ? (LIST ? (int) blockIdx.z : (int) blockIdx.x) : 0;
+    const int h0 = kvh * g_group + part * G, g_real = PART ? min(G, g_group - part * G) : g_group;  // the workgroup's first query head and how many it has
     // SKIP (a few query tokens, each seeing its own part of a unified cache): the workgroup first asks the mask whether its
     // token can see anything in its split — one 8-byte load per lane covers 256 positions — and leaves an empty record
     // if not: of the 64 x 32 (split, token) pairs of a -np 32 decode step only ~1/16 touch K/V at all
@@ -469,12 +474,17 @@ __global__ void __launch_bounds__(WV * 64) k_fattn_dec128(const tdesc q, const t
         if (ti >= ti1) {
             if (geo.n_splits == 1) {
                 // a token that sees nothing and no combine pass to say so: the CPU's result for such a row is 0 * (1 / 0) = NaN
+                if (PART && D == 64 && geo.q80) {
+                    for (int e = tid; e < g_real * (D / 32); e += WV * 64)
+                        *(float *) ((char *) geo.q80 + ((size_t) (tok >> 5) * (size_t) (geo.n_head * D / 32) + (size_t) (h0 * (D / 32) + e)) * 1152 + 1024 + (tok & 31) * 4) = __builtin_nanf("");
+                    return;
+                }
                 for (int e = tid; e < g_real * D; e += WV * 64) {
-                    float * out = (float *) (dst.data + (int64_t) (kvh * g_real + e / D) * dst.nb[1] + (int64_t) tok * dst.nb[2] + (int64_t) bat * dst.nb[3]);
+                    float * out = (float *) (dst.data + (int64_t) (h0 + e / D) * dst.nb[1] + (int64_t) tok * dst.nb[2] + (int64_t) bat * dst.nb[3]);
                     out[e % D] = __builtin_nanf("");
                 }
             } else if (tid < g_real) {
-                float * rec = ws + ((((int64_t) bat * geo.n_q + tok) * geo.n_head + kvh * g_real + tid) * geo.n_splits + split) * (D + 2);
+                float * rec = ws + ((((int64_t) bat * geo.n_q + tok) * geo.n_head + h0 + tid) * geo.n_splits + split) * (D + 2);
                 if (geo.arrive) { st_agent(rec + D, -INFINITY); st_agent(rec + D + 1, 0.0f); }
                 else { rec[D] = -INFINITY; rec[D + 1] = 0.0f; }
             }
@@ -497,7 +507,7 @@ __global__ void __launch_bounds__(WV * 64) k_fattn_dec128(const tdesc q, const t
         }
         if (!__any(any)) {  // every wave reaches the same verdict: no barrier has been passed yet
             if (tid < g_real) {
-                float * rec = ws + ((((int64_t) bat * geo.n_q + tok) * geo.n_head + kvh * g_real + tid) * geo.n_splits + split) * (D + 2);
+                float * rec = ws + ((((int64_t) bat * geo.n_q + tok) * geo.n_head + h0 + tid) * geo.n_splits + split) * (D + 2);
                 if (geo.arrive) { st_agent(rec + D, -INFINITY); st_agent(rec + D + 1, 0.0f); }
                 else { rec[D] = -INFINITY; rec[D + 1] = 0.0f; }
             }
@@ -575,7 +585,7 @@ __global__ void __launch_bounds__(WV * 64) k_fattn_dec128(const tdesc q, const t
     float qf[BF ? G : 1][8];  // bf16 cache: the query rounded to bf16, as f32
 #pragma unroll
     for (int g = 0; g < G; ++g) {
-        const int h = kvh * g_real + min(g, g_real - 1);
+        const int h = h0 + min(g, g_real - 1);
         const float4 * qp = (const float4 *) ((const float *) (q.data + (int64_t) tok * q.nb[1] + (int64_t) h * q.nb[2] + (int64_t) bat * q.nb[3]) + sl * 8);
         const float4 qa = qp[0], qb = qp[1];
         const float z = g < g_real ? 1.0f : 0.0f;
@@ -855,7 +865,7 @@ __global__ void __launch_bounds__(WV * 64) k_fattn_dec128(const tdesc q, const t
                 lt += sh[w][g][D + 1] * c;
             }
         }
-        const int h = kvh * g_real + g;
+        const int h = h0 + g;
         const float mt_e = mt * (1.0f / LOG2E);  // records and sinks use the natural-log domain of the generic kernel
         if (geo.n_splits == 1 && (!FAT || geo.rec_stride == D + 2)) {  // (the fat form always leaves records: its reader is the wo prologue, also for one split)
             if (sinks) {
@@ -866,7 +876,22 @@ __global__ void __launch_bounds__(WV * 64) k_fattn_dec128(const tdesc q, const t
                 lt = lt * c + expf(sk - mn);
             }
             if (!FAT && geo.q8) qv[g * D + dd] = a * (1.0f / lt);  // (quantised below, two heads per Q8_K block)
-            else {
+            else if constexpr (PART && LIST && D == 64) {
+                const float o = a * (1.0f / lt);
+                if (geo.q80) {  // a Q8_0 block = half a wave (e and D are multiples of 32 apart): k_quantize_q8_0's arithmetic, left in panel order
+                    float amax = fabsf(o);
+#pragma unroll
+                    for (int st = 1; st < 32; st <<= 1) amax = fmaxf(amax, __shfl_xor(amax, st, 64));
+                    const float d = amax / 127.0f, id = d != 0.0f ? 1.0f / d : 0.0f;
+                    const int e0 = h * D + dd, w = e0 & 31;
+                    char * tile = (char *) geo.q80 + ((size_t) (tok >> 5) * (size_t) (geo.n_head * D / 32) + (size_t) (e0 >> 5)) * 1152;
+                    tile[(w >> 4) * 512 + (tok & 31) * 16 + (w & 15)] = (char) (int8_t) (int) roundf(o * id);
+                    if (w == 0) *(float *) (tile + 1024 + (tok & 31) * 4) = h2f(f2h(d));
+                } else {
+                    float * out = (float *) (dst.data + (int64_t) h * dst.nb[1] + (int64_t) tok * dst.nb[2] + (int64_t) bat * dst.nb[3]);
+                    out[dd] = o;
+                }
+            } else {
                 float * out = (float *) (dst.data + (int64_t) h * dst.nb[1] + (int64_t) tok * dst.nb[2] + (int64_t) bat * dst.nb[3]);
                 out[dd] = a * (1.0f / lt);
             }
@@ -921,7 +946,7 @@ __global__ void __launch_bounds__(WV * 64) k_fattn_dec128(const tdesc q, const t
             if (wave < g_real / 2) {
                 const float4 t4 = ((const float4 *) (qv + wave * 256))[lane];
                 const float t[4] = {t4.x, t4.y, t4.z, t4.w};
-                wave_quantize_q8_K(t, lane, (q8k_dev *) geo.q8 + ((int64_t) bat * geo.n_q + tok) * (geo.n_head * D / 256) + (kvh * g_real) / 2 + wave);
+                wave_quantize_q8_K(t, lane, (q8k_dev *) geo.q8 + ((int64_t) bat * geo.n_q + tok) * (geo.n_head * D / 256) + h0 / 2 + wave);
             }
         }
         if constexpr (WV == 4)
@@ -1302,7 +1327,7 @@ bool fattn_q8_out_ok(const tdesc & q, const tdesc & k, const tdesc * mask, const
     return p.logit_softcap == 0.0f && p.max_bias == 0.0f && fa_g_ok(G) && (q.nb[1] % 16) == 0 && (q.nb[2] % 16) == 0 && ((uintptr_t) q.data & 15) == 0;
 }
 // the head_dim-64 forms that take p.lists (see launch_flash_attn)
-static bool dec64_applies(const tdesc & q, const tdesc & k, const tdesc & v, const fattn_params & p) {
+bool fattn_dec64_applies(const tdesc & q, const tdesc & k, const tdesc & v, const fattn_params & p) {
     static const bool on = !getenv("GGML_MI355X_FA_DEC64") || atoi(getenv("GGML_MI355X_FA_DEC64")) != 0;
     return on && k.ne[0] == 64 && k.type == GGML_TYPE_F16 && v.type == GGML_TYPE_F16 && (q.ne[1] == 1 || (p.lists && q.ne[3] == 1)) && p.logit_softcap == 0.0f && p.max_bias == 0.0f && fa_g_ok((int) (q.ne[2] / k.ne[2])) &&
            (q.nb[1] % 16) == 0 && (q.nb[2] % 16) == 0 && ((uintptr_t) q.data & 15) == 0 && (k.nb[1] % 16) == 0 && (v.nb[1] % 16) == 0 && (k.nb[2] % 16) == 0 && (v.nb[2] % 16) == 0 &&
@@ -1310,9 +1335,35 @@ static bool dec64_applies(const tdesc & q, const tdesc & k, const tdesc & v, con
 }
 // will launch_flash_attn end in the combine pass that leaves Q8_0 panel blocks? (mirrors its dispatch)
 bool fattn_q80_out_ok(const tdesc & q, const tdesc & k, const tdesc & v, const tdesc * mask, const float * sinks, const tdesc & dst, const fattn_params & p) {
-    if (k.ne[0] != 64 || k.ne[2] <= 0 || q.ne[2] % k.ne[2] != 0 || sinks || p.n_splits < 2 || p.n_splits > 8 || q.ne[3] != 1 || p.kv_type != GGML_TYPE_F16 || p.dq || p.fat) return false;
+    if (k.ne[0] != 64 || k.ne[2] <= 0 || q.ne[2] % k.ne[2] != 0 || sinks || p.n_splits < 1 || p.n_splits > 8 || q.ne[3] != 1 || p.kv_type != GGML_TYPE_F16 || p.dq || p.fat) return false;
+    if (p.n_splits == 1) return p.lists && p.head_pairs && fattn_dec64_applies(q, k, v, p);
     if (!p.lists && flash_attn_mma_applies(q, k, mask, sinks, dst, p)) return true;
-    return p.lists && dec64_applies(q, k, v, p);
+    return p.lists && fattn_dec64_applies(q, k, v, p);
+}
+// One pass over all cells instead of splits and a combine launch (4 us a layer)?  For pairs of query heads per workgroup (k_fattn_dec128: PART) where a token sees few cells: its rows are fetched once a
+// pair, 256 of them a trip on eight waves (128 on four), and a further trip costs what the lines below weigh against the launch saved.  us a step, splits + combine / one pass of pairs:
+//   one token, head_dim 64 (small model, 4 x 8 heads): 120 cells 916 / 800, 400 919 / 840, 1000 916 / 894, 1500 921 / 954 (whole groups in one pass: 923, 1035, 1280, 1527)
+//   one token, head_dim 128: Llama-3-8B 60 cells 1660 / 1563, 400 1662 / 1638, 700 1660 / 1702; Qwen2-7B (7 heads a group, whose splits run as 8) 100 1827 / 1675, 300 1823 / 1729, 600 1820 / 1784;
+//   Llama-3-8B over Q8_0 rows (four waves) 100 1745 / 1671, 300 1752 / 1810
+//   lists of n x cells, head_dim 64: 2 x 400 1115 / 1060, 2 x 900 1155 / 1127, 16 x 150 1209 / 1130, 16 x 500 1289 / 1222, 32 x 250 1542 / 1466; 9 drafts of 400 1308 / 1116
+//   lists, Llama-3-8B: 2 x 100 2453 / 2339, 2 x 450 2479 / 2510, 4 x 300 2513 / 2489, 8 x 350 2630 / 2566, 8 x 500 2641 / 2637, 16 x 400 2896 / 2839; Q8_0 rows 4 x 100 2542 / 2426, 4 x 300 2554 / 2582,
+//   16 x 200 2869 / 2779; 24 x 150 3208 / 3119 and 3063 as whole groups: from 128 (token, KV head) pairs on these fill the chip by themselves.
+// An odd group of heads does not leave whole Q8_K blocks (two heads of 128): its lists would trade the combine launch for a quantiser's.
+int fattn_one_pass(const tdesc & q, const tdesc & k, const fattn_params & p, bool list) {
+    const int64_t G = k.ne[2] > 0 ? q.ne[2] / k.ne[2] : 0, pairs = k.ne[2] * q.ne[1];
+    const bool q8 = p.kv_type == GGML_TYPE_Q8_0;
+    if (p.dq || p.fat || p.logit_softcap != 0.0f || p.max_bias != 0.0f || !fa_g_ok(G) || (q.nb[1] % 16) != 0 || (q.nb[2] % 16) != 0 || ((uintptr_t) q.data & 15) != 0 || (k.ne[0] != 64 && k.ne[0] != 128) ||
+        (k.ne[0] == 64 && q8) || q.ne[1] > 32)
+        return 0;
+    const int64_t cells = p.seen > 0 ? std::min<int64_t>(p.seen, k.ne[1]) : k.ne[1];
+    if (!list) {
+        if (q.ne[1] != 1) return 0;
+        return cells <= (k.ne[0] == 64 ? 1024 : q8 ? 256 : fa_gg(G) == 8 ? 768 : 512) ? 2 : 0;
+    }
+    if (k.ne[0] == 64) return cells <= (pairs * ((G + 1) / 2) <= 256 ? 1024 : 256) ? 2 : 0;
+    if (G & 1) return 0;
+    if (pairs > 128) return cells <= (q8 ? 256 : 384) ? 1 : 0;
+    return cells <= (q8 ? 256 : pairs >= 64 ? 512 : 384) ? 2 : 0;
 }
 void launch_flash_attn(hipStream_t s, const tdesc & q, const tdesc & k, const tdesc & v, const tdesc * mask, const float * sinks, const tdesc & dst,
                        const fattn_params & p, void * workspace) {
@@ -1392,6 +1443,7 @@ void launch_flash_attn(hipStream_t s, const tdesc & q, const tdesc & k, const td
         const bool merge2 = self_merge && !list && !skip && !q8 && !dq && p.q8_out == nullptr && geo.n_splits <= 32;
         const bool list8 = list_wv8 && list && !q8 && !dq && !p.arrive;
         const bool wide8 = wv8 && !q8 && !dq && !list && !skip && geo.n_q == 1 && geo.n_splits > 1 && (!p.arrive || merge2);
+        const int parts = p.head_pairs ? (G + 1) / 2 : 0;
 #define FA_DEC_T(GG, TT)                                                                                                                    \
     {                                                                                                                                       \
         if (list) hipLaunchKernelGGL((k_fattn_dec128<GG, 2, false, 4, TT>), grid, dim3(256), 0, s, q, k, v, mk, sinks, dst, geo, ws, G, p.lists, lstride);  \
@@ -1427,7 +1479,8 @@ void launch_flash_attn(hipStream_t s, const tdesc & q, const tdesc & k, const td
             const fa_geom geo0 = geo;
             float * const ws0 = ws;
             const int64_t nb_ = q0.ne[3];
-            const dim3 grid = list ? dim3((unsigned) geo0.n_kv_head, (unsigned) geo0.n_q, (unsigned) geo0.n_splits) : dim3((unsigned) geo0.n_splits, (unsigned) geo0.n_kv_head, (unsigned) geo0.n_q);
+            const unsigned inner = parts ? (unsigned) parts : (unsigned) geo0.n_splits;
+            const dim3 grid = list ? dim3((unsigned) geo0.n_kv_head, (unsigned) geo0.n_q, inner) : dim3(inner, (unsigned) geo0.n_kv_head, (unsigned) geo0.n_q);
             for (int64_t b = 0; b < nb_; ++b) {
                 tdesc q = q0, k = k0, v = v0, mk = mk0, dst = dst0;
                 fa_geom geo = geo0;
@@ -1440,7 +1493,12 @@ void launch_flash_attn(hipStream_t s, const tdesc & q, const tdesc & k, const td
                 float * ws = ws0 + (merge2 ? rows * geo0.n_kv_head * geo0.n_splits * G * FA_M2_REC : rows * geo0.n_head * geo0.n_splits * geo0.rec_stride);
                 if (geo.arrive) geo.arrive += rows * geo0.n_kv_head;
                 if (geo.q8) geo.q8 = (q8k_dev *) geo.q8 + rows * (geo0.n_head * 128 / 256);
-                if (fa_gg(G) == 2) FA_DEC(2) else if (fa_gg(G) == 4) FA_DEC(4) else FA_DEC(8)
+                if (parts) {
+                    if (list && q8) hipLaunchKernelGGL((k_fattn_dec128<2, 2, true, 4, 0, 128, true>), grid, dim3(256), 0, s, q, k, v, mk, sinks, dst, geo, ws, G, p.lists, lstride);
+                    else if (list) hipLaunchKernelGGL((k_fattn_dec128<2, 2, false, 4, 0, 128, true>), grid, dim3(256), 0, s, q, k, v, mk, sinks, dst, geo, ws, G, p.lists, lstride);
+                    else if (q8) hipLaunchKernelGGL((k_fattn_dec128<2, 0, true, 4, 0, 128, true>), grid, dim3(256), 0, s, q, k, v, mk, sinks, dst, geo, ws, G, nullptr, 0);
+                    else hipLaunchKernelGGL((k_fattn_dec128<2, 0, false, 8, 0, 128, true>), grid, dim3(512), 0, s, q, k, v, mk, sinks, dst, geo, ws, G, nullptr, 0);
+                } else if (fa_gg(G) == 2) FA_DEC(2) else if (fa_gg(G) == 4) FA_DEC(4) else FA_DEC(8)
             }
         }
 #undef FA_DEC
@@ -1458,14 +1516,17 @@ void launch_flash_attn(hipStream_t s, const tdesc & q, const tdesc & k, const td
     }
     // one decode token at head_dim 64 over an f16 cache (round 6): the lane-parallel kernel in its eight-lane-row form, records + combine pass
     // (generic kernel: 14.9 us per layer for TinyLlama at a 600-cell context; profiles/r06_secondary_kernel_stats.txt)
-    if (dec64_applies(q, k, v, p)) {
+    if (fattn_dec64_applies(q, k, v, p)) {
         geo.arrive = nullptr;
         geo.merge2 = 0;
         geo.q8 = nullptr;
         geo.per = (geo.n_kv + geo.n_splits - 1) / geo.n_splits;
         const tdesc q0 = q, k0 = k, v0 = v, mk0 = mk, dst0 = dst;
         const bool list = p.lists != nullptr;  // (2 .. 32 tokens of a -np decode step: each walks the list of its own visible cells, as at head_dim 128)
-        const dim3 grid = list ? dim3((unsigned) geo.n_kv_head, (unsigned) geo.n_q, (unsigned) geo.n_splits) : dim3((unsigned) geo.n_splits, (unsigned) geo.n_kv_head, (unsigned) geo.n_q);
+        const int parts = p.head_pairs ? (G + 1) / 2 : 0;
+        const unsigned inner = parts ? (unsigned) parts : (unsigned) geo.n_splits;
+        const dim3 grid = list ? dim3((unsigned) geo.n_kv_head, (unsigned) geo.n_q, inner) : dim3(inner, (unsigned) geo.n_kv_head, (unsigned) geo.n_q);
+        geo.q80 = parts && list ? p.q80_out : nullptr;
         const int lstride = geo.n_kv + 1;
         const bool wide = !list && geo.n_splits > 1;  // (eight waves: a trip covers 64 / 128 cells)
         for (int64_t b = 0; b < q0.ne[3]; ++b) {  // one launch per batch slice: the kernel has no batch arithmetic
@@ -1476,7 +1537,11 @@ void launch_flash_attn(hipStream_t s, const tdesc & q, const tdesc & k, const td
             if (mask) mb.data += (b % mk0.ne[3]) * mk0.nb[3];
             db.data += b * dst0.nb[3];
             float * wsb = ws + b * geo.n_head * geo.n_splits * geo.rec_stride;
-            if (list) {
+            if (parts) {
+                if (list && p.seen > 256) hipLaunchKernelGGL((k_fattn_dec128<2, 2, false, 8, 0, 64, true>), grid, dim3(512), 0, s, qb, kb, vb, mb, sinks, db, geo, wsb, G, p.lists, lstride);
+                else if (list) hipLaunchKernelGGL((k_fattn_dec128<2, 2, false, 4, 0, 64, true>), grid, dim3(256), 0, s, qb, kb, vb, mb, sinks, db, geo, wsb, G, p.lists, lstride);
+                else hipLaunchKernelGGL((k_fattn_dec128<2, 0, false, 8, 0, 64, true>), grid, dim3(512), 0, s, qb, kb, vb, mb, sinks, db, geo, wsb, G, nullptr, 0);
+            } else if (list) {
                 if (fa_gg(G) == 2) hipLaunchKernelGGL((k_fattn_dec128<2, 2, false, 4, 0, 64>), grid, dim3(256), 0, s, qb, kb, vb, mb, sinks, db, geo, wsb, G, p.lists, lstride);
                 else if (fa_gg(G) == 4) hipLaunchKernelGGL((k_fattn_dec128<4, 2, false, 4, 0, 64>), grid, dim3(256), 0, s, qb, kb, vb, mb, sinks, db, geo, wsb, G, p.lists, lstride);
                 else hipLaunchKernelGGL((k_fattn_dec128<8, 2, false, 4, 0, 64>), grid, dim3(256), 0, s, qb, kb, vb, mb, sinks, db, geo, wsb, G, p.lists, lstride);

@@ -466,8 +466,17 @@ static const void * mask_upload_ptr(const ggml_tensor * m) {
     }
     return m ? m->data : nullptr;
 }
+// the longest row of a mask, as the few steps that fattn_one_pass() tells apart: every step is a graph of its own (the hint is part of a graph's key)
+static constexpr int FA_SEEN[] = {256, 384, 512, 1024};
 static int fa_mask_hint(const ggml_tensor * n) {  // kernel choices that follow the CONTENT of the attention mask (common.h: mask_stats)
-    if (n->op == GGML_OP_FLASH_ATTN_EXT && n->src[3]) return n->src[0]->ne[1] >= 33 ? mask_sparse_hint(mask_upload_ptr(n->src[3])) : 0;
+    if (n->op == GGML_OP_FLASH_ATTN_EXT && n->src[3]) {
+        if (n->src[0]->ne[1] >= 33) return mask_sparse_hint(mask_upload_ptr(n->src[3]));
+        mask_stats ms;
+        if (n->src[0]->ne[1] < 2 || !lookup_mask_stats(mask_upload_ptr(n->src[3]), &ms)) return 0;
+        int step = 0;
+        while (step < 4 && ms.max_visible > FA_SEEN[step]) ++step;
+        return (step + 1) << 1;
+    }
     if (n->op == GGML_OP_SOFT_MAX && n->src[1] && n->src[0]->ne[1] >= 2 && n->src[0]->ne[1] <= 32) {
         mask_stats ms;
         return lookup_mask_stats(mask_upload_ptr(n->src[1]), &ms) ? (ms.max_visible > 1024 ? 2 : 1) : 0;
@@ -3651,7 +3660,9 @@ static int run_node(exec_state & st, int i) {
                 c->st.kv_image_nodes++;
             }
             const tdesc md0 = m ? TD(m) : qd;
-            p.mask_sparse = fa_mask_hint(n);
+            const int hint = fa_mask_hint(n);
+            p.mask_sparse = hint & 1;
+            p.seen = hint >> 1 == 0 ? 0 : hint >> 1 <= 4 ? FA_SEEN[(hint >> 1) - 1] : INT32_MAX;
             p.n_splits = std::min(64, c->opt.fa_splits > 0 ? c->opt.fa_splits : fattn_pick_splits(qd, kd, m ? &md0 : nullptr, p.mask_sparse));
             p.kv_type = (imaged || native_kv) ? (int) GGML_TYPE_F16 : (int) k->type;
             p.dq = native_kv ? 1 : 0;
@@ -3661,6 +3672,7 @@ static int run_node(exec_state & st, int i) {
             }
             const tdesc md = m ? TD(m) : qd;
             timed_scope ts(c, "flash_attn", (double) (k->ne[1] * k->ne[2] * k->ne[0] * 2 * 2));
+            int one_pass = a->ne[1] == 1 && a->ne[3] == 1 ? fattn_one_pass(qd, kd, p, false) : 0;
             if (c->fa_lists) {
                 const int tile = fattn_list_tile(qd, kd, m ? &md : nullptr, p, c->fa_lists_bytes);
                 if (tile > 0) {
@@ -3672,6 +3684,7 @@ static int run_node(exec_state & st, int i) {
                     }
                     p.lists = c->fa_lists;
                     c->st.fa_list_launches++;
+                    if (a->ne[1] <= 32) one_pass = fattn_one_pass(qd, kd, p, true);
                 } else if (m && a->ne[1] >= fattn_mma_min_q() && a->ne[3] == 1 && m->ne[3] == 1 && m->type == GGML_TYPE_F16 && (m->nb[1] % 8) == 0 && !(((uintptr_t) m->data) & 7) &&
                            (k->ne[1] % 4) == 0 && fattn_vis_bytes(qd, kd) <= c->fa_lists_bytes && flash_attn_mma_applies(qd, kd, &md, n->src[4] ? (const float *) n->src[4]->data : nullptr, TD(n), p)) {
                     // prompt batches on the matrix-core kernel: which (query tile, kv tile) pairs hold anything visible — once per graph run
@@ -3683,6 +3696,10 @@ static int run_node(exec_state & st, int i) {
                     }
                     p.tile_vis = (const uint8_t *) c->fa_lists;
                 }
+            }
+            if (one_pass && c->opt.fa_splits == 0 && (kd.ne[0] == 128 || fattn_dec64_applies(qd, kd, vd, p))) {
+                p.n_splits = 1;
+                p.head_pairs = one_pass == 2;
             }
             // one decode token whose attention result goes (through a reshape) straight into a quantised mat-vec — wo: few fat splits on
             // 8-wave workgroups, and the merge of their partial records is that mat-vec's prologue; the combine launch disappears

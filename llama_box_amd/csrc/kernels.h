@@ -383,6 +383,8 @@ struct fattn_params {
     unsigned * arrive = nullptr;  // zeroed counters (arrive_slots of them): lets the split kernel of the head_dim-128 decode path merge its own
     int arrive_slots = 0;         // partial records (last workgroup to arrive) instead of a second launch; the kernel leaves them at zero
     const uint8_t * tile_vis = nullptr;  // matrix-core kernel: [q tile of 32][kv tile of 64] visibility bytes (launch_fattn_vis_scan), or nullptr
+    int head_pairs = 0;   // 1: one pass (n_splits == 1), two query heads a workgroup: fattn_one_pass() said so
+    int seen = 0;         // cells the token that sees most can see, rounded up (graph.cpp: FA_SEEN), where the mask's content is known; else 0
     int mask_sparse = 0;  // 1: the mask's CONTENT is known (it passed through set_tensor, possibly behind the host's F32 -> F16 cast node) and at most a
                           // quarter of its cells are visible (common.h: mask_sparse_hint, resolved by graph.cpp) — position lists beat dense tiles
 };
@@ -406,6 +408,8 @@ int fattn_pick_splits(const tdesc & q, const tdesc & k, const tdesc * mask = nul
 // batches of many sequences over a unified cache, llama-box/httpserver.hpp:4042-4069) of up to 256 tokens walks per-token position lists instead
 bool fattn_prefers_lists(const tdesc & q, const tdesc * mask, int mask_sparse);
 int fattn_fat_splits(const tdesc & q, const tdesc & k, const tdesc * mask, const float * sinks, const fattn_params & p);  // 0 = the fat-split form does not apply
+bool fattn_dec64_applies(const tdesc & q, const tdesc & k, const tdesc & v, const fattn_params & p);  // the lane-parallel kernel at head_dim 64
+int fattn_one_pass(const tdesc & q, const tdesc & k, const fattn_params & p, bool list);  // instead of p.n_splits: 1: one pass of whole groups, 2: one pass of head pairs, 0: the splits
 bool fattn_q80_out_ok(const tdesc & q, const tdesc & k, const tdesc & v, const tdesc * mask, const float * sinks, const tdesc & dst, const fattn_params & p);
 bool fattn_q8_out_ok(const tdesc & q, const tdesc & k, const tdesc * mask, const float * sinks, const tdesc & dst, const fattn_params & p);  // will this launch end in the quantising combine?
 void launch_flash_attn(hipStream_t s, const tdesc & q, const tdesc & k, const tdesc & v, const tdesc * mask, const float * sinks,

@@ -319,6 +319,57 @@ def test_splits_of_few_tokens(backend, H, T_, n_kv, NH, NKV, HD, seen):
         assert np.abs(got[:, h] - ref).max() <= 2e-3 * np.abs(ref).max() + 1e-5, h
 
 
+# one pass over all cells, two heads of a key head a workgroup, at the lines between it and the splits; group sizes that leave a last pair in part, Q8_0 rows, sinks, tokens on lists
+@pytest.mark.parametrize("T_,n_kv,NH,NKV,HD,seen,q8,sinks,launches", [
+    (1, 1, 7, 1, 128, 0, False, False, 1), (1, 255, 14, 2, 128, 0, False, True, 1), (1, 768, 14, 2, 128, 0, False, False, 1), (1, 772, 14, 2, 128, 0, False, False, 2), (1, 512, 8, 2, 128, 0, False, False, 1),
+    (1, 513, 8, 2, 128, 0, False, False, 2), (1, 257, 5, 1, 128, 0, True, False, 2), (1, 256, 6, 2, 128, 0, True, True, 1), (1, 70, 3, 3, 64, 0, False, False, 1), (1, 1024, 32, 4, 64, 0, False, True, 1),
+    (1, 1025, 10, 2, 64, 0, False, False, 2), (2, 900, 8, 2, 128, 384, False, True, 2), (3, 900, 8, 2, 128, 385, False, False, 3), (17, 640, 16, 8, 128, 130, False, False, 2), (6, 500, 8, 2, 128, 256, True, False, 2),
+    (6, 500, 12, 2, 128, 257, True, False, 3), (4, 4096, 7, 1, 64, 1000, False, True, 2), (4, 4096, 8, 1, 64, 200, False, False, 2), (32, 640, 24, 8, 64, 256, False, False, 2), (32, 644, 24, 8, 64, 257, False, False, 2)])
+def test_one_pass_of_head_pairs(backend, H, T_, n_kv, NH, NKV, HD, seen, q8, sinks, launches):
+    """against float64 on the rows and queries as the kernel reads them (f16; Q8_0 rows: 8-bit queries); `launches`: the attention's own and the list scan's"""
+    rng = np.random.default_rng(T_ + n_kv + NH)
+    q = rng.standard_normal((NH, T_, HD)).astype(np.float32)
+    k, v = (rng.standard_normal((NKV, n_kv, HD)).astype(np.float32) for _ in range(2))
+    sk = rng.standard_normal(NH).astype(np.float32)
+    mask = np.full(((T_ + 63) // 64 * 64, n_kv), -np.inf, np.float16)
+    for t in range(T_):
+        if seen:
+            mask[t, rng.choice(n_kv, seen, replace=False)] = 0
+        else:
+            mask[t, : n_kv - T_ + t + 1] = 0
+    if q8:
+        def blocks(x):  # (bytes, values) of Q8_0 blocks
+            b = x.reshape(-1, 32)
+            d = (np.abs(b).max(1, keepdims=True) / 127).astype(np.float32)
+            i = np.rint(b / d).astype(np.int8)
+            return np.concatenate([d.astype(np.float16).view(np.uint8), i.view(np.uint8)], 1), (d.astype(np.float16).astype(np.float32) * i).reshape(x.shape)
+
+        (kr, k), (vr, v), (_, qx) = blocks(k), blocks(v), blocks(q)
+    else:
+        kr, vr = (x.astype(np.float16) for x in (k, v))
+        k, v, qx = kr, vr, q.astype(np.float16)
+
+    def build(g):
+        kt = L.Q8_0 if q8 else L.F16
+        a = H.ggml_flash_attn_ext(g.ctx, g.new(L.F32, [HD, T_, NH], q), g.new(kt, [HD, n_kv, NKV], kr), g.new(kt, [HD, n_kv, NKV], vr),
+                                  H.ggml_cast(g.ctx, g.new(L.F32, [n_kv, mask.shape[0]], mask.astype(np.float32), "KQ_mask"), L.F16), HD ** -0.5, 0.0, 0.0)
+        H.ggml_flash_attn_ext_set_prec(a, 10)
+        if sinks:
+            H.ggml_flash_attn_ext_add_sinks(a, g.new(L.F32, [NH], sk))
+        return a
+
+    n0 = backend.stat("kernel_launches")
+    got = T.run_case(build, backend)[0].reshape(T_, NH, HD)
+    assert backend.stat("kernel_launches") - n0 == launches + 1  # (the mask's conversion)
+    for h in range(NH):
+        z = qx[h].astype(np.float64) @ k[h // (NH // NKV)].astype(np.float64).T * HD ** -0.5 + mask[:T_].astype(np.float64)
+        m = np.maximum(z.max(1, keepdims=True), sk[h] if sinks else -np.inf)
+        p = np.exp(z - m)
+        ref = (p / (p.sum(1, keepdims=True) + (np.exp(sk[h] - m) if sinks else 0.0))) @ v[h // (NH // NKV)].astype(np.float64)
+        # (f32 sums and probabilities: 2^-11 of headroom over the query's own rounding, whose f16 scale a Q8_0 block holds)
+        assert np.abs(got[:, h] - ref).max() <= 1e-3 * np.abs(ref).max() + 1e-5, h
+
+
 # trips of 512 cells with eight waves (16, 32 and 64 rows of V^T a workgroup) and of 256 with four, the last tile and the last trip in part, waves without a tile; whole rows from 80 pairs of
 # a token and a key head and 64 cells a token on (their 256- and 512-cell limits on both sides)
 @pytest.mark.parametrize("T_,NKV,G,per", [
