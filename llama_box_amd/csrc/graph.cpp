@@ -2360,6 +2360,83 @@ static int try_fuse_qk_norm_store(exec_state & st, int i) {
     return k - i;
 }
 
+static void rope_params_of(const ggml_tensor * n, rope_params & p) {
+    p.n_dims = n->op_params[1]; p.mode = n->op_params[2]; p.n_ctx_orig = n->op_params[4];
+    p.freq_base = ggml_abi_op_param_f32(n, 5); p.freq_scale = ggml_abi_op_param_f32(n, 6); p.ext_factor = ggml_abi_op_param_f32(n, 7);
+    p.attn_factor = ggml_abi_op_param_f32(n, 8); p.beta_fast = ggml_abi_op_param_f32(n, 9); p.beta_slow = ggml_abi_op_param_f32(n, 10);
+    memcpy(p.sections, n->op_params + 11, sizeof(p.sections));
+    p.exact_freq = rope_exact_freq(n);
+}
+// ROPE(q), ROPE(k), [SCALE(v, a), SCALE(y, b), ADD,] SET_ROWS(k), SET_ROWS(v) (views and finished nodes between them skipped): one launch.  Returns the nodes consumed (0: no match)
+static int try_fuse_rope_rows(exec_state & st, int i) {
+    ggml_cgraph * g = st.g;
+    const ggml_tensor * rq = g->nodes[i];
+    int k = i + 1;
+    auto take = [&]() -> const ggml_tensor * {  // the next node with work left
+        while (k < g->n_nodes && (st.done[k] || is_view_op(g->nodes[k]))) ++k;
+        return k < g->n_nodes ? g->nodes[k++] : nullptr;
+    };
+    const ggml_tensor * rk = take();
+    if (!rk || rk->op != GGML_OP_ROPE || rq->src[2] || rk->src[2] || (rq->op_params[2] & GGML_ROPE_TYPE_MROPE) || memcmp(rq->op_params, rk->op_params, sizeof(rq->op_params)) != 0 || rq->src[1] != rk->src[1])
+        return 0;
+    const ggml_tensor * n1 = take(), * s1 = nullptr, * s2 = nullptr, * ad = nullptr;
+    if (n1 && n1->op == GGML_OP_SCALE) {
+        s1 = n1; s2 = take(); ad = take();
+        if (!s2 || !ad || s2->op != GGML_OP_SCALE || ad->op != GGML_OP_ADD || !((ad->src[0] == s1 && ad->src[1] == s2) || (ad->src[0] == s2 && ad->src[1] == s1)) || !single_use(st, s1) || !single_use(st, s2) ||
+            ggml_abi_op_param_f32(s1, 1) != 0.0f || ggml_abi_op_param_f32(s2, 1) != 0.0f || !same_shape(s1, s2) || !same_shape(s1, ad) || !is_f32_contig(s1->src[0]) || !is_f32_contig(s2->src[0]) ||
+            !is_f32_contig(ad) || ad->ne[2] != 1 || ad->ne[3] != 1)
+            return 0;
+        if (ad->src[0] != s1) std::swap(s1, s2);
+        n1 = take();
+    }
+    const ggml_tensor * sk = n1, * sv = take();
+    if (!sk || !sv || sk->op != GGML_OP_SET_ROWS || sv->op != GGML_OP_SET_ROWS) return 0;
+    const ggml_tensor * q = rq->src[0], * kx = rk->src[0], * v = sv->src[0], * idx = sk->src[1], * pos = rq->src[1];
+    const int64_t DK = q->ne[0], T = q->ne[2];
+    auto heads_ok = [&](const ggml_tensor * t) { return t->type == GGML_TYPE_F32 && t->nb[0] == 4 && (t->nb[1] % 4) == 0 && (t->nb[2] % 4) == 0 && t->ne[0] == DK && t->ne[2] == T && t->ne[3] == 1; };
+    if (!heads_ok(q) || !heads_ok(kx) || !is_f32_contig(rq) || !is_f32_contig(rk) || pos->type != GGML_TYPE_I32 || ggml_abi_nelements(pos) != T || rq->op_params[1] <= 0 || rq->op_params[1] > DK) return 0;
+    // the rotated keys and the blended values live in the cache alone
+    auto only_stored = [&](const ggml_tensor * t, const ggml_tensor * at) {  // `at`: t, seen through views
+        if (through_views(at) != t || use_count(st, t) != 1 || (t->flags & GGML_TENSOR_FLAG_OUTPUT)) return false;
+        for (const ggml_tensor * u = at; u != t; u = u->src[0])
+            if (!single_use(st, u)) return false;
+        return true;
+    };
+    if (!only_stored(rk, sk->src[0]) || (ad ? !only_stored(ad, v) : v->type != GGML_TYPE_F32 || v->nb[0] != 4 || (v->nb[1] % 4) != 0 || through_views(v) == rk || through_views(v) == rq)) return 0;
+    const int64_t row_v = sv->ne[0];
+    auto cache_ok = [&](const ggml_tensor * t, const ggml_tensor * src, int64_t n) {
+        return (t->type == GGML_TYPE_F32 || t->type == GGML_TYPE_BF16 || t->type == GGML_TYPE_F16) && t->nb[0] == ggml_abi_type_size(t->type) && t->ne[0] == n && t->ne[2] == 1 && t->ne[3] == 1 && src->ne[0] == n &&
+               src->ne[1] == T && src->ne[2] == 1 && src->ne[3] == 1;
+    };
+    if (!cache_ok(sk, sk->src[0], DK * kx->ne[1]) || !cache_ok(sv, v, row_v) || (ad && !ggml_abi_is_contiguous(v)) || idx != sv->src[1] || idx->type != GGML_TYPE_I64 || !ggml_abi_is_contiguous(idx) ||
+        ggml_abi_nelements(idx) != T || idx->op != GGML_OP_NONE)
+        return 0;
+    // (every wave reads its own head before it writes: the queries' result may be the projection's own block, nothing else that the launch reads)
+    const ggml_tensor * va = ad ? s1->src[0] : v, * vy = ad ? s2->src[0] : nullptr;
+    if (!(is_f32_contig(q) ? elementwise_safe(rq, q) : !ranges_overlap(rq, q))) return 0;
+    for (const ggml_tensor * t : {kx, va, vy, pos, idx})
+        if (t && ranges_overlap(rq, t)) return 0;
+    if (ranges_overlap(sk, sv)) return 0;
+    for (const ggml_tensor * c : {sk, sv})
+        for (const ggml_tensor * t : {q, kx, va, vy, pos, idx, rq})
+            if (t && ranges_overlap(c, t)) return 0;
+    rope_rows_args a{};
+    a.q = (const float *) q->data; a.qd = (float *) rq->data; a.k = (const float *) kx->data; a.v = (const float *) va->data; a.y = vy ? (const float *) vy->data : nullptr;
+    a.q_head = (int64_t) q->nb[1] / 4; a.q_tok = (int64_t) q->nb[2] / 4; a.k_head = (int64_t) kx->nb[1] / 4; a.k_tok = (int64_t) kx->nb[2] / 4;
+    a.v_tok = ad ? row_v : (int64_t) v->nb[1] / 4; a.y_tok = row_v;
+    if (ad) { a.va = ggml_abi_op_param_f32(s1, 0); a.vb = ggml_abi_op_param_f32(s2, 0); }
+    a.pos = (const char *) pos->data; a.pos_nb = (int64_t) pos->nb[0];
+    a.idx = (const int64_t *) idx->data;
+    a.k_cache = (char *) sk->data; a.v_cache = (char *) sv->data; a.kc_nb1 = (int64_t) sk->nb[1]; a.vc_nb1 = (int64_t) sv->nb[1];
+    a.H = (int) q->ne[1]; a.G = (int) kx->ne[1]; a.DK = (int) DK; a.NV = (int) row_v; a.k_type = sk->type; a.v_type = sv->type;
+    rope_params_of(rq, a.p);
+    timed_scope ts(st.c, "rope_rows", (double) (ggml_abi_nbytes(rq) * 2 + ggml_abi_nelements(kx) * 4 + row_v * T * 4));
+    launch_rope_rows(st.c->stream, a, T);
+    st.c->st.kernel_launches++;
+    st.c->st.fused_nodes += ad ? 6 : 3;
+    return k - i;
+}
+
 // [ADD(x, bias row) ->] SSM_CONV -> SSM_CONV (store) of one input: the bias goes into the loads of both; a batch of one token per sequence is ONE launch (a thread has read its channel's
 // history before it writes it).  Returns the nodes consumed at position i (0: no match)
 static int try_fuse_conv_store(exec_state & st, int i) {
@@ -3307,7 +3384,8 @@ static int run_node(exec_state & st, int i) {
                             same_shape(m2, ad) && !(ad->flags & GGML_TENSOR_FLAG_OUTPUT)) {
                             const ggml_tensor * w2 = m2->src[0] == n2 ? m2->src[1] : (m2->src[1] == n2 ? m2->src[0] : nullptr);
                             if (w2 && w2->type == GGML_TYPE_F32 && ggml_abi_is_contiguous(w2) && w2->ne[0] == n->ne[0] && ggml_abi_nelements(w2) == w2->ne[0] && !ranges_overlap(m2, ad) &&
-                                !(ranges_overlap(m2, a) && m2->data != a->data) && !ranges_overlap(m2, res)) {  // (a row's second output is written after the last read of that row of `a`: the allocator may hand `a`'s block to it)
+                                !(ranges_overlap(m2, a) && m2->data != a->data) && (!ranges_overlap(m2, res) || (m2->data == res->data && is_f32_contig(res) && is_f32_contig(m2)))) {
+                                // (a row's second output is written after the last read of that row of `a` and of the residual: the allocator may hand either's block to it)
                                 timed_scope ts(c, "layer_norm_mul_add_norm_mul", (double) ggml_abi_nbytes(a) * 4);
                                 const ggml_tensor * b16 = nullptr;
                                 const copy16 o16 = copy_16_for(st, i + 4, m2, &b16);
@@ -3578,16 +3656,16 @@ static int run_node(exec_state & st, int i) {
             }
             if (fuse && try_fuse_rope_store(st, i)) return 1;
             static const bool row_stores = !getenv("GGML_MI355X_ROW_STORES") || atoi(getenv("GGML_MI355X_ROW_STORES")) != 0;
+            if (fuse && row_stores) {
+                const int r = try_fuse_rope_rows(st, i);
+                if (r > 0) return r;
+            }
             if (fuse && row_stores && n->type == GGML_TYPE_F32 && a->type == GGML_TYPE_F32 && a->nb[0] == 4 && !(n->op_params[2] & GGML_ROPE_TYPE_MROPE) && !n->src[2] && n->ne[3] == 1 &&
                 ggml_abi_is_contiguous(n) && b->type == GGML_TYPE_I32) {
                 const int ks = sole_cache_store_of(st, i, n, n->ne[2]);
                 if (ks >= 0) {  // rope(k) lives only in the cache: rotate straight into the cache rows
                     rope_params p;
-                    p.n_dims = n->op_params[1]; p.mode = n->op_params[2]; p.n_ctx_orig = n->op_params[4];
-                    p.freq_base = ggml_abi_op_param_f32(n, 5); p.freq_scale = ggml_abi_op_param_f32(n, 6); p.ext_factor = ggml_abi_op_param_f32(n, 7);
-                    p.attn_factor = ggml_abi_op_param_f32(n, 8); p.beta_fast = ggml_abi_op_param_f32(n, 9); p.beta_slow = ggml_abi_op_param_f32(n, 10);
-                    memset(p.sections, 0, sizeof(p.sections));
-                    p.exact_freq = rope_exact_freq(n);
+                    rope_params_of(n, p);
                     const ggml_tensor * sr = g->nodes[ks];
                     timed_scope ts(c, "rope_store_rows", (double) ggml_abi_nbytes(n) * 2);
                     launch_rope_store(s, TD(a), TD(b), nullptr, (const int64_t *) sr->src[1]->data, TD(sr), p);
@@ -3598,17 +3676,7 @@ static int run_node(exec_state & st, int i) {
                 }
             }
             rope_params p;
-            p.n_dims = n->op_params[1];
-            p.mode = n->op_params[2];
-            p.n_ctx_orig = n->op_params[4];
-            p.freq_base = ggml_abi_op_param_f32(n, 5);
-            p.freq_scale = ggml_abi_op_param_f32(n, 6);
-            p.ext_factor = ggml_abi_op_param_f32(n, 7);
-            p.attn_factor = ggml_abi_op_param_f32(n, 8);
-            p.beta_fast = ggml_abi_op_param_f32(n, 9);
-            p.beta_slow = ggml_abi_op_param_f32(n, 10);
-            memcpy(p.sections, n->op_params + 11, sizeof(p.sections));
-            p.exact_freq = rope_exact_freq(n);
+            rope_params_of(n, p);
             timed_scope ts(c, "rope", (double) ggml_abi_nbytes(n) * 2);
             launch_rope(s, TD(a), TD(b), n->src[2] ? (const float *) n->src[2]->data : nullptr, TD(n), p);
             c->st.kernel_launches++;

@@ -364,6 +364,20 @@ void launch_rope_qk_store_vec(hipStream_t s, const rope_store_args & a, int n_to
 void launch_rope(hipStream_t s, const tdesc & src, const tdesc & pos, const float * freq_factors, const tdesc & dst, const rope_params & p);
 // ROPE (no frequency factors) + SET_ROWS into a cache kept in f32 / f16 / bf16, and a x + b y + SET_ROWS: the value goes straight into cache row idx[t]
 void launch_rope_store(hipStream_t s, const tdesc & src /* [D, heads, T] f32 */, const tdesc & pos, const float * freq /* exact_freq == 2 */, const int64_t * idx, const tdesc & cache, const rope_params & p);
+// ROPE(q), ROPE(k) -> SET_ROWS, v (or a v + b y) -> SET_ROWS: rotated queries to qd, keys and values into row idx[t] of their caches (f32 / f16 / bf16)
+struct rope_rows_args {
+    const float * q; float * qd; const float * k; const float * v; const float * y;  // qd [DK, H, T] contiguous; y: null, or as v
+    int64_t q_head, q_tok, k_head, k_tok, v_tok, y_tok;                              // floats from a head / a token to the next
+    float va, vb;
+    const char * pos; int64_t pos_nb;
+    const int64_t * idx;
+    char * k_cache; char * v_cache;
+    int64_t kc_nb1, vc_nb1;
+    int H, G, DK, NV, k_type, v_type;  // NV: values of a token
+    rope_params p;
+    float theta_scale, corr0, corr1;
+};
+void launch_rope_rows(hipStream_t s, rope_rows_args a, int64_t n_tok);
 void launch_axpby_store(hipStream_t s, const float * x, float a, const float * y, float b, int64_t n, int64_t n_tok, const int64_t * idx, const tdesc & cache);
 void launch_soft_max(hipStream_t s, const tdesc & src, const tdesc * mask, const float * sinks, const tdesc & dst, float scale, float max_bias);
 

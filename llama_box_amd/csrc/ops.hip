@@ -1972,6 +1972,73 @@ void launch_rope_store(hipStream_t s, const tdesc & a, const tdesc & pos, const 
     if (many) hipLaunchKernelGGL(k_rope_heads_store, grid, dim3(256), 0, s, a, pos, ff, idx, cache.data, cache.nb[1], cache.type, p, theta_scale, c0, c1);
     else hipLaunchKernelGGL(k_rope_store, grid, dim3(64), 0, s, a, pos, ff, idx, cache.data, cache.nb[1], cache.type, p, theta_scale, c0, c1);
 }
+// Queries, keys and values of a step between their projection and the attention, in one launch where there were three (four with a blend): such launches cost 4 us each whatever they hold, and the
+// queries and keys of a token share their angles.  The element formulas are k_rope's, k_rope_store's and k_axpby_store's.  A wave a head, and one for 256 values, while the chip holds them; else groups of
+// four waves a token (rope_many).  us: 16 + 4 heads of 128, 64 rotated, 2 tokens 13.3 (three launches) -> 4.6; 32 + 8 heads, 512 tokens 21.5 -> 11.9.
+__device__ __forceinline__ void rope_rows_values(const rope_rows_args & A, const int64_t t, const int i0, const int end, const int step) {
+    char * __restrict__ row = A.v_cache + A.idx[t] * A.vc_nb1;
+    const float * __restrict__ v = A.v + t * A.v_tok;
+    const float * __restrict__ y = A.y ? A.y + t * A.y_tok : nullptr;
+    for (int i = i0; i < end; i += 4 * step) {
+        float x[4], w[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int ik = min(i + k * step, end - 1);
+            x[k] = v[ik];
+            w[k] = y ? y[ik] : 0.0f;
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            float o = x[k];
+            if (y) {
+                const float pp = x[k] * A.va, q = w[k] * A.vb;
+                o = pp + q;
+            }
+            if (i + k * step < end) store_as(row, A.v_type, i + k * step, o);
+        }
+    }
+}
+__global__ void __launch_bounds__(64) k_rope_rows(const rope_rows_args A) {
+    const int h = blockIdx.x;
+    const int64_t t = blockIdx.y;
+    if (h >= A.H + A.G) {
+        const int i0 = (h - A.H - A.G) * 256 + (int) threadIdx.x;  // (256 values: one trip)
+        rope_rows_values(A, t, i0, min(A.NV, (h - A.H - A.G + 1) * 256), 64);
+        return;
+    }
+    const float pos_f = (float) *(const int32_t *) (A.pos + t * A.pos_nb);
+    const bool key = h >= A.H;
+    const float * src = key ? A.k + (h - A.H) * A.k_head + t * A.k_tok : A.q + h * A.q_head + t * A.q_tok;
+    float * qd = A.qd + (t * A.H + h) * A.DK;
+    char * row = key ? A.k_cache + A.idx[t] * A.kc_nb1 : nullptr;
+    const int64_t base = (int64_t) (h - A.H) * A.DK;
+    rope_heads(A.p, pos_f, nullptr, rope_consts{A.theta_scale, A.p.freq_scale, A.p.ext_factor, A.p.attn_factor, A.corr0, A.corr1}, A.DK, 1, 0, 1, [&](const int, const int i) { return src[i]; },
+               [&](const int, const int i, const float v) {
+                   if (key) store_as(row, A.k_type, base + i, v);
+                   else qd[i] = v;
+               });
+}
+__global__ void __launch_bounds__(256) k_rope_rows_many(const rope_rows_args A) {
+    const int64_t t = blockIdx.y;
+    const int wv = (int) (blockIdx.x * 4 + (threadIdx.x >> 6)), nw = (int) gridDim.x * 4;
+    const float pos_f = (float) *(const int32_t *) (A.pos + t * A.pos_nb);
+    const float * q = A.q + t * A.q_tok, * k = A.k + t * A.k_tok;
+    float * qd = A.qd + t * A.H * A.DK;
+    char * row = A.k_cache + A.idx[t] * A.kc_nb1;
+    rope_heads(A.p, pos_f, nullptr, rope_consts{A.theta_scale, A.p.freq_scale, A.p.ext_factor, A.p.attn_factor, A.corr0, A.corr1}, A.DK, A.H + A.G, wv, nw,
+               [&](const int h, const int i) { return h < A.H ? q[h * A.q_head + i] : k[(h - A.H) * A.k_head + i]; },
+               [&](const int h, const int i, const float v) {
+                   if (h < A.H) qd[h * A.DK + i] = v;
+                   else store_as(row, A.k_type, (int64_t) (h - A.H) * A.DK + i, v);
+               });
+    rope_rows_values(A, t, (int) (blockIdx.x * 256 + threadIdx.x), A.NV, (int) gridDim.x * 256);
+}
+void launch_rope_rows(hipStream_t s, rope_rows_args a, int64_t n_tok) {
+    if (n_tok == 0) return;
+    rope_host_consts(a.p, a.theta_scale, a.corr0, a.corr1);
+    if (rope_many(a.H + a.G, n_tok, false)) hipLaunchKernelGGL(k_rope_rows_many, dim3(rope_groups(a.H + a.G, n_tok), (unsigned) n_tok), dim3(256), 0, s, a);
+    else hipLaunchKernelGGL(k_rope_rows, dim3((unsigned) (a.H + a.G + (a.NV + 255) / 256), (unsigned) n_tok), dim3(64), 0, s, a);
+}
 // ------------------------------------------------------------------------------------------------ fused steps of models with token shift / latent attention
 // (each one the arithmetic of the unfused nodes it replaces, operation by operation: fused and unfused graphs agree bit for bit)
 // token shift: out[t] = h[t] + (prev - h[t]) * w, prev = row src[t] of [h rows | state rows] (CONCAT dim 1 -> GET_ROWS -> SUB -> MUL -> ADD)

@@ -425,6 +425,7 @@ struct llm_layer_cfg {
     bool no_pre_norm = false;                       // the sublayers read the stream itself (their outputs are normed: attn_post_norm, ffn_post_norm)
     bool ffn_silu_gated = false;                    // dense feed-forward W_down (silu(W_gate h) * W_up h)
     bool qkv_first = false;                         // the projections precede the per-head steps in the graph's order (which the backend then runs as one launch)
+    bool gate_first = false;                        // ... the output gate's among them
     bool rot_table = false;                         // rotation by a table of frequencies (rope_freq), cos and sin times rope_magnitude
     float band_factor = 0.0f, band_low = 1.0f, band_high = 1.0f, band_orig = 0.0f;  // band_factor > 0: frequencies divided by it, kept or blended by their wavelength
     bool qk_unit = false;                           // BEHIND the rotation every head's query and key is divided by its root mean square (no weight)
@@ -936,6 +937,7 @@ static bool parse_nigozen_config(const json_value & cfg, llm_model * m, std::str
         c.v_mix = num(mx, "v_mix", nullptr, 0) != 0;
         c.sink = true;      // the design's soft-max always carries the sink ...
         c.out_gate = true;  // ... and its heads always pass the sigmoid gate
+        c.qkv_first = c.gate_first = true;
         if (c.n_head <= 0 || c.n_head_kv <= 0 || c.n_head % c.n_head_kv || c.dk <= 0 || c.dv <= 0 || c.rot_dims < 0 || c.rot_dims > c.dk || (c.rot_dims & 1) || c.chunk < 0) {
             err = "config: layer " + std::to_string(il) + ": inconsistent attention sizes";
             return false;
@@ -2592,6 +2594,9 @@ static ggml_tensor * build_moe(ggml_context * ctx, ggml_cgraph * gf, const llm_l
     ggml_tensor * sel = named(ggml_top_k(ctx, logits, c.n_top), "ffn_moe_topk", il);            // [n_top, T] i32
     ggml_tensor * w = ggml_get_rows(ctx, ggml_reshape_3d(ctx, logits, 1, c.n_expert, T), sel);   // [1, n_top, T]
     w = named(ggml_soft_max(ctx, ggml_reshape_2d(ctx, named(w, "ffn_moe_sel_logits", il), c.n_top, T)), "ffn_moe_weights", il);  // soft-max over the chosen logits only
+    // (router and soft-max in front of the experts, and the weights' block given to nothing else: the backend runs the first as one launch and reads the weights in the launch that writes the sum)
+    ggml_set_output(w);
+    ggml_build_forward_expand(gf, w);
     ggml_tensor * up = named(ggml_mul_mat_id(ctx, L.ffn_up_exps, ggml_reshape_3d(ctx, cur, E, 1, T), sel), "ffn_moe_up", il);     // [n_ff, n_top, T]
     ggml_tensor * act = named(ggml_sqr(ctx, named(ggml_unary(ctx, up, GGML_UNARY_OP_RELU), "ffn_moe_relu", il)), "ffn_moe_act", il);
     ggml_tensor * down = named(ggml_mul_mat_id(ctx, L.ffn_down_exps, act, sel), "ffn_moe_down", il);                              // [E, n_top, T]
@@ -2675,7 +2680,7 @@ static ggml_tensor * build_mixer_attention(llm_context * c, ggml_context * ctx, 
                 ggml_build_forward_expand(gf, Kcur);
                 ggml_build_forward_expand(gf, Vcur);
             }
-            if (gate && lc.no_pre_norm) ggml_build_forward_expand(gf, gate);
+            if (gate && (lc.no_pre_norm || lc.gate_first)) ggml_build_forward_expand(gf, gate);
         }
         Qcur = ggml_reshape_3d(ctx, Qcur, DK, H, n_tokens);
         if (own_kv) Kcur = ggml_reshape_3d(ctx, Kcur, DK, G, n_tokens);

@@ -327,6 +327,27 @@ def test_layer_norm_two_stages_at_the_edges_of_its_pieces(backend, H, n):
     assert np.abs(got - R.layer_norm(s, w2.astype(np.float64), 1e-6)).max() <= 2e-5
 
 
+# the second stage's rows in the block that the residual is read from: still one launch
+@pytest.mark.parametrize("n", [260, 1027, 4096, 4100])
+def test_layer_norm_two_stages_over_the_residual(backend, H, n):
+    rng = np.random.default_rng(n)
+    rows = 3
+    x, r = ((rng.standard_normal((rows, n)) * 3 + 1.5).astype(np.float32) for _ in range(2))
+    w, w2 = (rng.standard_normal(n).astype(np.float32) for _ in range(2))
+    g = T.G(backend)
+    try:
+        res = g.new(L.F32, [n, rows], r)
+        s = H.ggml_add(g.ctx, H.ggml_mul(g.ctx, H.ggml_norm(g.ctx, g.new(L.F32, [n, rows], x), 1e-5), g.new(L.F32, [n], w)), res)
+        out = H.ggml_mul(g.ctx, H.ggml_norm(g.ctx, s, 1e-6), g.new(L.F32, [n], w2))
+        n0 = backend.stat("kernel_launches")
+        got = g.compute([out], same_block=[(out, res)])[0].reshape(rows, n)
+        assert backend.stat("kernel_launches") == n0 + 1
+    finally:
+        g.free()
+    ref = R.layer_norm(R.layer_norm(x.astype(np.float64), w.astype(np.float64), 1e-5) + r, w2.astype(np.float64), 1e-6)
+    assert np.abs(got - ref).max() <= 2e-5  # (as above)
+
+
 # rows of up to 4096 values that start at no multiple of 16 bytes, or whose weights do (single values a thread, 4, 8 or 16 of them)
 @pytest.mark.parametrize("n", [1, 63, 256, 1024, 1025, 2048, 2049, 4095, 4096])
 @pytest.mark.parametrize("shifted", ["rows", "weight"])
@@ -517,3 +538,54 @@ def test_random_configurations(backend, tmp_path, seed):
     if got2:
         assert row_err(np.concatenate(got2), ref2[:at2]).max() <= F32_GATE
     s.close()
+
+
+# rotated queries, keys and (blended) values of a step in one launch: a wave a head, or groups of waves a token from 4096 heads x tokens on; rotated parts of a head, f32 / f16 / bf16 caches, queries in place or not
+@pytest.mark.parametrize("T_,NH,NKV,D,rot,mode,exact,blend,kt,vt,launches", [
+    (1, 16, 4, 128, 64, 0, 1, True, L.BF16, L.BF16, 1), (2, 5, 1, 96, 96, 2, 0, False, L.F32, L.BF16, 1), (7, 3, 3, 80, 22, 0, 0, True, L.F16, L.F32, 1), (130, 32, 8, 128, 64, 0, 1, True, L.BF16, L.BF16, 1),
+    (515, 9, 3, 72, 40, 2, 1, False, L.BF16, L.BF16, 1), (203, 20, 4, 64, 64, 0, 0, True, L.F32, L.F16, 1)])
+def test_rows_of_a_step_in_one_launch(backend, H, T_, NH, NKV, D, rot, mode, exact, blend, kt, vt, launches):
+    rng = np.random.default_rng(T_ + NH)
+    q, k, v, y = (rng.standard_normal((T_, n * D)).astype(np.float32) for n in (NH, NKV, NKV, NKV))
+    idx = rng.permutation(T_ + 40)[:T_].astype(np.int64)
+    pos = rng.integers(0, 3000, T_).astype(np.int32)
+
+    def build(g):
+        p, rows = g.new(L.I32, [T_], pos), g.new(L.I64, [T_], idx)
+        caches = [g.new(t, [NKV * D, T_ + 40], np.zeros((T_ + 40, NKV * D), np.float32 if t == L.F32 else np.float16)) for t in (kt, vt)]
+
+        def rope(x):
+            r = H.ggml_rope_ext(g.ctx, x, p, None, rot, mode, 4096, 10000.0, 1.0, 0.0, 1.0, 32.0, 1.0)
+            if exact:
+                r.contents.op_params[3] = 1
+            return r
+
+        tq = g.new(L.F32, [D, NH, T_], q)
+        rq = rope(tq)
+        g.place = [(rq, tq)] if blend else []
+        rk = rope(g.new(L.F32, [D, NKV, T_], k))
+        val = g.new(L.F32, [NKV * D, T_], v)
+        if blend:
+            val = H.ggml_add(g.ctx, H.ggml_scale(g.ctx, val, 0.375), H.ggml_scale(g.ctx, g.new(L.F32, [NKV * D, T_], y), 0.7))
+        g.first = [rq, rk, val] if blend else [rq, rk]
+        return [H.ggml_set_rows(g.ctx, caches[0], H.ggml_reshape_2d(g.ctx, rk, NKV * D, T_), rows), H.ggml_set_rows(g.ctx, caches[1], val, rows), H.ggml_scale(g.ctx, rq, 1.0)]
+
+    def run():
+        g = T.G(backend)
+        try:
+            outs = build(g)
+            n0 = backend.stat("kernel_launches")
+            got = [np.asarray(o).copy() for o in g.compute(outs, expand_first=g.first, same_block=g.place)]
+            return got, backend.stat("kernel_launches") - n0
+        finally:
+            g.free()
+
+    got, n = run()
+    backend.set_option("fusion", 0)
+    try:
+        ref, n_ref = run()
+    finally:
+        backend.set_option("fusion", 1)
+    assert n == launches + 1 and n_ref == (8 if blend else 5), (n, n_ref)  # (+ the read of the queries)
+    for a, b in zip(got, ref):
+        assert np.array_equal(a.view(np.uint8), b.view(np.uint8))
