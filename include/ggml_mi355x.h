@@ -58,6 +58,7 @@ ggml_backend_reg_t ggml_backend_mi355x_reg(void);
  *   "ggml_backend_mi355x_scratch_probe"   ggml_backend_mi355x_scratch_probe_t   (tests: the scratch that a graph's partial products and records may take)
  *   "ggml_backend_mi355x_k_slices"        ggml_backend_mi355x_k_slices_t        (tests: K slices of a K-quant product)
  *   "ggml_backend_mi355x_prepare_columns" ggml_backend_mi355x_prepare_columns_t
+ *   "ggml_backend_mi355x_result_to"       ggml_backend_mi355x_result_to_t
  *   "ggml_backend_mi355x_decode_copy_read" ggml_backend_mi355x_decode_copy_read_t (tests: the plane-layout decode copy of a weight matrix, csrc/repack.hip)
  */
 
@@ -102,6 +103,10 @@ typedef int (*ggml_backend_mi355x_k_slices_t)(int type, int64_t K, int64_t n_row
  * stream.  A host that has loaded its weights may call it once per group of matrices, so that the first such batch does not have to make them; copies that exist are kept.  Returns the
  * number of matrices that have one, -1 on error. */
 typedef int (*ggml_backend_mi355x_prepare_columns_t)(ggml_backend_t backend, const struct ggml_tensor * const * matrices, int n, int64_t from, int64_t to);
+
+/* The bytes of tensor t (f32, dense, the result of the graph that the backend is given next) go to `host`, memory of the backend's host buffer type, as part of that graph: complete after
+ * ggml_backend_synchronize, as behind a get_tensor_async that it takes the place of; t's own memory may not hold them afterwards.  Returns 1 where the next graph_compute will do so, else 0. */
+typedef int (*ggml_backend_mi355x_result_to_t)(ggml_backend_t backend, const struct ggml_tensor * t, void * host, size_t size);
 
 /* The decode copy (round 6): K-quant weight matrices of a usage-WEIGHTS buffer are kept a second time in a line-aligned plane layout that the batch-1 mat-vec kernels
  * stream with non-temporal loads (csrc/repack.hip, csrc/mmvq_types.h; option "decode_copy", GGML_MI355X_DECODE_COPY).  The tensor the host uploaded stays as it is:

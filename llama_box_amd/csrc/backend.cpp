@@ -1015,6 +1015,18 @@ static int api_prepare_columns(ggml_backend_t be, const ggml_tensor * const * w,
     uploader_join(c->device, c->stream);  // (weights staged by set_tensor are complete before they are read)
     return prepare_columns(c, w, n, from, to);
 }
+// the graph computed next leaves tensor t's bytes at `host` (graph.cpp: result_node)
+static int api_result_to(ggml_backend_t be, const ggml_tensor * t, void * host, size_t size) {
+    if (!be_is_ours(be) || t == nullptr) return 0;
+    backend_ctx * c = (backend_ctx *) be->context;
+    c->result = {};
+    if (!c->opt.small_downloads || size == 0 || size != ggml_abi_nbytes(t) || t->type != GGML_TYPE_F32 || !ggml_abi_is_contiguous(t) || t->data == nullptr || t->ne[1] < 2 || ((uintptr_t) host & 15) || !is_pinned_range(host, size) || ip_any() || tp_active(c)) return 0;
+    note_download(c, host, size);
+    c->result.src = t->data;
+    c->result.host = (char *) host;
+    c->result.bytes = size;
+    return 1;
+}
 // tests: the decode copy of weight matrix t (repacking it first if need be) into `out`; returns its bytes, 0 when the tensor has / gets no copy, -1 on error
 static int64_t api_decode_copy_read(ggml_backend_t be, const ggml_tensor * t, void * out, size_t size) {
     if (!be_is_ours(be) || t == nullptr) return -1;
@@ -1159,6 +1171,7 @@ static void * reg_get_proc_address(ggml_backend_reg_t, const char * name) {
     if (n == "ggml_backend_mi355x_tp_rowpar_buffer_type") return (void *) api_tp_rowpar_buft;
     if (n == "ggml_backend_mi355x_set_option") return (void *) api_set_option;
     if (n == "ggml_backend_mi355x_prepare_columns") return (void *) api_prepare_columns;
+    if (n == "ggml_backend_mi355x_result_to") return (void *) api_result_to;
     if (n == "ggml_backend_mi355x_decode_copy_read") return (void *) api_decode_copy_read;
     if (n == "ggml_backend_mi355x_get_stat") return (void *) api_get_stat;
     if (n == "ggml_backend_mi355x_timing_report") return (void *) api_timing_report;

@@ -217,6 +217,12 @@ struct act_image {
         return ggml_abi_is_contiguous(t) && ne[1] * ne[2] * ne[3] == t->ne[1] * t->ne[2] * t->ne[3] && nb[2] == nb[1] * (size_t) ne[1] && nb[3] == nb[2] * (size_t) ne[2];
     }
 };
+// a graph's result in host memory of the pinned buffer type: written by the graph itself
+struct result_target {
+    const void * src = nullptr;  // the tensor's memory
+    char * host = nullptr;
+    size_t bytes = 0;
+};
 struct backend_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -256,6 +262,7 @@ struct backend_ctx {
     int up_used = 0;       // slots whose contents may not have been taken yet: since the last synchronize, or the last wait of up_stream for the stream
     bool up_behind = false;  // a graph entered the stream since the last synchronize
     bool up_off = false;     // (could not be set up)
+    result_target result;          // where the next graph's result goes besides (ggml_backend_mi355x_result_to), until that graph is computed
     bool downloads_open = false;  // get_tensor_async calls since the last synchronize (backend.cpp: note_download)
     upload_batch up_pending{};  // staged in the ring, not yet launched: flushed as ONE kernel before anything else enters the stream
     // attention over a unified cache with a few query tokens: per-token lists of visible tiles (fattn.hip, k_fattn_tile_scan),

@@ -2375,6 +2375,7 @@ struct llm_context {
     char * pin = nullptr;
     size_t pin_in_bytes = 0;   // per input slot
     int pin_out_rows = 0;
+    int (*result_to)(ggml_backend_t, const ggml_tensor *, void *, size_t) = nullptr;  // the backend's graph leaves the logits in the output area itself
     // micro-batches without outputs are not waited for (as llama.cpp: the wait happens when results are fetched); each
     // in-flight micro-batch keeps its own input slot, so the host builds and stages batch i+1 while the GPU runs batch i
     // (only the slot's own micro-batch is waited for, on its event: a full wait before the fourth of four micro-batches left the GPU idle while the host filled its masks, 213 of 2950 us)
@@ -3427,6 +3428,7 @@ extern "C" struct llm_context * llm_context_new(struct llm_model * m, ggml_backe
                 for (ggml_backend_event_t & e : c->pin_ev) e = ggml_backend_event_new(backend->device);
             }
         }
+        if (backend->device->reg) c->result_to = (decltype(c->result_to)) ggml_backend_reg_get_proc_address(backend->device->reg, "ggml_backend_mi355x_result_to");
         prepare_columns(backend, c->p.n_ubatch, column_groups(m, 0, (int) m->layers.size(), true));
     }
     return c;
@@ -3919,8 +3921,9 @@ static int decode_ubatch(llm_context * c, int n_tokens, const int32_t * tokens, 
     const bool async_out = async_io && n_outputs > 0 && (direct_out || n_outputs <= c->pin_out_rows);
     enum ggml_status st;
     if (async_io) {
+        const bool by_graph = async_out && direct_out && c->result_to && c->result_to(c->backend, c->t_logits, logits_out, logit_bytes);
         st = ggml_backend_graph_compute_async(c->backend, c->gf);
-        if (st == GGML_STATUS_SUCCESS && async_out) ggml_backend_tensor_get_async(c->backend, c->t_logits, direct_out ? (void *) logits_out : (void *) pin_out, 0, logit_bytes);
+        if (st == GGML_STATUS_SUCCESS && async_out && !by_graph) ggml_backend_tensor_get_async(c->backend, c->t_logits, direct_out ? (void *) logits_out : (void *) pin_out, 0, logit_bytes);
         if (n_outputs > 0 || st != GGML_STATUS_SUCCESS || !defer_sync) {
             ggml_backend_synchronize(c->backend);
             c->all_done();

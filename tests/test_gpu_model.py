@@ -1024,6 +1024,32 @@ def test_uploads_wait_for_the_download_that_fills_their_source(backend, H, nbyte
             other.close()
 
 
+# the logits of several columns, stored by the output product in the pinned output area (option small_downloads) or copied there: eager, captured and replayed steps, rows at the kernels' edges (2 .. 64 columns)
+@pytest.mark.parametrize("name", ["test-llama", "tinyllama-1.1b-q8_0", "llama3-8b-q4_k_m"])
+@pytest.mark.parametrize("cols", [1, 2, 9, 17, 33, 64, 70])
+def test_logits_stored_by_the_output_product(backend, H, name, cols):
+    m = Model(preset(name) if name == "test-llama" else preset(name, n_layer=1, n_vocab=4096), 5, backend.buft)
+    rng = np.random.default_rng(cols)
+    tok = rng.integers(0, m.n_vocab_local, (5, cols))
+    rows = []
+    try:
+        for on in (1, 0):
+            backend.set_option("small_downloads", on)
+            c = Context(m, backend=backend, n_ctx=512, flash_attn=1)
+            rows.append([])
+            for t in tok:  # (the same positions again: a graph seen before)
+                rc, lg = c.decode(t, range(cols))
+                assert rc == 0 and lg.shape[0] == cols
+                rows[-1].append(lg)
+                c.seq_rm(-1, 0, -1)
+            c.free()
+    finally:
+        backend.set_option("small_downloads", 1)
+        m.free()
+    for a, b in zip(*rows):
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+
+
 def test_copies_for_batches_are_made_with_the_context(backend, H):
     """The first step of a few sequences finds the panel copies that it reads (llama_lite.cpp: prepare_columns)."""
     hp = preset("llama3-8b-q4_k_m")
