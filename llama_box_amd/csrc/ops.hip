@@ -70,6 +70,38 @@ __global__ void __launch_bounds__(256) k_rms_norm(const tdesc a, const tdesc d, 
     const int64_t n = a.ne[0];
     const bool vec = (n & 3) == 0 && ((((uintptr_t) x) | ((uintptr_t) y) | ((uintptr_t) w)) & 15) == 0;
     double s = 0.0;
+    // up to 4096 entries: the row, its weights and what is added are requested together and held, one round trip instead of three in a row (16 rows of 2048 as panels: 4.9 -> 4.2 us)
+    if (vec && n <= 4096) {
+        const int n4 = (int) (n >> 2);
+        const float4 * x4 = (const float4 *) x, * w4 = (const float4 *) w, * e4 = (const float4 *) (res ? res + row * n : x);
+        float4 v[4], g[4], e[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            if (256 * u >= n4) break;
+            const int i = min((int) threadIdx.x + 256 * u, n4 - 1);  // (a thread behind the row's end holds its last entries and adds nothing)
+            v[u] = x4[i];
+            if (w) g[u] = w4[i];
+            if (res) e[u] = e4[i];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            if ((int) threadIdx.x + 256 * u < n4) s += (double) (v[u].x * v[u].x) + (double) (v[u].y * v[u].y) + (double) (v[u].z * v[u].z) + (double) (v[u].w * v[u].w);
+        }
+        s = block_sum_d(s, sh);
+        const float scale = 1.0f / sqrtf((float) (s / (double) n) + eps);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int i = (int) threadIdx.x + 256 * u;
+            if (i >= n4) break;
+            float4 r;
+            r.x = v[u].x * scale; r.y = v[u].y * scale; r.z = v[u].z * scale; r.w = v[u].w * scale;
+            if (w) { r.x = r.x * g[u].x; r.y = r.y * g[u].y; r.z = r.z * g[u].z; r.w = r.w * g[u].w; }
+            if (res) { r.x = r.x + e[u].x; r.y = r.y + e[u].y; r.z = r.z + e[u].z; r.w = r.w + e[u].w; }
+            if constexpr (Q80P) q80_panel_store(r.x, r.y, r.z, r.w, i & 7, row, i >> 3, n4 >> 3, q80);
+            else ((float4 *) y)[i] = r;
+        }
+        return;
+    }
     if (vec) {
         // up to 4 independent 16-byte loads per thread per trip: a 4096-wide row is ONE round trip to L2
         const float4 * x4 = (const float4 *) x;
@@ -991,22 +1023,44 @@ void launch_softcap(hipStream_t s, const float * x, float * d, int64_t n, float 
     hipLaunchKernelGGL(k_softcap, dim3((unsigned) std::min<int64_t>((n + 255) / 256, 4096)), dim3(256), 0, s, x, d, n, by, cap);
 }
 
-__global__ void __launch_bounds__(256) k_weighted_rows_sum(const tdesc rows, const tdesc w, const tdesc d) {
-    const int64_t t = blockIdx.x, n_used = rows.ne[1];
-    const float * __restrict__ wt = (const float *) (w.data + t * w.nb[2]);
-    float * __restrict__ out = (float *) (d.data + t * d.nb[1]);
-    for (int64_t i = threadIdx.x; i < rows.ne[0]; i += blockDim.x) {
-        float acc = 0.0f;
-        for (int64_t u = 0; u < n_used; ++u) {
-            const float p = *(const float *) (rows.data + i * 4 + u * rows.nb[1] + t * rows.nb[2]) * *(const float *) ((const char *) wt + u * w.nb[1]);
-            acc = u == 0 ? p : acc + p;
+// One thread holds V neighbouring entries of a token's sum: the rows of four experts are requested together, and a token's row is spread over workgroups (a step of two tokens would leave
+// two workgroups walking it: 2 x 2048, four experts, 6.7 -> 2.9 us)
+template <int V> __global__ void __launch_bounds__(256) k_weighted_rows_sum(const tdesc rows, const tdesc w, const tdesc d) {
+    const int64_t t = blockIdx.x, i = ((int64_t) blockIdx.y * 256 + threadIdx.x) * V;
+    const int n_used = (int) rows.ne[1];
+    if (i >= rows.ne[0]) return;
+    const char * wt = w.data + t * w.nb[2];
+    const char * x = rows.data + i * 4 + t * rows.nb[2];
+    float acc[V] = {};
+    for (int u0 = 0; u0 < n_used; u0 += 4) {
+        float f[4], v[4][V];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int64_t u = min(u0 + k, n_used - 1);
+            f[k] = *(const float *) (wt + u * w.nb[1]);
+            if constexpr (V == 4) *(float4 *) v[k] = *(const float4 *) (x + u * rows.nb[1]);
+            else v[k][0] = *(const float *) (x + u * rows.nb[1]);
         }
-        out[i] = acc;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            if (u0 + k >= n_used) break;
+#pragma unroll
+            for (int c = 0; c < V; ++c) {
+                const float p = v[k][c] * f[k];
+                acc[c] = u0 + k == 0 ? p : acc[c] + p;
+            }
+        }
     }
+    float * out = (float *) (d.data + t * d.nb[1]) + i;
+    if constexpr (V == 4) *(float4 *) out = *(const float4 *) acc;
+    else out[0] = acc[0];
 }
 void launch_weighted_rows_sum(hipStream_t s, const tdesc & rows, const tdesc & w, const tdesc & d) {
-    if (rows.ne[2] == 0) return;
-    hipLaunchKernelGGL(k_weighted_rows_sum, dim3((unsigned) rows.ne[2]), dim3(256), 0, s, rows, w, d);
+    if (rows.ne[2] == 0 || rows.ne[0] == 0) return;
+    const bool vec = (rows.ne[0] & 3) == 0 && ((((uintptr_t) rows.data) | ((uintptr_t) d.data) | (uintptr_t) rows.nb[1] | (uintptr_t) rows.nb[2] | (uintptr_t) d.nb[1]) & 15) == 0;
+    const dim3 grid((unsigned) rows.ne[2], (unsigned) ((rows.ne[0] + (vec ? 1023 : 255)) / (vec ? 1024 : 256)));
+    if (vec) hipLaunchKernelGGL(k_weighted_rows_sum<4>, grid, dim3(256), 0, s, rows, w, d);
+    else hipLaunchKernelGGL(k_weighted_rows_sum<1>, grid, dim3(256), 0, s, rows, w, d);
 }
 
 // ------------------------------------------------------------------------------------------------ ADD/SUB/MUL/DIV

@@ -438,6 +438,37 @@ def test_experts_router_and_weighted_sum(backend, H, wtype, T_, E, ff, n_exp, to
     assert np.abs(got - ref).max() <= tol * max(1.0, np.abs(ref).max())
 
 
+@pytest.mark.parametrize("n,top,T_", [(64, 1, 3), (1024, 2, 1), (1028, 3, 2), (2048, 4, 2), (36, 5, 70), (35, 9, 2), (4096, 8, 1)])
+def test_weighted_sum_of_expert_rows(backend, H, n, top, T_):
+    """MUL by the weights and the chain of ADDs in one launch against the same sum in that order: four experts at a time and a remainder, float4 and single entries, the edges of a workgroup"""
+    rng = np.random.default_rng(n + top)
+    n_exp, K = 9, 32
+    ups, x = rng.standard_normal((n_exp, n, K)).astype(np.float32), rng.standard_normal((T_, K)).astype(np.float32)
+    sel = np.stack([rng.permutation(n_exp)[:top] for _ in range(T_)]).astype(np.int32)
+    w = rng.standard_normal((T_, top)).astype(np.float32)
+
+    def build(g, chain):
+        ids = g.new(L.I32, [top, T_], sel)
+        rows = H.ggml_mul_mat_id(g.ctx, g.new(L.F32, [K, n, n_exp], ups), g.new(L.F32, [K, 1, T_], x), ids)
+        if not chain:
+            return [rows]
+        mul = H.ggml_mul(g.ctx, rows, g.new(L.F32, [1, top, T_], w))
+        acc = None
+        for u in range(top):
+            v = H.ggml_view_2d(g.ctx, mul, n, T_, top * n * 4, u * n * 4)
+            acc = v if acc is None else H.ggml_add(g.ctx, acc, v)
+        return [H.ggml_cont(g.ctx, acc) if top == 1 else acc]
+
+    rows = run(backend, lambda g: build(g, False))[0].reshape(T_, top, n)
+    f0 = backend.stat("fused_nodes")
+    got = run(backend, lambda g: build(g, True))[0].reshape(T_, n)
+    assert backend.stat("fused_nodes") > f0
+    ref = rows[:, 0] * w[:, :1]
+    for u in range(1, top):
+        ref = ref + rows[:, u] * w[:, u:u + 1]
+    assert np.array_equal(got, ref)  # the same products and additions in the same order
+
+
 def test_erf_gelu_and_squared_relu(backend, H):
     x = np.linspace(-6, 6, 1001).astype(np.float32)
 

@@ -520,6 +520,25 @@ def test_rms_norm_and_mul(backend, H, plog, ne):
     T.compare(f"rms_norm*2 (shared) {ne}", got[1], ref[1], max_nmse=1e-13, log=plog)
 
 
+@pytest.mark.parametrize("n", [4, 252, 1024, 1028, 2052, 4092, 4096, 4100, 4095])
+@pytest.mark.parametrize("form", ["plain", "weighted", "in place"])
+def test_rms_norm_row_lengths(backend, H, plog, n, form):
+    """rows of up to 4096 entries are held in registers, longer ones and those of no whole float4 are read twice; in place over the product that the norm reads"""
+    rng = np.random.default_rng(n)
+    x = (rng.standard_normal((3, n)) * 3).astype(np.float32)
+    w = rng.uniform(0.5, 1.5, n).astype(np.float32)
+
+    def build(g):
+        t = g.new(L.F32, [n, 3], x)
+        if form == "in place":
+            t = H.ggml_scale(g.ctx, t, 0.5)
+        y = H.ggml_rms_norm(g.ctx, t, 1e-5)
+        return y if form == "plain" else H.ggml_mul(g.ctx, y, g.new(L.F32, [n], w))
+
+    ref, got = both(build, backend)
+    T.compare(f"rms_norm {form} {n}", got[0], ref[0], max_nmse=1e-13, max_abs=2e-6, log=plog)
+
+
 @pytest.mark.parametrize("op", ["add", "sub", "mul", "div"])
 def test_binary_broadcast(backend, H, plog, op):
     rng = np.random.default_rng(11)
