@@ -17,6 +17,7 @@
 //     the result is written as float4 runs along d.
 // P is rounded to f16 for the second GEMM (the CPU path rounds the whole accumulation to f16 at every step).
 #include <algorithm>
+#include <type_traits>
 
 #include "dev_util.h"
 #include "kernels.h"
@@ -312,7 +313,7 @@ __global__ void __launch_bounds__(NW * 64, 2) k_fattn_mma(const tdesc q, const t
 // not an online one: PASS 1 leaves (max, sum of e^(w - max)) per (query, head, KV split); PASS 2 combines those into the row's maximum and sum,
 // recomputes the scores, takes p = e^(w - max) * (1 / sum) — rounded to f16 where the CPU's second MUL_MAT rounds its src1 — and multiplies with
 // the TRANSPOSED V cache, whose rows need no transposition on the way into LDS.  Partial outputs of KV splits simply add (k_fattn_combine_rows
-// with coefficients 1).  llama-box's zero-sum guard (ggml-cpu.patch:5-15) and the NaN row of a query that sees nothing are kept.
+// with coefficients 1).  (Head dimension 64 had the three launches until its own two passes: a 2000-token prompt of the small model 24.5 -> 15.5 ms, 14.8 with the one launch below.)  llama-box's zero-sum guard (ggml-cpu.patch:5-15) and the NaN row of a query that sees nothing are kept.
 template <int D, int NW, int PASS>
 __global__ void __launch_bounds__(NW * 64, 2) k_attn_nf_mma(const tdesc q, const tdesc k, const tdesc vt, const tdesc mask, const tdesc dst, const fam_geom geo, float * __restrict__ stats,
                                                          float * __restrict__ ws, const uint8_t * __restrict__ vis) {
@@ -556,6 +557,188 @@ __global__ void __launch_bounds__(NW * 64, 2) k_attn_nf_mma(const tdesc q, const
     }
 }
 
+// The same chain of a SHORT cache (up to 256 NT cells) in one launch, its scores made once (77 tokens of Llama-3-8B, a layer: 10.3 + 7.7 us of two passes and 4.8 of the quantiser behind them, now 7.3; the two passes
+// had 32 workgroups, a head each).
+// A workgroup owns 16 QT columns — 8 QT queries of HP = 2 heads of a group, or 16 QT of one — and its eight waves share the cells in blocks of 32 (block w, w + 8, ..), whose scores stay in
+// registers from K.q to V^T.p.  K and V^T come from memory as the matrix cores need them (16 rows of 64 bytes an instruction: with 32 rows of 32 the address pipeline took 15.0 us instead of 7.3): the rows
+// of a block's two K tiles are the cells that make a lane's eight scores eight consecutive cells, so V^T is read 16 bytes at a time.  The waves meet for the row's maximum, its sum and the result, which
+// leaves as Q8_K blocks (two heads of a token) where only quantised products read it.
+typedef float float4v __attribute__((ext_vector_type(4)));
+template <int D, int NT, int QT, int HP>
+__global__ void __launch_bounds__(512, 2) k_attn_nf_once(const tdesc q, const tdesc k, const tdesc vt, const tdesc mask, const tdesc dst, const fam_geom geo, q8k_dev * __restrict__ q8) {
+    constexpr int NS = D / 32, ND = D / 16, PS = D + 4, QS = D + 8, NC = 16 * QT, NQ = NC / HP;
+    constexpr float LOG2E = 1.4426950408889634f;
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    float * part = (float *) smem;          // [wave][column][PS], once the queries have been read:
+    _Float16 * qs = (_Float16 *) smem;      // [column][QS]
+    __shared__ float st_m[8][NC], st_l[8][NC];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int col = lane & 15, quad = lane >> 4;
+    const int h0 = HP * (int) blockIdx.y, kvh = h0 / (geo.n_head / geo.n_kv_head), q0 = (int) blockIdx.x * NQ;
+    auto col_q = [&](const int c) { return HP == 2 ? (c >> 4) * 8 + (c & 7) : c; };  // a column's query (of the workgroup's) and head (of its HP)
+    auto col_h = [&](const int c) { return HP == 2 ? (c >> 3) & 1 : 0; };
+    const char * kbase = k.data + (int64_t) kvh * k.nb[2] + 16 * quad;
+    const char * vbase = vt.data + (int64_t) kvh * vt.nb[2] + (int64_t) col * vt.nb[1];
+    const int cell = 8 * (col >> 2) + (col & 3);  // of a block, for row `col` of its first K tile (of the second: + 4): a lane's scores are then cells 8 quad .. + 7
+
+    half8 kf[NT][2][NS];
+    float4 mv[NT][QT][2];
+    auto load_k = [&](const int t) {  // (cells behind the cache's end: its last ones, hidden)
+        const int c0 = 32 * (wave + 8 * t);
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const char * kr = kbase + (int64_t) min(c0 + cell + 4 * u, geo.n_kv - 1) * k.nb[1];
+#pragma unroll
+            for (int s = 0; s < NS; ++s) kf[t][u][s] = *(const half8 *) (kr + 64 * s);
+        }
+#pragma unroll
+        for (int j = 0; j < QT; ++j) {
+            const float * mrow = (const float *) (mask.data + (int64_t) min(q0 + col_q(16 * j + col), geo.n_q - 1) * mask.nb[1]);
+#pragma unroll
+            for (int u = 0; u < 2; ++u) mv[t][j][u] = *(const float4 *) (mrow + min(c0 + 8 * quad + 4 * u, geo.n_kv - 4));
+        }
+    };
+#pragma unroll
+    for (int t = 0; t < NT && t < 2; ++t) load_k(t);
+    for (int i = tid; i < NC * (D / 4); i += 512) {
+        const int c = i / (D / 4), d = 4 * (i % (D / 4));
+        const float4 x = *(const float4 *) (q.data + (int64_t) min(q0 + col_q(c), geo.n_q - 1) * q.nb[1] + (int64_t) (h0 + col_h(c)) * q.nb[2] + (int64_t) d * 4);
+        *(half4v *) (qs + c * QS + d) = (half4v){(_Float16) x.x, (_Float16) x.y, (_Float16) x.z, (_Float16) x.w};
+    }
+    __syncthreads();
+    half8 qf[QT][NS];
+#pragma unroll
+    for (int j = 0; j < QT; ++j)
+#pragma unroll
+        for (int s = 0; s < NS; ++s) qf[j][s] = *(const half8 *) (qs + (16 * j + col) * QS + 32 * s + 8 * quad);
+    float S[NT][QT][8];
+    uint32_t seen = 0;  // (uniform) the blocks of which some query sees a cell: the others are not multiplied
+    float m[QT];
+#pragma unroll
+    for (int j = 0; j < QT; ++j) m[j] = -INFINITY;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        const bool in = 32 * (wave + 8 * t) + 8 * quad < geo.n_kv;  // (n_kv % 8 == 0)
+        bool any = false;
+#pragma unroll
+        for (int j = 0; j < QT; ++j)
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const float x[4] = {mv[t][j][u].x, mv[t][j][u].y, mv[t][j][u].z, mv[t][j][u].w};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    S[t][j][4 * u + e] = in ? x[e] : -INFINITY;
+                    any = any || S[t][j][4 * u + e] != -INFINITY;
+                }
+            }
+        if (__any(any)) {
+            seen |= 1u << t;
+#pragma unroll
+            for (int j = 0; j < QT; ++j)
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    float4v acc = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                    for (int s = 0; s < NS; ++s) acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[t][u][s], qf[j][s], acc, 0, 0, 0);
+                    // w = kq * scale + mask (two roundings, as SOFT_MAX computes it)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        S[t][j][4 * u + e] = acc[e] * geo.scale + S[t][j][4 * u + e];
+                        m[j] = fmaxf(m[j], S[t][j][4 * u + e]);
+                    }
+                }
+        }
+        if (t + 2 < NT) load_k(t + 2);
+    }
+    // V^T of a block: rows 16 d + col, cells 8 quad .. + 7 (cells past n_kv are given p = 0, and 0 x NaN must not happen)
+    half8 vf[NT][ND];
+    auto load_v = [&](const int t) {
+        const int c = 32 * (wave + 8 * t) + 8 * quad;
+#pragma unroll
+        for (int d = 0; d < ND; ++d) vf[t][d] = c < geo.n_kv ? *(const half8 *) (vbase + (int64_t) (16 * d) * vt.nb[1] + (int64_t) c * 2) : half8{};
+    };
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+        if (t < 2 && ((seen >> t) & 1)) load_v(t);  // (under way during the soft-max)
+#pragma unroll
+    for (int j = 0; j < QT; ++j) {
+        m[j] = fmaxf(m[j], __shfl_xor(m[j], 16, 64));
+        m[j] = fmaxf(m[j], __shfl_xor(m[j], 32, 64));
+        if (quad == 0) st_m[wave][16 * j + col] = m[j];
+    }
+    __syncthreads();
+    float l[QT], inv[QT];
+#pragma unroll
+    for (int j = 0; j < QT; ++j) {
+        float mg = -INFINITY;
+#pragma unroll
+        for (int w = 0; w < 8; ++w) mg = fmaxf(mg, st_m[w][16 * j + col]);
+        const float mref = mg == -INFINITY ? 0.0f : mg;  // (a query that sees nothing: zeros here, NaN below)
+        l[j] = 0.0f;
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+            if ((seen >> t) & 1) {
+#pragma unroll
+                for (int r = 0; r < 8; ++r) {
+                    S[t][j][r] = __builtin_amdgcn_exp2f((S[t][j][r] - mref) * LOG2E);
+                    l[j] += S[t][j][r];
+                }
+            }
+        l[j] += __shfl_xor(l[j], 16, 64);
+        l[j] += __shfl_xor(l[j], 32, 64);
+        if (quad == 0) st_l[wave][16 * j + col] = l[j];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < QT; ++j) {
+        double sum = 0.0;
+#pragma unroll
+        for (int w = 0; w < 8; ++w) sum += (double) st_l[w][16 * j + col];
+        if (isnan(sum) || sum == 0.0) sum = -INFINITY;
+        inv[j] = (float) (1.0 / sum);
+    }
+    float4v O[QT][ND];
+#pragma unroll
+    for (int j = 0; j < QT; ++j)
+#pragma unroll
+        for (int d = 0; d < ND; ++d) O[j][d] = (float4v){0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+        if ((seen >> t) & 1) {
+            if (t >= 2) load_v(t);
+#pragma unroll
+            for (int j = 0; j < QT; ++j) {
+                half8 pb;
+#pragma unroll
+                for (int u = 0; u < 8; ++u) pb[u] = (_Float16) (S[t][j][u] * inv[j]);
+#pragma unroll
+                for (int d = 0; d < ND; ++d) O[j][d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf[t][d], pb, O[j][d], 0, 0, 0);
+            }
+        }
+#pragma unroll
+    for (int j = 0; j < QT; ++j)
+#pragma unroll
+        for (int d = 0; d < ND; ++d) *(float4v *) (part + (wave * NC + 16 * j + col) * PS + 16 * d + 4 * quad) = O[j][d];
+    __syncthreads();
+    // a lane takes four entries of a column, a wave 256 of them (a Q8_K block: both heads of a query)
+    constexpr int LC = D / 4, CW = 64 / LC;
+    const int g = lane / LC, d0 = 4 * (lane % LC);
+    for (int i = wave; i < NC / CW; i += 8) {
+        const int c = HP == 2 && D == 128 ? 16 * (i >> 3) + (i & 7) + 8 * g : CW * i + g, qi = q0 + col_q(c);
+        float v[4] = {0.0f, 0.0f, 0.0f, 0.0f}, mg = -INFINITY;
+#pragma unroll
+        for (int w = 0; w < 8; ++w) {
+            const float4 x = *(const float4 *) (part + (w * NC + c) * PS + d0);
+            v[0] += x.x; v[1] += x.y; v[2] += x.z; v[3] += x.w;
+            mg = fmaxf(mg, st_m[w][c]);
+        }
+        if (mg == -INFINITY) v[0] = v[1] = v[2] = v[3] = __builtin_nanf("");  // (the CPU's row: NaN throughout)
+        if (qi >= geo.n_q) continue;  // (both heads of a query together)
+        if (HP == 2 && D == 128 && q8) wave_quantize_q8_K(v, lane, q8 + (int64_t) qi * (geo.n_head / 2) + blockIdx.y);
+        else *(float4 *) (dst.data + (int64_t) (h0 + col_h(c)) * dst.nb[1] + (int64_t) qi * dst.nb[2] + (int64_t) d0 * 4) = make_float4(v[0], v[1], v[2], v[3]);
+    }
+}
+
 // returns false when this variant does not apply (caller falls back to the split-KV kernel)
 int fattn_mma_pick_splits(const tdesc & q, const tdesc & k) {
     const int64_t qt = q.ne[1] >= 256 ? 128 : 64;
@@ -657,7 +840,7 @@ bool launch_flash_attn_mma(hipStream_t s, const tdesc & q, const tdesc & k, cons
 bool attn_nf_mma_applies(const tdesc & q, const tdesc & k, const tdesc & vt, const tdesc & mask) {
     static const bool on = !getenv("GGML_MI355X_ATTN_NF_MMA") || atoi(getenv("GGML_MI355X_ATTN_NF_MMA")) != 0;
     const int64_t D = k.ne[0];
-    if (!on || D != 128 || q.ne[1] < fattn_mma_min_q() || q.ne[3] != 1 || k.ne[3] != 1 || vt.ne[3] != 1 || k.type != GGML_TYPE_F16 || vt.type != GGML_TYPE_F16 || q.type != GGML_TYPE_F32 ||
+    if (!on || (D != 128 && D != 64) || q.ne[0] != D || q.ne[1] < fattn_mma_min_q() || q.ne[3] != 1 || k.ne[3] != 1 || vt.ne[3] != 1 || k.type != GGML_TYPE_F16 || vt.type != GGML_TYPE_F16 || q.type != GGML_TYPE_F32 ||
         mask.type != GGML_TYPE_F32)
         return false;
     if (k.ne[2] <= 0 || q.ne[2] % k.ne[2] != 0 || vt.ne[2] != k.ne[2] || vt.ne[0] != k.ne[1] || vt.ne[1] != D || (k.ne[1] % 8) != 0) return false;
@@ -685,14 +868,56 @@ void launch_attn_nf_mma(hipStream_t s, const tdesc & q, const tdesc & k, const t
     float * recs = (float *) ((char *) workspace + ((rows * (size_t) geo.n_splits * 2 * sizeof(float) + 255) & ~(size_t) 255));
     const int tiles_all = (geo.n_kv + 63) / 64, tps = (tiles_all + geo.n_splits - 1) / geo.n_splits;
     const uint8_t * const vis = tps <= 16384 ? tile_vis : nullptr;
-    const size_t lds = 64 * (128 + 8) * 2 + 128 * (64 + 4) * 2 + (vis ? (size_t) ((tps + 15) & ~15) : 0);
+    const int D = (int) k.ne[0];
+    const size_t lds = 64 * (D + 8) * 2 + D * (64 + 4) * 2 + (vis ? (size_t) ((tps + 15) & ~15) : 0);
     // (always 128-query workgroups: the 64-query form of pass 2 holds twice the staging registers per thread and spills 60 of them; a batch
     // of 64 tokens leaves two of the four waves multiplying clamped duplicates instead)
     constexpr int nw = 4;
     dim3 grid((unsigned) ((geo.n_q + nw * 32 - 1) / (nw * 32)), (unsigned) geo.n_head, (unsigned) geo.n_splits);
-    hipLaunchKernelGGL((k_attn_nf_mma<128, 4, 1>), grid, dim3(256), lds, s, q, k, vt, mask, dst, geo, stats, recs, vis);
-    hipLaunchKernelGGL((k_attn_nf_mma<128, 4, 2>), grid, dim3(256), lds, s, q, k, vt, mask, dst, geo, stats, recs, vis);
-    if (geo.n_splits > 1) launch_flash_attn_combine(s, 128, recs, nullptr, dst, geo.n_q, geo.n_head, 1, geo.n_splits, q8_out);  // (q8_out: only where the row-parallel form applies — the caller checked)
+    if (D == 64) {
+        hipLaunchKernelGGL((k_attn_nf_mma<64, 4, 1>), grid, dim3(256), lds, s, q, k, vt, mask, dst, geo, stats, recs, vis);
+        hipLaunchKernelGGL((k_attn_nf_mma<64, 4, 2>), grid, dim3(256), lds, s, q, k, vt, mask, dst, geo, stats, recs, vis);
+    } else {
+        hipLaunchKernelGGL((k_attn_nf_mma<128, 4, 1>), grid, dim3(256), lds, s, q, k, vt, mask, dst, geo, stats, recs, vis);
+        hipLaunchKernelGGL((k_attn_nf_mma<128, 4, 2>), grid, dim3(256), lds, s, q, k, vt, mask, dst, geo, stats, recs, vis);
+    }
+    if (geo.n_splits > 1) launch_flash_attn_combine(s, D, recs, nullptr, dst, geo.n_q, geo.n_head, 1, geo.n_splits, q8_out);  // (q8_out: only where the row-parallel form applies — the caller checked)
+}
+
+// One launch instead of the two passes?  It reads K and V^T once per 16 or 32 columns where they read them once per 128 queries: with many queries over many cells that is what it waits for.
+// Whole prompts, us, two passes / one launch (16 columns a workgroup, 32):
+//   head_dim 128, tokens = cells: Llama-3-8B 40 4189 / 3818, 3881; 77 5106 / 4643, 4697; 128 5613 / 5100, 5142; 200 8408 / 7835, 7778; 350 11379 / 11128, 11142; 512 12920 / 12952, 12686;
+//   700 (its second batch: 188 over 768) 20895 / 20692, 20167; 1000 (488 over 1024) 26157 / 26929, 25904, of which the first batch's 235 are most; Qwen2-7B (single heads) 100 6174 / 5800, 5843,
+//   500 15126 / 15315, 15069
+//   head_dim 64, small model: 512 3678 / 3420, 3310; 1000 7698 / 7327, 7019 (7260 with its second batch in two passes); beyond 1024 cells two passes
+bool attn_nf_once_applies(const tdesc & q, const tdesc & k) { return k.ne[1] <= (k.ne[0] == 64 || q.ne[1] <= 256 ? 1024 : 512); }
+bool attn_nf_once_q8(const tdesc & q, const tdesc & k) { return k.ne[0] == 128 && (q.ne[2] / k.ne[2]) % 2 == 0; }  // (pairs of heads of a group: their Q8_K blocks)
+template <int D, int NT, int QT, int HP>
+static void attn_nf_once_go(hipStream_t s, const tdesc & q, const tdesc & k, const tdesc & vt, const tdesc & mask, const tdesc & dst, const fam_geom & geo, void * q8_out) {
+    constexpr int NQ = 16 * QT / HP;
+    constexpr size_t lds = sizeof(float) * 8 * 16 * QT * (D + 4);
+    static std::atomic<uint32_t> raised{0};
+    (void) ensure_dyn_lds((const void *) k_attn_nf_once<D, NT, QT, HP>, lds, raised);
+    hipLaunchKernelGGL((k_attn_nf_once<D, NT, QT, HP>), dim3((unsigned) ((geo.n_q + NQ - 1) / NQ), (unsigned) (geo.n_head / HP)), dim3(512), lds, s, q, k, vt, mask, dst, geo, (q8k_dev *) q8_out);
+}
+void launch_attn_nf_once(hipStream_t s, const tdesc & q, const tdesc & k, const tdesc & vt, const tdesc & mask, const tdesc & dst, float scale, void * q8_out) {
+    const fam_geom geo{(int) q.ne[1], (int) q.ne[2], (int) k.ne[2], (int) k.ne[1], 1, 1, scale};
+    const bool pair = (q.ne[2] / k.ne[2]) % 2 == 0, two = q.ne[1] > 128;
+    const int nt = geo.n_kv <= 256 ? 1 : geo.n_kv <= 512 ? 2 : 4;
+    auto go = [&](auto d, auto t) {
+        constexpr int D = decltype(d)::value, NT = decltype(t)::value;
+        if (two && pair) attn_nf_once_go<D, NT, 2, 2>(s, q, k, vt, mask, dst, geo, q8_out);
+        else if (two) attn_nf_once_go<D, NT, 2, 1>(s, q, k, vt, mask, dst, geo, nullptr);
+        else if (pair) attn_nf_once_go<D, NT, 1, 2>(s, q, k, vt, mask, dst, geo, q8_out);
+        else attn_nf_once_go<D, NT, 1, 1>(s, q, k, vt, mask, dst, geo, nullptr);
+    };
+    auto of = [&](auto d) {
+        if (nt == 1) go(d, std::integral_constant<int, 1>{});
+        else if (nt == 2) go(d, std::integral_constant<int, 2>{});
+        else go(d, std::integral_constant<int, 4>{});
+    };
+    if (k.ne[0] == 64) of(std::integral_constant<int, 64>{});
+    else of(std::integral_constant<int, 128>{});
 }
 
 MI_TU_TOUCH(fattn_mma)

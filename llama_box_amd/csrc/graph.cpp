@@ -421,7 +421,7 @@ static ws_plan plan_ws(backend_ctx * c, const ggml_cgraph * g) {
             p.aux_bytes = std::max(p.aux_bytes, mul_mat_f_workspace_bytes(TD(n->src[0]), TD(n->src[1])));
             if (c->opt.attn_nf) p.aux_bytes = std::max(p.aux_bytes, attn_nf_list_scratch_bytes(TD(n->src[1]), TD(n->src[0]), nullptr));
             // (K.q of a prompt micro-batch on the non-flash path: statistics + partial records of the two-pass matrix-core form)
-            if (c->opt.attn_nf && n->src[1]->type == GGML_TYPE_F32 && n->src[1]->ne[1] >= fattn_mma_min_q() && n->src[0]->ne[0] == 128 && n->src[1]->ne[3] == 1)
+            if (c->opt.attn_nf && n->src[1]->type == GGML_TYPE_F32 && n->src[1]->ne[1] >= fattn_mma_min_q() && (n->src[0]->ne[0] == 128 || n->src[0]->ne[0] == 64) && n->src[1]->ne[3] == 1)
                 p.aux_bytes = std::max(p.aux_bytes, attn_nf_mma_ws_bytes(TD(n->src[1]), fattn_mma_pick_splits(TD(n->src[1]), TD(n->src[0]))));
         } else if (n->op == GGML_OP_MUL_MAT_ID && n->src[2]) {
             p.aux_bytes = std::max(p.aux_bytes, mul_mat_id_workspace_bytes(TD(n->src[0]), TD(n->src[2])));
@@ -1969,9 +1969,10 @@ static bool try_fuse_attn_nf_mma(exec_state & st, int i) {
     }
     if (jc < 0 && (ranges_overlap(kqv, Q) || (((uintptr_t) kqv->data) & 15) != 0)) return false;
     const int n_splits = fattn_mma_pick_splits(qd, kd);
+    const bool once = attn_nf_once_applies(qd, kd);
     const size_t need = attn_nf_mma_ws_bytes(qd, n_splits);
-    if (need > c->ws_size - st.aux_off) return false;
-    if (st.fa_list_mask != M->data || st.fa_list_tile != -1) {  // first attention of this graph run: the (query tile, kv tile) states
+    if (!once && need > c->ws_size - st.aux_off) return false;
+    if (!once && (st.fa_list_mask != M->data || st.fa_list_tile != -1)) {  // first attention of this graph run: the (query tile, kv tile) states
         launch_fattn_vis_scan(c->stream, md, (int) Q->ne[1], (int) K->ne[1], (uint8_t *) c->fa_lists);
         c->st.kernel_launches++;
         st.fa_list_mask = M->data;
@@ -1979,16 +1980,17 @@ static bool try_fuse_attn_nf_mma(exec_state & st, int i) {
     }
     // the copy is read only by quantised mat-muls (wo) and the splits' sum is the row-parallel combine: it writes the Q8_K blocks itself
     void * q8_out = nullptr;
-    if (jc >= 0 && n_splits > 1 && (Q->ne[2] % 2) == 0 && c->opt.prologue && !(g->nodes[jc]->flags & GGML_TENSOR_FLAG_OUTPUT) && quant_consumers_only(st, jc, g->nodes[jc]) &&
-        fattn_combine_rows_applies(128, Q->ne[1], Q->ne[2], 1, n_splits, nullptr))
+    if (jc >= 0 && (once ? attn_nf_once_q8(qd, kd) : n_splits > 1 && kd.ne[0] == 128) && (Q->ne[2] % 2) == 0 && c->opt.prologue && !(g->nodes[jc]->flags & GGML_TENSOR_FLAG_OUTPUT) && quant_consumers_only(st, jc, g->nodes[jc]) &&
+        (once || fattn_combine_rows_applies(128, Q->ne[1], Q->ne[2], 1, n_splits, nullptr)))
         q8_out = (char *) c->ws + st.act_off;
     timed_scope ts(c, "attn_nf_mma", (double) ggml_abi_nbytes(kqv));
-    launch_attn_nf_mma(c->stream, qd, kd, vd, md, od, ggml_abi_op_param_f32(sm, 0), n_splits, (const uint8_t *) c->fa_lists, (char *) c->ws + st.aux_off, q8_out);
+    if (once) launch_attn_nf_once(c->stream, qd, kd, vd, md, od, ggml_abi_op_param_f32(sm, 0), q8_out);
+    else launch_attn_nf_mma(c->stream, qd, kd, vd, md, od, ggml_abi_op_param_f32(sm, 0), n_splits, (const uint8_t *) c->fa_lists, (char *) c->ws + st.aux_off, q8_out);
     if (q8_out) {
         mark_q8_cache(st, g->nodes[jc]);
         c->st.fused_nodes++;
     }
-    c->st.kernel_launches += n_splits > 1 ? 3 : 2;
+    c->st.kernel_launches += once ? 1 : n_splits > 1 ? 3 : 2;
     c->st.nf_mma_chains++;
     mark_done(st, js);
     mark_done(st, jv);

@@ -407,6 +407,10 @@ bool attn_nf_mma_applies(const tdesc & q, const tdesc & k, const tdesc & vt, con
 size_t attn_nf_mma_ws_bytes(const tdesc & q, int n_splits);
 void launch_attn_nf_mma(hipStream_t s, const tdesc & q, const tdesc & k, const tdesc & vt, const tdesc & mask, const tdesc & dst, float scale, int n_splits, const uint8_t * tile_vis, void * workspace,
                         void * q8_out = nullptr);
+// ... over a short cache in one launch (k_attn_nf_once): shapes attn_nf_mma_applies accepts, no workspace
+bool attn_nf_once_applies(const tdesc & q, const tdesc & k);
+bool attn_nf_once_q8(const tdesc & q, const tdesc & k);  // can it leave Q8_K blocks?
+void launch_attn_nf_once(hipStream_t s, const tdesc & q, const tdesc & k, const tdesc & vt, const tdesc & mask, const tdesc & dst, float scale, void * q8_out);
 bool fattn_native_kv_ok(const tdesc & q, const tdesc & k, const tdesc & v, const fattn_params & p);  // may launch_flash_attn read this K / V pair in place (p.dq = 1)?
 bool fattn_combine_rows_applies(int D, int64_t n_q, int64_t n_head, int64_t n_batch, int n_splits, const float * sinks);  // the row-parallel combine pass (prompt micro-batches)
 size_t fattn_vis_bytes(const tdesc & q, const tdesc & k);

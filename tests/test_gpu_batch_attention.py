@@ -491,3 +491,94 @@ def test_few_tokens_over_runs_of_cells(backend, H, T_, NKV, G, per, first):
             ref = v[h // G][:, see].astype(np.float64) @ p
             # (as test_few_tokens_on_matrix_cores)
             assert np.abs(got[h, t] - ref).max() <= 2e-3 * np.abs(ref).max() + 1e-5, (t, h)
+
+
+# one launch over a short cache (attn_nf_once: 16 and 32 columns a workgroup, pairs and single heads, one, two and four blocks a wave) and two passes behind it; ragged batches, a last block in part
+@pytest.mark.parametrize("HD,NH,NKV,T_,n_kv", [
+    (128, 8, 2, 33, 40), (128, 8, 2, 77, 256), (128, 7, 1, 45, 264), (128, 4, 4, 129, 512), (128, 8, 2, 250, 520), (128, 14, 2, 130, 1024), (128, 4, 2, 257, 768),
+    (64, 8, 1, 33, 48), (64, 8, 2, 128, 512), (64, 6, 2, 140, 1000), (64, 3, 1, 65, 256), (64, 8, 2, 70, 1032), (64, 4, 1, 300, 1024)])
+@pytest.mark.parametrize("mask_kind", ["causal", "scattered"])
+def test_prompt_over_a_short_cache(backend, H, HD, NH, NKV, T_, n_kv, mask_kind):
+    """K.q -> SOFT_MAX -> V^T.p -> CONT of a prompt's batch; cells that no query sees hold infinities and NaN (whole blocks of 64 of them: such blocks are not multiplied), one query sees nothing: NaN.
+    Against float64 with the chain's two f16 roundings, as test_few_tokens_on_matrix_cores."""
+    rng = np.random.default_rng(HD + NH + T_ + n_kv)
+    G = NH // NKV
+    k = rng.standard_normal((n_kv, NKV, HD)).astype(np.float16)
+    v = rng.standard_normal((NKV, HD, n_kv)).astype(np.float16)
+    q = (2 * rng.standard_normal((T_, NH, HD))).astype(np.float32)
+    mask = np.full((T_, n_kv), -np.inf, np.float32)
+    for t in range(T_):
+        if mask_kind == "causal":
+            mask[t, :max(1, n_kv - T_ + t + 1 - 8)] = 0
+        else:
+            mask[t, rng.random(n_kv) < 0.2] = -0.5 * (t % 3)
+            mask[t, t % 8] = 0
+            if n_kv > 200:
+                mask[t, 64:128] = -np.inf
+    mask[T_ // 2] = -np.inf
+    if mask_kind == "scattered" and n_kv > 200:
+        k[64:128], v[:, :, 64:128] = np.inf, np.nan
+
+    def build(g):
+        kc, vc = g.new(L.F16, [NKV * HD, n_kv], k.reshape(n_kv, -1)), g.new(L.F16, [n_kv, NKV * HD], v.reshape(-1, n_kv))
+        qp = H.ggml_permute(g.ctx, g.new(L.F32, [HD, NH, T_], q), 0, 2, 1, 3)
+        kv = H.ggml_view_3d(g.ctx, kc, HD, n_kv, NKV, NKV * HD * 2, HD * 2, 0)
+        vv = H.ggml_view_3d(g.ctx, vc, n_kv, HD, NKV, n_kv * 2, n_kv * 2 * HD, 0)
+        p = H.ggml_soft_max_ext(g.ctx, H.ggml_mul_mat(g.ctx, kv, qp), g.new(L.F32, [n_kv, T_], mask), HD ** -0.5, 0.0)
+        return H.ggml_cont_2d(g.ctx, H.ggml_permute(g.ctx, H.ggml_mul_mat(g.ctx, vv, p), 0, 2, 1, 3), HD * NH, T_)
+
+    k0, c0 = backend.stat("kernel_launches"), backend.stat("nf_mma_chains")
+    got = T.run_case(build, backend)[0].reshape(T_, NH, HD)
+    launches = backend.stat("kernel_launches") - k0
+    once = n_kv <= (1024 if HD == 64 or T_ <= 256 else 512)
+    assert backend.stat("nf_mma_chains") - c0 == 1 and (launches == 1 if once else launches in (3, 4)), launches
+    qh = q.astype(np.float16).astype(np.float64)
+    for t in range(T_):
+        see = np.flatnonzero(mask[t] > -1e30)
+        if len(see) == 0:
+            assert np.isnan(got[t]).all()
+            continue
+        kt, vt = k[see].astype(np.float64), v[:, :, see].astype(np.float64)
+        for h in range(NH):
+            s = kt[:, h // G] @ qh[t, h] * HD ** -0.5 + mask[t, see]
+            p = np.exp(s - s.max())
+            p = (p / p.sum()).astype(np.float16).astype(np.float64)
+            ref = vt[h // G] @ p
+            assert np.abs(got[t, h] - ref).max() <= 2e-3 * np.abs(ref).max() + 1e-5, (t, h)
+
+
+@pytest.mark.parametrize("recycled", [False, True])
+@pytest.mark.parametrize("NH,NKV,T_", [(8, 2, 41), (8, 2, 160), (6, 2, 50)])
+def test_prompt_over_a_short_cache_feeds_a_quantised_matrix(backend, H, NH, NKV, T_, recycled):
+    """the same into a K-quant product: head pairs of a group leave as Q8_K blocks, an odd group's rows as the copy; only a Q8_K code next to a rounding boundary may differ from the graph run node by node"""
+    rng = np.random.default_rng(NH + T_)
+    HD, n_kv, N = 128, 256, 96
+    k, v = rng.standard_normal((n_kv, NKV * HD)).astype(np.float16), rng.standard_normal((NKV * HD, n_kv)).astype(np.float16)
+    wq, x = T.rand_weight(L.Q4_K, 256, NH * HD, rng), rng.standard_normal((T_, 256)).astype(np.float32)
+    wo = T.rand_weight(L.Q4_K, NH * HD, N, rng)
+    mask = np.where(np.arange(n_kv)[None, :] <= 30 + np.arange(T_)[:, None], 0, -np.inf).astype(np.float32)
+
+    def run():
+        g = T.G(backend)
+        try:
+            q = H.ggml_mul_mat(g.ctx, g.new(L.Q4_K, [256, NH * HD], wq), g.new(L.F32, [256, T_], x))
+            qp = H.ggml_permute(g.ctx, H.ggml_reshape_3d(g.ctx, q, HD, NH, T_), 0, 2, 1, 3)
+            kv = H.ggml_view_3d(g.ctx, g.new(L.F16, [NKV * HD, n_kv], k), HD, n_kv, NKV, NKV * HD * 2, HD * 2, 0)
+            vv = H.ggml_view_3d(g.ctx, g.new(L.F16, [n_kv, NKV * HD], v), n_kv, HD, NKV, n_kv * 2, n_kv * 2 * HD, 0)
+            p = H.ggml_soft_max_ext(g.ctx, H.ggml_mul_mat(g.ctx, kv, qp), g.new(L.F32, [n_kv, T_], mask), HD ** -0.5, 0.0)
+            o = H.ggml_cont_2d(g.ctx, H.ggml_permute(g.ctx, H.ggml_mul_mat(g.ctx, vv, p), 0, 2, 1, 3), NH * HD, T_)
+            r = H.ggml_mul_mat(g.ctx, g.new(L.Q4_K, [NH * HD, N], wo), o)
+            c0 = backend.stat("nf_mma_chains")
+            out = g.compute([r], same_block=[(o, q)] if recycled else [])[0]
+            return out, backend.stat("nf_mma_chains") - c0
+        finally:
+            g.free()
+
+    got, chains = run()
+    backend.set_option("fusion", 0)
+    try:
+        plain, plain_chains = run()
+    finally:
+        backend.set_option("fusion", 1)
+    assert chains == 1 and plain_chains == 0
+    assert T.nmse(got, plain) <= 1e-5
