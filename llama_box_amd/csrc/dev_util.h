@@ -148,6 +148,24 @@ template <typename Q8K> __device__ __forceinline__ void wave_quantize_q8_K(const
     }
 }
 
+// four neighbouring sums of ks >= 1 partial products, mn floats apart, added in their order; the loads of four are in flight together
+__device__ __forceinline__ float4 splitk_sum4(const float * part, const int64_t mn, const int ks) {
+    float4 acc;
+    for (int k = 0; k < ks; k += 4) {
+        float4 p[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (k + u < ks) p[u] = *(const float4 *) (part + (int64_t) (k + u) * mn);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            if (k + u >= ks) break;
+            if (k + u == 0) acc = p[0];
+            else { acc.x += p[u].x; acc.y += p[u].y; acc.z += p[u].z; acc.w += p[u].w; }
+        }
+    }
+    return acc;
+}
+
 // rotary-embedding angle for pair `ip` of a token at position pos_f: the same chain of f32 multiplies as ggml-cpu's
 // rope cache loop (theta *= theta_scale per pair), then the YaRN mix and the accurate cosf/sinf
 struct rope_consts {

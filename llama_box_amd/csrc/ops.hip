@@ -1860,17 +1860,29 @@ __global__ void __launch_bounds__(256) k_rope_qk_store(const rope_store_args a) 
 // rotation: two adjacent pairs) or 4 + 4 dims half a head apart (NeoX) — of every query / key / value head; ALL of a thread's loads are
 // requested first (the per-slot loop above waits one L2 round trip per head slot: 14 us for 512 tokens of Llama-3-8B against 23 MB of traffic),
 // and (cos, sin) come from the per-graph-run table of k_rope_table (the chain of multiplies and the accurate cosf / sinf once per run, not once
-// per layer).  Requires: whole heads rotated (n_dims == head_dim), head_dim % 8 == 0, projections in memory (no split-K partials); the V cache row-major, or transposed with llama.cpp's per-element indices (non-flash path).
+// per layer).  Requires: whole heads rotated (n_dims == head_dim), head_dim % 8 == 0; the V cache row-major, or transposed with llama.cpp's per-element indices (non-flash path).
 // The arithmetic per element is that of k_rope_qk_store (x0 cs - x1 sn, x0 sn + x1 cs; f2h for the cache rows).
-template <bool NEOX, bool Q8>
+// SKP: projections may be left as split-K partial products, summed here in k_splitk_reduce's order; a thread takes ONE chunk then and blockIdx.y the chunks of a token, so that all partial
+// sums of a chunk are one round trip (77 tokens of Llama-3-8B: 9.2 us a launch of k_rope_qk_store, 6.5 here).
+template <bool NEOX, bool Q8, bool SKP>
 __global__ void __launch_bounds__(256) k_rope_qk_store_vec(const rope_store_args a, const float * __restrict__ tab) {
     const int64_t t = blockIdx.x;
     const int tid = threadIdx.x, hd = a.head_dim, half = hd >> 1;
     const int64_t row = a.idx[t];
     const int cph = NEOX ? hd / 8 : hd / 4;            // chunks per head
     const int n_rot = (a.nh + a.nkv) * cph, n_v = a.nkv * (hd / 4);
-    constexpr int MAXC = 6;                            // chunks per thread and pass (Llama-3-8B: 1280 rotated chunks -> 5, + 1 value chunk)
-    for (int c0 = 0; c0 < n_rot + n_v; c0 += 256 * MAXC) {
+    constexpr int MAXC = SKP ? 1 : 6;                  // chunks per thread and pass (Llama-3-8B: 1280 rotated chunks -> 5, + 1 value chunk)
+    // four neighbouring values of head h of source sidx (0 q, 1 k, 2 v)
+    auto ld4 = [&](const int sidx, const float * src, const int h, const int i) -> float4 {
+        if (!SKP || a.sk[sidx].part == nullptr) return *(const float4 *) (src + i);
+        const int e = h * hd + i;
+        float4 b;
+        if (a.sk[sidx].bias) b = *(const float4 *) (a.sk[sidx].bias + e);
+        float4 v = splitk_sum4(a.sk[sidx].part + t * a.sk[sidx].n + e, a.sk[sidx].mn, a.ks);
+        if (a.sk[sidx].bias) { v.x += b.x; v.y += b.y; v.z += b.z; v.w += b.w; }
+        return v;
+    };
+    for (int c0 = SKP ? (int) blockIdx.y * 256 : 0; c0 < n_rot + n_v; c0 += 256 * MAXC * (SKP ? (int) gridDim.y : 1)) {
         float4 lo[MAXC], hi[MAXC], cs[MAXC], cs2[MAXC];
 #pragma unroll
         for (int k = 0; k < MAXC; ++k) {
@@ -1878,17 +1890,18 @@ __global__ void __launch_bounds__(256) k_rope_qk_store_vec(const rope_store_args
             if (c < n_rot) {
                 const int slot = c / cph, j = c - slot * cph;
                 const float * src = slot < a.nh ? (const float *) (a.q_src + (int64_t) slot * a.q_nb1 + t * a.q_nb2) : (const float *) (a.k_src + (int64_t) (slot - a.nh) * a.k_nb1 + t * a.k_nb2);
-                lo[k] = *(const float4 *) (src + 4 * j);
                 if (NEOX) {
-                    hi[k] = *(const float4 *) (src + half + 4 * j);
                     cs[k] = *(const float4 *) (tab + ((size_t) t * half + 4 * j) * 2);       // pairs 4j, 4j + 1
                     cs2[k] = *(const float4 *) (tab + ((size_t) t * half + 4 * j + 2) * 2);  // pairs 4j + 2, 4j + 3
                 } else {
                     cs[k] = *(const float4 *) (tab + ((size_t) t * half + 2 * j) * 2);       // pairs 2j, 2j + 1
                 }
+                const int sidx = slot < a.nh ? 0 : 1, h = slot < a.nh ? slot : slot - a.nh;
+                lo[k] = ld4(sidx, src, h, 4 * j);
+                if (NEOX) hi[k] = ld4(sidx, src, h, half + 4 * j);
             } else if (c < n_rot + n_v) {
                 const int cv = c - n_rot, h = cv / (hd / 4), j = cv - h * (hd / 4);
-                lo[k] = *(const float4 *) ((const float *) (a.v_src + (int64_t) h * a.v_nb1 + t * a.v_nb2) + 4 * j);
+                lo[k] = ld4(2, (const float *) (a.v_src + (int64_t) h * a.v_nb1 + t * a.v_nb2), h, 4 * j);
             }
         }
 #pragma unroll
@@ -1938,21 +1951,27 @@ __global__ void __launch_bounds__(256) k_rope_qk_store_vec(const rope_store_args
 }
 bool rope_qk_store_vec_ok(const rope_store_args & a, int n_tokens) {
     static const bool on = !getenv("GGML_MI355X_ROPE_VEC") || atoi(getenv("GGML_MI355X_ROPE_VEC")) != 0;
-    if (!on || n_tokens < 33 || a.ks > 1 || a.sk[0].part || a.sk[1].part || a.sk[2].part) return false;
+    if (!on || n_tokens < 33) return false;
     if ((a.p.mode & ~GGML_ROPE_TYPE_NEOX) != 0 || a.p.n_dims != a.head_dim || (a.head_dim % 8) != 0) return false;
     auto al16 = [](const void * p) { return (((uintptr_t) p) & 15) == 0; };
     if (!al16(a.q_src) || !al16(a.q_dst) || !al16(a.k_src) || !al16(a.v_src) || (!a.k_q8 && !al16(a.k_cache)) || (!a.v_q8 && !al16(a.v_cache))) return false;
     for (int64_t v : {a.q_nb1, a.q_nb2, a.qd_nb1, a.qd_nb2, a.k_nb1, a.k_nb2, a.v_nb1, a.v_nb2})
         if (v % 16) return false;
+    for (const auto & sk : a.sk)
+        if (sk.part && (!al16(sk.part) || !al16(sk.bias) || (sk.mn % 4) || (sk.n % 4))) return false;
     return (a.k_q8 || (a.kc_nb1 % 8) == 0) && (a.v_idx != nullptr || a.v_q8 || (a.vc_nb1 % 8) == 0);
 }
 void launch_rope_qk_store_vec(hipStream_t s, const rope_store_args & a, int n_tokens, const float * tab) {
     const bool neox = (a.p.mode & GGML_ROPE_TYPE_NEOX) != 0, q8 = a.k_q8 || a.v_q8;
-    const dim3 grid((unsigned) n_tokens), block(256);
-    if (neox && q8) hipLaunchKernelGGL((k_rope_qk_store_vec<true, true>), grid, block, 0, s, a, tab);
-    else if (neox) hipLaunchKernelGGL((k_rope_qk_store_vec<true, false>), grid, block, 0, s, a, tab);
-    else if (q8) hipLaunchKernelGGL((k_rope_qk_store_vec<false, true>), grid, block, 0, s, a, tab);
-    else hipLaunchKernelGGL((k_rope_qk_store_vec<false, false>), grid, block, 0, s, a, tab);
+    const bool skp = a.sk[0].part || a.sk[1].part || a.sk[2].part;
+    const int chunks = (a.nh + a.nkv) * (a.head_dim / (neox ? 8 : 4)) + a.nkv * (a.head_dim / 4);
+    const dim3 grid((unsigned) n_tokens, skp ? (unsigned) ((chunks + 255) / 256) : 1u), block(256);
+#define ROPE_VEC(N, Q) { if (skp) hipLaunchKernelGGL((k_rope_qk_store_vec<N, Q, true>), grid, block, 0, s, a, tab); else hipLaunchKernelGGL((k_rope_qk_store_vec<N, Q, false>), grid, block, 0, s, a, tab); }
+    if (neox && q8) ROPE_VEC(true, true)
+    else if (neox) ROPE_VEC(true, false)
+    else if (q8) ROPE_VEC(false, true)
+    else ROPE_VEC(false, false)
+#undef ROPE_VEC
 }
 void launch_rope_qk_store(hipStream_t s, rope_store_args a, int n_tokens) {
     rope_host_consts(a.p, a.theta_scale, a.corr0, a.corr1);

@@ -1465,6 +1465,55 @@ def test_batch_rope_and_cache_stores_one_launch(backend, H, plog, mode, n_dims, 
                   max_nmse=1e-6 if name != "q_rope" else 1e-10, log=plog)
 
 
+# projections of a short prompt left as K slices' partial sums: neighbouring pairs and halves, biases, f16 / Q8_0 / transposed cache rows, chunks of a token that end inside a workgroup; 32 tokens: below the vectorised form
+@pytest.mark.parametrize("M,mode,NH,NKV,HD,bias,store", [(33, 0, 8, 2, 128, False, "rows"), (77, 0, 32, 8, 128, False, "transposed"), (50, L.ROPE_NEOX, 28, 4, 128, True, "rows"), (130, 0, 6, 2, 64, True, "q8"),
+                                                         (96, L.ROPE_NEOX, 12, 4, 64, False, "q8"), (40, 0, 6, 3, 128, True, "transposed")])
+def test_rope_and_stores_over_partial_sums(backend, H, plog, M, mode, NH, NKV, HD, bias, store):
+    rng = np.random.default_rng(M + NH)
+    E, NCTX, tq = 2048, M + 40, L.Q4_K
+    x = rng.standard_normal((M, E)).astype(np.float32)
+    N = (NH * HD, NKV * HD, NKV * HD)
+    w = [T.rand_weight(tq, E, n, rng) for n in N]
+    b = [rng.standard_normal(n).astype(np.float32) for n in N]
+    pos = rng.integers(0, 5000, M).astype(np.int32)
+    rows = rng.permutation(NCTX)[:M].astype(np.int64)
+    kvt = L.Q8_0 if store == "q8" else L.F16
+    c0 = np.zeros((NCTX, NKV * HD // 32 * 34), np.uint8) if store == "q8" else np.zeros((NCTX, NKV * HD), np.float16)
+    v_idx = (np.arange(NKV * HD, dtype=np.int64)[None, :] * NCTX + rows[:, None]).reshape(-1)
+
+    def build(g):
+        cur = g.new(L.F32, [E, M], x)
+        q, k, v = (H.ggml_mul_mat(g.ctx, g.new(tq, [E, n], m), cur) for n, m in zip(N, w))
+        if bias:
+            q, k, v = (H.ggml_add(g.ctx, y, g.new(L.F32, [n], z)) for y, n, z in zip((q, k, v), N, b))
+        tp, idx = g.new(L.I32, [M], pos), g.new(L.I64, [M], rows)
+        q = H.ggml_rope_ext(g.ctx, H.ggml_reshape_3d(g.ctx, q, HD, NH, M), tp, None, HD, mode, 8192, 500000.0, 1.0, 0.0, 1.0, 32.0, 1.0)
+        k = H.ggml_rope_ext(g.ctx, H.ggml_reshape_3d(g.ctx, k, HD, NKV, M), tp, None, HD, mode, 8192, 500000.0, 1.0, 0.0, 1.0, 32.0, 1.0)
+        ks = H.ggml_set_rows(g.ctx, g.new(kvt, [NKV * HD, NCTX], c0), H.ggml_reshape_2d(g.ctx, k, NKV * HD, M), idx)
+        if store == "transposed":
+            view = H.ggml_reshape_2d(g.ctx, g.new(L.F16, [NCTX, NKV * HD], np.zeros((NKV * HD, NCTX), np.float16)), 1, NCTX * NKV * HD)
+            vs = H.ggml_set_rows(g.ctx, view, H.ggml_reshape_2d(g.ctx, v, 1, M * NKV * HD), g.new(L.I64, [M * NKV * HD], v_idx))
+        else:
+            vs = H.ggml_set_rows(g.ctx, g.new(kvt, [NKV * HD, NCTX], c0), v, idx)
+        return [q, ks, vs]
+
+    ref = T.run_case(build, "oracle", expand_first=())
+    k0 = backend.stat("kernel_launches")
+    got = T.run_case(build, backend)
+    assert backend.stat("kernel_launches") - k0 == 4  # quantiser, products, (cos, sin) table, rotation with both stores
+
+    def values(a):
+        a = np.asarray(a)
+        if store != "q8" or a.dtype == np.float32:
+            return a.astype(np.float32)
+        blk = a.reshape(-1).view(np.uint8).reshape(-1, 34)
+        return blk[:, :2].copy().view(np.float16).astype(np.float32) * blk[:, 2:].view(np.int8)
+
+    for name, a, r in zip(("q_rope", "k_cache", "v_cache"), got, ref):
+        # (f32 sums in another order than the oracle's; f16 and 8-bit rows: a value next to a rounding boundary)
+        T.compare(f"rope + stores over partial sums M={M} {store}: {name}", values(a), values(r), max_nmse=1e-10 if name == "q_rope" else 1e-6, log=plog)
+
+
 @pytest.mark.parametrize("T_", [32, 130, 512])
 def test_batch_rope_and_transposed_v_store_one_launch(backend, H, plog, T_):
     """The same window on the non-flash path: the V store is a scatter of single elements into the transposed cache (an index per element)."""
