@@ -241,26 +241,42 @@ __global__ void __launch_bounds__(256) k_attn_f32_rows(const tdesc q, const tdes
 // the merge of k_attn_f32_rows' partial records: one workgroup per (token, head).  gate (may be null): the output is multiplied by sigmoid(gate), one number per head or per entry
 __global__ void __launch_bounds__(128) k_attn_f32_combine(const float * __restrict__ parts, const int S, const int H, const int DV, const tdesc dst, const int sgm, const float * __restrict__ gate,
                                                           const int gate_heads) {
-    __shared__ float cw[ATTN_F32_MAX_SPLITS];
-    const int64_t t = blockIdx.x, h = blockIdx.y;
-    const float * rec = parts + (t * H + h) * S * (int64_t) (DV + 2);
-    float M = rec[0];
-    for (int s = 1; s < S; ++s) M = fmaxf(M, rec[s * (int64_t) (DV + 2)]);
-    float L = 0.0f;
-    for (int s = 0; s < S; ++s) {
-        const float c = expf(rec[s * (int64_t) (DV + 2)] - M);
-        if (threadIdx.x == 0) cw[s] = c;
-        L += rec[s * (int64_t) (DV + 2) + 1] * c;
+    // Lane s of each wave holds split s's (maximum, sum); they, the values of the first eight splits and the gate are requested together.  (One after the other, a round trip a split: 2 tokens x 16 heads
+    // in 8 splits 6.0 us a launch; so 4.4.)
+    static_assert(ATTN_F32_MAX_SPLITS <= 64, "a lane a split");
+    const int64_t t = blockIdx.x, h = blockIdx.y, DR = DV + 2;
+    const int lane = threadIdx.x & 63;
+    const float * rec = parts + (t * H + h) * S * DR;
+    const float ms = lane < S ? rec[lane * DR] : -INFINITY, ls = lane < S ? rec[lane * DR + 1] : 0.0f;
+    float v[8], gt = 0.0f;
+    auto request = [&](const int d, const int s0) {
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = rec[min(s0 + u, S - 1) * DR + 2 + d];
+    };
+    if ((int) threadIdx.x < DV) {
+        request(threadIdx.x, 0);
+        if (gate) gt = gate[gate_heads ? t * H + h : (t * H + h) * DV + threadIdx.x];
     }
-    __syncthreads();
+    const float M = wave_max(ms), c = expf(ms - M), lc = ls * c;
+    float L = 0.0f;
+    for (int s = 0; s < S; ++s) L += readlane_f32(lc, s);
     const float inv = sgm ? 1.0f : (L > 0.0f ? 1.0f / L : 0.0f);
     float * out = (float *) (dst.data + h * dst.nb[1] + t * dst.nb[2]);
-    for (int d = threadIdx.x; d < DV; d += 128) {
+    for (int d0 = 0; d0 < DV; d0 += 128) {  // (whole waves stay: the coefficients come out of their lanes)
+        const int d = d0 + (int) threadIdx.x, dl = min(d, DV - 1);
         float o = 0.0f;
-        for (int s = 0; s < S; ++s) o += rec[s * (int64_t) (DV + 2) + 2 + d] * cw[s];
+        for (int s0 = 0; s0 < S; s0 += 8) {
+            if (d0 > 0 || s0 > 0) request(dl, s0);
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+                if (s0 + u < S) o += v[u] * readlane_f32(c, s0 + u);
+        }
         o = o * inv;
-        if (gate) o = o * (1.f / (1.f + expf(-gate[gate_heads ? t * H + h : (t * H + h) * DV + d])));
-        out[d] = o;
+        if (gate) {
+            if (d0 > 0) gt = gate[gate_heads ? t * H + h : (t * H + h) * DV + dl];
+            o = o * (1.f / (1.f + expf(-gt)));
+        }
+        if (d < DV) out[d] = o;
     }
 }
 

@@ -268,6 +268,16 @@ def test_attention_alone(backend, H, kv_type, n_q, n_kv, heads, kv_heads, dk, dv
     assert np.abs(got - ref).max() <= 2e-5 * max(1.0, np.abs(ref).max())
 
 
+# records of 2, 8, 9, 20 and 32 splits (one for 256 cells), value rows on both sides of the merge's 128 threads, splits without a visible cell
+@pytest.mark.parametrize("n_q,n_kv,heads,kv_heads,dv,chunk,sink", [
+    (2, 300, 16, 4, 128, 0, True), (1, 2048, 3, 1, 40, 0, False), (1, 2049, 2, 2, 129, 0, True), (2, 5000, 2, 1, 256, 500, True), (1, 9000, 1, 1, 200, 0, False), (3, 700, 5, 5, 1, 64, True)])
+def test_merge_of_split_records(backend, H, n_q, n_kv, heads, kv_heads, dv, chunk, sink):
+    rng = np.random.default_rng(n_kv + dv)
+    q, k, v = (rng.standard_normal(z).astype(np.float32) for z in ((n_q, heads, 64), (n_kv, kv_heads, 64), (n_kv, kv_heads, dv)))
+    got, ref = attention_case(backend, H, L.F32, n_q, n_kv, heads, kv_heads, 64, dv, chunk, sink, q, k, v, np.arange(n_kv - n_q, n_kv))
+    assert np.abs(got - ref).max() <= 2e-5 * max(1.0, np.abs(ref).max())  # (as test_attention_alone: f32 sums of thousands of terms, each to 2^-24)
+
+
 @pytest.mark.parametrize("n_q", [1, 40])
 def test_a_far_key_a_chunk_edge_and_the_sink_show(backend, H, n_q):
     """bf16 cache, one key made to dominate: the output is that key's value row when the rule lets the query see it, and not when it lies one position
