@@ -2329,6 +2329,15 @@ struct graph_key {
     bool operator==(const graph_key & o) const { return n_tokens == o.n_tokens && n_kv == o.n_kv && n_outputs == o.n_outputs && n_seqs == o.n_seqs; }
 };
 
+// a graph and the tensors of it that the host fills and reads
+struct built_graph {
+    graph_key key;
+    ggml_context * ctx = nullptr;
+    ggml_cgraph * gf = nullptr;
+    seg_io io;
+    uint64_t used = 0;
+};
+
 struct llm_context {
     llm_model * model = nullptr;
     ggml_backend_t backend = nullptr;
@@ -2353,9 +2362,13 @@ struct llm_context {
     int used_max = 0;           // one past the highest occupied cell; < 0: unknown (cells were freed), recounted by the next batch
     // compute graph
     ggml_gallocr_t galloc = nullptr;
-    ggml_context * ctx_compute = nullptr;
     ggml_cgraph * gf = nullptr;
     graph_key key;
+    // the graphs of the shapes used last, all of them laid out in galloc's one buffer: the micro-batches of one prompt after the other come round to the same few (building one took 9 us a layer,
+    // in front of a prompt's first micro-batch with the GPU idle: 700 tokens of a 22-layer model in two micro-batches 5625 us, 5425 with its graphs kept; 8 graphs take a few MB of host memory)
+    static constexpr size_t GRAPHS_KEPT = 8;
+    std::vector<built_graph> built;
+    uint64_t graph_tick = 0;
     ggml_tensor *inp_tokens = nullptr, *inp_pos = nullptr, *inp_mask = nullptr, *inp_k_idxs = nullptr, *inp_v_idxs = nullptr, *inp_out_ids = nullptr;
     ggml_tensor *inp_bigram = nullptr, *inp_shift_src = nullptr, *inp_shift_last = nullptr, *inp_shift_slot = nullptr;
     ggml_tensor *inp_seq_hist = nullptr, *inp_seq_upd = nullptr, *inp_seq_tok = nullptr, *inp_seq_info = nullptr;
@@ -3251,14 +3264,19 @@ static void build_layerwise(llm_context * c, ggml_context * ctx, ggml_cgraph * g
     io.out = cur;
 }
 
-static void build_graph(llm_context * c, int n_tokens, int n_kv, int n_outputs, int n_seqs = 0) {
-    if (c->ctx_compute) ggml_free(c->ctx_compute);
-    c->ctx_compute = ggml_init({0, nullptr, true});
-    ggml_cgraph * gf = ggml_new_graph_custom(c->ctx_compute, 8192, false);
-    seg_io io;
-    make_inputs(c, c->ctx_compute, 0, c->model->hp.n_layer, true, n_tokens, n_kv, n_outputs, io, n_seqs);
-    if (!c->model->lcfg.empty()) build_layerwise(c, c->ctx_compute, gf, n_tokens, n_kv, io);
-    else build_segment(c, c->ctx_compute, gf, 0, c->model->hp.n_layer, true, n_tokens, n_kv, io);
+static built_graph build_graph(llm_context * c, const graph_key & key) {
+    built_graph b;
+    b.key = key;
+    b.ctx = ggml_init({0, nullptr, true});
+    b.gf = ggml_new_graph_custom(b.ctx, 8192, false);
+    make_inputs(c, b.ctx, 0, c->model->hp.n_layer, true, key.n_tokens, key.n_kv, key.n_outputs, b.io, key.n_seqs);
+    if (!c->model->lcfg.empty()) build_layerwise(c, b.ctx, b.gf, key.n_tokens, key.n_kv, b.io);
+    else build_segment(c, b.ctx, b.gf, 0, c->model->hp.n_layer, true, key.n_tokens, key.n_kv, b.io);
+    return b;
+}
+static void use_graph(llm_context * c, built_graph & b) {
+    const seg_io & io = b.io;
+    b.used = ++c->graph_tick;
     c->inp_masks = io.masks;
     c->inp_q_temps = io.q_temps;
     c->inp_tokens = io.tokens;
@@ -3276,7 +3294,39 @@ static void build_graph(llm_context * c, int n_tokens, int n_kv, int n_outputs, 
     c->inp_seq_tok = io.seq_tok;
     c->inp_seq_info = io.seq_info;
     c->t_logits = io.out;
-    c->gf = gf;
+    c->gf = b.gf;
+    c->key = b.key;
+}
+static void drop_graph(llm_context * c, size_t i) {
+    if (c->built[i].gf == c->gf) {
+        c->gf = nullptr;
+        c->key = graph_key();
+    }
+    ggml_free(c->built[i].ctx);
+    c->built.erase(c->built.begin() + (ptrdiff_t) i);
+}
+// makes the graph of this shape the current one
+static bool switch_graph(llm_context * c, const graph_key & key) {
+    if (c->p.graph_reuse)
+        for (built_graph & b : c->built)
+            if (b.key == key) {
+                use_graph(c, b);
+                return true;
+            }
+    while (c->built.size() >= (c->p.graph_reuse ? llm_context::GRAPHS_KEPT : 1))
+        drop_graph(c, (size_t) (std::min_element(c->built.begin(), c->built.end(), [](const built_graph & x, const built_graph & y) { return x.used < y.used; }) - c->built.begin()));
+    built_graph b = build_graph(c, key);
+    const size_t size = ggml_gallocr_get_buffer_size(c->galloc, 0);
+    const bool ok = ggml_gallocr_alloc_graph(c->galloc, b.gf);
+    if (!ok || ggml_gallocr_get_buffer_size(c->galloc, 0) != size)  // (the buffer that the other graphs lie in is gone)
+        while (!c->built.empty()) drop_graph(c, c->built.size() - 1);
+    if (!ok) {
+        ggml_free(b.ctx);
+        return false;
+    }
+    c->built.push_back(std::move(b));
+    use_graph(c, c->built.back());
+    return true;
 }
 
 // the second copies that the device's kernels for batches of a few columns read are made with the context, not in front of the first such batch
@@ -3401,14 +3451,15 @@ extern "C" struct llm_context * llm_context_new(struct llm_model * m, ggml_backe
     c->used_max = 0;
     c->galloc = ggml_gallocr_new(c->buft);
     // reserve the worst-case graph (full micro-batch over the full cache) so later graphs re-use one buffer
-    build_graph(c, std::min(c->p.n_ubatch, c->p.n_ctx), c->p.n_ctx, std::min(c->p.n_ubatch, c->p.n_ctx),
-                (m->has_shift || m->has_seq_state) ? std::min(c->n_seq_max, std::min(c->p.n_ubatch, c->p.n_ctx)) : 0);
+    const int n_most = std::min(c->p.n_ubatch, c->p.n_ctx);
+    c->built.push_back(build_graph(c, {n_most, c->p.n_ctx, n_most, (m->has_shift || m->has_seq_state) ? std::min(c->n_seq_max, n_most) : 0}));
+    use_graph(c, c->built[0]);
     if (!ggml_gallocr_reserve(c->galloc, c->gf)) {
         fprintf(stderr, "llm_context_new: failed to reserve the compute buffer\n");
         llm_context_free(c);
         return nullptr;
     }
-    c->key = graph_key();
+    c->key = c->built[0].key = graph_key();  // (measured, not laid out)
     if (backend) {
         ggml_backend_buffer_type_t hbuft = ggml_backend_dev_host_buffer_type(backend->device);
         if (hbuft) {
@@ -3448,7 +3499,7 @@ extern "C" void llm_context_free(struct llm_context * c) {
         if (d.buf_kv) ggml_backend_buffer_free(d.buf_kv);
         if (d.ctx_kv) ggml_free(d.ctx_kv);
     }
-    if (c->ctx_compute) ggml_free(c->ctx_compute);
+    for (built_graph & b : c->built) ggml_free(b.ctx);
     if (c->galloc) ggml_gallocr_free(c->galloc);
     for (ggml_backend_event_t e : c->pin_ev)
         if (e) ggml_backend_event_free(e);
@@ -3810,9 +3861,7 @@ static int decode_ubatch(llm_context * c, int n_tokens, const int32_t * tokens, 
     bool rebuilt = false;
     if (!(c->p.graph_reuse && key == c->key && c->gf)) {
         rebuilt = true;
-        build_graph(c, n_tokens, n_kv, n_out_graph, n_seqs);
-        if (!ggml_gallocr_alloc_graph(c->galloc, c->gf)) return -2;
-        c->key = key;
+        if (!switch_graph(c, key)) return -2;
     }
     const double t1 = now_us();
 

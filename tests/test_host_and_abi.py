@@ -192,6 +192,26 @@ def test_driver_on_oracle_determinism_reuse_and_batching(H):
         m.free()
 
 
+def test_graphs_of_several_shapes_are_kept(H):
+    """prompts of more shapes than a context keeps graphs for, in an order that meets kept, dropped and never built ones: the logits of a context that builds every graph anew"""
+    fn = T.oracle_compute_fn(2)
+    m = Model(preset("test-llama"), 5, H.ggml_backend_cpu_buffer_type())
+    kept, anew = Context(m, compute=fn, graph_reuse=1, n_ubatch=16), Context(m, compute=fn, graph_reuse=0, n_ubatch=16)
+    rng = np.random.default_rng(3)
+    for n in [3, 40, 1, 37, 3, 5, 6, 40, 7, 8, 9, 10, 11, 12, 3, 37, 1, 40, 12]:
+        tok = rng.integers(0, 500, n)
+        rows = []
+        for c in (kept, anew):
+            H.llm_kv_seq_rm(c.c, -1, 0, -1)
+            rc, lg = c.decode(tok, range(n), want=[0] * (n - 1) + [1])
+            assert rc == 0
+            rows.append(lg)
+        assert np.array_equal(*rows), n
+    kept.free()
+    anew.free()
+    m.free()
+
+
 @pytest.mark.parametrize("name,type_k", [("test-llama", 0), ("test-qwen2", 0), ("test-llama", L.Q8_0), ("test-llama", L.Q5_1), ("test-llama", L.Q4_0), ("test-llama", L.IQ4_NL), ("test-llama", -1)])
 def test_context_shift_k_shift_oracle(H, name, type_k):
     """llama-box context shift (httpserver.hpp:3453-3537): seq_rm of [n_keep, n_keep + n_discard) + seq_add of the rest by
