@@ -2141,6 +2141,23 @@ static int sole_cache_store_of(const exec_state & st, int i, const ggml_tensor *
 // ------------------------------------------------------------------------------------------------ fused steps of models with token shift / latent attention
 // elementwise result `d` written while `x` is read: legal when they are the same block (every thread reads its own element before it writes it) or apart
 static bool elementwise_safe(const ggml_tensor * d, const ggml_tensor * x) { return d->data == x->data || !ranges_overlap(d, x); }
+// the activation that alone reads product i, in the nodes right behind it (the erf form of GELU, or RELU -> SQR): how many nodes, and which.  Its rows may lie over the product's own, which nobody
+// else reads, but not over what the product still reads while the first sums are stored
+static int act_behind(const exec_state & st, int i, int & act) {
+    const ggml_cgraph * g = st.g;
+    const ggml_tensor * n = g->nodes[i], * u = i + 1 < g->n_nodes ? g->nodes[i + 1] : nullptr, * q = i + 2 < g->n_nodes ? g->nodes[i + 2] : nullptr;
+    if (!u || u->op != GGML_OP_UNARY || u->src[0] != n || st.done[i + 1] || !single_use(st, n)) return 0;
+    const ggml_tensor * out = u;
+    if (u->op_params[0] == GGML_UNARY_OP_GELU_ERF) act = GGML_UNARY_OP_GELU_ERF;
+    else if (u->op_params[0] == GGML_UNARY_OP_RELU && q && q->op == GGML_OP_SQR && q->src[0] == u && !st.done[i + 2] && single_use(st, u)) {
+        act = MI_UNARY_RELU_SQR;
+        out = q;
+    } else return 0;
+    bool ok = is_f32_contig(n) && is_f32_contig(out) && same_shape(out, n);
+    for (int s = 0; s < 3; ++s) ok = ok && !(n->src[s] && ranges_overlap(out, n->src[s]));
+    if (!ok) act = -1;
+    return ok ? (out == u ? 1 : 2) : 0;
+}
 static bool is_row_of(const ggml_tensor * b, const ggml_tensor * x) { return is_f32_contig(b) && b->ne[0] == x->ne[0] && ggml_abi_nelements(b) == b->ne[0]; }
 
 // CONCAT(h, state; dim 1) -> GET_ROWS(., src) -> SUB(., h) -> MUL(., w) -> ADD(h, .): the token shift in one launch.  Returns the nodes consumed (0: no match)
@@ -3003,9 +3020,12 @@ static int run_node(exec_state & st, int i) {
             }
             if (!is_quant(a->type)) {
                 timed_scope ts(c, "mul_mat_f", (double) ggml_abi_nbytes(a));
-                launch_mul_mat_f(s, TD(a), TD(b), TD(n), (float *) ((char *) c->ws + st.aux_off), c->ws ? c->ws_size - st.aux_off : 0);
+                int act = -1;
+                const int behind = fuse && mul_mat_f_takes_act(TD(a), TD(b)) ? act_behind(st, i, act) : 0;
+                launch_mul_mat_f(s, TD(a), TD(b), TD(g->nodes[i + behind]), (float *) ((char *) c->ws + st.aux_off), c->ws ? c->ws_size - st.aux_off : 0, act);
                 c->st.kernel_launches++;
-                return 1;
+                c->st.fused_nodes += behind;
+                return 1 + behind;
             }
             if (buffer_is_split(a->buffer)) {  // weights in the split buffer type (-sm row): split.cpp
                 const split_tensor_info * si = split_info(a);
@@ -3430,11 +3450,14 @@ static int run_node(exec_state & st, int i) {
             void * ws = (c->ws && st.aux_off + need <= c->ws_size) ? (char *) c->ws + st.aux_off : nullptr;
             timed_scope ts(c, "mul_mat_id", (double) ggml_abi_nbytes(a) / (double) std::max<int64_t>(1, a->ne[2]) * (double) std::min<int64_t>(a->ne[2], ggml_abi_nelements(ids)));
             const void * x16 = (ws && mm_id_tile_applies(n)) ? rounded_src1(st, b, a->type) : nullptr;
-            const bool grouped = launch_mul_mat_id(s, TD(a), TD(b), TD(ids), TD(n), ws, ws ? c->ws_size - st.aux_off : 0, valid && ws, x16);
+            int act = -1;
+            const int behind = fuse && !is_quant(a->type) && mul_mat_id_takes_act(TD(a), TD(b), TD(ids)) ? act_behind(st, i, act) : 0;
+            const bool grouped = launch_mul_mat_id(s, TD(a), TD(b), TD(ids), TD(g->nodes[i + behind]), ws, ws ? c->ws_size - st.aux_off : 0, valid && ws, x16, act);
             st.moe_ids = grouped ? ids : nullptr;  // (only a launch that made or used the lists vouches for them: the per-column forms leave the scratch alone)
             st.moe_node = grouped ? i : -1;
             c->st.kernel_launches++;
-            return 1;
+            c->st.fused_nodes += behind;
+            return 1 + behind;
         }
         case GGML_OP_GLU: {
             const tdesc bd = b ? TD(b) : TD(a);

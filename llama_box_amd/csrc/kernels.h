@@ -160,7 +160,8 @@ void launch_qkv(hipStream_t s, const qkv_args & a, int type_a, int type_b);
 
 // ---- f16 / f32 weights (K cache, V cache, small dense) (mmf.hip): dst = src0 · src1 with ggml broadcasting;
 // src1 rounded to f16 first when src0 is f16 (ggml-cpu vec_dot_type semantics)
-void launch_mul_mat_f(hipStream_t s, const tdesc & src0, const tdesc & src1, const tdesc & dst, float * ws = nullptr, size_t ws_bytes = 0);  // ws: scratch for K-split partial tiles
+void launch_mul_mat_f(hipStream_t s, const tdesc & src0, const tdesc & src1, const tdesc & dst, float * ws = nullptr, size_t ws_bytes = 0, int act = -1);  // ws: scratch for K-split partial tiles; act: GELU_ERF or MI_UNARY_RELU_SQR on the sums, where ...
+bool mul_mat_f_takes_act(const tdesc & src0, const tdesc & src1);  // ... this says so
 size_t mul_mat_f_workspace_bytes(const tdesc & src0, const tdesc & src1);
 // up to four bf16 matrices (rows of K values, 16-byte aligned) against ONE f32 column of K values (K a multiple of 8), one launch
 // a batch of M columns by up to four f16 / bf16 matrices of K columns, LDS-tiled (mmf_tile.hip); x16: the columns in the matrices' type, dense rows (launch_to_16; x rows 16-byte aligned)
@@ -185,7 +186,8 @@ void launch_mul_mat_bf16_multi(hipStream_t s, matvec_multi mm, const char * x, i
 // MUL_MAT_ID: as [K, N, n_expert] (f32 / f16 / bf16), b [K, 1 or n_used, T] f32, ids [n_used, T] i32 -> d [N, n_used, T].  ws: scratch for the
 // per-expert column lists of the batched form; lists_valid: an earlier call left the lists of these same ids there
 size_t mul_mat_id_workspace_bytes(const tdesc & as, const tdesc & ids);
-bool launch_mul_mat_id(hipStream_t s, const tdesc & as, const tdesc & b, const tdesc & ids, const tdesc & d, void * ws, size_t ws_bytes, bool lists_valid, const void * x16 = nullptr);  // x16: src1 in the experts' 16-bit type (mmf_tile.hip); true: the batched form ran and left the lists in ws
+bool mul_mat_id_takes_act(const tdesc & as, const tdesc & b, const tdesc & ids);
+bool launch_mul_mat_id(hipStream_t s, const tdesc & as, const tdesc & b, const tdesc & ids, const tdesc & d, void * ws, size_t ws_bytes, bool lists_valid, const void * x16 = nullptr, int act = -1);  // act: as launch_mul_mat_f; x16: src1 in the experts' 16-bit type (mmf_tile.hip); true: the batched form ran and left the lists in ws
 // MUL_MAT of ONE column / MUL_MAT_ID of few columns by a bf16 matrix whose operand is silu(g f) (u f) of rows gu [2 K, n_used, T] (f: one factor per row, or null)
 bool matvec_glu_ok(const tdesc & a, const void * gu, const tdesc * ids);
 void launch_matvec_glu(hipStream_t s, const tdesc & a, const float * gu, const float * f, const tdesc * ids, const tdesc & d);

@@ -267,8 +267,14 @@ template <int NWK, bool BF> __device__ __forceinline__ mmf_float4 mma16_tile(con
     }
     return acc;
 }
+// An activation on the sums of a few columns, where they are stored (graph.cpp: act_behind; k_unary's formulas): its own launch is 4 us with one value a thread in it.  Two sequences of a layered
+// model, four such launches a step: 376 us, 369 without them.
+__device__ __forceinline__ float mmf_act(const int act, const float v) {
+    if (act == MI_UNARY_RELU_SQR) return v > 0.f ? v * v : 0.f;
+    return act == GGML_UNARY_OP_GELU_ERF ? 0.5f * v * (1.0f + erff(v * 0.70710678118654752440f)) : v;
+}
 template <int NWK, bool BF>
-__global__ void __launch_bounds__(64 * NWK) k_mul_mat_f16_mma16(const tdesc a, const tdesc b, const tdesc d) {
+__global__ void __launch_bounds__(64 * NWK) k_mul_mat_f16_mma16(const tdesc a, const tdesc b, const tdesc d, const int act) {
     __shared__ mmf_float4 red[NWK][64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int r16 = lane & 15, kg = lane >> 4;
@@ -286,7 +292,7 @@ __global__ void __launch_bounds__(64 * NWK) k_mul_mat_f16_mma16(const tdesc a, c
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const int64_t col = col0 + 4 * kg + i;
-        if (col < b.ne[1]) *(float *) (out + col * d.nb[1]) = acc[i];
+        if (col < b.ne[1]) *(float *) (out + col * d.nb[1]) = mmf_act(act, acc[i]);
     }
 }
 // ... up to four bf16 matrices against the same 2 .. 16 columns in one launch (a step's q / k / v / gate projections: four launches of 8.7 us each, of which the weights'
@@ -466,7 +472,7 @@ __global__ void __launch_bounds__(256) k_mul_mat_f16_gqa_short(const tdesc a, co
     }
 }
 template <int G, bool BF = false>
-__global__ void __launch_bounds__(256) k_mul_mat_f16_gqa_long(const tdesc a, const tdesc b, const tdesc d) {
+__global__ void __launch_bounds__(256) k_mul_mat_f16_gqa_long(const tdesc a, const tdesc b, const tdesc d, const int act) {
     __shared__ float part[4][4 * G];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int64_t i02 = blockIdx.y, K = a.ne[0], row0 = (int64_t) blockIdx.x * 4;
@@ -502,7 +508,7 @@ __global__ void __launch_bounds__(256) k_mul_mat_f16_gqa_long(const tdesc a, con
     if (threadIdx.x < 4 * G) {
         const int r = threadIdx.x / G, g = threadIdx.x % G;
         const float v = ((part[0][threadIdx.x] + part[1][threadIdx.x]) + part[2][threadIdx.x]) + part[3][threadIdx.x];
-        if (row0 + r < a.ne[1]) *(float *) (d.data + (row0 + r) * d.nb[0] + (i02 * G + g) * d.nb[2]) = v;
+        if (row0 + r < a.ne[1]) *(float *) (d.data + (row0 + r) * d.nb[0] + (i02 * G + g) * d.nb[2]) = mmf_act(act, v);
     }
 }
 // ---- SOFT_MAX(K.q) folded into V^T.p (a decode step on the non-flash path): the long-row layout above with 8 waves, whose 512 threads
@@ -737,7 +743,7 @@ bool launch_soft_max_mul_mat_f16(hipStream_t s, const tdesc & a, const tdesc & k
 }
 
 // one column against a bf16 matrix (a decode step's projections): the same two forms on bf16 rows
-static void launch_matvec_bf16(hipStream_t s, const tdesc & a, const tdesc & b, const tdesc & d) {
+static void launch_matvec_bf16(hipStream_t s, const tdesc & a, const tdesc & b, const tdesc & d, const int act) {
     const int64_t K = a.ne[0];
     if (K <= 512) {
         int lpr = 64;
@@ -752,7 +758,7 @@ static void launch_matvec_bf16(hipStream_t s, const tdesc & a, const tdesc & b, 
         }
     } else {
         dim3 grid((unsigned) ((a.ne[1] + 3) / 4), (unsigned) a.ne[2]);
-        hipLaunchKernelGGL((k_mul_mat_f16_gqa_long<1, true>), grid, dim3(256), 0, s, a, b, d);
+        hipLaunchKernelGGL((k_mul_mat_f16_gqa_long<1, true>), grid, dim3(256), 0, s, a, b, d, act);
     }
 }
 template <int G> static void launch_gqa_t(hipStream_t s, const tdesc & a, const tdesc & b, const tdesc & d) {
@@ -770,19 +776,31 @@ template <int G> static void launch_gqa_t(hipStream_t s, const tdesc & a, const 
         }
     } else {
         dim3 grid((unsigned) ((a.ne[1] + 3) / 4), (unsigned) a.ne[2]);
-        hipLaunchKernelGGL(k_mul_mat_f16_gqa_long<G>, grid, dim3(256), 0, s, a, b, d);
+        hipLaunchKernelGGL(k_mul_mat_f16_gqa_long<G>, grid, dim3(256), 0, s, a, b, d, -1);
     }
 }
 
-void launch_mul_mat_f(hipStream_t s, const tdesc & a, const tdesc & b, const tdesc & d, float * ws, size_t ws_bytes) {
+// 16-byte vector path: contiguous dim 0 on both sides, K multiple of 8, every row start 16-byte aligned
+static bool mmf_vec_ok(const tdesc & a, const tdesc & b, int esz) {
+    bool ok = a.nb[0] == esz && b.nb[0] == 4 && (a.ne[0] % 8) == 0 && (((uintptr_t) a.data) & 15) == 0 && (((uintptr_t) b.data) & 15) == 0;
+    for (int i = 1; i < 4; ++i) ok = ok && (a.nb[i] % 16) == 0 && (b.nb[i] % 16) == 0;
+    return ok;
+}
+static bool mmf_matvec_bf16_ok(const tdesc & a, const tdesc & b) { return b.ne[1] == 1 && a.ne[3] == 1 && b.ne[3] == 1 && b.ne[2] == a.ne[2] && a.ne[1] >= 64; }
+// does launch_mul_mat_f choose a kernel that applies an activation to its sums?
+bool mul_mat_f_takes_act(const tdesc & a, const tdesc & b) {
+    if (a.type != GGML_TYPE_BF16 || a.ne[1] == 0 || b.ne[1] * b.ne[2] * b.ne[3] == 0 || !mmf_vec_ok(a, b, 2)) return false;
+    if (b.ne[1] >= 2) return mma16_applies(b.ne[1], a.ne[0], ((a.ne[1] + 31) / 32) * ((b.ne[1] + 31) / 32) * b.ne[2] * b.ne[3]);
+    return mmf_matvec_bf16_ok(a, b) && a.ne[0] > 512;
+}
+void launch_mul_mat_f(hipStream_t s, const tdesc & a, const tdesc & b, const tdesc & d, float * ws, size_t ws_bytes, int act) {
+    if (act >= 0 && !mul_mat_f_takes_act(a, b)) { MI_ERR("launch_mul_mat_f: no activation on the sums of this product"); abort(); }
     const int64_t K = a.ne[0];
     const bool bf = a.type == GGML_TYPE_BF16;           // bf16 src0: the same tilings on the bf16 matrix-core instructions
     const bool w16 = a.type == GGML_TYPE_F16 || bf;     // a 2-byte src0
     const int esz = w16 ? 2 : 4;
     if (a.ne[1] == 0 || b.ne[1] * b.ne[2] * b.ne[3] == 0) return;
-    // 16-byte vector path: contiguous dim 0 on both sides, K multiple of 8, every row start 16-byte aligned
-    bool vec_ok = a.nb[0] == esz && b.nb[0] == 4 && (K % 8) == 0 && (((uintptr_t) a.data) & 15) == 0 && (((uintptr_t) b.data) & 15) == 0;
-    for (int i = 1; i < 4; ++i) vec_ok = vec_ok && (a.nb[i] % 16) == 0 && (b.nb[i] % 16) == 0;
+    const bool vec_ok = mmf_vec_ok(a, b, esz);
     if (w16 && !bf && vec_ok && ws && d.nb[0] == 4 && d.nb[1] == d.ne[0] * 4 && d.nb[2] == d.nb[1] * d.ne[1] && d.nb[3] == d.nb[2] * d.ne[2]) {
         int64_t Kc = 0;
         const int ks = mmf_ksplit_slices(a, b, &Kc);
@@ -800,10 +818,10 @@ void launch_mul_mat_f(hipStream_t s, const tdesc & a, const tdesc & b, const tde
         if (mma16_applies(b.ne[1], K, waves32)) {  // few tiles, long rows (or a handful of columns): split K inside the workgroup
             dim3 grid((unsigned) ((a.ne[1] + 15) / 16), (unsigned) ((b.ne[1] + 15) / 16), (unsigned) (b.ne[2] * b.ne[3]));
             if (bf) {
-                if (K >= 4096) hipLaunchKernelGGL((k_mul_mat_f16_mma16<16, true>), grid, dim3(1024), 0, s, a, b, d);
-                else hipLaunchKernelGGL((k_mul_mat_f16_mma16<8, true>), grid, dim3(512), 0, s, a, b, d);
-            } else if (K >= 4096) hipLaunchKernelGGL((k_mul_mat_f16_mma16<16, false>), grid, dim3(1024), 0, s, a, b, d);
-            else hipLaunchKernelGGL((k_mul_mat_f16_mma16<8, false>), grid, dim3(512), 0, s, a, b, d);
+                if (K >= 4096) hipLaunchKernelGGL((k_mul_mat_f16_mma16<16, true>), grid, dim3(1024), 0, s, a, b, d, act);
+                else hipLaunchKernelGGL((k_mul_mat_f16_mma16<8, true>), grid, dim3(512), 0, s, a, b, d, act);
+            } else if (K >= 4096) hipLaunchKernelGGL((k_mul_mat_f16_mma16<16, false>), grid, dim3(1024), 0, s, a, b, d, act);
+            else hipLaunchKernelGGL((k_mul_mat_f16_mma16<8, false>), grid, dim3(512), 0, s, a, b, d, act);
             return;
         }
     }
@@ -819,8 +837,8 @@ void launch_mul_mat_f(hipStream_t s, const tdesc & a, const tdesc & b, const tde
         else hipLaunchKernelGGL(k_mul_mat_f16_mma<false>, grid, dim3(256), 0, s, a, b, d);
         return;
     }
-    if (bf && vec_ok && b.ne[1] == 1 && a.ne[3] == 1 && b.ne[3] == 1 && b.ne[2] == a.ne[2] && a.ne[1] >= 64) {
-        launch_matvec_bf16(s, a, b, d);
+    if (bf && vec_ok && mmf_matvec_bf16_ok(a, b)) {
+        launch_matvec_bf16(s, a, b, d, act);
         return;
     }
     if (w16 && !bf && vec_ok && b.ne[1] == 1 && a.ne[3] == 1 && b.ne[3] == 1 && b.ne[2] % a.ne[2] == 0 && a.ne[1] >= 64) {  // a decode step's K.q / V^T.p
@@ -972,7 +990,7 @@ __global__ void __launch_bounds__(256) k_mul_mat_id_mma(const tdesc a, const tde
 // a few columns (a decode step): four rows of the column's expert per workgroup, the four waves take slices of K with 16-byte loads (the form of
 // k_mul_mat_f16_gqa_long), so an expert's matrix streams at the rate of a plain mat-vec
 template <bool BF>
-__global__ void __launch_bounds__(256) k_mul_mat_id_vec(const tdesc a, const tdesc b, const tdesc ids, const tdesc d) {
+__global__ void __launch_bounds__(256) k_mul_mat_id_vec(const tdesc a, const tdesc b, const tdesc ids, const tdesc d, const int act) {
     __shared__ float part[4][4];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int64_t u = blockIdx.y, t = blockIdx.z, K = a.ne[0], row0 = (int64_t) blockIdx.x * 4;
@@ -1002,7 +1020,7 @@ __global__ void __launch_bounds__(256) k_mul_mat_id_vec(const tdesc a, const tde
     if (threadIdx.x < 4) {
         const int r = threadIdx.x;
         const float v = ((part[0][r] + part[1][r]) + part[2][r]) + part[3][r];
-        if (row0 + r < a.ne[1]) *(float *) (d.data + (row0 + r) * d.nb[0] + u * d.nb[1] + t * d.nb[2]) = v;
+        if (row0 + r < a.ne[1]) *(float *) (d.data + (row0 + r) * d.nb[0] + u * d.nb[1] + t * d.nb[2]) = mmf_act(act, v);
     }
 }
 
@@ -1116,7 +1134,11 @@ static bool mul_mat_id_vec_ok(const tdesc & as, const tdesc & b) {
     return ok;
 }
 bool mul_mat_id_batched(const tdesc & as, const tdesc & b, const tdesc & ids) { return mul_mat_id_vec_ok(as, b) && ids.ne[0] * ids.ne[1] >= 64 && as.ne[2] <= 65535; }
-bool launch_mul_mat_id(hipStream_t s, const tdesc & as, const tdesc & b, const tdesc & ids, const tdesc & d, void * ws, size_t ws_bytes, bool lists_valid, const void * x16) {
+bool mul_mat_id_takes_act(const tdesc & as, const tdesc & b, const tdesc & ids) {
+    return as.ne[1] > 0 && ids.ne[0] * ids.ne[1] > 0 && mul_mat_id_vec_ok(as, b) && as.ne[0] >= 256 && !mul_mat_id_batched(as, b, ids);
+}
+bool launch_mul_mat_id(hipStream_t s, const tdesc & as, const tdesc & b, const tdesc & ids, const tdesc & d, void * ws, size_t ws_bytes, bool lists_valid, const void * x16, int act) {
+    if (act >= 0 && !mul_mat_id_takes_act(as, b, ids)) { MI_ERR("launch_mul_mat_id: no activation on the sums of this product"); abort(); }
     const int64_t K = as.ne[0], n_used = ids.ne[0], T = ids.ne[1];
     if (as.ne[1] == 0 || n_used * T == 0) return false;
     const bool bf = as.type == GGML_TYPE_BF16, w16 = bf || as.type == GGML_TYPE_F16;
@@ -1137,8 +1159,8 @@ bool launch_mul_mat_id(hipStream_t s, const tdesc & as, const tdesc & b, const t
     }
     if (vec_ok && K >= 256) {
         const dim3 grid((unsigned) ((as.ne[1] + 3) / 4), (unsigned) n_used, (unsigned) T);
-        if (bf) hipLaunchKernelGGL(k_mul_mat_id_vec<true>, grid, dim3(256), 0, s, as, b, ids, d);
-        else hipLaunchKernelGGL(k_mul_mat_id_vec<false>, grid, dim3(256), 0, s, as, b, ids, d);
+        if (bf) hipLaunchKernelGGL(k_mul_mat_id_vec<true>, grid, dim3(256), 0, s, as, b, ids, d, act);
+        else hipLaunchKernelGGL(k_mul_mat_id_vec<false>, grid, dim3(256), 0, s, as, b, ids, d, act);
         return false;
     }
     int lpr = 64;

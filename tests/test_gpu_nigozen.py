@@ -479,6 +479,31 @@ def test_weighted_sum_of_expert_rows(backend, H, n, top, T_):
     assert np.array_equal(got, ref)  # the same products and additions in the same order
 
 
+@pytest.mark.parametrize("act,experts", [("gelu", 0), ("relu2", 0), ("relu2", 4)])
+@pytest.mark.parametrize("K,N,M,fused", [(1024, 96, 1, 1), (520, 65, 1, 1), (512, 96, 1, 0), (264, 17, 2, 1), (4096, 33, 15, 1), (1024, 50, 20, 1), (64, 300, 40, 0)])
+def test_activation_on_the_sums_of_a_product(backend, H, act, experts, K, N, M, fused):
+    """(14: GELU_ERF, 6: RELU) the activation in the product's own launch where its kernel takes it, at the edges of its rows and columns: bit for bit the product, then the activation"""
+    if experts:
+        fused = int(K >= 256 and 2 * M < 64)
+    rng = np.random.default_rng(K + N + M)
+    w = bf16_bits(rng.standard_normal((max(1, experts), N, K)).astype(np.float32))
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    sel = np.stack([rng.permutation(experts)[:2] for _ in range(M)]).astype(np.int32) if experts else None
+
+    def product(g):
+        t = g.new(L.BF16, [K, N, experts] if experts else [K, N], w)
+        return H.ggml_mul_mat_id(g.ctx, t, g.new(L.F32, [K, 1, M], x), g.new(L.I32, [2, M], sel)) if experts else H.ggml_mul_mat(g.ctx, t, g.new(L.F32, [K, M], x))
+
+    def activation(g, y):
+        return H.ggml_unary(g.ctx, y, 14) if act == "gelu" else H.ggml_sqr(g.ctx, H.ggml_unary(g.ctx, y, 6))
+
+    f0 = backend.stat("fused_nodes")
+    got = run(backend, lambda g: activation(g, product(g)))[0]
+    assert (backend.stat("fused_nodes") - f0) == (0 if act == "gelu" and not fused else 1 if act == "gelu" or not fused else 2)  # (RELU -> SQR alone is one launch as well)
+    y = run(backend, product)[0]
+    assert np.array_equal(got, run(backend, lambda g: activation(g, g.new(L.F32, [N, y.size // N], y)))[0].reshape(got.shape))
+
+
 def test_erf_gelu_and_squared_relu(backend, H):
     x = np.linspace(-6, 6, 1001).astype(np.float32)
 
