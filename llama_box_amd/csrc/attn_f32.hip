@@ -238,6 +238,136 @@ __global__ void __launch_bounds__(256) k_attn_f32_rows(const tdesc q, const tdes
     }
 }
 
+// k_attn_f32_rows for what a decode step of most models is: 2-byte rows of up to 128 entries that vector loads reach, the soft-max alone (no distance penalty, sigmoid or cap).  What bounds such a
+// launch is its chain of round trips and the instructions between them, not bytes: the general kernel fetches its arguments in five rounds round two 64-bit divisions, then the query, then the mask,
+// then a K row in loads that wait for one another, then the values in two trips, out of 40 KB of code of which each launch runs a tenth.  Here the arguments are one struct with the group size in it,
+// query and mask are requested together, a block's K rows (sixteen lanes a row) and its values (a lane two neighbouring columns) in one trip each; sums across lanes by DPP.
+// 2 tokens x 16 heads of 128 over 1800 cells, 900 of them visible, in 8 splits: 11.2 us, 7.9 here (9.9 with a lane fetching a row); one token x 32 heads over 300 cells 11.2, 7.5.
+struct attn_rows_args {
+    const char * q, * k, * v, * mask;
+    const float * sinks;
+    char * dst;
+    float * parts;
+    int64_t q_nb1, q_nb2, k_nb1, k_nb2, v_nb1, v_nb2, mask_nb1, dst_nb1, dst_nb2;
+    int n_kv, DK, DV, H, gq, mask_f16;
+    float scale;
+};
+template <int T>  // K and V rows: bf16 or f16
+__global__ void __launch_bounds__(256) k_attn_f32_rows128(const attn_rows_args a) {
+    __shared__ float part_acc[4][128], part_m[4], part_l[4];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int t = blockIdx.x, h = blockIdx.y, g = h / a.gq, DK = a.DK, DV = a.DV, n_kv = a.n_kv;
+    const int c16 = lane & 15, r16 = lane >> 4;  // sixteen lanes fetch a K row, 16 bytes each; the lane's own cell of a block is 4 c16 + r16
+    const char * const mrow = a.mask ? a.mask + t * a.mask_nb1 : nullptr;
+    auto mask_at = [&](const int j) -> float {
+        if (j >= n_kv) return -INFINITY;
+        if (!mrow) return 0.0f;
+        return a.mask_f16 ? h2f(((const uint16_t *) mrow)[j]) : ((const float *) mrow)[j];
+    };
+    auto two = [](const uint32_t w, float & lo, float & hi) {
+        if constexpr (T == GGML_TYPE_BF16) { lo = __uint_as_float(w << 16); hi = __uint_as_float(w & 0xFFFF0000u); }
+        else { lo = h2f((uint16_t) (w & 0xFFFFu)); hi = h2f((uint16_t) (w >> 16)); }
+    };
+    int j0 = ((int) blockIdx.z * 4 + wave) * 64;
+    float mv_next = mask_at(j0 + 4 * c16 + r16);
+    const bool has_q = 8 * c16 < DK;
+    const float4 * const qrow = (const float4 *) (a.q + t * a.q_nb1 + h * a.q_nb2) + (has_q ? 2 * c16 : 0);
+    const float4 qa = qrow[0], qb = qrow[1];
+    const float qv[8] = {qa.x, qa.y, qa.z, qa.w, qb.x, qb.y, qb.z, qb.w};
+    const char * const kbase = a.k + g * a.k_nb2 + (has_q ? 16 * c16 : 0), * const vbase = a.v + g * a.v_nb2 + 2 * min(2 * lane, DV - 2);
+    float m = ATTN_F32_LOW, l = 0.0f, acc0 = 0.0f, acc1 = 0.0f;
+    if (a.sinks && wave == 0 && blockIdx.z == 0) { m = a.sinks[h]; l = 1.0f; }  // the sink: exp(sink - m) = 1 in the denominator, nothing in the numerator
+    for (; j0 < n_kv; j0 += 256 * (int) gridDim.z) {
+        const float mv = mv_next;
+        mv_next = mask_at(j0 + 256 * (int) gridDim.z + 4 * c16 + r16);
+        const bool vis = mv > -INFINITY;
+        const uint64_t live = __ballot(vis);
+        if (!live) continue;
+        uint4 w[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i)  // cells 4 i .. 4 i + 3
+            if ((live >> i) & 0x0001000100010001ull) w[i] = *(const uint4 *) (kbase + (int64_t) min(j0 + 4 * i + r16, n_kv - 1) * a.k_nb1);
+        float s = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            if (((live >> i) & 0x0001000100010001ull) == 0) continue;
+            const uint32_t u[4] = {w[i].x, w[i].y, w[i].z, w[i].w};
+            float d = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                float lo, hi;
+                two(u[e], lo, hi);
+                d = fmaf(qv[2 * e], lo, d);
+                d = fmaf(qv[2 * e + 1], hi, d);
+            }
+            d = row16_sum(has_q ? d : 0.0f);
+            s = c16 == i ? d : s;
+        }
+        s = vis ? s * a.scale + mv : -INFINITY;
+        const float m_new = fmaxf(m, wave_max(s));
+        const float p = vis ? expf(s - m_new) : 0.0f, corr = expf(m - m_new);
+        l = l * corr + wave_sum(p);
+        m = m_new;
+        acc0 *= corr;
+        acc1 *= corr;
+        uint32_t vv[4][16];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {  // cells 16 c .. 16 c + 15
+            if (((live >> (4 * c)) & 0x000F000F000F000Full) == 0) continue;
+#pragma unroll
+            for (int u = 0; u < 16; ++u) vv[c][u] = *(const uint32_t *) (vbase + (int64_t) min(j0 + 16 * c + u, n_kv - 1) * a.v_nb1);
+        }
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            if (((live >> (4 * c)) & 0x000F000F000F000Full) == 0) continue;
+#pragma unroll
+            for (int u = 0; u < 16; ++u) {
+                const float pj = readlane_f32(p, 4 * c + (u >> 2) + 16 * (u & 3));
+                float lo, hi;
+                two(vv[c][u], lo, hi);
+                acc0 = fmaf(pj, lo, acc0);
+                acc1 = fmaf(pj, hi, acc1);
+            }
+        }
+    }
+    if (lane == 0) { part_m[wave] = m; part_l[wave] = l; }
+    part_acc[wave][2 * lane] = acc0;
+    part_acc[wave][2 * lane + 1] = acc1;
+    __syncthreads();
+    if (wave != 0) return;
+    float M = part_m[0];
+#pragma unroll
+    for (int w = 1; w < 4; ++w) M = fmaxf(M, part_m[w]);
+    float L = 0.0f, cw[4];
+#pragma unroll
+    for (int w = 0; w < 4; ++w) { cw[w] = expf(part_m[w] - M); L += part_l[w] * cw[w]; }
+    float o[2] = {0.0f, 0.0f};
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+        o[0] += part_acc[w][lane] * cw[w];
+        o[1] += part_acc[w][lane + 64] * cw[w];
+    }
+    float * out = (float *) (a.dst + h * a.dst_nb1 + t * a.dst_nb2);
+    if (gridDim.z > 1) {  // one of several workgroups over the cells of this (token, head): its record for the merge
+        out = a.parts + (((int64_t) t * a.H + h) * gridDim.z + blockIdx.z) * (DV + 2);
+        if (lane == 0) { out[0] = M; out[1] = L; }
+        out += 2;
+    } else {
+        const float inv = L > 0.0f ? 1.0f / L : 0.0f;
+        o[0] *= inv;
+        o[1] *= inv;
+    }
+    if (lane < DV) out[lane] = o[0];
+    if (lane + 64 < DV) out[lane + 64] = o[1];
+}
+// (what the general kernel reads entry by entry stays with it)
+static bool attn_f32_rows128_ok(const tdesc & q, const tdesc & k, const tdesc & v, const float * r12, const float * sig, float softcap) {
+    if (k.type != v.type || (k.type != GGML_TYPE_BF16 && k.type != GGML_TYPE_F16) || r12 || sig || softcap > 0.0f) return false;
+    if (q.ne[0] < 8 || q.ne[0] > 128 || (q.ne[0] % 8) || v.ne[0] < 2 || v.ne[0] > 128 || (v.ne[0] % 2) || k.ne[1] < 1 || k.ne[1] > (1 << 30)) return false;
+    if ((q.nb[1] % 16) || (q.nb[2] % 16) || (((uintptr_t) q.data) & 15) || (k.nb[1] % 16) || (k.nb[2] % 16) || (((uintptr_t) k.data) & 15) || (v.nb[1] % 4) || (v.nb[2] % 4) || (((uintptr_t) v.data) & 3)) return false;
+    return true;
+}
+
 // the merge of k_attn_f32_rows' partial records: one workgroup per (token, head).  gate (may be null): the output is multiplied by sigmoid(gate), one number per head or per entry
 __global__ void __launch_bounds__(128) k_attn_f32_combine(const float * __restrict__ parts, const int S, const int H, const int DV, const tdesc dst, const int sgm, const float * __restrict__ gate,
                                                           const int gate_heads) {
@@ -1045,7 +1175,18 @@ static void attn_f32_launch_t(hipStream_t s, const tdesc & q, const tdesc & k, c
     }
     const int S = attn_f32_row_splits(q, k, v, mask, dst);
     const bool split = S > 1 && x.ws && attn_f32_workspace_bytes(q, k, v, mask, dst) <= x.ws_bytes;
-    hipLaunchKernelGGL((k_attn_f32_rows<KT, VT>), dim3((unsigned) n_q, (unsigned) H, split ? (unsigned) S : 1u), dim3(256), 0, s, q, k, v, mask ? *mask : q, mask ? 1 : 0, sinks, r12, dst, scale, sig,
+    const dim3 grid((unsigned) n_q, (unsigned) H, split ? (unsigned) S : 1u);
+    bool served = false;
+    if constexpr (KT == VT && KT != GGML_TYPE_F32) {
+        if (attn_f32_rows128_ok(q, k, v, r12, sig, softcap)) {
+            const attn_rows_args a{q.data, k.data, v.data, mask ? mask->data : nullptr, sinks, dst.data, (float *) x.ws, q.nb[1], q.nb[2], k.nb[1], k.nb[2], v.nb[1], v.nb[2], mask ? mask->nb[1] : 0,
+                                   dst.nb[1], dst.nb[2], (int) k.ne[1], DK, DV, (int) H, (int) (H / k.ne[2]), mask && mask->type == GGML_TYPE_F16 ? 1 : 0, scale};
+            hipLaunchKernelGGL(k_attn_f32_rows128<KT>, grid, dim3(256), 0, s, a);
+            served = true;
+        }
+    }
+    if (!served)
+        hipLaunchKernelGGL((k_attn_f32_rows<KT, VT>), grid, dim3(256), 0, s, q, k, v, mask ? *mask : q, mask ? 1 : 0, sinks, r12, dst, scale, sig,
                        softcap, pen_kind, (float *) x.ws);
     if (!split) return;
     tdesc o = dst;

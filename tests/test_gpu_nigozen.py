@@ -278,6 +278,49 @@ def test_merge_of_split_records(backend, H, n_q, n_kv, heads, kv_heads, dv, chun
     assert np.abs(got - ref).max() <= 2e-5 * max(1.0, np.abs(ref).max())  # (as test_attention_alone: f32 sums of thousands of terms, each to 2^-24)
 
 
+# 2-byte rows of up to 128 entries: the edges of a row's 16-byte pieces and of a lane's two columns, the last cells of a block, blocks and groups of 16 without a visible cell, one and several splits, masks of
+# the type's lowest value and of zeros; what does not fit (an odd number of value entries, key rows that are no whole pieces) goes to the general kernel and meets the same bound
+@pytest.mark.parametrize("kv_type", [L.BF16, L.F16])
+@pytest.mark.parametrize("n_q,n_kv,heads,kv_heads,dk,dv,how", [
+    (1, 1, 4, 4, 128, 128, "causal"), (2, 63, 4, 2, 8, 2, "causal"), (1, 65, 3, 1, 120, 126, "sink"), (3, 257, 8, 2, 128, 128, "sink"), (31, 300, 2, 1, 64, 40, "sink"), (2, 1800, 16, 4, 128, 128, "half"),
+    (1, 2049, 2, 2, 24, 66, "half"), (2, 200, 2, 1, 128, 128, "lowest"), (1, 130, 4, 1, 128, 64, "all seen"), (2, 300, 4, 2, 128, 33, "causal"), (2, 300, 4, 2, 20, 64, "sink")])
+def test_rows_of_up_to_128_entries(backend, H, kv_type, n_q, n_kv, heads, kv_heads, dk, dv, how):
+    rng = np.random.default_rng(n_kv + dk + dv)
+    q, k, v = (rng.standard_normal(z).astype(np.float32) for z in ((n_q, heads, dk), (n_kv, kv_heads, dk), (n_kv, kv_heads, dv)))
+    k, v = (R.bf16_round(y) if kv_type == L.BF16 else y.astype(np.float16).astype(np.float32) for y in (k, v))
+    raw = (lambda y: bf16_bits(y)) if kv_type == L.BF16 else (lambda y: y.astype(np.float16))
+    mask = np.full((64, n_kv), -np.inf, np.float32)
+    for t in range(n_q):
+        if how == "half":
+            mask[t, (np.arange(n_kv) // 37) % 2 == t % 2] = 0.0
+        else:
+            mask[t, : n_kv - n_q + t + 1] = 0.0
+    if how == "lowest":
+        mask[:, n_kv // 2:] = np.finfo(np.float32).min
+
+    def build(g):
+        tk, tv = g.new(kv_type, [dk * kv_heads, n_kv], raw(k)), g.new(kv_type, [dv * kv_heads, n_kv], raw(v))
+        kk = H.ggml_view_3d(g.ctx, tk, dk, n_kv, kv_heads, dk * kv_heads * 2, dk * 2, 0)
+        vv = H.ggml_view_3d(g.ctx, tv, dv, n_kv, kv_heads, dv * kv_heads * 2, dv * 2, 0)
+        m = g.new(L.F32, [n_kv, 64], np.zeros_like(mask) if how == "all seen" else mask)
+        r = H.ggml_flash_attn_ext(g.ctx, H.ggml_permute(g.ctx, g.new(L.F32, [dk, heads, n_q], q), 0, 2, 1, 3), kk, vv, m, 0.25, 0.0, 0.0)
+        H.ggml_flash_attn_ext_set_prec(r, 10)
+        if how == "sink":
+            H.ggml_flash_attn_ext_add_sinks(r, g.new(L.F32, [heads], np.linspace(-1, 1, heads).astype(np.float32)))
+        return r
+
+    got = run(backend, build)[0].reshape(n_q, heads, dv)
+    for h in range(heads):
+        s = q[:, h].astype(np.float64) @ k[:, h // (heads // kv_heads)].astype(np.float64).T * 0.25
+        if how != "all seen":
+            s = s + mask[:n_q].astype(np.float64)
+        top = np.maximum(s.max(axis=-1, keepdims=True), np.linspace(-1, 1, heads)[h]) if how == "sink" else s.max(axis=-1, keepdims=True)
+        p = np.exp(s - top)
+        z = p.sum(axis=-1, keepdims=True) + (np.exp(np.linspace(-1, 1, heads)[h].astype(np.float32) - top) if how == "sink" else 0.0)
+        ref = (p / z) @ v[:, h // (heads // kv_heads)].astype(np.float64)
+        assert np.abs(got[:, h] - ref).max() <= 2e-5 * max(1.0, np.abs(ref).max()), h  # (f32 sums, as test_attention_alone)
+
+
 @pytest.mark.parametrize("n_q", [1, 40])
 def test_a_far_key_a_chunk_edge_and_the_sink_show(backend, H, n_q):
     """bf16 cache, one key made to dominate: the output is that key's value row when the rule lets the query see it, and not when it lies one position
