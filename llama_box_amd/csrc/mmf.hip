@@ -13,6 +13,15 @@
 
 namespace mi355x {
 
+// the batch of this workgroup (grid.z) in b and in a, whose matrices it shares; one matrix by one needs no divisions in front of the first load
+__device__ __forceinline__ void mmf_batch(const tdesc & a, const tdesc & b, int64_t & i12, int64_t & i13, int64_t & i02, int64_t & i03) {
+    i12 = i13 = i02 = i03 = 0;
+    if (b.ne[2] == 1 && b.ne[3] == 1) return;
+    i12 = blockIdx.z % b.ne[2];
+    i13 = blockIdx.z / b.ne[2];
+    i02 = i12 / (b.ne[2] / a.ne[2]);
+    i03 = i13 / (b.ne[3] / a.ne[3]);
+}
 // f32 -> bf16, nearest even (what ggml-cpu's from_float does to src1 when src0 is bf16), returned widened again
 __device__ __forceinline__ uint32_t mmf_bf16_bits(const float f) {
     const uint32_t u = __float_as_uint(f);
@@ -28,8 +37,8 @@ __global__ void __launch_bounds__(256) k_mul_mat_f(const tdesc a, const tdesc b,
     const int sub = lane / lpr, sl = lane % lpr;
     const int64_t i01 = ((int64_t) blockIdx.x * 4 + wave) * rpw + sub;
     const int64_t i11 = blockIdx.y;
-    const int64_t i12 = blockIdx.z % b.ne[2], i13 = blockIdx.z / b.ne[2];
-    const int64_t i02 = i12 / (b.ne[2] / a.ne[2]), i03 = i13 / (b.ne[3] / a.ne[3]);
+    int64_t i12, i13, i02, i03;
+    mmf_batch(a, b, i12, i13, i02, i03);
     const int64_t K = a.ne[0];
     const bool live = i01 < a.ne[1];
     const int64_t r = live ? i01 : a.ne[1] - 1;
@@ -122,8 +131,8 @@ __global__ void __launch_bounds__(256) k_mul_mat_f16_mma(const tdesc a, const td
     const int r32 = lane & 31, g = lane >> 5;
     const int64_t row0 = ((int64_t) blockIdx.x * 2 + (wave & 1)) * 32, col0 = ((int64_t) blockIdx.y * 2 + (wave >> 1)) * 32;
     if (row0 >= a.ne[1] || col0 >= b.ne[1]) return;
-    const int64_t i12 = blockIdx.z % b.ne[2], i13 = blockIdx.z / b.ne[2];
-    const int64_t i02 = i12 / (b.ne[2] / a.ne[2]), i03 = i13 / (b.ne[3] / a.ne[3]);
+    int64_t i12, i13, i02, i03;
+    mmf_batch(a, b, i12, i13, i02, i03);
     const int64_t K = a.ne[0];
     const char * wrow = a.data + std::min<int64_t>(row0 + r32, a.ne[1] - 1) * a.nb[1] + i02 * a.nb[2] + i03 * a.nb[3] + g * 16;  // this lane's src0 row, its k-group
     const char * xcol = b.data + std::min<int64_t>(col0 + r32, b.ne[1] - 1) * b.nb[1] + i12 * b.nb[2] + i13 * b.nb[3] + g * 32;  // this lane's src1 column
@@ -279,8 +288,8 @@ __global__ void __launch_bounds__(64 * NWK) k_mul_mat_f16_mma16(const tdesc a, c
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int r16 = lane & 15, kg = lane >> 4;
     const int64_t row0 = (int64_t) blockIdx.x * 16, col0 = (int64_t) blockIdx.y * 16;
-    const int64_t i12 = blockIdx.z % b.ne[2], i13 = blockIdx.z / b.ne[2];
-    const int64_t i02 = i12 / (b.ne[2] / a.ne[2]), i03 = i13 / (b.ne[3] / a.ne[3]);
+    int64_t i12, i13, i02, i03;
+    mmf_batch(a, b, i12, i13, i02, i03);
     const char * wrow = a.data + std::min<int64_t>(row0 + r16, a.ne[1] - 1) * a.nb[1] + i02 * a.nb[2] + i03 * a.nb[3] + kg * 16;
     const char * xcol = b.data + std::min<int64_t>(col0 + r16, b.ne[1] - 1) * b.nb[1] + i12 * b.nb[2] + i13 * b.nb[3] + kg * 32;
     const mmf_float4 acc = mma16_tile<NWK, BF>(wrow, xcol, a.ne[0], red);

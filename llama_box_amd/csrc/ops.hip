@@ -64,7 +64,8 @@ __global__ void __launch_bounds__(256) k_rms_norm(const tdesc a, const tdesc d, 
                                                   const float * res = nullptr /* rows like d's, contiguous: added to the normed, weighted row (the ADD behind the MUL) */) {
     __shared__ double sh[4];
     const int64_t row = blockIdx.x;
-    const int64_t i1 = row % a.ne[1], i2 = (row / a.ne[1]) % a.ne[2], i3 = row / (a.ne[1] * a.ne[2]);
+    int64_t i1, i2, i3;
+    split_row(a, row, i1, i2, i3);
     const float * __restrict__ x = (const float *) (a.data + i1 * a.nb[1] + i2 * a.nb[2] + i3 * a.nb[3]);
     float * __restrict__ y = (float *) (d.data + i1 * d.nb[1] + i2 * d.nb[2] + i3 * d.nb[3]);
     const int64_t n = a.ne[0];
@@ -195,7 +196,8 @@ __global__ void __launch_bounds__(256) k_layer_norm_held(const tdesc a, const td
     static_assert(V == 1 || V == 4, "single values or quads");
     __shared__ double sh[4][4];
     const int64_t row = blockIdx.x;
-    const int64_t i1 = row % a.ne[1], i2 = (row / a.ne[1]) % a.ne[2], i3 = row / (a.ne[1] * a.ne[2]);
+    int64_t i1, i2, i3;
+    split_row(a, row, i1, i2, i3);
     const float * const x = (const float *) (a.data + i1 * a.nb[1] + i2 * a.nb[2] + i3 * a.nb[3]);
     const float * const rr = (const float *) (r.data + i1 * r.nb[1] + i2 * r.nb[2] + i3 * r.nb[3]);
     const int np = (int) (a.ne[0] / V);
@@ -295,7 +297,8 @@ __global__ void __launch_bounds__(256) k_layer_norm(const tdesc a, const tdesc d
                                                     const float * __restrict__ w2, const float eps2, const tdesc d2) {
     __shared__ double sh[4];
     const int64_t row = blockIdx.x;
-    const int64_t i1 = row % a.ne[1], i2 = (row / a.ne[1]) % a.ne[2], i3 = row / (a.ne[1] * a.ne[2]);
+    int64_t i1, i2, i3;
+    split_row(a, row, i1, i2, i3);
     const float * x = (const float *) (a.data + i1 * a.nb[1] + i2 * a.nb[2] + i3 * a.nb[3]);
     float * y = (float *) (d.data + i1 * d.nb[1] + i2 * d.nb[2] + i3 * d.nb[3]);
     const float * rr = has_r ? (const float *) (r.data + i1 * r.nb[1] + i2 * r.nb[2] + i3 * r.nb[3]) : nullptr;
@@ -496,7 +499,8 @@ void launch_router_sigmoid_topk(hipStream_t s, const tdesc & logits, const float
 __global__ void __launch_bounds__(256) k_sum_rows(const tdesc a, const tdesc d) {
     const int64_t row = (int64_t) blockIdx.x * 4 + (threadIdx.x >> 6);
     if (row >= a.ne[1] * a.ne[2] * a.ne[3]) return;
-    const int64_t i1 = row % a.ne[1], i2 = (row / a.ne[1]) % a.ne[2], i3 = row / (a.ne[1] * a.ne[2]);
+    int64_t i1, i2, i3;
+    split_row(a, row, i1, i2, i3);
     const float * x = (const float *) (a.data + i1 * a.nb[1] + i2 * a.nb[2] + i3 * a.nb[3]);
     double s = 0.0;
     for (int64_t i = threadIdx.x & 63; i < a.ne[0]; i += 64) s += (double) x[i];
@@ -695,7 +699,8 @@ void launch_head_norm_gate(hipStream_t s, const tdesc & o, const float * w, int 
 // stable sort's permutation; rows of up to a few thousand entries (router logits)
 __global__ void __launch_bounds__(256) k_argsort(const tdesc a, const tdesc d, const int descending) {
     const int64_t row = blockIdx.x;
-    const int64_t i1 = row % a.ne[1], i2 = (row / a.ne[1]) % a.ne[2], i3 = row / (a.ne[1] * a.ne[2]);
+    int64_t i1, i2, i3;
+    split_row(a, row, i1, i2, i3);
     const float * __restrict__ x = (const float *) (a.data + i1 * a.nb[1] + i2 * a.nb[2] + i3 * a.nb[3]);
     int32_t * __restrict__ y = (int32_t *) (d.data + i1 * d.nb[1] + i2 * d.nb[2] + i3 * d.nb[3]);
     const int n = (int) a.ne[0];
@@ -722,7 +727,8 @@ __global__ void __launch_bounds__(256) k_argsort_grouped(const tdesc a, const td
     __shared__ float gmax[256];
     __shared__ int gkeep[256];
     const int64_t row = blockIdx.x;
-    const int64_t i1 = row % a.ne[1], i2 = (row / a.ne[1]) % a.ne[2], i3 = row / (a.ne[1] * a.ne[2]);
+    int64_t i1, i2, i3;
+    split_row(a, row, i1, i2, i3);
     const float * __restrict__ x = (const float *) (a.data + i1 * a.nb[1] + i2 * a.nb[2] + i3 * a.nb[3]);
     int32_t * __restrict__ y = (int32_t *) (d.data + i1 * d.nb[1] + i2 * d.nb[2] + i3 * d.nb[3]);
     const int n = (int) a.ne[0], per = n / groups;
@@ -1066,7 +1072,8 @@ void launch_weighted_rows_sum(hipStream_t s, const tdesc & rows, const tdesc & w
 // ------------------------------------------------------------------------------------------------ ADD/SUB/MUL/DIV
 __global__ void __launch_bounds__(256) k_binary(const int op, const tdesc a, const tdesc b, const tdesc d) {
     const int64_t row = blockIdx.x;
-    const int64_t i1 = row % a.ne[1], i2 = (row / a.ne[1]) % a.ne[2], i3 = row / (a.ne[1] * a.ne[2]);
+    int64_t i1, i2, i3;
+    split_row(a, row, i1, i2, i3);
     const char * pa = a.data + i1 * a.nb[1] + i2 * a.nb[2] + i3 * a.nb[3];
     const char * pb = b.data + (i1 % b.ne[1]) * b.nb[1] + (i2 % b.ne[2]) * b.nb[2] + (i3 % b.ne[3]) * b.nb[3];
     char * pd = d.data + i1 * d.nb[1] + i2 * d.nb[2] + i3 * d.nb[3];
@@ -1382,7 +1389,12 @@ __device__ __forceinline__ float dequant_elem(const int type, const uint8_t * __
 // (a decode step gathers ONE row: 1024 threads and independent iterations keep its chain of dependent byte loads short)
 __global__ void __launch_bounds__(1024) k_get_rows(const tdesc a, const tdesc idx, const tdesc d) {
     const int64_t r = blockIdx.x;
-    const int64_t i10 = r % idx.ne[0], i11 = (r / idx.ne[0]) % idx.ne[1], i12 = r / (idx.ne[0] * idx.ne[1]);
+    int64_t i10 = r, i11 = 0, i12 = 0;
+    if (idx.ne[1] != 1 || idx.ne[2] != 1) {
+        i10 = r % idx.ne[0];
+        i11 = (r / idx.ne[0]) % idx.ne[1];
+        i12 = r / (idx.ne[0] * idx.ne[1]);
+    }
     const int32_t i01 = *(const int32_t *) (idx.data + i10 * idx.nb[0] + i11 * idx.nb[1] + i12 * idx.nb[2]);
     const uint8_t * row = (const uint8_t *) (a.data + (int64_t) i01 * a.nb[1] + i11 * a.nb[2] + i12 * a.nb[3]);
     float * y = (float *) (d.data + i10 * d.nb[1] + i11 * d.nb[2] + i12 * d.nb[3]);
@@ -2257,7 +2269,8 @@ __global__ void __launch_bounds__(256) k_soft_max(const tdesc a, const tdesc m, 
     __shared__ double shd[4];
     __shared__ float shf[4];
     const int64_t row = blockIdx.x;
-    const int64_t i1 = row % a.ne[1], i2 = (row / a.ne[1]) % a.ne[2], i3 = row / (a.ne[1] * a.ne[2]);
+    int64_t i1, i2, i3;
+    split_row(a, row, i1, i2, i3);
     const float * x = (const float *) (a.data + i1 * a.nb[1] + i2 * a.nb[2] + i3 * a.nb[3]);
     float * y = (float *) (d.data + i1 * d.nb[1] + i2 * d.nb[2] + i3 * d.nb[3]);
     const char * mp = has_mask ? m.data + i1 * m.nb[1] + (i2 % m.ne[2]) * m.nb[2] + (i3 % m.ne[3]) * m.nb[3] : nullptr;
@@ -2297,7 +2310,8 @@ __global__ void __launch_bounds__(256) k_soft_max_reg(const tdesc a, const tdesc
     __shared__ double shd[4];
     __shared__ float shf[4];
     const int64_t row = blockIdx.x;
-    const int64_t i1 = row % a.ne[1], i2 = (row / a.ne[1]) % a.ne[2], i3 = row / (a.ne[1] * a.ne[2]);
+    int64_t i1, i2, i3;
+    split_row(a, row, i1, i2, i3);
     const float * x = (const float *) (a.data + i1 * a.nb[1] + i2 * a.nb[2] + i3 * a.nb[3]);
     float * y = (float *) (d.data + i1 * d.nb[1] + i2 * d.nb[2] + i3 * d.nb[3]);
     const char * mp = has_mask ? m.data + i1 * m.nb[1] + (i2 % m.ne[2]) * m.nb[2] + (i3 % m.ne[3]) * m.nb[3] : nullptr;
