@@ -46,6 +46,7 @@ template <int CT> constexpr int mp_sb_bytes() { return CT * (4096 + 512 + 64); }
 
 template <int QT, int CT, int NW>
 __global__ void __launch_bounds__(NW * 64) k_mmq_panel(const mmqp_args a) {
+    args_ahead<sizeof(mmqp_args)>();
     constexpr int DEPTH = CT == 2 && NW == 16 ? 2 : 4, NT = NW * 64, NP = CT == 1 ? 5 : 9;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);

@@ -182,6 +182,7 @@ template <bool WP, bool EPI> __global__ void __launch_bounds__(Q80S_WV * 64, 2) 
 // lanes, and v_permlane32_swap turns them into the operands of the two blocks (the K order inside a block is the same on both sides, so the integer sums are).  One v_mfma_f32_16x16x1 (four outer
 // products) gives d_w * d_x of a chunk's four blocks.  The chunks go to the eight sums, and these are added, as above: the same bits.
 template <int CT, bool EPI> __global__ void __launch_bounds__(Q80S_WV * 64, 2) k_mmq_q80_rows16(const mmq80s_args a, const mmq_epi epi) {
+    args_ahead<sizeof(mmq80s_args)>();
     constexpr int DEPTH = 4;
     __shared__ float red[Q80S_WV][4 * CT][64];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -297,6 +298,7 @@ template <int CT, bool EPI> __global__ void __launch_bounds__(Q80S_WV * 64, 2) k
 // with the factors on the VALU: 40 / 66 us / 9.1 ms; as it is: 15 / 44 us / 5.9 ms (23.6 GFLOP in 44 us: 0.53 POP/s).
 constexpr int Q80C_WV = 4;
 template <bool WP> __global__ void __launch_bounds__(Q80C_WV * 64, 3) k_mmq_q80_cols(const mmq80s_args a, const int n_panels, const int m_tiles) {
+    args_ahead<sizeof(mmq80s_args) + 8>();
     __shared__ float red[Q80C_WV][16][65];                         // the waves' partial tiles, one 32-column half at a time
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int fr = lane & 31, kg = lane >> 5;

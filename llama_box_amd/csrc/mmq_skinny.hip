@@ -190,6 +190,7 @@ template <int QT, int TQ> __device__ __forceinline__ void sk_unit_k45(const char
 // copy the block into scratch memory — 408 bytes per lane — and read every pointer of the launch from there)
 template <int QA, int QB, int EPI, int TQ, bool TILE = false>
 __global__ void __launch_bounds__(SK_NW * 64, 1) k_mmq_skinny(const mmq8_args a) {
+    args_ahead<sizeof(mmq8_args)>();
     extern __shared__ __attribute__((aligned(16))) char smem[];
     constexpr bool MIXED = QA != QB;
     auto pass = [&](auto qt_tag) __attribute__((always_inline)) {
@@ -638,6 +639,7 @@ template <int QT, int TQ> constexpr int tp8_lds_bytes() { return TP8_NSB * (2 * 
 
 template <int QT, int TQ>
 __global__ void __launch_bounds__(TP8_NW * 64, 1) k_mmq_skinny_tp8(const mmq8_args a) {
+    args_ahead<sizeof(mmq8_args)>();
     extern __shared__ __attribute__((aligned(16))) char smem[];
     typedef sk_fmt<QT> F;
     constexpr int NPA = 32 * F::PIECES, NLA = (NPA + 63) / 64;  // weight pieces per unit and the wave-instructions fetching them
@@ -1189,6 +1191,7 @@ __global__ void __launch_bounds__((NW + NL) * 64, NSA == 2 ? 2 : 1) k_mmq_wide(c
 // ffn_down Q6_K 39 .. 51 -> 29, wq + wk (+ wv) 22 -> 17.  (At 512 columns the chunks gain nothing over k_mmq_wide.)
 template <int QT, int TT, bool LAP>
 __global__ void __launch_bounds__((WD_NW + WD_NL) * 64, 1) k_mmq_wide_few(const mmq8_args a) {
+    args_ahead<sizeof(mmq8_args)>();
     extern __shared__ __attribute__((aligned(16))) char smem[];
     typedef sk_fmt<QT> F;
     constexpr int NP = QT == 5 ? 3 : 2;

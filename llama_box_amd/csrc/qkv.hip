@@ -84,6 +84,7 @@ template <typename T, bool PIPE> __device__ __forceinline__ void qkv_unit(qkv_re
 // a launch with a scratch frame pays for it at every dispatch); Qwen2-7B's launches use 9 waves, so the Q5_K forms also exist compiled for 640 threads (round 6)
 template <typename TA, typename TB, bool Q8S, bool PIPE = false, int BND = 1024>
 __global__ void __launch_bounds__(PIPE ? 512 : BND) k_qkv_stream2(const qkv_args a) {
+    args_ahead<sizeof(qkv_args)>();
     extern __shared__ __attribute__((aligned(16))) char smem[];
     // (a generic lambda, not a device function: passing the kernel-argument struct to a function copies it to scratch)
     // (u_first / GW: this wave's first unit among the segments of its format, and the number of waves that share them)
