@@ -254,6 +254,7 @@ struct attn_rows_args {
 };
 template <int T>  // K and V rows: bf16 or f16
 __global__ void __launch_bounds__(256) k_attn_f32_rows128(const attn_rows_args a) {
+    args_ahead<sizeof(attn_rows_args)>();
     __shared__ float part_acc[4][128], part_m[4], part_l[4];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int t = blockIdx.x, h = blockIdx.y, g = h / a.gq, DK = a.DK, DV = a.DV, n_kv = a.n_kv;
@@ -569,6 +570,7 @@ constexpr int ATT_SCAN_BITS = 16384;  // blocks beyond these are taken as visibl
 template <int DK16, int DVT, bool PLAIN>
 __global__ void __launch_bounds__(256, 2) k_attn_mma_bf16(const tdesc q, const tdesc k, const tdesc v, const tdesc mask, const float * __restrict__ sinks, const float * __restrict__ r12, const tdesc dst,
                                                        const float scale, const float * __restrict__ sig, const float softcap, const int pen_kind) {
+    args_ahead<args_bytes<tdesc, tdesc, tdesc, tdesc, const float *, const float *, tdesc, float>()>();
     constexpr int W = 4;  // waves
     // 16-byte pieces of a cell's K and V rows in LDS, a piece's index XORed by the cell's: the 16 K rows read at once, and the 4 x 64 bytes of V, hit all banks once
     constexpr int CP = DK16 <= 2 ? 4 : DK16 <= 4 ? 8 : 16, CV = DVT <= 1 ? 4 : DVT <= 2 ? 8 : 16;

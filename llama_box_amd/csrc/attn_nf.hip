@@ -29,6 +29,7 @@ struct __attribute__((packed, aligned(2))) u32x4a { uint32_t x, y, z, w; };  // 
 template <int G, int NW>
 __global__ void __launch_bounds__(NW * 64) k_attn_nf_list(const tdesc q, const tdesc k, const tdesc v, const tdesc mask, const tdesc dst, const int * __restrict__ lists,
                                                       const int list_stride, float * __restrict__ scratch, const float scale, const int dq_n, q8k_dev * __restrict__ q8, const int nf_groups_on) {
+    args_ahead<args_bytes<tdesc, tdesc, tdesc, tdesc, tdesc, const int *>()>();
     // q8 != null (only with dq_n == 1 and an even G): the result's only readers are quantised mat-muls (wo) — it leaves the kernel as the
     // Q8_K blocks quantize_row_q8_K builds of the token's row (a block = two heads), through the q area of the LDS, and not as f32
     constexpr int D = 128, NT = NW * 64;

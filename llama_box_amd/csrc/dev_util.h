@@ -149,16 +149,16 @@ template <typename Q8K> __device__ __forceinline__ void wave_quantize_q8_K(const
 }
 
 // The kernel's arguments (BYTES of them) into the scalar cache in ONE round of requests: fetched where they are used, a struct of several cache lines is that many misses one after the other
-// in front of the first load (K-quant products of a few columns fetched theirs in four or five rounds: a step of 3 sequences of an 8B model 2714 us, 2641 so; of 32 3156, 3096)
+// in front of the first load (K-quant products of a few columns fetched theirs in four or five rounds: a step of 3 sequences of an 8B model 2714 us, 2641 so; of 32 3156, 3096; the mat-vecs of one sequence 1725, 1684)
 template <int BYTES> __device__ __forceinline__ void args_ahead() {
-    static_assert(BYTES <= 512, "eight lines");
+    constexpr int N = BYTES > 640 ? 10 : (BYTES + 63) / 64;  // (ten lines at the most)
     const __attribute__((address_space(4))) uint32_t * const ka = (const __attribute__((address_space(4))) uint32_t *) __builtin_amdgcn_kernarg_segment_ptr();
-    constexpr int N = (BYTES + 63) / 64;
-    uint32_t t[8];
+    uint32_t t[10];
 #pragma unroll
-    for (int k = 0; k < 8; ++k) t[k] = ka[16 * (k < N ? k : N - 1)];
-    asm volatile("" ::"s"(t[0]), "s"(t[1]), "s"(t[2]), "s"(t[3]), "s"(t[4]), "s"(t[5]), "s"(t[6]), "s"(t[7]));
+    for (int k = 0; k < 10; ++k) t[k] = ka[16 * (k < N ? k : N - 1)];
+    asm volatile("" ::"s"(t[0]), "s"(t[1]), "s"(t[2]), "s"(t[3]), "s"(t[4]), "s"(t[5]), "s"(t[6]), "s"(t[7]), "s"(t[8]), "s"(t[9]));
 }
+template <typename... A> constexpr int args_bytes() { return (0 + ... + (int) sizeof(A)); }  // (a kernel's arguments are at least that far apart)
 
 // row number -> its indices in dimensions 1 .. 3 of `a`.  Rows of one matrix, which most launches walk, need none of the 64-bit divisions in front of a kernel's first load (a norm of 2 rows
 // of 2048 values 4.9 us a launch with them, 4.2 without; steps of 1.1B models 2 to 4 % shorter)

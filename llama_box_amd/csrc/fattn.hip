@@ -416,6 +416,7 @@ template <int G, int MODE, bool Q8, int WV = 4, int KVT = 0, int D = 128, bool P
 __global__ void __launch_bounds__(WV * 64) k_fattn_dec128(const tdesc q, const tdesc k, const tdesc v, const tdesc mask, const float * __restrict__ sinks,
                                                       const tdesc dst, const fa_geom geo, float * __restrict__ ws, const int g_group,
                                                       const int * __restrict__ lists, const int list_stride) {
+    args_ahead<args_bytes<tdesc, tdesc, tdesc, tdesc, const float *, tdesc, fa_geom, float *>()>();
     constexpr bool SKIP = MODE == 1, LIST = MODE == 2;
     constexpr int LPR = D / 8, RPW = 64 / LPR, NG = LPR / G;  // lanes per K / V row, rows per wave-instruction, row groups per trip
     static_assert(D == 128 || (D == 64 && !Q8 && KVT == 0 && G <= 8), "head_dim 64: f16 cache only");
@@ -976,6 +977,7 @@ __global__ void __launch_bounds__(WV * 64) k_fattn_dec128(const tdesc q, const t
 // the kernel as Q8_K blocks (one block = the 256 values of the two heads of a (token, head pair)), not as f32
 template <int D, bool Q8OUT = false> __global__ void __launch_bounds__(Q8OUT ? 256 : D) k_fattn_combine(const float * __restrict__ ws, const float * __restrict__ sinks, const tdesc dst, const fa_geom geo,
                                                                                                  q8k_dev * __restrict__ q8 = nullptr) {
+    args_ahead<args_bytes<const float *, const float *, tdesc, fa_geom>()>();
     // one thread per output dimension; every wave recomputes the (<= 64) split coefficients lane-parallel (lane s owns
     // split s: ONE round trip fetches every (m, l) pair), then the coefficients come out of their lanes through SGPRs
     // (v_readlane with compile-time indices) while up to 32 partial values per thread are in flight at once
@@ -1039,6 +1041,7 @@ template <int D, bool Q8OUT = false> __global__ void __launch_bounds__(Q8OUT ? 2
 // 4.9 for the quantiser behind it -> 6.3; 16 tokens 3.8 and 2.7 -> 4.5.
 template <int D, int S, int OUT = 0>
 __global__ void __launch_bounds__(256) k_fattn_combine_rows(const float * __restrict__ ws, const tdesc dst, const fa_geom geo, const int n_rows, q8k_dev * __restrict__ q8 = nullptr) {
+    args_ahead<args_bytes<const float *, tdesc, fa_geom>()>();
     constexpr int CPR = D / 4;            // chunks (threads) per row
     constexpr int RPB = 256 / CPR;        // rows per workgroup
     const int r = (int) blockIdx.x * RPB + (int) threadIdx.x / CPR, j = (int) threadIdx.x % CPR;

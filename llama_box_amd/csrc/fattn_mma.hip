@@ -37,6 +37,7 @@ struct fam_geom {
 template <int D, int NW>
 __global__ void __launch_bounds__(NW * 64, 2) k_fattn_mma(const tdesc q, const tdesc k, const tdesc v, const tdesc mask, const tdesc dst, const fam_geom geo, float * __restrict__ ws,
                                                        const uint8_t * __restrict__ vis) {
+    args_ahead<args_bytes<tdesc, tdesc, tdesc, tdesc, tdesc, fam_geom>()>();
     constexpr int BKV = 64;
     constexpr int KS = (D + 8) * 2;    // K tile row stride (bytes): odd multiple of 16 -> conflict-free ds_read_b128
     constexpr int VS = (BKV + 4) * 2;  // V^T tile row stride (bytes): 34 dwords -> conflict-free ds_read_b64 across 32 rows
@@ -317,6 +318,7 @@ __global__ void __launch_bounds__(NW * 64, 2) k_fattn_mma(const tdesc q, const t
 template <int D, int NW, int PASS>
 __global__ void __launch_bounds__(NW * 64, 2) k_attn_nf_mma(const tdesc q, const tdesc k, const tdesc vt, const tdesc mask, const tdesc dst, const fam_geom geo, float * __restrict__ stats,
                                                          float * __restrict__ ws, const uint8_t * __restrict__ vis) {
+    args_ahead<args_bytes<tdesc, tdesc, tdesc, tdesc, tdesc, fam_geom>()>();
     constexpr int BKV = 64;
     constexpr int KS = (D + 8) * 2, VS = (BKV + 4) * 2, NS = D / 16, ND = D / 32;
     constexpr int T = NW * 64;
@@ -566,6 +568,7 @@ __global__ void __launch_bounds__(NW * 64, 2) k_attn_nf_mma(const tdesc q, const
 typedef float float4v __attribute__((ext_vector_type(4)));
 template <int D, int NT, int QT, int HP>
 __global__ void __launch_bounds__(512, 2) k_attn_nf_once(const tdesc q, const tdesc k, const tdesc vt, const tdesc mask, const tdesc dst, const fam_geom geo, q8k_dev * __restrict__ q8) {
+    args_ahead<args_bytes<tdesc, tdesc, tdesc, tdesc, tdesc, fam_geom>()>();
     constexpr int NS = D / 32, ND = D / 16, PS = D + 4, QS = D + 8, NC = 16 * QT, NQ = NC / HP;
     constexpr float LOG2E = 1.4426950408889634f;
     extern __shared__ __attribute__((aligned(16))) char smem[];

@@ -64,7 +64,7 @@ struct mmvq_args {
     float * x_out;
     float * norm_out;  // norm_w != null: where RMS_NORM(x) * norm_w itself belongs (the graph's MUL node); written by workgroup 0 so that
                        // the fusion never leaves a tensor of the graph unwritten (readers in another split, or the host, may exist)
-    int balance_tail;  // set by the launcher: spread the last, partial pass of rows evenly over the workgroups
+    int full_rows, rem_per;  // set by the launcher: rows of the whole passes, and of the last, partial pass those of each workgroup (spread evenly)
     // sum of squares of the result row, handed from the mat-vec that WRITES a residual stream to the RMS_NORM prologue that READS it (round 4):
     //   ss_out != null (single column, f32 result, no SwiGLU): workgroup b writes the sum of (double) (v * v) over the rows it produced to ss_out[b];
     //     launch_mmvq_ss_count() tells how many workgroups that is

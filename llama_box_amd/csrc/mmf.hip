@@ -31,6 +31,7 @@ __device__ __forceinline__ float mmf_bf16_round(const float f) { return __uint_a
 // WT: 0 = f32 src0 (true 32-bit products), 1 = f16, 2 = bf16 (src1 rounded to the same type first; f32 accumulation)
 template <int WT>
 __global__ void __launch_bounds__(256) k_mul_mat_f(const tdesc a, const tdesc b, const tdesc d, const int lpr, const int vec_ok) {
+    args_ahead<args_bytes<tdesc, tdesc, tdesc, int, int>()>();
     constexpr bool W16 = WT != 0;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int rpw = 64 / lpr;  // rows per wave
@@ -284,6 +285,7 @@ __device__ __forceinline__ float mmf_act(const int act, const float v) {
 }
 template <int NWK, bool BF>
 __global__ void __launch_bounds__(64 * NWK) k_mul_mat_f16_mma16(const tdesc a, const tdesc b, const tdesc d, const int act) {
+    args_ahead<args_bytes<tdesc, tdesc, tdesc, int>()>();
     __shared__ mmf_float4 red[NWK][64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int r16 = lane & 15, kg = lane >> 4;
@@ -308,6 +310,7 @@ __global__ void __launch_bounds__(64 * NWK) k_mul_mat_f16_mma16(const tdesc a, c
 // bytes are 1 .. 2): the workgroups are dealt over the matrices' 16-row tiles; results dense rows
 template <int NWK>
 __global__ void __launch_bounds__(64 * NWK) k_mul_mat_bf16_mma16_multi(const matvec_multi mm, const char * __restrict__ x, const int64_t x_nb1, const int64_t K, const int M) {
+    args_ahead<args_bytes<matvec_multi, const char *, int64_t, int64_t, int>()>();
     __shared__ mmf_float4 red[NWK][64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int r16 = lane & 15, kg = lane >> 4;
@@ -482,6 +485,7 @@ __global__ void __launch_bounds__(256) k_mul_mat_f16_gqa_short(const tdesc a, co
 }
 template <int G, bool BF = false>
 __global__ void __launch_bounds__(256) k_mul_mat_f16_gqa_long(const tdesc a, const tdesc b, const tdesc d, const int act) {
+    args_ahead<args_bytes<tdesc, tdesc, tdesc, int>()>();
     __shared__ float part[4][4 * G];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int64_t i02 = blockIdx.y, K = a.ne[0], row0 = (int64_t) blockIdx.x * 4;
@@ -1000,6 +1004,7 @@ __global__ void __launch_bounds__(256) k_mul_mat_id_mma(const tdesc a, const tde
 // k_mul_mat_f16_gqa_long), so an expert's matrix streams at the rate of a plain mat-vec
 template <bool BF>
 __global__ void __launch_bounds__(256) k_mul_mat_id_vec(const tdesc a, const tdesc b, const tdesc ids, const tdesc d, const int act) {
+    args_ahead<args_bytes<tdesc, tdesc, tdesc, tdesc, int>()>();
     __shared__ float part[4][4];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int64_t u = blockIdx.y, t = blockIdx.z, K = a.ne[0], row0 = (int64_t) blockIdx.x * 4;
@@ -1095,6 +1100,7 @@ void launch_matvec_glu(hipStream_t s, const tdesc & a, const float * gu, const f
 // up to four bf16 matrices against the same single column (a decode step's q / k / v / gate projections) in one launch: the workgroups are dealt over
 // the matrices' rows, four rows each, the waves taking slices of K (k_mul_mat_f16_gqa_long's form and arithmetic)
 __global__ void __launch_bounds__(256) k_matvec_bf16_multi(const matvec_multi mm, const char * __restrict__ x, const int64_t K) {
+    args_ahead<args_bytes<matvec_multi, const char *, int64_t>()>();
     __shared__ float part[4][4];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     int q = 0;

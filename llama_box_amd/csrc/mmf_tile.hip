@@ -72,6 +72,7 @@ struct mt_args {
 };
 
 template <bool BF, int TM, int TN, int S, bool ID> __global__ void __launch_bounds__(256, 1) k_mul_mat_tile(const mt_args a) {
+    args_ahead<sizeof(mt_args)>();
     constexpr int MT = TM / 64, NT = TN / 64;
     constexpr int STAGE = (TM + TN) * 128, L = (TM + TN) / 32, Q = L / 4;  // bytes of a stage, DMA instructions per wave and stage, of which the first quarter
     static_assert(S >= 2 && S <= 5 && (S - 1) * L <= 63, "ring");

@@ -58,6 +58,7 @@ __device__ __forceinline__ int sw_off(const int row, const int chunk) { return r
 // LDS-read and fold work shrinks with the tile instead of multiplying zeros; the two partial sums meet in LDS at the end.
 template <int QT, int BN, int BM = 128>
 __global__ void __launch_bounds__(BN * 4, BN == 64 ? (BM == 32 ? 3 : 2) : 1) k_mmq_i8(const mmq8_args a) {
+    args_ahead<sizeof(mmq8_args)>();
     extern __shared__ __attribute__((aligned(16))) char smem[];
     constexpr int NT = BN * 4;
     constexpr int NP = QT == 5 ? 3 : 2;

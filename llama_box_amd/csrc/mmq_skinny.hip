@@ -919,6 +919,7 @@ template <> struct sk_conv<6> {
 // Q4_K with more items than CUs: 28672 x 4096 at 512 columns 155 -> 149 us, a 2048-token prompt of Llama-3-8B 52.7 -> 51.9 ms.  (Q5_K's units do not fit twice.)
 template <int QT, int TT, int NW, int NL, int NSA>
 __global__ void __launch_bounds__((NW + NL) * 64, NSA == 2 ? 2 : 1) k_mmq_wide(const mmq8_args a) {
+    args_ahead<sizeof(mmq8_args)>();
     constexpr bool SELF = NL == 0;
     constexpr int NLD = SELF ? NW : NL;  // waves that request
     extern __shared__ __attribute__((aligned(16))) char smem[];

@@ -204,6 +204,7 @@ __global__ void __launch_bounds__(WAVES * 64) k_mmvq(const mmvq_args a) {
 //     RMS-norm reduction, CPU-identical Q8_K quantisation straight into LDS.
 template <typename T, bool GLU, int PRO>
 __global__ void __launch_bounds__(1024) k_mmvq_stream(const mmvq_args a) {
+    args_ahead<sizeof(mmvq_args)>();
     extern __shared__ __attribute__((aligned(16))) char smem[];
     typedef typename T::act act;
     // pairs per item: ~16 dwords of weights per lane per matrix (8 for the two-matrix GLU form).  Measured on MI355X:
@@ -217,8 +218,8 @@ __global__ void __launch_bounds__(1024) k_mmvq_stream(const mmvq_args a) {
     // rows are dealt one per wave and pass (row = pass*GW + block*16 + wave); the LAST, partial pass is spread evenly over
     // the workgroups instead (rem_per rows each), so that every CU streams until the end: with N = 14336 (3.5 passes)
     // the natural order left half of the CUs idle for the final eighth of the launch
-    const int full = a.balance_tail ? (a.N / GW) * GW : ((a.N + GW - 1) / GW) * GW, rem = a.N - (a.balance_tail ? full : a.N);
-    const int rem_per = (rem + (int) gridDim.x - 1) / (int) gridDim.x;
+    // (both from the launcher: two divisions in front of the first load otherwise)
+    const int full = a.full_rows, rem_per = a.rem_per;
     auto next_row = [&](const int r) {
         const int nr = r + GW;
         if (nr < full) return nr;
@@ -478,7 +479,9 @@ template <typename T, bool GLU, int PRO> static void launch_stream(hipStream_t s
     const unsigned grid = (unsigned) std::min<int64_t>(256, ((int64_t) a.N + 15) / 16);
     static const int bal = getenv("GGML_MI355X_BALANCE_TAIL") ? atoi(getenv("GGML_MI355X_BALANCE_TAIL")) : 1;
     mmvq_args a2 = a;
-    a2.balance_tail = bal;
+    const int GW = (int) grid * 16;
+    a2.full_rows = bal ? (a.N / GW) * GW : ((a.N + GW - 1) / GW) * GW;
+    a2.rem_per = bal ? (a.N - a2.full_rows + (int) grid - 1) / (int) grid : 0;
     if (g_launch_probe.armed && !g_launch_probe.used) {
         hipExtLaunchKernelGGL((k_mmvq_stream<T, GLU, PRO>), dim3(grid), dim3(1024), lds, s, g_launch_probe.e0, g_launch_probe.e1, 0, a2);
         g_launch_probe.used = true;

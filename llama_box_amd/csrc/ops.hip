@@ -62,6 +62,7 @@ __device__ __forceinline__ void q80_panel_store(const float r0, const float r1, 
 template <bool Q80P>
 __global__ void __launch_bounds__(256) k_rms_norm(const tdesc a, const tdesc d, const float eps, const float * __restrict__ w, char * __restrict__ q80 = nullptr,
                                                   const float * res = nullptr /* rows like d's, contiguous: added to the normed, weighted row (the ADD behind the MUL) */) {
+    args_ahead<args_bytes<tdesc, tdesc, float, const float *, char *, const float *>()>();
     __shared__ double sh[4];
     const int64_t row = blockIdx.x;
     int64_t i1, i2, i3;
@@ -193,6 +194,7 @@ __device__ __forceinline__ uint2 round4_16(const float4 v, const int type) {
 template <int R, int V>
 __global__ void __launch_bounds__(256) k_layer_norm_held(const tdesc a, const tdesc d, const float eps, const float * __restrict__ w, const tdesc r, const int has_r,
                                                          const float * __restrict__ w2, const float eps2, const tdesc d2, const copy16 o16) {
+    args_ahead<args_bytes<tdesc, tdesc, float, const float *, tdesc, int, const float *, float, tdesc, copy16>()>();
     static_assert(V == 1 || V == 4, "single values or quads");
     __shared__ double sh[4][4];
     const int64_t row = blockIdx.x;
@@ -367,6 +369,7 @@ bool launch_layer_norm_twice(hipStream_t s, const tdesc & src, const tdesc & dst
 // one workgroup per token: ranks by counting (k_argsort's stable order), the whole permutation is written (the top-k view reads its first columns), and the
 // soft-max over the k largest logits goes to `wts` [k, T] — ARGSORT, GET_ROWS of the chosen logits and SOFT_MAX in one pass
 __global__ void __launch_bounds__(256) k_topk_softmax(const tdesc a, const tdesc ids, const tdesc wts, const int k) {
+    args_ahead<args_bytes<tdesc, tdesc, tdesc, int>()>();
     __shared__ float top[256];
     __shared__ float red[2];
     const int64_t t = blockIdx.x;
@@ -1032,6 +1035,7 @@ void launch_softcap(hipStream_t s, const float * x, float * d, int64_t n, float 
 // One thread holds V neighbouring entries of a token's sum: the rows of four experts are requested together, and a token's row is spread over workgroups (a step of two tokens would leave
 // two workgroups walking it: 2 x 2048, four experts, 6.7 -> 2.9 us)
 template <int V> __global__ void __launch_bounds__(256) k_weighted_rows_sum(const tdesc rows, const tdesc w, const tdesc d) {
+    args_ahead<args_bytes<tdesc, tdesc, tdesc>()>();
     const int64_t t = blockIdx.x, i = ((int64_t) blockIdx.y * 256 + threadIdx.x) * V;
     const int n_used = (int) rows.ne[1];
     if (i >= rows.ne[0]) return;
@@ -1388,6 +1392,7 @@ __device__ __forceinline__ float dequant_elem(const int type, const uint8_t * __
 }
 // (a decode step gathers ONE row: 1024 threads and independent iterations keep its chain of dependent byte loads short)
 __global__ void __launch_bounds__(1024) k_get_rows(const tdesc a, const tdesc idx, const tdesc d) {
+    args_ahead<args_bytes<tdesc, tdesc, tdesc>()>();
     const int64_t r = blockIdx.x;
     int64_t i10 = r, i11 = 0, i12 = 0;
     if (idx.ne[1] != 1 || idx.ne[2] != 1) {
@@ -1681,6 +1686,7 @@ struct step_head_args {
     float * tab;
 };
 __global__ void __launch_bounds__(1024) k_step_head(const step_head_args h) {
+    args_ahead<sizeof(step_head_args)>();
     int b = (int) blockIdx.x;
     if (b < h.n_rows) {
         const tdesc & a = h.gr_a, & idx = h.gr_idx, & d = h.gr_d;
@@ -1878,6 +1884,7 @@ __global__ void __launch_bounds__(256) k_rope_qk_store(const rope_store_args a) 
 // sums of a chunk are one round trip (77 tokens of Llama-3-8B: 9.2 us a launch of k_rope_qk_store, 6.5 here).
 template <bool NEOX, bool Q8, bool SKP>
 __global__ void __launch_bounds__(256) k_rope_qk_store_vec(const rope_store_args a, const float * __restrict__ tab) {
+    args_ahead<sizeof(rope_store_args)>();
     const int64_t t = blockIdx.x;
     const int tid = threadIdx.x, hd = a.head_dim, half = hd >> 1;
     const int64_t row = a.idx[t];
@@ -2084,6 +2091,7 @@ __device__ __forceinline__ void rope_rows_values(const rope_rows_args & A, const
     }
 }
 __global__ void __launch_bounds__(64) k_rope_rows(const rope_rows_args A) {
+    args_ahead<sizeof(rope_rows_args)>();
     const int h = blockIdx.x;
     const int64_t t = blockIdx.y;
     if (h >= A.H + A.G) {
@@ -2104,6 +2112,7 @@ __global__ void __launch_bounds__(64) k_rope_rows(const rope_rows_args A) {
                });
 }
 __global__ void __launch_bounds__(256) k_rope_rows_many(const rope_rows_args A) {
+    args_ahead<sizeof(rope_rows_args)>();
     const int64_t t = blockIdx.y;
     const int wv = (int) (blockIdx.x * 4 + (threadIdx.x >> 6)), nw = (int) gridDim.x * 4;
     const float pos_f = (float) *(const int32_t *) (A.pos + t * A.pos_nb);

@@ -78,6 +78,7 @@ __global__ void __launch_bounds__(64) k_quantize_q8_0(const char * __restrict__ 
 template <bool SK>
 __global__ void __launch_bounds__(1024) k_rms_norm_mul_q8_K(const char * __restrict__ src, const int64_t nb1, const float * __restrict__ w, const float eps, const int K,
                                                             q8k_dev * __restrict__ dst, const splitk_src sk) {
+    args_ahead<args_bytes<const char *, int64_t, const float *, float, int, q8k_dev *, splitk_src>()>();
     __shared__ double red[16];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int nblk = K / 256;
