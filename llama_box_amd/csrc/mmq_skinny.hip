@@ -197,7 +197,9 @@ __global__ void __launch_bounds__(SK_NW * 64, 1) k_mmq_skinny(const mmq8_args a)
     constexpr int QT = decltype(qt_tag)::value;
     typedef sk_fmt<QT> F;
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    // (a wave's walk over units in scalar registers: up to 8 columns, where it is what a unit waits for, 3 sequences of an 8B model 2642 -> 2571 us a step, 4 of Qwen2-7B 2686 -> 2599; 9 and 32 columns
+    // 2871 -> 2877 and 3100 -> 3115 with it)
+    const int tid = threadIdx.x, lane = tid & 63, wave = TQ == 1 ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6;
     const int row = lane & 31, g = lane >> 5;
     const int nblk = a.K / 256;
     // work items = (32-row tile, K slice); workgroup j serves items j, j + gridDim.x, ..  (one resident workgroup per CU: the loads
