@@ -474,15 +474,26 @@ __global__ void __launch_bounds__(WV * 64) k_fattn_dec128(const tdesc q, const t
         ti1 = min(trips, ti + share);
         if (ti >= ti1) {
             if (geo.n_splits == 1) {
-                // a token that sees nothing and no combine pass to say so: the CPU's result for such a row is 0 * (1 / 0) = NaN
+                // a token that sees nothing and no combine pass to say so, in the forms a combine pass leaves: with a sink 0 / e^(sink - sink) = 0, else 0 * (1 / 0) = NaN, of which the
+                // quantisers make Q8_K blocks of zeros and Q8_0 blocks whose scale is NaN
+                auto none = [&](const int g) { const float sk = sinks ? sinks[h0 + g] : -INFINITY; return 0.0f / expf(sk - sk); };
+                if constexpr (D == 128 && !FAT) {
+                    if (geo.q8) {
+                        if (wave < g_real / 2) {
+                            const float e = none(2 * wave + (lane >> 5)), t[4] = {e, e, e, e};
+                            wave_quantize_q8_K(t, lane, (q8k_dev *) geo.q8 + ((int64_t) bat * geo.n_q + tok) * (geo.n_head * D / 256) + h0 / 2 + wave);
+                        }
+                        return;
+                    }
+                }
                 if (PART && D == 64 && geo.q80) {
                     for (int e = tid; e < g_real * (D / 32); e += WV * 64)
-                        *(float *) ((char *) geo.q80 + ((size_t) (tok >> 5) * (size_t) (geo.n_head * D / 32) + (size_t) (h0 * (D / 32) + e)) * 1152 + 1024 + (tok & 31) * 4) = __builtin_nanf("");
+                        *(float *) ((char *) geo.q80 + ((size_t) (tok >> 5) * (size_t) (geo.n_head * D / 32) + (size_t) (h0 * (D / 32) + e)) * 1152 + 1024 + (tok & 31) * 4) = none(e / (D / 32));
                     return;
                 }
                 for (int e = tid; e < g_real * D; e += WV * 64) {
                     float * out = (float *) (dst.data + (int64_t) (h0 + e / D) * dst.nb[1] + (int64_t) tok * dst.nb[2] + (int64_t) bat * dst.nb[3]);
-                    out[e % D] = __builtin_nanf("");
+                    out[e % D] = none(e / D);
                 }
             } else if (tid < g_real) {
                 float * rec = ws + ((((int64_t) bat * geo.n_q + tok) * geo.n_head + h0 + tid) * geo.n_splits + split) * (D + 2);

@@ -370,6 +370,54 @@ def test_one_pass_of_head_pairs(backend, H, T_, n_kv, NH, NKV, HD, seen, q8, sin
         assert np.abs(got[:, h] - ref).max() <= 1e-3 * np.abs(ref).max() + 1e-5, h
 
 
+# one token of a batch on lists sees nothing: with sinks its result is zero (all weight is the sink's), without them NaN, of which quantisers make Q8_K blocks of zeros and Q8_0 scales of NaN; f32 rows and
+# such blocks (whose scratch holds another step's before), pairs of heads and whole groups
+@pytest.mark.parametrize("T_,n_kv,NH,NKV,HD,seen,kq,sinks,reader", [
+    (3, 900, 8, 2, 128, 300, False, True, None), (3, 900, 8, 2, 128, 300, False, False, None), (5, 500, 8, 2, 128, 200, True, True, None), (4, 1024, 7, 1, 64, 200, False, True, None), (4, 1024, 8, 2, 64, 900, False, False, None),
+    (24, 640, 32, 8, 128, 100, False, True, None), (3, 900, 8, 2, 128, 300, False, True, "Q4_K"), (3, 900, 8, 2, 128, 300, False, False, "Q4_K"), (24, 640, 32, 8, 128, 100, False, False, "Q4_K"),
+    (24, 640, 16, 8, 128, 100, True, True, "Q6_K"), (4, 1024, 8, 2, 64, 200, False, False, "Q8_0"), (4, 1024, 8, 2, 64, 900, False, False, "Q8_0"), (4, 1024, 8, 2, 64, 200, False, True, "Q8_0")])
+def test_token_without_cells(backend, H, T_, n_kv, NH, NKV, HD, seen, kq, sinks, reader):
+    """one pass against splits and their merge (option fa_splits), where the merge speaks for such a token"""
+    rng = np.random.default_rng(T_ + n_kv + NH)
+    q = rng.standard_normal((NH, T_, HD)).astype(np.float32)
+    k, v = (T.rand_weight(L.Q8_0, HD, n_kv * NKV, rng) if kq else rng.standard_normal((NKV, n_kv, HD)).astype(np.float16) for _ in range(2))
+    sk = rng.standard_normal(NH).astype(np.float32)
+    w = T.rand_weight(getattr(L, reader), NH * HD, 96, rng) if reader else None
+    full = np.full((64, n_kv), -np.inf, np.float32)
+    for t in range(T_):
+        full[t, rng.choice(n_kv, seen, replace=False)] = 0
+    blind = full.copy()
+    blind[T_ // 2] = -np.inf
+
+    def build(mask):
+        def f(g):
+            kt = L.Q8_0 if kq else L.F16
+            a = H.ggml_flash_attn_ext(g.ctx, g.new(L.F32, [HD, T_, NH], q), g.new(kt, [HD, n_kv, NKV], k), g.new(kt, [HD, n_kv, NKV], v), H.ggml_cast(g.ctx, g.new(L.F32, [n_kv, 64], mask, "KQ_mask"), L.F16),
+                                      HD ** -0.5, 0.0, 0.0)
+            H.ggml_flash_attn_ext_set_prec(a, 10)
+            if sinks:
+                H.ggml_flash_attn_ext_add_sinks(a, g.new(L.F32, [NH], sk))
+            return H.ggml_mul_mat(g.ctx, g.new(getattr(L, reader), [NH * HD, 96], w), H.ggml_reshape_2d(g.ctx, a, NH * HD, T_)) if reader else a
+        return f
+
+    def run(mask):
+        k0 = backend.stat("kernel_launches")
+        return T.run_case(build(mask), backend)[0].reshape(T_, -1), backend.stat("kernel_launches") - k0
+
+    run(full)
+    got, n_got = run(blind)
+    backend.set_option("fa_splits", 3)
+    try:
+        ref, n_ref = run(blind)
+    finally:
+        backend.set_option("fa_splits", 0)
+    assert n_got < n_ref or (sinks and reader == "Q8_0")
+    t = T_ // 2
+    assert np.array_equal(got[t], ref[t], equal_nan=True) and (np.isnan(ref[t]).all() if not sinks and reader in (None, "Q8_0") else (ref[t] == 0).all())
+    # (f32 sums in another order; an 8-bit value next to a rounding boundary moves by 1 / 127 of its block's largest, few of them)
+    assert T.nmse(np.delete(got, t, 0), np.delete(ref, t, 0)) <= 1e-6
+
+
 # trips of 512 cells with eight waves (16, 32 and 64 rows of V^T a workgroup) and of 256 with four, the last tile and the last trip in part, waves without a tile; whole rows from 80 pairs of
 # a token and a key head and 64 cells a token on (their 256- and 512-cell limits on both sides)
 @pytest.mark.parametrize("T_,NKV,G,per", [
