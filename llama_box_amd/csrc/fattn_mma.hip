@@ -314,7 +314,17 @@ __global__ void __launch_bounds__(NW * 64, 2) k_fattn_mma(const tdesc q, const t
 // not an online one: PASS 1 leaves (max, sum of e^(w - max)) per (query, head, KV split); PASS 2 combines those into the row's maximum and sum,
 // recomputes the scores, takes p = e^(w - max) * (1 / sum) — rounded to f16 where the CPU's second MUL_MAT rounds its src1 — and multiplies with
 // the TRANSPOSED V cache, whose rows need no transposition on the way into LDS.  Partial outputs of KV splits simply add (k_fattn_combine_rows
-// with coefficients 1).  (Head dimension 64 had the three launches until its own two passes: a 2000-token prompt of the small model 24.5 -> 15.5 ms, 14.8 with the one launch below.)  llama-box's zero-sum guard (ggml-cpu.patch:5-15) and the NaN row of a query that sees nothing are kept.
+// with coefficients 1).  (Head dimension 64 had the three launches until its own two passes: a 2000-token prompt of the small model 24.5 -> 15.4 ms, with the one launch below for its first half.)  llama-box's zero-sum guard (ggml-cpu.patch:5-15) and the NaN row of a query that sees nothing are kept.
+// What a row's soft-max is made of.  Heads of 64 were served by the three launches before, whose SOFT_MAX takes expf and adds in 64 bits: so they do here (in 32 bits, 31 weights of 2^-24.1 behind one of 1
+// in one lane were lost: 1.3e-6 of the sum).  A small model's prompts with 32-bit sums and powers of two / so, us: 250 tokens 2273 / 2289, 512 3280 / 3324, 1000 6750 / 6845, 2000 14510 / 15370.  Heads of 128
+// have had two passes with 32-bit statistics from the start.
+template <int D> struct nf_stat { typedef float sum; float m; sum l; };
+template <> struct nf_stat<64> { typedef double sum; float m; sum l; };
+template <int D> __device__ __forceinline__ float nf_exp(const float x) { return D == 64 ? expf(x) : __builtin_amdgcn_exp2f(x * 1.4426950408889634f); }
+template <int D> __device__ __forceinline__ typename nf_stat<D>::sum nf_scale(const float from, const float to) {  // e^(from - to)
+    if constexpr (D == 64) return exp((double) from - (double) to);
+    else return __builtin_amdgcn_exp2f((from - to) * 1.4426950408889634f);
+}
 template <int D, int NW, int PASS>
 __global__ void __launch_bounds__(NW * 64, 2) k_attn_nf_mma(const tdesc q, const tdesc k, const tdesc vt, const tdesc mask, const tdesc dst, const fam_geom geo, float * __restrict__ stats,
                                                          float * __restrict__ ws, const uint8_t * __restrict__ vis) {
@@ -346,18 +356,18 @@ __global__ void __launch_bounds__(NW * 64, 2) k_attn_nf_mma(const tdesc q, const
     const float * mrow = (const float *) (mask.data + (int64_t) qrow * mask.nb[1] + (int64_t) (bat % mask.ne[3]) * mask.nb[3]);
     const char * kbase = k.data + (int64_t) kvh * k.nb[2] + kb * k.nb[3];
     const char * vtbase = vt.data + (int64_t) kvh * vt.nb[2] + vb * vt.nb[3];  // row d of the head at + d * vt.nb[1], cells contiguous
-    constexpr float LOG2E = 1.4426950408889634f;
     const int64_t srow_id = ((int64_t) bat * geo.n_q + qrow) * geo.n_head + h;  // this lane's (query, head) row of the statistics / records
 
     // PASS 2: the row's maximum and sum from the splits' statistics (ggml: max over the row, sum of expf(w - max), 1 / sum; zero-sum guard)
+    typedef nf_stat<D> stat;
+    stat * const st = (stat *) stats + srow_id * geo.n_splits;
     float m_g = -INFINITY, inv = 0.0f;
     if constexpr (PASS == 2) {
-        const float * st = stats + srow_id * geo.n_splits * 2;
-        for (int u = 0; u < geo.n_splits; ++u) m_g = fmaxf(m_g, st[2 * u]);
+        for (int u = 0; u < geo.n_splits; ++u) m_g = fmaxf(m_g, st[u].m);
         double sum = 0.0;
         for (int u = 0; u < geo.n_splits; ++u) {
-            const float mu = st[2 * u];
-            if (mu != -INFINITY) sum += (double) st[2 * u + 1] * (double) __builtin_amdgcn_exp2f((mu - m_g) * LOG2E);
+            const float mu = st[u].m;
+            if (mu != -INFINITY) sum += (double) st[u].l * nf_scale<D>(mu, m_g);
         }
         if (m_g == -INFINITY) sum = __builtin_nan("");  // expf(-inf - -inf) in every cell
         if (isnan(sum) || sum == 0.0) sum = -INFINITY;
@@ -370,7 +380,8 @@ __global__ void __launch_bounds__(NW * 64, 2) k_attn_nf_mma(const tdesc q, const
 #pragma unroll
         for (int r = 0; r < 16; ++r) O[dt][r] = 0.0f;
     const float16v zero = O[0];
-    float m = -INFINITY, l = 0.0f;
+    float m = -INFINITY;
+    typename stat::sum l = 0;
 
     const int srow = tid / NW, spart = tid % NW;
     constexpr int CH = D / (8 * NW);
@@ -492,14 +503,14 @@ __global__ void __launch_bounds__(NW * 64, 2) k_attn_nf_mma(const tdesc q, const
             const float m_new = fmaxf(m, mx);
             if (__all(m_new == -INFINITY)) continue;
             const float mref = m_new == -INFINITY ? 0.0f : m_new;
-            const float alpha = __builtin_amdgcn_exp2f((m - mref) * LOG2E);
-            float rs = 0.0f;
+            typename stat::sum rs = 0;
 #pragma unroll
             for (int t = 0; t < 2; ++t)
 #pragma unroll
-                for (int r = 0; r < 16; ++r) rs += __builtin_amdgcn_exp2f((S[t][r] - mref) * LOG2E);
+                for (int r = 0; r < 16; ++r) rs += nf_exp<D>(S[t][r] - mref);
             rs += __shfl_xor(rs, 32, 64);
-            l = l * alpha + rs;
+            if (D != 64 || __any(m != mref)) l *= nf_scale<D>(m, mref);
+            l += rs;
             m = m_new;
         } else {
             if (__all(m_g == -INFINITY)) continue;
@@ -509,7 +520,7 @@ __global__ void __launch_bounds__(NW * 64, 2) k_attn_nf_mma(const tdesc q, const
                 for (int s2 = 0; s2 < 2; ++s2) {
                     half8 pb;
 #pragma unroll
-                    for (int u = 0; u < 8; ++u) pb[u] = (_Float16) (__builtin_amdgcn_exp2f((S[t][8 * s2 + u] - m_g) * LOG2E) * inv);
+                    for (int u = 0; u < 8; ++u) pb[u] = (_Float16) (nf_exp<D>(S[t][8 * s2 + u] - m_g) * inv);
                     const int kvg = 8 * t + 4 * s2 + kg;
 #pragma unroll
                     for (int dt = 0; dt < ND; ++dt) {
@@ -524,11 +535,7 @@ __global__ void __launch_bounds__(NW * 64, 2) k_attn_nf_mma(const tdesc q, const
     }
     if (qi >= geo.n_q) return;
     if constexpr (PASS == 1) {
-        if (kg == 0) {
-            float * st = stats + (srow_id * geo.n_splits + split) * 2;
-            st[0] = m;
-            st[1] = l;
-        }
+        if (kg == 0) st[split] = {m, l};
     } else {
         const bool nan_row = m_g == -INFINITY;  // the query sees nothing: the CPU's row is NaN throughout
         if (geo.n_splits == 1) {
@@ -570,11 +577,12 @@ template <int D, int NT, int QT, int HP>
 __global__ void __launch_bounds__(512, 2) k_attn_nf_once(const tdesc q, const tdesc k, const tdesc vt, const tdesc mask, const tdesc dst, const fam_geom geo, q8k_dev * __restrict__ q8) {
     args_ahead<args_bytes<tdesc, tdesc, tdesc, tdesc, tdesc, fam_geom>()>();
     constexpr int NS = D / 32, ND = D / 16, PS = D + 4, QS = D + 8, NC = 16 * QT, NQ = NC / HP;
-    constexpr float LOG2E = 1.4426950408889634f;
+    typedef typename nf_stat<D>::sum sum_t;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     float * part = (float *) smem;          // [wave][column][PS], once the queries have been read:
     _Float16 * qs = (_Float16 *) smem;      // [column][QS]
-    __shared__ float st_m[8][NC], st_l[8][NC];
+    __shared__ float st_m[8][NC];
+    __shared__ sum_t st_l[8][NC];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int col = lane & 15, quad = lane >> 4;
     const int h0 = HP * (int) blockIdx.y, kvh = h0 / (geo.n_head / geo.n_kv_head), q0 = (int) blockIdx.x * NQ;
@@ -670,20 +678,21 @@ __global__ void __launch_bounds__(512, 2) k_attn_nf_once(const tdesc q, const td
         if (quad == 0) st_m[wave][16 * j + col] = m[j];
     }
     __syncthreads();
-    float l[QT], inv[QT];
+    sum_t l[QT];
+    float inv[QT];
 #pragma unroll
     for (int j = 0; j < QT; ++j) {
         float mg = -INFINITY;
 #pragma unroll
         for (int w = 0; w < 8; ++w) mg = fmaxf(mg, st_m[w][16 * j + col]);
         const float mref = mg == -INFINITY ? 0.0f : mg;  // (a query that sees nothing: zeros here, NaN below)
-        l[j] = 0.0f;
+        l[j] = 0;
 #pragma unroll
         for (int t = 0; t < NT; ++t)
             if ((seen >> t) & 1) {
 #pragma unroll
                 for (int r = 0; r < 8; ++r) {
-                    S[t][j][r] = __builtin_amdgcn_exp2f((S[t][j][r] - mref) * LOG2E);
+                    S[t][j][r] = nf_exp<D>(S[t][j][r] - mref);
                     l[j] += S[t][j][r];
                 }
             }
@@ -851,9 +860,13 @@ bool attn_nf_mma_applies(const tdesc & q, const tdesc & k, const tdesc & vt, con
     if (vt.nb[0] != 2 || (vt.nb[1] % 16) || (vt.nb[2] % 16) || (((uintptr_t) vt.data) & 15) || (mask.nb[1] % 16) || (((uintptr_t) mask.data) & 15) || mask.ne[0] < k.ne[1] || mask.ne[1] < q.ne[1]) return false;
     return true;
 }
-size_t attn_nf_mma_ws_bytes(const tdesc & q, int n_splits) {  // [statistics: rows x splits x 2][records: rows x splits x (D + 2)]
+static size_t nf_stats_bytes(const tdesc & q, int n_splits) {
     const size_t rows = (size_t) q.ne[1] * (size_t) q.ne[2];
-    return ((rows * (size_t) n_splits * 2 * sizeof(float) + 255) & ~(size_t) 255) + (n_splits > 1 ? rows * (size_t) n_splits * (128 + 2) * sizeof(float) : 0);
+    return (rows * (size_t) n_splits * (q.ne[0] == 64 ? sizeof(nf_stat<64>) : sizeof(nf_stat<128>)) + 255) & ~(size_t) 255;
+}
+size_t attn_nf_mma_ws_bytes(const tdesc & q, int n_splits) {  // [statistics: rows x splits][records: rows x splits x (D + 2)]
+    const size_t rows = (size_t) q.ne[1] * (size_t) q.ne[2];
+    return nf_stats_bytes(q, n_splits) + (n_splits > 1 ? rows * (size_t) n_splits * (128 + 2) * sizeof(float) : 0);
 }
 // dst: the result as [D, head, token] strides in nb[1] (head) / nb[2] (token) — the caller passes kqv's or the CONT copy's layout that way
 void launch_attn_nf_mma(hipStream_t s, const tdesc & q, const tdesc & k, const tdesc & vt, const tdesc & mask, const tdesc & dst, float scale, int n_splits, const uint8_t * tile_vis, void * workspace,
@@ -866,9 +879,8 @@ void launch_attn_nf_mma(hipStream_t s, const tdesc & q, const tdesc & k, const t
     geo.has_mask = 1;
     geo.scale = scale;
     geo.n_splits = std::max(1, n_splits);
-    const size_t rows = (size_t) q.ne[1] * (size_t) q.ne[2];
     float * stats = (float *) workspace;
-    float * recs = (float *) ((char *) workspace + ((rows * (size_t) geo.n_splits * 2 * sizeof(float) + 255) & ~(size_t) 255));
+    float * recs = (float *) ((char *) workspace + nf_stats_bytes(q, geo.n_splits));
     const int tiles_all = (geo.n_kv + 63) / 64, tps = (tiles_all + geo.n_splits - 1) / geo.n_splits;
     const uint8_t * const vis = tps <= 16384 ? tile_vis : nullptr;
     const int D = (int) k.ne[0];

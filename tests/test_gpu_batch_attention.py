@@ -595,6 +595,35 @@ def test_prompt_over_a_short_cache(backend, H, HD, NH, NKV, T_, n_kv, mask_kind)
             assert np.abs(got[t, h] - ref).max() <= 2e-3 * np.abs(ref).max() + 1e-5, (t, h)
 
 
+# heads of 64: the sum of a row's weights is made in 64 bits, as SOFT_MAX makes it.  One weight of 1 and 31 of 2^-24.1 in the cells that one lane adds up (in 32 bits each of them is lost behind the 1), another
+# cell's weight chosen so that the large probability lies 8e-7 of itself below a rounding boundary of f16: without the small ones it would round up
+@pytest.mark.parametrize("NH,NKV,T_,n_kv", [(8, 2, 33, 1024), (3, 1, 40, 1024), (8, 2, 200, 1024), (6, 2, 130, 1000), (8, 2, 40, 2048), (8, 2, 300, 1032), (8, 1, 130, 4096)])
+def test_sums_of_prompt_probabilities(backend, H, NH, NKV, T_, n_kv):
+    HD = 64
+    small = [1, 2, 3] + [8 * i + j for i in range(1, 8) for j in range(4)] if n_kv > 1024 else list(range(1, 8)) + [256 * i + j for i in range(1, 4) for j in range(8)]
+    row = np.full(n_kv, -np.inf, np.float32)
+    row[0], row[small] = 0, -16.7
+    edge = 0.75 + 2.0 ** -12
+    row[63] = np.log((1 + 8e-7) / edge - 1 - np.exp(row[small].astype(np.float64)).sum())
+    p = 1 / np.exp(row.astype(np.float64)).sum()
+    assert len(small) == 31 and 7e-7 < 1 - p / edge < 9e-7 and 3e-7 < p * (1 + 31 * p * np.exp(-16.7)) / edge - 1
+    v = np.zeros((NKV, HD, n_kv), np.float16)
+    v[:, :, 0] = 1 + np.arange(HD) % 2
+
+    def build(g):
+        kc, vc = g.new(L.F16, [NKV * HD, n_kv], np.ones((n_kv, NKV * HD), np.float16)), g.new(L.F16, [n_kv, NKV * HD], v.reshape(-1, n_kv))
+        qp = H.ggml_permute(g.ctx, g.new(L.F32, [HD, NH, T_], np.zeros((T_, NH, HD), np.float32)), 0, 2, 1, 3)
+        kv = H.ggml_view_3d(g.ctx, kc, HD, n_kv, NKV, NKV * HD * 2, HD * 2, 0)
+        vv = H.ggml_view_3d(g.ctx, vc, n_kv, HD, NKV, n_kv * 2, n_kv * 2 * HD, 0)
+        p = H.ggml_soft_max_ext(g.ctx, H.ggml_mul_mat(g.ctx, kv, qp), g.new(L.F32, [n_kv, T_], np.tile(row, (T_, 1))), HD ** -0.5, 0.0)
+        return H.ggml_cont_2d(g.ctx, H.ggml_permute(g.ctx, H.ggml_mul_mat(g.ctx, vv, p), 0, 2, 1, 3), HD * NH, T_)
+
+    c0 = backend.stat("nf_mma_chains")
+    got = T.run_case(build, backend)[0].reshape(T_, NH, HD)
+    assert backend.stat("nf_mma_chains") == c0 + 1
+    assert np.array_equal(got, np.broadcast_to(np.float16(p).astype(np.float32) * v[0, :, 0].astype(np.float32), got.shape))
+
+
 @pytest.mark.parametrize("recycled", [False, True])
 @pytest.mark.parametrize("NH,NKV,T_", [(8, 2, 41), (8, 2, 160), (6, 2, 50)])
 def test_prompt_over_a_short_cache_feeds_a_quantised_matrix(backend, H, NH, NKV, T_, recycled):
