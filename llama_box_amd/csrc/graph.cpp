@@ -2427,7 +2427,7 @@ static int try_fuse_rope_rows(exec_state & st, int i) {
         return (t->type == GGML_TYPE_F32 || t->type == GGML_TYPE_BF16 || t->type == GGML_TYPE_F16) && t->nb[0] == ggml_abi_type_size(t->type) && t->ne[0] == n && t->ne[2] == 1 && t->ne[3] == 1 && src->ne[0] == n &&
                src->ne[1] == T && src->ne[2] == 1 && src->ne[3] == 1;
     };
-    if (!cache_ok(sk, sk->src[0], DK * kx->ne[1]) || !cache_ok(sv, v, row_v) || (ad && !ggml_abi_is_contiguous(v)) || idx != sv->src[1] || idx->type != GGML_TYPE_I64 || !ggml_abi_is_contiguous(idx) ||
+    if (!cache_ok(sk, sk->src[0], DK * kx->ne[1]) || !ggml_abi_is_contiguous(sk->src[0]) /* a token's heads, not other rows of the same block */ || !cache_ok(sv, v, row_v) || (ad && !ggml_abi_is_contiguous(v)) || idx != sv->src[1] || idx->type != GGML_TYPE_I64 || !ggml_abi_is_contiguous(idx) ||
         ggml_abi_nelements(idx) != T || idx->op != GGML_OP_NONE)
         return 0;
     // (every wave reads its own head before it writes: the queries' result may be the projection's own block, nothing else that the launch reads)
