@@ -823,6 +823,7 @@ static enum ggml_status be_graph_compute(ggml_backend_t be, ggml_cgraph * g) {
     flush_uploads(c);
     uploader_join(c->device, c->stream);  // weights staged by set_tensor are complete before the first kernel reads them
     c->up_behind = true;
+    if (c->result.host) note_download(c, c->result.host, c->result.bytes);  // (here, not where it was asked for: a synchronize between the two has nothing to wait for)
     return graph_compute(c, g);
 }
 static void be_event_record(ggml_backend_t be, ggml_backend_event_t ev) {
@@ -1021,7 +1022,6 @@ static int api_result_to(ggml_backend_t be, const ggml_tensor * t, void * host, 
     backend_ctx * c = (backend_ctx *) be->context;
     c->result = {};
     if (!c->opt.small_downloads || size == 0 || size != ggml_abi_nbytes(t) || t->type != GGML_TYPE_F32 || !ggml_abi_is_contiguous(t) || t->data == nullptr || t->ne[1] < 2 || ((uintptr_t) host & 15) || !is_pinned_range(host, size) || ip_any() || tp_active(c)) return 0;
-    note_download(c, host, size);
     c->result.src = t->data;
     c->result.host = (char *) host;
     c->result.bytes = size;

@@ -1024,6 +1024,45 @@ def test_uploads_wait_for_the_download_that_fills_their_source(backend, H, nbyte
             other.close()
 
 
+def result_to(backend):
+    return backend.proc("ggml_backend_mi355x_result_to", C.c_int, [C.c_void_p, L.TP, C.c_void_p, C.c_size_t])
+
+
+@pytest.mark.parametrize("product", [True, False])
+def test_uploads_wait_for_the_result_that_fills_their_source(backend, H, product):
+    """... asked for before a synchronize that the graph itself comes behind; stored by the graph's last product, or copied behind the graph"""
+    P, SZ = C.c_void_p, C.c_size_t
+    H.ggml_backend_tensor_set_async.argtypes = [P, L.TP, P, SZ, SZ]
+    H.ggml_backend_graph_compute_async.argtypes = [P, C.POINTER(L.CGraph)]
+    rng = np.random.default_rng(2)
+    K, M = 8192, 64
+    g = T.G(backend)
+    pin = None
+    try:
+        w = g.new(L.Q8_0, [K, K], T.rand_weight(L.Q8_0, K, K, rng))
+        cur = g.new(L.F32, [K, M], rng.standard_normal((M, K)).astype(np.float32))
+        for _ in range(60):
+            cur = H.ggml_mul_mat(g.ctx, w, cur)
+        if not product:
+            cur = H.ggml_scale(g.ctx, cur, 0.5)
+        u = g.new(L.F32, [K, M], np.zeros((M, K), np.float32))
+        ref = g.compute([cur])[0].view(np.uint8)
+        pin = H.ggml_backend_buft_alloc_buffer(H.ggml_backend_dev_host_buffer_type(backend.dev), M * K * 4)
+        base = H.ggml_backend_buffer_get_base(pin)
+        for _ in range(3):
+            C.memset(base, 0x55, M * K * 4)
+            assert result_to(backend)(backend.backend, cur, base, M * K * 4) == 1
+            H.ggml_backend_synchronize(backend.backend)
+            assert H.ggml_backend_graph_compute_async(backend.backend, g.gf) == 0
+            H.ggml_backend_tensor_set_async(backend.backend, u, base, 0, M * K * 4)
+            H.ggml_backend_synchronize(backend.backend)
+            assert np.array_equal(g.read(u).view(np.uint8).ravel(), ref.ravel())
+    finally:
+        if pin:
+            H.ggml_backend_buffer_free(pin)
+        g.free()
+
+
 # the logits of several columns, stored by the output product in the pinned output area (option small_downloads) or copied there: eager, captured and replayed steps, rows at the kernels' edges (2 .. 64 columns)
 @pytest.mark.parametrize("name", ["test-llama", "tinyllama-1.1b-q8_0", "llama3-8b-q4_k_m"])
 @pytest.mark.parametrize("cols", [1, 2, 9, 17, 33, 64, 70])
