@@ -757,6 +757,17 @@ static void be_set_tensor_async(ggml_backend_t be, ggml_tensor * t, const void *
     if (at_once && stage_upload(c, (char *) t->data + offset, data, size)) return;
     HIP_SOFT(hipMemcpyAsync((char *) t->data + offset, data, size, hipMemcpyHostToDevice, c->stream));
 }
+// n bytes of device memory to the host, in the stream.  The logits of a decode step (513 KB per sequence, llama.cpp's pinned output buffer): a blit through hipMemcpyAsync starts ~20 us after
+// the graph's last kernel and takes 10 us; a copy kernel writing the mapped pinned memory is an ordinary
+// launch behind that kernel.  Only into memory of OUR host buffer type (known to be device-mapped), up to 8 MiB.
+void download(backend_ctx * c, void * host, const void * src, size_t n) {
+    if (c->opt.small_downloads && n > 0 && n <= ((size_t) 8 << 20) && is_pinned_range(host, n)) {
+        launch_upload_small(c->stream, host, src, n);
+        c->st.kernel_downloads++;
+        return;
+    }
+    HIP_SOFT(hipMemcpyAsync(host, src, n, hipMemcpyDeviceToHost, c->stream));
+}
 static void be_get_tensor_async(ggml_backend_t be, const ggml_tensor * t, void * data, size_t offset, size_t size) {
     backend_ctx * c = (backend_ctx *) be->context;
     if (ip_any()) ip_host_access(t->view_src ? t->view_src->buffer : t->buffer, false);
@@ -764,15 +775,7 @@ static void be_get_tensor_async(ggml_backend_t be, const ggml_tensor * t, void *
     flush_uploads(c);
     uploader_join(c->device, c->stream);
     note_download(c, data, size);
-    // The logits of a decode step (513 KB per sequence, llama.cpp's pinned output buffer): a blit through hipMemcpyAsync starts ~20 us after
-    // the graph's last kernel and takes 10 us (profiles/r05_decode_gaps_*.txt); a copy kernel writing the mapped pinned memory is an ordinary
-    // launch behind that kernel.  Only into memory of OUR host buffer type (known to be device-mapped), up to 8 MiB.
-    if (c->opt.small_downloads && size > 0 && size <= ((size_t) 8 << 20) && is_pinned_range(data, size)) {
-        launch_upload_small(c->stream, data, (const char *) t->data + offset, size);
-        c->st.kernel_downloads++;
-        return;
-    }
-    HIP_SOFT(hipMemcpyAsync(data, (const char *) t->data + offset, size, hipMemcpyDeviceToHost, c->stream));
+    download(c, data, (const char *) t->data + offset, size);
 }
 static bool be_is_ours(ggml_backend_t be);
 static bool be_cpy_tensor_async(ggml_backend_t be_src, ggml_backend_t be_dst, const ggml_tensor * src, ggml_tensor * dst) {

@@ -369,6 +369,7 @@ void free_split_helpers(backend_ctx * c);
 // ---- graph execution (graph.cpp) ----
 bool supports_op(const ggml_tensor * op);
 enum ggml_status graph_compute(backend_ctx * ctx, ggml_cgraph * g);
+void download(backend_ctx * c, void * host, const void * src, size_t n);  // device memory to the host, behind what the stream holds (backend.cpp)
 void free_graph_cache(backend_ctx * ctx);
 bool graph_key_equals(const ggml_cgraph * g, const std::vector<uint64_t> & key);  // the graph-key words (graph.cpp: walk_key), compared in place ...
 int64_t partials_reserved(const ggml_cgraph * g);  // bytes of scratch behind the activations that a backend with the default options sets aside for the graph

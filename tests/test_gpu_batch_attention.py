@@ -322,7 +322,7 @@ def test_splits_of_few_tokens(backend, H, T_, n_kv, NH, NKV, HD, seen):
 # one pass over all cells, two heads of a key head a workgroup, at the lines between it and the splits; group sizes that leave a last pair in part, Q8_0 rows, sinks, tokens on lists
 @pytest.mark.parametrize("T_,n_kv,NH,NKV,HD,seen,q8,sinks,launches", [
     (1, 1, 7, 1, 128, 0, False, False, 1), (1, 255, 14, 2, 128, 0, False, True, 1), (1, 768, 14, 2, 128, 0, False, False, 1), (1, 772, 14, 2, 128, 0, False, False, 2), (1, 512, 8, 2, 128, 0, False, False, 1),
-    (1, 513, 8, 2, 128, 0, False, False, 2), (1, 257, 5, 1, 128, 0, True, False, 2), (1, 256, 6, 2, 128, 0, True, True, 1), (1, 70, 3, 3, 64, 0, False, False, 1), (1, 1024, 32, 4, 64, 0, False, True, 1),
+    (1, 513, 8, 2, 128, 0, False, False, 2), (1, 1, 4, 1, 128, 0, False, False, 1), (1, 256, 32, 8, 128, 0, False, True, 1), (1, 200, 6, 2, 128, 0, False, False, 1), (1, 257, 5, 1, 128, 0, True, False, 2), (1, 256, 6, 2, 128, 0, True, True, 1), (1, 70, 3, 3, 64, 0, False, False, 1), (1, 1024, 32, 4, 64, 0, False, True, 1),
     (1, 1025, 10, 2, 64, 0, False, False, 2), (2, 900, 8, 2, 128, 384, False, True, 2), (3, 900, 8, 2, 128, 385, False, False, 3), (17, 640, 16, 8, 128, 130, False, False, 2), (6, 500, 8, 2, 128, 256, True, False, 2),
     (6, 500, 12, 2, 128, 257, True, False, 3), (4, 4096, 7, 1, 64, 1000, False, True, 2), (4, 4096, 8, 1, 64, 200, False, False, 2), (32, 640, 24, 8, 64, 256, False, False, 2), (32, 644, 24, 8, 64, 257, False, False, 2)])
 def test_one_pass_of_head_pairs(backend, H, T_, n_kv, NH, NKV, HD, seen, q8, sinks, launches):

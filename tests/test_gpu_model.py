@@ -1028,6 +1028,34 @@ def result_to(backend):
     return backend.proc("ggml_backend_mi355x_result_to", C.c_int, [C.c_void_p, L.TP, C.c_void_p, C.c_size_t])
 
 
+@pytest.mark.parametrize("cols,launches", [(2, 1), (64, 1), (600, 0)])
+def test_result_behind_a_graph_that_ends_in_no_product(backend, H, cols, launches):
+    """a target of a graph whose last node cannot store it itself (logits scaled or capped behind their product): copied behind the graph as get_tensor_async copies, up to 8 MiB by a copy kernel"""
+    H.ggml_backend_graph_compute_async.argtypes = [C.c_void_p, C.POINTER(L.CGraph)]
+    K, N = 256, 4096
+    rng = np.random.default_rng(cols)
+    g = T.G(backend)
+    pin = None
+    try:
+        w, x = g.new(L.Q4_K, [K, N], T.rand_weight(L.Q4_K, K, N, rng)), g.new(L.F32, [K, cols], rng.standard_normal((cols, K)).astype(np.float32))
+        out = H.ggml_scale(g.ctx, H.ggml_mul_mat(g.ctx, w, x), 0.5)
+        ref = g.compute([out])[0].reshape(cols, N)
+        pin = H.ggml_backend_buft_alloc_buffer(H.ggml_backend_dev_host_buffer_type(backend.dev), cols * N * 4)
+        base = H.ggml_backend_buffer_get_base(pin)
+        for _ in range(3):
+            C.memset(base, 0x55, cols * N * 4)
+            d0 = backend.stat("kernel_downloads")
+            assert result_to(backend)(backend.backend, out, base, cols * N * 4) == 1
+            assert H.ggml_backend_graph_compute_async(backend.backend, g.gf) == 0
+            H.ggml_backend_synchronize(backend.backend)
+            assert np.array_equal(np.ctypeslib.as_array(C.cast(base, C.POINTER(C.c_float)), (cols, N)), ref)
+            assert backend.stat("kernel_downloads") - d0 == launches
+    finally:
+        if pin:
+            H.ggml_backend_buffer_free(pin)
+        g.free()
+
+
 @pytest.mark.parametrize("product", [True, False])
 def test_uploads_wait_for_the_result_that_fills_their_source(backend, H, product):
     """... asked for before a synchronize that the graph itself comes behind; stored by the graph's last product, or copied behind the graph"""
