@@ -82,9 +82,13 @@ template <typename T, bool PIPE> __device__ __forceinline__ void qkv_unit(qkv_re
 // f16-cache kernel does not have to spare)
 // BND: the workgroup size the kernel is compiled for.  1024 caps a wave at 128 registers, which the Q5_K register sets exceed by a few (6 .. 16 dwords of scratch:
 // a launch with a scratch frame pays for it at every dispatch); Qwen2-7B's launches use 9 waves, so the Q5_K forms also exist compiled for 640 threads (round 6)
+// The arguments are fetched ahead except by the pairs of formats that fill the 128 registers of 1024 threads: there it cost 4 .. 16 bytes of scratch.  us a launch with it / without (16 layers of one width):
+// 4096 x (4096 + 2 x 4096) Q4_K + Q6_K 14.20 / 13.62, 5120 x 3 x 5120 Q5_K 22.84 / 22.36, Q5_K + Q6_K 23.81 / 23.75, 4096 x (4096 + 2 x 1024) Q6_K 8.87 / 8.93 (a step of that model 953 / 948 us).
+template <typename TA, typename TB> constexpr bool qkv_full_of = std::is_same<TA, T_Q5KP>::value || std::is_same<TA, T_Q5KS>::value || std::is_same<TB, T_Q5KP>::value || std::is_same<TB, T_Q5KS>::value ||
+                                                                 std::is_same<TB, T_Q6KP>::value || std::is_same<TB, T_Q6KS>::value || (std::is_same<TA, T_Q4K>::value && std::is_same<TB, T_Q5K>::value);
 template <typename TA, typename TB, bool Q8S, bool PIPE = false, int BND = 1024>
 __global__ void __launch_bounds__(PIPE ? 512 : BND) k_qkv_stream2(const qkv_args a) {
-    args_ahead<sizeof(qkv_args)>();
+    if constexpr (PIPE || BND < 1024 || Q8S || !qkv_full_of<TA, TB>) args_ahead<sizeof(qkv_args)>();
     extern __shared__ __attribute__((aligned(16))) char smem[];
     // (a generic lambda, not a device function: passing the kernel-argument struct to a function copies it to scratch)
     // (u_first / GW: this wave's first unit among the segments of its format, and the number of waves that share them)

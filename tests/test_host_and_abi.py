@@ -3,6 +3,7 @@ the host-side mirror (graph construction, allocator, GGUF, llama_decode-shaped d
 import ctypes as C
 import os
 import re
+import struct
 import tempfile
 
 import numpy as np
@@ -532,3 +533,42 @@ def test_scratch_holds_the_slices_of_merged_launches():
                 short.append((K, nq, nkv, M, types, need, got))
             H.ggml_free(ctx)
     assert not short, (len(short), short[:5])
+
+
+def built_kernels():
+    """{symbol: metadata} of the gfx950 kernels in the built library (the code objects' AMDGPU metadata notes)"""
+    msgpack = pytest.importorskip("msgpack")
+    with open(L.BACKEND_SO, "rb") as f:
+        d = f.read()
+    out, magic, at = {}, b"__CLANG_OFFLOAD_BUNDLE__", -1
+    while (at := d.find(magic, at + 1)) >= 0:
+        n, p = struct.unpack_from("<Q", d, at + 24)[0], at + 32
+        for _ in range(n):
+            off, size, chars = struct.unpack_from("<QQQ", d, p)
+            target = d[p + 24:p + 24 + chars]
+            p += 24 + chars
+            if size == 0 or b"gfx950" not in target:
+                continue
+            elf = d[at + off:at + off + size]
+            headers, = struct.unpack_from("<Q", elf, 32)
+            for k in range(struct.unpack_from("<H", elf, 56)[0]):
+                kind, _, q, _, _, length = struct.unpack_from("<IIQQQQ", elf, headers + 56 * k)
+                end = q + length
+                while kind == 4 and q < end:  # PT_NOTE
+                    name, desc, note = struct.unpack_from("<III", elf, q)
+                    q += 12 + (name + 3 & ~3)
+                    if note == 32:
+                        out.update((m[".name"], m) for m in msgpack.unpackb(elf[q:q + desc])["amdhsa.kernels"])
+                    q += desc + 3 & ~3
+    return out
+
+
+def test_scratch_of_the_fused_projections():
+    """bytes of scratch a lane of the 1024-thread builds of k_qkv_stream2 (f16 cache), which have no register to spare: a launch with a scratch frame pays for it at every dispatch"""
+    pairs = {"Q4K Q5K": 0, "Q4KP Q5KP": 16, "Q4KP Q6KP": 8, "Q4KS Q5KS": 40, "Q4KS Q6KS": 32, "Q5KP Q6KP": 24, "Q5KP Q5KP": 16, "Q5KS Q6KS": 48, "Q5KS Q5KS": 40, "Q6KP Q6KP": 0, "Q6KS Q6KS": 16,
+             "Q4K Q6K": 0, "Q4K Q4K": 0, "Q5K Q6K": 0, "Q5K Q5K": 0, "Q6K Q6K": 0, "Q80 Q80": 0, "Q4KP Q4KP": 0, "Q4KS Q4KS": 0}
+    kernels = built_kernels()
+    for pair, scratch in pairs.items():
+        a, b = pair.split()
+        symbol = "_ZN6mi355x13k_qkv_stream2INS_%dT_%sE%sLb0ELb0ELi1024EEEvNS_8qkv_argsE" % (len(a) + 2, a, "S1_" if a == b else "NS_%dT_%sE" % (len(b) + 2, b))
+        assert kernels[symbol][".private_segment_fixed_size"] <= scratch, pair
