@@ -1357,7 +1357,7 @@ bool fattn_q80_out_ok(const tdesc & q, const tdesc & k, const tdesc & v, const t
 // One pass over all cells instead of splits and a combine launch (4 us a layer)?  For pairs of query heads per workgroup (k_fattn_dec128: PART) where a token sees few cells: its rows are fetched once a
 // pair, 256 of them a trip on eight waves (128 on four), and a further trip costs what the lines below weigh against the launch saved.  us a step, splits + combine / one pass of pairs:
 //   one token, head_dim 64 (small model, 4 x 8 heads): 120 cells 916 / 800, 400 919 / 840, 1000 916 / 894, 1500 921 / 954 (whole groups in one pass: 923, 1035, 1280, 1527)
-//   one token, head_dim 128: Llama-3-8B 60 cells 1660 / 1563 (not taken, below), 400 1662 / 1638, 700 1660 / 1702; Qwen2-7B (7 heads a group, whose splits run as 8) 100 1827 / 1675, 300 1823 / 1729, 600 1820 / 1784;
+//   one token, head_dim 128: Llama-3-8B 17 cells 1615 / 1526, 60 1614 / 1522, 250 1615 / 1525, 400 1662 / 1638, 700 1660 / 1702; Qwen2-7B (7 heads a group, whose splits run as 8) 100 1827 / 1675, 300 1823 / 1729, 600 1820 / 1784;
 //   Llama-3-8B over Q8_0 rows (four waves) 100 1745 / 1671, 300 1752 / 1810
 //   lists of n x cells, head_dim 64: 2 x 400 1115 / 1060, 2 x 900 1155 / 1127, 16 x 150 1209 / 1130, 16 x 500 1289 / 1222, 32 x 250 1542 / 1466; 9 drafts of 400 1308 / 1116
 //   lists, Llama-3-8B: 2 x 100 2453 / 2339, 2 x 450 2479 / 2510, 4 x 300 2513 / 2489, 8 x 350 2630 / 2566, 8 x 500 2641 / 2637, 16 x 400 2896 / 2839; Q8_0 rows 4 x 100 2542 / 2426, 4 x 300 2554 / 2582,
@@ -1372,7 +1372,6 @@ int fattn_one_pass(const tdesc & q, const tdesc & k, const fattn_params & p, boo
     const int64_t cells = p.seen > 0 ? std::min<int64_t>(p.seen, k.ne[1]) : k.ne[1];
     if (!list) {
         if (q.ne[1] != 1) return 0;
-        if (k.ne[0] == 128 && !q8 && fa_gg(G) == 4 && cells <= 256) return 0;  // (the combine pass stays there: the merge in wo's prologue is checked against it at this size too)
         return cells <= (k.ne[0] == 64 ? 1024 : q8 ? 256 : fa_gg(G) == 8 ? 768 : 512) ? 2 : 0;
     }
     if (k.ne[0] == 64) return cells <= (pairs * ((G + 1) / 2) <= 256 ? 1024 : 256) ? 2 : 0;
