@@ -2369,6 +2369,7 @@ struct llm_context {
     static constexpr size_t GRAPHS_KEPT = 8;
     std::vector<built_graph> built;
     uint64_t graph_tick = 0;
+    int64_t graph_stats[3] = {0, 0, 0};  // llm_graph_stats
     ggml_tensor *inp_tokens = nullptr, *inp_pos = nullptr, *inp_mask = nullptr, *inp_k_idxs = nullptr, *inp_v_idxs = nullptr, *inp_out_ids = nullptr;
     ggml_tensor *inp_bigram = nullptr, *inp_shift_src = nullptr, *inp_shift_last = nullptr, *inp_shift_slot = nullptr;
     ggml_tensor *inp_seq_hist = nullptr, *inp_seq_upd = nullptr, *inp_seq_tok = nullptr, *inp_seq_info = nullptr;
@@ -3311,15 +3312,20 @@ static bool switch_graph(llm_context * c, const graph_key & key) {
         for (built_graph & b : c->built)
             if (b.key == key) {
                 use_graph(c, b);
+                c->graph_stats[1]++;
                 return true;
             }
     while (c->built.size() >= (c->p.graph_reuse ? llm_context::GRAPHS_KEPT : 1))
         drop_graph(c, (size_t) (std::min_element(c->built.begin(), c->built.end(), [](const built_graph & x, const built_graph & y) { return x.used < y.used; }) - c->built.begin()));
     built_graph b = build_graph(c, key);
+    c->graph_stats[0]++;
     const size_t size = ggml_gallocr_get_buffer_size(c->galloc, 0);
     const bool ok = ggml_gallocr_alloc_graph(c->galloc, b.gf);
     if (!ok || ggml_gallocr_get_buffer_size(c->galloc, 0) != size)  // (the buffer that the other graphs lie in is gone)
-        while (!c->built.empty()) drop_graph(c, c->built.size() - 1);
+        while (!c->built.empty()) {
+            drop_graph(c, c->built.size() - 1);
+            c->graph_stats[2]++;
+        }
     if (!ok) {
         ggml_free(b.ctx);
         return false;
@@ -3452,14 +3458,16 @@ extern "C" struct llm_context * llm_context_new(struct llm_model * m, ggml_backe
     c->galloc = ggml_gallocr_new(c->buft);
     // reserve the worst-case graph (full micro-batch over the full cache) so later graphs re-use one buffer
     const int n_most = std::min(c->p.n_ubatch, c->p.n_ctx);
-    c->built.push_back(build_graph(c, {n_most, c->p.n_ctx, n_most, (m->has_shift || m->has_seq_state) ? std::min(c->n_seq_max, n_most) : 0}));
-    use_graph(c, c->built[0]);
-    if (!ggml_gallocr_reserve(c->galloc, c->gf)) {
-        fprintf(stderr, "llm_context_new: failed to reserve the compute buffer\n");
-        llm_context_free(c);
-        return nullptr;
+    if (c->p.graph_reuse != 2) {
+        c->built.push_back(build_graph(c, {n_most, c->p.n_ctx, n_most, (m->has_shift || m->has_seq_state) ? std::min(c->n_seq_max, n_most) : 0}));
+        use_graph(c, c->built[0]);
+        if (!ggml_gallocr_reserve(c->galloc, c->gf)) {
+            fprintf(stderr, "llm_context_new: failed to reserve the compute buffer\n");
+            llm_context_free(c);
+            return nullptr;
+        }
+        c->key = c->built[0].key = graph_key();  // (measured, not laid out)
     }
-    c->key = c->built[0].key = graph_key();  // (measured, not laid out)
     if (backend) {
         ggml_backend_buffer_type_t hbuft = ggml_backend_dev_host_buffer_type(backend->device);
         if (hbuft) {
@@ -3645,6 +3653,9 @@ extern "C" struct llm_context * llm_context_new_layer_split(struct llm_model * m
     c->used_max = 0;
     c->key = graph_key();
     return c;
+}
+extern "C" void llm_graph_stats(const struct llm_context * c, int64_t out[3]) {
+    for (int k = 0; k < 3; ++k) out[k] = c->graph_stats[k];
 }
 extern "C" void llm_layer_split_stats(const struct llm_context * c, int64_t out[4]) {
     for (int k = 0; k < 4; ++k) out[k] = c->ls_stats[k];

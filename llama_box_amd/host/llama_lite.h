@@ -88,7 +88,7 @@ struct llm_context_params {
     int32_t n_ubatch;   /* micro-batch (graph) size; batches are sliced into views of this many tokens */
     int32_t flash_attn; /* 1: FLASH_ATTN_EXT, 0: MUL_MAT/SOFT_MAX/MUL_MAT with transposed V cache */
     int32_t n_threads;  /* for the external compute function */
-    int32_t graph_reuse; /* keep the built graph while the topology key is unchanged */
+    int32_t graph_reuse; /* 1: keep the graphs of the shapes used last, in a compute buffer reserved for the largest; 2: in one that grows with them; 0: build every graph anew */
     int32_t type_k, type_v; /* ggml type of the K / V cache rows (llama-box -ctk / -ctv, engine_param.hpp:51-54): 0 or GGML_TYPE_F16 = f16; GGML_TYPE_Q8_0,
                                Q4_0, Q4_1, IQ4_NL, Q5_0, Q5_1, BF16; LLM_KV_TYPE_F32 = f32 (a V cache other than f16 needs flash_attn, as in llama.cpp) */
     int32_t n_seq_max;  /* sequence ids are 0 .. n_seq_max - 1 for models that keep state per sequence (0 = 8) */
@@ -127,6 +127,8 @@ int llm_kv_seq_rm(struct llm_context * c, int seq_id, int p0, int p1);
 int llm_kv_seq_add(struct llm_context * c, int seq_id, int p0, int p1, int delta);
 /* the graph of the last micro-batch (for inspection / per-node comparison in tests) */
 struct ggml_cgraph * llm_last_graph(struct llm_context * c);
+/* [graphs built for a shape, kept graphs taken again, kept graphs dropped with the buffer that they lay in] since the context was made */
+void llm_graph_stats(const struct llm_context * c, int64_t out[3]);
 struct ggml_tensor * llm_context_cache_tensor(struct llm_context * c, int il, int which); /* K (0) / V (1) cache tensor of layer il */
 /* host-side time split of the last llm_decode, microseconds: [build+alloc, set inputs, compute+sync, get logits] */
 void llm_last_timings(const struct llm_context * c, double out[4]);

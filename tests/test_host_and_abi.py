@@ -193,13 +193,22 @@ def test_driver_on_oracle_determinism_reuse_and_batching(H):
         m.free()
 
 
-def test_graphs_of_several_shapes_are_kept(H):
-    """prompts of more shapes than a context keeps graphs for, in an order that meets kept, dropped and never built ones: the logits of a context that builds every graph anew"""
+@pytest.mark.parametrize("reuse", [1, 2])
+def test_graphs_of_several_shapes_are_kept(H, reuse):
+    """prompts of more shapes than a context keeps graphs for, in an order that meets kept, dropped and never built ones: the logits of a context that builds every graph anew.  (A shape: the tokens of a
+    micro-batch and its cells, up to 256 for all of these.)  In a buffer that grows (2), a larger graph takes the others' memory with it: they are built anew where they come again."""
     fn = T.oracle_compute_fn(2)
     m = Model(preset("test-llama"), 5, H.ggml_backend_cpu_buffer_type())
-    kept, anew = Context(m, compute=fn, graph_reuse=1, n_ubatch=16), Context(m, compute=fn, graph_reuse=0, n_ubatch=16)
+    kept, anew = Context(m, compute=fn, graph_reuse=reuse, n_ubatch=16), Context(m, compute=fn, graph_reuse=0, n_ubatch=16)
     rng = np.random.default_rng(3)
-    for n in [3, 40, 1, 37, 3, 5, 6, 40, 7, 8, 9, 10, 11, 12, 3, 37, 1, 40, 12]:
+
+    def stats(c):
+        out = (C.c_int64 * 3)()
+        H.llm_graph_stats(c.c, out)
+        return list(out)
+
+    held, now, largest, count, anew_count = [None] * (reuse == 1), None, 0, [0, 0, 0], 0  # shapes held, used last at the end (None: the graph that the buffer is reserved for)
+    for n in [3, 1, 2, 5, 3, 40, 1, 37, 3, 5, 6, 40, 7, 8, 9, 10, 11, 12, 3, 37, 1, 40, 12]:
         tok = rng.integers(0, 500, n)
         rows = []
         for c in (kept, anew):
@@ -208,6 +217,24 @@ def test_graphs_of_several_shapes_are_kept(H):
             assert rc == 0
             rows.append(lg)
         assert np.array_equal(*rows), n
+        for at in range(0, n, 16):
+            shape = (min(16, n - at), at + 16 >= n)
+            anew_count += 1
+            if shape == now:
+                continue
+            if shape in held:
+                held.remove(shape)
+                count[1] += 1
+            else:
+                count[0] += 1
+                held = held[-7:]
+                if reuse == 2 and shape[0] > largest:
+                    count[2] += len(held)
+                    held, largest = [], shape[0]
+            held.append(shape)
+            now = shape
+        assert stats(kept) == count and stats(anew) == [anew_count, 0, 0], n
+    assert count[1] > 5 and (count[2] > 3) == (reuse == 2)
     kept.free()
     anew.free()
     m.free()
