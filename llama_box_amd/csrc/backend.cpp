@@ -1109,6 +1109,7 @@ static int64_t api_get_stat(ggml_backend_t be, const char * key) {
     if (k == "graph_launch_host_ns") return c->st.graph_launch_host_ns;
     if (k == "staged_uploads") return c->st.staged_uploads;
     if (k == "kernel_downloads") return c->st.kernel_downloads;
+    if (k == "results_by_graph") return c->st.results_by_graph;
     if (k == "kv_image_nodes") return c->st.kv_image_nodes;
     if (k == "kv_native_nodes") return c->st.kv_native_nodes;
     if (k == "attn_f32_nodes") return c->st.attn_f32_nodes;

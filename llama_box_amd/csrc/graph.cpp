@@ -4031,6 +4031,7 @@ enum ggml_status graph_compute(backend_ctx * c, ggml_cgraph * g) {
     c->result = {};
     const bool inside = want.host && result_node(g, want) >= 0;
     const enum ggml_status st = compute_to(c, g, inside ? want : result_target{});
+    if (st == GGML_STATUS_SUCCESS && inside) c->st.results_by_graph++;
     if (st == GGML_STATUS_SUCCESS && want.host && !inside) download(c, want.host, want.src, want.bytes);
     return st;
 }

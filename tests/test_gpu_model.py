@@ -9,6 +9,7 @@ it.  So the e2e gate is RELATIVE to the oracle's own sensitivity to summation or
 absolute NMSE cap of 1e-3, and greedy ids must match wherever the top-2 margin exceeds the observed deviation.
 The FLASH_ATTN_EXT path is gated against the CPU's own FA-vs-softmax gap (ggml-cpu accumulates V in f16 there)."""
 import ctypes as C
+import json
 import os
 import tempfile
 
@@ -1092,10 +1093,15 @@ def test_uploads_wait_for_the_result_that_fills_their_source(backend, H, product
 
 
 # the logits of several columns, stored by the output product in the pinned output area (option small_downloads) or copied there: eager, captured and replayed steps, rows at the kernels' edges (2 .. 64 columns)
-@pytest.mark.parametrize("name", ["test-llama", "tinyllama-1.1b-q8_0", "llama3-8b-q4_k_m"])
+@pytest.mark.parametrize("name", ["test-llama", "tinyllama-1.1b-q8_0", "llama3-8b-q4_k_m", "nigozen"])
 @pytest.mark.parametrize("cols", [1, 2, 9, 17, 33, 64, 70])
 def test_logits_stored_by_the_output_product(backend, H, name, cols):
-    m = Model(preset(name) if name == "test-llama" else preset(name, n_layer=1, n_vocab=4096), 5, backend.buft)
+    if name == "nigozen":  # (bf16 matrices)
+        mixer = {"heads": 4, "kv_heads": 2, "dim": 64, "vdim": 64, "mask": {"size": 256}, "rot": {"base": 1e6, "dims": 32}, "scale": 0.125, "v_mix": True}
+        m = Model(config_json=json.dumps({"architecture": "Nigozen", "embedding": {"scale": 1.0}, "layers": [{"type": "attention", "mixer": mixer, "mlp": {"kind": "dense", "ff": 512}}], "norm": {"eps": 1e-5},
+                                          "vocab": 4096, "width": 256}), seed=5, buft=backend.buft, wtype=L.BF16)
+    else:
+        m = Model(preset(name) if name == "test-llama" else preset(name, n_layer=1, n_vocab=4096), 5, backend.buft)
     rng = np.random.default_rng(cols)
     tok = rng.integers(0, m.n_vocab_local, (5, cols))
     rows = []
@@ -1105,8 +1111,11 @@ def test_logits_stored_by_the_output_product(backend, H, name, cols):
             c = Context(m, backend=backend, n_ctx=512, flash_attn=1)
             rows.append([])
             for t in tok:  # (the same positions again: a graph seen before)
+                n0 = [backend.stat(k) for k in ("results_by_graph", "kernel_downloads")]
                 rc, lg = c.decode(t, range(cols))
                 assert rc == 0 and lg.shape[0] == cols
+                # (one row: the copy kernel behind the graph; more rows than the output area has: copied to ordinary memory)
+                assert [backend.stat(k) - n for k, n in zip(("results_by_graph", "kernel_downloads"), n0)] == [int(on and 2 <= cols <= 64), int(on and cols == 1)]
                 rows[-1].append(lg)
                 c.seq_rm(-1, 0, -1)
             c.free()
