@@ -904,7 +904,7 @@ void launch_attn_nf_mma(hipStream_t s, const tdesc & q, const tdesc & k, const t
 //   head_dim 128, tokens = cells: Llama-3-8B 40 4189 / 3818, 3881; 77 5106 / 4643, 4697; 128 5613 / 5100, 5142; 200 8408 / 7835, 7778; 350 11379 / 11128, 11142; 512 12920 / 12952, 12686;
 //   700 (its second batch: 188 over 768) 20895 / 20692, 20167; 1000 (488 over 1024) 26157 / 26929, 25904, of which the first batch's 235 are most; Qwen2-7B (single heads) 100 6174 / 5800, 5843,
 //   500 15126 / 15315, 15069
-//   head_dim 64, small model: 512 3678 / 3420, 3310; 1000 7698 / 7327, 7019 (7260 with its second batch in two passes); beyond 1024 cells two passes
+//   head_dim 64, small model, two passes / as chosen: 250 2668 / 2287, 512 3822 / 3362, 1000 7700 / 6921 (7263 with its second batch in two passes); beyond 1024 cells two passes
 bool attn_nf_once_applies(const tdesc & q, const tdesc & k) { return k.ne[1] <= (k.ne[0] == 64 || q.ne[1] <= 256 ? 1024 : 512); }
 bool attn_nf_once_q8(const tdesc & q, const tdesc & k) { return k.ne[0] == 128 && (q.ne[2] / k.ne[2]) % 2 == 0; }  // (pairs of heads of a group: their Q8_K blocks)
 template <int D, int NT, int QT, int HP>

@@ -375,7 +375,8 @@ def test_one_pass_of_head_pairs(backend, H, T_, n_kv, NH, NKV, HD, seen, q8, sin
 @pytest.mark.parametrize("T_,n_kv,NH,NKV,HD,seen,kq,sinks,reader", [
     (3, 900, 8, 2, 128, 300, False, True, None), (3, 900, 8, 2, 128, 300, False, False, None), (5, 500, 8, 2, 128, 200, True, True, None), (4, 1024, 7, 1, 64, 200, False, True, None), (4, 1024, 8, 2, 64, 900, False, False, None),
     (24, 640, 32, 8, 128, 100, False, True, None), (3, 900, 8, 2, 128, 300, False, True, "Q4_K"), (3, 900, 8, 2, 128, 300, False, False, "Q4_K"), (24, 640, 32, 8, 128, 100, False, False, "Q4_K"),
-    (24, 640, 16, 8, 128, 100, True, True, "Q6_K"), (4, 1024, 8, 2, 64, 200, False, False, "Q8_0"), (4, 1024, 8, 2, 64, 900, False, False, "Q8_0"), (4, 1024, 8, 2, 64, 200, False, True, "Q8_0")])
+    (24, 640, 16, 8, 128, 100, True, True, "Q6_K"), (4, 1024, 8, 2, 64, 200, False, False, "Q8_0"), (4, 1024, 8, 2, 64, 900, False, False, "Q8_0"), (4, 1024, 8, 2, 64, 200, False, True, "Q8_0"), (1, 256, 8, 2, 128, 100, False, True, None),
+    (1, 256, 8, 2, 128, 100, False, False, None), (1, 300, 14, 2, 128, 100, False, True, "Q4_K"), (1, 200, 8, 2, 128, 100, True, True, None), (1, 700, 8, 1, 64, 100, False, True, None), (1, 700, 8, 1, 64, 100, False, False, None)])
 def test_token_without_cells(backend, H, T_, n_kv, NH, NKV, HD, seen, kq, sinks, reader):
     """one pass against splits and their merge (option fa_splits), where the merge speaks for such a token"""
     rng = np.random.default_rng(T_ + n_kv + NH)
