@@ -1702,7 +1702,7 @@ static bool plan_rope_store(const exec_state & st, int i, rope_store_plan & pl) 
     // cache stores: f16 or Q8_0 rows of NKV * HD values, one I64 index per token, both stores through the same indices
     auto q8_rows = [&](const ggml_tensor * sr) { return sr->type == GGML_TYPE_Q8_0 && (HD % 64) == 0 && rq->op_params[1] == HD && (sr->nb[1] % 2) == 0 && ((uintptr_t) sr->data & 1) == 0; };
     auto store_ok = [&](const ggml_tensor * sr, const ggml_tensor * src) {
-        return ((sr->type == GGML_TYPE_F16 && sr->nb[0] == 2) || q8_rows(sr)) && sr->ne[0] == NKV * HD && src->ne[0] == NKV * HD && ggml_abi_nelements(src) == NKV * HD * T &&
+        return ((sr->type == GGML_TYPE_F16 && sr->nb[0] == 2) || q8_rows(sr)) && sr->ne[0] == NKV * HD && src->ne[0] == NKV * HD && ggml_abi_nelements(src) == NKV * HD * T && ggml_abi_is_contiguous(src) &&
                sr->src[1]->type == GGML_TYPE_I64 && ggml_abi_nelements(sr->src[1]) == T && ggml_abi_is_contiguous(sr->src[1]);
     };
     // ... or, on the non-flash path, V transposed: the projection viewed as rows of ONE element, an index per element

@@ -700,8 +700,9 @@ def test_rows_of_a_step_in_one_launch(backend, H, T_, NH, NKV, D, rot, mode, exa
         assert np.array_equal(a.view(np.uint8), b.view(np.uint8))
 
 
-def test_rows_of_a_step_stored_from_a_strided_view(backend, H):
-    """the rotated keys' rows for the cache overlap (a view with a row stride of one head): not the rows that the launch of a step stores"""
+@pytest.mark.parametrize("kv_type", [L.BF16, L.F16])
+def test_rows_of_a_step_stored_from_a_strided_view(backend, H, kv_type):
+    """the rotated keys' rows for the cache overlap (a view with a row stride of one head): not the rows that the launches of a step store"""
     T_, NH, NKV, D = 6, 4, 3, 64
     rng = np.random.default_rng(3)
     q, k, v = (rng.standard_normal((T_, n * D)).astype(np.float32) for n in (NH, NKV, NKV))
@@ -709,7 +710,7 @@ def test_rows_of_a_step_stored_from_a_strided_view(backend, H):
 
     def build(g):
         p, rows = g.new(L.I32, [T_], pos), g.new(L.I64, [T_], idx)
-        caches = [g.new(L.BF16, [NKV * D, 20], np.zeros((20, NKV * D), np.uint16)) for _ in range(2)]
+        caches = [g.new(kv_type, [NKV * D, 20], np.zeros((20, NKV * D), np.uint16)) for _ in range(2)]
         rq, rk = (H.ggml_rope_ext(g.ctx, g.new(L.F32, [D, n, T_], x), p, None, D, 0, 4096, 10000.0, 1.0, 0.0, 1.0, 32.0, 1.0) for n, x in ((NH, q), (NKV, k)))
         g.first = [rq, rk]
         return [H.ggml_set_rows(g.ctx, caches[0], H.ggml_view_2d(g.ctx, rk, NKV * D, T_, D * 4, 0), rows), H.ggml_set_rows(g.ctx, caches[1], g.new(L.F32, [NKV * D, T_], v), rows), H.ggml_scale(g.ctx, rq, 1.0)]
