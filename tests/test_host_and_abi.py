@@ -562,6 +562,39 @@ def test_scratch_holds_the_slices_of_merged_launches():
     assert not short, (len(short), short[:5])
 
 
+def test_kept_graphs_when_the_buffer_cannot_grow(H):
+    """no memory for a larger shape: the call fails, the graphs kept in the buffer that was given up go with it, and later calls build theirs anew"""
+    fn = T.oracle_compute_fn(2)
+    buft = H.ggml_backend_cpu_buffer_type()
+    m = Model(preset("test-llama"), 5, buft)
+    c, anew = Context(m, compute=fn, graph_reuse=2), Context(m, compute=fn, graph_reuse=0)
+    out = (C.c_int64 * 3)()
+
+    def step(ctx, n):
+        H.llm_kv_seq_rm(ctx.c, -1, 0, -1)
+        return ctx.decode(np.arange(n) + 7, range(n), want=[0] * (n - 1) + [1])
+
+    fields = C.cast(buft, C.POINTER(C.c_void_p))  # (the type's interface: name, allocation, ..)
+    alloc, none = fields[1], C.CFUNCTYPE(C.c_void_p, C.c_void_p, C.c_size_t)(lambda buft, size: None)
+    for n in (5, 3, 1):
+        assert step(c, n)[0] == 0
+    fields[1] = C.cast(none, C.c_void_p).value
+    try:
+        for _ in range(2):
+            assert step(c, 12)[0] == -2
+    finally:
+        fields[1] = alloc
+    H.llm_graph_stats(c.c, out)
+    assert list(out) == [5, 0, 3]
+    for n in (3, 12, 5, 3):
+        (rc, got), (_, ref) = step(c, n), step(anew, n)
+        assert rc == 0 and np.array_equal(got, ref)
+    H.llm_graph_stats(c.c, out)
+    assert list(out) == [9, 0, 4]  # (the graph of 3 goes as 12 tokens come)
+    for x in (c, anew, m):
+        x.free()
+
+
 def built_kernels():
     """{symbol: metadata} of the gfx950 kernels in the built library (the code objects' AMDGPU metadata notes)"""
     msgpack = pytest.importorskip("msgpack")
